@@ -34,7 +34,7 @@ class Params(ctypes.Structure):
                               "initial_f", "initial_b", "dfinal_f", "dfinal_b", "dinitial_f", "dinitial_b", "seq_idx",
                               "states16_f", "states16_b", "dstates16_f", "dstates16_b", "workspace")]
         + [("workspace_bytes", ctypes.c_size_t), ("stream", _vp)]
-        + [(n, _i64) for n in ("dx_sb", "dx_sl", "dB_sb", "dB_sl", "dC_sb", "dC_sl")]
+        + [(n, _i64) for n in ("dx_sb", "dx_sl", "dB_sb", "dB_sl", "dC_sb", "dC_sl", "ddt_sb", "ddt_sl")]
     )
 
 
@@ -49,7 +49,7 @@ ENTRY_POINTS = (
 NORM_ENTRY_POINTS = ("bimamba2_rmsnorm_gated_fwd", "bimamba2_rmsnorm_gated_bwd")
 CONV_ENTRY_POINTS = ("bimamba2_conv1d_silu_fwd", "bimamba2_conv1d_silu_bwd")
 ALL_SYMBOLS = ENTRY_POINTS + ("bimamba2_strerror", "bimamba2_version", "bimamba2_params_size",
-                              "bimamba2_workspace_bytes", "bimamba2_chunk_scan_reads_cb", "bimamba2_state_copies",
+                              "bimamba2_workspace_bytes", "bimamba2_seq_boundaries", "bimamba2_chunk_scan_reads_cb", "bimamba2_state_copies",
                               "bimamba2_chunk_scan_heads_per_workgroup", "bimamba2_ddt_direct_planes", "bimamba2_norm_params_size",
                               "bimamba2_rmsnorm_gated_workspace_bytes", "bimamba2_conv_params_size",
                               "bimamba2_conv1d_silu_workspace_bytes", "bimamba2_cast_params_size",
@@ -116,6 +116,8 @@ def load():
     lib.bimamba2_chunk_scan_heads_per_workgroup.restype = ctypes.c_int
     lib.bimamba2_ddt_direct_planes.argtypes = [ctypes.POINTER(Params)]
     lib.bimamba2_ddt_direct_planes.restype = ctypes.c_int
+    lib.bimamba2_seq_boundaries.argtypes = [ctypes.POINTER(Params), _vp]
+    lib.bimamba2_seq_boundaries.restype = ctypes.c_int
     lib.bimamba2_state_copies.argtypes = [ctypes.POINTER(Params)]
     lib.bimamba2_state_copies.restype = ctypes.c_int
     lib.bimamba2_params_size.restype = ctypes.c_size_t
@@ -148,6 +150,25 @@ def load():
     lib.bimamba2_cast_many.restype = ctypes.c_int
     _lib = lib
     return lib
+
+
+_host = None
+
+
+def host():
+    """The native host path (csrc/host.cpp, built beside the library): the operator's and the layer's autograd functions.
+    Raises RuntimeError when it or the library is missing."""
+    global _host
+    if _host is None:
+        load()
+        try:
+            from . import _host as module
+        except ImportError as exc:
+            raise RuntimeError(f"bi_mamba2_amd/_host.so is missing or does not load ({exc}): run `make -C {_HERE}/csrc`. "
+                               "There is no CPU or PyTorch fallback for this operator.") from exc
+        module.load(LIB_PATH)
+        _host = module
+    return _host
 
 
 def call(name, params):

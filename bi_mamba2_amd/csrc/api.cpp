@@ -217,6 +217,13 @@ int bimamba2_ddt_direct_planes(const bimamba2_params *p) {
     return ddt_direct_planes(*p);
 }
 
+int bimamba2_seq_boundaries(const bimamba2_params *p, int32_t *counts) {
+    TRY(check_problem(p));
+    REQUIRE(p->seq_idx); REQUIRE(counts);
+    if (p->batch > 65535) return BIMAMBA2_EUNSUPPORTED;
+    return launch_seq_boundaries(p, counts);
+}
+
 int bimamba2_chunk_cumsum_fwd(const bimamba2_params *p) {
     TRY(check_problem(p));
     REQUIRE(p->dt); REQUIRE(p->A); REQUIRE(p->dt_out); REQUIRE(p->cs_f); REQUIRE(p->cs_b);

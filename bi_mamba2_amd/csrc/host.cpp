@@ -1,0 +1,757 @@
+// The host path of the operator and of the BiMamba2 layer in native code: argument checks, parameter block, memory and the
+// autograd functions around bimamba2_fwd / bimamba2_bwd and the layer's other kernels.
+//
+// Why it exists: a forward + backward pass through Python (ctypes parameter block, autograd functions whose backward needs
+// the interpreter lock, one torch op per small map) took the host 0.18 - 0.37 ms, the layer's 1.0 ms, which is more than the
+// kernels take at every small or ordinary size.  The functions here do the same checks, make the same launches and leave the
+// same tensors for the backward pass; the interpreter lock is released while they run.
+//
+// Built as a Python module (bi_mamba2_amd/_host.so); load(path) opens libbimamba2_hip.so and resolves the C ABI, so the
+// module follows the library the Python side was told to use.
+#include <dlfcn.h>
+#include <torch/extension.h>
+#include <c10/hip/HIPStream.h>
+#include <c10/hip/HIPGuard.h>
+#include <hip/hip_runtime_api.h>
+
+#include <algorithm>
+#include <array>
+#include <optional>
+#include <string>
+#include <vector>
+
+#include "../../include/bimamba2.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+using OptTensor = std::optional<Tensor>;
+
+struct AssertionFailure : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+#define BM2_ASSERT(cond, what) \
+    do {                       \
+        if (!(cond)) throw AssertionFailure(what); \
+    } while (0)
+
+struct Api {
+    decltype(&bimamba2_fwd) fwd = nullptr;
+    decltype(&bimamba2_bwd) bwd = nullptr;
+    decltype(&bimamba2_workspace_bytes) workspace_bytes = nullptr;
+    decltype(&bimamba2_state_copies) state_copies = nullptr;
+    decltype(&bimamba2_seq_boundaries) seq_boundaries = nullptr;
+    decltype(&bimamba2_strerror) strerror = nullptr;
+    decltype(&bimamba2_rmsnorm_gated_fwd) norm_fwd = nullptr;
+    decltype(&bimamba2_rmsnorm_gated_bwd) norm_bwd = nullptr;
+    decltype(&bimamba2_rmsnorm_gated_workspace_bytes) norm_workspace = nullptr;
+    decltype(&bimamba2_conv1d_silu_fwd) conv_fwd = nullptr;
+    decltype(&bimamba2_conv1d_silu_bwd) conv_bwd = nullptr;
+    decltype(&bimamba2_conv1d_silu_workspace_bytes) conv_workspace = nullptr;
+    decltype(&bimamba2_cast_many) cast_many = nullptr;
+} api;
+
+void load(const std::string &path) {
+    void *lib = dlopen(path.c_str(), RTLD_NOW | RTLD_LOCAL);
+    TORCH_CHECK(lib, "cannot open ", path, ": ", dlerror());
+    auto get = [&](auto &fn, const char *name) {
+        fn = reinterpret_cast<std::remove_reference_t<decltype(fn)>>(dlsym(lib, name));
+        TORCH_CHECK(fn, path, " does not export ", name);
+    };
+    size_t (*params_size)() = nullptr, (*norm_size)() = nullptr, (*conv_size)() = nullptr, (*cast_size)() = nullptr;
+    get(params_size, "bimamba2_params_size");
+    get(norm_size, "bimamba2_norm_params_size");
+    get(conv_size, "bimamba2_conv_params_size");
+    get(cast_size, "bimamba2_cast_params_size");
+    TORCH_CHECK(params_size() == sizeof(bimamba2_params) && norm_size() == sizeof(bimamba2_norm_params) &&
+                    conv_size() == sizeof(bimamba2_conv_params) && cast_size() == sizeof(bimamba2_cast_params),
+                path, " was built from another version of include/bimamba2.h");
+    get(api.fwd, "bimamba2_fwd");
+    get(api.bwd, "bimamba2_bwd");
+    get(api.workspace_bytes, "bimamba2_workspace_bytes");
+    get(api.state_copies, "bimamba2_state_copies");
+    get(api.seq_boundaries, "bimamba2_seq_boundaries");
+    get(api.strerror, "bimamba2_strerror");
+    get(api.norm_fwd, "bimamba2_rmsnorm_gated_fwd");
+    get(api.norm_bwd, "bimamba2_rmsnorm_gated_bwd");
+    get(api.norm_workspace, "bimamba2_rmsnorm_gated_workspace_bytes");
+    get(api.conv_fwd, "bimamba2_conv1d_silu_fwd");
+    get(api.conv_bwd, "bimamba2_conv1d_silu_bwd");
+    get(api.conv_workspace, "bimamba2_conv1d_silu_workspace_bytes");
+    get(api.cast_many, "bimamba2_cast_many");
+}
+
+void check(int rc, const char *entry) {
+    if (rc == BIMAMBA2_OK) return;
+    const std::string msg = std::string(entry) + ": " + api.strerror(rc) + " (code " + std::to_string(rc) + ")";
+    if (rc == BIMAMBA2_EINVAL || rc == BIMAMBA2_EUNSUPPORTED || rc == BIMAMBA2_ESCRATCH) TORCH_CHECK_VALUE(false, msg);
+    TORCH_CHECK(false, msg);
+}
+
+void *stream_of(const Tensor &t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
+
+int dtype_code(at::ScalarType t, const char *what) {
+    switch (t) {
+        case at::kFloat: return BIMAMBA2_F32;
+        case at::kBFloat16: return BIMAMBA2_BF16;
+        case at::kHalf: return BIMAMBA2_F16;
+        default: TORCH_CHECK_VALUE(false, "unsupported ", what, " ", t, " (need float32, bfloat16 or float16)"); return -1;
+    }
+}
+
+void require_gpu(const Tensor &t, const char *name) {
+    TORCH_CHECK(t.is_cuda(), name, " is on ", t.device(),
+                ": the bidirectional SSD kernels run on an AMD GPU only (there is no CPU fallback)");
+}
+
+inline bool aligned16(const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; }
+inline size_t round_up(size_t n, size_t to) { return (n + to - 1) / to * to; }
+inline Tensor as_type(const Tensor &t, at::ScalarType dtype) { return t.scalar_type() == dtype ? t : t.to(dtype); }
+inline Tensor undef(const OptTensor &t) { return t ? *t : Tensor(); }
+
+// float32 contiguous form of a parameter (A, D, dt_bias) or state
+inline Tensor f32c(const Tensor &t) { return as_type(t, at::kFloat).contiguous(); }
+
+// ---------------------------------------------------------------------------------------------------------------------
+// the operator
+// ---------------------------------------------------------------------------------------------------------------------
+struct ScanOpts : torch::CustomClassHolder {
+    int64_t chunk = 0;
+    bool dt_softplus = false, want_final = false;
+    bool copies = false;          // the forward kept the states in 16 bits
+    double dt_min = 0, dt_max = 0;
+};
+
+// The operands in the form the kernels take (16-bit or float32 rows with the last dimension contiguous, float32
+// parameters) and the parameter block that points at them.
+struct Problem {
+    bimamba2_params p{};
+    Tensor x, dt, A, B, C, D, z, bias, init_f, init_b, seq;
+
+    Tensor strided(const Tensor &t, const char *name, const void *&ptr, int64_t &s0, int64_t &s1, int64_t &s2) {
+        require_gpu(t, name);
+        Tensor r = as_type(t, x.scalar_type());
+        if (r.stride(-1) != 1) r = r.contiguous();
+        ptr = r.const_data_ptr();
+        s0 = r.stride(0);
+        s1 = r.stride(1);
+        s2 = r.stride(2);
+        return r;
+    }
+    Tensor param(const Tensor &t, const char *name, const float *&ptr) {
+        require_gpu(t, name);
+        Tensor r = f32c(t);
+        ptr = r.const_data_ptr<float>();
+        return r;
+    }
+
+    Problem(const Tensor &x_, const Tensor &dt_, const Tensor &A_, const Tensor &B_, const Tensor &C_, const Tensor &D_,
+            const Tensor &z_, const Tensor &bias_, const Tensor &init_f_, const Tensor &init_b_, const Tensor &seq_,
+            const ScanOpts &o) {
+        BM2_ASSERT(x_.dim() == 4 && B_.dim() == 4, "x: expected (batch, seqlen, nheads, headdim), B: (batch, seqlen, ngroups, dstate)");
+        const int64_t batch = x_.size(0), seqlen = x_.size(1), nheads = x_.size(2), headdim = x_.size(3);
+        const int64_t ngroups = B_.size(2), dstate = B_.size(3);
+        BM2_ASSERT(ngroups > 0 && nheads % ngroups == 0, "nheads must be a multiple of ngroups");
+        BM2_ASSERT(B_.size(0) == batch && B_.size(1) == seqlen, "B: expected (batch, seqlen, ngroups, dstate)");
+        BM2_ASSERT(dt_.sizes() == at::IntArrayRef({batch, seqlen, nheads}), "dt: expected (batch, seqlen, nheads)");
+        BM2_ASSERT(A_.sizes() == at::IntArrayRef({nheads}), "A: expected (nheads,)");
+        BM2_ASSERT(C_.sizes() == B_.sizes(), "C: expected the shape of B");
+        BM2_ASSERT(o.chunk >= 32, "chunk_size must be at least 32 (as in the reference) and at most 256");
+        BM2_ASSERT(!z_.defined() || z_.sizes() == x_.sizes(), "z: expected the shape of x");
+        BM2_ASSERT(!D_.defined() || D_.sizes() == at::IntArrayRef({nheads}) || D_.sizes() == at::IntArrayRef({nheads, headdim}),
+                   "D: expected (nheads,) or (nheads, headdim)");
+        BM2_ASSERT(!bias_.defined() || bias_.sizes() == at::IntArrayRef({nheads}), "dt_bias: expected (nheads,)");
+        require_gpu(x_, "x");
+        p.batch = batch; p.seqlen = seqlen; p.nheads = nheads; p.headdim = headdim;
+        p.ngroups = ngroups; p.dstate = dstate; p.chunk_size = o.chunk;
+        p.dtype = dtype_code(x_.scalar_type(), "dtype");
+        p.dt_dtype = dtype_code(dt_.scalar_type(), "dt dtype");
+        p.dt_softplus = o.dt_softplus;
+        p.dt_min = (float)o.dt_min;
+        p.dt_max = (float)o.dt_max;
+        x = x_;
+        x = strided(x_, "x", p.x, p.x_sb, p.x_sl, p.x_sh);
+        require_gpu(dt_, "dt");
+        dt = dt_;
+        p.dt = dt.const_data_ptr();
+        p.dt_sb = dt.stride(0); p.dt_sl = dt.stride(1); p.dt_sh = dt.stride(2);
+        A = param(A_, "A", p.A);
+        B = strided(B_, "Bm", p.Bm, p.B_sb, p.B_sl, p.B_sg);
+        C = strided(C_, "Cm", p.Cm, p.C_sb, p.C_sl, p.C_sg);
+        if (D_.defined()) {
+            p.has_D = 1;
+            p.D_has_hdim = D_.dim() == 2;
+            D = param(D_, "D", p.D);
+        }
+        if (z_.defined()) {
+            p.has_z = 1;
+            z = strided(z_, "z", p.z, p.z_sb, p.z_sl, p.z_sh);
+        }
+        if (bias_.defined()) {
+            p.has_dt_bias = 1;
+            bias = param(bias_, "dt_bias", p.dt_bias);
+        }
+        if (init_f_.defined()) {
+            BM2_ASSERT(init_f_.sizes() == at::IntArrayRef({batch, nheads, headdim, dstate}), "initial_f: expected (batch, nheads, headdim, dstate)");
+            init_f = param(init_f_, "initial_f", p.initial_f);
+        }
+        if (init_b_.defined()) {
+            BM2_ASSERT(init_b_.sizes() == at::IntArrayRef({batch, nheads, headdim, dstate}), "initial_b: expected (batch, nheads, headdim, dstate)");
+            init_b = param(init_b_, "initial_b", p.initial_b);
+        }
+        if (seq_.defined()) {
+            BM2_ASSERT(seq_.sizes() == at::IntArrayRef({batch, seqlen}), "seq_idx: expected (batch, seqlen)");
+            require_gpu(seq_, "seq_idx");
+            seq = as_type(seq_, at::kInt).contiguous();
+            p.seq_idx = seq.const_data_ptr<int32_t>();
+        }
+        p.stream = stream_of(x);
+    }
+};
+
+// What the forward pass leaves for the backward pass besides its operands, in one float32 allocation: dt_out, cs_f, cs_b and
+// the states entering the chunks (copies: in the operands' 16-bit type, where the kernels can keep them that way).
+struct Kept {
+    size_t n1 = 0, ns = 0;
+    bool copies = false;
+    Kept(const bimamba2_params &p, bool copies_) : copies(copies_) {
+        const size_t nc = (p.seqlen + p.chunk_size - 1) / p.chunk_size;
+        n1 = round_up((size_t)p.batch * p.nheads * nc * p.chunk_size, 64);
+        ns = round_up((size_t)p.batch * nc * p.nheads * p.headdim * p.dstate, 64);
+        if (copies) ns /= 2;
+    }
+    int64_t floats() const { return (int64_t)(3 * n1 + 2 * ns); }
+    void point(bimamba2_params &p, float *base) const {
+        p.dt_out = base;
+        p.cs_f = base + n1;
+        p.cs_b = base + 2 * n1;
+        float *st = base + 3 * n1;
+        if (copies) {
+            p.states16_f = st;
+            p.states16_b = st + ns;
+        } else {
+            p.states_f = st;
+            p.states_b = st + ns;
+        }
+    }
+};
+
+Tensor attach_workspace(bimamba2_params &p, bool bwd, const at::TensorOptions &like) {
+    Tensor ws = at::empty({(int64_t)std::max<size_t>(api.workspace_bytes(&p, bwd), 1)}, like.dtype(at::kByte));
+    p.workspace = ws.mutable_data_ptr();
+    p.workspace_bytes = ws.numel();
+    return ws;
+}
+
+struct ScanResult {
+    Tensor out, out_x, final_f, final_b, kept;
+};
+
+ScanResult scan_forward(Problem &q, ScanOpts &o, bool keep) {
+    bimamba2_params &p = q.p;
+    ScanResult r;
+    const auto f32 = q.x.options().dtype(at::kFloat);
+    if (keep) {
+        o.copies = api.state_copies(&p) != 0;
+        const Kept k(p, o.copies);
+        r.kept = at::empty({k.floats()}, f32);
+        k.point(p, r.kept.mutable_data_ptr<float>());
+    }
+    r.out = at::empty(q.x.sizes(), q.x.options());
+    p.out = r.out.mutable_data_ptr();
+    if (keep && p.has_z) {        // the pre-gate output is what a backward pass needs; without one the store is skipped
+        r.out_x = at::empty(q.x.sizes(), q.x.options());
+        p.out_x = r.out_x.mutable_data_ptr();
+    }
+    if (o.want_final) {
+        const std::array<int64_t, 4> st = {p.batch, p.nheads, p.headdim, p.dstate};
+        r.final_f = at::empty(st, f32);
+        r.final_b = at::empty(st, f32);
+        p.final_f = r.final_f.mutable_data_ptr<float>();
+        p.final_b = r.final_b.mutable_data_ptr<float>();
+    }
+    const Tensor ws = attach_workspace(p, false, q.x.options());
+    check(api.fwd(&p), "bimamba2_fwd");
+    return r;
+}
+
+// Packed sequences: the largest number of boundaries that falls into one chunk.  The count is taken on the device and written
+// to pinned host memory; the host waits for that kernel only, after it has enqueued the forward pass at the caller's chunk
+// size, so that the GPU has work while the host reads the answer (which nearly always is that the chunk size may stay).
+constexpr int64_t max_boundaries = BIMAMBA2_MAX_SEQ_BOUNDARIES;
+
+struct EventCache {
+    std::vector<hipEvent_t> of_device;
+    hipEvent_t get(int device) {
+        if ((int)of_device.size() <= device) of_device.resize(device + 1, nullptr);
+        if (!of_device[device]) TORCH_CHECK(hipEventCreateWithFlags(&of_device[device], hipEventDisableTiming) == hipSuccess, "hipEventCreate failed");
+        return of_device[device];
+    }
+    ~EventCache() {
+        for (hipEvent_t e : of_device)
+            if (e) (void)hipEventDestroy(e);
+    }
+};
+
+struct BoundaryCount {
+    Tensor counts;
+    hipEvent_t event = nullptr;
+    explicit BoundaryCount(const bimamba2_params &p, int device) {
+        static thread_local EventCache events;
+        const int64_t nc = (p.seqlen + p.chunk_size - 1) / p.chunk_size;
+        counts = at::empty({p.batch * nc}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
+        check(api.seq_boundaries(&p, counts.mutable_data_ptr<int32_t>()), "bimamba2_seq_boundaries");
+        event = events.get(device);
+        TORCH_CHECK(hipEventRecord(event, static_cast<hipStream_t>(p.stream)) == hipSuccess, "hipEventRecord failed");
+    }
+    int64_t wait() {
+        TORCH_CHECK(hipEventSynchronize(event) == hipSuccess, "waiting for the count of sequence boundaries failed");
+        const int32_t *c = counts.const_data_ptr<int32_t>();
+        return counts.numel() ? *std::max_element(c, c + counts.numel()) : 0;
+    }
+};
+
+template <typename MakeProblem> ScanResult scan_checked(MakeProblem make, ScanOpts &o, bool keep) {
+    Problem q = make(o);
+    if (!q.p.seq_idx || o.chunk <= max_boundaries) return scan_forward(q, o, keep);
+    BoundaryCount first(q.p, q.x.device().index());
+    ScanResult r = scan_forward(q, o, keep);
+    if (first.wait() <= max_boundaries) return r;
+    for (int64_t c : {128, 64, 32}) {
+        if (c >= o.chunk) continue;
+        o.chunk = c;
+        Problem smaller = make(o);
+        if (c <= max_boundaries || BoundaryCount(smaller.p, smaller.x.device().index()).wait() <= max_boundaries) return scan_forward(smaller, o, keep);
+    }
+    TORCH_CHECK_VALUE(false, "seq_idx puts more than ", max_boundaries, " sequence boundaries into every chunk size down to 32 positions");
+}
+
+class ScanFn : public torch::autograd::Function<ScanFn> {
+public:
+    static variable_list forward(AutogradContext *ctx, const Tensor &x, const Tensor &dt, const Tensor &A, const Tensor &B,
+                                 const Tensor &C, const OptTensor &D, const OptTensor &z, const OptTensor &bias,
+                                 const OptTensor &init_f, const OptTensor &init_b, const OptTensor &seq,
+                                 c10::intrusive_ptr<ScanOpts> o) {
+        ScanResult r = scan_checked([&](const ScanOpts &opts) {
+            return Problem(x, dt, A, B, C, undef(D), undef(z), undef(bias), undef(init_f), undef(init_b), undef(seq), opts);
+        }, *o, true);
+        ctx->save_for_backward({x, dt, A, B, C, undef(D), undef(z), undef(bias), undef(init_f), undef(init_b), undef(seq), r.out_x, r.kept});
+        ctx->saved_data["opts"] = c10::IValue::make_capsule(o);
+        ctx->set_materialize_grads(false);
+        if (!o->want_final) return {r.out};
+        return {r.out, r.final_f, r.final_b};
+    }
+
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const variable_list s = ctx->get_saved_variables();
+        const auto capsule = ctx->saved_data["opts"].toCapsule();
+        const ScanOpts &o = *static_cast<const ScanOpts *>(capsule.get());
+        const Tensor &x = s[0], &dt = s[1], &A = s[2], &B = s[3], &C = s[4], &D = s[5], &bias = s[7];
+        const c10::DeviceGuard guard(x.device());
+        Problem q(x, dt, A, B, C, D, s[6], bias, s[8], s[9], s[10], o);
+        bimamba2_params &p = q.p;
+        const auto f32 = q.x.options().dtype(at::kFloat);
+        Tensor dout = grads[0].defined() ? grads[0] : at::zeros(x.sizes(), q.x.options());
+        BM2_ASSERT(dout.sizes() == x.sizes(), "gradient of the output: expected the shape of x");
+        dout = as_type(dout, x.scalar_type());
+        // the kernels that read the kept 16-bit states take aligned rows: a gradient view that is not (a slice of a wider
+        // tensor at an odd offset) is copied
+        bool even = dout.stride(-1) == 1;
+        if (even && p.dtype != BIMAMBA2_F32)
+            even = aligned16(dout.const_data_ptr()) && dout.stride(0) % 8 == 0 && dout.stride(1) % 8 == 0 && dout.stride(2) % 8 == 0;
+        if (!even) dout = dout.contiguous();
+        p.dout = dout.const_data_ptr();
+        p.dout_sb = dout.stride(0); p.dout_sl = dout.stride(1); p.dout_sh = dout.stride(2);
+        Tensor dfin_f, dfin_b, dinit_f, dinit_b;
+        if (grads.size() > 1 && grads[1].defined()) dfin_f = q.param(grads[1], "dfinal_f", p.dfinal_f);
+        if (grads.size() > 2 && grads[2].defined()) dfin_b = q.param(grads[2], "dfinal_b", p.dfinal_b);
+        const std::array<int64_t, 4> st = {p.batch, p.nheads, p.headdim, p.dstate};
+        if (q.init_f.defined()) {
+            dinit_f = at::empty(st, f32);
+            p.dinitial_f = dinit_f.mutable_data_ptr<float>();
+        }
+        if (q.init_b.defined()) {
+            dinit_b = at::empty(st, f32);
+            p.dinitial_b = dinit_b.mutable_data_ptr<float>();
+        }
+        Tensor kept = s[12];
+        Kept(p, o.copies).point(p, kept.mutable_data_ptr<float>());
+        p.fwd_saved = 1;
+        Tensor dz, dD, dbias, out_x = s[11];
+        if (p.has_z) {
+            out_x = out_x.contiguous();
+            p.out_x = out_x.mutable_data_ptr();
+            dz = at::empty(x.sizes(), q.x.options());
+            p.dz = dz.mutable_data_ptr();
+        }
+        Tensor dx = at::empty(x.sizes(), q.x.options()), ddt = at::empty(dt.sizes(), dt.options()), dB = at::empty(B.sizes(), q.x.options()),
+               dC = at::empty(C.sizes(), q.x.options()), dA = at::empty(A.sizes(), f32);
+        p.dx = dx.mutable_data_ptr();
+        p.ddt = ddt.mutable_data_ptr();
+        p.dB = dB.mutable_data_ptr();
+        p.dC = dC.mutable_data_ptr();
+        p.dA = dA.mutable_data_ptr<float>();
+        if (D.defined()) {
+            dD = at::empty(D.sizes(), f32);
+            p.dD = dD.mutable_data_ptr<float>();
+        }
+        if (bias.defined()) {
+            dbias = at::empty(bias.sizes(), f32);
+            p.ddt_bias = dbias.mutable_data_ptr<float>();
+        }
+        const Tensor ws = attach_workspace(p, true, q.x.options());
+        check(api.bwd(&p), "bimamba2_bwd");
+        auto like = [](const Tensor &g, const Tensor &t) { return g.defined() ? as_type(g, t.scalar_type()) : g; };
+        return {dx, ddt, like(dA, A), like(dB, B), like(dC, C), like(dD, D), dz.defined() ? like(dz, s[6]) : dz, like(dbias, bias),
+                dinit_f, dinit_b, Tensor(), Tensor()};
+    }
+};
+
+inline bool wants_grad(std::initializer_list<const Tensor *> ts) {
+    if (!at::GradMode::is_enabled()) return false;
+    for (const Tensor *t : ts)
+        if (t->defined() && t->requires_grad()) return true;
+    return false;
+}
+
+variable_list scan(const Tensor &x, const Tensor &dt, const Tensor &A, const Tensor &B, const Tensor &C, int64_t chunk,
+                   const OptTensor &D, const OptTensor &z, const OptTensor &bias, bool dt_softplus, double dt_min, double dt_max,
+                   bool want_final, const OptTensor &init_f, const OptTensor &init_b, const OptTensor &seq) {
+    const Tensor D_ = undef(D), z_ = undef(z), b_ = undef(bias), f_ = undef(init_f), r_ = undef(init_b);
+    auto o = c10::make_intrusive<ScanOpts>();
+    o->chunk = chunk;
+    o->dt_softplus = dt_softplus;
+    o->want_final = want_final;
+    o->dt_min = dt_min;
+    o->dt_max = dt_max;
+    c10::OptionalDeviceGuard guard;
+    if (x.is_cuda()) guard.reset_device(x.device());
+    if (wants_grad({&x, &dt, &A, &B, &C, &D_, &z_, &b_, &f_, &r_})) return ScanFn::apply(x, dt, A, B, C, D, z, bias, init_f, init_b, seq, o);
+    at::AutoDispatchBelowADInplaceOrView below;
+    ScanResult r = scan_checked([&](const ScanOpts &opts) { return Problem(x, dt, A, B, C, D_, z_, b_, f_, r_, undef(seq), opts); }, *o, false);
+    if (!want_final) return {r.out};
+    return {r.out, r.final_f, r.final_b};
+}
+
+// ---------------------------------------------------------------------------------------------------------------------
+// the BiMamba2 layer: in_proj -> [z | xBC | dt] -> conv + SiLU -> operator -> gated RMS norm -> out_proj
+// ---------------------------------------------------------------------------------------------------------------------
+struct LayerOpts : torch::CustomClassHolder {
+    int64_t inner = 0, nheads = 0, headdim = 0, ngroups = 0, dstate = 0, chunk = 0, norm_group = 0;
+    bool norm_before_gate = true;
+    uint32_t needs = 0;           // bit i: input i of LayerFn takes a gradient
+    bool copies = false;          // the forward kept the states in 16 bits
+    double dt_min = 0, dt_max = 0, eps = 0;
+};
+
+// The layer's small parameters as the kernels take them: float32, A = -exp(A_log).  One launch for all of them.
+struct Params32 {
+    // A_log, D, dt_bias, conv weight, conv bias, norm weight
+    static constexpr int N = 6;
+    std::array<const float *, N> ptr{};
+    Tensor buf;       // holds what had to be converted; null where the parameters are used as they are
+};
+
+void add_cast(bimamba2_cast_params &c, const Tensor &src, void *dst, int dst_dtype, int op, const float *aux = nullptr) {
+    bimamba2_cast_item &it = c.item[c.count++];
+    it.src = src.const_data_ptr();
+    it.dst = dst;
+    it.aux = aux;
+    it.n = src.numel();
+    it.src_dtype = dtype_code(src.scalar_type(), "parameter dtype");
+    it.dst_dtype = dst_dtype;
+    it.op = op;
+}
+
+// offsets (in floats, 256-byte steps so that every piece is aligned for vector loads) of the pieces in Params32::buf; the
+// backward pass finds them again from the same parameters
+std::array<int64_t, Params32::N + 1> param_offsets(const std::array<Tensor, Params32::N> &prm) {
+    std::array<int64_t, Params32::N + 1> off{};
+    for (int i = 0; i < Params32::N; ++i) {
+        const bool converted = prm[i].defined() && (i == 0 || prm[i].scalar_type() != at::kFloat || !prm[i].is_contiguous());
+        off[i + 1] = off[i] + (converted ? (int64_t)round_up(prm[i].numel(), 64) : 0);
+    }
+    return off;
+}
+
+Params32 point_params(const std::array<Tensor, Params32::N> &prm, const Tensor &buf) {
+    const auto off = param_offsets(prm);
+    Params32 r;
+    r.buf = buf;
+    float *base = buf.mutable_data_ptr<float>();
+    for (int i = 0; i < Params32::N; ++i)
+        if (prm[i].defined()) r.ptr[i] = off[i + 1] > off[i] ? base + off[i] : prm[i].const_data_ptr<float>();
+    return r;
+}
+
+Params32 params_as_float32(std::array<Tensor, Params32::N> &prm, void *stream) {
+    const auto off = param_offsets(prm);
+    const Tensor buf = at::empty({off.back()}, prm[0].options().dtype(at::kFloat));
+    Params32 r = point_params(prm, buf);
+    bimamba2_cast_params c{};
+    c.stream = stream;
+    std::array<Tensor, Params32::N> rows;
+    for (int i = 0; i < Params32::N; ++i)
+        if (off[i + 1] > off[i]) {
+            rows[i] = prm[i].contiguous();
+            add_cast(c, rows[i], const_cast<float *>(r.ptr[i]), BIMAMBA2_F32, i == 0 ? BIMAMBA2_CAST_NEG_EXP : BIMAMBA2_CAST_COPY);
+        }
+    check(api.cast_many(&c), "bimamba2_cast_many");
+    return r;
+}
+
+struct LayerShape {
+    int64_t batch, seqlen, rows, inner, conv, proj, width;
+    size_t e;
+    LayerShape(const Tensor &u, const Tensor &cw, const LayerOpts &o)
+        : batch(u.size(0)), seqlen(u.size(1)), rows(batch * seqlen), inner(o.inner), conv(o.inner + 2 * o.ngroups * o.dstate),
+          proj(o.inner + conv + o.nheads), width(cw.size(-1)), e(u.element_size()) {}
+};
+
+inline char *at_byte(const Tensor &t, size_t elements) { return static_cast<char *>(t.mutable_data_ptr()) + elements * t.element_size(); }
+
+bimamba2_conv_params conv_params(const LayerShape &s, const Tensor &zx, const Params32 &w, void *stream) {
+    bimamba2_conv_params c{};
+    c.batch = s.batch; c.seqlen = s.seqlen; c.channels = s.conv; c.width = s.width;
+    c.dtype = dtype_code(zx.scalar_type(), "dtype");
+    c.has_bias = w.ptr[4] != nullptr;
+    c.x = at_byte(zx, s.inner);
+    c.x_sb = s.seqlen * s.proj;
+    c.x_sl = s.proj;
+    c.weight = w.ptr[3];
+    c.bias = w.ptr[4];
+    c.stream = stream;
+    return c;
+}
+
+bimamba2_params layer_scan_params(const LayerShape &s, const LayerOpts &o, const Tensor &zx, const Tensor &xbc, const Params32 &w, void *stream) {
+    bimamba2_params p{};
+    p.batch = s.batch; p.seqlen = s.seqlen; p.nheads = o.nheads; p.headdim = o.headdim;
+    p.ngroups = o.ngroups; p.dstate = o.dstate; p.chunk_size = o.chunk;
+    p.dtype = p.dt_dtype = dtype_code(zx.scalar_type(), "dtype");
+    p.dt_softplus = 1;
+    p.dt_min = (float)o.dt_min; p.dt_max = (float)o.dt_max;
+    p.has_D = 1; p.has_dt_bias = 1;
+    p.x = at_byte(xbc, 0);
+    p.x_sb = s.seqlen * s.conv; p.x_sl = s.conv; p.x_sh = o.headdim;
+    p.Bm = at_byte(xbc, s.inner);
+    p.Cm = at_byte(xbc, s.inner + o.ngroups * o.dstate);
+    p.B_sb = p.C_sb = s.seqlen * s.conv; p.B_sl = p.C_sl = s.conv; p.B_sg = p.C_sg = o.dstate;
+    p.dt = at_byte(zx, s.inner + s.conv);
+    p.dt_sb = s.seqlen * s.proj; p.dt_sl = s.proj; p.dt_sh = 1;
+    p.A = w.ptr[0]; p.D = w.ptr[1]; p.dt_bias = w.ptr[2];
+    p.stream = stream;
+    return p;
+}
+
+bimamba2_norm_params layer_norm_params(const LayerShape &s, const LayerOpts &o, const Tensor &zx, const Tensor &y, const Params32 &w, void *stream) {
+    bimamba2_norm_params n{};
+    n.rows = s.rows; n.cols = s.inner; n.group_size = o.norm_group;
+    n.dtype = dtype_code(zx.scalar_type(), "dtype");
+    n.has_z = 1;
+    n.norm_before_gate = o.norm_before_gate;
+    n.eps = (float)o.eps;
+    n.x = y.const_data_ptr(); n.x_rs = s.inner;
+    n.z = at_byte(zx, 0); n.z_rs = s.proj;
+    n.weight = w.ptr[5];
+    n.stream = stream;
+    return n;
+}
+
+struct LayerKept {
+    Tensor zx, xbc, y, yn, rstd, kept, prm32;
+};
+
+Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, std::array<Tensor, Params32::N> prm, const Tensor &w_out,
+                     const Tensor &b_out, LayerOpts &o, bool keep, LayerKept *left) {
+    const LayerShape s(u, prm[3], o);
+    void *stream = stream_of(u);
+    const Tensor u2 = u.reshape({s.rows, u.size(2)});
+    const Tensor zx = b_in.defined() ? at::addmm(b_in, u2, w_in.t()) : at::mm(u2, w_in.t());
+    const Params32 w = params_as_float32(prm, stream);
+    const auto f32 = u.options().dtype(at::kFloat);
+
+    const Tensor xbc = at::empty({s.rows, s.conv}, u.options());
+    bimamba2_conv_params c = conv_params(s, zx, w, stream);
+    c.out = xbc.mutable_data_ptr();
+    check(api.conv_fwd(&c), "bimamba2_conv1d_silu_fwd");
+
+    const Tensor y = at::empty({s.rows, s.inner}, u.options());
+    bimamba2_params p = layer_scan_params(s, o, zx, xbc, w, stream);
+    p.out = y.mutable_data_ptr();
+    Tensor kept;
+    if (keep) {
+        o.copies = api.state_copies(&p) != 0;
+        const Kept k(p, o.copies);
+        kept = at::empty({k.floats()}, f32);
+        k.point(p, kept.mutable_data_ptr<float>());
+    }
+    const Tensor ws = attach_workspace(p, false, u.options());
+    check(api.fwd(&p), "bimamba2_fwd");
+
+    const Tensor yn = at::empty({s.rows, s.inner}, u.options());
+    Tensor rstd;
+    bimamba2_norm_params n = layer_norm_params(s, o, zx, y, w, stream);
+    n.out = yn.mutable_data_ptr();
+    n.out_rs = s.inner;
+    if (keep) {
+        rstd = at::empty({s.rows, s.inner / o.norm_group}, f32);
+        n.rstd = rstd.mutable_data_ptr<float>();
+    }
+    check(api.norm_fwd(&n), "bimamba2_rmsnorm_gated_fwd");
+    const Tensor out = b_out.defined() ? at::addmm(b_out, yn, w_out.t()) : at::mm(yn, w_out.t());
+    if (left) *left = {zx, xbc, y, yn, rstd, kept, w.buf};
+    return out.view({s.batch, s.seqlen, w_out.size(0)});
+}
+
+class LayerFn : public torch::autograd::Function<LayerFn> {
+public:
+    static Tensor forward(AutogradContext *ctx, const Tensor &u, const Tensor &w_in, const OptTensor &b_in, const Tensor &A_log,
+                          const Tensor &D, const Tensor &dt_bias, const Tensor &cw, const OptTensor &cb, const Tensor &nw,
+                          const Tensor &w_out, const OptTensor &b_out, c10::intrusive_ptr<LayerOpts> o) {
+        LayerKept k;
+        const Tensor out = layer_forward(u, w_in, undef(b_in), {A_log, D, dt_bias, cw, undef(cb), nw}, w_out, undef(b_out), *o, true, &k);
+        ctx->save_for_backward({u, w_in, A_log, D, dt_bias, cw, undef(cb), nw, w_out, k.zx, k.xbc, k.y, k.yn, k.rstd, k.kept, k.prm32});
+        ctx->saved_data["opts"] = c10::IValue::make_capsule(o);
+        return out;
+    }
+
+    // The gradient of the projection's output is one buffer: the norm writes dz, the operator ddt and the convolution dxBC
+    // into its columns (and the operator dx, dB and dC into the columns of the gradient of the convolution's output), so
+    // nothing is concatenated.
+    static variable_list backward(AutogradContext *ctx, variable_list grads) {
+        const variable_list v = ctx->get_saved_variables();
+        const auto capsule = ctx->saved_data["opts"].toCapsule();
+        const LayerOpts &o = *static_cast<const LayerOpts *>(capsule.get());
+        auto needs = [&](int i) { return (o.needs >> i & 1) != 0; };
+        const Tensor &u = v[0], &w_in = v[1], &w_out = v[8], &zx = v[9], &xbc = v[10], &y = v[11], &yn = v[12], &rstd = v[13];
+        Tensor kept = v[14];
+        const std::array<Tensor, Params32::N> prm = {v[2], v[3], v[4], v[5], v[6], v[7]};
+        const c10::DeviceGuard guard(u.device());
+        void *stream = stream_of(u);
+        const LayerShape s(u, prm[3], o);
+        const Params32 w = point_params(prm, v[15]);
+        const auto f32 = u.options().dtype(at::kFloat);
+        const Tensor dout = as_type(grads[0], u.scalar_type()).reshape({s.rows, w_out.size(0)});
+        Tensor dw_in, db_in, dw_out, db_out, du;
+        if (needs(9)) dw_out = at::mm(dout.t(), yn);
+        if (needs(10)) db_out = dout.sum(0);
+
+        // float32 gradients of the small parameters, one buffer: A, D, dt_bias, conv weight, conv bias, norm weight
+        std::array<int64_t, Params32::N + 1> off{};
+        for (int i = 0; i < Params32::N; ++i) off[i + 1] = off[i] + (prm[i].defined() ? (int64_t)round_up(prm[i].numel(), 64) : 0);
+        const Tensor g32 = at::empty({off.back()}, f32);
+        float *g = g32.mutable_data_ptr<float>();
+
+        const Tensor dyn = at::mm(dout, w_out), dy = at::empty({s.rows, s.inner}, u.options()), dzx = at::empty({s.rows, s.proj}, u.options());
+        {
+            bimamba2_norm_params n = layer_norm_params(s, o, zx, y, w, stream);
+            n.rstd = rstd.mutable_data_ptr<float>();
+            n.dout = dyn.const_data_ptr(); n.dout_rs = s.inner;
+            n.dx = dy.mutable_data_ptr(); n.dx_rs = s.inner;
+            n.dz = at_byte(dzx, 0); n.dz_rs = s.proj;
+            n.dweight = g + off[5];
+            const Tensor ws = at::empty({(int64_t)std::max<size_t>(api.norm_workspace(&n), 1)}, u.options().dtype(at::kByte));
+            n.workspace = ws.mutable_data_ptr();
+            n.workspace_bytes = ws.numel();
+            check(api.norm_bwd(&n), "bimamba2_rmsnorm_gated_bwd");
+        }
+        const Tensor dxbc = at::empty({s.rows, s.conv}, u.options());
+        {
+            bimamba2_params p = layer_scan_params(s, o, zx, xbc, w, stream);
+            Kept(p, o.copies).point(p, kept.mutable_data_ptr<float>());
+            p.fwd_saved = 1;
+            p.dout = dy.const_data_ptr();
+            p.dout_sb = s.seqlen * s.inner; p.dout_sl = s.inner; p.dout_sh = o.headdim;
+            p.dx = at_byte(dxbc, 0);
+            p.dB = at_byte(dxbc, s.inner);
+            p.dC = at_byte(dxbc, s.inner + o.ngroups * o.dstate);
+            p.dx_sb = p.dB_sb = p.dC_sb = s.seqlen * s.conv;
+            p.dx_sl = p.dB_sl = p.dC_sl = s.conv;
+            p.ddt = at_byte(dzx, s.inner + s.conv);
+            p.ddt_sb = s.seqlen * s.proj; p.ddt_sl = s.proj;
+            p.dA = g + off[0]; p.dD = g + off[1]; p.ddt_bias = g + off[2];
+            const Tensor ws = attach_workspace(p, true, u.options());
+            check(api.bwd(&p), "bimamba2_bwd");
+        }
+        {
+            bimamba2_conv_params c = conv_params(s, zx, w, stream);
+            c.dout = dxbc.const_data_ptr();
+            c.dout_sb = s.seqlen * s.conv; c.dout_sl = s.conv;
+            c.dx = at_byte(dzx, s.inner);
+            c.dx_sb = s.seqlen * s.proj; c.dx_sl = s.proj;
+            c.dweight = g + off[3];
+            if (prm[4].defined()) c.dbias = g + off[4];
+            const Tensor ws = at::empty({(int64_t)std::max<size_t>(api.conv_workspace(&c), 1)}, u.options().dtype(at::kByte));
+            c.workspace = ws.mutable_data_ptr();
+            c.workspace_bytes = ws.numel();
+            check(api.conv_bwd(&c), "bimamba2_conv1d_silu_bwd");
+        }
+        // the small gradients into their parameters' types, one launch; dA_log = dA * A
+        std::array<Tensor, Params32::N> dprm;
+        bimamba2_cast_params c{};
+        c.stream = stream;
+        static constexpr int input_of[Params32::N] = {3, 4, 5, 6, 7, 8};
+        for (int i = 0; i < Params32::N; ++i) {
+            if (!prm[i].defined() || !needs(input_of[i])) continue;
+            const Tensor part = g32.narrow(0, off[i], prm[i].numel());
+            if (i && prm[i].scalar_type() == at::kFloat) {
+                dprm[i] = part.view(prm[i].sizes());
+                continue;
+            }
+            dprm[i] = at::empty(prm[i].sizes(), prm[i].options());
+            add_cast(c, part, dprm[i].mutable_data_ptr(), dtype_code(prm[i].scalar_type(), "parameter dtype"),
+                     i == 0 ? BIMAMBA2_CAST_MUL : BIMAMBA2_CAST_COPY, i == 0 ? w.ptr[0] : nullptr);
+        }
+        if (c.count) check(api.cast_many(&c), "bimamba2_cast_many");
+        if (needs(0)) du = at::mm(dzx, w_in).view(u.sizes());
+        if (needs(1)) dw_in = at::mm(dzx.t(), u.reshape({s.rows, u.size(2)}));
+        if (needs(2)) db_in = dzx.sum(0);
+        return {du, dw_in, db_in, dprm[0], dprm[1], dprm[2], dprm[3], dprm[4], dprm[5], dw_out, db_out, Tensor()};
+    }
+};
+
+Tensor layer(const Tensor &u, const Tensor &w_in, const OptTensor &b_in, const Tensor &A_log, const Tensor &D, const Tensor &dt_bias,
+             const Tensor &cw, const OptTensor &cb, const Tensor &nw, const Tensor &w_out, const OptTensor &b_out, int64_t headdim,
+             int64_t ngroups, int64_t dstate, int64_t chunk, double dt_min, double dt_max, double eps, int64_t norm_group, bool norm_before_gate) {
+    auto o = c10::make_intrusive<LayerOpts>();
+    o->inner = w_out.size(1);
+    o->headdim = headdim;
+    o->nheads = o->inner / headdim;
+    o->ngroups = ngroups;
+    o->dstate = dstate;
+    o->chunk = chunk;
+    o->dt_min = dt_min;
+    o->dt_max = dt_max;
+    o->eps = eps;
+    o->norm_group = norm_group;
+    o->norm_before_gate = norm_before_gate;
+    const c10::DeviceGuard guard(u.device());
+    const Tensor bi = undef(b_in), bc = undef(cb), bo = undef(b_out);
+    int i = 0;
+    for (const Tensor *t : {&u, &w_in, &bi, &A_log, &D, &dt_bias, &cw, &bc, &nw, &w_out, &bo}) {
+        if (at::GradMode::is_enabled() && t->defined() && t->requires_grad()) o->needs |= 1u << i;
+        ++i;
+    }
+    if (o->needs)
+        return LayerFn::apply(u, w_in, b_in, A_log, D, dt_bias, cw, cb, nw, w_out, b_out, o);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return layer_forward(u, w_in, bi, {A_log, D, dt_bias, cw, bc, nw}, w_out, bo, *o, false, nullptr);
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+    py::register_exception_translator([](std::exception_ptr e) {
+        try {
+            if (e) std::rethrow_exception(e);
+        } catch (const AssertionFailure &f) {
+            PyErr_SetString(PyExc_AssertionError, f.what());
+        }
+    });
+    m.def("load", &load);
+    m.def("scan", &scan, py::call_guard<py::gil_scoped_release>());
+    m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
+}

@@ -2208,7 +2208,8 @@ __device__ __forceinline__ void chunk_cumsum_bwd_body(const bimamba2_params &p, 
             ex_vb += vb[e];
         }
     }
-    DT *ddt = reinterpret_cast<DT *>(p.ddt);
+    const int64_t ddt_sl = p.ddt_sl ? p.ddt_sl : H, ddt_sb = p.ddt_sl ? p.ddt_sb : (int64_t)p.seqlen * H;
+    DT *ddt = reinterpret_cast<DT *>(p.ddt) + b * ddt_sb + (int64_t)c * Q * ddt_sl + h;
     float sA = 0.f, sb = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -2222,7 +2223,7 @@ __device__ __forceinline__ void chunk_cumsum_bwd_body(const bimamba2_params &p, 
             float g = da[e] * A + ddr[e];
             if (clamped) g = 0.f;
             if (p.dt_softplus && pre <= 20.f) g *= 1.f / (1.f + expf(-pre));
-            ddt[((int64_t)b * p.seqlen + (int64_t)c * Q + q) * H + h] = from_f<DT>(g);
+            ddt[q * ddt_sl] = from_f<DT>(g);
             sA += da[e] * d;
             sb += g;
         }

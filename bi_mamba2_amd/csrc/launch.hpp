@@ -20,6 +20,7 @@ __host__ __device__ inline int ddt_direct_planes(const bimamba2_params &p) {
 }
 
 int launch_chunk_cumsum_fwd(const bimamba2_params *p);
+int launch_seq_boundaries(const bimamba2_params *p, int32_t *counts);
 int launch_bmm_chunk_fwd(const bimamba2_params *p);
 int launch_chunk_state(const bimamba2_params *p, bool dstates, bool cumsum = false);   // cumsum: also does the chunk cumsum
 bool chunk_state_does_cumsum(const bimamba2_params *p);

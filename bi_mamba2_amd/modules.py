@@ -4,7 +4,7 @@ Same constructor keywords, parameter names/shapes (so state_dicts interchange) a
 reference layer (src/ssd/modules.py:17-187): in_proj -> split [z | xBC | dt] -> softplus(dt + dt_bias) ->
 non-causal depthwise conv1d + SiLU -> split x, B, C -> bidirectional SSD with D -> gated RMSNorm(y, z) ->
 out_proj.  Parameters are created in the reference's order, so a seeded construction draws the same values.
-The projections and the convolution are ordinary torch ops; the SSD and the gated RMS norm are the HIP operators.
+The projections are torch GEMMs; the convolution, the SSD and the gated RMS norm are the HIP operators.
 """
 import ctypes
 import math
@@ -16,7 +16,7 @@ import torch.nn.functional as F
 from . import _lib
 from .conv1d import conv1d_silu_fn
 from .layernorm_gated import RMSNorm, rmsnorm_fn
-from .ops import _DT, bimamba_chunk_scan_combined
+from .ops import _DT, MAX_CHUNK_SIZE, MAX_DSTATE, MAX_HEADDIM, bimamba_chunk_scan_combined
 
 
 # the gated RMS norm of the layer runs on the HIP kernels (bi_mamba2_amd/layernorm_gated.py)
@@ -133,7 +133,8 @@ class _SplitInto(torch.autograd.Function):
             dst = pieces.piece(i)
             if g is None:
                 dst.zero_()
-            elif not (g.data_ptr() == dst.data_ptr() and g.shape == dst.shape and g.stride() == dst.stride() and g.dtype == dst.dtype):
+            elif not (g.data_ptr() == dst.data_ptr() and g.shape == dst.shape and g.dtype == dst.dtype
+                      and all(a == b for a, b, n in zip(g.stride(), dst.stride(), g.shape) if n > 1)):
                 dst.copy_(g)
                 copied.append(i)
         if _GradPieces.on_copied is not None:
@@ -191,7 +192,35 @@ class BiMamba2(nn.Module):
         self.norm = RMSNormGated(self.d_inner, eps=1e-5, norm_before_gate=True, **fk)
         self.out_proj = nn.Linear(self.d_inner, d_model, bias=bias, **fk)
 
+    def _takes_native_path(self, u):
+        """Whether forward() may run as ONE native autograd function (csrc/host.cpp: the two GEMMs and this library's kernels,
+        no Python between them): what the kernels take in one piece, and nobody who expects the projections to be called as
+        modules, or the gradients' pieces as separate tensors (_GradPieces.on_copied) - hooks, replaced or patched
+        projections, autocast."""
+        if not (u.is_cuda and u.dim() == 3 and u.dtype in _DT and self.headdim <= MAX_HEADDIM and self.d_state <= MAX_DSTATE
+                and self.chunk_size >= 32) or _GradPieces.on_copied is not None or torch.is_autocast_enabled("cuda"):
+            return False
+        m = torch.nn.modules.module
+        if m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks:
+            return False
+        for lin in (self.in_proj, self.out_proj):
+            if (type(lin) is not nn.Linear or lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks
+                    or lin._backward_pre_hooks or "forward" in lin.__dict__ or lin.weight.dtype != u.dtype):
+                return False
+        if self.norm.bias is not None or self.conv1d.weight.dim() != 3:
+            return False
+        return all(type(t) in (nn.Parameter, torch.Tensor) and t.dtype in _DT for t in self._native_tensors() if t is not None)
+
+    def _native_tensors(self):
+        return (self.in_proj.weight, self.in_proj.bias, self.A_log, self.D, self.dt_bias, self.conv1d.weight, self.conv1d.bias,
+                self.norm.weight, self.out_proj.weight, self.out_proj.bias)
+
     def forward(self, u):
+        if self._takes_native_path(u):
+            norm = self.norm
+            return _lib.host().layer(u, *self._native_tensors(), self.headdim, self.ngroups, self.d_state, min(self.chunk_size, MAX_CHUNK_SIZE),
+                                     self.dt_limit[0], self.dt_limit[1], norm.eps, norm.group_size or self.d_inner,
+                                     norm.norm_before_gate)
         bc = self.ngroups * self.d_state
         zxbcdt = self.in_proj(u)
         prm = (self.A_log, self.D, self.dt_bias, self.conv1d.weight, self.conv1d.bias, self.norm.weight)

@@ -56,6 +56,7 @@ enum {
  * boundaries: a caller whose sequences can be shorter than chunk_size / 32 positions on average picks a smaller chunk_size
  * (the result does not depend on it); the Python host does so for at most 32 boundaries per chunk. */
 #define BIMAMBA2_SEQ_CUT (-20.0f)
+#define BIMAMBA2_MAX_SEQ_BOUNDARIES 32  /* boundaries per chunk that the hosts of this library allow */
 
 typedef struct bimamba2_params {
     /* problem */
@@ -157,6 +158,7 @@ typedef struct bimamba2_params {
        slices of the convolution's output in the BiMamba2 layer: no concatenation of the gradients afterwards.  Multiples of
        8 elements (16 bytes) where the vector kernels are to run. */
     int64_t dx_sb, dx_sl, dB_sb, dB_sl, dC_sb, dC_sl;
+    int64_t ddt_sb, ddt_sl;         /* likewise of ddt (batch, seqlen, nheads): 0 means contiguous */
 } bimamba2_params;
 
 /* text of an error code */
@@ -168,6 +170,13 @@ size_t bimamba2_params_size(void);
 
 /* bytes of workspace the composite entry points need (is_bwd = 0: forward, 1: backward) */
 size_t bimamba2_workspace_bytes(const bimamba2_params *p, int is_bwd);
+
+/* Packed sequences: counts[b * nchunks + c] = the larger of the numbers of sequence boundaries that the forward and the reverse
+ * cumulative sums of chunk c of row b see at this chunk_size (a change of seq_idx between positions l - 1 and l belongs to the
+ * chunk of l in the forward sums and to the chunk of l - 1 in the reverse ones).  `counts` may be pinned host memory.  Needs
+ * seq_idx.  A caller that finds more than BIMAMBA2_SEQ_CUT's resolution allows (see there) takes a smaller chunk_size.  No
+ * counterpart in the reference. */
+int bimamba2_seq_boundaries(const bimamba2_params *p, int32_t *counts);
 
 /* 1 if the kernels of this problem can keep the entering states in 16-bit copies (see states16_f), else 0 */
 int bimamba2_state_copies(const bimamba2_params *p);

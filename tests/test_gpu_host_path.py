@@ -1,0 +1,89 @@
+"""GPU tests of the native host path (csrc/host.cpp): the layer as one autograd function against the same layer composed of
+its pieces, with frozen parameters and projection biases; the count of packed sequences' boundaries that decides the chunk
+size, and gradients that arrive as views the kernels cannot read in place."""
+import pytest
+import torch
+
+from tests.helpers import assert_close, make_case, to_dev
+
+pytestmark = pytest.mark.gpu
+
+LAYERS = [
+    # batch, seqlen, kwargs, dtype, bias of the projections, frozen parameters
+    (2, 70, dict(d_model=64, d_state=16, headdim=16, chunk_size=64), torch.float32, True, ()),
+    (1, 1, dict(d_model=64, d_state=16, headdim=32, ngroups=2), torch.float32, False, ("A_log", "conv1d.weight")),
+    (2, 300, dict(d_model=128, d_state=64, headdim=64), torch.bfloat16, True, ("in_proj.weight", "norm.weight", "D")),
+    (1, 257, dict(d_model=128, d_state=128, headdim=64, conv_bias=False), torch.float16, False, ("out_proj.weight",)),
+]
+
+
+@pytest.mark.parametrize("case", LAYERS)
+def test_layer_equals_its_composition(case, monkeypatch):
+    from bi_mamba2_amd.modules import BiMamba2, _GradPieces
+    batch, seqlen, kw, dtype, bias, frozen = case
+    torch.manual_seed(0)
+    m = BiMamba2(bias=bias, **kw).cuda().to(dtype)
+    for name, p in m.named_parameters():
+        p.requires_grad_(name not in frozen)
+    u = torch.randn(batch, seqlen, kw["d_model"], device="cuda").to(dtype).requires_grad_(True)
+    dy = torch.randn_like(u)
+    live = {"u": u, **{n: p for n, p in m.named_parameters() if p.requires_grad and n != "fc_D.weight"}}
+
+    def step():
+        out = m(u)
+        with torch.no_grad():
+            assert_close(m(u), out.detach().double(), dtype, "output without autograd", scaled=True)
+        return (out.detach(),) + torch.autograd.grad(out, list(live.values()), dy)
+
+    assert m._takes_native_path(u)
+    native = step()
+    monkeypatch.setattr(_GradPieces, "on_copied", staticmethod(lambda copied: None))      # (its observer gets the composition)
+    assert not m._takes_native_path(u)
+    for name, a, b in zip(["out"] + list(live), native, step()):
+        assert a.shape == b.shape and a.dtype == b.dtype, name
+        assert_close(a, b.double(), dtype, name, scaled=True)
+
+
+def test_layer_with_hooks_or_autocast_is_composed():
+    from bi_mamba2_amd.modules import BiMamba2
+    m = BiMamba2(d_model=64, d_state=16, headdim=16, chunk_size=64).cuda()
+    u = torch.randn(1, 40, 64, device="cuda")
+    seen = []
+    handle = m.in_proj.register_forward_hook(lambda mod, args, out: seen.append(out.shape))
+    with torch.no_grad():
+        hooked = m(u)
+        handle.remove()
+        assert len(seen) == 1 and torch.allclose(hooked, m(u), rtol=1e-4, atol=1e-5)
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            assert m(u).dtype == torch.bfloat16
+
+
+@pytest.mark.parametrize("chunk", [32, 48, 256])
+def test_boundary_count(chunk):
+    from bi_mamba2_amd import _lib, ops
+    g = torch.Generator().manual_seed(1)
+    seq = (torch.rand(3, 521, generator=g) < 0.3).cumsum(1).to(torch.int32)
+    seq[1] = 0
+    seq[2, 256:] += 1
+    p = _lib.Params()
+    for k, v in dict(batch=3, seqlen=521, nheads=1, headdim=1, ngroups=1, dstate=1, chunk_size=chunk).items():
+        setattr(p, k, v)
+    dev, counts = seq.cuda(), torch.empty(3 * -(-521 // chunk), dtype=torch.int32, pin_memory=True)
+    p.seq_idx, p.stream = dev.data_ptr(), torch.cuda.current_stream().cuda_stream
+    assert _lib.load().bimamba2_seq_boundaries(p, counts.data_ptr()) == 0
+    torch.cuda.synchronize()
+    want = [ops.seq_boundaries_per_chunk(seq[b:b + 1], chunk) for b in range(3)]
+    assert counts.view(3, -1).amax(1).tolist() == want
+
+
+def test_gradient_views_that_break_the_alignment_are_copied():
+    from bi_mamba2_amd import ops
+    d = to_dev(make_case(1, 300, 2, 64, 1, 64, torch.bfloat16, with_z=False))
+    leaves = [d[k].clone().requires_grad_(True) for k in ("x", "dt", "A", "B", "C")]
+    out = ops.bimamba_chunk_scan_combined(*leaves, 256, D=d["D"], dt_bias=d["dt_bias"], dt_softplus=True)
+    wide = torch.randn(1, 300, 131, device="cuda", dtype=torch.bfloat16)
+    odd = wide[..., 3:].unflatten(-1, (2, 64))
+    for view in (odd, odd.transpose(2, 3).contiguous().transpose(2, 3)):
+        got = torch.autograd.grad(out, leaves, view, retain_graph=True)
+        for a, b in zip(got, torch.autograd.grad(out, leaves, view.contiguous(), retain_graph=True)):
+            assert torch.equal(a, b)
