@@ -193,13 +193,18 @@ template <bool RAW = true, typename V> __device__ __forceinline__ void raw_lds_u
 // A operand: lane l holds KPL consecutive k of row l%16 starting at KPL*(l/16); B operand likewise for
 // column l%16.  Both operands use the same k mapping, so any consistent mapping gives the same product.
 template <typename T> struct Mma;
+// float32: the matrix instruction takes one k per lane (four per instruction).  Which k that is does not matter as long as both
+// operands agree, so a lane owns four consecutive ones and a fragment feeds four instructions: operands arrive as 16-byte
+// accesses (one element per access before: the float32 kernels spent their time on four times the loads).
 template <> struct Mma<float> {
-    static constexpr int KPL = 1, KSTEP = 4, LD = BK + 4;
-    typedef float Frag;
-    static __device__ __forceinline__ Frag load(const float *p) { return *p; }
-    static __device__ __forceinline__ Frag pack(const float *a) { return a[0]; }
+    static constexpr int KPL = 4, KSTEP = 16, LD = BK + 4;
+    typedef f32x4 Frag;
+    static __device__ __forceinline__ Frag load(const float *p) { return *reinterpret_cast<const f32x4 *>(p); }
+    static __device__ __forceinline__ Frag pack(const float *a) { return f32x4{a[0], a[1], a[2], a[3]}; }
     static __device__ __forceinline__ f32x4 mma(Frag a, Frag b, f32x4 c) {
-        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i], b[i], c, 0, 0, 0);
+        return c;
     }
 };
 template <> struct Mma<bf16_t> {
@@ -267,10 +272,18 @@ template <typename T, typename S, int ROWS, int KW = BK, class F>
 __device__ __forceinline__ void tile_load_kcontig(T *dst, const S *src, int64_t rs, int rvalid, int kvalid, F f) {
     constexpr int VS = 16 / sizeof(S), KV = KW / VS, LD = Mma<T>::LD - BK + KW;
     const bool vec = aligned16(src, rs);
+    // whole vectors only: the loads are unconditional, from clamped addresses (a conditional load is waited for on the spot),
+    // and what lies outside is replaced by 0 afterwards
+    const bool whole = vec && kvalid % VS == 0 && kvalid > 0 && rvalid > 0;
     for (int idx = threadIdx.x; idx < ROWS * KV; idx += blockDim.x) {
         const int r = idx / KV, k0 = (idx % KV) * VS;
         float v[VS];
-        if (vec && r < rvalid && k0 + VS <= kvalid) {
+        if (whole) {
+            const Vec16<S> raw = *reinterpret_cast<const Vec16<S> *>(src + min(r, rvalid - 1) * rs + min(k0, kvalid - VS));
+            const bool in = r < rvalid && k0 < kvalid;
+#pragma unroll
+            for (int i = 0; i < VS; ++i) v[i] = in ? to_f(raw.v[i]) : 0.f;
+        } else if (vec && r < rvalid && k0 + VS <= kvalid) {
             Vec16<S> raw = *reinterpret_cast<const Vec16<S> *>(src + r * rs + k0);
 #pragma unroll
             for (int i = 0; i < VS; ++i) v[i] = to_f(raw.v[i]);
@@ -282,52 +295,6 @@ __device__ __forceinline__ void tile_load_kcontig(T *dst, const S *src, int64_t 
 #pragma unroll
         for (int i = 0; i < VS; ++i) o.v[i] = from_f<T>(f(r, k0 + i, v[i]));
         *reinterpret_cast<Out *>(dst + r * LD + k0) = o;
-    }
-}
-
-// dst[r][k] = f(r, k, src[k*ks + r]): the source is contiguous along r (transposing load).
-template <typename T, typename S, int ROWS, class F>
-__device__ __forceinline__ void tile_load_rcontig(T *dst, const S *src, int64_t ks, int rvalid, int kvalid, F f) {
-    constexpr int VS = 16 / sizeof(S), RV = ROWS / VS, LD = Mma<T>::LD;
-    const bool vec = aligned16(src, ks);
-    for (int idx = threadIdx.x; idx < BK * RV; idx += blockDim.x) {
-        const int k = idx / RV, r0 = (idx % RV) * VS;
-        float v[VS];
-        if (vec && k < kvalid && r0 + VS <= rvalid) {
-            Vec16<S> raw = *reinterpret_cast<const Vec16<S> *>(src + k * ks + r0);
-#pragma unroll
-            for (int i = 0; i < VS; ++i) v[i] = to_f(raw.v[i]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < VS; ++i) v[i] = (k < kvalid && r0 + i < rvalid) ? to_f(src[k * ks + r0 + i]) : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < VS; ++i) dst[(r0 + i) * LD + k] = from_f<T>(f(r0 + i, k, v[i]));
-    }
-}
-
-// same, writing two tiles with two functors from one read of the source
-template <typename T, typename S, int ROWS, class F1, class F2>
-__device__ __forceinline__ void tile_load_rcontig2(T *dst1, T *dst2, const S *src, int64_t ks, int rvalid,
-                                                   int kvalid, F1 f1, F2 f2) {
-    constexpr int VS = 16 / sizeof(S), RV = ROWS / VS, LD = Mma<T>::LD;
-    const bool vec = aligned16(src, ks);
-    for (int idx = threadIdx.x; idx < BK * RV; idx += blockDim.x) {
-        const int k = idx / RV, r0 = (idx % RV) * VS;
-        float v[VS];
-        if (vec && k < kvalid && r0 + VS <= rvalid) {
-            Vec16<S> raw = *reinterpret_cast<const Vec16<S> *>(src + k * ks + r0);
-#pragma unroll
-            for (int i = 0; i < VS; ++i) v[i] = to_f(raw.v[i]);
-        } else {
-#pragma unroll
-            for (int i = 0; i < VS; ++i) v[i] = (k < kvalid && r0 + i < rvalid) ? to_f(src[k * ks + r0 + i]) : 0.f;
-        }
-#pragma unroll
-        for (int i = 0; i < VS; ++i) {
-            dst1[(r0 + i) * LD + k] = from_f<T>(f1(r0 + i, k, v[i]));
-            dst2[(r0 + i) * LD + k] = from_f<T>(f2(r0 + i, k, v[i]));
-        }
     }
 }
 
@@ -353,9 +320,24 @@ template <typename T, int KTOT, int RTOT, int LDX, bool FAST, typename S, class 
 __device__ __forceinline__ void stage_transposed(T *dst, const S *src, int64_t ks, int kvalid, int rvalid, F scale) {
     constexpr int VK = 16 / sizeof(T), VR = 16 / sizeof(S), RB = RTOT / VR, NB = (KTOT / VK) * RB;
     const bool vec = FAST || aligned16(src, ks);
+    const bool whole = !FAST && vec && rvalid % VR == 0;      // whole vectors: unconditional loads (see tile_load_kcontig)
     for (int blk = threadIdx.x; blk < NB; blk += blockDim.x) {
         const int rb = blk % RB, kb = blk / RB;
         float v[VK][VR];
+        if (whole) {
+            Vec16<S> raw[VK];
+#pragma unroll
+            for (int kk = 0; kk < VK; ++kk)
+                raw[kk] = *reinterpret_cast<const Vec16<S> *>(src + (int64_t)min(kb * VK + kk, kvalid - 1) * ks + min(rb * VR, rvalid - VR));
+#pragma unroll
+            for (int kk = 0; kk < VK; ++kk) {
+                const int k = kb * VK + kk;
+                const bool in = k < kvalid && rb * VR < rvalid;
+                const float sc = scale(k);
+#pragma unroll
+                for (int i = 0; i < VR; ++i) v[kk][i] = in ? to_f(raw[kk].v[i]) * sc : 0.f;
+            }
+        } else
 #pragma unroll
         for (int kk = 0; kk < VK; ++kk) {
             const int k = kb * VK + kk;
@@ -388,9 +370,25 @@ __device__ __forceinline__ void stage_transposed2(T *dst1, T *dst2, const S *src
                                                   F1 scale1, F2 scale2) {
     constexpr int VK = 16 / sizeof(T), VR = 16 / sizeof(S), RB = RTOT / VR, NB = (KTOT / VK) * RB;
     const bool vec = FAST || aligned16(src, ks);
+    const bool whole = !FAST && vec && rvalid % VR == 0;
     for (int blk = threadIdx.x; blk < NB; blk += blockDim.x) {
         const int rb = blk % RB, kb = blk / RB;
         float v[VK][VR], s1[VK], s2[VK];
+        if (whole) {
+            Vec16<S> raw[VK];
+#pragma unroll
+            for (int kk = 0; kk < VK; ++kk)
+                raw[kk] = *reinterpret_cast<const Vec16<S> *>(src + (int64_t)min(kb * VK + kk, kvalid - 1) * ks + min(rb * VR, rvalid - VR));
+#pragma unroll
+            for (int kk = 0; kk < VK; ++kk) {
+                const int k = kb * VK + kk;
+                const bool in = k < kvalid && rb * VR < rvalid;
+#pragma unroll
+                for (int i = 0; i < VR; ++i) v[kk][i] = in ? to_f(raw[kk].v[i]) : 0.f;
+                s1[kk] = scale1(k);
+                s2[kk] = scale2(k);
+            }
+        } else
 #pragma unroll
         for (int kk = 0; kk < VK; ++kk) {
             const int k = kb * VK + kk;

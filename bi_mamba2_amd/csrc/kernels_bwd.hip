@@ -373,8 +373,32 @@ int launch_state_passing_bwd(const bimamba2_params *p) {
 //   tmp_f = x_h[r,:] . dS_f[h],  dBs[r,n] += dt[r] (e^{cs_f[Q-1]-cs_f[r]} tmp_f + e^{cs_b[0]-cs_b[r]} tmp_b)
 //   v_f[h,r] = dt[r] e^{cs_f[Q-1]-cs_f[r]} sum_n tmp_f[r,n] B[r,n]
 // =========================================================================================================
-constexpr int DBDC_HEADS = 8;         // heads per slice (measured against 4 with 256-row tiles: dB / dC / tail 0.323 -> 0.316 ms per step)
-static inline int dbdc_slices(const bimamba2_params *p) { return (p->nheads / p->ngroups + DBDC_HEADS - 1) / DBDC_HEADS; }
+constexpr int DBDC_HEADS = 8;         // heads per slice at most (measured against 4 with 256-row tiles: dB / dC / tail 0.323 -> 0.316 ms per step)
+constexpr int DBDC_SLICES_MAX = 8;    // what bmm_chunk_bwd adds up in its fast variant
+static inline int dbdc_heads(const bimamba2_params *p) { return p->dbdc_heads > 0 ? p->dbdc_heads : DBDC_HEADS; }
+static inline int dbdc_slices(const bimamba2_params *p) { return (p->nheads / p->ngroups + dbdc_heads(p) - 1) / dbdc_heads(p); }
+
+// Heads per slice where the caller leaves the choice (the partial sums are bimamba2_bwd's own).  A workgroup of the dB / dC
+// kernels fills a CU, needs about three head steps to start (measured: 17 us for 8 heads, of which 5 before the first) and
+// then one per head; each slice more is a partial sum of each of dB and dC that is written and read again.  With eight heads
+// a slice, small problems leave most of the chip idle: 24 workgroups at batch 2 x 1500 with 8 heads of 128 channels, where the
+// two kernels took 22 us each and take 12 with one head a slice.
+int choose_dbdc_heads(const bimamba2_params *p) {
+    const int hpg = p->nheads / p->ngroups, nc = nchunks(p);
+    const int64_t tiles = (int64_t)p->batch * nc * p->ngroups * ((p->chunk_size + 127) / 128);
+    const double steps = ((p->headdim + 63) / 64) * ((p->dstate + 63) / 64);                             // per head
+    const double slice_cost = (double)p->batch * p->seqlen * p->ngroups * p->dstate * 8 / 5e6 / 1.5;     // one partial sum at 5 TB/s, in steps of 1.5 us
+    int best = DBDC_HEADS;
+    double best_cost = 0;
+    for (int k = DBDC_HEADS; k >= 1; --k) {
+        const int slices = (hpg + k - 1) / k;
+        if (k < DBDC_HEADS && (slices > DBDC_SLICES_MAX || (hpg + slices - 1) / slices != k)) continue;  // (the fewest heads for this many slices)
+        const double rounds = (double)((tiles * slices + 255) / 256);
+        const double cost = rounds * (3 + steps * std::min(k, hpg)) + slices * slice_cost;
+        if (k == DBDC_HEADS || cost < best_cost) { best = k; best_cost = cost; }
+    }
+    return best;
+}
 
 // The A operand (x or dout rows, K = headdim contiguous) is read from global memory straight into MFMA operand
 // registers; the states, stored [p][n], are staged transposed ([n][p], 64 x 64 at a time) in LDS, double-buffered for
@@ -387,7 +411,7 @@ constexpr int DBDC_WAVES = 8, DBDC_THREADS = 64 * DBDC_WAVES;
 // only then written to the LDS image.
 // UNI: the forward direction's state only (single-direction comparator).
 template <typename T, int NT, int QT, bool IS_DB, bool FAST, bool UNI = false>
-__global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_params p, int nc) {
+__global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_params p, int nc, int hps) {
     typedef Mma<T> M;
     constexpr int KPL = M::KPL, KSTEP = M::KSTEP, KC = 64, NKS = KC / KSTEP;
     constexpr int VK = 16 / (int)sizeof(T);                                // image rows (k) per staged block; 4 columns (n)
@@ -408,9 +432,9 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_p
     const int Q = p.chunk_size, N = p.dstate, P = p.headdim, H = p.nheads, hpg = H / p.ngroups;
     const int limit = min(Q, p.seqlen - c * Q);
     const int r0 = rt * ROWS;
-    // blockIdx.z selects a slice of DBDC_HEADS heads of the group; its partial sum goes to slice blockIdx.z of the
-    // output, and bmm_chunk_bwd adds the slices up
-    const int hh0 = blockIdx.z * DBDC_HEADS, hh_end = min(hpg, hh0 + DBDC_HEADS);
+    // blockIdx.z selects a slice of hps (at most DBDC_HEADS) heads of the group; its partial sum goes to slice blockIdx.z of
+    // the output, and bmm_chunk_bwd adds the slices up
+    const int hh0 = blockIdx.z * hps, hh_end = min(hpg, hh0 + hps);
     const int nkc = (P + KC - 1) / KC, nnt = (N + 63) / 64;
     const int per_head = nnt * nkc, nsteps = (hh_end - hh0) * per_head;
 
@@ -422,8 +446,16 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_p
     for (int q = 0; q < QT; ++q) arow[q] = min(r0 + (wave * QT + q) * 16 + lr, limit - 1);
     const int sblk = threadIdx.x % NBLK, stile = threadIdx.x / NBLK;       // stile 0: forward state, 1: reverse state
     const int s_rb = sblk % 16, s_kb = sblk / 16;
+    // without FAST: whole vectors of the states (columns) and of the x / dout rows, or element by element
+    const bool whole_s = !FAST && N % 4 == 0 && aligned16(IS_DB ? p.dstates_f : p.states_f, 0) && aligned16(IS_DB ? p.dstates_b : p.states_b, 0);
+    const bool whole_a = !FAST && P % KPL == 0 &&
+                         (IS_DB ? aligned16(reinterpret_cast<const T *>(p.x), p.x_sb | p.x_sl | p.x_sh)
+                                : p.has_z ? aligned16(reinterpret_cast<const T *>(p.dout_x), P) : aligned16(reinterpret_cast<const T *>(p.dout), p.dout_sb | p.dout_sl | p.dout_sh));
+    int s_kc = 0, s_nt = 0;                                                // the step whose state block sreg holds
     auto request = [&](int step) __attribute__((always_inline)) {
         const int hh = hh0 + step / per_head, rem = step % per_head, nt = rem / nkc, kc = rem % nkc;
+        s_kc = kc;
+        s_nt = nt;
         const int h = g * hpg + hh;
         if (stile < (UNI ? 1 : 2)) {
             const int64_t so = ((int64_t)(b * nc + c) * H + h) * P * N;
@@ -432,7 +464,9 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_p
             for (int kk = 0; kk < VK; ++kk) {
                 const int pp = kc * KC + s_kb * VK + kk, n = nt * 64 + s_rb * 4;
                 if (FAST) sreg[kk] = *reinterpret_cast<const Vec16<float> *>(st + (int64_t)pp * N + n);
-                else
+                else if (whole_s) {                        // unconditional, from clamped addresses; zeroed in commit()
+                    sreg[kk] = *reinterpret_cast<const Vec16<float> *>(st + (int64_t)min(pp, P - 1) * N + min(n, N - 4));
+                } else
 #pragma unroll
                     for (int i = 0; i < 4; ++i) sreg[kk].v[i] = (pp < P && n + i < N) ? st[(int64_t)pp * N + n + i] : 0.f;
             }
@@ -449,7 +483,10 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_p
                 const int kb = kc * KC + ks * KSTEP + lg * KPL;
                 const T *row = ap + (int64_t)arow[q] * as;
                 if (FAST) af[q][ks] = M::load(row + kb);
-                else {
+                else if (whole_a) {
+                    af[q][ks] = M::load(row + min(kb, P - KPL));
+                    if (kb >= P) af[q][ks] = typename M::Frag{};
+                } else {
                     float v[KPL];
 #pragma unroll
                     for (int i = 0; i < KPL; ++i) v[i] = kb + i < P ? to_f(row[kb + i]) : 0.f;
@@ -465,7 +502,10 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_p
             for (int rr = 0; rr < 4; ++rr) {
                 Vec16<T> o;
 #pragma unroll
-                for (int kk = 0; kk < VK; ++kk) o.v[kk] = from_f<T>(sreg[kk].v[rr]);
+                for (int kk = 0; kk < VK; ++kk) {
+                    const bool in = FAST || (s_kc * KC + s_kb * VK + kk < P && s_nt * 64 + s_rb * 4 + rr < N);
+                    o.v[kk] = from_f<T>(in ? sreg[kk].v[rr] : 0.f);
+                }
                 *reinterpret_cast<Vec16<T> *>(dst + xt_index<T, LDX>(s_rb * 4 + rr, s_kb * VK)) = o;
             }
         }
@@ -542,9 +582,11 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_p
                 if (step + 1 < nsteps) request(step + 1);  // in flight while this step is multiplied
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) {
+                    if (!FAST && kc * KC + ks * KSTEP >= P) continue;      // (uniform) nothing there: narrow heads and states
                     const int kq = ks * KSTEP + lg * KPL;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
+                        if (!FAST && nt * 64 + j * 16 >= N) continue;
                         const typename M::Frag bff = M::load(sF[buf] + xt_index<T, LDX>(j * 16 + lr, kq));
                         const typename M::Frag bfb = UNI ? bff : M::load(sB[buf] + xt_index<T, LDX>(j * 16 + lr, kq));
 #pragma unroll
@@ -596,7 +638,7 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_p
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// The same for 16-bit types with dstate 64 and headdim % 64 == 0, with every load of the head loop taken out of the
+// The same for 16-bit types with dstate 64 or 128 and headdim % 64 == 0, with every load of the head loop taken out of the
 // compiler's hands.  The workgroup is alone on its CU (register-bound), so nothing hides a load it waits for; here the
 // float32 state tiles of a step travel straight into a 3-slot LDS ring (no registers), two steps ahead of their use, and
 // the x / dout fragments into registers, likewise two steps ahead, from inline assembly.  A step then reads its tiles
@@ -608,8 +650,9 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_p
 // S16: the state tiles come from their 16-bit copies (states16_* / dstates16_*).  They lie in the ring as they lie in
 // memory ([p][n], 16-byte chunks swizzled as tile64_request does), and the operand fragments are LDS transpose reads
 // straight from the ring slot: no operand image, one barrier per step, a third of the LDS.
-template <typename T, int QT, bool IS_DB, bool UNI, bool S16>
-__global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamba2_params p, int nc) {
+// NT: 64-column tiles of the state dimension (1 or 2).  A step multiplies one of them: step = (head, n tile, headdim chunk).
+template <typename T, int QT, bool IS_DB, bool UNI, bool S16, int NT = 1>
+__global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamba2_params p, int nc, int hps) {
     typedef Mma<T> M;
     typedef typename M::Frag Frag;
     static_assert(sizeof(T) == 2, "16-bit operands");
@@ -621,6 +664,7 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamb
     constexpr int IMG_B = 64 * LDX * 2;                        // bytes of a 16-bit operand image
     constexpr int PER_STEP = NDIR * (S16 ? 1 : 2) + QT * NKS;  // vector memory operations of a wave per step
     static_assert(NDIR * NBLK <= DBDC_THREADS, "one block per thread");
+    static_assert(NT == 1 || NT == 2, "state dimension 64 or 128");
     static_assert(DBDC_WAVES == 8, "a wave brings 8 (16-bit) resp. 2 x 4 (float32) rows of each tile");
     __shared__ __attribute__((aligned(16))) unsigned char ring[RING * NDIR * TILE_B];
     __shared__ __attribute__((aligned(16))) unsigned char img[S16 ? 16 : 2 * NDIR * IMG_B];
@@ -635,35 +679,35 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamb
     const int Q = p.chunk_size, N = p.dstate, P = p.headdim, H = p.nheads, hpg = H / p.ngroups;
     const int limit = min(Q, p.seqlen - c * Q);
     const int r0 = rt * ROWS;
-    const int hh0 = blockIdx.z * DBDC_HEADS, hh_end = min(hpg, hh0 + DBDC_HEADS);
-    const int nkc = P / KC, nsteps = (hh_end - hh0) * nkc;
+    const int hh0 = blockIdx.z * hps, hh_end = min(hpg, hh0 + hps);
+    const int nkc = P / KC, per_head = nkc * NT, nsteps = (hh_end - hh0) * per_head;
     int arow[QT];
 #pragma unroll
     for (int q = 0; q < QT; ++q) arow[q] = min(r0 + (wave * QT + q) * 16 + lr, limit - 1);
 
     // requests of a step: this wave's two 4-row units of each state tile, then its fragments
     auto issue_states = [&](int step) {
-        const int hh = hh0 + step / nkc, kc = step % nkc, h = g * hpg + hh;
-        const int64_t so = ((int64_t)(b * nc + c) * H + h) * P * N + (int64_t)kc * KC * N;
+        const int hh = hh0 + step / per_head, kc = step % nkc, nt = NT == 1 ? 0 : (step / nkc) % NT, h = g * hpg + hh;
+        const int64_t so = ((int64_t)(b * nc + c) * H + h) * P * N + (int64_t)kc * KC * N + nt * 64;
 #pragma unroll
         for (int d = 0; d < NDIR; ++d) {
             if constexpr (S16) {
                 // rows 8 wave .. 8 wave + 7, 16-byte chunk (lane % 8) ^ swizzle(row) at chunk position lane % 8
                 const T *st = reinterpret_cast<const T *>(IS_DB ? (d ? p.dstates16_b : p.dstates16_f) : (d ? p.states16_b : p.states16_f)) + so;
                 const int row = wave * 8 + (lane >> 3);
-                load16_to_lds(st + row * 64 + (((lane & 7) ^ tile64_swz(row)) << 3), ring + ((step % RING) * NDIR + d) * TILE_B + wave * 1024);
+                load16_to_lds(st + row * (64 * NT) + (((lane & 7) ^ tile64_swz(row)) << 3), ring + ((step % RING) * NDIR + d) * TILE_B + wave * 1024);
             } else {
                 const float *st = (IS_DB ? (d ? p.dstates_b : p.dstates_f) : (d ? p.states_b : p.states_f)) + so;
 #pragma unroll
                 for (int uu = 0; uu < 2; ++uu) {
                     const int u = wave * 2 + uu;
-                    load16_to_lds(st + (4 * u + (lane >> 4)) * 64 + (lane & 15) * 4, ring + ((step % RING) * NDIR + d) * TILE_B + u * 1024);
+                    load16_to_lds(st + (4 * u + (lane >> 4)) * (64 * NT) + (lane & 15) * 4, ring + ((step % RING) * NDIR + d) * TILE_B + u * 1024);
                 }
             }
         }
     };
     auto issue_frags = [&](int step, Frag (&af)[QT][NKS]) {
-        const int hh = hh0 + step / nkc, kc = step % nkc, h = g * hpg + hh;
+        const int hh = hh0 + step / per_head, kc = step % nkc, h = g * hpg + hh;
         const T *ap;
         int64_t as;
         if (IS_DB) { as = p.x_sl; ap = reinterpret_cast<const T *>(p.x) + b * p.x_sb + (int64_t)c * Q * as + h * p.x_sh; }
@@ -705,20 +749,24 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamb
     int64_t cbs;
     if (IS_DB) { cbs = p.B_sl; cbp = reinterpret_cast<const T *>(p.Bm) + b * p.B_sb + ((int64_t)c * Q + r0) * cbs + g * p.B_sg; }
     else { cbs = p.C_sl; cbp = reinterpret_cast<const T *>(p.Cm) + b * p.C_sb + ((int64_t)c * Q + r0) * cbs + g * p.C_sg; }
-    float creg[QT][4][4];
+    float creg[NT][QT][4][4];
 #pragma unroll
-    for (int q = 0; q < QT; ++q)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int q = 0; q < QT; ++q)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) creg[q][j][i] = to_f(cbp[(int64_t)min(tl[q][i], limit - 1 - r0) * cbs + j * 16 + lr]);
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
-    for (int q = 0; q < QT; ++q)
+                for (int i = 0; i < 4; ++i) creg[nt][q][j][i] = to_f(cbp[(int64_t)min(tl[q][i], limit - 1 - r0) * cbs + nt * 64 + j * 16 + lr]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (r0 + tl[q][i] >= limit) creg[q][j][i] = 0.f;
+        for (int q = 0; q < QT; ++q)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (r0 + tl[q][i] >= limit) creg[nt][q][j][i] = 0.f;
 #pragma unroll
     for (int it = 0; it < NTAB; ++it) {
         const int idx = threadIdx.x + it * DBDC_THREADS;
@@ -738,7 +786,7 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamb
             sbs[hh][rl] = rv;
         }
     }
-    f32x4 tot[QT][4] = {};
+    f32x4 tot[NT][QT][4] = {};
     __syncthreads();
 
     // ---- the head loop: raw LDS accesses and counted waits only ----
@@ -768,10 +816,11 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamb
         }
     }
     f32x4 tf[QT][4], tb[QT][4];
+    float uf[NT == 1 ? 1 : QT][4], ub[NT == 1 ? 1 : QT][4];     // (NT > 1: decay-gradient sums over the n tiles of a head)
     // SLOT = step % RING as a compile-time value: the slot's offset goes into the offset field of the LDS reads
     auto step_body = [&](int step, Frag (&af)[QT][NKS], auto SLOT) {
         constexpr int RB = decltype(SLOT)::value * NDIR * TILE_B;
-        const int hh = hh0 + step / nkc, kc = step % nkc;
+        const int hh = hh0 + step / per_head, kc = step % nkc;
         // this wave's requests of the step have landed (those of the next step may be outstanding) ...
         if (step + 1 < nsteps) wait_vmcnt<PER_STEP>();
         else wait_vmcnt<0>();
@@ -880,32 +929,47 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamb
         // the fragments of step + 2 take the place of the ones just used
         if (step + 2 < nsteps) issue_frags(step + 2, af);
         if (kc == nkc - 1) {
-            // ---- end of a head: its share of dB / dC and of the decay gradients
+            // ---- end of a head's n tile: its share of dB / dC and of the decay gradients.  (The tile's registers are picked by
+            // a compile-time index: the caller's branch on the tile is uniform.)
+            auto finish = [&](auto NTI) {
+                constexpr int nt = decltype(NTI)::value;
 #pragma unroll
-            for (int q = 0; q < QT; ++q) {
-                f32x4 sf4 = raw_lds_read_at<f32x4, 0>(sfs_a + ((hh - hh0) * ROWS + q * 16) * 4);
-                f32x4 sb4 = raw_lds_read_at<f32x4, 0>(sbs_a + ((hh - hh0) * ROWS + q * 16) * 4);
-                raw_lds_wait();
-                raw_lds_use(sf4); raw_lds_use(sb4);
-                f32x4 av, bv;
+                for (int q = 0; q < QT; ++q) {
+                    f32x4 sf4 = raw_lds_read_at<f32x4, 0>(sfs_a + ((hh - hh0) * ROWS + q * 16) * 4);
+                    f32x4 sb4 = raw_lds_read_at<f32x4, 0>(sbs_a + ((hh - hh0) * ROWS + q * 16) * 4);
+                    raw_lds_wait();
+                    raw_lds_use(sf4); raw_lds_use(sb4);
+                    f32x4 av, bv;
+                    constexpr int UQ = NT == 1 ? 0 : 1;
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    float uf = 0.f, ub = 0.f;
+                    for (int i = 0; i < 4; ++i) {
+                        float fs = nt == 0 ? 0.f : uf[q * UQ][i], bs = nt == 0 ? 0.f : ub[q * UQ][i];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        uf += tf[q][j][i] * creg[q][j][i];
-                        if (!UNI) ub += tb[q][j][i] * creg[q][j][i];
-                        tot[q][j][i] += UNI ? sf4[i] * tf[q][j][i] : sf4[i] * tf[q][j][i] + sb4[i] * tb[q][j][i];
+                        for (int j = 0; j < 4; ++j) {
+                            fs += tf[q][j][i] * creg[nt][q][j][i];
+                            if (!UNI) bs += tb[q][j][i] * creg[nt][q][j][i];
+                            tot[nt][q][j][i] += UNI ? sf4[i] * tf[q][j][i] : sf4[i] * tf[q][j][i] + sb4[i] * tb[q][j][i];
+                        }
+                        if constexpr (nt < NT - 1) {
+                            uf[q * UQ][i] = fs;
+                            ub[q * UQ][i] = bs;
+                        } else {
+                            av[i] = row16_sum(fs) * sf4[i];
+                            bv[i] = UNI ? 0.f : row16_sum(bs) * sb4[i];
+                        }
                     }
-                    av[i] = row16_sum(uf) * sf4[i];
-                    bv[i] = UNI ? 0.f : row16_sum(ub) * sb4[i];
+                    if constexpr (nt == NT - 1) {
+                        if (lr == 0) {
+                            const unsigned ua = uvs_a + (((hh - hh0) * NDIR) * ROWS + q * 16) * 4;
+                            raw_lds_write128_at<0>(ua, av);
+                            if (!UNI) raw_lds_write128_at<ROWS * 4>(ua, bv);
+                        }
+                    }
                 }
-                if (lr == 0) {
-                    const unsigned ua = uvs_a + (((hh - hh0) * NDIR) * ROWS + q * 16) * 4;
-                    raw_lds_write128_at<0>(ua, av);
-                    if (!UNI) raw_lds_write128_at<ROWS * 4>(ua, bv);
-                }
-            }
+            };
+            if constexpr (NT == 1) finish(std::integral_constant<int, 0>());
+            else if ((step / nkc) % NT == 0) finish(std::integral_constant<int, 0>());
+            else finish(std::integral_constant<int, 1>());
         }
     };
     static_assert(RING == 3, "six steps = one round of ring slots and of the two fragment sets");
@@ -928,21 +992,25 @@ __global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_dma_kernel(const bimamb
     }
     float *out = (IS_DB ? p.dBs : p.dCs) + (int64_t)blockIdx.z * p.batch * p.seqlen * p.ngroups * N;
 #pragma unroll
-    for (int q = 0; q < QT; ++q)
+    for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int q = 0; q < QT; ++q)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int n = j * 16 + lr, r = r0 + tl[q][i];
-                if (r < limit) out[(((int64_t)b * p.seqlen + (int64_t)c * Q + r) * p.ngroups + g) * N + n] = tot[q][j][i];
-            }
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int n = nt * 64 + j * 16 + lr, r = r0 + tl[q][i];
+                    if (r < limit) out[(((int64_t)b * p.seqlen + (int64_t)c * Q + r) * p.ngroups + g) * N + n] = tot[nt][q][j][i];
+                }
 }
 
 template <typename T, bool IS_DB>
 static int launch_dbdc_t(const bimamba2_params *p) {
     const int nc = nchunks(p);
+    if (dbdc_heads(p) > DBDC_HEADS) return BIMAMBA2_EINVAL;
     const int nt = (p->dstate + 63) / 64;
-    int qt = (p->chunk_size > 128 && nt == 1) ? 2 : 1;                // 16-row tiles per wave
+    // 16-row tiles per wave: two (a 256-row chunk reads each state once) where that still gives every CU a workgroup
+    int qt = (p->chunk_size > 128 && nt == 1 && (int64_t)p->batch * nc * p->ngroups * dbdc_slices(p) >= 256) ? 2 : 1;
     const int rows = DBDC_WAVES * 16 * qt;
     dim3 grid(p->batch * nc * p->ngroups, (p->chunk_size + rows - 1) / rows, dbdc_slices(p));
     constexpr int VS = 16 / (int)sizeof(T);
@@ -952,14 +1020,20 @@ static int launch_dbdc_t(const bimamba2_params *p) {
     else fast = fast && (p->has_z ? al(p->dout_x) : (al(p->dout) && p->dout_sb % VS == 0 && p->dout_sl % VS == 0 && p->dout_sh % VS == 0));
 #define BM2_DBDC(NTV, QTV)                                                                                                    \
     do {                                                                                                                  \
-        if (fast) hipLaunchKernelGGL((bwd_dbdc_kernel<T, NTV, QTV, IS_DB, true>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc); \
-        else hipLaunchKernelGGL((bwd_dbdc_kernel<T, NTV, QTV, IS_DB, false>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc);     \
+        if (fast) hipLaunchKernelGGL((bwd_dbdc_kernel<T, NTV, QTV, IS_DB, true>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p)); \
+        else hipLaunchKernelGGL((bwd_dbdc_kernel<T, NTV, QTV, IS_DB, false>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));     \
     } while (0)
     if constexpr (sizeof(T) == 2) {
-        // dstate 64: the variant with the ring of state tiles (16-byte aligned state tensors)
+        // dstate 64 and 128: the variant with the ring of state tiles (16-byte aligned state tensors)
         const void *c16f = IS_DB ? p->dstates16_f : p->states16_f, *c16b = IS_DB ? p->dstates16_b : p->states16_b;
         const bool st_al = c16f ? al(c16f) && al(c16b) && (p->causal || c16b)
                                 : (IS_DB ? al(p->dstates_f) && al(p->dstates_b) : al(p->states_f) && al(p->states_b));
+        if (fast && p->dstate == 128 && st_al && !p->causal) {
+            grid.y = (p->chunk_size + DBDC_WAVES * 16 - 1) / (DBDC_WAVES * 16);
+            if (c16f) hipLaunchKernelGGL((bwd_dbdc_dma_kernel<T, 1, IS_DB, false, true, 2>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));
+            else hipLaunchKernelGGL((bwd_dbdc_dma_kernel<T, 1, IS_DB, false, false, 2>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));
+            return check_launch();
+        }
         if (fast && p->dstate == 64 && st_al) {
             // 128-row tiles here: with eight heads per slice that is still one workgroup per CU at the usual sizes, and
             // the partial sums the slices leave behind (and bmm_chunk_bwd reads again) are half of what four heads give
@@ -967,8 +1041,8 @@ static int launch_dbdc_t(const bimamba2_params *p) {
             grid.y = (p->chunk_size + DBDC_WAVES * 16 - 1) / (DBDC_WAVES * 16);
 #define BM2_DMA(QTV, UNIV)                                                                                                                  \
     do {                                                                                                                                    \
-        if (c16f) hipLaunchKernelGGL((bwd_dbdc_dma_kernel<T, QTV, IS_DB, UNIV, true>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc);   \
-        else hipLaunchKernelGGL((bwd_dbdc_dma_kernel<T, QTV, IS_DB, UNIV, false>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc);       \
+        if (c16f) hipLaunchKernelGGL((bwd_dbdc_dma_kernel<T, QTV, IS_DB, UNIV, true>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));   \
+        else hipLaunchKernelGGL((bwd_dbdc_dma_kernel<T, QTV, IS_DB, UNIV, false>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));       \
     } while (0)
             if (p->causal) { BM2_DMA(1, true); }
             else { BM2_DMA(1, false); }
@@ -980,8 +1054,8 @@ static int launch_dbdc_t(const bimamba2_params *p) {
     if (p->causal) {
         if constexpr (sizeof(T) == 2) {
             if (fast && nt == 1) {
-                if (qt == 2) hipLaunchKernelGGL((bwd_dbdc_kernel<T, 1, 2, IS_DB, true, true>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc);
-                else hipLaunchKernelGGL((bwd_dbdc_kernel<T, 1, 1, IS_DB, true, true>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc);
+                if (qt == 2) hipLaunchKernelGGL((bwd_dbdc_kernel<T, 1, 2, IS_DB, true, true>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));
+                else hipLaunchKernelGGL((bwd_dbdc_kernel<T, 1, 1, IS_DB, true, true>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));
                 return check_launch();
             }
         }
@@ -1157,6 +1231,9 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_kernel(const bimamba2_params
 #pragma unroll
     for (int j = 0; j < 4; ++j) brow[j] = min(s0 + j * 16 + lr, limit - 1);
     const int nkc = (P + KC - 1) / KC;
+    // without FAST: whole vectors of the rows (unconditional loads from clamped addresses), or element by element
+    const bool whole = !FAST && P % KPL == 0 && aligned16(reinterpret_cast<const T *>(p.x), p.x_sb | p.x_sl | p.x_sh) &&
+                       (p.has_z ? aligned16(reinterpret_cast<const T *>(p.dout_x), P) : aligned16(reinterpret_cast<const T *>(p.dout), p.dout_sb | p.dout_sl | p.dout_sh));
 
     // blockIdx.z selects a slice of the group's heads; its dCB partial sum goes to slice blockIdx.z of the output
     const int hps = (hpg + gridDim.z - 1) / gridDim.z;
@@ -1207,8 +1284,11 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_kernel(const bimamba2_params
 #pragma unroll
             for (int ks = 0; ks < NKS; ++ks) {
                 const int kb = k0 + ks * KSTEP + lg * KPL;
-                if (FAST || ((reinterpret_cast<uintptr_t>(ar + kb) & 15) == 0 && kb + KPL <= P)) af[B_][ks] = M::load(ar + kb);
-                else {
+                if (FAST) af[B_][ks] = M::load(ar + kb);
+                else if (whole) {
+                    af[B_][ks] = M::load(ar + min(kb, P - KPL));
+                    if (kb >= P) af[B_][ks] = typename M::Frag{};
+                } else {
                     float v[KPL];
 #pragma unroll
                     for (int i = 0; i < KPL; ++i) v[i] = kb + i < P ? to_f(ar[kb + i]) : 0.f;
@@ -1221,8 +1301,11 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_kernel(const bimamba2_params
 #pragma unroll
                 for (int ks = 0; ks < NKS; ++ks) {
                     const int kb = k0 + ks * KSTEP + lg * KPL;
-                    if (FAST || ((reinterpret_cast<uintptr_t>(br + kb) & 15) == 0 && kb + KPL <= P)) bf[B_][j][ks] = M::load(br + kb);
-                    else {
+                    if (FAST) bf[B_][j][ks] = M::load(br + kb);
+                    else if (whole) {
+                        bf[B_][j][ks] = M::load(br + min(kb, P - KPL));
+                        if (kb >= P) bf[B_][j][ks] = typename M::Frag{};
+                    } else {
                         float v[KPL];
 #pragma unroll
                         for (int i = 0; i < KPL; ++i) v[i] = kb + i < P ? to_f(br[kb + i]) : 0.f;
@@ -1246,9 +1329,11 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_kernel(const bimamba2_params
             }
             if (it + 1 < nit) issue(it + 1);                // requested now, needed in the next iteration
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks)
+            for (int ks = 0; ks < NKS; ++ks) {
+                if (!FAST && (it % nkc) * KC + ks * KSTEP >= P) continue;      // (uniform) narrow heads
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc[j] = M::mma(afc[ks], bfc[j][ks], acc[j]);
+            }
             if (it % nkc == nkc - 1) {
                 // rows past the end of the sequence were read from a valid row: drop them
 #pragma unroll
@@ -1734,8 +1819,7 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_ring_kernel(const bimamba2_p
     bwd_dcb_ring_body<T, UNI>(p, nc, nqt, bid, gridDim.x, gridDim.z);
 }
 
-// The dCB kernel and the backward state passing as roles of one launch (16-bit copies of the entering states on both sides
-// of the state passing, one head slice): the first is bound by instruction issue and moves little data, the second streams
+// The dCB kernel and the backward state passing as roles of one launch (one head slice): the first is bound by instruction issue and moves little data, the second streams
 // 70 MB and needs few instructions, and the two depend on different kernels before them.  The first ndcb blocks are the
 // dCB tiles in the order of their own grid (so they are placed first, two per CU as when alone), the rest are the state
 // passing's blocks, which take what is left of each CU.
@@ -1748,6 +1832,7 @@ __device__ __forceinline__ void bwd_dcb_sp_body(const bimamba2_params &p, int nc
         const int k = id - ndcb;                  // grid (nsplit, nheads, batch * ndir) of the state passing
         const BlockId sb{k % nsplit, (k / nsplit) % p.nheads, k / (nsplit * p.nheads)};
         if (p.dstates_f == nullptr) state_passing_bwd_vec_body<T, true, true, true>(p, nc, nsplit, ndir, sb);
+        else if (p.dstates16_f == nullptr) state_passing_bwd_vec_body<T, false, false>(p, nc, nsplit, ndir, sb);
         else state_passing_bwd_vec_body<T, true, true>(p, nc, nsplit, ndir, sb);
     }
 }
@@ -1808,12 +1893,16 @@ static int launch_dcb_t(const bimamba2_params *p) {
 }
 
 // whether bwd_dcb_sp_kernel exists for the problem (the ring variant of the dCB kernel with one head slice, the vector
-// variant of the state passing, 16-bit copies of the entering states and of their gradients)
+// variant of the state passing)
 bool bwd_dcb_sp_merged(const bimamba2_params *p) {
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     if (p->dtype != BIMAMBA2_BF16 && p->dtype != BIMAMBA2_F16) return false;
     if (!dcb_recomputes_cb(p) || dcb_slices(p) != 1) return false;       // (implies the conditions of the ring variant)
-    if (!p->states16_f || !p->dstates16_f || !(p->causal || (p->states16_b && p->dstates16_b))) return false;
+    // the entering states and their gradients both in 16 bits, or (state dimension 128) both in float32
+    if (p->states16_f && p->dstates16_f ? !(p->causal || (p->states16_b && p->dstates16_b))
+                                        : p->states16_f || p->dstates16_f || p->causal || !p->states_f || !p->states_b || !p->dstates_f || !p->dstates_b)
+        return false;
+    if (!al(p->states_f) || !al(p->states_b)) return false;
     if ((p->headdim * p->dstate) % 4) return false;
     return al(p->states16_f) && al(p->states16_b) && al(p->dstates16_f) && al(p->dstates16_b) && al(p->dstates_f) && al(p->dstates_b) &&
            al(p->dfinal_f) && al(p->dfinal_b) && al(p->dinitial_f) && al(p->dinitial_b);
@@ -2249,11 +2338,12 @@ __global__ __launch_bounds__(NTHREADS) void bwd_tail_kernel(const bimamba2_param
                                                             int bmm_gy, int cs_gx, bool in16) {
     const int id = blockIdx.x;
     if (id < nbmm) {
-        // bmm grid (1, bmm_gy, z).  The bmm_gy row tiles of one z = (which, b, c, g) stage the same K operand (the chunk's C or
-        // B rows): consecutive ids are dealt round-robin to the 8 XCDs, so eight z at a time, one per XCD, go through their
+        // bmm grid (n tiles, bmm_gy, z), bmm_gy here counting both.  The bmm_gy tiles of one z = (which, b, c, g) stage the same
+        // K operand (the chunk's C or B rows, or the 64 columns of them that the n tile takes): consecutive ids are dealt round-robin to the 8 XCDs, so eight z at a time, one per XCD, go through their
         // row tiles (with the row tile fastest every XCD fetched every K operand: +100 MB of reads at 8 groups)
         const int nz = nbmm / bmm_gy, k = id >> 3;
-        const BlockId bb = nz % 8 == 0 ? BlockId{0, k % bmm_gy, (k / bmm_gy) * 8 + (id & 7)} : BlockId{0, id % bmm_gy, id / bmm_gy};
+        const int t = nz % 8 == 0 ? k % bmm_gy : id % bmm_gy, ntiles = p.dstate >> 6;
+        const BlockId bb{t % ntiles, t / ntiles, nz % 8 == 0 ? (k / bmm_gy) * 8 + (id & 7) : id / bmm_gy};
         bmm_chunk_bwd_body<T, 256, true, SLIM>(p, nc, nslices, bb, in16);
     } else {
         const int k = id - nbmm;                  // cumsum grid (cs_gx, nc, batch)
@@ -2271,11 +2361,11 @@ static bool bmm_bwd_fast(const bimamba2_params *p) {
 }
 
 // whether launch_bwd_tail() exists for this problem
-bool bwd_tail_merged(const bimamba2_params *p) { return bmm_bwd_fast(p) && p->chunk_size == 256 && p->dstate == 64; }
+bool bwd_tail_merged(const bimamba2_params *p) { return bmm_bwd_fast(p) && p->chunk_size == 256 && (p->dstate == 64 || p->dstate == 128); }
 
 template <typename T>
 static int launch_bwd_tail_t(const bimamba2_params *p, int nc, int nqt, int nsplit, bool in16) {
-    const int bmm_gy = (p->chunk_size + 63) / 64, nbmm = bmm_gy * p->batch * nc * p->ngroups * 2;
+    const int bmm_gy = (p->chunk_size + 63) / 64 * (p->dstate / 64), nbmm = bmm_gy * p->batch * nc * p->ngroups * 2;
     const int cs_gx = (p->nheads + 3) / 4, ncs = cs_gx * nc * p->batch;
     dim3 grid(nbmm + ncs);
     const int nsl = dbdc_slices(p);

@@ -129,9 +129,17 @@ __global__ __launch_bounds__(NTHREADS) void bmm_chunk_fwd_kernel(const bimamba2_
             const int t = tt * 64 + wave * 16 + (lane >> 4) * 4 + i, s = st * 64 + j * 16 + (lane & 15);
             if (t < Q && s < Q) {
                 out[(int64_t)t * Q + s] = acc[j][i];
-                if (outT) outT[(int64_t)s * Q + t] = acc[j][i];
+                if (outT && Q % 4) outT[(int64_t)s * Q + t] = acc[j][i];
             }
         }
+    if (outT && Q % 4 == 0) {
+        // a lane's four rows of the tile are four consecutive columns of the transposed one
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int t = tt * 64 + wave * 16 + (lane >> 4) * 4, s = st * 64 + j * 16 + (lane & 15);
+            if (t < Q && s < Q) *reinterpret_cast<f32x4 *>(outT + (int64_t)s * Q + t) = acc[j];
+        }
+    }
 }
 
 // =========================================================================================================
@@ -207,6 +215,7 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_kernel(const bimamba2_pa
             const typename M::Frag a = M::load(xT + xt_index<T, LDX>(wave * 16 + lr, kq));
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
+                if (!FAST && nt * 64 + j * 16 >= N) continue;      // (uniform) narrow states: nothing in this column tile
                 accf[j] = M::mma(a, M::load(Bf + xt_index<T, LDX>(j * 16 + lr, kq)), accf[j]);
                 accb[j] = M::mma(a, M::load(Bb + xt_index<T, LDX>(j * 16 + lr, kq)), accb[j]);
             }
@@ -1134,8 +1143,9 @@ int launch_bwd_dz_dstates(const bimamba2_params *p) {
 // together, unconditionally (past the last chunk a valid chunk is read again and not used).  Needs P*N % 4 == 0 and
 // 16-byte aligned tensors.
 // ndir = 1: the forward recurrence only (blockIdx.z = b).
-// T16 != void: the entering states go to the 16-bit copies (states16_*) and the per-chunk states stay as they are.
-template <typename T16>
+// T16 != void: the entering states go to the 16-bit copies (states16_*) and the per-chunk states stay as they are; with BOTH
+// they are replaced by the float32 entering states as well.
+template <typename T16, bool BOTH = false>
 __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_vec_kernel(const bimamba2_params p, int nc, int ndir) {
     const int PN = p.headdim * p.dstate;
     const int e = (blockIdx.x * NTHREADS + threadIdx.x) * 4;
@@ -1171,7 +1181,8 @@ __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_vec_kernel(const b
 #pragma unroll
                     for (int k = 0; k < 4; ++k) o.v[k] = from_f<TC>(s[k]);
                     *reinterpret_cast<Out4 *>(st16 + c * cstride) = o;
-                } else {
+                }
+                if constexpr (!COPY || BOTH) {
                     *reinterpret_cast<f32x4 *>(st + c * cstride) = s;
                 }
                 s = __expf(d[i]) * s + v[i];
@@ -1231,7 +1242,7 @@ __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_inplace16_kernel(c
     }
 }
 
-int launch_state_passing_fwd(const bimamba2_params *p) {
+int launch_state_passing_fwd(const bimamba2_params *p, bool both) {
     const int nc = nchunks(p), PN = p->headdim * p->dstate;
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     const int ndir = p->causal ? 1 : 2;
@@ -1247,7 +1258,11 @@ int launch_state_passing_fwd(const bimamba2_params *p) {
         dim3 grid((PN / 4 + NTHREADS - 1) / NTHREADS, p->nheads, p->batch * ndir);
         if (p->states16_f) {
             if (!(p->causal || p->states16_b) || !al(p->states16_f) || !al(p->states16_b)) return BIMAMBA2_EINVAL;
-            if (p->dtype == BIMAMBA2_BF16) hipLaunchKernelGGL(state_passing_fwd_vec_kernel<bf16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
+            if (both) {
+                if (p->dtype == BIMAMBA2_BF16) hipLaunchKernelGGL((state_passing_fwd_vec_kernel<bf16_t, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
+                else if (p->dtype == BIMAMBA2_F16) hipLaunchKernelGGL((state_passing_fwd_vec_kernel<f16_t, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
+                else return BIMAMBA2_EUNSUPPORTED;
+            } else if (p->dtype == BIMAMBA2_BF16) hipLaunchKernelGGL(state_passing_fwd_vec_kernel<bf16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
             else if (p->dtype == BIMAMBA2_F16) hipLaunchKernelGGL(state_passing_fwd_vec_kernel<f16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
             else return BIMAMBA2_EUNSUPPORTED;
         } else {
@@ -1255,7 +1270,7 @@ int launch_state_passing_fwd(const bimamba2_params *p) {
         }
         return check_launch();
     }
-    if (p->states16_f) return BIMAMBA2_EUNSUPPORTED;
+    if (p->states16_f) return BIMAMBA2_EUNSUPPORTED;     // (so that `both` is never dropped)
     if (p->causal) return BIMAMBA2_EUNSUPPORTED;
     dim3 grid((PN + NTHREADS - 1) / NTHREADS, p->nheads, p->batch);
     hipLaunchKernelGGL(state_passing_fwd_kernel, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc);

@@ -27,7 +27,7 @@ static inline hipStream_t stream_of(const bimamba2_params *p) { return reinterpr
 constexpr int SCAN_WAVES = 8, SCAN_THREADS = 64 * SCAN_WAVES;
 
 // FAST = true is chosen by the launcher when chunk_size % 32 == 0, headdim is a multiple of the column tile,
-// dstate % 64 == 0 and every operand is 16-byte aligned with strides that keep rows aligned: all guarded scalar
+// dstate a multiple of the elements in 16 bytes and every operand is 16-byte aligned with strides that keep rows aligned: all guarded scalar
 // fallbacks compile away and loads become unconditional (rows past the end of the sequence are read from a valid
 // row and never stored).
 //
@@ -122,10 +122,15 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
 #pragma unroll
             for (int s = 0; s < NW / KSTEP; ++s) {
                 const int r = rowi[rt], kb = n0 + s * KSTEP + lg * KPL;
-                if (FAST && KPL == 1) {
-                    arow[rt][s][0] = to_f(ap[(int64_t)min(r, limit - 1) * as + kb]);
-                } else if (KPL > 1 && (FAST || (r < limit && avec && kb + KPL <= N))) {
-                    Vec16<T> raw = *reinterpret_cast<const Vec16<T> *>(ap + (int64_t)(FAST ? min(r, limit - 1) : r) * as + kb);
+                if (FAST) {
+                    // (zeros behind the state dimension by masking the 16 bytes: a select per element cost the kernel 20 of 55 us)
+                    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+                    const u32x4 bits = *reinterpret_cast<const u32x4 *>(ap + (int64_t)min(r, limit - 1) * as + min(kb, N - KPL));
+                    const Vec16<T> raw = __builtin_bit_cast(Vec16<T>, bits & (kb < N ? ~0u : 0u));
+#pragma unroll
+                    for (int i = 0; i < KPL; ++i) arow[rt][s][i] = to_f(raw.v[i]);
+                } else if (r < limit && avec && kb + KPL <= N) {
+                    Vec16<T> raw = *reinterpret_cast<const Vec16<T> *>(ap + (int64_t)r * as + kb);
 #pragma unroll
                     for (int i = 0; i < KPL; ++i) arow[rt][s][i] = to_f(raw.v[i % Vec16<T>::N]);
                 } else {
@@ -342,8 +347,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
     };
     typedef std::integral_constant<int, 0> B0;
     typedef std::integral_constant<int, 1> B1;
-    // ---- part 2: inside the chunk.  A built in registers from CB (forward) or CB^T (mirror); the CB rows of
-    // the next K step are requested before the current step is consumed (two register buffers) ----
+    // ---- part 2: inside the chunk.  A built in registers from CB (forward) or CB^T (mirror) ----
     {
         const float *cb = (BWD ? p.CBT : p.CB) + ((int64_t)(b * nc + c) * p.ngroups + g) * Q * Q;
         const bool cvec = (Q % 4 == 0);
@@ -355,7 +359,10 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
             upr[rt] = up[rowi[rt]];
             rowp[rt] = cb + (int64_t)min(rowi[rt], Q - 1) * Q;
         }
-        float cbv[1][QT][KPL];
+        // two register buffers where there is room for them: the CB rows of the next K step are on their way while the current
+        // step is consumed (with 2 x 4 tiles of accumulators the kernel is at its 128 registers)
+        constexpr bool AHEAD = QT * NJ <= 4;
+        float cbv[AHEAD ? 2 : 1][QT][KPL];
         auto issue = [&](auto BUF, int k0) {
             constexpr int B_ = decltype(BUF)::value;
             const int kb = k0 + lg * KPL;
@@ -528,9 +535,21 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
             wait_vmcnt<0>();
             __syncthreads();
         } else {
-            for (int k0 = 0; k0 < limit; k0 += KSTEP) {
-                issue(B0(), k0);
-                process(B0(), k0);
+            if constexpr (AHEAD) {
+                issue(B0(), 0);
+                for (int k0 = 0; k0 < limit; k0 += 2 * KSTEP) {
+                    if (k0 + KSTEP < limit) issue(B1(), k0 + KSTEP);
+                    process(B0(), k0);
+                    if (k0 + KSTEP < limit) {
+                        if (k0 + 2 * KSTEP < limit) issue(B0(), k0 + 2 * KSTEP);
+                        process(B1(), k0 + KSTEP);
+                    }
+                }
+            } else {
+                for (int k0 = 0; k0 < limit; k0 += KSTEP) {
+                    issue(B0(), k0);
+                    process(B0(), k0);
+                }
             }
         }
     }
@@ -670,7 +689,7 @@ static inline int scan_col_tile(const bimamba2_params *p) {
 // whether the kernels without guarded fallbacks apply (vs = elements per 16 bytes)
 static bool scan_fast(const bimamba2_params *p, bool bwd, int pw, int vs) {
     auto mult = [vs](int64_t a, int64_t b, int64_t c) { return a % vs == 0 && b % vs == 0 && c % vs == 0; };
-    bool fast = p->chunk_size % 32 == 0 && p->headdim % pw == 0 && p->dstate % 64 == 0 && al16(p->x) && mult(p->x_sb, p->x_sl, p->x_sh);
+    bool fast = p->chunk_size % 32 == 0 && p->headdim % pw == 0 && p->dstate % vs == 0 && al16(p->x) && mult(p->x_sb, p->x_sl, p->x_sh);
     if (bwd) {
         fast = fast && al16(p->Bm) && mult(p->B_sb, p->B_sl, p->B_sg) && al16(p->dx) && mult(p->dx_sb, p->dx_sl, 0);
         fast = fast && (p->has_z ? al16(p->dout_x) : (al16(p->dout) && mult(p->dout_sb, p->dout_sl, p->dout_sh)));
@@ -687,7 +706,7 @@ static bool scan_rebuild_shape(const bimamba2_params *p, bool bwd) {
     auto mult = [](int64_t a, int64_t b, int64_t c) { return a % 8 == 0 && b % 8 == 0 && c % 8 == 0; };
     if (p->B_sl <= 0 || p->C_sl <= 0 || p->B_sl > (1 << 21) || p->C_sl > (1 << 21)) return false;   // 256 rows in 32-bit byte offsets
     if (!(bwd ? al16(p->dstates_f) && al16(p->dstates_b) : al16(p->states_f) && al16(p->states_b))) return false;
-    return scan_fast(p, bwd, 64, 8) && al16(p->Bm) && mult(p->B_sb, p->B_sl, p->B_sg) && al16(p->Cm) && mult(p->C_sb, p->C_sl, p->C_sg);
+    return p->dstate % 64 == 0 && scan_fast(p, bwd, 64, 8) && al16(p->Bm) && mult(p->B_sb, p->B_sl, p->B_sg) && al16(p->Cm) && mult(p->C_sb, p->C_sl, p->C_sg);
 }
 
 bool scan_recomputes_cb(const bimamba2_params *p, bool bwd) { return p->dstate == 64 && scan_rebuild_shape(p, bwd); }

@@ -29,7 +29,8 @@ bool chunk_states_in_16bit(const bimamba2_params *p);
 // the chunk-state kernel whose workgroups walk through several heads of one (batch, chunk): where it is used, and its launch
 bool chunk_state_uses_heads_kernel(const bimamba2_params *p);
 int launch_chunk_state_heads(const bimamba2_params *p);
-int launch_state_passing_fwd(const bimamba2_params *p);
+// both: the entering states in float32 (in place of the per-chunk states) and in the 16-bit copies
+int launch_state_passing_fwd(const bimamba2_params *p, bool both = false);
 int launch_chunk_scan(const bimamba2_params *p, bool bwd);
 // the 16-bit kernel of kernels_scan16.hip (launch_chunk_scan picks it where it applies)
 int launch_chunk_scan16(const bimamba2_params *p, bool bwd);
@@ -46,6 +47,7 @@ int launch_bwd_dz(const bimamba2_params *p);
 bool bwd_dz_dstates_fused(const bimamba2_params *p);   // dz and dstates as one launch
 int launch_bwd_dz_dstates(const bimamba2_params *p);
 int launch_state_passing_bwd(const bimamba2_params *p);
+int choose_dbdc_heads(const bimamba2_params *p);   // heads per slice of the dB / dC partial sums
 int launch_bwd_dbdc(const bimamba2_params *p, bool is_db);
 int launch_bwd_dcb(const bimamba2_params *p);
 int dcb_slices(const bimamba2_params *p);   // head slices whose dCB partial sums the kernel keeps apart

@@ -101,7 +101,7 @@ typedef struct bimamba2_params {
     float *ddt_direct, *u_f, *u_b, *v_f, *v_b;     /* ddt_direct: bimamba2_ddt_direct_planes() planes of (B, H, nc, Q) */
     float *da_intra;                    /* (B, H, nc, T*T, 2, 64), T = ceil(Q/64): per-tile column / row sums */
     float *ddA_chunk_f, *ddA_chunk_b;   /* (B, H, nc, ceil(P*N/1024)) partial sums */
-    float *dBs, *dCs;                   /* (S, B, L, G, N) float32 partial gradients, S = ceil(H/G/8) head slices */
+    float *dBs, *dCs;                   /* (S, B, L, G, N) float32 partial gradients, S = ceil(H/G/8) head slices (see dbdc_heads) */
     float *red;                         /* scratch for two-stage reductions: max(B*nc*H*P, 2*B*nc*H) floats for the single
                                            stages, B*nc*H*P + 2*B*nc*H for bimamba2_bwd */
     /* States at the ends of the sequence, all (B, H, P, N) float32, all optional (NULL = absent).  The reference's
@@ -159,6 +159,9 @@ typedef struct bimamba2_params {
        8 elements (16 bytes) where the vector kernels are to run. */
     int64_t dx_sb, dx_sl, dB_sb, dB_sl, dC_sb, dC_sl;
     int64_t ddt_sb, ddt_sl;         /* likewise of ddt (batch, seqlen, nheads): 0 means contiguous */
+    int32_t dbdc_heads;             /* heads per slice of dBs / dCs (1..8): S = ceil(H/G/dbdc_heads); 0 means 8.  bimamba2_bwd
+                                       chooses it itself where dBs and dCs are its own. */
+    int32_t reserved;
 } bimamba2_params;
 
 /* text of an error code */
