@@ -192,33 +192,40 @@ class BiMamba2(nn.Module):
         self.norm = RMSNormGated(self.d_inner, eps=1e-5, norm_before_gate=True, **fk)
         self.out_proj = nn.Linear(self.d_inner, d_model, bias=bias, **fk)
 
-    def _takes_native_path(self, u):
-        """Whether forward() may run as ONE native autograd function (csrc/host.cpp: the two GEMMs and this library's kernels,
-        no Python between them): what the kernels take in one piece, and nobody who expects the projections to be called as
-        modules, or the gradients' pieces as separate tensors (_GradPieces.on_copied) - hooks, replaced or patched
-        projections, autocast."""
+    def _native_tensors(self, u):
+        """The layer's parameters if forward() may run as ONE native autograd function (csrc/host.cpp: the two GEMMs and this
+        library's kernels, no Python between them), else None.  It may for what the kernels take in one piece, where nobody
+        expects the projections to be called as modules, or the gradients' pieces as separate tensors
+        (_GradPieces.on_copied): no hooks, no replaced or patched projections, no autocast."""
         if not (u.is_cuda and u.dim() == 3 and u.dtype in _DT and self.headdim <= MAX_HEADDIM and self.d_state <= MAX_DSTATE
                 and self.chunk_size >= 32) or _GradPieces.on_copied is not None or torch.is_autocast_enabled("cuda"):
-            return False
+            return None
         m = torch.nn.modules.module
         if m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks:
-            return False
-        for lin in (self.in_proj, self.out_proj):
+            return None
+        # (straight from the modules' tables: attribute access on a module costs a microsecond each)
+        parts, own = self._modules, self._parameters
+        in_proj, out_proj, norm = parts["in_proj"], parts["out_proj"], parts["norm"]
+        for lin in (in_proj, out_proj):
             if (type(lin) is not nn.Linear or lin._forward_hooks or lin._forward_pre_hooks or lin._backward_hooks
-                    or lin._backward_pre_hooks or "forward" in lin.__dict__ or lin.weight.dtype != u.dtype):
-                return False
-        if self.norm.bias is not None or self.conv1d.weight.dim() != 3:
-            return False
-        return all(type(t) in (nn.Parameter, torch.Tensor) and t.dtype in _DT for t in self._native_tensors() if t is not None)
-
-    def _native_tensors(self):
-        return (self.in_proj.weight, self.in_proj.bias, self.A_log, self.D, self.dt_bias, self.conv1d.weight, self.conv1d.bias,
-                self.norm.weight, self.out_proj.weight, self.out_proj.bias)
+                    or lin._backward_pre_hooks or "forward" in lin.__dict__):
+                return None
+        ip, op, conv, nrm = in_proj._parameters, out_proj._parameters, parts["conv1d"]._parameters, norm._parameters
+        get = lambda table, name: table.get(name, False)
+        tensors = (get(ip, "weight"), get(ip, "bias"), get(own, "A_log"), get(own, "D"), get(own, "dt_bias"), get(conv, "weight"),
+                   get(conv, "bias"), get(nrm, "weight"), get(op, "weight"), get(op, "bias"))
+        for t in tensors:                # (False: not a plain parameter of its module - parametrised, replaced, removed)
+            if t is not None and (type(t) is not nn.Parameter or t.dtype not in _DT):
+                return None
+        if tensors[0].dtype != u.dtype or tensors[8].dtype != u.dtype or nrm.get("bias") is not None:
+            return None
+        return tensors
 
     def forward(self, u):
-        if self._takes_native_path(u):
-            norm = self.norm
-            return _lib.host().layer(u, *self._native_tensors(), self.headdim, self.ngroups, self.d_state, min(self.chunk_size, MAX_CHUNK_SIZE),
+        tensors = self._native_tensors(u)
+        if tensors is not None:
+            norm = self._modules["norm"]
+            return _lib.host().layer(u, *tensors, self.headdim, self.ngroups, self.d_state, min(self.chunk_size, MAX_CHUNK_SIZE),
                                      self.dt_limit[0], self.dt_limit[1], norm.eps, norm.group_size or self.d_inner,
                                      norm.norm_before_gate)
         bc = self.ngroups * self.d_state

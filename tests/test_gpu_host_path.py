@@ -35,10 +35,10 @@ def test_layer_equals_its_composition(case, monkeypatch):
             assert_close(m(u), out.detach().double(), dtype, "output without autograd", scaled=True)
         return (out.detach(),) + torch.autograd.grad(out, list(live.values()), dy)
 
-    assert m._takes_native_path(u)
+    assert m._native_tensors(u) is not None
     native = step()
     monkeypatch.setattr(_GradPieces, "on_copied", staticmethod(lambda copied: None))      # (its observer gets the composition)
-    assert not m._takes_native_path(u)
+    assert m._native_tensors(u) is None
     for name, a, b in zip(["out"] + list(live), native, step()):
         assert a.shape == b.shape and a.dtype == b.dtype, name
         assert_close(a, b.double(), dtype, name, scaled=True)
