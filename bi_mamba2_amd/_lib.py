@@ -54,7 +54,7 @@ ALL_SYMBOLS = ENTRY_POINTS + ("bimamba2_strerror", "bimamba2_version", "bimamba2
                               "bimamba2_chunk_scan_heads_per_workgroup", "bimamba2_ddt_direct_planes", "bimamba2_norm_params_size",
                               "bimamba2_rmsnorm_gated_workspace_bytes", "bimamba2_conv_params_size",
                               "bimamba2_conv1d_silu_workspace_bytes", "bimamba2_cast_params_size",
-                              "bimamba2_cast_many") + NORM_ENTRY_POINTS + CONV_ENTRY_POINTS
+                              "bimamba2_cast_many", "bimamba2_gemm_params_size", "bimamba2_gemm_workspace_bytes", "bimamba2_gemm") + NORM_ENTRY_POINTS + CONV_ENTRY_POINTS
 
 _lib = None
 
@@ -92,6 +92,12 @@ class CastItem(ctypes.Structure):
 class CastParams(ctypes.Structure):
     """Mirror of ``struct bimamba2_cast_params`` (several small conversions in one launch)."""
     _fields_ = [("count", _i32), ("reserved", _i32), ("item", CastItem * CAST_MAX), ("stream", _vp)]
+
+
+class GemmParams(ctypes.Structure):
+    """Mirror of ``struct bimamba2_gemm_params`` (matrix product of the layer's projections)."""
+    _fields_ = ([(n, _i32) for n in ("m", "n", "k", "dtype", "a_kcontig", "b_kcontig")] + [(n, _i64) for n in ("lda", "ldb", "ldc")]
+                + [(n, _vp) for n in ("a", "b", "bias", "c", "partial")] + [("partial_bytes", ctypes.c_size_t), ("stream", _vp)])
 
 
 def load():
@@ -147,6 +153,13 @@ def load():
     lib.bimamba2_cast_params_size.restype = ctypes.c_size_t
     if lib.bimamba2_cast_params_size() != ctypes.sizeof(CastParams):
         raise RuntimeError("bimamba2_cast_params layout mismatch between the library and its Python mirror")
+    lib.bimamba2_gemm_params_size.restype = ctypes.c_size_t
+    if lib.bimamba2_gemm_params_size() != ctypes.sizeof(GemmParams):
+        raise RuntimeError("bimamba2_gemm_params layout mismatch between the library and its Python mirror")
+    lib.bimamba2_gemm_workspace_bytes.argtypes = [ctypes.POINTER(GemmParams)]
+    lib.bimamba2_gemm_workspace_bytes.restype = ctypes.c_size_t
+    lib.bimamba2_gemm.argtypes = [ctypes.POINTER(GemmParams)]
+    lib.bimamba2_gemm.restype = ctypes.c_int
     lib.bimamba2_cast_many.argtypes = [ctypes.POINTER(CastParams)]
     lib.bimamba2_cast_many.restype = ctypes.c_int
     _lib = lib

@@ -564,4 +564,32 @@ int bimamba2_conv1d_silu_bwd(const bimamba2_conv_params *p) {
     return launch_conv1d_silu(p, true);
 }
 
+size_t bimamba2_gemm_params_size(void) { return sizeof(bimamba2_gemm_params); }
+
+static int check_gemm(const bimamba2_gemm_params *p) {
+    if (!p || p->m <= 0 || p->n <= 0 || p->k <= 0 || !p->a || !p->b || !p->c) return BIMAMBA2_EINVAL;
+    if (p->dtype != BIMAMBA2_BF16 && p->dtype != BIMAMBA2_F16) return BIMAMBA2_EUNSUPPORTED;
+    auto al16 = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    if (!al16(p->a) || !al16(p->b) || !al16(p->c) || p->lda % 8 || p->ldb % 8 || p->ldc < p->n) return BIMAMBA2_EUNSUPPORTED;
+    auto up8 = [](int64_t v) { return (v + 7) / 8 * 8; };
+    if (p->lda < up8(p->a_kcontig ? p->k : p->m) || p->ldb < up8(p->b_kcontig ? p->k : p->n)) return BIMAMBA2_EUNSUPPORTED;
+    // offsets inside a tile are 32-bit products of 24-bit factors: 256 rows of k, or the whole k range of rows
+    if (p->lda >= (1 << 23) || p->ldb >= (1 << 23) || p->k >= (1 << 24)) return BIMAMBA2_EUNSUPPORTED;
+    const int64_t most = int64_t(1) << 31;
+    if ((p->a_kcontig ? 256 : (int64_t)p->k) * p->lda * 2 + 2 * (int64_t)p->k >= 2 * most) return BIMAMBA2_EUNSUPPORTED;
+    if ((p->b_kcontig ? 256 : (int64_t)p->k) * p->ldb * 2 + 2 * (int64_t)p->k >= 2 * most) return BIMAMBA2_EUNSUPPORTED;
+    if (!p->a_kcontig && p->b_kcontig) return BIMAMBA2_EUNSUPPORTED;
+    if (p->b_kcontig && p->k % 8) return BIMAMBA2_EUNSUPPORTED;   // what lies behind a row of B is multiplied by zero: it must be numbers
+    return BIMAMBA2_OK;
+}
+
+size_t bimamba2_gemm_workspace_bytes(const bimamba2_gemm_params *p) { return check_gemm(p) ? 0 : gemm_workspace_bytes(p); }
+
+int bimamba2_gemm(const bimamba2_gemm_params *p) {
+    TRY(check_gemm(p));
+    const size_t need = gemm_workspace_bytes(p);
+    if (need && (!p->partial || p->partial_bytes < need)) return BIMAMBA2_EWORKSPACE;
+    return launch_gemm(p);
+}
+
 }  // extern "C"

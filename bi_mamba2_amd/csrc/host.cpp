@@ -52,6 +52,8 @@ struct Api {
     decltype(&bimamba2_conv1d_silu_bwd) conv_bwd = nullptr;
     decltype(&bimamba2_conv1d_silu_workspace_bytes) conv_workspace = nullptr;
     decltype(&bimamba2_cast_many) cast_many = nullptr;
+    decltype(&bimamba2_gemm) gemm = nullptr;
+    decltype(&bimamba2_gemm_workspace_bytes) gemm_workspace = nullptr;
 } api;
 
 void load(const std::string &path) {
@@ -61,13 +63,15 @@ void load(const std::string &path) {
         fn = reinterpret_cast<std::remove_reference_t<decltype(fn)>>(dlsym(lib, name));
         TORCH_CHECK(fn, path, " does not export ", name);
     };
-    size_t (*params_size)() = nullptr, (*norm_size)() = nullptr, (*conv_size)() = nullptr, (*cast_size)() = nullptr;
+    size_t (*params_size)() = nullptr, (*norm_size)() = nullptr, (*conv_size)() = nullptr, (*cast_size)() = nullptr, (*gemm_size)() = nullptr;
     get(params_size, "bimamba2_params_size");
     get(norm_size, "bimamba2_norm_params_size");
     get(conv_size, "bimamba2_conv_params_size");
     get(cast_size, "bimamba2_cast_params_size");
+    get(gemm_size, "bimamba2_gemm_params_size");
     TORCH_CHECK(params_size() == sizeof(bimamba2_params) && norm_size() == sizeof(bimamba2_norm_params) &&
-                    conv_size() == sizeof(bimamba2_conv_params) && cast_size() == sizeof(bimamba2_cast_params),
+                    conv_size() == sizeof(bimamba2_conv_params) && cast_size() == sizeof(bimamba2_cast_params) &&
+                    gemm_size() == sizeof(bimamba2_gemm_params),
                 path, " was built from another version of include/bimamba2.h");
     get(api.fwd, "bimamba2_fwd");
     get(api.bwd, "bimamba2_bwd");
@@ -82,6 +86,8 @@ void load(const std::string &path) {
     get(api.conv_bwd, "bimamba2_conv1d_silu_bwd");
     get(api.conv_workspace, "bimamba2_conv1d_silu_workspace_bytes");
     get(api.cast_many, "bimamba2_cast_many");
+    get(api.gemm, "bimamba2_gemm");
+    get(api.gemm_workspace, "bimamba2_gemm_workspace_bytes");
 }
 
 void check(int rc, const char *entry) {
@@ -508,10 +514,11 @@ Params32 params_as_float32(std::array<Tensor, Params32::N> &prm, void *stream) {
 
 struct LayerShape {
     int64_t batch, seqlen, rows, inner, conv, proj, width;
+    int64_t pitch;      // of the rows of the projection's output: whole cache lines, and aligned for vector loads whatever nheads is
     size_t e;
     LayerShape(const Tensor &u, const Tensor &cw, const LayerOpts &o)
         : batch(u.size(0)), seqlen(u.size(1)), rows(batch * seqlen), inner(o.inner), conv(o.inner + 2 * o.ngroups * o.dstate),
-          proj(o.inner + conv + o.nheads), width(cw.size(-1)), e(u.element_size()) {}
+          proj(o.inner + conv + o.nheads), width(cw.size(-1)), pitch((proj + 63) / 64 * 64), e(u.element_size()) {}
 };
 
 inline char *at_byte(const Tensor &t, size_t elements) { return static_cast<char *>(t.mutable_data_ptr()) + elements * t.element_size(); }
@@ -522,8 +529,8 @@ bimamba2_conv_params conv_params(const LayerShape &s, const Tensor &zx, const Pa
     c.dtype = dtype_code(zx.scalar_type(), "dtype");
     c.has_bias = w.ptr[4] != nullptr;
     c.x = at_byte(zx, s.inner);
-    c.x_sb = s.seqlen * s.proj;
-    c.x_sl = s.proj;
+    c.x_sb = s.seqlen * s.pitch;
+    c.x_sl = s.pitch;
     c.weight = w.ptr[3];
     c.bias = w.ptr[4];
     c.stream = stream;
@@ -544,7 +551,7 @@ bimamba2_params layer_scan_params(const LayerShape &s, const LayerOpts &o, const
     p.Cm = at_byte(xbc, s.inner + o.ngroups * o.dstate);
     p.B_sb = p.C_sb = s.seqlen * s.conv; p.B_sl = p.C_sl = s.conv; p.B_sg = p.C_sg = o.dstate;
     p.dt = at_byte(zx, s.inner + s.conv);
-    p.dt_sb = s.seqlen * s.proj; p.dt_sl = s.proj; p.dt_sh = 1;
+    p.dt_sb = s.seqlen * s.pitch; p.dt_sl = s.pitch; p.dt_sh = 1;
     p.A = w.ptr[0]; p.D = w.ptr[1]; p.dt_bias = w.ptr[2];
     p.stream = stream;
     return p;
@@ -558,10 +565,77 @@ bimamba2_norm_params layer_norm_params(const LayerShape &s, const LayerOpts &o, 
     n.norm_before_gate = o.norm_before_gate;
     n.eps = (float)o.eps;
     n.x = y.const_data_ptr(); n.x_rs = s.inner;
-    n.z = at_byte(zx, 0); n.z_rs = s.proj;
+    n.z = at_byte(zx, 0); n.z_rs = s.pitch;
     n.weight = w.ptr[5];
     n.stream = stream;
     return n;
+}
+
+// ---- the projections' matrix products -------------------------------------------------------------------------------
+// c (m x n, row pitch ldc) = sum_k A(m, k) B(n, k) (+ bias), by this library's kernel; false where it does not take the problem.
+// a, b: 2-d with unit stride along columns; a_kc: k along a's columns (else along its rows), b_kc likewise.
+bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const Tensor &bias, const Tensor &c) {
+    if (c.scalar_type() == at::kFloat || a.stride(1) != 1 || b.stride(1) != 1 || c.stride(1) != 1) return false;
+    bimamba2_gemm_params g{};
+    g.m = c.size(0);
+    g.n = c.size(1);
+    g.k = a.size(a_kc ? 1 : 0);
+    g.dtype = dtype_code(c.scalar_type(), "dtype");
+    g.a_kcontig = a_kc;
+    g.b_kcontig = b_kc;
+    g.lda = a.stride(0);
+    g.ldb = b.stride(0);
+    g.ldc = c.stride(0);
+    g.a = a.const_data_ptr();
+    g.b = b.const_data_ptr();
+    g.bias = bias.defined() ? bias.const_data_ptr() : nullptr;
+    g.c = c.mutable_data_ptr();
+    g.stream = stream_of(c);
+    const size_t need = api.gemm_workspace(&g);
+    Tensor ws;
+    if (need) {
+        ws = device_empty({(int64_t)need}, at::kByte, c);
+        g.partial = static_cast<float *>(ws.mutable_data_ptr());
+        g.partial_bytes = need;
+    }
+    const int rc = api.gemm(&g);
+    if (rc == BIMAMBA2_EUNSUPPORTED) return false;
+    check(rc, "bimamba2_gemm");
+    return true;
+}
+
+// Operations up to which the own kernel takes a product whose library call would be as fast or faster on the GPU: the call
+// costs the host 22 us, and up to here the own kernel ends within that time (3.5 GFLOP: 14 us).
+constexpr double OWN_PRODUCT_FLOPS = 5e9;
+
+// c = x w^T (+ bias): the forward product.  c may be a view with a row pitch.
+void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c) {
+    const double flops = 2.0 * c.size(0) * c.size(1) * x.size(1);
+    if (flops <= OWN_PRODUCT_FLOPS && own_product(x, true, w, true, bias, c)) return;
+    // The library's kernels work at full rate on output columns in multiples of 256 and at half of it otherwise (16384 x 768 by
+    // 3072 columns 72 us, by 3224 columns 147 us): the remaining columns go to the own kernel (16 us there).
+    const int64_t n = c.size(1), whole = n / 256 * 256;
+    if (whole && whole != n && c.scalar_type() != at::kFloat && !bias.defined() &&
+        own_product(x, true, w.narrow(0, whole, n - whole), true, Tensor(), c.narrow(1, whole, n - whole))) {
+        Tensor front = c.narrow(1, 0, whole);
+        at::mm_out(front, x, w.narrow(0, 0, whole).t());
+        return;
+    }
+    if (bias.defined()) at::addmm_out(c, bias, x, w.t());
+    else at::mm_out(c, x, w.t());
+}
+
+// c = dy w: the gradient of a projection's input
+void product_nn(const Tensor &dy, const Tensor &w, Tensor c) {
+    if (2.0 * c.size(0) * c.size(1) * dy.size(1) <= OWN_PRODUCT_FLOPS && own_product(dy, true, w, false, Tensor(), c)) return;
+    at::mm_out(c, dy, w);
+}
+
+// c = dy^T x: the gradient of a projection's weight.  Always the own kernel where it exists: the library does not cut the long
+// sum over the rows (3224 x 768 over 16384 rows: 157 us against 93).
+void product_tn(const Tensor &dy, const Tensor &x, Tensor c) {
+    if (own_product(dy, false, x, false, Tensor(), c)) return;
+    at::mm_out(c, dy.t(), x);
 }
 
 struct LayerKept {
@@ -573,7 +647,8 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
     const LayerShape s(u, prm[3], o);
     void *stream = stream_of(u);
     const Tensor u2 = u.reshape({s.rows, u.size(2)});
-    const Tensor zx = b_in.defined() ? at::addmm(b_in, u2, w_in.t()) : at::mm(u2, w_in.t());
+    const Tensor zx = device_empty({s.rows, s.pitch}, u.scalar_type(), u).narrow(1, 0, s.proj);
+    product_nt(u2, w_in, b_in, zx);
     const Params32 w = params_as_float32(prm, stream);
 
     const Tensor xbc = device_empty({s.rows, s.conv}, u.scalar_type(), u);
@@ -604,9 +679,10 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
         n.rstd = rstd.mutable_data_ptr<float>();
     }
     check(api.norm_fwd(&n), "bimamba2_rmsnorm_gated_fwd");
-    const Tensor out = b_out.defined() ? at::addmm(b_out, yn, w_out.t()) : at::mm(yn, w_out.t());
+    const Tensor out = device_empty({s.batch, s.seqlen, w_out.size(0)}, u.scalar_type(), u);
+    product_nt(yn, w_out, b_out, out.view({s.rows, w_out.size(0)}));
     if (left) *left = {zx, xbc, y, yn, rstd, kept, w.buf};
-    return out.view({s.batch, s.seqlen, w_out.size(0)});
+    return out;
 }
 
 class LayerFn : public torch::autograd::Function<LayerFn> {
@@ -634,11 +710,12 @@ public:
         const std::array<Tensor, Params32::N> prm = {v[2], v[3], v[4], v[5], v[6], v[7]};
         const c10::DeviceGuard guard(u.device());
         void *stream = stream_of(u);
+        at::AutoDispatchBelowADInplaceOrView below;
         const LayerShape s(u, prm[3], o);
         const Params32 w = point_params(prm, v[15]);
         const Tensor dout = as_type(grads[0], u.scalar_type()).reshape({s.rows, w_out.size(0)});
         Tensor dw_in, db_in, dw_out, db_out, du;
-        if (needs(9)) dw_out = at::mm(dout.t(), yn);
+        if (needs(9)) product_tn(dout, yn, dw_out = device_empty(w_out.sizes(), u.scalar_type(), u));
         if (needs(10)) db_out = dout.sum(0);
 
         // float32 gradients of the small parameters, one buffer: A, D, dt_bias, conv weight, conv bias, norm weight
@@ -647,13 +724,15 @@ public:
         const Tensor g32 = device_empty({off.back()}, at::kFloat, u);
         float *g = g32.mutable_data_ptr<float>();
 
-        const Tensor dyn = at::mm(dout, w_out), dy = device_empty({s.rows, s.inner}, u.scalar_type(), u), dzx = device_empty({s.rows, s.proj}, u.scalar_type(), u);
+        const Tensor dyn = device_empty({s.rows, s.inner}, u.scalar_type(), u), dy = device_empty({s.rows, s.inner}, u.scalar_type(), u);
+        const Tensor dzx = device_empty({s.rows, s.pitch}, u.scalar_type(), u).narrow(1, 0, s.proj);
+        product_nn(dout, w_out, dyn);
         {
             bimamba2_norm_params n = layer_norm_params(s, o, zx, y, w, stream);
             n.rstd = rstd.mutable_data_ptr<float>();
             n.dout = dyn.const_data_ptr(); n.dout_rs = s.inner;
             n.dx = dy.mutable_data_ptr(); n.dx_rs = s.inner;
-            n.dz = at_byte(dzx, 0); n.dz_rs = s.proj;
+            n.dz = at_byte(dzx, 0); n.dz_rs = s.pitch;
             n.dweight = g + off[5];
             const Tensor ws = device_empty({(int64_t)std::max<size_t>(api.norm_workspace(&n), 1)}, at::kByte, u);
             n.workspace = ws.mutable_data_ptr();
@@ -673,7 +752,7 @@ public:
             p.dx_sb = p.dB_sb = p.dC_sb = s.seqlen * s.conv;
             p.dx_sl = p.dB_sl = p.dC_sl = s.conv;
             p.ddt = at_byte(dzx, s.inner + s.conv);
-            p.ddt_sb = s.seqlen * s.proj; p.ddt_sl = s.proj;
+            p.ddt_sb = s.seqlen * s.pitch; p.ddt_sl = s.pitch;
             p.dA = g + off[0]; p.dD = g + off[1]; p.ddt_bias = g + off[2];
             const Tensor ws = attach_workspace(p, true, u);
             check(api.bwd(&p), "bimamba2_bwd");
@@ -683,7 +762,7 @@ public:
             c.dout = dxbc.const_data_ptr();
             c.dout_sb = s.seqlen * s.conv; c.dout_sl = s.conv;
             c.dx = at_byte(dzx, s.inner);
-            c.dx_sb = s.seqlen * s.proj; c.dx_sl = s.proj;
+            c.dx_sb = s.seqlen * s.pitch; c.dx_sl = s.pitch;
             c.dweight = g + off[3];
             if (prm[4].defined()) c.dbias = g + off[4];
             const Tensor ws = device_empty({(int64_t)std::max<size_t>(api.conv_workspace(&c), 1)}, at::kByte, u);
@@ -708,8 +787,11 @@ public:
                      i == 0 ? BIMAMBA2_CAST_MUL : BIMAMBA2_CAST_COPY, i == 0 ? w.ptr[0] : nullptr);
         }
         if (c.count) check(api.cast_many(&c), "bimamba2_cast_many");
-        if (needs(0)) du = at::mm(dzx, w_in).view(u.sizes());
-        if (needs(1)) dw_in = at::mm(dzx.t(), u.reshape({s.rows, u.size(2)}));
+        if (needs(0)) {
+            du = device_empty(u.sizes(), u.scalar_type(), u);
+            product_nn(dzx, w_in, du.view({s.rows, u.size(2)}));
+        }
+        if (needs(1)) product_tn(dzx, u.reshape({s.rows, u.size(2)}), dw_in = device_empty(w_in.sizes(), u.scalar_type(), u));
         if (needs(2)) db_in = dzx.sum(0);
         return {du, dw_in, db_in, dprm[0], dprm[1], dprm[2], dprm[3], dprm[4], dprm[5], dw_out, db_out, Tensor()};
     }

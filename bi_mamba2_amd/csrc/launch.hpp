@@ -82,4 +82,8 @@ size_t conv_workspace_bytes(const bimamba2_conv_params *p);
 // several small element-wise conversions in one launch (kernels_conv.hip)
 int launch_cast_many(const bimamba2_cast_params *p);
 
+// matrix products of the layer's projections (kernels_gemm.hip)
+int launch_gemm(const bimamba2_gemm_params *p);
+size_t gemm_workspace_bytes(const bimamba2_gemm_params *p);
+
 }  // namespace bm2

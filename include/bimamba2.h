@@ -390,6 +390,29 @@ typedef struct bimamba2_cast_params {
 size_t bimamba2_cast_params_size(void);
 int bimamba2_cast_many(const bimamba2_cast_params *p);
 
+/* ---------------------------------------------------------------------------------------------------------
+ * Matrix product for the layer's projections, 16-bit operands, float32 accumulation:
+ *   c[m, n] = sum_k A(m, k) B(n, k) (+ bias[n])
+ * a_kcontig: A(m, k) = a[m * lda + k], else a[k * lda + m]; b_kcontig likewise for B(n, k) (a_kcontig = 0 with b_kcontig = 1 is
+ * not built).  lda, ldb multiples of 8, a, b and c 16-byte aligned; an operand is read in whole 16-byte pieces of its contiguous
+ * dimension, so its last row must hold that dimension rounded up to 8 elements.  `partial`: bimamba2_gemm_workspace_bytes()
+ * bytes.  The reference has torch linear layers there (src/ssd/modules.py:63-64, :115-116).
+ * ------------------------------------------------------------------------------------------------------- */
+typedef struct bimamba2_gemm_params {
+    int32_t m, n, k;
+    int32_t dtype;              /* BIMAMBA2_BF16 or BIMAMBA2_F16: a, b, bias, c */
+    int32_t a_kcontig, b_kcontig;
+    int64_t lda, ldb, ldc;      /* elements */
+    const void *a, *b, *bias;   /* bias (n) or NULL */
+    void *c;
+    float *partial;
+    size_t partial_bytes;
+    void *stream;               /* hipStream_t */
+} bimamba2_gemm_params;
+size_t bimamba2_gemm_params_size(void);
+size_t bimamba2_gemm_workspace_bytes(const bimamba2_gemm_params *p);
+int bimamba2_gemm(const bimamba2_gemm_params *p);
+
 #ifdef __cplusplus
 }
 #endif
