@@ -579,7 +579,7 @@ static int check_gemm(const bimamba2_gemm_params *p) {
     if ((p->a_kcontig ? 256 : (int64_t)p->k) * p->lda * 2 + 2 * (int64_t)p->k >= 2 * most) return BIMAMBA2_EUNSUPPORTED;
     if ((p->b_kcontig ? 256 : (int64_t)p->k) * p->ldb * 2 + 2 * (int64_t)p->k >= 2 * most) return BIMAMBA2_EUNSUPPORTED;
     if (!p->a_kcontig && p->b_kcontig) return BIMAMBA2_EUNSUPPORTED;
-    if (p->b_kcontig && p->k % 8) return BIMAMBA2_EUNSUPPORTED;   // what lies behind a row of B is multiplied by zero: it must be numbers
+    if (p->b_kcontig && p->k % 8) return BIMAMBA2_EUNSUPPORTED;   // (no caller has such rows of B)
     return BIMAMBA2_OK;
 }
 

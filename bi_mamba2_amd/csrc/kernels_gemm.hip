@@ -68,7 +68,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const bimamba2_gemm_
     const int mvalid = p.m - m0, nvalid = p.n - n0;
 
     // one request: unit u (1 KB) of an operand tile, step it.  k contiguous: 16 rows x 64 bytes; else 8 k x 128 bytes of a
-    // 64-column block.  Rows, columns and k outside the matrix read a valid neighbour (the k of the A side is masked later).
+    // 64-column block.  Rows, columns and k outside the matrix read a valid neighbour (k is masked later, in the fragments).
     auto request = [&](auto KC, const char *base, unsigned ld, int valid, int u, int it, unsigned char *dst) __attribute__((always_inline)) {
         if constexpr (decltype(KC)::value) {
             const int row = u * 16 + (lane >> 2), chunk = (lane & 3) ^ ((row >> 2) & 3);
@@ -163,7 +163,8 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const bimamba2_gemm_
         for (int j = 0; j < (BKC ? 0 : NT); ++j) { raw_lds_use(f.bl[j]); raw_lds_use(f.bh[j]); }
     };
     f32x4 acc[MT][NT] = {};
-    // the last step of a k that is no multiple of 32: the A side's elements behind the end become zero
+    // the last step of a k that is no multiple of 32: the elements behind the end become zero on both sides (what the loads
+    // found there may be an infinity, or no number at all)
     auto mask_tail = [&](Frags &f) __attribute__((always_inline)) {
         typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
         typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -175,6 +176,13 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const bimamba2_gemm_
         for (int j = 0; j < (AKC ? 0 : MT); ++j) {
             f.al[j] = __builtin_bit_cast(i16x4, __builtin_bit_cast(u32x2, f.al[j]) & u32x2{msk[0], msk[1]});
             f.ah[j] = __builtin_bit_cast(i16x4, __builtin_bit_cast(u32x2, f.ah[j]) & u32x2{msk[2], msk[3]});
+        }
+#pragma unroll
+        for (int j = 0; j < (BKC ? NT : 0); ++j) f.b[j] = __builtin_bit_cast(Frag, __builtin_bit_cast(u32x4, f.b[j]) & msk);
+#pragma unroll
+        for (int j = 0; j < (BKC ? 0 : NT); ++j) {
+            f.bl[j] = __builtin_bit_cast(i16x4, __builtin_bit_cast(u32x2, f.bl[j]) & u32x2{msk[0], msk[1]});
+            f.bh[j] = __builtin_bit_cast(i16x4, __builtin_bit_cast(u32x2, f.bh[j]) & u32x2{msk[2], msk[3]});
         }
     };
     auto multiply = [&](Frags &f) __attribute__((always_inline)) {

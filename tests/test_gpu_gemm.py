@@ -50,6 +50,23 @@ def test_product(m, n, k, a_kc, b_kc, dtype):
     assert (got - want).abs().max() <= (8e-3 if dtype == torch.bfloat16 else 1e-3) * want.abs().max()
 
 
+@pytest.mark.parametrize("b_kc", [1, 0])
+def test_infinities_in_the_last_step(b_kc):
+    """what the loads find behind a k that is no multiple of a step takes no part, infinities included"""
+    m, n, k = 70, 66, 40
+    a = torch.ones(m, k, device="cuda", dtype=torch.bfloat16)
+    b = torch.ones(n, k, device="cuda", dtype=torch.bfloat16)
+    b[3, 36], b[5, k - 1] = float("inf"), float("-inf")
+    rows = b if b_kc else torch.cat([b.t(), b.new_zeros(k, 6)], 1)
+    c = torch.empty(m, 72, device="cuda", dtype=torch.bfloat16)
+    lib, p = _lib.load(), _lib.GemmParams()
+    p.m, p.n, p.k, p.a_kcontig, p.b_kcontig, p.dtype = m, n, k, 1, b_kc, _lib.BF16
+    p.lda, p.ldb, p.ldc = k, rows.stride(0), 72
+    p.a, p.b, p.c, p.stream = a.data_ptr(), rows.data_ptr(), c.data_ptr(), torch.cuda.current_stream().cuda_stream
+    assert lib.bimamba2_gemm_workspace_bytes(ctypes.byref(p)) == 0 and lib.bimamba2_gemm(ctypes.byref(p)) == 0
+    assert torch.equal(c[:, :n], (a.float() @ b.float().t()).bfloat16())
+
+
 def test_rejects():
     lib, p = _lib.load(), _lib.GemmParams()
     x = torch.zeros(64, 64, device="cuda", dtype=torch.bfloat16)
