@@ -10,6 +10,7 @@
 // module follows the library the Python side was told to use.
 #include <dlfcn.h>
 #include <torch/extension.h>
+#include <torch/csrc/Exceptions.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/hip/HIPGuard.h>
@@ -314,11 +315,19 @@ struct BoundaryCount {
         const int64_t nc = (p.seqlen + p.chunk_size - 1) / p.chunk_size;
         counts = at::empty({p.batch * nc}, at::TensorOptions().dtype(at::kInt).pinned_memory(true));
         check(api.seq_boundaries(&p, counts.mutable_data_ptr<int32_t>()), "bimamba2_seq_boundaries");
-        event = events.get(device);
-        TORCH_CHECK(hipEventRecord(event, static_cast<hipStream_t>(p.stream)) == hipSuccess, "hipEventRecord failed");
+        const hipEvent_t e = events.get(device);
+        TORCH_CHECK(hipEventRecord(e, static_cast<hipStream_t>(p.stream)) == hipSuccess, "hipEventRecord failed");
+        event = e;
+    }
+    BoundaryCount(const BoundaryCount &) = delete;
+    // (an exception between the launch and wait(): the pinned memory goes back only when the kernel has written it)
+    ~BoundaryCount() {
+        if (event) (void)hipEventSynchronize(event);
     }
     int64_t wait() {
-        TORCH_CHECK(hipEventSynchronize(event) == hipSuccess, "waiting for the count of sequence boundaries failed");
+        const hipEvent_t recorded = event;
+        event = nullptr;
+        TORCH_CHECK(hipEventSynchronize(recorded) == hipSuccess, "waiting for the count of sequence boundaries failed");
         const int32_t *c = counts.const_data_ptr<int32_t>();
         return counts.numel() ? *std::max_element(c, c + counts.numel()) : 0;
     }
@@ -386,7 +395,7 @@ public:
             dinit_b = device_empty(st, at::kFloat, q.x);
             p.dinitial_b = dinit_b.mutable_data_ptr<float>();
         }
-        Tensor kept = s[12];
+        Tensor kept = s[12].contiguous();
         Kept(p, o.copies).point(p, kept.mutable_data_ptr<float>());
         p.fwd_saved = 1;
         Tensor dz, dD, dbias, out_x = s[11];
@@ -419,10 +428,14 @@ public:
     }
 };
 
-inline bool wants_grad(std::initializer_list<const Tensor *> ts) {
-    if (!at::GradMode::is_enabled()) return false;
+// forward-mode tangents: the call goes through the autograd function whether or not gradients are enabled, which says that
+// there is no such derivative
+inline bool has_tangent(const Tensor &t) { return t.defined() && t._fw_grad(0).defined(); }
+
+inline bool wants_autograd(std::initializer_list<const Tensor *> ts) {
+    const bool grads = at::GradMode::is_enabled();
     for (const Tensor *t : ts)
-        if (t->defined() && t->requires_grad()) return true;
+        if ((grads && t->defined() && t->requires_grad()) || has_tangent(*t)) return true;
     return false;
 }
 
@@ -438,7 +451,7 @@ variable_list scan(const Tensor &x, const Tensor &dt, const Tensor &A, const Ten
     o->dt_max = dt_max;
     c10::OptionalDeviceGuard guard;
     if (x.is_cuda()) guard.reset_device(x.device());
-    if (wants_grad({&x, &dt, &A, &B, &C, &D_, &z_, &b_, &f_, &r_})) return ScanFn::apply(x, dt, A, B, C, D, z, bias, init_f, init_b, seq, o);
+    if (wants_autograd({&x, &dt, &A, &B, &C, &D_, &z_, &b_, &f_, &r_})) return ScanFn::apply(x, dt, A, B, C, D, z, bias, init_f, init_b, seq, o);
     at::AutoDispatchBelowADInplaceOrView below;
     ScanResult r = scan_checked([&](const ScanOpts &opts) { return Problem(x, dt, A, B, C, D_, z_, b_, f_, r_, undef(seq), opts); }, *o, false);
     if (!want_final) return {r.out};
@@ -452,6 +465,7 @@ struct LayerOpts : torch::CustomClassHolder {
     int64_t inner = 0, nheads = 0, headdim = 0, ngroups = 0, dstate = 0, chunk = 0, norm_group = 0;
     bool norm_before_gate = true;
     uint32_t needs = 0;           // bit i: input i of LayerFn takes a gradient
+    uint32_t converted = 0;       // bit i: the forward took small parameter i from its float32 copy
     bool copies = false;          // the forward kept the states in 16 bits
     double dt_min = 0, dt_max = 0, eps = 0;
 };
@@ -475,36 +489,42 @@ void add_cast(bimamba2_cast_params &c, const Tensor &src, void *dst, int dst_dty
     it.op = op;
 }
 
+// The parameters that need a float32 copy (bit i: parameter i; A = -exp(A_log) always is one).
+uint32_t params_to_convert(const std::array<Tensor, Params32::N> &prm) {
+    uint32_t mask = 0;
+    for (int i = 0; i < Params32::N; ++i)
+        if (prm[i].defined() && (i == 0 || prm[i].scalar_type() != at::kFloat || !prm[i].is_contiguous())) mask |= 1u << i;
+    return mask;
+}
+
 // offsets (in floats, 256-byte steps so that every piece is aligned for vector loads) of the pieces in Params32::buf; the
-// backward pass finds them again from the same parameters
-std::array<int64_t, Params32::N + 1> param_offsets(const std::array<Tensor, Params32::N> &prm) {
+// backward pass finds them again from the forward's mask
+std::array<int64_t, Params32::N + 1> param_offsets(const std::array<Tensor, Params32::N> &prm, uint32_t converted) {
     std::array<int64_t, Params32::N + 1> off{};
-    for (int i = 0; i < Params32::N; ++i) {
-        const bool converted = prm[i].defined() && (i == 0 || prm[i].scalar_type() != at::kFloat || !prm[i].is_contiguous());
-        off[i + 1] = off[i] + (converted ? (int64_t)round_up(prm[i].numel(), 64) : 0);
-    }
+    for (int i = 0; i < Params32::N; ++i) off[i + 1] = off[i] + (converted >> i & 1 ? (int64_t)round_up(prm[i].numel(), 64) : 0);
     return off;
 }
 
-Params32 point_params(const std::array<Tensor, Params32::N> &prm, const Tensor &buf) {
-    const auto off = param_offsets(prm);
+// (a parameter that is used as it is has to be contiguous; the caller holds it)
+Params32 point_params(const std::array<Tensor, Params32::N> &prm, uint32_t converted, const Tensor &buf) {
+    const auto off = param_offsets(prm, converted);
     Params32 r;
     r.buf = buf;
     float *base = buf.mutable_data_ptr<float>();
     for (int i = 0; i < Params32::N; ++i)
-        if (prm[i].defined()) r.ptr[i] = off[i + 1] > off[i] ? base + off[i] : prm[i].const_data_ptr<float>();
+        if (prm[i].defined()) r.ptr[i] = converted >> i & 1 ? base + off[i] : prm[i].const_data_ptr<float>();
     return r;
 }
 
-Params32 params_as_float32(std::array<Tensor, Params32::N> &prm, void *stream) {
-    const auto off = param_offsets(prm);
+Params32 params_as_float32(std::array<Tensor, Params32::N> &prm, uint32_t converted, void *stream) {
+    const auto off = param_offsets(prm, converted);
     const Tensor buf = device_empty({off.back()}, at::kFloat, prm[0]);
-    Params32 r = point_params(prm, buf);
+    Params32 r = point_params(prm, converted, buf);
     bimamba2_cast_params c{};
     c.stream = stream;
     std::array<Tensor, Params32::N> rows;
     for (int i = 0; i < Params32::N; ++i)
-        if (off[i + 1] > off[i]) {
+        if (converted >> i & 1) {
             rows[i] = prm[i].contiguous();
             add_cast(c, rows[i], const_cast<float *>(r.ptr[i]), BIMAMBA2_F32, i == 0 ? BIMAMBA2_CAST_NEG_EXP : BIMAMBA2_CAST_COPY);
         }
@@ -639,7 +659,7 @@ void product_tn(const Tensor &dy, const Tensor &x, Tensor c) {
 }
 
 struct LayerKept {
-    Tensor zx, xbc, y, yn, rstd, kept, prm32;
+    Tensor zx_rows, xbc, y, yn, rstd, kept, prm32;
 };
 
 Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, std::array<Tensor, Params32::N> prm, const Tensor &w_out,
@@ -647,9 +667,10 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
     const LayerShape s(u, prm[3], o);
     void *stream = stream_of(u);
     const Tensor u2 = u.reshape({s.rows, u.size(2)});
-    const Tensor zx = device_empty({s.rows, s.pitch}, u.scalar_type(), u).narrow(1, 0, s.proj);
+    const Tensor zx_rows = device_empty({s.rows, s.pitch}, u.scalar_type(), u), zx = zx_rows.narrow(1, 0, s.proj);
     product_nt(u2, w_in, b_in, zx);
-    const Params32 w = params_as_float32(prm, stream);
+    o.converted = params_to_convert(prm);
+    const Params32 w = params_as_float32(prm, o.converted, stream);
 
     const Tensor xbc = device_empty({s.rows, s.conv}, u.scalar_type(), u);
     bimamba2_conv_params c = conv_params(s, zx, w, stream);
@@ -681,7 +702,7 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
     check(api.norm_fwd(&n), "bimamba2_rmsnorm_gated_fwd");
     const Tensor out = device_empty({s.batch, s.seqlen, w_out.size(0)}, u.scalar_type(), u);
     product_nt(yn, w_out, b_out, out.view({s.rows, w_out.size(0)}));
-    if (left) *left = {zx, xbc, y, yn, rstd, kept, w.buf};
+    if (left) *left = {zx_rows, xbc, y, yn, rstd, kept, w.buf};
     return out;
 }
 
@@ -692,7 +713,7 @@ public:
                           const Tensor &w_out, const OptTensor &b_out, c10::intrusive_ptr<LayerOpts> o) {
         LayerKept k;
         const Tensor out = layer_forward(u, w_in, undef(b_in), {A_log, D, dt_bias, cw, undef(cb), nw}, w_out, undef(b_out), *o, true, &k);
-        ctx->save_for_backward({u, w_in, A_log, D, dt_bias, cw, undef(cb), nw, w_out, k.zx, k.xbc, k.y, k.yn, k.rstd, k.kept, k.prm32});
+        ctx->save_for_backward({u, w_in, A_log, D, dt_bias, cw, undef(cb), nw, w_out, k.zx_rows, k.xbc, k.y, k.yn, k.rstd, k.kept, k.prm32});
         ctx->saved_data["opts"] = c10::IValue::make_capsule(o);
         return out;
     }
@@ -705,14 +726,19 @@ public:
         const auto capsule = ctx->saved_data["opts"].toCapsule();
         const LayerOpts &o = *static_cast<const LayerOpts *>(capsule.get());
         auto needs = [&](int i) { return (o.needs >> i & 1) != 0; };
-        const Tensor &u = v[0], &w_in = v[1], &w_out = v[8], &zx = v[9], &xbc = v[10], &y = v[11], &yn = v[12], &rstd = v[13];
-        Tensor kept = v[14];
-        const std::array<Tensor, Params32::N> prm = {v[2], v[3], v[4], v[5], v[6], v[7]};
+        const Tensor &u = v[0], &w_in = v[1], &w_out = v[8];
+        // (a saved-tensor hook may hand back another layout than it was given: zx is kept with its padding columns, so that
+        // contiguous is the layout the kernels were told)
+        const Tensor zx = v[9].contiguous(), xbc = v[10].contiguous(), y = v[11].contiguous(), yn = v[12].contiguous(),
+                     rstd = v[13].contiguous(), kept = v[14].contiguous(), prm32 = v[15].contiguous();
+        std::array<Tensor, Params32::N> prm = {v[2], v[3], v[4], v[5], v[6], v[7]};
+        for (int i = 0; i < Params32::N; ++i)
+            if (prm[i].defined() && !(o.converted >> i & 1)) prm[i] = prm[i].contiguous();
         const c10::DeviceGuard guard(u.device());
         void *stream = stream_of(u);
         at::AutoDispatchBelowADInplaceOrView below;
         const LayerShape s(u, prm[3], o);
-        const Params32 w = point_params(prm, v[15]);
+        const Params32 w = point_params(prm, o.converted, prm32);
         const Tensor dout = as_type(grads[0], u.scalar_type()).reshape({s.rows, w_out.size(0)});
         Tensor dw_in, db_in, dw_out, db_out, du;
         if (needs(9)) product_tn(dout, yn, dw_out = device_empty(w_out.sizes(), u.scalar_type(), u));
@@ -797,7 +823,31 @@ public:
     }
 };
 
-Tensor layer(const Tensor &u, const Tensor &w_in, const OptTensor &b_in, const Tensor &A_log, const Tensor &D, const Tensor &dt_bias,
+// Whether the layer's tensors have the shapes, the device and the types that its kernels are told; what does not (a parameter
+// that was replaced, an input of another width, no rows at all) is left to the composition of the operators, whose own checks
+// say what is wrong with it.
+bool layer_fits(const Tensor &u, const Tensor &w_in, const Tensor &b_in, const std::array<Tensor, Params32::N> &prm, const Tensor &w_out,
+                const Tensor &b_out, const LayerOpts &o) {
+    if (u.dim() != 3 || u.numel() == 0 || w_in.dim() != 2 || w_out.dim() != 2 || w_out.numel() == 0) return false;
+    if (o.headdim <= 0 || o.ngroups <= 0 || o.nheads * o.headdim != o.inner || o.nheads % o.ngroups || o.norm_group <= 0 || o.inner % o.norm_group)
+        return false;
+    const int64_t conv = o.inner + 2 * o.ngroups * o.dstate;
+    auto is = [](const Tensor &t, at::IntArrayRef sizes) { return !t.defined() || t.sizes() == sizes; };
+    if (!is(w_in, {o.inner + conv + o.nheads, u.size(2)}) || !is(b_in, {w_in.size(0)}) || !is(b_out, {w_out.size(0)})) return false;
+    for (int i = 0; i < 3; ++i)
+        if (!is(prm[i], {o.nheads})) return false;
+    const Tensor &cw = prm[3];
+    if (cw.dim() != 3 || cw.size(0) != conv || cw.size(1) != 1 || !is(prm[4], {conv}) || !is(prm[5], {o.inner})) return false;
+    for (const Tensor *t : {&w_in, &b_in, &w_out, &b_out})
+        if (t->defined() && t->scalar_type() != u.scalar_type()) return false;
+    auto here = [&](const Tensor &t) { return !t.defined() || (t.device() == u.device() && t.layout() == at::kStrided); };
+    for (const Tensor *t : {&u, &w_in, &b_in, &w_out, &b_out})
+        if (!here(*t)) return false;
+    return std::all_of(prm.begin(), prm.end(), here);
+}
+
+// nullopt: see layer_fits
+OptTensor layer(const Tensor &u, const Tensor &w_in, const OptTensor &b_in, const Tensor &A_log, const Tensor &D, const Tensor &dt_bias,
              const Tensor &cw, const OptTensor &cb, const Tensor &nw, const Tensor &w_out, const OptTensor &b_out, int64_t headdim,
              int64_t ngroups, int64_t dstate, int64_t chunk, double dt_min, double dt_max, double eps, int64_t norm_group, bool norm_before_gate) {
     auto o = c10::make_intrusive<LayerOpts>();
@@ -812,14 +862,17 @@ Tensor layer(const Tensor &u, const Tensor &w_in, const OptTensor &b_in, const T
     o->eps = eps;
     o->norm_group = norm_group;
     o->norm_before_gate = norm_before_gate;
-    const c10::DeviceGuard guard(u.device());
     const Tensor bi = undef(b_in), bc = undef(cb), bo = undef(b_out);
+    if (!layer_fits(u, w_in, bi, {A_log, D, dt_bias, cw, bc, nw}, w_out, bo, *o)) return std::nullopt;
+    const c10::DeviceGuard guard(u.device());
+    bool tangents = false;
     int i = 0;
     for (const Tensor *t : {&u, &w_in, &bi, &A_log, &D, &dt_bias, &cw, &bc, &nw, &w_out, &bo}) {
         if (at::GradMode::is_enabled() && t->defined() && t->requires_grad()) o->needs |= 1u << i;
+        tangents |= has_tangent(*t);
         ++i;
     }
-    if (o->needs)
+    if (o->needs || tangents)
         return LayerFn::apply(u, w_in, b_in, A_log, D, dt_bias, cw, cb, nw, w_out, b_out, o);
     at::AutoDispatchBelowADInplaceOrView below;
     return layer_forward(u, w_in, bi, {A_log, D, dt_bias, cw, bc, nw}, w_out, bo, *o, false, nullptr);
@@ -833,6 +886,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
             if (e) std::rethrow_exception(e);
         } catch (const AssertionFailure &f) {
             PyErr_SetString(PyExc_AssertionError, f.what());
+        } catch (python_error &f) {              // raised by a saved-tensor hook: the hook's own exception goes on
+            f.restore();
         }
     });
     m.def("load", &load);

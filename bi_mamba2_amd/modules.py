@@ -196,9 +196,11 @@ class BiMamba2(nn.Module):
         """The layer's parameters if forward() may run as ONE native autograd function (csrc/host.cpp: the two GEMMs and this
         library's kernels, no Python between them), else None.  It may for what the kernels take in one piece, where nobody
         expects the projections to be called as modules, or the gradients' pieces as separate tensors
-        (_GradPieces.on_copied): no hooks, no replaced or patched projections, no autocast."""
+        (_GradPieces.on_copied): no hooks, no replaced or patched projections, no autocast, no tracing (a trace records the
+        composition's operators and autograd functions)."""
         if not (u.is_cuda and u.dim() == 3 and u.dtype in _DT and self.headdim <= MAX_HEADDIM and self.d_state <= MAX_DSTATE
-                and self.chunk_size >= 32) or _GradPieces.on_copied is not None or torch.is_autocast_enabled("cuda"):
+                and self.chunk_size >= 32) or _GradPieces.on_copied is not None or torch.is_autocast_enabled("cuda") \
+                or torch._C._get_tracing_state() is not None:
             return None
         m = torch.nn.modules.module
         if m._global_forward_hooks or m._global_forward_pre_hooks or m._global_backward_hooks or m._global_backward_pre_hooks:
@@ -225,9 +227,11 @@ class BiMamba2(nn.Module):
         tensors = self._native_tensors(u)
         if tensors is not None:
             norm = self._modules["norm"]
-            return _lib.host().layer(u, *tensors, self.headdim, self.ngroups, self.d_state, min(self.chunk_size, MAX_CHUNK_SIZE),
-                                     self.dt_limit[0], self.dt_limit[1], norm.eps, norm.group_size or self.d_inner,
-                                     norm.norm_before_gate)
+            out = _lib.host().layer(u, *tensors, self.headdim, self.ngroups, self.d_state, min(self.chunk_size, MAX_CHUNK_SIZE),
+                                    self.dt_limit[0], self.dt_limit[1], norm.eps, norm.group_size or self.d_inner,
+                                    norm.norm_before_gate)
+            if out is not None:          # (None: shapes or devices that do not belong together)
+                return out
         bc = self.ngroups * self.d_state
         zxbcdt = self.in_proj(u)
         prm = (self.A_log, self.D, self.dt_bias, self.conv1d.weight, self.conv1d.bias, self.norm.weight)

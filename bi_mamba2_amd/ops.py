@@ -845,7 +845,8 @@ def bimamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_b
     # The result does not depend on the chunk size (it only sets where the kernels cut the sequence), and the kernels'
     # chunks hold at most 256 positions: a larger chunk_size, which the reference accepts, runs with 256.
     chunk_size = min(chunk_size, MAX_CHUNK_SIZE)
-    if grad_places is None and KEEP_FORWARD_INTERMEDIATES and x.shape[-1] <= MAX_HEADDIM and B.shape[-1] <= MAX_DSTATE:
+    if grad_places is None and KEEP_FORWARD_INTERMEDIATES and x.shape[-1] <= MAX_HEADDIM and B.shape[-1] <= MAX_DSTATE \
+            and torch._C._get_tracing_state() is None:         # (a trace records the Python autograd function)
         # what the kernels take in one piece: checks, memory, launches and autograd in native code (csrc/host.cpp), the choice
         # of the chunk size for packed sequences included
         res = _lib.host().scan(x, dt, A, B, C, chunk_size, D, z, dt_bias, dt_softplus, dt_limit[0], dt_limit[1],
@@ -902,7 +903,7 @@ def bimamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_b
         if not return_final_states:
             return out
         return out, torch.cat([f[0] for f in fins], dim=-1), torch.cat([f[1] for f in fins], dim=-1)
-    # gradients into places of the caller's, or KEEP_FORWARD_INTERMEDIATES off
+    # gradients into places of the caller's, KEEP_FORWARD_INTERMEDIATES off, or a trace
     return MambaChunkScanCombinedFn.apply(x, dt, A, B, C, chunk_size, D, z, dt_bias, dt_softplus, dt_limit,
                                           return_final_states, initial_states_f, initial_states_b, seq_idx, grad_places)
 

@@ -87,3 +87,58 @@ def test_gradient_views_that_break_the_alignment_are_copied():
         got = torch.autograd.grad(out, leaves, view, retain_graph=True)
         for a, b in zip(got, torch.autograd.grad(out, leaves, view.contiguous(), retain_graph=True)):
             assert torch.equal(a, b)
+
+
+def small_layer(**kw):
+    """a layer whose projection has 296 columns: no multiple of the 64 its rows are padded to"""
+    from bi_mamba2_amd.modules import BiMamba2
+    torch.manual_seed(0)
+    m = BiMamba2(d_model=64, d_state=16, headdim=16, chunk_size=64, **kw).cuda().to(torch.bfloat16)
+    u = torch.randn(2, 100, 64, device="cuda").to(torch.bfloat16).requires_grad_(True)
+    return m, u, [u] + [p for n, p in m.named_parameters() if n != "fc_D.weight"]
+
+
+def scan_of(d, leaves):
+    from bi_mamba2_amd import ops
+    return ops.bimamba_chunk_scan_combined(*leaves, 64, D=d["D"], z=d["z"], dt_bias=d["dt_bias"], dt_softplus=True)
+
+
+@pytest.mark.parametrize("how", ["layer", "scan"])
+def test_saved_tensor_hooks_and_checkpointing(how):
+    from torch.utils.checkpoint import checkpoint
+    if how == "layer":
+        m, u, leaves = small_layer()
+        fn = lambda: m(u)
+    else:
+        d = to_dev(make_case(2, 100, 4, 16, 2, 16, torch.bfloat16, with_z=True))
+        leaves = [d[k].clone().requires_grad_(True) for k in ("x", "dt", "A", "B", "C")]
+        fn = lambda: scan_of(d, leaves)
+    out = fn()
+    dy = torch.randn_like(out)
+    want = torch.autograd.grad(out, leaves, dy)
+    with torch.autograd.graph.save_on_cpu():
+        out = fn()
+    kept = torch.autograd.grad(out, leaves, dy)
+    for a, b, c in zip(want, kept, torch.autograd.grad(checkpoint(fn, use_reentrant=False), leaves, dy)):
+        assert torch.equal(a, b) and torch.equal(a, c)
+
+
+def test_forward_mode_is_refused():
+    import torch.autograd.forward_ad as fwAD
+    m, u, _ = small_layer()
+    d = to_dev(make_case(1, 64, 2, 16, 1, 16, torch.bfloat16, with_z=True))
+    with fwAD.dual_level(), torch.no_grad():
+        for call in (lambda: m(fwAD.make_dual(u.detach(), torch.ones_like(u))),
+                     lambda: scan_of(d, [fwAD.make_dual(d["x"], d["x"])] + [d[k] for k in ("dt", "A", "B", "C")])):
+            with pytest.raises((RuntimeError, NotImplementedError)):
+                call()
+
+
+def test_layer_parameters_of_other_shapes():
+    m, u, _ = small_layer()
+    with torch.no_grad():
+        want = m(u)
+        m.D = torch.nn.Parameter(m.D[:, None].expand(-1, 16).contiguous())          # one value a channel: the composition takes it
+        assert_close(m(u), want.double(), torch.bfloat16, "D per channel", scaled=True)
+        with pytest.raises(RuntimeError):
+            m(torch.zeros(2, 100, 72, device="cuda", dtype=torch.bfloat16))
