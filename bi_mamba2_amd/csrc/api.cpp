@@ -23,16 +23,6 @@ inline bool fwd_scan_rebuilds_cb(const bimamba2_params *p) {
     return chunk_scan_uses_scan16(p, false) && p->states16_f && (p->causal || p->states16_b);
 }
 
-// State dimension 128 in training: the states that enter the chunks are kept in float32 for the backward pass, and the scan
-// kernel, which rounds them to the input's type for its MFMA anyway, gets a 16-bit copy beside them: half the bytes for it, the
-// kernel with direct loads, no C.B^T launch, bit for bit the same operands of the state product.  bfloat16 only: that scan
-// kernel holds C.B^T in float16, three bits more than bfloat16 operands resolve but no more than float16 ones do.
-inline bool forward_adds_copies(const bimamba2_params *p) {
-    auto al16 = [](const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
-    return p->dtype == BIMAMBA2_BF16 && p->dstate == 128 && !p->causal && p->states_f && p->states_b && !p->states16_f &&
-           chunk_scan_uses_scan16(p, false) && al16(p->final_f) && al16(p->final_b) && al16(p->initial_f) && al16(p->initial_b);
-}
-
 int check_problem(const bimamba2_params *p) {
     if (!p) return BIMAMBA2_EINVAL;
     if (p->batch <= 0 || p->seqlen <= 0 || p->nheads <= 0 || p->headdim <= 0 || p->ngroups <= 0 || p->dstate <= 0)
@@ -93,7 +83,7 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     const bool fwd_only_copies = !is_bwd && !q->causal && (q->dtype == BIMAMBA2_BF16 || q->dtype == BIMAMBA2_F16) &&
                                  (q->headdim * q->dstate) % 4 == 0 && al16(q->final_f) && al16(q->final_b) &&
                                  al16(q->initial_f) && al16(q->initial_b) && !q->states_b && !q->states16_b;
-    const bool carve16 = ((copies || fwd_only_copies) && !q->states_f && !q->states16_f) || (!is_bwd && forward_adds_copies(q));
+    const bool carve16 = (copies || fwd_only_copies) && !q->states_f && !q->states16_f;
     // CB: read by the forward scan and by the dCB kernel unless they rebuild it; CB^T: by the dx kernel, likewise.  (The
     // forward scan kernel for state dimension 128 rebuilds it as well, and runs where the entering states travel as copies.)
     const bool fwd_scan16 = !is_bwd && chunk_scan_uses_scan16(q, false) && (carve16 || q->states16_f) && (q->causal || carve16 || q->states16_b);
@@ -383,8 +373,7 @@ int bimamba2_fwd(const bimamba2_params *p) {
     if (need > 256 && (!p->workspace || p->workspace_bytes < need)) return BIMAMBA2_EWORKSPACE;
     TRY(forward_cumsum_and_states(&q));
     if (q.CB) TRY(bimamba2_bmm_chunk_fwd(&q));     // given by the caller, or carved because the scan kernel reads it
-    if (q.states_f && q.states16_f && !p->states16_f) TRY(launch_state_passing_fwd(&q, true));   // forward_adds_copies()
-    else TRY(bimamba2_state_passing_fwd(&q));
+    TRY(bimamba2_state_passing_fwd(&q));
     if (scan_recomputes_cb(&q, false) || fwd_scan_rebuilds_cb(&q)) q.CB = nullptr;
     TRY(bimamba2_chunk_scan_fwd(&q));
     return BIMAMBA2_OK;
@@ -424,7 +413,9 @@ int bimamba2_bwd(const bimamba2_params *p) {
     // merged ones (their reader rounds them to that type for its MFMA anyway)
     const bool dcb16 = !p->dCB && !p->dCBT && bwd_dcb_sp_merged(&q) && bwd_tail_merged(&q);
     const bool need_cbt = !scan_recomputes_cb(&q, true), need_cb = need_cbt || !dcb_recomputes_cb(&q);
-    if (need_cb) TRY(bimamba2_bmm_chunk_fwd(&q));  // CB for the dCB kernel, CB^T for the dx kernel, unless they rebuild it
+    const bool saved_cb = (p->fwd_saved & 2) && p->CB && p->CBT;
+    if (need_cb && saved_cb) {}                    // left there by the forward pass
+    else if (need_cb) TRY(bimamba2_bmm_chunk_fwd(&q));  // CB for the dCB kernel, CB^T for the dx kernel, unless they rebuild it
     else q.CB = nullptr;
     // dz and dstates as one launch where the kernel for it exists (dout_x goes from the first to the second inside the workgroup)
     const bool dz_dstates = q.has_z && bwd_dz_dstates_fused(&q);

@@ -44,6 +44,7 @@ struct Api {
     decltype(&bimamba2_bwd) bwd = nullptr;
     decltype(&bimamba2_workspace_bytes) workspace_bytes = nullptr;
     decltype(&bimamba2_state_copies) state_copies = nullptr;
+    decltype(&bimamba2_chunk_scan_reads_cb) reads_cb = nullptr;
     decltype(&bimamba2_seq_boundaries) seq_boundaries = nullptr;
     decltype(&bimamba2_strerror) strerror = nullptr;
     decltype(&bimamba2_rmsnorm_gated_fwd) norm_fwd = nullptr;
@@ -78,6 +79,7 @@ void load(const std::string &path) {
     get(api.bwd, "bimamba2_bwd");
     get(api.workspace_bytes, "bimamba2_workspace_bytes");
     get(api.state_copies, "bimamba2_state_copies");
+    get(api.reads_cb, "bimamba2_chunk_scan_reads_cb");
     get(api.seq_boundaries, "bimamba2_seq_boundaries");
     get(api.strerror, "bimamba2_strerror");
     get(api.norm_fwd, "bimamba2_rmsnorm_gated_fwd");
@@ -134,6 +136,7 @@ struct ScanOpts : torch::CustomClassHolder {
     int64_t chunk = 0;
     bool dt_softplus = false, want_final = false;
     bool copies = false;          // the forward kept the states in 16 bits
+    bool cb = false;              // the forward kept C.B^T
     double dt_min = 0, dt_max = 0;
 };
 
@@ -224,18 +227,29 @@ struct Problem {
     }
 };
 
-// What the forward pass leaves for the backward pass besides its operands, in one float32 allocation: dt_out, cs_f, cs_b and
-// the states entering the chunks (copies: in the operands' 16-bit type, where the kernels can keep them that way).
+// Whether the forward pass keeps C.B^T and its transpose for the backward pass: where the backward's kernels read them and
+// they take no more memory than x, or little (64 MiB).  It forms the product for itself there; the backward's launch for both
+// took 9 to 13 us (float32 with 16 heads in 2 groups over 2 x 1111 positions, bfloat16 at state dimension 128 over 2 x 3001).
+bool keeps_cb(const bimamba2_params &p) {
+    const size_t nc = (p.seqlen + p.chunk_size - 1) / p.chunk_size, e = p.dtype == BIMAMBA2_F32 ? 4 : 2;
+    const size_t bytes = 8 * (size_t)p.batch * nc * p.ngroups * p.chunk_size * p.chunk_size;
+    return api.reads_cb(&p, 0) && api.reads_cb(&p, 1) && bytes <= std::max(e * p.batch * p.seqlen * p.nheads * p.headdim, size_t(64) << 20);
+}
+
+// What the forward pass leaves for the backward pass besides its operands, in one float32 allocation: dt_out, cs_f, cs_b, the
+// states entering the chunks (copies: in the operands' 16-bit type, where the kernels can keep them that way) and, with cb,
+// C.B^T and its transpose.
 struct Kept {
-    size_t n1 = 0, ns = 0;
+    size_t n1 = 0, ns = 0, ncb = 0;
     bool copies = false;
-    Kept(const bimamba2_params &p, bool copies_) : copies(copies_) {
+    Kept(const bimamba2_params &p, bool copies_, bool cb) : copies(copies_) {
         const size_t nc = (p.seqlen + p.chunk_size - 1) / p.chunk_size;
         n1 = round_up((size_t)p.batch * p.nheads * nc * p.chunk_size, 64);
         ns = round_up((size_t)p.batch * nc * p.nheads * p.headdim * p.dstate, 64);
         if (copies) ns /= 2;
+        if (cb) ncb = round_up((size_t)p.batch * nc * p.ngroups * p.chunk_size * p.chunk_size, 64);
     }
-    int64_t floats() const { return (int64_t)(3 * n1 + 2 * ns); }
+    int64_t floats() const { return (int64_t)(3 * n1 + 2 * ns + 2 * ncb); }
     void point(bimamba2_params &p, float *base) const {
         p.dt_out = base;
         p.cs_f = base + n1;
@@ -248,7 +262,13 @@ struct Kept {
             p.states_f = st;
             p.states_b = st + ns;
         }
+        if (ncb) {
+            p.CB = st + 2 * ns;
+            p.CBT = p.CB + ncb;
+        }
     }
+    // what bimamba2_bwd is told about these
+    int saved() const { return ncb ? 3 : 1; }
 };
 
 Tensor attach_workspace(bimamba2_params &p, bool bwd, const Tensor &like) {
@@ -267,7 +287,8 @@ ScanResult scan_forward(Problem &q, ScanOpts &o, bool keep) {
     ScanResult r;
     if (keep) {
         o.copies = api.state_copies(&p) != 0;
-        const Kept k(p, o.copies);
+        o.cb = !o.copies && keeps_cb(p);
+        const Kept k(p, o.copies, o.cb);
         r.kept = device_empty({k.floats()}, at::kFloat, q.x);
         k.point(p, r.kept.mutable_data_ptr<float>());
     }
@@ -396,8 +417,9 @@ public:
             p.dinitial_b = dinit_b.mutable_data_ptr<float>();
         }
         Tensor kept = s[12].contiguous();
-        Kept(p, o.copies).point(p, kept.mutable_data_ptr<float>());
-        p.fwd_saved = 1;
+        const Kept k(p, o.copies, o.cb);
+        k.point(p, kept.mutable_data_ptr<float>());
+        p.fwd_saved = k.saved();
         Tensor dz, dD, dbias, out_x = s[11];
         if (p.has_z) {
             out_x = out_x.contiguous();
@@ -467,6 +489,7 @@ struct LayerOpts : torch::CustomClassHolder {
     uint32_t needs = 0;           // bit i: input i of LayerFn takes a gradient
     uint32_t converted = 0;       // bit i: the forward took small parameter i from its float32 copy
     bool copies = false;          // the forward kept the states in 16 bits
+    bool cb = false;              // the forward kept C.B^T
     double dt_min = 0, dt_max = 0, eps = 0;
 };
 
@@ -683,7 +706,8 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
     Tensor kept;
     if (keep) {
         o.copies = api.state_copies(&p) != 0;
-        const Kept k(p, o.copies);
+        o.cb = !o.copies && keeps_cb(p);
+        const Kept k(p, o.copies, o.cb);
         kept = device_empty({k.floats()}, at::kFloat, u);
         k.point(p, kept.mutable_data_ptr<float>());
     }
@@ -768,8 +792,9 @@ public:
         const Tensor dxbc = device_empty({s.rows, s.conv}, u.scalar_type(), u);
         {
             bimamba2_params p = layer_scan_params(s, o, zx, xbc, w, stream);
-            Kept(p, o.copies).point(p, kept.mutable_data_ptr<float>());
-            p.fwd_saved = 1;
+            const Kept k(p, o.copies, o.cb);
+            k.point(p, kept.mutable_data_ptr<float>());
+            p.fwd_saved = k.saved();
             p.dout = dy.const_data_ptr();
             p.dout_sb = s.seqlen * s.inner; p.dout_sl = s.inner; p.dout_sh = o.headdim;
             p.dx = at_byte(dxbc, 0);

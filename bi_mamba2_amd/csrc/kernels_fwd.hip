@@ -1143,9 +1143,8 @@ int launch_bwd_dz_dstates(const bimamba2_params *p) {
 // together, unconditionally (past the last chunk a valid chunk is read again and not used).  Needs P*N % 4 == 0 and
 // 16-byte aligned tensors.
 // ndir = 1: the forward recurrence only (blockIdx.z = b).
-// T16 != void: the entering states go to the 16-bit copies (states16_*) and the per-chunk states stay as they are; with BOTH
-// they are replaced by the float32 entering states as well.
-template <typename T16, bool BOTH = false>
+// T16 != void: the entering states go to the 16-bit copies (states16_*) and the per-chunk states stay as they are.
+template <typename T16>
 __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_vec_kernel(const bimamba2_params p, int nc, int ndir) {
     const int PN = p.headdim * p.dstate;
     const int e = (blockIdx.x * NTHREADS + threadIdx.x) * 4;
@@ -1181,8 +1180,7 @@ __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_vec_kernel(const b
 #pragma unroll
                     for (int k = 0; k < 4; ++k) o.v[k] = from_f<TC>(s[k]);
                     *reinterpret_cast<Out4 *>(st16 + c * cstride) = o;
-                }
-                if constexpr (!COPY || BOTH) {
+                } else {
                     *reinterpret_cast<f32x4 *>(st + c * cstride) = s;
                 }
                 s = __expf(d[i]) * s + v[i];
@@ -1242,7 +1240,7 @@ __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_inplace16_kernel(c
     }
 }
 
-int launch_state_passing_fwd(const bimamba2_params *p, bool both) {
+int launch_state_passing_fwd(const bimamba2_params *p) {
     const int nc = nchunks(p), PN = p->headdim * p->dstate;
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     const int ndir = p->causal ? 1 : 2;
@@ -1258,11 +1256,7 @@ int launch_state_passing_fwd(const bimamba2_params *p, bool both) {
         dim3 grid((PN / 4 + NTHREADS - 1) / NTHREADS, p->nheads, p->batch * ndir);
         if (p->states16_f) {
             if (!(p->causal || p->states16_b) || !al(p->states16_f) || !al(p->states16_b)) return BIMAMBA2_EINVAL;
-            if (both) {
-                if (p->dtype == BIMAMBA2_BF16) hipLaunchKernelGGL((state_passing_fwd_vec_kernel<bf16_t, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
-                else if (p->dtype == BIMAMBA2_F16) hipLaunchKernelGGL((state_passing_fwd_vec_kernel<f16_t, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
-                else return BIMAMBA2_EUNSUPPORTED;
-            } else if (p->dtype == BIMAMBA2_BF16) hipLaunchKernelGGL(state_passing_fwd_vec_kernel<bf16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
+            if (p->dtype == BIMAMBA2_BF16) hipLaunchKernelGGL(state_passing_fwd_vec_kernel<bf16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
             else if (p->dtype == BIMAMBA2_F16) hipLaunchKernelGGL(state_passing_fwd_vec_kernel<f16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, ndir);
             else return BIMAMBA2_EUNSUPPORTED;
         } else {
@@ -1270,7 +1264,7 @@ int launch_state_passing_fwd(const bimamba2_params *p, bool both) {
         }
         return check_launch();
     }
-    if (p->states16_f) return BIMAMBA2_EUNSUPPORTED;     // (so that `both` is never dropped)
+    if (p->states16_f) return BIMAMBA2_EUNSUPPORTED;
     if (p->causal) return BIMAMBA2_EUNSUPPORTED;
     dim3 grid((PN + NTHREADS - 1) / NTHREADS, p->nheads, p->batch);
     hipLaunchKernelGGL(state_passing_fwd_kernel, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc);

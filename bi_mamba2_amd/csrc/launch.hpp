@@ -29,8 +29,7 @@ bool chunk_states_in_16bit(const bimamba2_params *p);
 // the chunk-state kernel whose workgroups walk through several heads of one (batch, chunk): where it is used, and its launch
 bool chunk_state_uses_heads_kernel(const bimamba2_params *p);
 int launch_chunk_state_heads(const bimamba2_params *p);
-// both: the entering states in float32 (in place of the per-chunk states) and in the 16-bit copies
-int launch_state_passing_fwd(const bimamba2_params *p, bool both = false);
+int launch_state_passing_fwd(const bimamba2_params *p);
 int launch_chunk_scan(const bimamba2_params *p, bool bwd);
 // the 16-bit kernel of kernels_scan16.hip (launch_chunk_scan picks it where it applies)
 int launch_chunk_scan16(const bimamba2_params *p, bool bwd);

@@ -65,7 +65,8 @@ typedef struct bimamba2_params {
     int32_t dt_dtype;       /* BIMAMBA2_* : dt and ddt */
     int32_t has_D, D_has_hdim, has_z, has_dt_bias, dt_softplus;
     int32_t fwd_saved;      /* bimamba2_bwd only: dt_out, cs_f, cs_b, states_f, states_b hold what bimamba2_fwd left in
-                               them, so the backward pass does not recompute them (CB is always recomputed) */
+                               them, so the backward pass does not recompute them.  3: CB and CBT hold what it left there too
+                               (1: they are recomputed where a kernel reads them) */
     int32_t causal;         /* 0: the bidirectional operator.  1: the single-direction (causal) operator built from the same
                                kernels with the reverse direction left out - the comparator the bidirectional pass is
                                timed against.  Every entry point follows it, but only for the shapes whose scan
@@ -230,7 +231,7 @@ int bimamba2_fwd_static(const bimamba2_params *p);
 /* Whole backward; replaces _mamba_chunk_scan_combined_bwd (src/ssd/bi/ssd_combined.py:334-475).
  * Needs: the forward inputs, dout, out_x (pre-gate output, when has_z), dx ddt dA dB dC [dD dz ddt_bias],
  * workspace.  With fwd_saved = 0 it recomputes the forward intermediates as the reference does; with
- * fwd_saved = 1 it reads them from the five pointers named at that flag. */
+ * fwd_saved = 1 it reads them from the five pointers named at that flag (3: from seven). */
 int bimamba2_bwd(const bimamba2_params *p);
 
 /* ---- single stages (each is also what the composites run) ------------------------------------------ */

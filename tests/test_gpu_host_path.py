@@ -142,3 +142,20 @@ def test_layer_parameters_of_other_shapes():
         assert_close(m(u), want.double(), torch.bfloat16, "D per channel", scaled=True)
         with pytest.raises(RuntimeError):
             m(torch.zeros(2, 100, 72, device="cuda", dtype=torch.bfloat16))
+
+
+def test_cb_kept_or_formed_again():
+    """C.B^T of one row of 2304 positions and 8 groups (38 MB with its transpose) is kept for the backward pass, that of two rows
+    is formed again there: the gradients of a row are the same, bit for bit"""
+    d = to_dev(make_case(2, 2304, 8, 16, 8, 16, torch.bfloat16, with_z=True))
+    from bi_mamba2_amd import ops
+    dy = torch.randn_like(d["x"])
+
+    def grads(rows):
+        leaves = [d[k][rows].clone().requires_grad_(True) for k in ("x", "dt", "B", "C", "z")]
+        x, dt, B, C, z = leaves
+        out = ops.bimamba_chunk_scan_combined(x, dt, d["A"], B, C, 256, D=d["D"], z=z, dt_bias=d["dt_bias"], dt_softplus=True)
+        return (out.detach(),) + torch.autograd.grad(out, leaves, dy[rows])
+
+    for both, one in zip(grads(slice(0, 2)), grads(slice(1, 2))):
+        assert torch.equal(both[1:], one)
