@@ -14,6 +14,8 @@
 // dweight[c, k] = sum_{b, l} g[l] * x[l + k - W/2];  dbias[c] = sum g.  A second rotating window holds g.  Each thread
 // leaves its dweight / dbias partial sums (over its own positions) in the workspace, [tile][channel][W + 1], and a
 // column-parallel fixed-order sum adds the tiles up (no atomics).
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 
@@ -27,6 +29,29 @@ template <typename T, int VS> struct alignas(sizeof(T) * VS) ConvVec {
 
 template <typename T, int VS> __device__ __forceinline__ ConvVec<T, VS> conv_load(const T *p) {
     return *reinterpret_cast<const ConvVec<T, VS> *>(p);
+}
+
+// VS elements as they travel: one register of packed 16-bit values (a struct of two is loaded in halves, a register each)
+template <int BYTES> struct ConvRawOf;
+template <> struct ConvRawOf<2> { typedef unsigned short Type; };
+template <> struct ConvRawOf<4> { typedef unsigned Type; };
+template <> struct ConvRawOf<8> { typedef unsigned Type __attribute__((ext_vector_type(2))); };
+template <typename T, int VS> using ConvRaw = typename ConvRawOf<sizeof(T) * VS>::Type;
+
+// a row's scalar address plus the lane's byte offset
+template <typename R> __device__ __forceinline__ R conv_row_load(const char *row, unsigned off) {
+    return *reinterpret_cast<const __attribute__((address_space(1))) R *>(reinterpret_cast<uintptr_t>(uniform_ptr(row)) + off);
+}
+template <typename R> __device__ __forceinline__ void conv_row_store(const char *row, unsigned off, R v) {
+    *reinterpret_cast<__attribute__((address_space(1))) R *>(reinterpret_cast<uintptr_t>(uniform_ptr(row)) + off) = v;
+}
+
+// f(integral_constant<int, 0>) .. f(integral_constant<int, N - 1>)
+template <int N, int I = 0, class F> __device__ __forceinline__ void conv_steps(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>());
+        conv_steps<N, I + 1>(f);
+    }
 }
 
 }  // namespace
@@ -154,17 +179,24 @@ __global__ __launch_bounds__(NTHREADS) void conv1d_silu_fwd_tiled_kernel(const b
 }
 
 // Steps t = 0 .. TL + 2H - 1 visit positions l = l0 - H + t: g[l] is formed (needs x[l - H .. l + H]) and dx[l - H] leaves.
+//
+// Bound by instruction issue: 21 multiply-adds and a sigmoid per element against 6 bytes.  So the unit of work is a wave, 64
+// runs of VS channels over one tile of positions (nwc waves side by side): positions, row addresses and the edge conditions
+// are scalar, a row costs no vector instruction, and the filter widths that lie inside the tile and the sequence run without
+// masks.  16 x 1024 positions x 1664 channels in bfloat16: 64 -> 51 us (59 with tiles of 56 positions).
 template <typename T, int W, int VS>
-__global__ __launch_bounds__(NTHREADS) void conv1d_silu_bwd_kernel(const bimamba2_conv_params p, int ntl, int TL, float *part) {
+__global__ __launch_bounds__(NTHREADS) void conv1d_silu_bwd_kernel(const bimamba2_conv_params p, int ntl, int TL, int nwc, float *part) {
     constexpr int H = W / 2;
+    typedef ConvRaw<T, VS> Raw;
+    typedef ConvVec<T, VS> Vec;
     const int CV = p.channels / VS;
-    const int64_t id = (int64_t)blockIdx.x * NTHREADS + threadIdx.x;
-    const int cv = (int)(id % CV);
-    const int64_t tile = id / CV;
+    const int lane = threadIdx.x & 63, wid = blockIdx.x * (NTHREADS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // (readfirstlane: a division's result lives in a vector register, and every address formed from it would too)
+    const int tile = __builtin_amdgcn_readfirstlane(wid / nwc), cv = (wid - tile * nwc) * 64 + lane;
     if (tile >= p.batch * ntl) return;
-    const int lt = (int)(tile % ntl);
-    const int64_t b = tile / ntl;
-    const int L = (int)p.seqlen, c0 = cv * VS, l0 = lt * TL, l1 = min(l0 + TL, L);
+    const int b = __builtin_amdgcn_readfirstlane(tile / ntl), lt = tile - b * ntl;
+    const bool live = cv < CV;                        // (the others load what the last run loads and store nothing)
+    const int L = (int)p.seqlen, c0 = min(cv, CV - 1) * VS, l0 = lt * TL, l1 = min(l0 + TL, L);
     float w[W][VS], bias[VS];
 #pragma unroll
     for (int i = 0; i < VS; ++i) {
@@ -172,12 +204,15 @@ __global__ __launch_bounds__(NTHREADS) void conv1d_silu_bwd_kernel(const bimamba
 #pragma unroll
         for (int k = 0; k < W; ++k) w[k][i] = p.weight[(int64_t)(c0 + i) * W + k];
     }
-    const T *xin = reinterpret_cast<const T *>(p.x) + b * p.x_sb + c0;
-    const T *din = reinterpret_cast<const T *>(p.dout) + b * p.dout_sb + c0;
+    const unsigned co = (unsigned)(c0 * sizeof(T));   // a row's address is scalar, plus this
+    const char *xin = uniform_ptr(reinterpret_cast<const T *>(p.x) + b * p.x_sb);
+    const char *din = uniform_ptr(reinterpret_cast<const T *>(p.dout) + b * p.dout_sb);
+    const int64_t x_row = p.x_sl * (int64_t)sizeof(T), d_row = p.dout_sl * (int64_t)sizeof(T);
     const int64_t dx_sl = p.dx_sl ? p.dx_sl : p.channels, dx_sb = p.dx_sl ? p.dx_sb : p.seqlen * p.channels;
-    T *dx = reinterpret_cast<T *>(p.dx) + b * dx_sb + c0;
-    auto ldx = [&](int l) { return conv_load<T, VS>(xin + (int64_t)min(max(l, 0), L - 1) * p.x_sl); };
-    auto ldd = [&](int l) { return conv_load<T, VS>(din + (int64_t)min(max(l, 0), L - 1) * p.dout_sl); };
+    char *dx = const_cast<char *>(uniform_ptr(reinterpret_cast<T *>(p.dx) + b * dx_sb));
+    const int64_t dx_row = dx_sl * (int64_t)sizeof(T);
+    auto ldx = [&](int l) __attribute__((always_inline)) { return conv_row_load<Raw>(xin + min(max(l, 0), L - 1) * x_row, co); };
+    auto ldd = [&](int l) __attribute__((always_inline)) { return conv_row_load<Raw>(din + min(max(l, 0), L - 1) * d_row, co); };
     float xw[W][VS], gw[W][VS], dw[W][VS], db[VS];
 #pragma unroll
     for (int i = 0; i < VS; ++i) {
@@ -189,57 +224,57 @@ __global__ __launch_bounds__(NTHREADS) void conv1d_silu_bwd_kernel(const bimamba
 #pragma unroll
     for (int j = 0; j < W - 1; ++j) {
         const int l = lb - H + j;
-        const ConvVec<T, VS> r = ldx(l);
+        const Vec r = __builtin_bit_cast(Vec, ldx(l));
 #pragma unroll
         for (int i = 0; i < VS; ++i) xw[j][i] = (l >= 0 && l < L) ? to_f(r.v[i]) : 0.f;
     }
-    ConvVec<T, VS> nx[W], nd[W];
+    Raw nx[W], nd[W];
 #pragma unroll
     for (int u = 0; u < W; ++u) { nx[u] = ldx(lb + u + H); nd[u] = ldd(lb + u); }
     const int lend = l1 + H;                          // one past the last position visited
-    for (int s0 = lb; s0 < lend; s0 += W) {
-        ConvVec<T, VS> cx[W], cd[W];
+    // step u of the filter width that starts at s0; EDGE: at an end of the tile or of the sequence
+    auto step = [&](auto EDGE, auto U, int s0) __attribute__((always_inline)) {
+        constexpr bool E = decltype(EDGE)::value;
+        constexpr int u = decltype(U)::value;
+        const int l = s0 + u, j = l - H;              // dx[j] = sum_k w[k] g[l - k]
+        const bool xin_ok = l + H >= 0 && l + H < L, lin = l >= 0 && l < L, own = l >= l0 && l < l1;
+        const Vec cx = __builtin_bit_cast(Vec, nx[u]), cd = __builtin_bit_cast(Vec, nd[u]);
+        nx[u] = ldx(l + W + H);                       // needed a filter width later
+        nd[u] = ldd(l + W);
+        Vec o;
 #pragma unroll
-        for (int u = 0; u < W; ++u) { cx[u] = nx[u]; cd[u] = nd[u]; }
+        for (int i = 0; i < VS; ++i) {
+            const float xn = to_f(cx.v[i]);
+            xw[(u + W - 1) % W][i] = E ? (xin_ok ? xn : 0.f) : xn;
+            float a = bias[i];
 #pragma unroll
-        for (int u = 0; u < W; ++u) { nx[u] = ldx(s0 + W + u + H); nd[u] = ldd(s0 + W + u); }
+            for (int k = 0; k < W; ++k) a = __builtin_fmaf(w[k][i], xw[(u + k) % W][i], a);
+            const float sg = sigmoid_f(a);
+            float g = to_f(cd.v[i]) * sg * (1.f + a * (1.f - sg));
+            if (E && !lin) g = 0.f;
+            gw[u][i] = g;
+            if (!E || own) {
+                db[i] += g;
 #pragma unroll
-        for (int u = 0; u < W; ++u) {
-            const int l = s0 + u;
-            if (l < lend) {
-                const bool xin_ok = l + H >= 0 && l + H < L, lin = l >= 0 && l < L, own = l >= l0 && l < l1;
-#pragma unroll
-                for (int i = 0; i < VS; ++i) xw[(u + W - 1) % W][i] = xin_ok ? to_f(cx[u].v[i]) : 0.f;
-#pragma unroll
-                for (int i = 0; i < VS; ++i) {
-                    float a = bias[i];
-#pragma unroll
-                    for (int k = 0; k < W; ++k) a = __builtin_fmaf(w[k][i], xw[(u + k) % W][i], a);
-                    const float sg = sigmoid_f(a);
-                    const float g = lin ? to_f(cd[u].v[i]) * sg * (1.f + a * (1.f - sg)) : 0.f;
-                    gw[u][i] = g;
-                    if (own) {
-                        db[i] += g;
-#pragma unroll
-                        for (int k = 0; k < W; ++k) dw[k][i] = __builtin_fmaf(g, xw[(u + k) % W][i], dw[k][i]);
-                    }
-                }
-                const int j = l - H;                  // dx[j] = sum_k w[k] g[l - k]
-                if (j >= l0 && j < l1) {
-                    ConvVec<T, VS> o;
-#pragma unroll
-                    for (int i = 0; i < VS; ++i) {
-                        float a = 0.f;
-#pragma unroll
-                        for (int k = 0; k < W; ++k) a = __builtin_fmaf(w[k][i], gw[(u - k + W) % W][i], a);
-                        o.v[i] = from_f<T>(a);
-                    }
-                    *reinterpret_cast<ConvVec<T, VS> *>(dx + (int64_t)j * dx_sl) = o;
-                }
+                for (int k = 0; k < W; ++k) dw[k][i] = __builtin_fmaf(g, xw[(u + k) % W][i], dw[k][i]);
             }
+            a = 0.f;
+#pragma unroll
+            for (int k = 0; k < W; ++k) a = __builtin_fmaf(w[k][i], gw[(u - k + W) % W][i], a);
+            o.v[i] = from_f<T>(a);
         }
+        if (live && (!E || (j >= l0 && j < l1))) conv_row_store<Raw>(dx + j * dx_row, co, __builtin_bit_cast(Raw, o));
+        __builtin_amdgcn_sched_barrier(0);            // (interleaved steps would need more registers than four waves per SIMD leave)
+    };
+    for (int s0 = lb; s0 < lend; s0 += W) {
+        if (s0 - H >= l0 && s0 + W <= l1 && s0 + W + H <= L) conv_steps<W>([&](auto U) __attribute__((always_inline)) { step(std::false_type(), U, s0); });
+        else
+            conv_steps<W>([&](auto U) __attribute__((always_inline)) {
+                if (s0 + decltype(U)::value < lend) step(std::true_type(), U, s0);
+            });
     }
-    float *pp = part + (tile * p.channels + c0) * (W + 1);
+    if (!live) return;
+    float *pp = part + ((int64_t)tile * p.channels + c0) * (W + 1);
 #pragma unroll
     for (int i = 0; i < VS; ++i) {
 #pragma unroll
@@ -248,25 +283,56 @@ __global__ __launch_bounds__(NTHREADS) void conv1d_silu_bwd_kernel(const bimamba
     }
 }
 
-// positions per thread: forward 4 filter widths, backward 8 (fewer, longer runs: fewer partial sums to add up)
-static inline int conv_tile_len(const bimamba2_conv_params *p, bool bwd) { return p->width * (bwd ? 8 : 4); }
+// Positions per thread: forward 4 filter widths; backward 2 to 16, by the time that the rounds of workgroups take (256 CUs,
+// as many workgroups each as the kernel's registers leave: 147 at width 7): a workgroup costs its positions, the filter's reach
+// and a start worth about 12 more.  Few positions where the grid is small, and tiles that end with a round where it is not
+// (16 x 1024 x 1664: 59 us with 56 positions, 988 workgroups in two rounds; 51 us with the 77 chosen, 728 in one).
+static int conv_tile_len(const bimamba2_conv_params *p, bool bwd) {
+    if (!bwd) return p->width * 4;
+    const int64_t across = (p->channels / 2 + 63) / 64, slots = 256 * (p->width <= 5 ? 4 : p->width == 7 ? 3 : 2);
+    int64_t best = 0, best_cost = 0;
+    for (int k = 2; k <= 16; ++k) {
+        const int64_t tl = (int64_t)p->width * k, wgs = (p->batch * ((p->seqlen + tl - 1) / tl) * across + 3) / 4;
+        const int64_t cost = (wgs + slots - 1) / slots * (tl + p->width + 12);
+        if (!best || cost <= best_cost) { best = tl; best_cost = cost; }
+    }
+    return (int)best;
+}
 static inline int conv_ntl(const bimamba2_conv_params *p, bool bwd) {
     const int tl = conv_tile_len(p, bwd);
     return (int)((p->seqlen + tl - 1) / tl);
 }
 
 size_t conv_workspace_bytes(const bimamba2_conv_params *p) {
-    // backward: [batch * ntl][channels][width + 1] partial sums, then the summed [channels][width + 1]
-    return ((size_t)p->batch * conv_ntl(p, true) + 1) * p->channels * (p->width + 1) * sizeof(float);
+    // backward: [batch * ntl][channels][width + 1] partial sums
+    return (size_t)p->batch * conv_ntl(p, true) * p->channels * (p->width + 1) * sizeof(float);
 }
 
-// sums[c][W + 1] -> dweight[c][W], dbias[c]
-__global__ void conv_split_kernel(const float *sums, float *dweight, float *dbias, int channels, int W) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= channels * (W + 1)) return;
-    const int c = i / (W + 1), k = i % (W + 1);
-    if (k < W) dweight[c * W + k] = sums[i];
-    else if (dbias) dbias[c] = sums[i];
+// dweight[c][k], dbias[c] = sums over the tiles of part[tile][c][W + 1]: 16 columns x 16 slices of the tiles per workgroup, the
+// slices added in a fixed order
+__global__ __launch_bounds__(NTHREADS) void conv_sums_kernel(const float *part, float *dweight, float *dbias, int ntiles, int channels, int W) {
+    __shared__ float red[16][17];
+    const int jl = threadIdx.x & 15, sl = threadIdx.x >> 4, j = blockIdx.x * 16 + jl, nj = channels * (W + 1);
+    float s = 0.f;
+    if (j < nj) {
+        int i = sl;
+        for (; i + 48 < ntiles; i += 64) {
+            const float a = part[(int64_t)i * nj + j], b = part[(int64_t)(i + 16) * nj + j], c = part[(int64_t)(i + 32) * nj + j],
+                        d = part[(int64_t)(i + 48) * nj + j];
+            s += (a + b) + (c + d);
+        }
+        for (; i < ntiles; i += 16) s += part[(int64_t)i * nj + j];
+    }
+    red[sl][jl] = s;
+    __syncthreads();
+    if (sl == 0 && j < nj) {
+        float t = 0.f;
+#pragma unroll
+        for (int q = 0; q < 16; ++q) t += red[q][jl];
+        const int c = j / (W + 1), k = j - c * (W + 1);
+        if (k < W) dweight[(int64_t)c * W + k] = t;
+        else if (dbias) dbias[c] = t;
+    }
 }
 
 template <typename T, int W, int VS>
@@ -291,14 +357,15 @@ static int launch_conv_w(const bimamba2_conv_params *p, bool bwd) {
     float *part = reinterpret_cast<float *>(p->workspace);
     const int64_t ntiles = (int64_t)p->batch * ntl;
     const int nj = p->channels * (W + 1);
-    float *sums = part + ntiles * nj;
-    hipLaunchKernelGGL((conv1d_silu_bwd_kernel<T, W, VS>), dim3((unsigned)blocks), dim3(NTHREADS), 0, s, *p, ntl, tl, part);
+    const int nwc = (p->channels / VS + 63) / 64;                  // waves side by side over the channels
+    const int64_t waves = ntiles * nwc;
+    if (waves > 0x7fffff00) return BIMAMBA2_EUNSUPPORTED;
+    hipLaunchKernelGGL((conv1d_silu_bwd_kernel<T, W, VS>), dim3((unsigned)((waves + NTHREADS / 64 - 1) / (NTHREADS / 64))), dim3(NTHREADS), 0, s,
+                       *p, ntl, tl, nwc, part);
     int rc = check_launch();
     if (rc) return rc;
-    rc = launch_colsum(part, sums, (int)ntiles, nj, s);
-    if (rc) return rc;
-    hipLaunchKernelGGL(conv_split_kernel, dim3((nj + 255) / 256), dim3(256), 0, s, sums, p->dweight, p->has_bias ? p->dbias : nullptr,
-                       p->channels, W);
+    hipLaunchKernelGGL(conv_sums_kernel, dim3((nj + 15) / 16), dim3(NTHREADS), 0, s, part, p->dweight, p->has_bias ? p->dbias : nullptr,
+                       (int)ntiles, p->channels, W);
     return check_launch();
 }
 

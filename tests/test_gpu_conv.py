@@ -53,6 +53,15 @@ def test_conv1d_silu_forward_and_backward(case):
         assert_close(bd.grad, b64.grad, dtype, "dbias")
 
 
+# tiles of the backward kernel: one position in the last tile, one more or less than a whole number of tiles, channels that leave
+# lanes without work in the last wave, and a grid that takes longer tiles (35 positions instead of 14)
+@pytest.mark.parametrize("case", [(1, 1, 2, 7, torch.bfloat16, True, False), (2, 29, 130, 7, torch.bfloat16, True, True),
+                                  (1, 27, 258, 7, torch.float32, True, False), (3, 28, 129, 5, torch.float16, False, False),
+                                  (16, 1100, 640, 7, torch.bfloat16, True, False)])
+def test_backward_tiles(case):
+    test_conv1d_silu_forward_and_backward(case)
+
+
 @pytest.mark.parametrize("dtype,C", [(torch.bfloat16, 64), (torch.float32, 5)])
 def test_conv1d_silu_gradient_into_a_slice(dtype, C):
     """dx_place: the gradient of x lands in a slice of a wider buffer (the layer's use), bit for bit what the plain call
