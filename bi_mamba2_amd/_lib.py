@@ -35,7 +35,7 @@ class Params(ctypes.Structure):
                               "states16_f", "states16_b", "dstates16_f", "dstates16_b", "workspace")]
         + [("workspace_bytes", ctypes.c_size_t), ("stream", _vp)]
         + [(n, _i64) for n in ("dx_sb", "dx_sl", "dB_sb", "dB_sl", "dC_sb", "dC_sl", "ddt_sb", "ddt_sl")]
-        + [("dbdc_heads", _i32), ("reserved", _i32)]
+        + [("dbdc_heads", _i32), ("dcb_slices", _i32)]
     )
 
 

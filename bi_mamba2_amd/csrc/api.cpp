@@ -106,6 +106,7 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     }
     if (is_bwd) {
         const size_t nqt = (Q + 63) / 64;
+        if (!q->dCB && !q->dCBT) q->dcb_slices = choose_dcb_slices(q);
         need_f(q->dCB, cbn * dcb_slices(q));
         need_f(q->dCBT, cbn * dcb_slices(q));
         if (!scan_recomputes_cb(q, true)) need_f(q->CBT, cbn);

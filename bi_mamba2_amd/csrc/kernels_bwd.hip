@@ -1368,9 +1368,9 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_kernel(const bimamba2_params
     }
 }
 
-// dst[i] += sum_{s=1..nslices-1} dst[s*n + i]
-__global__ __launch_bounds__(NTHREADS) void sum_slices_kernel(float *dst, size_t n4, int nslices) {
-    float4 *d = reinterpret_cast<float4 *>(dst);
+// dst[i] += sum_{s=1..nslices-1} dst[s*n + i], for dst0 and dst1 (blockIdx.y)
+__global__ __launch_bounds__(NTHREADS) void sum_slices_kernel(float *dst0, float *dst1, size_t n4, int nslices) {
+    float4 *d = reinterpret_cast<float4 *>(blockIdx.y ? dst1 : dst0);
     for (size_t i = blockIdx.x * (size_t)NTHREADS + threadIdx.x; i < n4; i += (size_t)gridDim.x * NTHREADS) {
         float4 v = d[i];
         for (int s = 1; s < nslices; ++s) {
@@ -1381,8 +1381,10 @@ __global__ __launch_bounds__(NTHREADS) void sum_slices_kernel(float *dst, size_t
     }
 }
 
-// head slices of the dCB kernel: one per 32 heads of a group (more slices only cost traffic: measured)
+// Head slices of the dCB kernel: one per 32 heads of a group (more slices only cost traffic: measured with the ring variant,
+// which has several workgroups on every CU).
 int dcb_slices(const bimamba2_params *p) {
+    if (p->dcb_slices > 0) return p->dcb_slices;
     const int hpg = p->nheads / p->ngroups;
     return std::max(1, std::min(DCB_SLICES_MAX, hpg / DCB_SLICE_HEADS));
 }
@@ -1886,10 +1888,21 @@ static int launch_dcb_t(const bimamba2_params *p) {
         const size_t n = (size_t)p->batch * nc * p->ngroups * p->chunk_size * p->chunk_size;
         if (n % 4) return BIMAMBA2_EUNSUPPORTED;
         const int blocks = (int)std::min<size_t>((n / 4 + NTHREADS - 1) / NTHREADS, 4096);
-        hipLaunchKernelGGL(sum_slices_kernel, dim3(blocks), dim3(NTHREADS), 0, stream_of(p), p->dCB, n / 4, slices);
-        hipLaunchKernelGGL(sum_slices_kernel, dim3(blocks), dim3(NTHREADS), 0, stream_of(p), p->dCBT, n / 4, slices);
+        hipLaunchKernelGGL(sum_slices_kernel, dim3(blocks, 2), dim3(NTHREADS), 0, stream_of(p), p->dCB, p->dCBT, n / 4, slices);
     }
     return check_launch();
+}
+
+// The same for the variant through registers (float32, and 16-bit shapes without the ring): a wave of it is one chain of loads,
+// products and exponentials, 5 to 7 us a head, and leaves three quarters of its SIMD to others, so slices pay until there are
+// three workgroups on every CU, down to two heads a slice: adding them up costs a launch.
+// 2 x 1111 positions, 16 heads in 2 groups, float32: 56 us in 320 workgroups of eight heads, 42 + 6 us in two slices, 43 + 9 us in four.
+int choose_dcb_slices(const bimamba2_params *p) {
+    const int usual = dcb_slices(p), hpg = p->nheads / p->ngroups, nqt = (p->chunk_size + 63) / 64;
+    const int64_t n = (int64_t)p->batch * nchunks(p) * p->ngroups * p->chunk_size * p->chunk_size;
+    if (dcb_recomputes_cb(p) || p->causal || n % 4) return usual;
+    const int64_t wgs = (int64_t)p->batch * nchunks(p) * p->ngroups * nqt * nqt;
+    return (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, 768 / wgs}));
 }
 
 // whether bwd_dcb_sp_kernel exists for the problem (the ring variant of the dCB kernel with one head slice, the vector

@@ -49,6 +49,7 @@ int launch_state_passing_bwd(const bimamba2_params *p);
 int choose_dbdc_heads(const bimamba2_params *p);   // heads per slice of the dB / dC partial sums
 int launch_bwd_dbdc(const bimamba2_params *p, bool is_db);
 int launch_bwd_dcb(const bimamba2_params *p);
+int choose_dcb_slices(const bimamba2_params *p);
 int dcb_slices(const bimamba2_params *p);   // head slices whose dCB partial sums the kernel keeps apart
 int launch_bmm_chunk_bwd(const bimamba2_params *p);
 // out[j] = sum_i sum_k in[(i*nj + j)*nk + k]

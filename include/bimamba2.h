@@ -93,7 +93,7 @@ typedef struct bimamba2_params {
     /* intermediates (caller-owned; the composite entry points carve them from `workspace` when NULL) */
     float *dt_out, *cs_f, *cs_b;
     float *CB;
-    float *dCB;                     /* room for min(4, max(1, H/G/32)) copies: head-slice partial sums, added up in place */
+    float *dCB;                     /* room for min(4, max(1, H/G/32)) copies (see dcb_slices): head-slice partial sums, added up in place */
     float *CBT;                     /* optional: CB transposed per chunk, CBT[.., s, l] = CB[.., l, s] */
     float *dCBT;                    /* dCB transposed per chunk (same number of copies as dCB) */
     float *states_f, *states_b;     /* chunk states, overwritten in place by the inter-chunk scan */
@@ -162,7 +162,8 @@ typedef struct bimamba2_params {
     int64_t ddt_sb, ddt_sl;         /* likewise of ddt (batch, seqlen, nheads): 0 means contiguous */
     int32_t dbdc_heads;             /* heads per slice of dBs / dCs (1..8): S = ceil(H/G/dbdc_heads); 0 means 8.  bimamba2_bwd
                                        chooses it itself where dBs and dCs are its own. */
-    int32_t reserved;
+    int32_t dcb_slices;             /* head slices of dCB / dCBT, one copy of each per slice; 0 means min(4, max(1, H/G/32)).
+                                       bimamba2_bwd chooses it itself where dCB and dCBT are its own. */
 } bimamba2_params;
 
 /* text of an error code */

@@ -45,3 +45,11 @@ def test_shapes_between_the_tiles(case):
     assert_close(out, ref["out"], dtype, "out", scaled=big)
     for k, g in zip(names, grads):
         assert_close(g, ref["d" + k], dtype, "d" + k, scaled=big or is_reduced("d" + k, dtype))
+
+
+# dCB in head slices where the grid is small: 11 heads in slices of three (of five slices the last is empty), 5 in slices of two
+# and three, a 16-bit shape, and a chunk whose square is no multiple of four (no slices)
+@pytest.mark.parametrize("case", [(1, 200, 11, 64, 1, 64, 64, torch.float32, True, "h"), (1, 300, 5, 32, 1, 16, 256, torch.float32, False, "none"),
+                                  (2, 130, 10, 32, 2, 16, 64, torch.float16, True, "hp"), (1, 130, 8, 16, 1, 16, 65, torch.float32, False, "h")])
+def test_dcb_head_slices(case):
+    test_shapes_between_the_tiles(case)
