@@ -4,7 +4,8 @@ Same constructor keywords, parameter names/shapes (so state_dicts interchange) a
 reference layer (src/ssd/modules.py:17-187): in_proj -> split [z | xBC | dt] -> softplus(dt + dt_bias) ->
 non-causal depthwise conv1d + SiLU -> split x, B, C -> bidirectional SSD with D -> gated RMSNorm(y, z) ->
 out_proj.  Parameters are created in the reference's order, so a seeded construction draws the same values.
-The projections are torch GEMMs; the convolution, the SSD and the gated RMS norm are the HIP operators.
+The projections run on this library's matrix product and, for large outputs, on torch's; the convolution, the SSD and the
+gated RMS norm are the HIP operators.
 """
 import ctypes
 import math
