@@ -1460,13 +1460,14 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
     const int Q = p.chunk_size, P = p.headdim, H = p.nheads, hpg = H / p.ngroups;
     const int limit = min(Q, p.seqlen - c * Q);
     const int t0 = tt * 64, s0 = st * 64;
-    const bool live = t0 < limit && s0 < limit && !(UNI && st > tt);
     const int trow = wave * 16 + lg * 4;                       // first of this lane's four accumulator rows
     f32x4 cbr[4] = {}, dcb[4] = {};
     const int hps = (hpg + gdz - 1) / gdz;
     const int h_begin = bid.z * hps, h_end = min(hpg, h_begin + hps);
     const int nkc = P / KC, nhs = h_end - h_begin, nit = nhs * nkc;
     const int h0 = g * hpg + h_begin;
+    // (a caller's dcb_slices may leave a slice without heads: it writes zeros and requests nothing, its h0 may lie behind the last head)
+    const bool live = t0 < limit && s0 < limit && !(UNI && st > tt) && nhs > 0;
     const int64_t tv_head = (int64_t)nc * nqt * nqt * DCB_VEC;
     float *tv0 = p.da_intra + ((((int64_t)b * H + h0) * nc + c) * nqt * nqt + tile) * DCB_VEC;
     if (!live) {
@@ -1902,7 +1903,9 @@ int choose_dcb_slices(const bimamba2_params *p) {
     const int64_t n = (int64_t)p->batch * nchunks(p) * p->ngroups * p->chunk_size * p->chunk_size;
     if (dcb_recomputes_cb(p) || p->causal || n % 4) return usual;
     const int64_t wgs = (int64_t)p->batch * nchunks(p) * p->ngroups * nqt * nqt;
-    return (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, 768 / wgs}));
+    const int wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, 768 / wgs}));
+    const int heads = (hpg + wanted - 1) / wanted;               // (9 heads in 4 slices: three of 3, the fourth would be empty)
+    return (hpg + heads - 1) / heads;
 }
 
 // whether bwd_dcb_sp_kernel exists for the problem (the ring variant of the dCB kernel with one head slice, the vector

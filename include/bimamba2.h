@@ -163,6 +163,7 @@ typedef struct bimamba2_params {
     int32_t dbdc_heads;             /* heads per slice of dBs / dCs (1..8): S = ceil(H/G/dbdc_heads); 0 means 8.  bimamba2_bwd
                                        chooses it itself where dBs and dCs are its own. */
     int32_t dcb_slices;             /* head slices of dCB / dCBT, one copy of each per slice; 0 means min(4, max(1, H/G/32)).
+                                       A slice holds ceil(H/G/dcb_slices) heads; one that is left without any adds zeros.
                                        bimamba2_bwd chooses it itself where dCB and dCBT are its own. */
 } bimamba2_params;
 

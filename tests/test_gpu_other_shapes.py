@@ -47,9 +47,39 @@ def test_shapes_between_the_tiles(case):
         assert_close(g, ref["d" + k], dtype, "d" + k, scaled=big or is_reduced("d" + k, dtype))
 
 
-# dCB in head slices where the grid is small: 11 heads in slices of three (of five slices the last is empty), 5 in slices of two
-# and three, a 16-bit shape, and a chunk whose square is no multiple of four (no slices)
+# dCB in head slices where the grid is small: 11 heads in slices of three (the last of two), 5 in slices of two and three, a 16-bit
+# shape, a chunk whose square is no multiple of four (no slices), and the ring of direct loads with a narrow state (9 heads of 64)
 @pytest.mark.parametrize("case", [(1, 200, 11, 64, 1, 64, 64, torch.float32, True, "h"), (1, 300, 5, 32, 1, 16, 256, torch.float32, False, "none"),
-                                  (2, 130, 10, 32, 2, 16, 64, torch.float16, True, "hp"), (1, 130, 8, 16, 1, 16, 65, torch.float32, False, "h")])
+                                  (2, 130, 10, 32, 2, 16, 64, torch.float16, True, "hp"), (1, 130, 8, 16, 1, 16, 65, torch.float32, False, "h"),
+                                  (2, 130, 9, 64, 1, 16, 64, torch.bfloat16, False, "h")])
 def test_dcb_head_slices(case):
     test_shapes_between_the_tiles(case)
+
+
+@pytest.mark.parametrize("headdim,dtype", [(64, torch.bfloat16), (128, torch.float16), (64, torch.float32), (32, torch.bfloat16)])
+def test_dcb_slices_of_the_callers_choice(headdim, dtype):
+    """9 heads in 4 slices start at 0, 3, 6 and 9: the last one is empty and adds nothing, with the ring of direct loads (16 bits,
+    whole 64-column tiles) and through registers"""
+    from bi_mamba2_amd import ops
+    b, L, H, Q = 2, 100, 9, 64
+    d = to_dev(make_case(b, L, H, headdim, 1, 16, dtype))
+    csf, csb, dt = ops._chunk_cumsum_fwd(d["dt"], d["A"], Q, dt_bias=d["dt_bias"], dt_softplus=True)
+    CB = ops._bmm_chunk_fwd(d["C"], d["B"], Q)
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(3)).to(dtype).cuda()
+
+    def dcb(slices):
+        c = ops._Call(b, L, H, headdim, 1, 1, Q, dtype, dout.device)
+        c.set_x(d["x"]); c.set_dout(dout)
+        for name, t in (("CB", CB), ("dt_out", dt), ("cs_f", csf), ("cs_b", csb)):
+            c.put(name, t, torch.float32)
+        c.p.dcb_slices = slices
+        dCB, dCBT = (c.new(name, (slices, b, 2, 1, Q, Q))[0] for name in ("dCB", "dCBT"))
+        da = c.new("da_intra", (b, H, 2, 1, 2, 64))
+        c.run("bimamba2_chunk_scan_bwd_dcb")
+        return dCB, dCBT, da
+
+    (one, oneT, da1), (four, fourT, da4) = dcb(1), dcb(4)
+    assert torch.equal(da1, da4)
+    # the same nine float32 terms an element, added in another order
+    assert (four - one).norm() <= 1e-6 * one.norm() and torch.equal(fourT, four.transpose(-1, -2))
+    assert torch.equal(oneT, one.transpose(-1, -2))

@@ -199,3 +199,32 @@ def test_chunk_size_follows_the_number_of_sequence_boundaries():
     mixed = torch.cat([torch.zeros(1, 256, dtype=torch.int64), 1 + torch.arange(256)[None].div(5, rounding_mode="floor")], dim=1)
     assert ops.chunk_size_for_seq_idx(mixed, 256) == 128                    # the densest chunk decides
     assert ops.chunk_size_for_seq_idx(four, 64) == 64                       # never above what the caller asked for
+
+
+def _dcb_slices(**kw):
+    """head slices of dCB that bimamba2_bwd works with: what its workspace holds beside a caller's dCB and dCBT"""
+    lib = _lib.load()
+    own, brought = (lib.bimamba2_workspace_bytes(ctypes.byref(_params(**kw, **extra)), 1) for extra in ({}, dict(dCB=256, dCBT=256)))
+    nc = -(-kw["seqlen"] // kw["chunk_size"])
+    slices, rest = divmod(own - brought, 2 * 4 * kw["batch"] * nc * kw["ngroups"] * kw["chunk_size"] ** 2)
+    assert rest == 0
+    return slices
+
+
+def _contiguous(batch, seqlen, nheads, headdim, ngroups, dstate, chunk_size, dtype):
+    return dict(batch=batch, seqlen=seqlen, nheads=nheads, headdim=headdim, ngroups=ngroups, dstate=dstate, chunk_size=chunk_size,
+                dtype=dtype, x_sb=seqlen * nheads * headdim, x_sl=nheads * headdim, x_sh=headdim, B_sb=seqlen * ngroups * dstate,
+                B_sl=ngroups * dstate, B_sg=dstate, C_sb=seqlen * ngroups * dstate, C_sl=ngroups * dstate, C_sg=dstate)
+
+
+def test_no_head_slice_of_dcb_is_empty():
+    """a slice starts at its number times ceil(heads / slices): 9 heads in 4 slices, 11 in 5 and 17 in 8 would leave the last one
+    behind the end of the group"""
+    cut = set()
+    for dtype, headdim, dstate in ((_lib.F32, 64, 64), (_lib.BF16, 64, 16), (_lib.F16, 32, 16)):
+        for rows in (1, 3, 30, 192, 400, 800):                     # (batch, chunk) pairs
+            for hpg in range(1, 257):
+                n = _dcb_slices(**_contiguous(rows, 64, 2 * hpg, headdim, 2, dstate, 64, dtype))
+                assert 1 <= n <= max(8, hpg // 32) and (n - 1) * -(-hpg // n) < hpg, (dtype, rows, hpg, n)
+                cut.add(n)
+    assert {1, 2, 3, 4, 8} <= cut
