@@ -1381,8 +1381,8 @@ __global__ __launch_bounds__(NTHREADS) void sum_slices_kernel(float *dst0, float
     }
 }
 
-// Head slices of the dCB kernel: one per 32 heads of a group (more slices only cost traffic: measured with the ring variant,
-// which has several workgroups on every CU).
+// Head slices of the dCB kernel unless the caller says otherwise: one per 32 heads of a group (on grids that fill the chip more
+// slices only cost traffic: 512 tiles of 24 heads 38 us in one slice, 42 in two; for small grids see choose_dcb_slices).
 int dcb_slices(const bimamba2_params *p) {
     if (p->dcb_slices > 0) return p->dcb_slices;
     const int hpg = p->nheads / p->ngroups;
@@ -1894,16 +1894,26 @@ static int launch_dcb_t(const bimamba2_params *p) {
     return check_launch();
 }
 
-// The same for the variant through registers (float32, and 16-bit shapes without the ring): a wave of it is one chain of loads,
-// products and exponentials, 5 to 7 us a head, and leaves three quarters of its SIMD to others, so slices pay until there are
-// three workgroups on every CU, down to two heads a slice: adding them up costs a launch.
-// 2 x 1111 positions, 16 heads in 2 groups, float32: 56 us in 320 workgroups of eight heads, 42 + 6 us in two slices, 43 + 9 us in four.
+// Head slices where bimamba2_bwd owns dCB and the kernel reads C.B^T: float32, and 16-bit shapes whose state or headdim is no
+// multiple of what the rebuilding kernel takes (through registers, or the ring with a narrow state).  Where C.B^T is rebuilt the
+// number is dcb_slices()'s: every slice would rebuild it, and one slice shares its launch with the state passing.
+// A workgroup is one chain over its heads, 5 to 7 us a head through registers in float32, 3 to 5 in 16 bits and 1.5 in the ring,
+// so slices pay on a small grid until there are three workgroups on every CU; against them stands a launch that adds them up
+// (4 us, and 0.03 us per tile and slice), which few heads do not earn: in 16 bits a slice wants a head per 32 tiles of the grid,
+// in float32 fewer than six heads are cut only where all slices are on the chip at once.  us with one slice -> with the number
+// chosen here (-> with as many as three workgroups a CU would allow, where that is another number), the adding up included:
+//   float32, headdim 64: 16 heads in 2 groups, 320 tiles 56 -> 42 + 6; 24 heads, 256 tiles 112 -> 82; 4 heads, 192 tiles 23 (-> 28)
+//   16 bits, headdim 32 or 16: 24 heads, 64 tiles 94 -> 30; 17 heads, 240 tiles 70 -> 51 (-> 62); 8 heads, 320 tiles 43 (-> 49);
+//     6 heads, 384 tiles 33 (-> 46); the rule loses at 7 heads, 176 tiles (32 -> 29) and 15 heads, 256 tiles (62 -> 56)
+//   ring, headdim 64, state 16: 48 heads, 64 tiles 62 -> 22; 24 heads, 256 tiles 36 -> 31; 16 heads, 160 tiles 26 -> 20 (-> 21);
+//     8 heads, 320 tiles 17 (-> 22); 4 heads, 192 tiles 10 (-> 17); 8 heads, 128 tiles 15 -> 16 (-> 19)
 int choose_dcb_slices(const bimamba2_params *p) {
     const int usual = dcb_slices(p), hpg = p->nheads / p->ngroups, nqt = (p->chunk_size + 63) / 64;
     const int64_t n = (int64_t)p->batch * nchunks(p) * p->ngroups * p->chunk_size * p->chunk_size;
     if (dcb_recomputes_cb(p) || p->causal || n % 4) return usual;
     const int64_t wgs = (int64_t)p->batch * nchunks(p) * p->ngroups * nqt * nqt;
-    const int wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, 768 / wgs}));
+    const int most = p->dtype == BIMAMBA2_F32 ? (hpg < 6 ? 256 : 768) : std::min(768, 32 * hpg);      // workgroups
+    const int wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, most / wgs}));
     const int heads = (hpg + wanted - 1) / wanted;               // (9 heads in 4 slices: three of 3, the fourth would be empty)
     return (hpg + heads - 1) / heads;
 }

@@ -207,7 +207,7 @@ def _dcb_slices(**kw):
     own, brought = (lib.bimamba2_workspace_bytes(ctypes.byref(_params(**kw, **extra)), 1) for extra in ({}, dict(dCB=256, dCBT=256)))
     nc = -(-kw["seqlen"] // kw["chunk_size"])
     slices, rest = divmod(own - brought, 2 * 4 * kw["batch"] * nc * kw["ngroups"] * kw["chunk_size"] ** 2)
-    assert rest == 0
+    assert rest < 512                      # (each piece begins at a multiple of 256)
     return slices
 
 
@@ -228,3 +228,14 @@ def test_no_head_slice_of_dcb_is_empty():
                 assert 1 <= n <= max(8, hpg // 32) and (n - 1) * -(-hpg // n) < hpg, (dtype, rows, hpg, n)
                 cut.add(n)
     assert {1, 2, 3, 4, 8} <= cut
+
+
+# heads in one group, (batch, chunk) pairs, chunk, headdim, dstate, dtype -> slices.  Cut only where the kernel reads C.B^T (dstate
+# 64 and 16 bits rebuilds it), where the grid is small, and in 16 bits (in float32 below six heads) only with heads enough for it.
+@pytest.mark.parametrize("heads,rows,chunk,headdim,dstate,dtype,slices", [
+    (24, 16, 256, 64, 16, _lib.BF16, 3), (24, 16, 256, 64, 64, _lib.BF16, 1), (128, 16, 256, 64, 64, _lib.BF16, 4),
+    (24, 32, 256, 64, 16, _lib.BF16, 1), (8, 20, 256, 64, 16, _lib.BF16, 1), (8, 20, 256, 32, 16, _lib.F16, 1),
+    (24, 4, 256, 32, 64, _lib.BF16, 8), (8, 20, 256, 64, 64, _lib.F32, 2), (4, 12, 256, 64, 64, _lib.F32, 1),
+    (4, 4, 256, 64, 64, _lib.F32, 2), (64, 64, 256, 64, 64, _lib.F32, 2), (24, 64, 65, 64, 64, _lib.F32, 3), (25, 63, 65, 64, 64, _lib.F32, 1)])
+def test_head_slices_of_dcb(heads, rows, chunk, headdim, dstate, dtype, slices):
+    assert _dcb_slices(**_contiguous(rows, chunk, heads, headdim, 1, dstate, chunk, dtype)) == slices
