@@ -227,15 +227,6 @@ struct Problem {
     }
 };
 
-// Whether the forward pass keeps C.B^T and its transpose for the backward pass: where the backward's kernels read them and
-// they take no more memory than x, or little (64 MiB).  It forms the product for itself there; the backward's launch for both
-// took 9 to 13 us (float32 with 16 heads in 2 groups over 2 x 1111 positions, bfloat16 at state dimension 128 over 2 x 3001).
-bool keeps_cb(const bimamba2_params &p) {
-    const size_t nc = (p.seqlen + p.chunk_size - 1) / p.chunk_size, e = p.dtype == BIMAMBA2_F32 ? 4 : 2;
-    const size_t bytes = 8 * (size_t)p.batch * nc * p.ngroups * p.chunk_size * p.chunk_size;
-    return api.reads_cb(&p, 0) && api.reads_cb(&p, 1) && bytes <= std::max(e * p.batch * p.seqlen * p.nheads * p.headdim, size_t(64) << 20);
-}
-
 // What the forward pass leaves for the backward pass besides its operands, in one float32 allocation: dt_out, cs_f, cs_b, the
 // states entering the chunks (copies: in the operands' 16-bit type, where the kernels can keep them that way) and, with cb,
 // C.B^T and its transpose.
@@ -270,6 +261,18 @@ struct Kept {
     // what bimamba2_bwd is told about these
     int saved() const { return ncb ? 3 : 1; }
 };
+
+// Whether the forward pass keeps C.B^T and its transpose for the backward pass: where the backward's kernels read them and they
+// are no larger than what the call holds between the passes anyway (x, the decays and the states), so that a model's layers
+// hold at most twice as much.  The forward pass forms the product for itself there; the backward's launch for both took 9 to 13 us
+// (float32 with 16 heads in 2 groups over 2 x 1111 positions, 10 MB beside 15; bfloat16 at state dimension 128 over 2 x 3001, 13
+// MB beside 57).  With few narrow heads per group it would be many times that: 17 MB beside 1.5 at 4 heads of 16 in 4 groups.
+bool keeps_cb(const bimamba2_params &p) {
+    if (!api.reads_cb(&p, 0) || !api.reads_cb(&p, 1)) return false;
+    const size_t e = p.dtype == BIMAMBA2_F32 ? 4 : 2, x = e * p.batch * p.seqlen * p.nheads * p.headdim;
+    const Kept without(p, false, false), with(p, false, true);
+    return 8 * with.ncb <= x + 4 * (size_t)without.floats();
+}
 
 Tensor attach_workspace(bimamba2_params &p, bool bwd, const Tensor &like) {
     Tensor ws = device_empty({(int64_t)std::max<size_t>(api.workspace_bytes(&p, bwd), 1)}, at::kByte, like);

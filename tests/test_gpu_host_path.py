@@ -144,18 +144,45 @@ def test_layer_parameters_of_other_shapes():
             m(torch.zeros(2, 100, 72, device="cuda", dtype=torch.bfloat16))
 
 
+def held_for_backward(fn):
+    """bytes that the result of fn() keeps besides the tensors it returns"""
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated()
+    out = fn()
+    return torch.cuda.memory_allocated() - before - out.untyped_storage().nbytes(), out
+
+
 def test_cb_kept_or_formed_again():
-    """C.B^T of one row of 2304 positions and 8 groups (38 MB with its transpose) is kept for the backward pass, that of two rows
-    is formed again there: the gradients of a row are the same, bit for bit"""
-    d = to_dev(make_case(2, 2304, 8, 16, 8, 16, torch.bfloat16, with_z=True))
+    """C.B^T is kept for the backward pass with eight heads in a group of 64-position chunks (8 KB for each group and position
+    beside 9.5) and formed again there with two (beside 2.4): what belongs to one head is the same, bit for bit"""
+    b, L, P, G, N, Q = 2, 200, 16, 2, 16, 64
+    d = to_dev(make_case(b, L, 16, P, G, N, torch.bfloat16, with_z=True))
     from bi_mamba2_amd import ops
     dy = torch.randn_like(d["x"])
+    nc, cb = -(-L // Q), 2 * 4 * b * -(-L // Q) * G * Q * Q
 
-    def grads(rows):
-        leaves = [d[k][rows].clone().requires_grad_(True) for k in ("x", "dt", "B", "C", "z")]
-        x, dt, B, C, z = leaves
-        out = ops.bimamba_chunk_scan_combined(x, dt, d["A"], B, C, 256, D=d["D"], z=z, dt_bias=d["dt_bias"], dt_softplus=True)
-        return (out.detach(),) + torch.autograd.grad(out, leaves, dy[rows])
+    def grads(heads):
+        x, dt, z = (d[k][:, :, heads].clone().requires_grad_(True) for k in ("x", "dt", "z"))
+        A, D, bias = (d[k][heads].clone() for k in ("A", "D", "dt_bias"))
+        held, out = held_for_backward(lambda: ops.bimamba_chunk_scan_combined(x, dt, A, d["B"], d["C"], Q, D=D, z=z, dt_bias=bias, dt_softplus=True))
+        H = len(heads)
+        own = 4 * (3 * b * H * nc * Q + 2 * b * nc * H * P * N) + 2 * x.numel()            # decays, states, the result in front of the gate
+        return held, own, (out.detach(),) + torch.autograd.grad(out, (x, dt, z), dy[:, :, heads])
 
-    for both, one in zip(grads(slice(0, 2)), grads(slice(1, 2))):
-        assert torch.equal(both[1:], one)
+    held, own, all_heads = grads(list(range(16)))
+    assert own + cb <= held <= own + cb + 4096
+    few = [0, 1, 8, 9]
+    held, own, some = grads(few)
+    assert own <= held <= own + 4096
+    for a, s in zip(all_heads, some):
+        assert torch.equal(a[:, :, few], s)
+
+
+def test_memory_held_for_the_backward_pass():
+    """what a call keeps follows its operands, however large C.B^T is beside them (17 MB beside an x of 1 MB)"""
+    d = to_dev(make_case(2, 2048, 4, 16, 4, 16, torch.float32, with_z=True))
+    from bi_mamba2_amd import ops
+    x = d["x"].clone().requires_grad_(True)
+    held, out = held_for_backward(lambda: ops.bimamba_chunk_scan_combined(x, d["dt"], d["A"], d["B"], d["C"], 128, D=d["D"], z=d["z"],
+                                                                          dt_bias=d["dt_bias"], dt_softplus=True))
+    assert held <= 4 * x.numel() * 4
