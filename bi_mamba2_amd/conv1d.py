@@ -11,6 +11,7 @@ There is no CPU or PyTorch fallback: CPU tensors raise, a missing library raises
 import ctypes
 
 import torch
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 from .ops import _DT, _require_gpu
@@ -92,6 +93,7 @@ class Conv1dSiluFn(torch.autograd.Function):
         return _conv1d_silu_fwd(x, weight, bias)
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, dout):
         x, weight, bias = ctx.saved_tensors
         dx, dw, db = _conv1d_silu_bwd(dout, x, weight, bias, dx_out=ctx.dx_place() if ctx.dx_place is not None else None)

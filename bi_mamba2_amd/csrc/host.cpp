@@ -11,6 +11,7 @@
 #include <dlfcn.h>
 #include <torch/extension.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/autograd/functions/utils.h>
 #include <ATen/hip/EmptyTensor.h>
 #include <c10/hip/HIPStream.h>
 #include <c10/hip/HIPGuard.h>
@@ -128,6 +129,27 @@ inline Tensor undef(const OptTensor &t) { return t ? *t : Tensor(); }
 
 // float32 contiguous form of a parameter (A, D, dt_bias) or state
 inline Tensor f32c(const Tensor &t) { return as_type(t, at::kFloat).contiguous(); }
+
+// The gradients that the kernels write have no history.  Where a backward pass is itself recorded (create_graph), they are given
+// one that leads back to what they were computed from and refuses to be differentiated: as one term of a loss they would
+// otherwise count as constants without a word.
+struct NoSecondDerivative : torch::autograd::Node {
+    const char *of;
+    explicit NoSecondDerivative(const char *of_) : of(of_) {}
+    std::string name() const override { return "NoSecondDerivative"; }
+    variable_list apply(variable_list &&) override { TORCH_CHECK(false, of, " has no second derivative: its gradients cannot be differentiated again"); }
+};
+
+variable_list once_differentiable(variable_list grads, const variable_list &from, const variable_list &upstream, const char *of) {
+    if (!at::GradMode::is_enabled()) return grads;
+    variable_list all = from;
+    all.insert(all.end(), upstream.begin(), upstream.end());
+    const std::shared_ptr<torch::autograd::Node> node(new NoSecondDerivative(of), torch::autograd::deleteNode);
+    node->set_next_edges(torch::autograd::collect_next_edges(all));
+    for (Tensor &g : grads)
+        if (g.defined()) torch::autograd::set_history(g, node);
+    return grads;
+}
 
 // ---------------------------------------------------------------------------------------------------------------------
 // the operator
@@ -448,8 +470,8 @@ public:
         const Tensor ws = attach_workspace(p, true, q.x);
         check(api.bwd(&p), "bimamba2_bwd");
         auto like = [](const Tensor &g, const Tensor &t) { return g.defined() ? as_type(g, t.scalar_type()) : g; };
-        return {dx, ddt, like(dA, A), like(dB, B), like(dC, C), like(dD, D), dz.defined() ? like(dz, s[6]) : dz, like(dbias, bias),
-                dinit_f, dinit_b, Tensor(), Tensor()};
+        return once_differentiable({dx, ddt, like(dA, A), like(dB, B), like(dC, C), like(dD, D), dz.defined() ? like(dz, s[6]) : dz,
+                                    like(dbias, bias), dinit_f, dinit_b, Tensor(), Tensor()}, s, grads, "bimamba_chunk_scan_combined");
     }
 };
 
@@ -847,7 +869,8 @@ public:
         }
         if (needs(1)) product_tn(dzx, u.reshape({s.rows, u.size(2)}), dw_in = device_empty(w_in.sizes(), u.scalar_type(), u));
         if (needs(2)) db_in = dzx.sum(0);
-        return {du, dw_in, db_in, dprm[0], dprm[1], dprm[2], dprm[3], dprm[4], dprm[5], dw_out, db_out, Tensor()};
+        return once_differentiable({du, dw_in, db_in, dprm[0], dprm[1], dprm[2], dprm[3], dprm[4], dprm[5], dw_out, db_out, Tensor()},
+                                   v, grads, "BiMamba2");
     }
 };
 

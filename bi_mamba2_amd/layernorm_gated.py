@@ -12,6 +12,7 @@ There is no CPU or PyTorch fallback: CPU tensors raise, a missing library raises
 import ctypes
 
 import torch
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 from .ops import _DT, _require_gpu
@@ -131,6 +132,7 @@ class LayerNormFn(torch.autograd.Function):
         return out.reshape(shape)
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, dy):
         x2, w32, b32, rstd, z2, mean = ctx.saved_tensors
         dy2 = _rows(dy, "dy")

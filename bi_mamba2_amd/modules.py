@@ -13,6 +13,7 @@ import math
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 from .conv1d import conv1d_silu_fn
@@ -99,6 +100,7 @@ class _ParamsAsFloat32(torch.autograd.Function):
         return tuple(outs)
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, *grads):
         (A,) = ctx.saved_tensors
         res, items = [], []
@@ -127,6 +129,7 @@ class _SplitInto(torch.autograd.Function):
         return tuple(t[..., b[i]:b[i + 1]] for i in range(len(b) - 1))
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, *grads):
         pieces = ctx.pieces
         copied = []

@@ -15,6 +15,7 @@ Reference interface mirrored here (paths relative to the reference's root):
 import math
 
 import torch
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 from ._lib import Params
@@ -770,6 +771,7 @@ class MambaChunkScanCombinedFn(torch.autograd.Function):
         return out, ff, fb
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, dout, *dfinal):
         out_x, x, dt, A, B, C, D, z, dt_bias, init_f, init_b, blob = ctx.saved_tensors
         saved = ("blob", blob, ctx.snap) if blob is not None else None
@@ -927,6 +929,7 @@ class CausalChunkScanCombinedFn(torch.autograd.Function):
         return res[0]
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, dout):
         out_x, x, dt, A, B, C, D, z, dt_bias, blob = ctx.saved_tensors
         saved = ("blob", blob, ctx.snap) if blob is not None else None

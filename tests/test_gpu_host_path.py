@@ -123,6 +123,36 @@ def test_saved_tensor_hooks_and_checkpointing(how):
         assert torch.equal(a, b) and torch.equal(a, c)
 
 
+@pytest.mark.parametrize("how", ["layer", "composed layer", "scan", "scan without kept intermediates"])
+def test_second_derivatives_are_refused(how, monkeypatch):
+    """the gradients of a recorded backward pass are the same values, and no constants in a loss"""
+    from bi_mamba2_amd import ops
+    from bi_mamba2_amd.modules import _GradPieces
+    if "layer" in how:
+        m, u, leaves = small_layer()
+        fn = lambda: m(u)
+        if how.startswith("composed"):
+            monkeypatch.setattr(_GradPieces, "on_copied", staticmethod(lambda copied: None))
+    else:
+        if "without" in how:
+            monkeypatch.setattr(ops, "KEEP_FORWARD_INTERMEDIATES", False)
+        d = to_dev(make_case(2, 100, 4, 16, 2, 16, torch.bfloat16, with_z=True))
+        leaves = [d[k].clone().requires_grad_(True) for k in ("x", "dt", "A", "B", "C")]
+        fn = lambda: scan_of(d, leaves)
+    out = fn()
+    dy = torch.randn_like(out).requires_grad_("kept" in how)         # (Python functions see it by what comes from upstream)
+    recorded = torch.autograd.grad(out, leaves, dy, create_graph=True)
+    for a, b in zip(torch.autograd.grad(fn(), leaves, dy.detach()), recorded):
+        assert torch.equal(a, b)
+    penalty = recorded[0].float().pow(2).sum()
+    for loss in (penalty, fn().float().sum() + penalty):
+        with pytest.raises(RuntimeError, match="no second derivative|differentiate twice"):
+            loss.backward(retain_graph=True)
+        if "kept" not in how and "composed" not in how:
+            with pytest.raises(RuntimeError, match="no second derivative"):
+                torch.autograd.grad(loss, leaves[0], retain_graph=True)
+
+
 def test_forward_mode_is_refused():
     import torch.autograd.forward_ad as fwAD
     m, u, _ = small_layer()
