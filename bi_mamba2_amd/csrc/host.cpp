@@ -380,11 +380,13 @@ struct BoundaryCount {
 };
 
 template <typename MakeProblem> ScanResult scan_checked(MakeProblem make, ScanOpts &o, bool keep) {
-    Problem q = make(o);
-    if (!q.p.seq_idx || o.chunk <= max_boundaries) return scan_forward(q, o, keep);
-    BoundaryCount first(q.p, q.x.device().index());
-    ScanResult r = scan_forward(q, o, keep);
-    if (first.wait() <= max_boundaries) return r;
+    {
+        Problem q = make(o);
+        if (!q.p.seq_idx || o.chunk <= max_boundaries) return scan_forward(q, o, keep);
+        BoundaryCount first(q.p, q.x.device().index());
+        ScanResult r = scan_forward(q, o, keep);
+        if (first.wait() <= max_boundaries) return r;
+    }        // (the pass that does not count gives its memory back before the one that does takes its own)
     for (int64_t c : {128, 64, 32}) {
         if (c >= o.chunk) continue;
         o.chunk = c;

@@ -831,8 +831,10 @@ def bimamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_b
         seq_idx: (batch, seqlen) integers, optional - not in the bidirectional reference (its causal sibling has it):
             constant over each of several sequences packed one behind the other; positions with different seq_idx do
             not interact in either direction.  When some chunk would hold more than MAX_SEQ_BOUNDARIES_PER_CHUNK (32)
-            sequence boundaries the call runs with a smaller chunk size (the result does not depend on it), which costs
-            one device-to-host synchronisation per call with seq_idx (chunk_size_for_seq_idx).
+            sequence boundaries the call runs with a smaller chunk size (the result does not depend on it).  The
+            count costs one device-to-host synchronisation per call with seq_idx, behind the pass at the caller's chunk
+            size; a pack that needs a smaller one pays for that pass as well (chunk_size_for_seq_idx tells the size to
+            pass instead).
         grad_places: {"dx": f, "dB": f, "dC": f}, optional - not in the reference: callables asked in the backward pass for
             the tensors these gradients are to be written into (shaped like x / B / C, the two inner dimensions contiguous;
             e.g. slices of one buffer, which saves concatenating them when x, B, C are pieces of one tensor).  A destination

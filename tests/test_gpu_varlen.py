@@ -76,3 +76,25 @@ def test_packed_equals_one_by_one(ops):
         alone = ops.bimamba_chunk_scan_combined(d["x"][:, s], d["dt"][:, s], d["A"], d["B"][:, s], d["C"][:, s], Q,
                                                 z=d["z"][:, s], **kw)
         assert_close(packed[:, s], alone, dtype, f"sequence {i}")
+
+
+@pytest.mark.parametrize("training", [False, True])
+def test_dense_packs_take_no_more_memory(ops, training):
+    """sequences of four positions put 64 boundaries into 256 positions: the call falls back to chunks of 128 after a first pass,
+    whose memory it does not hold on to (24 MB here: the result, the one in front of the gate, the states)"""
+    b, L, H, P = 1, 8192, 8, 64
+    d = to_dev(make_case(b, L, H, P, 1, 64, torch.bfloat16, with_z=True))
+    d["x"].requires_grad_(training)
+    dense, one = (torch.arange(L, device="cuda", dtype=torch.int32)[None].div(n, rounding_mode="floor") for n in (4, L))
+
+    def peak(seq_idx, chunk):
+        torch.cuda.synchronize()
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        out = ops.bimamba_chunk_scan_combined(d["x"], d["dt"], d["A"], d["B"], d["C"], chunk, D=d["D"], z=d["z"], dt_bias=d["dt_bias"],
+                                              dt_softplus=True, seq_idx=seq_idx)
+        return torch.cuda.max_memory_allocated() - before, out.detach()
+
+    (_, _), (wide, _), (narrow, want), (both, got) = (peak(one, 256), peak(one, 256), peak(dense, 128), peak(dense, 256))
+    assert torch.equal(got, want)
+    assert both <= max(wide, narrow) + (4 << 20)         # (large blocks may be given out up to 1 MB larger than asked for)
