@@ -674,18 +674,29 @@ bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const T
     return true;
 }
 
-// Operations up to which the own kernel takes a product whose library call would be as fast or faster on the GPU: the call
-// costs the host 22 us, and up to here the own kernel ends within that time (3.5 GFLOP: 14 us).
-constexpr double OWN_PRODUCT_FLOPS = 5e9;
+// Which products the own kernel takes.  A library call costs the host 22 us more, which counts where a layer is small enough that
+// its kernels do not hide it; the library's kernel is the faster one where the product is large.  One layer of d_model columns
+// and dstate 64 over so many rows in bfloat16, us a pass (eager / replayed graph):
+//   forward products, own up to 1 GFLOP: 197 x 384 (0.25 and 0.12 GFLOP) library 67 / 47, own 51 / 48; 197 x 768 (0.98 and 0.46)
+//     67 / 50, own 55 / 52; 512 x 768 (2.5 and 1.2) 66 / 58, own 63 / 63; 1024 x 768 (5.1 and 2.4) 66 / 65, own for the second 71 / 69;
+//     512 x 1024 (4.5 and 2.2) 66 / 64, own 72 / 73
+//   gradients of the inputs, own up to 5 GFLOP (a training step): 197 x 384 library 241 / 170, own 214 / 163; 512 x 768 240 / 231,
+//     own 230 / 228; 512 x 1024 273 / 270, own 264 / 262; 2048 x 768 (4.8 for the second) 314 / 313, own 316 / 314
+constexpr double OWN_FORWARD_FLOPS = 1e9, OWN_GRADIENT_FLOPS = 5e9;
+
+// From here on the columns of a forward product behind the last multiple of 256 go to the own kernel.  The library works in tiles of
+// 256 columns: where they fill the chip, a tile more for a few columns is a round more, else it is not.  us with 8 / 152 / 248
+// columns over, library alone -> in two: 16384 x 768 by 3072: 123 / 128 / 144 -> 75 / 84 / 86; 8192 x 384 by 2048 (12.9 GFLOP): 36 / 34 / 34
+// -> 24 / 26 / 26; 4096 x 768 by 2048 (12.9): 27 / 26 / 28 -> 26 / 25 / 25; 2048 x 1024 by 3072 (12.9): 23 / 24 / 25 -> 24 / 26 / 27;
+// 8192 x 384 by 1536 (9.7): 27 / 28 / 28 -> 28 / 30 / 31; 4096 x 1024 by 768 (6.4): 16 / 16 / 16 -> 20 / 22 / 22.
+constexpr double SPLIT_FLOPS = 12e9;
 
 // c = x w^T (+ bias): the forward product.  c may be a view with a row pitch.
 void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c) {
-    const double flops = 2.0 * c.size(0) * c.size(1) * x.size(1);
-    if (flops <= OWN_PRODUCT_FLOPS && own_product(x, true, w, true, bias, c)) return;
-    // The library's kernels work at full rate on output columns in multiples of 256 and at half of it otherwise (16384 x 768 by
-    // 3072 columns 72 us, by 3224 columns 147 us): the remaining columns go to the own kernel (16 us there).
+    const double per_column = 2.0 * c.size(0) * x.size(1);
     const int64_t n = c.size(1), whole = n / 256 * 256;
-    if (whole && whole != n && c.scalar_type() != at::kFloat && !bias.defined() &&
+    if (per_column * n <= OWN_FORWARD_FLOPS && own_product(x, true, w, true, bias, c)) return;
+    if (per_column * whole >= SPLIT_FLOPS && whole != n && c.scalar_type() != at::kFloat && !bias.defined() &&
         own_product(x, true, w.narrow(0, whole, n - whole), true, Tensor(), c.narrow(1, whole, n - whole))) {
         Tensor front = c.narrow(1, 0, whole);
         at::mm_out(front, x, w.narrow(0, 0, whole).t());
@@ -697,12 +708,13 @@ void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c) 
 
 // c = dy w: the gradient of a projection's input
 void product_nn(const Tensor &dy, const Tensor &w, Tensor c) {
-    if (2.0 * c.size(0) * c.size(1) * dy.size(1) <= OWN_PRODUCT_FLOPS && own_product(dy, true, w, false, Tensor(), c)) return;
+    if (2.0 * c.size(0) * c.size(1) * dy.size(1) <= OWN_GRADIENT_FLOPS && own_product(dy, true, w, false, Tensor(), c)) return;
     at::mm_out(c, dy, w);
 }
 
 // c = dy^T x: the gradient of a projection's weight.  Always the own kernel where it exists: the library does not cut the long
-// sum over the rows (3224 x 768 over 16384 rows: 157 us against 93).
+// sum over the rows.  us, library -> own: 3224 x 768 over 16384 rows 149 -> 94, over 4096 43 -> 35, over 1024 16 -> 19, over 197
+// 10 -> 10; 768 x 1536 122 -> 51, 34 -> 25, 13 -> 12, 8 -> 7; 4384 x 1024 over 65536 693 -> 554; 644 x 128 over 4096 31 -> 11.
 void product_tn(const Tensor &dy, const Tensor &x, Tensor c) {
     if (own_product(dy, false, x, false, Tensor(), c)) return;
     at::mm_out(c, dy.t(), x);

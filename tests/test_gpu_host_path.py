@@ -14,6 +14,9 @@ LAYERS = [
     (1, 1, dict(d_model=64, d_state=16, headdim=32, ngroups=2), torch.float32, False, ("A_log", "conv1d.weight")),
     (2, 300, dict(d_model=128, d_state=64, headdim=64), torch.bfloat16, True, ("in_proj.weight", "norm.weight", "D")),
     (1, 257, dict(d_model=128, d_state=128, headdim=64, conv_bias=False), torch.float16, False, ("out_proj.weight",)),
+    # in_proj as one library product (1.6 GFLOP), and with its last 144 columns by the own kernel (2048 columns: 12.2 GFLOP)
+    (1, 700, dict(d_model=512), torch.bfloat16, False, ()),
+    (2, 2900, dict(d_model=512), torch.bfloat16, False, ()),
 ]
 
 
