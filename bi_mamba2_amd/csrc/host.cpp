@@ -674,29 +674,33 @@ bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const T
     return true;
 }
 
-// Which products the own kernel takes.  A library call costs the host 22 us more, which counts where a layer is small enough that
-// its kernels do not hide it; the library's kernel is the faster one where the product is large.  One layer of d_model columns
-// and dstate 64 over so many rows in bfloat16, us a pass (eager / replayed graph):
-//   forward products, own up to 1 GFLOP: 197 x 384 (0.25 and 0.12 GFLOP) library 67 / 47, own 51 / 48; 197 x 768 (0.98 and 0.46)
-//     67 / 50, own 55 / 52; 512 x 768 (2.5 and 1.2) 66 / 58, own 63 / 63; 1024 x 768 (5.1 and 2.4) 66 / 65, own for the second 71 / 69;
-//     512 x 1024 (4.5 and 2.2) 66 / 64, own 72 / 73
-//   gradients of the inputs, own up to 5 GFLOP (a training step): 197 x 384 library 241 / 170, own 214 / 163; 512 x 768 240 / 231,
-//     own 230 / 228; 512 x 1024 273 / 270, own 264 / 262; 2048 x 768 (4.8 for the second) 314 / 313, own 316 / 314
-constexpr double OWN_FORWARD_FLOPS = 1e9, OWN_GRADIENT_FLOPS = 5e9;
+// Which products the own kernel takes, in operations.  A library call costs the host 18 us, which shows where a layer's kernels do not
+// hide it: a forward pass without gradients up to some 65 us, a training step up to some 230.  Where the host is hidden, or a
+// replayed graph does without it, the library's kernel is the faster one of the large products.  One layer of dstate 64 in bfloat16
+// over rows x d_model, us a pass with the library -> with the own kernel (eager, as a replayed graph):
+//   without gradients: 197 x 384 (0.25 and 0.12 GFLOP) 67 -> 51, 47 -> 48; 197 x 768 (0.98 and 0.46) 67 -> 55, 50 -> 52; 1024 x 384 (1.3
+//     and 0.6) 67 -> 58, 56 -> 56; above the line 1024 x 768 (5.1, 2.4) 66 -> 70, 65 -> 70 for the second, 512 x 1024 (4.5, 2.2) 65 -> 72, 64 -> 73
+//   forward products of a training step: 2048 x 384 (2.6, 1.2) 255 -> 228, 223 -> 223; 1024 x 576 (2.9, 1.4) 247 -> 232, 227 -> 229; 512 x 1024
+//     (4.5, 2.2) 257 -> 262, 251 -> 259 for the second; above the line 2048 x 768 (10, 4.8) 308 -> 315, 307 -> 314
+//   gradients of the inputs: 197 x 384 241 -> 214, 170 -> 163; 512 x 768 240 -> 230, 231 -> 228; 512 x 1024 273 -> 264, 270 -> 262; 2048 x 768 (4.8 for
+//     the second) 314 -> 316, 313 -> 314
+constexpr double OWN_INFERENCE_FLOPS = 1.5e9, OWN_TRAINING_FLOPS = 3e9, OWN_GRADIENT_FLOPS = 5e9;
 
-// From here on the columns of a forward product behind the last multiple of 256 go to the own kernel.  The library works in tiles of
-// 256 columns: where they fill the chip, a tile more for a few columns is a round more, else it is not.  us with 8 / 152 / 248
-// columns over, library alone -> in two: 16384 x 768 by 3072: 123 / 128 / 144 -> 75 / 84 / 86; 8192 x 384 by 2048 (12.9 GFLOP): 36 / 34 / 34
-// -> 24 / 26 / 26; 4096 x 768 by 2048 (12.9): 27 / 26 / 28 -> 26 / 25 / 25; 2048 x 1024 by 3072 (12.9): 23 / 24 / 25 -> 24 / 26 / 27;
-// 8192 x 384 by 1536 (9.7): 27 / 28 / 28 -> 28 / 30 / 31; 4096 x 1024 by 768 (6.4): 16 / 16 / 16 -> 20 / 22 / 22.
-constexpr double SPLIT_FLOPS = 12e9;
+// From so many rows or operations on, the columns of a forward product behind the last multiple of 256 go to the own kernel where the
+// number of columns is no multiple of 64: the library has fast kernels for some of these numbers only.  us, library alone -> in
+// two: 16384 x 768 by 3224 columns 128 -> 84; 24063 x 384 by 2060 109 -> 73; 4715 x 832 by 3482 53 -> 36; 19687 x 128 by 772 47 -> 20; but 5044 x 448
+// by 1934 27 -> 33, 8931 x 704 by 2966 58 -> 71.  315 such products of layers of 128 to 1024 columns, operands from memory, above 1
+// GFLOP: 0.92 of the library's time (0.89 with the better of both each time).  Fewer rows: 3233 x 896 by 3740 35 -> 48, 1658 x 768 by 3352
+// 20 -> 27.  A multiple of 64 columns stays whole at any size: 188 products would take 1.2 times as long (15642 x 768 by 384 18 -> 35).
+constexpr int64_t SPLIT_ROWS = 4096;
+constexpr double SPLIT_FLOPS = 25e9;
 
 // c = x w^T (+ bias): the forward product.  c may be a view with a row pitch.
-void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c) {
-    const double per_column = 2.0 * c.size(0) * x.size(1);
-    const int64_t n = c.size(1), whole = n / 256 * 256;
-    if (per_column * n <= OWN_FORWARD_FLOPS && own_product(x, true, w, true, bias, c)) return;
-    if (per_column * whole >= SPLIT_FLOPS && whole != n && c.scalar_type() != at::kFloat && !bias.defined() &&
+void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c, bool training) {
+    const int64_t m = c.size(0), n = c.size(1), whole = n / 256 * 256;
+    const double per_column = 2.0 * m * x.size(1);
+    if (per_column * n <= (training ? OWN_TRAINING_FLOPS : OWN_INFERENCE_FLOPS) && own_product(x, true, w, true, bias, c)) return;
+    if ((m >= SPLIT_ROWS || per_column * whole >= SPLIT_FLOPS) && n % 64 && whole && c.scalar_type() != at::kFloat && !bias.defined() &&
         own_product(x, true, w.narrow(0, whole, n - whole), true, Tensor(), c.narrow(1, whole, n - whole))) {
         Tensor front = c.narrow(1, 0, whole);
         at::mm_out(front, x, w.narrow(0, 0, whole).t());
@@ -730,7 +734,7 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
     void *stream = stream_of(u);
     const Tensor u2 = u.reshape({s.rows, u.size(2)});
     const Tensor zx_rows = device_empty({s.rows, s.pitch}, u.scalar_type(), u), zx = zx_rows.narrow(1, 0, s.proj);
-    product_nt(u2, w_in, b_in, zx);
+    product_nt(u2, w_in, b_in, zx, keep);
     o.converted = params_to_convert(prm);
     const Params32 w = params_as_float32(prm, o.converted, stream);
 
@@ -764,7 +768,7 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
     }
     check(api.norm_fwd(&n), "bimamba2_rmsnorm_gated_fwd");
     const Tensor out = device_empty({s.batch, s.seqlen, w_out.size(0)}, u.scalar_type(), u);
-    product_nt(yn, w_out, b_out, out.view({s.rows, w_out.size(0)}));
+    product_nt(yn, w_out, b_out, out.view({s.rows, w_out.size(0)}), keep);
     if (left) *left = {zx_rows, xbc, y, yn, rstd, kept, w.buf};
     return out;
 }
