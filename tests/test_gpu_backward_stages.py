@@ -188,3 +188,29 @@ def test_dz_and_dstates_in_one_launch(ops, case):
     assert torch.equal(dpf1, dpf) and torch.equal(dpb1, dpb)
     with pytest.raises(ValueError):                             # float32: the two separate kernels only (unsupported)
         ops._chunk_scan_bwd_dz_dstates(z.float(), out_x.float(), dout.float(), C.float(), csf, csb)
+
+
+@pytest.mark.parametrize("N,dtype,z", [(64, torch.bfloat16, True), (128, torch.bfloat16, False), (128, torch.float16, True)])
+def test_dcb_between_the_merged_launches_in_sixteen_bits(ops, monkeypatch, N, dtype, z):
+    """Inside bimamba2_bwd dCB travels in the operands' type, at state dimension 128 too: its reader rounded the float32 values to
+    that type before its product anyway, so a caller who brings float32 dCB and dCBT gets the same bits."""
+    b, L, H, P, G, Q = 2, 600, 8, 64, 2, 256
+    d = to_dev(make_case(b, L, H, P, G, N, dtype, with_z=z))
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(7)).to(dtype).cuda()
+    args = (d["x"], d["dt"], d["A"], d["B"], d["C"])
+    kw = dict(D=d["D"], z=d["z"], dt_bias=d["dt_bias"], dt_softplus=True)
+    res = ops._mamba_chunk_scan_combined_fwd(*args, Q, return_intermediates=False, keep_for_bwd=True, **kw)
+
+    def bwd():
+        return ops._mamba_chunk_scan_combined_bwd(dout, *args, res[1], Q, saved=res[9], **kw)
+
+    own, ws = bwd(), ops._Call.workspace
+
+    def with_dcb(call, is_bwd):
+        for field in ("dCB", "dCBT"):
+            call.new(field, (b, -(-L // Q), G, Q, Q))
+        return ws(call, is_bwd)
+
+    monkeypatch.setattr(ops._Call, "workspace", with_dcb)
+    for a, c in zip(own, bwd()):
+        assert (a is None and c is None) or torch.equal(a, c)
