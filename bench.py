@@ -426,7 +426,7 @@ def layer_line(dev, steps, warmup, spin=False):
             "eager_ms_per_step": round(t_eager * 1e3, 4), "fwd_ms": round(t_fwd * 1e3, 4),
             "operator_ms_per_step": round(t_op * 1e3, 4), "operator_share": round(t_op / t, 3),
             "rest": "in_proj / out_proj products (this library's kernel and hipBLASLt), conv1d + SiLU and gated RMSNorm (this library's kernels), "
-                    "splits and the dt_bias / A_log parameter maps (torch)"}
+                    "the parameter maps (one launch each way); the splits are views"}
 
 
 def main():
