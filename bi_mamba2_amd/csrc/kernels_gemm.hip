@@ -4,7 +4,7 @@
 //
 // Either operand may have k contiguous in memory (x and W of a forward product) or its rows contiguous (W in an input
 // gradient, both operands of a weight gradient).  What it replaces at these places is a library product whose call costs the
-// host 22 us - more than the product at small sizes - and whose weight gradients (few output tiles, a long sum) ran at 330 to
+// host 18 to 22 us - more than the product at small sizes - and whose weight gradients (few output tiles, a long sum) ran at 330 to
 // 460 TFLOP/s.
 //
 // A workgroup owns a BM x BN tile and goes through k in steps of 32.  The operand tiles of a step travel straight into a ring

@@ -46,3 +46,41 @@ def test_forward_backward_replays_match_eager(shape):
         torch.cuda.synchronize()
         for name, a, e in zip(("out",) + tuple("d" + k for k in names), captured, eager):
             assert torch.equal(a, e), f"replay {rep}: {name} differs from the eager result"
+
+
+# the layer with its products by the own kernel, as whole library products, and cut in two (d_model 512: 2192 columns)
+@pytest.mark.parametrize("rows,d_model,training", [(200, 384, True), (1024, 768, False), (1500, 512, True), (4100, 512, True), (4100, 512, False)])
+def test_layer_replays_match_eager(rows, d_model, training):
+    from bi_mamba2_amd.modules import BiMamba2
+    torch.manual_seed(0)
+    m = BiMamba2(d_model=d_model).cuda().to(torch.bfloat16)
+    params = [p for n, p in m.named_parameters() if not n.startswith("fc_D")]
+    static = torch.randn(1, rows, d_model, device="cuda").bfloat16().requires_grad_(training)
+    dy = torch.randn_like(static)
+
+    def step(u):
+        if not training:
+            with torch.no_grad():
+                return (m(u),)
+        out = m(u)
+        return (out.detach(),) + torch.autograd.grad(out, [u] + params, dy)
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(3):
+            step(static)
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        captured = step(static)
+    for rep in range(4):
+        fresh = torch.randn(1, rows, d_model, device="cuda").bfloat16()
+        with torch.no_grad():
+            static.copy_(fresh)
+        graph.replay()
+        torch.cuda.synchronize()
+        for i, (a, e) in enumerate(zip(captured, step(fresh.requires_grad_(training)))):
+            assert torch.equal(a, e), f"replay {rep}: output {i} differs from the eager result by {(a.float() - e.float()).norm() / e.float().norm()}"
+        torch.cuda.synchronize()
