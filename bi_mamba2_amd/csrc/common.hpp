@@ -450,18 +450,18 @@ __device__ __forceinline__ float row16_max(float v) {
     return v;
 }
 // inclusive prefix / suffix sums over the 64 lanes
-__device__ __forceinline__ float wave_incl_prefix(float v, int lane) {
+template <typename F> __device__ __forceinline__ F wave_incl_prefix(F v, int lane) {
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        float o = __shfl_up(v, d, 64);
+        const F o = __shfl_up(v, d, 64);
         if (lane >= d) v += o;
     }
     return v;
 }
-__device__ __forceinline__ float wave_incl_suffix(float v, int lane) {
+template <typename F> __device__ __forceinline__ F wave_incl_suffix(F v, int lane) {
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) {
-        float o = __shfl_down(v, d, 64);
+        const F o = __shfl_down(v, d, 64);
         if (lane + d < 64) v += o;
     }
     return v;

@@ -1968,6 +1968,22 @@ int launch_bwd_dcb(const bimamba2_params *p) {
 // of a thread (its dCB row pieces, the slices it adds, the K operand) is requested before the first one is used.
 
 
+// A float32 operand of a 16-bit product as two 16-bit ones, the value rounded and what the rounding left: dCB in float32 enters
+// with 16 (22) bits instead of 8 (11).  The kernel waits for memory, the second product costs it nothing that can be measured,
+// and dB and dC are a fifth closer to the exact ones.
+template <typename T> __device__ __forceinline__ void split_operand(const float (&v)[Mma<T>::KPL], typename Mma<T>::Frag &hi, typename Mma<T>::Frag &rest) {
+    hi = Mma<T>::pack(v);
+    if constexpr (sizeof(T) == 2) {
+        float r[Mma<T>::KPL];
+#pragma unroll
+        for (int i = 0; i < Mma<T>::KPL; ++i) {
+            const float h = to_f(from_f<T>(v[i]));
+            r[i] = __builtin_isfinite(h) ? v[i] - h : 0.f;          // (what overflows the 16-bit type stays an infinity)
+        }
+        rest = Mma<T>::pack(r);
+    }
+}
+
 // SLIM (with FAST): dCB / dCBT hold 16-bit elements (in16) and there are at most two slices to add: a quarter of the
 // registers, and the staging tile of the result shares the LDS of the K operand, so that three workgroups fit a CU where
 // the general variant fits two (with few heads per group the launch has thousands of workgroups: 83 -> 76 us at 8 groups
@@ -2042,17 +2058,23 @@ __device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int
 #pragma unroll
         for (int s = 0; s < NS; ++s) {
             if (s * KSTEP < limit) {
-                typename M::Frag af;
+                // (chunks of 256 take dCB in 16 bits where it is bimamba2_bwd's own, and give the same bits where a caller brings it)
+                constexpr bool SPLIT = QP < 256 && !SLIM;
+                typename M::Frag af, rest{};
                 if constexpr (SLIM) {
                     static_assert(!SLIM || sizeof(typename M::Frag) == 16, "16-bit operands");
                     af = __builtin_bit_cast(typename M::Frag, raw[s][0]);
                 } else {
                     float v[KPL] = {raw[s][0].x, raw[s][0].y, raw[s][0].z, raw[s][0].w, raw[s][1].x, raw[s][1].y, raw[s][1].z, raw[s][1].w};
-                    if constexpr (sizeof(typename M::Frag) == 16) af = in16 ? __builtin_bit_cast(typename M::Frag, raw[s][0]) : M::pack(v);
-                    else af = M::pack(v);
+                    if constexpr (SPLIT) split_operand<T>(v, af, rest);
+                    else if constexpr (sizeof(typename M::Frag) == 16) af = in16 ? __builtin_bit_cast(typename M::Frag, raw[s][0]) : M::pack(v);
                 }
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[j] = M::mma(af, M::load(kT + xt_index<T, LDX>(j * 16 + lr, s * KSTEP + lg * KPL)), acc[j]);
+                for (int j = 0; j < 4; ++j) {
+                    const typename M::Frag bf = M::load(kT + xt_index<T, LDX>(j * 16 + lr, s * KSTEP + lg * KPL));
+                    acc[j] = M::mma(af, bf, acc[j]);
+                    if constexpr (SPLIT) acc[j] = M::mma(rest, bf, acc[j]);
+                }
             }
         }
         float4 sw[NIT][HSL][2] = {};
@@ -2117,9 +2139,14 @@ __device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int
 #pragma unroll
             for (int i = 0; i < KPL; ++i) v[i] = kb + i < Q ? arow[kb + i] : 0.f;
         }
-        const typename M::Frag af = M::pack(v);
+        typename M::Frag af, rest{};
+        split_operand<T>(v, af, rest);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[j] = M::mma(af, M::load(kT + xt_index<T, LDX>(j * 16 + lr, kb)), acc[j]);
+        for (int j = 0; j < 4; ++j) {
+            const typename M::Frag bf = M::load(kT + xt_index<T, LDX>(j * 16 + lr, kb));
+            acc[j] = M::mma(af, bf, acc[j]);
+            if constexpr (sizeof(T) == 2) acc[j] = M::mma(rest, bf, acc[j]);
+        }
     }
     // pass the tile through LDS so that the slices are read and the result is written
     // as 16-byte vectors along dstate

@@ -13,7 +13,10 @@ namespace bm2 {
 // =========================================================================================================
 // chunk cumsum: one wave per (b, c, h); lane i owns positions 4i..4i+3 of the chunk (Q <= 256)
 // =========================================================================================================
-template <typename DT>
+// ACC: the type of the sums.  float32 problems take them in 64 bits and round once: a result there is off by little else than the
+// resolution of these sums (their differences are exponents), and with every addition rounded it was off by 1.7 times as much.
+// 16-bit results are not, and 64 bits would cost them 2 of 13 us over 2 x 16384 positions of 48 heads.
+template <typename DT, typename ACC>
 __global__ __launch_bounds__(NTHREADS) void chunk_cumsum_fwd_kernel(const bimamba2_params p, int nc) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = blockIdx.x * 4 + wave, c = blockIdx.y, b = blockIdx.z;
@@ -23,7 +26,8 @@ __global__ __launch_bounds__(NTHREADS) void chunk_cumsum_fwd_kernel(const bimamb
     const DT *dt = reinterpret_cast<const DT *>(p.dt) + b * p.dt_sb + (int64_t)c * Q * p.dt_sl + h * p.dt_sh;
     const float A = p.A[h];
     const float bias = p.has_dt_bias ? p.dt_bias[h] : 0.f;
-    float v[4], a[4], ar[4];                          // ar: exponents of the reverse direction (differ with seq_idx only)
+    float v[4];
+    ACC a[4], ar[4];                                  // ar: exponents of the reverse direction (differ with seq_idx only)
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int q = lane * 4 + e;
@@ -34,7 +38,7 @@ __global__ __launch_bounds__(NTHREADS) void chunk_cumsum_fwd_kernel(const bimamb
             d = fminf(fmaxf(d, p.dt_min), p.dt_max);
         }
         v[e] = d;
-        a[e] = ar[e] = d * A;
+        a[e] = ar[e] = (ACC)d * A;
         if (p.seq_idx && q < limit) {
             // packed sequences: cut the forward recurrence in front of a sequence's first position, the reverse one
             // behind its last
@@ -46,21 +50,18 @@ __global__ __launch_bounds__(NTHREADS) void chunk_cumsum_fwd_kernel(const bimamb
         }
     }
     // forward inclusive scan, reverse inclusive scan
-    float pf[4], sb[4];
+    ACC pf[4], sb[4];
     pf[0] = a[0]; pf[1] = pf[0] + a[1]; pf[2] = pf[1] + a[2]; pf[3] = pf[2] + a[3];
     sb[3] = ar[3]; sb[2] = sb[3] + ar[2]; sb[1] = sb[2] + ar[1]; sb[0] = sb[1] + ar[0];
-    const float tot = pf[3], tot_r = sb[0];
-    const float incl = wave_incl_prefix(tot, lane);
-    const float before = incl - tot;
-    const float incl_s = wave_incl_suffix(tot_r, lane);
-    const float after = incl_s - tot_r;
+    const ACC tot = pf[3], tot_r = sb[0];
+    const ACC before = wave_incl_prefix(tot, lane) - tot, after = wave_incl_suffix(tot_r, lane) - tot_r;
     const int64_t o = (((int64_t)b * p.nheads + h) * nc + c) * Q;
     if (Q % 4 == 0) {
         // a lane's four positions are contiguous: 16-byte stores (the three tensors are contiguous and Q * 4 bytes per row)
         if (lane * 4 < Q) {
             *reinterpret_cast<f32x4 *>(p.dt_out + o + lane * 4) = f32x4{v[0], v[1], v[2], v[3]};
-            *reinterpret_cast<f32x4 *>(p.cs_f + o + lane * 4) = f32x4{before + pf[0], before + pf[1], before + pf[2], before + pf[3]};
-            *reinterpret_cast<f32x4 *>(p.cs_b + o + lane * 4) = f32x4{after + sb[0], after + sb[1], after + sb[2], after + sb[3]};
+            *reinterpret_cast<f32x4 *>(p.cs_f + o + lane * 4) = f32x4{(float)(before + pf[0]), (float)(before + pf[1]), (float)(before + pf[2]), (float)(before + pf[3])};
+            *reinterpret_cast<f32x4 *>(p.cs_b + o + lane * 4) = f32x4{(float)(after + sb[0]), (float)(after + sb[1]), (float)(after + sb[2]), (float)(after + sb[3])};
         }
         return;
     }
@@ -69,8 +70,8 @@ __global__ __launch_bounds__(NTHREADS) void chunk_cumsum_fwd_kernel(const bimamb
         const int q = lane * 4 + e;
         if (q < Q) {
             p.dt_out[o + q] = v[e];
-            p.cs_f[o + q] = before + pf[e];
-            p.cs_b[o + q] = after + sb[e];
+            p.cs_f[o + q] = (float)(before + pf[e]);
+            p.cs_b[o + q] = (float)(after + sb[e]);
         }
     }
 }
@@ -785,12 +786,18 @@ static inline hipStream_t stream_of(const bimamba2_params *p) { return reinterpr
 int launch_chunk_cumsum_fwd(const bimamba2_params *p) {
     const int nc = nchunks(p);
     dim3 grid((p->nheads + 3) / 4, nc, p->batch);
+#define BM2_CS(DT)                                                                                                                          \
+    do {                                                                                                                                    \
+        if (p->dtype == BIMAMBA2_F32) hipLaunchKernelGGL((chunk_cumsum_fwd_kernel<DT, double>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc); \
+        else hipLaunchKernelGGL((chunk_cumsum_fwd_kernel<DT, float>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc);                       \
+    } while (0)
     switch (p->dt_dtype) {
-        case BIMAMBA2_F32: hipLaunchKernelGGL(chunk_cumsum_fwd_kernel<float>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc); break;
-        case BIMAMBA2_BF16: hipLaunchKernelGGL(chunk_cumsum_fwd_kernel<bf16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc); break;
-        case BIMAMBA2_F16: hipLaunchKernelGGL(chunk_cumsum_fwd_kernel<f16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc); break;
+        case BIMAMBA2_F32: BM2_CS(float); break;
+        case BIMAMBA2_BF16: BM2_CS(bf16_t); break;
+        case BIMAMBA2_F16: BM2_CS(f16_t); break;
         default: return BIMAMBA2_EUNSUPPORTED;
     }
+#undef BM2_CS
     return check_launch();
 }
 

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
     constexpr int STG_BYTES = SCAN_WAVES * 16 * SLD * 4;
     // the operand images (xT and the two state tiles) and the per-wave epilogue staging patches are never live together
     __shared__ __attribute__((aligned(16))) char shared_u[XT_BYTES + ST_BYTES > STG_BYTES ? XT_BYTES + ST_BYTES : STG_BYTES];
-    __shared__ float lo[QP], up[QP];              // decay exponents (times log2 e), see below
+    __shared__ __attribute__((aligned(16))) float lo[QP], up[QP];   // decay exponents, see below
     __shared__ float glo[QP], gup[QP];            // their column factors relative to the edge of the 16-block, see below
     __shared__ float dtl[BWD ? 4 : QP];           // forward: dt of the columns, for the step across the diagonal
     __shared__ float red[SCAN_WAVES][PW];
@@ -115,27 +115,28 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
     if (BWD) { as = p.B_sl; ap = reinterpret_cast<const T *>(p.Bm) + b * p.B_sb + (int64_t)c * Q * as + g * p.B_sg; }
     else { as = p.C_sl; ap = reinterpret_cast<const T *>(p.Cm) + b * p.C_sb + (int64_t)c * Q * as + g * p.C_sg; }
     const bool avec = aligned16(ap, as) && (N % VS == 0);
-    float arow[QT][NW / KSTEP][KPL];               // rows of the first NW dstate columns, requested up front
+    // rows of NW dstate columns, as they are (the row factors go onto the accumulators: a factor on a 16-bit operand would be
+    // one more rounding of it), the first ones requested up front
+    typename M::Frag own[QT][NW / KSTEP];
     auto load_arows = [&](int n0) {
 #pragma unroll
         for (int rt = 0; rt < QT; ++rt)
 #pragma unroll
             for (int s = 0; s < NW / KSTEP; ++s) {
                 const int r = rowi[rt], kb = n0 + s * KSTEP + lg * KPL;
-                if (FAST) {
+                if (NF > 0) own[rt][s] = M::load(ap + (int64_t)min(r, limit - 1) * as + kb);
+                else if (FAST) {
                     // (zeros behind the state dimension by masking the 16 bytes: a select per element cost the kernel 20 of 55 us)
                     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
                     const u32x4 bits = *reinterpret_cast<const u32x4 *>(ap + (int64_t)min(r, limit - 1) * as + min(kb, N - KPL));
-                    const Vec16<T> raw = __builtin_bit_cast(Vec16<T>, bits & (kb < N ? ~0u : 0u));
-#pragma unroll
-                    for (int i = 0; i < KPL; ++i) arow[rt][s][i] = to_f(raw.v[i]);
+                    own[rt][s] = __builtin_bit_cast(typename M::Frag, bits & (kb < N ? ~0u : 0u));
                 } else if (r < limit && avec && kb + KPL <= N) {
-                    Vec16<T> raw = *reinterpret_cast<const Vec16<T> *>(ap + (int64_t)r * as + kb);
-#pragma unroll
-                    for (int i = 0; i < KPL; ++i) arow[rt][s][i] = to_f(raw.v[i % Vec16<T>::N]);
+                    own[rt][s] = M::load(ap + (int64_t)r * as + kb);
                 } else {
+                    float v[KPL];
 #pragma unroll
-                    for (int i = 0; i < KPL; ++i) arow[rt][s][i] = (r < limit && kb + i < N) ? to_f(ap[(int64_t)r * as + kb + i]) : 0.f;
+                    for (int i = 0; i < KPL; ++i) v[i] = (r < limit && kb + i < N) ? to_f(ap[(int64_t)r * as + kb + i]) : 0.f;
+                    own[rt][s] = M::pack(v);
                 }
             }
     };
@@ -143,19 +144,21 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
     // forward: k<r uses lo[r]-lo[k] with lo = cs_f, k>r uses up[r]-up[k] with up = cs_b
     // mirror : k<r uses e^{cs_b[k]-cs_b[r]} -> lo = -cs_b;  k>r uses e^{cs_f[k]-cs_f[r]} -> up = -cs_f
     // Away from the diagonal the factor separates: with m = lo at the last position of k's block of 16 (which lies
-    // between k and r), 2^{lo[r]-lo[k]} = 2^{lo[r]-m} * glo[k], glo[k] = 2^{m-lo[k]}, both factors <= 1 for A <= 0;
-    // likewise gup[k] = 2^{up[first of k's block] - up[k]}.  One exponential per lane and K step instead of one per element.
+    // between k and r), e^{lo[r]-lo[k]} = e^{lo[r]-m} * glo[k], glo[k] = e^{m-lo[k]}, both factors <= 1 for A <= 0;
+    // likewise gup[k] = e^{up[first of k's block] - up[k]}.  One exponential per lane and K step instead of one per element.
+    // (The sums stay as they are here and only their differences are scaled to base 2: scaled first, each would be rounded
+    // once more at the size of the sum, which is most of what a float32 result is off by.)
     for (int q = threadIdx.x; q < QP; q += SCAN_THREADS) {
         const int qq = min(q, Q - 1), qe = min(q | 15, Q - 1), qs = min(q & ~15, Q - 1);
-        const float f = csf[qq] * LOG2E, r = csb[qq] * LOG2E;
+        const float f = csf[qq], r = csb[qq];
         const float l = BWD ? -r : f, u = BWD ? -f : r;
         lo[q] = l;
         up[q] = u;
         // forward: dt[k] of the source position rides on the column factors (and on the diagonal step through dtl), so
         // that the operand image holds x as it is and the D term can take x from there
         const float dtq = BWD ? 1.f : dto[qq];
-        glo[q] = __builtin_amdgcn_exp2f((BWD ? -csb[qe] : csf[qe]) * LOG2E - l) * dtq;
-        gup[q] = __builtin_amdgcn_exp2f((BWD ? -csf[qs] : csb[qs]) * LOG2E - u) * dtq;
+        glo[q] = __expf((BWD ? -csb[qe] : csf[qe]) - l) * dtq;
+        gup[q] = __expf((BWD ? -csf[qs] : csb[qs]) - u) * dtq;
         if (!BWD) dtl[q] = dtq;
     }
     // K operand of part 2, transposed into LDS
@@ -166,36 +169,52 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
     else { ks = p.dout_sl; kp = reinterpret_cast<const T *>(p.dout) + b * p.dout_sb + (int64_t)c * Q * ks + h * p.dout_sh; }
     stage_transposed<T, QP, PW, LDX, FAST>(xT, kp + p0, ks, limit, P - p0, [&](int k) { return k < limit ? 1.f : 0.f; });
 
-    typename M::Frag own[QT][NF > 0 ? NF : 1];     // NF > 0: this lane's rows, 32 dstate columns per fragment
-    if constexpr (NF > 0) {
-#pragma unroll
-        for (int rt = 0; rt < QT; ++rt)
-#pragma unroll
-            for (int f = 0; f < NF; ++f) own[rt][f] = M::load(ap + (int64_t)min(rowi[rt], limit - 1) * as + f * KSTEP + lg * KPL);
-    } else {
-        load_arows(0);
-    }
+    // (two row tiles of four column tiles have no registers to hold them over the loads of the state tiles)
+    constexpr bool ROWS_FIRST = NF > 0 || QT * NJ <= 4;
+    if (ROWS_FIRST) load_arows(0);
     f32x4 acc[QT][NJ] = {};
 
     // ---- part 1: states.  A = (C or B rows) * row scale, K = dstate; B operand = state tiles [p][n] in LDS ----
     {
         const int64_t so = ((int64_t)(b * nc + c) * H + h) * P * N + (int64_t)p0 * N;
         const float *stf = (BWD ? p.dstates_f : p.states_f) + so, *stb = (BWD ? p.dstates_b : p.states_b) + so;
-        float rsf[QT], rsb[QT];
+        // one direction's product of the rows with the state tile in LDS, scaled row by row (rows 4*(l/16)+i of each tile) on
+        // its way to acc; one direction after the other, and without CB fragments to spare registers for also one row tile
+        // after the other, to keep one small set of temporaries (both row tiles at once: 32 registers spilled)
+        constexpr int RT = NF == 0 && QT * NJ > 4 ? 1 : QT;
+        auto state_product = [&](int dir, int nleft) __attribute__((always_inline)) {
+            const T *st = dir ? sB : sF;
+            // forward: e^{cs_f[r]}, e^{cs_b[r]}; mirror: e^{cs_f[Q-1] - cs_f[r]}, e^{cs_b[0] - cs_b[r]} (lo, up: see above)
+            const float ref = BWD ? (dir ? lo[0] : up[Q - 1]) : 0.f;
+            const float *tab = BWD ? (dir ? lo : up) : (dir ? up : lo);
 #pragma unroll
-        for (int rt = 0; rt < QT; ++rt) {
-            const int r = rowi[rt];
-            float ef = 0.f, eb = 0.f;
-            if (r < limit) {
-                ef = BWD ? __expf(csf[Q - 1] - csf[r]) : __expf(csf[r]);
-                eb = BWD ? __expf(csb[0] - csb[r]) : __expf(csb[r]);
+            for (int r0 = 0; r0 < QT; r0 += RT) {
+                if (RT < QT) __builtin_amdgcn_sched_barrier(0);
+                f32x4 tmp[RT][NJ] = {};
+#pragma unroll
+                for (int s = 0; s < NW / KSTEP; ++s) {
+                    if (NF == 0 && s * KSTEP >= nleft) break;
+                    typename M::Frag bfs[NJ];
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) bfs[j] = M::load(st + (j * 16 + lr) * LDS_ + s * KSTEP + lg * KPL);
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) tmp[rt][j] = M::mma(own[r0 + rt][s], bfs[j], tmp[rt][j]);
+                }
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt) {
+                    const f32x4 cs4 = *reinterpret_cast<const f32x4 *>(tab + (wave * QT + r0 + rt) * 16 + lg * 4);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const float e = __expf(cs4[i] - ref);
+#pragma unroll
+                        for (int j = 0; j < NJ; ++j) acc[r0 + rt][j][i] = __builtin_fmaf(tmp[rt][j][i], e, acc[r0 + rt][j][i]);
+                    }
+                }
             }
-            rsf[rt] = ef;
-            rsb[rt] = eb;
-        }
+        };
         if constexpr (NF > 0) {
-            // raw rows as the A operand; the row factors go onto the accumulators (rows 4*(l/16)+i of each tile).
-            // One direction after the other, to keep one set of temporaries.
             static_assert(NF == 0 || NF * KSTEP == NW, "one round of state tiles");
             // full 64 x 64 float tiles (the launcher checked it): every 16-byte load of both tiles goes out
             // before the first one is converted
@@ -230,37 +249,13 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
                 }
             }
             __syncthreads();
-#pragma unroll
-            for (int dir = 0; dir < (UNI ? 1 : 2); ++dir) {
-                const T *st = dir ? sB : sF;
-                f32x4 tmp[QT][NJ] = {};
-#pragma unroll
-                for (int s = 0; s < NW / KSTEP; ++s) {
-                    typename M::Frag bfs[NJ];
-#pragma unroll
-                    for (int j = 0; j < NJ; ++j) bfs[j] = M::load(st + (j * 16 + lr) * LDS_ + s * KSTEP + lg * KPL);
-#pragma unroll
-                    for (int rt = 0; rt < QT; ++rt)
-#pragma unroll
-                        for (int j = 0; j < NJ; ++j) tmp[rt][j] = M::mma(own[rt][s], bfs[j], tmp[rt][j]);
-                }
-#pragma unroll
-                for (int rt = 0; rt < QT; ++rt)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        const int r = (wave * QT + rt) * 16 + lg * 4 + i, rc = min(r, limit - 1);
-                        const float *cs = dir ? csb : csf;
-                        float e = BWD ? __expf(cs[dir ? 0 : Q - 1] - cs[rc]) : __expf(cs[rc]);
-                        if (r >= limit) e = 0.f;
-#pragma unroll
-                        for (int j = 0; j < NJ; ++j) acc[rt][j][i] = dir ? __builtin_fmaf(tmp[rt][j][i], e, acc[rt][j][i]) : tmp[rt][j][i] * e;
-                    }
-            }
+            state_product(0, NW);
+            if (!UNI) state_product(1, NW);
         } else
         for (int n0 = 0; n0 < N; n0 += NW) {
             if (n0) {
                 __syncthreads();
-                load_arows(n0);
+                if (ROWS_FIRST) load_arows(n0);
             }
             if (sizeof(T) == 2 && !BWD && p.states16_f) {
                 // the 16-bit copies of the entering states (a forward pass whose caller keeps no states: half the bytes)
@@ -270,30 +265,10 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
                 tile_load_kcontig<T, float, PW, NW>(sF, stf + n0, N, P - p0, N - n0, Ident());
                 tile_load_kcontig<T, float, PW, NW>(sB, stb + n0, N, P - p0, N - n0, Ident());
             }
+            if (!ROWS_FIRST) load_arows(n0);
             __syncthreads();
-#pragma unroll
-            for (int s = 0; s < NW / KSTEP; ++s) {
-                if (n0 + s * KSTEP >= N) break;
-                const int kq = s * KSTEP + lg * KPL;
-                typename M::Frag bff[NJ], bfb[NJ];
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-                    bff[j] = M::load(sF + (j * 16 + lr) * LDS_ + kq);
-                    bfb[j] = M::load(sB + (j * 16 + lr) * LDS_ + kq);
-                }
-#pragma unroll
-                for (int rt = 0; rt < QT; ++rt) {
-                    float vf[KPL], vb[KPL];
-#pragma unroll
-                    for (int i = 0; i < KPL; ++i) { vf[i] = arow[rt][s][i] * rsf[rt]; vb[i] = arow[rt][s][i] * rsb[rt]; }
-                    const typename M::Frag aff = M::pack(vf), afb = M::pack(vb);
-#pragma unroll
-                    for (int j = 0; j < NJ; ++j) {
-                        acc[rt][j] = M::mma(aff, bff[j], acc[rt][j]);
-                        acc[rt][j] = M::mma(afb, bfb[j], acc[rt][j]);
-                    }
-                }
-            }
+            state_product(0, N - n0);
+            state_product(1, N - n0);
         }
     }
 
@@ -397,11 +372,11 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
                 const int r = rowi[rt], r0 = (wave * QT + rt) * 16;
                 float v[KPL];
                 if (k0 + KSTEP - 1 < r0) {            // every k of this step is below every row of the tile
-                    const float rf = __builtin_amdgcn_exp2f(lor[rt] - lo[kb | 15]);
+                    const float rf = __expf(lor[rt] - lo[kb | 15]);
 #pragma unroll
                     for (int i = 0; i < KPL; ++i) v[i] = cbv[B_][rt][i] * rf * glo[kb + i];
                 } else if (k0 > r0 + 15) {            // every k above every row
-                    const float rf = __builtin_amdgcn_exp2f(upr[rt] - up[kb & ~15]);
+                    const float rf = __expf(upr[rt] - up[kb & ~15]);
 #pragma unroll
                     for (int i = 0; i < KPL; ++i) v[i] = cbv[B_][rt][i] * rf * gup[kb + i];
                 } else {
@@ -409,7 +384,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
                     for (int i = 0; i < KPL; ++i) {
                         const int k = kb + i;
                         const float e = k < r ? lor[rt] - lo[k] : upr[rt] - up[k];
-                        v[i] = cbv[B_][rt][i] * ((k == r) ? 2.f : __builtin_amdgcn_exp2f(e));
+                        v[i] = cbv[B_][rt][i] * ((k == r) ? 2.f : __expf(e));
                         if (!BWD) v[i] *= dtl[min(k, QP - 1)];
                     }
                 }
@@ -472,7 +447,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
                     raw_lds_use(ga0); raw_lds_use(ga1); raw_lds_use(mref);
 #pragma unroll
                     for (int rt = 0; rt < QT; ++rt) {
-                        const float rf = __builtin_amdgcn_exp2f((cls == 0 ? lor[rt] : upr[rt]) - mref);
+                        const float rf = __expf((cls == 0 ? lor[rt] : upr[rt]) - mref);
                         float v[KPL];
 #pragma unroll
                         for (int i = 0; i < 4; ++i) { v[i] = cb1[rt][i] * rf * ga0[i]; v[i + 4] = cb2[rt][i] * rf * ga1[i]; }
@@ -501,7 +476,7 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
                             const int k = kb + i;
                             const float lk = i < 4 ? l0[i & 3] : l1[i & 3], uk = i < 4 ? u0[i & 3] : u1[i & 3];
                             const float e = k < r ? lor[rt] - lk : upr[rt] - uk;
-                            float w = (k == r) ? (UNI ? 1.f : 2.f) : __builtin_amdgcn_exp2f(e);
+                            float w = (k == r) ? (UNI ? 1.f : 2.f) : __expf(e);
                             if (UNI && (BWD ? k < r : k > r)) w = 0.f;
                             if (!BWD) w *= i < 4 ? d0[i & 3] : d1[i & 3];
                             v[i] = (i < 4 ? cb1[rt][i & 3] : cb2[rt][i & 3]) * w;
@@ -682,7 +657,6 @@ __global__ __launch_bounds__(SCAN_THREADS, 4) void chunk_scan_kernel(const bimam
 static inline bool al16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
 
 static inline int scan_col_tile(const bimamba2_params *p) {
-    // headdim tile: the widest the LDS image allows (64 columns for 16-bit types, 32 for float32)
     return scan_col_tile_of(p->headdim, p->dtype);
 }
 
@@ -716,7 +690,7 @@ bool chunk_scan_uses_scan16(const bimamba2_params *p, bool bwd) {
     return scan_rebuild_shape(p, bwd) && (p->headdim == 64 || p->headdim == 128) && (p->dstate == 64 || (p->dstate == 128 && !bwd));
 }
 
-template <typename T, int NJMAX, bool BWD>
+template <typename T, bool BWD>
 static int launch_scan_t(const bimamba2_params *p) {
     const int nc = nchunks(p);
     const int P = p->headdim, Q = p->chunk_size, N = p->dstate;
@@ -735,7 +709,7 @@ static int launch_scan_t(const bimamba2_params *p) {
     // 16-bit copies of the entering states: known to the kernels that rebuild CB only
     const void *c16f = BWD ? p->dstates16_f : p->states16_f, *c16b = BWD ? p->dstates16_b : p->states16_b;
     if (c16f && (!al16(c16f) || !al16(c16b) || !(p->causal || c16b))) return BIMAMBA2_EINVAL;
-    if constexpr (sizeof(T) == 2 && NJMAX == 4) {
+    if constexpr (sizeof(T) == 2) {
         // the shapes of the 16-bit kernel with transposed products and a raw operand tile: it needs the 16-bit copies of the
         // entering states (the composites keep them at these shapes) and no CB
         if (c16f && (BWD ? p->CBT : p->CB) == nullptr && chunk_scan_uses_scan16(p, BWD) && (p->causal || c16b))
@@ -758,16 +732,16 @@ static int launch_scan_t(const bimamba2_params *p) {
     if ((BWD ? p->CBT : p->CB) == nullptr) return BIMAMBA2_EINVAL;
     if (pw == 16) { if (qt == 1) BM2_SCAN(1, 1); else BM2_SCAN(2, 1); }
     else if (pw == 32) { if (qt == 1) BM2_SCAN(1, 2); else BM2_SCAN(2, 2); }
-    else { if (qt == 1) BM2_SCAN(1, NJMAX); else BM2_SCAN(2, NJMAX); }
+    else if constexpr (sizeof(T) == 2) { if (qt == 1) BM2_SCAN(1, 4); else BM2_SCAN(2, 4); }   // (float32: 32 columns at most)
 #undef BM2_SCAN
     return check_launch();
 }
 
 int launch_chunk_scan(const bimamba2_params *p, bool bwd) {
     switch (p->dtype) {
-        case BIMAMBA2_F32: return bwd ? launch_scan_t<float, 2, true>(p) : launch_scan_t<float, 2, false>(p);
-        case BIMAMBA2_BF16: return bwd ? launch_scan_t<bf16_t, 4, true>(p) : launch_scan_t<bf16_t, 4, false>(p);
-        case BIMAMBA2_F16: return bwd ? launch_scan_t<f16_t, 4, true>(p) : launch_scan_t<f16_t, 4, false>(p);
+        case BIMAMBA2_F32: return bwd ? launch_scan_t<float, true>(p) : launch_scan_t<float, false>(p);
+        case BIMAMBA2_BF16: return bwd ? launch_scan_t<bf16_t, true>(p) : launch_scan_t<bf16_t, false>(p);
+        case BIMAMBA2_F16: return bwd ? launch_scan_t<f16_t, true>(p) : launch_scan_t<f16_t, false>(p);
         default: return BIMAMBA2_EUNSUPPORTED;
     }
 }
