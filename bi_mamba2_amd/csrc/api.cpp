@@ -215,6 +215,35 @@ int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd) {
     return chunk_scan_uses_scan16(p, bwd != 0) ? chunk_scan16_heads_per_workgroup(p) : 1;
 }
 
+// Where the lines lie, us a pass with chunks of 64 / 128 / 256 (z gate, D; forward alone and, second, with the backward pass; one
+// group unless said otherwise).  A chunk costs its pairs of positions (they grow with the chunk) and its states (which do not);
+// small calls want many workgroups, i.e. small chunks.
+//  * float32: pairs run at the float32 matrix rate.  4 x 2048, 16 heads of 64, dstate 64: 147 / 111 / 129, 526 / 412 / 488; heads of 16,
+//    dstate 16: 58 / 49 / 56, 240 / 211 / 252; 2 x 512, 8 heads of 64, dstate 64: 34 / 37 / 55, 141 / 143 / 185; 4 x 1024, 8 heads of 32:
+//    45 / 43 / 61.  Never above the caller's: the result is off by the resolution of sums over a chunk (1.6 times as much in
+//    chunks twice as long).
+//  * 16 bits, the kernels that rebuild C.B^T (dstate 64, headdim 64 or 128; forward also dstate 128): 4 x 2048, 16 heads of 64, dstate 64:
+//    61 / 44 / 39, 206 / 163 / 153; 4 x 1024, 8 heads: 31 / 25 / 29, 133 / 126 / 125; 2 x 512: 22 / 22 / 27; dstate 128, 4 x 2048: 86 / 65 / 63.
+//    Never below the caller's (their states are kept in 16 bits: a rounding per chunk).
+//  * other 16-bit shapes: 4 x 2048, 16 heads of 32, dstate 32: 66 / 52 / 53, 267 / 222 / 258; 8 groups, 4 x 4096: 126 / 101 / 119, 583 / 545 /
+//    719; 4 x 1024, 8 heads: 31 / 29 / 40, 139 / 129 / 167; 2 x 512: 27 / 28 / 38.  Training at dstate 128: 4 x 2048, 16 heads of 64: 433 / 278 /
+//    251; of 128: 894 / 496 / 408; 16 heads in 8 groups, 4 x 4096, of 64: 1093 / 783 / 877, of 128: 1903 / 1253 / 1218.
+int bimamba2_chunk_for(const bimamba2_params *p, int training) {
+    if (check_problem(p)) return p ? p->chunk_size : 0;
+    const int Q = p->chunk_size, P = p->headdim, N = p->dstate;
+    // (packed sequences that need no count of their boundaries keep their size: counting them synchronises)
+    if (p->causal || Q % 32 || (p->seq_idx && Q <= BIMAMBA2_MAX_SEQ_BOUNDARIES)) return Q;
+    auto workgroups = [&](int q, int columns) {       // of one launch over (batch, chunk, head, headdim tile)
+        return (int64_t)p->batch * ((p->seqlen + q - 1) / q) * p->nheads * ((P + columns - 1) / columns);
+    };
+    constexpr int CUS = 256;
+    if (p->dtype == BIMAMBA2_F32) return Q > 64 ? std::min(Q, workgroups(128, 32) >= CUS ? 128 : 64) : Q;
+    const bool whole = P == 64 || P == 128;
+    if (whole && (N == 64 || (N == 128 && (!training || P == 128 || p->nheads >= 8 * p->ngroups))))
+        return std::max(Q, workgroups(256, 64) >= CUS ? 256 : workgroups(128, 64) >= CUS / 2 ? 128 : Q);
+    return Q > 128 || workgroups(128, 64) >= CUS ? 128 : Q;
+}
+
 int bimamba2_ddt_direct_planes(const bimamba2_params *p) {
     if (check_problem(p)) return 1;
     return ddt_direct_planes(*p);

@@ -46,6 +46,7 @@ struct Api {
     decltype(&bimamba2_workspace_bytes) workspace_bytes = nullptr;
     decltype(&bimamba2_state_copies) state_copies = nullptr;
     decltype(&bimamba2_chunk_scan_reads_cb) reads_cb = nullptr;
+    decltype(&bimamba2_chunk_for) chunk_for = nullptr;
     decltype(&bimamba2_seq_boundaries) seq_boundaries = nullptr;
     decltype(&bimamba2_strerror) strerror = nullptr;
     decltype(&bimamba2_rmsnorm_gated_fwd) norm_fwd = nullptr;
@@ -81,6 +82,7 @@ void load(const std::string &path) {
     get(api.workspace_bytes, "bimamba2_workspace_bytes");
     get(api.state_copies, "bimamba2_state_copies");
     get(api.reads_cb, "bimamba2_chunk_scan_reads_cb");
+    get(api.chunk_for, "bimamba2_chunk_for");
     get(api.seq_boundaries, "bimamba2_seq_boundaries");
     get(api.strerror, "bimamba2_strerror");
     get(api.norm_fwd, "bimamba2_rmsnorm_gated_fwd");
@@ -336,7 +338,7 @@ ScanResult scan_forward(Problem &q, ScanOpts &o, bool keep) {
 }
 
 // Packed sequences: the largest number of boundaries that falls into one chunk.  The count is taken on the device and written
-// to pinned host memory; the host waits for that kernel only, after it has enqueued the forward pass at the caller's chunk
+// to pinned host memory; the host waits for that kernel only, after it has enqueued the forward pass at the usual chunk
 // size, so that the GPU has work while the host reads the answer (which nearly always is that the chunk size may stay).
 constexpr int64_t max_boundaries = BIMAMBA2_MAX_SEQ_BOUNDARIES;
 
@@ -382,6 +384,7 @@ struct BoundaryCount {
 template <typename MakeProblem> ScanResult scan_checked(MakeProblem make, ScanOpts &o, bool keep) {
     {
         Problem q = make(o);
+        q.p.chunk_size = o.chunk = api.chunk_for(&q.p, keep);
         if (!q.p.seq_idx || o.chunk <= max_boundaries) return scan_forward(q, o, keep);
         BoundaryCount first(q.p, q.x.device().index());
         ScanResult r = scan_forward(q, o, keep);
@@ -745,6 +748,7 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
 
     const Tensor y = device_empty({s.rows, s.inner}, u.scalar_type(), u);
     bimamba2_params p = layer_scan_params(s, o, zx, xbc, w, stream);
+    p.chunk_size = o.chunk = api.chunk_for(&p, keep);
     p.out = y.mutable_data_ptr();
     Tensor kept;
     if (keep) {

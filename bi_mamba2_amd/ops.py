@@ -557,6 +557,18 @@ def _point_into(c, blob, offs, fields=_BLOB_FIELDS):
 MAX_SEQ_BOUNDARIES_PER_CHUNK = 32
 
 
+def _chunk_for(x, dt, A, B, C, chunk_size, D, z, dt_bias, seq_idx):
+    """The chunk size that the kernels run the problem with (bimamba2_chunk_for), as the native route chooses it."""
+    if x.shape[-1] > MAX_HEADDIM or B.shape[-1] > MAX_DSTATE or x.dtype not in _DT:
+        return chunk_size                                          # (the pieces that such a call is made of choose theirs)
+    p = _lib.Params()
+    p.batch, p.seqlen, p.nheads, p.headdim = (int(n) for n in x.shape)
+    p.ngroups, p.dstate, p.chunk_size, p.dtype = int(B.shape[2]), int(B.shape[3]), chunk_size, _DT[x.dtype]
+    p.seq_idx = seq_idx.data_ptr() if seq_idx is not None else None
+    training = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, dt, A, B, C, D, z, dt_bias))
+    return int(_lib.load().bimamba2_chunk_for(p, 1 if training else 0))
+
+
 def seq_boundaries_per_chunk(seq_idx, chunk_size):
     """Largest number of sequence boundaries that fall into one chunk of `chunk_size` positions, as the kernels count
     them: a change of seq_idx between positions l - 1 and l offsets the forward sums of the chunk of l and the reverse
@@ -817,7 +829,8 @@ def bimamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_b
         A: (nheads)
         B: (batch, seqlen, ngroups, dstate)
         C: (batch, seqlen, ngroups, dstate)   (dstate above the kernels' 256: computed in pieces of the state dimension)
-        chunk_size: int, at least 32 (above 256 the kernels use 256: the result does not depend on it)
+        chunk_size: int, at least 32.  The result does not depend on it, and the kernels may run with another one (at most 256) that
+            is faster for the problem and no less exact
         D: (nheads, headdim) or (nheads,)
         z: (batch, seqlen, nheads, headdim)
         dt_bias: (nheads,)
@@ -856,6 +869,7 @@ def bimamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_b
         res = _lib.host().scan(x, dt, A, B, C, chunk_size, D, z, dt_bias, dt_softplus, dt_limit[0], dt_limit[1],
                                return_final_states, initial_states_f, initial_states_b, seq_idx)
         return tuple(res) if return_final_states else res[0]
+    chunk_size = _chunk_for(x, dt, A, B, C, chunk_size, D, z, dt_bias, seq_idx)
     if seq_idx is not None:
         # many short packed sequences: a smaller chunk keeps the boundaries per chunk inside what the mechanism resolves
         chunk_size = chunk_size_for_seq_idx(seq_idx, chunk_size)

@@ -1,0 +1,46 @@
+"""The chunk size that the kernels run with instead of the caller's (bimamba2_chunk_for): out and every gradient against float64
+autograd of the oracle's recurrence, at sizes where the rule takes another one, through the native route and the Python one."""
+import pytest
+import torch
+
+from oracle import bimamba2_oracle as O
+from helpers import make_case
+
+pytestmark = pytest.mark.gpu
+
+# as elsewhere: float32 differs by the order of sums; 16-bit operands enter every product rounded (2^-9 resp. 2^-12) and the results
+# are rounded once more, a few roundings one after the other
+REL = {torch.float32: 2e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}
+
+
+@pytest.mark.parametrize("b,L,H,P,G,N,Q,runs,dtype,z,pack", [
+    (1, 385, 4, 16, 2, 16, 256, 64, torch.float32, True, False),         # down to 64, one position in the last chunk
+    (2, 260, 64, 32, 1, 16, 256, 128, torch.float32, False, False),      # down to 128
+    (1, 300, 6, 32, 2, 32, 256, 128, torch.bfloat16, True, False),       # another 16-bit shape: down
+    (2, 257, 64, 16, 8, 80, 64, 128, torch.float16, True, False),        # and up, dstate no multiple of 32
+    (2, 300, 64, 64, 8, 64, 64, 256, torch.bfloat16, True, False),       # kernels that rebuild C.B^T: up
+    (2, 300, 64, 64, 64, 128, 256, 128, torch.bfloat16, False, False),   # state dimension 128 with one head a group
+    (2, 300, 64, 16, 8, 16, 64, 128, torch.bfloat16, False, True),       # packed sequences
+])
+def test_results_do_not_depend_on_the_choice(monkeypatch, b, L, H, P, G, N, Q, runs, dtype, z, pack):
+    from bi_mamba2_amd import ops
+    inp = make_case(b, L, H, P, G, N, dtype, with_z=z)
+    d = {k: None if v is None else v.cuda().requires_grad_(True) for k, v in inp.items()}
+    si = (torch.arange(L) // 45).expand(b, L).contiguous() if pack else None
+    si_gpu = si.to(torch.int32).cuda() if pack else None
+    assert ops._chunk_for(d["x"], d["dt"], d["A"], d["B"], d["C"], Q, d["D"], d["z"], d["dt_bias"], si_gpu) == runs
+    dout = torch.randn(inp["x"].shape, generator=torch.Generator().manual_seed(3)).to(dtype)
+    # (the recurrence step by step in float64, on the GPU: many heads, where the rule chooses by the size of the launch)
+    r = {k: None if v is None else v.detach().double().cuda().requires_grad_(True) for k, v in inp.items()}
+    want = O.bimamba2_sequential(r["x"], r["dt"], r["A"], r["B"], r["C"], D=r["D"], z=r["z"], dt_bias=r["dt_bias"], dt_softplus=True,
+                                 **({"seq_idx": si.cuda()} if pack else {}))[0]
+    names = [k for k, v in r.items() if v is not None]
+    want = (want.detach(),) + torch.autograd.grad(want, [r[k] for k in names], dout.double().cuda())
+    for keep in (True, False):                                           # native route, Python route
+        monkeypatch.setattr(ops, "KEEP_FORWARD_INTERMEDIATES", keep)
+        out = ops.bimamba_chunk_scan_combined(d["x"], d["dt"], d["A"], d["B"], d["C"], Q, D=d["D"], z=d["z"], dt_bias=d["dt_bias"],
+                                              dt_softplus=True, seq_idx=si_gpu)
+        got = (out.detach(),) + torch.autograd.grad(out, [d[k] for k in names], dout.cuda())
+        for name, g, w in zip(["out"] + names, got, want):
+            err = (g.double() - w).norm() / w.norm()
+            assert err < REL[dtype], (name, float(err))

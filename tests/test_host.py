@@ -239,3 +239,31 @@ def test_no_head_slice_of_dcb_is_empty():
     (4, 4, 256, 64, 64, _lib.F32, 2), (64, 64, 256, 64, 64, _lib.F32, 2), (24, 64, 65, 64, 64, _lib.F32, 3), (25, 63, 65, 64, 64, _lib.F32, 1)])
 def test_head_slices_of_dcb(heads, rows, chunk, headdim, dstate, dtype, slices):
     assert _dcb_slices(**_contiguous(rows, chunk, heads, headdim, 1, dstate, chunk, dtype)) == slices
+
+
+# what a caller asks for -> what the kernels run with, at the lines of the rule: workgroups of one launch against the chip's 256
+@pytest.mark.parametrize("batch,seqlen,heads,headdim,groups,dstate,dtype,training,chunk,runs", [
+    # float32: down to 128 where that fills the chip, else to 64; never up
+    (2, 1111, 16, 64, 2, 64, "F32", 1, 256, 128), (1, 8192, 4, 32, 1, 16, "F32", 1, 256, 128), (1, 8064, 4, 32, 1, 16, "F32", 0, 256, 64),
+    (1, 100, 1, 16, 1, 16, "F32", 0, 128, 64), (4, 2048, 16, 64, 1, 64, "F32", 1, 64, 64), (4, 2048, 16, 64, 1, 64, "F32", 1, 32, 32),
+    # kernels that rebuild C.B^T: up to 256 or 128 where that leaves enough workgroups; never down
+    (4, 1024, 16, 64, 1, 64, "BF16", 1, 64, 256), (4, 1024, 15, 64, 1, 64, "BF16", 1, 64, 128), (1, 300, 4, 64, 1, 64, "F16", 0, 64, 64),
+    (1, 300, 4, 64, 1, 64, "F16", 0, 256, 256), (4, 1024, 8, 128, 1, 64, "F16", 1, 128, 256),
+    # state dimension 128: training with few heads of 64 in a group stays at 128
+    (4, 2048, 16, 64, 8, 128, "BF16", 0, 64, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 256, 128), (4, 2048, 16, 64, 2, 128, "BF16", 1, 64, 256),
+    (4, 2048, 16, 128, 8, 128, "BF16", 1, 64, 256),
+    # the other 16-bit shapes: 128, from below only where that fills the chip
+    (1, 300, 4, 16, 1, 16, "BF16", 1, 256, 128), (1, 300, 4, 16, 1, 16, "BF16", 1, 64, 64), (4, 1024, 8, 32, 1, 16, "BF16", 0, 64, 128),
+    (4, 1024, 8, 96, 1, 64, "BF16", 0, 224, 128), (4, 1024, 8, 64, 1, 80, "F16", 1, 32, 128),
+    # sizes that are no whole steps of the kernels stay
+    (4, 2048, 16, 64, 1, 64, "F32", 1, 200, 200), (4, 2048, 16, 16, 1, 64, "BF16", 1, 33, 33),
+])
+def test_chunk_size_that_the_kernels_run_with(batch, seqlen, heads, headdim, groups, dstate, dtype, training, chunk, runs):
+    lib = _lib.load()
+    p = _params(batch=batch, seqlen=seqlen, nheads=heads, headdim=headdim, ngroups=groups, dstate=dstate, dtype=getattr(_lib, dtype), chunk_size=chunk)
+    assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == runs
+    p.causal = 1                                                               # (the comparator runs as it is asked to)
+    assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == chunk
+    p.causal, p.seq_idx = 0, 4096
+    assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == (chunk if chunk <= 32 else runs)   # 32: needs no count of boundaries
+    assert lib.bimamba2_chunk_for(ctypes.byref(_params(chunk_size=16)), training) == 16            # (refused by the entry points)
