@@ -1390,10 +1390,10 @@ int dcb_slices(const bimamba2_params *p) {
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Variant for 16-bit types with headdim % 64 == 0, chunk_size % 64 == 0 and aligned operands.
+// Variant for 16-bit types with headdim % 8 == 0, chunk_size % 64 == 0 and aligned operands.
 //
 // The kernel is bound by its instruction count, not by memory, so everything per head is pared down:
-//  * the dout tile, the x tile and the decay vectors of each (head, 64-wide headdim chunk) step travel from global memory
+//  * the dout tile, the x tile and the decay vectors of each (head, KC-wide headdim chunk) step travel from global memory
 //    straight into a ring of LDS slots (global_load_lds, 16 bytes per lane, no registers, no address arithmetic beyond
 //    one 64-bit add per request), one step ahead of the one being multiplied; 16-byte units are XOR-swizzled by the row
 //    so that the fragment reads spread over the banks;
@@ -1415,11 +1415,7 @@ __device__ __forceinline__ float lanegroup_sum_mfma(float v) {
 // its slot) measured 60 us against 62 us for three slots requested two steps ahead.
 constexpr int DCB_RING = 2;
 constexpr int DCB_RESIDENT_BLOCKS = 1024;                 // a dCB grid up to this size is on the chip all at once
-constexpr int DCB_TILE_B = 64 * 64 * 2;                    // one 64 x 64 tile of 16-bit elements
-constexpr int DCB_CS_OFF = 2 * DCB_TILE_B;                 // cs_f[t], cs_b[t], cs_f[s], cs_b[s], dt[s]: 5 x 64 floats
-constexpr int DCB_SLOT_B = DCB_CS_OFF + 5 * 64 * 4;
-constexpr int DCB_PART_OFF = DCB_RING * DCB_SLOT_B;        // per-wave column sums (f: 0-3, b: 4-7), row sums (f: 8, b: 9)
-constexpr int DCB_PART_B = 10 * 64 * 4;
+constexpr int DCB_PART_B = 10 * 64 * 4;                   // per-wave column sums (f: 0-3, b: 4-7), row sums (f: 8, b: 9)
 
 
 // UNI: the single-direction operator - tiles above the diagonal are empty, tiles on it keep the forward half.
@@ -1437,12 +1433,21 @@ __device__ __forceinline__ BlockId dcb_block_of(int id, int gdx, int ntiles, int
     return BlockId{(k / ntiles) * 8 + (id & 7), k % ntiles, 0};
 }
 
-template <typename T, bool UNI>
+// KC: headdim columns per step, 64 (headdim above 32), or 32.  WHOLE: headdim is a multiple of it.  Otherwise (a multiple of 8) the
+// rest of a row's units in LDS stays as it was cleared before the first request: a step with such a rest is always the same
+// slot's (headdim <= 128, two slots), so nothing else is ever put there.
+template <typename T, bool UNI, int KC, bool WHOLE>
 __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int nc, int nqt, BlockId bid, int gdx, int gdz, bool out16 = false) {
     typedef Mma<T> M;
     typedef typename M::Frag Frag;
-    static_assert(sizeof(T) == 2, "ring variant is for 16-bit operands");
-    constexpr int KC = 64, NKS = 2;                            // 64 headdim columns = 8 units of 16 bytes per row
+    static_assert(sizeof(T) == 2 && DCB_RING == 2, "ring variant is for 16-bit operands");
+    constexpr int NKS = KC / 32, UNITS = KC / 8;               // 16-byte units per row
+    constexpr int DCB_TILE_B = 64 * KC * 2;                    // one 64-row tile of 16-bit elements
+    constexpr int DCB_CS_OFF = 2 * DCB_TILE_B;                 // cs_f[t], cs_b[t], cs_f[s], cs_b[s], dt[s]: 5 x 64 floats
+    constexpr int DCB_SLOT_B = DCB_CS_OFF + 5 * 64 * 4;
+    constexpr int DCB_PART_OFF = DCB_RING * DCB_SLOT_B;
+    // position of a row's unit among its units: neighbouring rows' accesses to one unit fall on different banks
+    auto unit_at = [](int row, int unit) { return unit ^ (KC == 64 ? row & 7 : (row >> 1) & 3); };
     __shared__ __attribute__((aligned(16))) unsigned char smem[DCB_PART_OFF + 2 * DCB_PART_B];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 15, lg = lane >> 4;
@@ -1464,7 +1469,7 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
     f32x4 cbr[4] = {}, dcb[4] = {};
     const int hps = (hpg + gdz - 1) / gdz;
     const int h_begin = bid.z * hps, h_end = min(hpg, h_begin + hps);
-    const int nkc = P / KC, nhs = h_end - h_begin, nit = nhs * nkc;
+    const int nkc = (P + KC - 1) / KC, nhs = h_end - h_begin, nit = nhs * nkc;
     const int h0 = g * hpg + h_begin;
     // (a caller's dcb_slices may leave a slice without heads: it writes zeros and requests nothing, its h0 may lie behind the last head)
     const bool live = t0 < limit && s0 < limit && !(UNI && st > tt) && nhs > 0;
@@ -1475,12 +1480,18 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
             for (int i = threadIdx.x; i < DCB_VEC; i += NTHREADS) tv0[hh * tv_head + i] = 0.f;
     } else {
         const unsigned sbase = lds_addr(smem);
-        // ---- requests: unit u = i*256 + thread of a 64 x 64 tile is row r = u / 8, 16-byte chunk (u % 8) ^ (r % 8).
+        if constexpr (!WHOLE) {
+            for (int i = threadIdx.x; i < DCB_PART_OFF / 16; i += NTHREADS) reinterpret_cast<f32x4 *>(smem)[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+            __syncthreads();
+        }
+        // ---- requests: unit u = i*256 + thread of a tile lies at position u % UNITS of row r = u / UNITS.
         // Addresses are a wave-uniform base (scalar registers, moved on from head to head) plus this lane's 32-bit byte offset
         // (the launcher checks that the rows of a chunk lie within 32 bits of each other): six vector registers less than
         // four per-lane pointers (126 registers instead of 138: four workgroups fit a CU where the grid has them).
         const char *ybase, *xbase;
-        unsigned yoff[2], xoff[2];
+        constexpr int NREQ = 64 * UNITS / NTHREADS;            // per thread and tile
+        unsigned yoff[NREQ], xoff[NREQ];
+        int ucol[NREQ];                                        // headdim column of the unit inside the step
         int64_t y_head, y_row;
         {
             const T *yp;
@@ -1490,8 +1501,9 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
             ybase = uniform_ptr(yp);
             xbase = uniform_ptr(xp);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const int u = i * NTHREADS + threadIdx.x, r = u >> 3, col = ((u & 7) ^ (r & 7)) * 8;
+            for (int i = 0; i < NREQ; ++i) {
+                const int u = i * NTHREADS + threadIdx.x, r = u / UNITS, col = unit_at(r, u % UNITS) * 8;
+                ucol[i] = col;
                 yoff[i] = (unsigned)(((int64_t)min(t0 + r, limit - 1) * y_row + col) * (int64_t)sizeof(T));
                 xoff[i] = (unsigned)(((int64_t)min(s0 + r, limit - 1) * p.x_sl + col) * (int64_t)sizeof(T));
             }
@@ -1507,10 +1519,19 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
         // requests one step into `slot` and moves the source pointers on to the next step
         auto issue = [&](int slot) __attribute__((always_inline)) {
             unsigned char *sl = smem + slot * DCB_SLOT_B + wave * 1024;
-            load16_to_lds_at(ybase, yoff[0], sl);
-            load16_to_lds_at(ybase, yoff[1], sl + 4096);
-            load16_to_lds_at(xbase, xoff[0], sl + DCB_TILE_B);
-            load16_to_lds_at(xbase, xoff[1], sl + DCB_TILE_B + 4096);
+            if constexpr (WHOLE) {
+#pragma unroll
+                for (int i = 0; i < NREQ; ++i) load16_to_lds_at(ybase, yoff[i], sl + i * 4096);
+#pragma unroll
+                for (int i = 0; i < NREQ; ++i) load16_to_lds_at(xbase, xoff[i], sl + DCB_TILE_B + i * 4096);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NREQ; ++i)
+                    if (ikc * KC + ucol[i] < P) {
+                        load16_to_lds_at(ybase, yoff[i], sl + i * 4096);
+                        load16_to_lds_at(xbase, xoff[i], sl + DCB_TILE_B + i * 4096);
+                    }
+            }
             if (threadIdx.x < 80) __builtin_amdgcn_global_load_lds((gbl_ptr_t)csrc, (lds_ptr_t)(sl + DCB_CS_OFF), 16, 0, 0);
             const bool last = ++ikc == nkc;
             if (last) ikc = 0;
@@ -1523,9 +1544,9 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
         unsigned a_off[NKS], b_off[NKS];
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) {
-            const int ch = (ks * 4 + lg) ^ (lr & 7);
-            a_off[ks] = ((wave * 16 + lr) * 8 + ch) * 16;
-            b_off[ks] = DCB_TILE_B + (lr * 8 + ch) * 16;       // column block j adds j * 2048
+            const int ch = unit_at(lr, ks * 4 + lg);
+            a_off[ks] = ((wave * 16 + lr) * UNITS + ch) * 16;
+            b_off[ks] = DCB_TILE_B + (lr * UNITS + ch) * 16;   // column block j adds j * 16 rows
         }
         const unsigned ct_off = DCB_CS_OFF + trow * 4, cc_off = DCB_CS_OFF + lr * 4, cm_off = DCB_CS_OFF + wave * 64;
         const int rows_left = limit - t0 - trow;               // accumulator rows i >= rows_left lie past the sequence end
@@ -1597,8 +1618,8 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
         // The head loop is compiled once per kind of tile: off the diagonal (KIND = -1), and on it once per wave (KIND = the
         // wave's index, which decides for every column block whether it lies below, on or above the wave's rows), so that
         // none of these decisions is taken, and no register moved to a common place, inside the loop.
-        auto run = [&](auto KC) __attribute__((always_inline)) {
-            constexpr int KIND = decltype(KC)::value;
+        auto run = [&](auto TILE_KIND) __attribute__((always_inline)) {
+            constexpr int KIND = decltype(TILE_KIND)::value;
             constexpr bool DIAG = KIND >= 0;
             constexpr bool LOWER = KIND == -1;             // off the diagonal: -1 below it (forward direction), -2 above
         for (int it = 0; it < nit; ++it) {
@@ -1624,9 +1645,9 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
             for (int ks = 0; ks < NKS; ++ks) {
                 af[ks] = raw_lds_read_at<Frag, 0>(sb + a_off[ks]);
                 bf[0][ks] = raw_lds_read_at<Frag, 0>(sb + b_off[ks]);
-                bf[1][ks] = raw_lds_read_at<Frag, 2048>(sb + b_off[ks]);
-                bf[2][ks] = raw_lds_read_at<Frag, 4096>(sb + b_off[ks]);
-                bf[3][ks] = raw_lds_read_at<Frag, 6144>(sb + b_off[ks]);
+                bf[1][ks] = raw_lds_read_at<Frag, 256 * UNITS>(sb + b_off[ks]);
+                bf[2][ks] = raw_lds_read_at<Frag, 512 * UNITS>(sb + b_off[ks]);
+                bf[3][ks] = raw_lds_read_at<Frag, 768 * UNITS>(sb + b_off[ks]);
             }
             raw_lds_wait();
             // (the first product of a head starts from a literal zero: no registers to clear between heads)
@@ -1815,11 +1836,11 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
     }
 }
 
-template <typename T, bool UNI = false>
+template <typename T, bool UNI = false, int KC = 64, bool WHOLE = true>
 __global__ __launch_bounds__(NTHREADS) void bwd_dcb_ring_kernel(const bimamba2_params p, int nc, int nqt) {
     BlockId bid = dcb_block_of(blockIdx.x + gridDim.x * blockIdx.y, gridDim.x, gridDim.y, gridDim.x * gridDim.y);
     bid.z = blockIdx.z;
-    bwd_dcb_ring_body<T, UNI>(p, nc, nqt, bid, gridDim.x, gridDim.z);
+    bwd_dcb_ring_body<T, UNI, KC, WHOLE>(p, nc, nqt, bid, gridDim.x, gridDim.z);
 }
 
 // The dCB kernel and the backward state passing as roles of one launch (one head slice): the first is bound by instruction issue and moves little data, the second streams
@@ -1830,7 +1851,7 @@ template <typename T, bool UNI>
 __device__ __forceinline__ void bwd_dcb_sp_body(const bimamba2_params &p, int nc, int nqt, int gdx, int ndcb, int nsplit, int ndir, bool out16) {
     const int id = blockIdx.x;
     if (id < ndcb) {
-        bwd_dcb_ring_body<T, UNI>(p, nc, nqt, dcb_block_of(id, gdx, nqt * nqt, ndcb), gdx, 1, out16);
+        bwd_dcb_ring_body<T, UNI, 64, true>(p, nc, nqt, dcb_block_of(id, gdx, nqt * nqt, ndcb), gdx, 1, out16);
     } else {
         const int k = id - ndcb;                  // grid (nsplit, nheads, batch * ndir) of the state passing
         const BlockId sb{k % nsplit, (k / nsplit) % p.nheads, k / (nsplit * p.nheads)};
@@ -1844,9 +1865,13 @@ template <typename T, bool UNI>
 __global__ __launch_bounds__(NTHREADS) void bwd_dcb_sp_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int ndcb, int nsplit, int ndir, bool out16) {
     bwd_dcb_sp_body<T, UNI>(p, nc, nqt, gdx, ndcb, nsplit, ndir, out16);
 }
+// Narrow heads (16-bit) take the ring as well: through registers a workgroup waits for its operands head by head.  4 x 2048 in chunks of
+// 128, 16 heads of 16: 46 -> 21 us; 48 heads of 16: the whole pass 497 -> 389 us; in 8 groups (two heads a tile) 43 -> 28 us.
 template <typename T> static void launch_dcb_ring(dim3 grid, const bimamba2_params *p, int nc, int nqt) {
     if constexpr (sizeof(T) == 2) {
         if (p->causal) hipLaunchKernelGGL((bwd_dcb_ring_kernel<T, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
+        else if (p->headdim <= 32) hipLaunchKernelGGL((bwd_dcb_ring_kernel<T, false, 32, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
+        else if (p->headdim % 64) hipLaunchKernelGGL((bwd_dcb_ring_kernel<T, false, 64, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
         else hipLaunchKernelGGL((bwd_dcb_ring_kernel<T>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
     }
 }
@@ -1876,11 +1901,12 @@ static int launch_dcb_t(const bimamba2_params *p) {
     dim3 grid(p->batch * nc * p->ngroups, nqt * nqt, slices);
     constexpr int VS = 16 / (int)sizeof(T);
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    bool fast = p->headdim % (sizeof(T) == 2 ? 64 : 16) == 0 && al(p->x) && p->x_sb % VS == 0 && p->x_sl % VS == 0 && p->x_sh % VS == 0;
-    fast = fast && (p->has_z ? al(p->dout_x) : (al(p->dout) && p->dout_sb % VS == 0 && p->dout_sl % VS == 0 && p->dout_sh % VS == 0));
+    bool aligned = al(p->x) && p->x_sb % VS == 0 && p->x_sl % VS == 0 && p->x_sh % VS == 0;
+    aligned = aligned && (p->has_z ? al(p->dout_x) : (al(p->dout) && p->dout_sb % VS == 0 && p->dout_sl % VS == 0 && p->dout_sh % VS == 0));
+    const bool fast = aligned && p->headdim % (sizeof(T) == 2 ? 64 : 16) == 0;
     if (!p->CB && !dcb_recomputes_cb(p)) return BIMAMBA2_EINVAL;
-    const bool ring = fast && sizeof(T) == 2 && p->chunk_size % 64 == 0 && dcb_rows_in_32bit(p);
-    if (p->causal && !ring) return BIMAMBA2_EUNSUPPORTED;
+    const bool ring = aligned && sizeof(T) == 2 && p->chunk_size % 64 == 0 && p->headdim % 8 == 0 && dcb_rows_in_32bit(p);
+    if (p->causal && !(ring && fast)) return BIMAMBA2_EUNSUPPORTED;
     if (ring) launch_dcb_ring<T>(grid, p, nc, nqt);
     else if (fast) hipLaunchKernelGGL((bwd_dcb_kernel<T, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
     else hipLaunchKernelGGL((bwd_dcb_kernel<T, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
@@ -1895,7 +1921,8 @@ static int launch_dcb_t(const bimamba2_params *p) {
 }
 
 // Head slices where bimamba2_bwd owns dCB and the kernel reads C.B^T: float32, and 16-bit shapes whose state or headdim is no
-// multiple of what the rebuilding kernel takes (through registers, or the ring with a narrow state).  Where C.B^T is rebuilt the
+// multiple of what the rebuilding kernel takes (the ring with a narrow state or narrow heads; through registers where rows are
+// not aligned).  Where C.B^T is rebuilt the
 // number is dcb_slices()'s: every slice would rebuild it, and one slice shares its launch with the state passing.
 // A workgroup is one chain over its heads, 5 to 7 us a head through registers in float32, 3 to 5 in 16 bits and 1.5 in the ring,
 // so slices pay on a small grid until there are three workgroups on every CU; against them stands a launch that adds them up
@@ -1903,7 +1930,7 @@ static int launch_dcb_t(const bimamba2_params *p) {
 // in float32 fewer than six heads are cut only where all slices are on the chip at once.  us with one slice -> with the number
 // chosen here (-> with as many as three workgroups a CU would allow, where that is another number), the adding up included:
 //   float32, headdim 64: 16 heads in 2 groups, 320 tiles 56 -> 42 + 6; 24 heads, 256 tiles 112 -> 82; 4 heads, 192 tiles 23 (-> 28)
-//   16 bits, headdim 32 or 16: 24 heads, 64 tiles 94 -> 30; 17 heads, 240 tiles 70 -> 51 (-> 62); 8 heads, 320 tiles 43 (-> 49);
+//   16 bits through registers, headdim 32 or 16: 24 heads, 64 tiles 94 -> 30; 17 heads, 240 tiles 70 -> 51 (-> 62); 8 heads, 320 tiles 43 (-> 49);
 //     6 heads, 384 tiles 33 (-> 46); the rule loses at 7 heads, 176 tiles (32 -> 29) and 15 heads, 256 tiles (62 -> 56)
 //   ring, headdim 64, state 16: 48 heads, 64 tiles 62 -> 22; 24 heads, 256 tiles 36 -> 31; 16 heads, 160 tiles 26 -> 20 (-> 21);
 //     8 heads, 320 tiles 17 (-> 22); 4 heads, 192 tiles 10 (-> 17); 8 heads, 128 tiles 15 -> 16 (-> 19)

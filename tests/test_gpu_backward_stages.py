@@ -214,3 +214,20 @@ def test_dcb_between_the_merged_launches_in_sixteen_bits(ops, monkeypatch, N, dt
     monkeypatch.setattr(ops._Call, "workspace", with_dcb)
     for a, c in zip(own, bwd()):
         assert (a is None and c is None) or torch.equal(a, c)
+
+
+@pytest.mark.parametrize("P", [8, 16, 24, 32, 40, 64, 72, 128])
+@pytest.mark.parametrize("L,Q,dtype", [(64, 64, torch.bfloat16), (130, 128, torch.bfloat16), (449, 256, torch.float16)])
+def test_dcb_of_heads_that_are_no_whole_steps(ops, P, L, Q, dtype):
+    """The ring kernel brings rows in steps of 32 or 64 columns; what a narrower head leaves of them counts as zero.  Against the
+    float32 kernel on the same values: products of 16-bit values are exact in float32, so both differ by the order of sums over
+    P terms and by a unit in the last place of the exponentials (1e-6 of a value each)."""
+    b, H, G = 2, 6, 2
+    d = to_dev(make_case(b, L, H, P, G, 16, dtype))
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(5)).to(dtype).cuda()
+    csf, csb, dt = ops._chunk_cumsum_fwd(d["dt"], d["A"], Q, dt_bias=d["dt_bias"], dt_softplus=True)
+    CB = torch.randn(b, -(-L // Q), G, Q, Q, generator=torch.Generator().manual_seed(6)).cuda()
+    want = ops._chunk_scan_bwd_dcb(d["x"].float(), dt, csf, csb, dout.float(), CB, ngroups=G)
+    got = ops._chunk_scan_bwd_dcb(d["x"], dt, csf, csb, dout, CB, ngroups=G)
+    for g, w in zip(got, want):
+        assert float((g - w).norm() / w.norm()) < 4e-6

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 from oracle import bimamba2_oracle as O
-from helpers import make_case
+from tests.helpers import make_case
 
 pytestmark = pytest.mark.gpu
 
