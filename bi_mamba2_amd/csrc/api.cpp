@@ -401,8 +401,14 @@ int bimamba2_fwd(const bimamba2_params *p) {
     bimamba2_params q = *p;
     const size_t need = carve(&q, 0, p->workspace);
     if (need > 256 && (!p->workspace || p->workspace_bytes < need)) return BIMAMBA2_EWORKSPACE;
-    TRY(forward_cumsum_and_states(&q));
-    if (q.CB) TRY(bimamba2_bmm_chunk_fwd(&q));     // given by the caller, or carved because the scan kernel reads it
+    if (fwd_front_merged(&q)) {
+        REQUIRE(q.dt); REQUIRE(q.A); REQUIRE(q.x); REQUIRE(q.Bm); REQUIRE(q.Cm);
+        if (q.has_dt_bias) REQUIRE(q.dt_bias);
+        TRY(launch_fwd_front(&q));
+    } else {
+        TRY(forward_cumsum_and_states(&q));
+        if (q.CB) TRY(bimamba2_bmm_chunk_fwd(&q));     // given by the caller, or carved because the scan kernel reads it
+    }
     TRY(bimamba2_state_passing_fwd(&q));
     if (scan_recomputes_cb(&q, false) || fwd_scan_rebuilds_cb(&q)) q.CB = nullptr;
     TRY(bimamba2_chunk_scan_fwd(&q));

@@ -316,12 +316,14 @@ __device__ __forceinline__ int xt_index(int r, int k) {
 // last valid row and zeroed by scale().
 // The source element type S may differ from T (float32 states staged as 16-bit operands): a thread moves a block of
 // VK = 16/sizeof(T) rows (k) by VR = 16/sizeof(S) columns (r).
-template <typename T, int KTOT, int RTOT, int LDX, bool FAST, typename S, class F>
+// ROT (workgroups of NTHREADS only): the thread that takes the first block, so that several stages of few blocks each are
+// different threads' work.
+template <typename T, int KTOT, int RTOT, int LDX, bool FAST, int ROT = 0, typename S, class F>
 __device__ __forceinline__ void stage_transposed(T *dst, const S *src, int64_t ks, int kvalid, int rvalid, F scale) {
     constexpr int VK = 16 / sizeof(T), VR = 16 / sizeof(S), RB = RTOT / VR, NB = (KTOT / VK) * RB;
     const bool vec = FAST || aligned16(src, ks);
     const bool whole = !FAST && vec && rvalid % VR == 0;      // whole vectors: unconditional loads (see tile_load_kcontig)
-    for (int blk = threadIdx.x; blk < NB; blk += blockDim.x) {
+    for (int blk = ROT ? (threadIdx.x - ROT) & (NTHREADS - 1) : threadIdx.x; blk < NB; blk += blockDim.x) {
         const int rb = blk % RB, kb = blk / RB;
         float v[VK][VR];
         if (whole) {
@@ -365,13 +367,13 @@ __device__ __forceinline__ void stage_transposed(T *dst, const S *src, int64_t k
 }
 
 // same read of the source, two scaled images (used where both directions weight one operand differently)
-template <typename T, int KTOT, int RTOT, int LDX, bool FAST, typename S, class F1, class F2>
+template <typename T, int KTOT, int RTOT, int LDX, bool FAST, int ROT = 0, typename S, class F1, class F2>
 __device__ __forceinline__ void stage_transposed2(T *dst1, T *dst2, const S *src, int64_t ks, int kvalid, int rvalid,
                                                   F1 scale1, F2 scale2) {
     constexpr int VK = 16 / sizeof(T), VR = 16 / sizeof(S), RB = RTOT / VR, NB = (KTOT / VK) * RB;
     const bool vec = FAST || aligned16(src, ks);
     const bool whole = !FAST && vec && rvalid % VR == 0;
-    for (int blk = threadIdx.x; blk < NB; blk += blockDim.x) {
+    for (int blk = ROT ? (threadIdx.x - ROT) & (NTHREADS - 1) : threadIdx.x; blk < NB; blk += blockDim.x) {
         const int rb = blk % RB, kb = blk / RB;
         float v[VK][VR], s1[VK], s2[VK];
         if (whole) {

@@ -7,73 +7,19 @@
 // (the chunk-scan kernel itself lives in kernels_scan.hip)
 #include "common.hpp"
 #include "launch.hpp"
+#include "chunk_state_body.hpp"
 
 namespace bm2 {
 
-// =========================================================================================================
-// chunk cumsum: one wave per (b, c, h); lane i owns positions 4i..4i+3 of the chunk (Q <= 256)
-// =========================================================================================================
-// ACC: the type of the sums.  float32 problems take them in 64 bits and round once: a result there is off by little else than the
-// resolution of these sums (their differences are exponents), and with every addition rounded it was off by 1.7 times as much.
-// 16-bit results are not, and 64 bits would cost them 2 of 13 us over 2 x 16384 positions of 48 heads.
+// (what a wave of the chunk cumsum and a workgroup of the generic chunk-state kernel do: chunk_state_body.hpp)
 template <typename DT, typename ACC>
 __global__ __launch_bounds__(NTHREADS) void chunk_cumsum_fwd_kernel(const bimamba2_params p, int nc) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int h = blockIdx.x * 4 + wave, c = blockIdx.y, b = blockIdx.z;
     if (h >= p.nheads) return;
-    const int Q = p.chunk_size;
-    const int limit = min(Q, p.seqlen - c * Q);
-    const DT *dt = reinterpret_cast<const DT *>(p.dt) + b * p.dt_sb + (int64_t)c * Q * p.dt_sl + h * p.dt_sh;
-    const float A = p.A[h];
-    const float bias = p.has_dt_bias ? p.dt_bias[h] : 0.f;
-    float v[4];
-    ACC a[4], ar[4];                                  // ar: exponents of the reverse direction (differ with seq_idx only)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int q = lane * 4 + e;
-        float d = 0.f;
-        if (q < limit) {
-            d = to_f(dt[(int64_t)q * p.dt_sl]) + bias;
-            if (p.dt_softplus) d = d > 20.f ? d : log1pf(expf(d));
-            d = fminf(fmaxf(d, p.dt_min), p.dt_max);
-        }
-        v[e] = d;
-        a[e] = ar[e] = (ACC)d * A;
-        if (p.seq_idx && q < limit) {
-            // packed sequences: cut the forward recurrence in front of a sequence's first position, the reverse one
-            // behind its last
-            const int l = c * Q + q;
-            const int32_t *si = p.seq_idx + (int64_t)b * p.seqlen + l;
-            const int32_t cur = si[0];
-            if (l > 0 && si[-1] != cur) a[e] += BIMAMBA2_SEQ_CUT;
-            if (l + 1 < p.seqlen && si[1] != cur) ar[e] += BIMAMBA2_SEQ_CUT;
-        }
-    }
-    // forward inclusive scan, reverse inclusive scan
-    ACC pf[4], sb[4];
-    pf[0] = a[0]; pf[1] = pf[0] + a[1]; pf[2] = pf[1] + a[2]; pf[3] = pf[2] + a[3];
-    sb[3] = ar[3]; sb[2] = sb[3] + ar[2]; sb[1] = sb[2] + ar[1]; sb[0] = sb[1] + ar[0];
-    const ACC tot = pf[3], tot_r = sb[0];
-    const ACC before = wave_incl_prefix(tot, lane) - tot, after = wave_incl_suffix(tot_r, lane) - tot_r;
-    const int64_t o = (((int64_t)b * p.nheads + h) * nc + c) * Q;
-    if (Q % 4 == 0) {
-        // a lane's four positions are contiguous: 16-byte stores (the three tensors are contiguous and Q * 4 bytes per row)
-        if (lane * 4 < Q) {
-            *reinterpret_cast<f32x4 *>(p.dt_out + o + lane * 4) = f32x4{v[0], v[1], v[2], v[3]};
-            *reinterpret_cast<f32x4 *>(p.cs_f + o + lane * 4) = f32x4{(float)(before + pf[0]), (float)(before + pf[1]), (float)(before + pf[2]), (float)(before + pf[3])};
-            *reinterpret_cast<f32x4 *>(p.cs_b + o + lane * 4) = f32x4{(float)(after + sb[0]), (float)(after + sb[1]), (float)(after + sb[2]), (float)(after + sb[3])};
-        }
-        return;
-    }
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        const int q = lane * 4 + e;
-        if (q < Q) {
-            p.dt_out[o + q] = v[e];
-            p.cs_f[o + q] = (float)(before + pf[e]);
-            p.cs_b[o + q] = (float)(after + sb[e]);
-        }
-    }
+    float v[4], cf[4], cb[4];
+    chunk_cumsum_wave<DT, ACC>(p, b, c, h, lane, v, cf, cb);
+    chunk_cumsum_store(p, (((int64_t)b * p.nheads + h) * nc + c) * p.chunk_size, lane, v, cf, cb);
 }
 
 // Boundaries of the packed sequences per chunk, for the host's choice of the chunk size: a wave per (batch, chunk) reads its
@@ -101,14 +47,14 @@ __global__ __launch_bounds__(64) void seq_boundaries_kernel(const bimamba2_param
 // =========================================================================================================
 // CB[t, s] = sum_n C[t, n] B[s, n]
 // =========================================================================================================
+template <typename T> constexpr int BMM_FWD_LDS = 2 * 64 * Mma<T>::LD * (int)sizeof(T);
+// lds: BMM_FWD_LDS bytes; st, tt: tile of columns and of rows; bcg: (batch, chunk, group)
 template <typename T>
-__global__ __launch_bounds__(NTHREADS) void bmm_chunk_fwd_kernel(const bimamba2_params p, int nc) {
+__device__ __forceinline__ void bmm_chunk_fwd_body(const bimamba2_params &p, int nc, int st, int tt, int bcg, char *lds) {
     constexpr int LD = Mma<T>::LD;
-    __shared__ __attribute__((aligned(16))) T As[64 * LD];
-    __shared__ __attribute__((aligned(16))) T Bs[64 * LD];
+    T *As = reinterpret_cast<T *>(lds), *Bs = As + 64 * LD;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int st = blockIdx.x, tt = blockIdx.y;
-    const int g = blockIdx.z % p.ngroups, bc = blockIdx.z / p.ngroups, c = bc % nc, b = bc / nc;
+    const int g = bcg % p.ngroups, bc = bcg / p.ngroups, c = bc % nc, b = bc / nc;
     const int Q = p.chunk_size, N = p.dstate;
     const int limit = min(Q, p.seqlen - c * Q);
     const T *Cp = reinterpret_cast<const T *>(p.Cm) + b * p.C_sb + ((int64_t)c * Q + tt * 64) * p.C_sl + g * p.C_sg;
@@ -121,8 +67,8 @@ __global__ __launch_bounds__(NTHREADS) void bmm_chunk_fwd_kernel(const bimamba2_
         __syncthreads();
         mma_tile<T, 4>(acc, As + wave * 16 * LD, Bs, lane);
     }
-    float *out = p.CB + (int64_t)blockIdx.z * Q * Q;
-    float *outT = p.CBT ? p.CBT + (int64_t)blockIdx.z * Q * Q : nullptr;   // CBT[s, t] = CB[t, s], read by the dx kernel
+    float *out = p.CB + (int64_t)bcg * Q * Q;
+    float *outT = p.CBT ? p.CBT + (int64_t)bcg * Q * Q : nullptr;   // CBT[s, t] = CB[t, s], read by the dx kernel
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
@@ -143,97 +89,31 @@ __global__ __launch_bounds__(NTHREADS) void bmm_chunk_fwd_kernel(const bimamba2_
     }
 }
 
-// =========================================================================================================
-// chunk state (DSTATES = false):  S_f[p,n] = sum_k x[k,p] B[k,n] e^{cs_f[Q-1]-cs_f[k]} dt[k],  S_b with
-//                                 e^{cs_b[0]-cs_b[k]}
-// gradient of the chunk-entry states (DSTATES = true):  dprev_f[p,n] = sum_k dy[k,p] C[k,n] e^{cs_f[k]},
-//                                 dprev_b with e^{cs_b[k]}
-// =========================================================================================================
-// Both operands have K = chunk position as their slow dimension, so both are staged transposed (8x8 in-register
-// transposes) into LDS, KH positions at a time; the decay weights are applied to the B-side image while staging.
+template <typename T>
+__global__ __launch_bounds__(NTHREADS) void bmm_chunk_fwd_kernel(const bimamba2_params p, int nc) {
+    __shared__ __attribute__((aligned(16))) char lds[BMM_FWD_LDS<T>];
+    bmm_chunk_fwd_body<T>(p, nc, blockIdx.x, blockIdx.y, blockIdx.z, lds);
+}
+
 template <typename T, bool DSTATES, bool FAST>
 __global__ __launch_bounds__(NTHREADS) void chunk_state_kernel(const bimamba2_params p, int nc) {
-    typedef Mma<T> M;
-    constexpr int KPL = M::KPL, KSTEP = M::KSTEP;
-    constexpr int KH = sizeof(T) == 2 ? 128 : 64;          // chunk positions staged per round
-    constexpr int LDX = KH + 16 / (int)sizeof(T);
-    __shared__ __attribute__((aligned(16))) T xT[64 * LDX];
-    __shared__ __attribute__((aligned(16))) T Bf[64 * LDX];
-    __shared__ __attribute__((aligned(16))) T Bb[64 * LDX];
-    __shared__ float wf[BIMAMBA2_MAX_CHUNK], wb[BIMAMBA2_MAX_CHUNK];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int lr = lane & 15, lg = lane >> 4;
-    const int nt = blockIdx.x, pt = blockIdx.y;
-    const int h = blockIdx.z % p.nheads, bc = blockIdx.z / p.nheads, c = bc % nc, b = bc / nc;
-    const int g = h / (p.nheads / p.ngroups);
-    const int Q = p.chunk_size, N = p.dstate, P = p.headdim;
-    const int limit = min(Q, p.seqlen - c * Q);
-    const int64_t o = (((int64_t)b * p.nheads + h) * nc + c) * Q;
-    for (int q = threadIdx.x; q < Q; q += NTHREADS) {
-        float f = 0.f, r = 0.f;
-        if (q < limit) {
-            if (DSTATES) {
-                f = __expf(p.cs_f[o + q]);
-                r = __expf(p.cs_b[o + q]);
-            } else {
-                const float d = p.dt_out[o + q];
-                f = __expf(p.cs_f[o + Q - 1] - p.cs_f[o + q]) * d;
-                r = __expf(p.cs_b[o] - p.cs_b[o + q]) * d;
-            }
-        }
-        wf[q] = f;
-        wb[q] = r;
+    __shared__ __attribute__((aligned(16))) char lds[ChunkStateMap<T>::LDS];
+    chunk_state_body<T, DSTATES, FAST>(p, nc, blockIdx.x, blockIdx.y, blockIdx.z, lds);
+}
+
+// The forward pass's first kernels in one launch, where the scan kernel reads C.B^T: the first nstate workgroups form chunk states
+// (and the cumulative sums), the others the tiles of C.B^T.  Neither needs the other, none of them fills the chip at the sizes
+// where it matters, and a launch is 3 to 5 us.
+template <typename T, bool FAST>
+__global__ __launch_bounds__(NTHREADS) void fwd_front_kernel(const bimamba2_params p, int nc, int nnt, int npt, int nstate, int nqt) {
+    constexpr int LDS = ChunkStateMap<T>::LDS > BMM_FWD_LDS<T> ? ChunkStateMap<T>::LDS : BMM_FWD_LDS<T>;
+    __shared__ __attribute__((aligned(16))) char lds[LDS];
+    const int id = blockIdx.x;
+    if (id < nstate) chunk_state_body<T, false, FAST, true>(p, nc, id % nnt, id / nnt % npt, id / (nnt * npt), lds);
+    else {
+        const int k = id - nstate;
+        bmm_chunk_fwd_body<T>(p, nc, k % nqt, k / nqt % nqt, k / (nqt * nqt), lds);
     }
-    const T *xp;
-    int64_t xs;
-    if (DSTATES) {
-        const T *src = reinterpret_cast<const T *>(p.has_z ? p.dout_x : p.dout);
-        if (p.has_z) { xs = (int64_t)p.nheads * P; xp = src + ((int64_t)b * p.seqlen + (int64_t)c * Q) * xs + (int64_t)h * P; }
-        else { xs = p.dout_sl; xp = src + b * p.dout_sb + (int64_t)c * Q * xs + h * p.dout_sh; }
-    } else {
-        xs = p.x_sl;
-        xp = reinterpret_cast<const T *>(p.x) + b * p.x_sb + (int64_t)c * Q * xs + h * p.x_sh;
-    }
-    xp += pt * 64;
-    const T *bp;
-    int64_t bs;
-    if (DSTATES) { bs = p.C_sl; bp = reinterpret_cast<const T *>(p.Cm) + b * p.C_sb + (int64_t)c * Q * bs + g * p.C_sg; }
-    else { bs = p.B_sl; bp = reinterpret_cast<const T *>(p.Bm) + b * p.B_sb + (int64_t)c * Q * bs + g * p.B_sg; }
-    bp += nt * 64;
-    f32x4 accf[4] = {}, accb[4] = {};
-    for (int k0 = 0; k0 < limit; k0 += KH) {
-        __syncthreads();       // weights written / previous round consumed
-        const int kv = limit - k0;
-        stage_transposed<T, KH, 64, LDX, FAST>(xT, xp + (int64_t)k0 * xs, xs, kv, P - pt * 64,
-                                               [&](int k) { return k < kv ? 1.f : 0.f; });
-        stage_transposed2<T, KH, 64, LDX, FAST>(Bf, Bb, bp + (int64_t)k0 * bs, bs, kv, N - nt * 64,
-                                                [&](int k) { return k < kv ? wf[k0 + k] : 0.f; },
-                                                [&](int k) { return k < kv ? wb[k0 + k] : 0.f; });
-        __syncthreads();
-        const int kend = min(KH, (kv + KSTEP - 1) / KSTEP * KSTEP);
-        for (int ks = 0; ks < kend; ks += KSTEP) {
-            const int kq = ks + lg * KPL;
-            const typename M::Frag a = M::load(xT + xt_index<T, LDX>(wave * 16 + lr, kq));
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (!FAST && nt * 64 + j * 16 >= N) continue;      // (uniform) narrow states: nothing in this column tile
-                accf[j] = M::mma(a, M::load(Bf + xt_index<T, LDX>(j * 16 + lr, kq)), accf[j]);
-                accb[j] = M::mma(a, M::load(Bb + xt_index<T, LDX>(j * 16 + lr, kq)), accb[j]);
-            }
-        }
-    }
-    float *of = (DSTATES ? p.dstates_f : p.states_f) + (int64_t)blockIdx.z * P * N;
-    float *ob = (DSTATES ? p.dstates_b : p.states_b) + (int64_t)blockIdx.z * P * N;
-#pragma unroll
-    for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int pp = pt * 64 + wave * 16 + lg * 4 + i, n = nt * 64 + j * 16 + lr;
-            if (pp < P && n < N) {
-                of[(int64_t)pp * N + n] = accf[j][i];
-                ob[(int64_t)pp * N + n] = accb[j][i];
-            }
-        }
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -1107,6 +987,46 @@ int launch_chunk_state(const bimamba2_params *p, bool dstates, bool cumsum) {
         case BIMAMBA2_F32: return launch_chunk_state_t<float>(p, dstates, cumsum);
         case BIMAMBA2_BF16: return launch_chunk_state_t<bf16_t>(p, dstates, cumsum);
         case BIMAMBA2_F16: return launch_chunk_state_t<f16_t>(p, dstates, cumsum);
+        default: return BIMAMBA2_EUNSUPPORTED;
+    }
+}
+
+// whether the generic chunk-state kernel is the one that runs for float32 per-chunk states, and whether its loads are unconditional
+static bool chunk_state_generic(const bimamba2_params *p, bool &fast) {
+    const int vs = p->dtype == BIMAMBA2_F32 ? 4 : 8;
+    auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    auto mult = [vs](int64_t a, int64_t b, int64_t c) { return a % vs == 0 && b % vs == 0 && c % vs == 0; };
+    fast = p->headdim % 64 == 0 && p->dstate % 64 == 0 && al(p->Bm) && mult(p->B_sb, p->B_sl, p->B_sg) && al(p->x) && mult(p->x_sb, p->x_sl, p->x_sh);
+    return !p->causal && !(fast && p->dtype != BIMAMBA2_F32 && p->chunk_size % 32 == 0);
+}
+
+// chunk cumsum, chunk states and C.B^T as one launch
+bool fwd_front_merged(const bimamba2_params *p) {
+    bool fast;
+    return p->CB && p->states_f && p->states_b && chunk_state_generic(p, fast);
+}
+
+template <typename T> static int launch_fwd_front_t(const bimamba2_params *p, bool fast) {
+    const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, nnt = (p->dstate + 63) / 64, npt = (p->headdim + 63) / 64;
+    const int nstate = nnt * npt * p->batch * nc * p->nheads;
+    const dim3 grid(nstate + nqt * nqt * p->batch * nc * p->ngroups);
+    if constexpr (sizeof(T) == 4) {
+        if (fast) {
+            hipLaunchKernelGGL((fwd_front_kernel<T, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
+            return check_launch();
+        }
+    }
+    hipLaunchKernelGGL((fwd_front_kernel<T, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
+    return check_launch();
+}
+
+int launch_fwd_front(const bimamba2_params *p) {
+    bool fast;
+    if (!chunk_state_generic(p, fast)) return BIMAMBA2_EINVAL;          // (the caller checked fwd_front_merged())
+    switch (p->dtype) {
+        case BIMAMBA2_F32: return launch_fwd_front_t<float>(p, fast);
+        case BIMAMBA2_BF16: return launch_fwd_front_t<bf16_t>(p, fast);
+        case BIMAMBA2_F16: return launch_fwd_front_t<f16_t>(p, fast);
         default: return BIMAMBA2_EUNSUPPORTED;
     }
 }

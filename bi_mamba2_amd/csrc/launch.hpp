@@ -6,6 +6,8 @@
 
 namespace bm2 {
 
+struct BlockId { int x, y, z; };      // a workgroup's place in the grid of its kernel, or of its role in a launch of several
+
 static inline int check_launch() { return hipGetLastError() == hipSuccess ? BIMAMBA2_OK : BIMAMBA2_ELAUNCH; }
 
 // Width of the headdim column tile of the chunk-scan kernels (64 columns for 16-bit types, 32 for float32, less for narrow
@@ -24,6 +26,9 @@ int launch_seq_boundaries(const bimamba2_params *p, int32_t *counts);
 int launch_bmm_chunk_fwd(const bimamba2_params *p);
 int launch_chunk_state(const bimamba2_params *p, bool dstates, bool cumsum = false);   // cumsum: also does the chunk cumsum
 bool chunk_state_does_cumsum(const bimamba2_params *p);
+// chunk cumsum, chunk states and C.B^T as one launch, where fwd_front_merged() says it exists
+bool fwd_front_merged(const bimamba2_params *p);
+int launch_fwd_front(const bimamba2_params *p);
 // the forward pass may keep its per-chunk states in states16_f/b only (16-bit type, no float32 state tensors)
 bool chunk_states_in_16bit(const bimamba2_params *p);
 // the chunk-state kernel whose workgroups walk through several heads of one (batch, chunk): where it is used, and its launch

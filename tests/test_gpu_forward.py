@@ -152,3 +152,32 @@ def test_stages_rebuild_cb_when_it_is_not_given(ops, dtype):
     # shapes whose kernels cannot rebuild CB refuse a missing CB instead of reading a null pointer
     with pytest.raises(ValueError):
         ops._chunk_scan_fwd(None, d["x"].float(), dt_out, csf, csb, d["C"].float(), pf, pb, B=d["B"].float())
+
+
+@pytest.mark.parametrize("b,L,H,P,G,N,Q,dtype,dt_dtype", [
+    (2, 130, 3, 16, 3, 16, 64, torch.float32, torch.float32),        # several tiles of C.B^T, one of states
+    (1, 257, 2, 72, 1, 80, 256, torch.float32, torch.float16),       # four tiles of states: the first one's workgroup writes the sums
+    (1, 64, 2, 64, 1, 64, 64, torch.float32, torch.bfloat16),
+    (2, 75, 4, 24, 2, 24, 50, torch.bfloat16, torch.bfloat16),       # chunk no multiple of 4 positions a lane
+    (1, 300, 2, 8, 1, 136, 100, torch.float16, torch.float32),
+])
+def test_first_kernels_in_one_launch(b, L, H, P, G, N, Q, dtype, dt_dtype):
+    """bimamba2_fwd's launch of cumulative sums, chunk states and C.B^T against the stages one by one"""
+    from bi_mamba2_amd import ops
+    d = to_dev(make_case(b, L, H, P, G, N, dtype))
+    dt = d["dt"].to(dt_dtype)
+    res = ops._mamba_chunk_scan_combined_fwd(d["x"], dt, d["A"], d["B"], d["C"], Q, D=d["D"], dt_bias=d["dt_bias"], dt_softplus=True)
+    csf, csb, dt_out = ops._chunk_cumsum_fwd(dt, d["A"], Q, dt_bias=d["dt_bias"], dt_softplus=True)
+    for got, want in zip(res[2:5], (dt_out, csf, csb)):
+        if dtype == torch.float32:
+            assert torch.equal(got, want)
+        else:                                # (that stage alone always sums in 64 bits: up to 256 additions rounded to 24 bits here)
+            torch.testing.assert_close(got, want, rtol=256 * 2.0 ** -24, atol=0)
+    dt_out, csf, csb = res[2:5]
+    sf, sb = ops._chunk_state_fwd(d["B"], d["x"], dt_out, csf, csb)
+    sf, sb = ops._state_passing_fwd(sf, sb, csf, csb)[:2]
+    CB = ops._bmm_chunk_fwd(d["C"], d["B"], Q)
+    out = ops._chunk_scan_fwd(CB, d["x"], dt_out, csf, csb, d["C"], sf, sb, D=d["D"])[0]
+    # the weights of the states come from the sums in registers instead of memory: the same values, the same order of products
+    for got, want in zip((res[5], res[6], res[0]), (sf, sb, out)):
+        assert torch.equal(got, want)
