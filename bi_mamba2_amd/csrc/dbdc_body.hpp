@@ -33,7 +33,10 @@ template <typename T, int QT> struct DbdcMap {
     static constexpr int SB = NBUF * IMAGE, SFS = 2 * NBUF * IMAGE, SBS = SFS + 4 * DBDC_HEADS * ROWS, LDS = SBS + 4 * DBDC_HEADS * ROWS;
 };
 // lds: DbdcMap::LDS bytes, 16-byte aligned; bid: (batch, chunk, group), row tile, head slice
-template <typename T, int NT, int QT, bool IS_DB, bool FAST, bool UNI = false>
+// NT: 64-column tiles of the state dimension, NJ: 16-column tiles in use of each (below 4 with NT = 1 only): a narrow state does not
+// hold registers for 64 columns, and two workgroups fit a CU, which cover each other's waits (one step of one head is a chain of
+// 2 to 3 us: requests, LDS image, barrier, products, sums).  4 x 2048, bfloat16, 16 heads of 16, dstate 16: 17 -> 11 us each.
+template <typename T, int NT, int QT, bool IS_DB, bool FAST, bool UNI = false, int NJ = 4>
 __device__ __forceinline__ void bwd_dbdc_body(const bimamba2_params &p, int nc, int hps, BlockId bid, char *lds) {
     typedef Mma<T> M;
     typedef DbdcMap<T, QT> Map;
@@ -161,13 +164,13 @@ __device__ __forceinline__ void bwd_dbdc_body(const bimamba2_params &p, int nc, 
     int64_t cbs;
     if (IS_DB) { cbs = p.B_sl; cbp = reinterpret_cast<const T *>(p.Bm) + b * p.B_sb + ((int64_t)c * Q + r0) * cbs + g * p.B_sg; }
     else { cbs = p.C_sl; cbp = reinterpret_cast<const T *>(p.Cm) + b * p.C_sb + ((int64_t)c * Q + r0) * cbs + g * p.C_sg; }
-    float creg[NT][QT][4][4];
+    float creg[NT][QT][NJ][4];
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
         for (int q = 0; q < QT; ++q)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     // unconditional loads from clamped addresses (conditional ones are waited for one by one), masked after
@@ -175,7 +178,7 @@ __device__ __forceinline__ void bwd_dbdc_body(const bimamba2_params &p, int nc, 
                     const float v = to_f(cbp[(int64_t)min(tl[q][i], limit - 1 - r0) * cbs + min(n, N - 1)]);
                     creg[nt][q][j][i] = (r0 + tl[q][i] < limit && n < N) ? v : 0.f;
                 }
-    f32x4 tot[NT][QT][4] = {};
+    f32x4 tot[NT][QT][NJ] = {};
 
     int step = 0;
     for (int hh = hh0; hh < hh_end; ++hh) {
@@ -189,7 +192,7 @@ __device__ __forceinline__ void bwd_dbdc_body(const bimamba2_params &p, int nc, 
 #pragma unroll
         for (int nt = 0; nt < NT; ++nt) {
             if (nt >= nnt) break;
-            f32x4 tf[QT][4] = {}, tb[QT][4] = {};
+            f32x4 tf[QT][NJ] = {}, tb[QT][NJ] = {};
             for (int kc = 0; kc < nkc; ++kc, ++step) {
                 const int buf = NBUF == 2 ? (step & 1) : 0;
                 if (NBUF == 1) __syncthreads();            // the single image is still being read by slower waves
@@ -206,7 +209,7 @@ __device__ __forceinline__ void bwd_dbdc_body(const bimamba2_params &p, int nc, 
                     if (!FAST && kc * KC + ks * KSTEP >= P) continue;      // (uniform) nothing there: narrow heads and states
                     const int kq = ks * KSTEP + lg * KPL;
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
+                    for (int j = 0; j < NJ; ++j) {
                         if (!FAST && nt * 64 + j * 16 >= N) continue;
                         const typename M::Frag bff = M::load(sF[buf] + xt_index<T, LDX>(j * 16 + lr, kq));
                         const typename M::Frag bfb = UNI ? bff : M::load(sB[buf] + xt_index<T, LDX>(j * 16 + lr, kq));
@@ -224,7 +227,7 @@ __device__ __forceinline__ void bwd_dbdc_body(const bimamba2_params &p, int nc, 
                 for (int i = 0; i < 4; ++i) {
                     const float sf = sfs[hh - hh0][tl[q][i]], sb = sbs[hh - hh0][tl[q][i]];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
+                    for (int j = 0; j < NJ; ++j) {
                         uf[q][i] += tf[q][j][i] * creg[nt][q][j][i];
                         ub[q][i] += tb[q][j][i] * creg[nt][q][j][i];
                         tot[nt][q][j][i] += sf * tf[q][j][i] + sb * tb[q][j][i];
@@ -249,7 +252,7 @@ __device__ __forceinline__ void bwd_dbdc_body(const bimamba2_params &p, int nc, 
 #pragma unroll
         for (int q = 0; q < QT; ++q)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int j = 0; j < NJ; ++j)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int n = nt * 64 + j * 16 + lr, r = r0 + tl[q][i];

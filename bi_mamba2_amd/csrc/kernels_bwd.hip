@@ -382,22 +382,26 @@ int choose_dbdc_heads(const bimamba2_params *p) {
     const int64_t tiles = (int64_t)p->batch * nc * p->ngroups * ((p->chunk_size + 127) / 128);
     const double steps = ((p->headdim + 63) / 64) * ((p->dstate + 63) / 64);                             // per head
     const double slice_cost = (double)p->batch * p->seqlen * p->ngroups * p->dstate * 8 / 5e6 / 1.5;     // one partial sum at 5 TB/s, in steps of 1.5 us
+    const int64_t places = p->dstate <= 32 ? 512 : 256;       // workgroups on the chip at once (narrow states: two to a CU)
     int best = DBDC_HEADS;
     double best_cost = 0;
     for (int k = DBDC_HEADS; k >= 1; --k) {
         const int slices = (hpg + k - 1) / k;
         if (k < DBDC_HEADS && (slices > DBDC_SLICES_MAX || (hpg + slices - 1) / slices != k)) continue;  // (the fewest heads for this many slices)
-        const double rounds = (double)((tiles * slices + 255) / 256);
+        const double rounds = (double)((tiles * slices + places - 1) / places);
         const double cost = rounds * (3 + steps * std::min(k, hpg)) + slices * slice_cost;
         if (k == DBDC_HEADS || cost < best_cost) { best = k; best_cost = cost; }
     }
     return best;
 }
 
-template <typename T, int NT, int QT, bool IS_DB, bool FAST, bool UNI = false>
-__global__ __launch_bounds__(DBDC_THREADS) void bwd_dbdc_kernel(const bimamba2_params p, int nc, int hps) {
+// Two waves to a SIMD, said explicitly: with the bound left out the two-tile variant takes 140 us instead of 40 (float32, heads of 16,
+// dstate 128, 4 x 2048, 16 heads; the same registers, another order of instructions).  With all four column tiles the registers do not allow more: held to
+// four waves it spills 17 to 43 of them (33 -> 54 us).
+template <typename T, int NT, int QT, bool IS_DB, bool FAST, bool UNI = false, int NJ = 4>
+__global__ __launch_bounds__(DBDC_THREADS, NJ < 4 ? 4 : 2) void bwd_dbdc_kernel(const bimamba2_params p, int nc, int hps) {
     __shared__ __attribute__((aligned(16))) char lds[DbdcMap<T, QT>::LDS];
-    bwd_dbdc_body<T, NT, QT, IS_DB, FAST, UNI>(p, nc, hps, BlockId{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z}, lds);
+    bwd_dbdc_body<T, NT, QT, IS_DB, FAST, UNI, NJ>(p, nc, hps, BlockId{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z}, lds);
 }
 
 // ---------------------------------------------------------------------------------------------------------
@@ -825,6 +829,8 @@ static int launch_dbdc_t(const bimamba2_params *p) {
         return BIMAMBA2_EUNSUPPORTED;
     }
     if (nt == 1 && qt == 2) BM2_DBDC(1, 2);
+    else if (p->dstate <= 16) hipLaunchKernelGGL((bwd_dbdc_kernel<T, 1, 1, IS_DB, false, false, 1>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));
+    else if (p->dstate <= 32) hipLaunchKernelGGL((bwd_dbdc_kernel<T, 1, 1, IS_DB, false, false, 2>), grid, dim3(DBDC_THREADS), 0, stream_of(p), *p, nc, dbdc_heads(p));
     else if (nt == 1) BM2_DBDC(1, 1);
     else if (nt == 2) BM2_DBDC(2, 1);
     else if (nt <= 4) BM2_DBDC(4, 1);

@@ -231,3 +231,31 @@ def test_dcb_of_heads_that_are_no_whole_steps(ops, P, L, Q, dtype):
     got = ops._chunk_scan_bwd_dcb(d["x"], dt, csf, csb, dout, CB, ngroups=G)
     for g, w in zip(got, want):
         assert float((g - w).norm() / w.norm()) < 4e-6
+
+
+@pytest.mark.parametrize("N", [8, 16, 20, 32, 36, 64])
+@pytest.mark.parametrize("H,G,P,L,Q,dtype", [(6, 2, 16, 130, 128, torch.bfloat16), (8, 1, 72, 75, 64, torch.float32), (3, 3, 32, 257, 256, torch.float16)])
+def test_state_parts_of_db_and_dc_with_narrow_states(ops, N, H, G, P, L, Q, dtype):
+    """one, two or four column tiles of the state: dB's and dC's state parts and the decays' gradients against float64"""
+    b, hpg = 2, H // G
+    d = to_dev(make_case(b, L, H, P, G, N, dtype))
+    gen = torch.Generator().manual_seed(9)
+    csf, csb, dt = ops._chunk_cumsum_fwd(d["dt"], d["A"], Q, dt_bias=d["dt_bias"], dt_softplus=True)
+    nc = csf.shape[2]
+    sf, sb = (torch.randn(b, nc, H, P, N, generator=gen).cuda() for _ in range(2))
+    dout = torch.randn(b, L, H, P, generator=gen).to(dtype).cuda()
+    pad = lambda t: F.pad(t.double(), (0, 0, 0, 0, 0, nc * Q - L)).view(b, nc, Q, *t.shape[2:])
+    # the kernels' operands: states rounded to the inputs' type; products in float32, rows scaled afterwards
+    r = lambda s: s.to(dtype).double()
+    scale = lambda e: e.double().exp().permute(0, 2, 3, 1)                                 # (b, nc, Q, H)
+    grp = lambda t: t.view(b, nc, Q, G, hpg, N).sum(4)
+    wide = lambda t: pad(t).repeat_interleave(hpg, 3)
+    for got, rows, mate, wf, wb in (
+            (ops._chunk_state_bwd_db(d["x"], dt, csf, csb, sf, sb, B=d["B"], ngroups=G), d["x"], d["B"], dt.double().permute(0, 2, 3, 1) * scale(csf[..., -1:] - csf), dt.double().permute(0, 2, 3, 1) * scale(csb[..., :1] - csb)),
+            (ops._chunk_scan_bwd_dC(sf, sb, csf, csb, dout, C=d["C"], ngroups=G), dout, d["C"], scale(csf), scale(csb))):
+        tf, tb = (torch.einsum("bcqhp,bchpn->bcqhn", pad(rows), r(s)) for s in (sf, sb))
+        want = grp(wf[..., None] * tf + wb[..., None] * tb).reshape(b, nc * Q, G, N)[:, :L]
+        assert float((got[0].sum(0) if got[0].dim() == 5 else got[0]).sub(want).norm() / want.norm()) < 1e-5
+        for g, w, t in ((got[1], wf, tf), (got[2], wb, tb)):
+            want = (w * (t * wide(mate)).sum(-1)).permute(0, 3, 1, 2).reshape(b, H, -1)[:, :, :L]
+            assert float((g.reshape(b, H, -1)[:, :, :L] - want).norm() / want.norm()) < 1e-5
