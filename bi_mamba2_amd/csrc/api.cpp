@@ -361,12 +361,17 @@ int bimamba2_chunk_scan_bwd_dc(const bimamba2_params *p) {
     return launch_bwd_dbdc(p, false);
 }
 
-int bimamba2_chunk_scan_bwd_dcb(const bimamba2_params *p) {
+static int check_bwd_dcb(const bimamba2_params *p) {
     TRY(check_problem(p));
     REQUIRE(p->x); REQUIRE(p->dt_out); REQUIRE(p->cs_f); REQUIRE(p->cs_b);
     if (!p->CB && !(p->Cm && p->Bm && dcb_recomputes_cb(p))) return BIMAMBA2_EINVAL;   // without CB the kernel rebuilds it from Cm, Bm
     REQUIRE(p->dCB); REQUIRE(p->dCBT); REQUIRE(p->da_intra);
     if (p->has_z) REQUIRE(p->dout_x); else REQUIRE(p->dout);
+    return BIMAMBA2_OK;
+}
+
+int bimamba2_chunk_scan_bwd_dcb(const bimamba2_params *p) {
+    TRY(check_bwd_dcb(p));
     return launch_bwd_dcb(p);
 }
 
@@ -450,13 +455,19 @@ int bimamba2_bwd(const bimamba2_params *p) {
     const bool dcb16 = !p->dCB && !p->dCBT && bwd_dcb_sp_merged(&q) && bwd_tail_merged(&q);
     const bool need_cbt = !scan_recomputes_cb(&q, true), need_cb = need_cbt || !dcb_recomputes_cb(&q);
     const bool saved_cb = (p->fwd_saved & 2) && p->CB && p->CBT;
-    if (need_cb && saved_cb) {}                    // left there by the forward pass
-    else if (need_cb) TRY(bimamba2_bmm_chunk_fwd(&q));  // CB for the dCB kernel, CB^T for the dx kernel, unless they rebuild it
-    else q.CB = nullptr;
+    const bool form_cb = need_cb && !saved_cb;     // (else left there by the forward pass)
+    if (!need_cb) q.CB = nullptr;
     // dz and dstates as one launch where the kernel for it exists (dout_x goes from the first to the second inside the workgroup)
-    const bool dz_dstates = q.has_z && bwd_dz_dstates_fused(&q);
+    const bool dz_dstates = q.has_z && bwd_dz_dstates_fused(&q), dz_bmm = q.has_z && !dz_dstates && form_cb;
+    if (form_cb && !dz_bmm) TRY(bimamba2_bmm_chunk_fwd(&q));  // CB for the dCB kernel, CB^T for the dx kernel, unless they rebuild it
     if (dz_dstates) TRY(bimamba2_chunk_scan_bwd_dz_dstates(&q));
-    else if (q.has_z) TRY(bimamba2_chunk_scan_bwd_dz(&q));
+    else if (dz_bmm) {
+        REQUIRE(q.z); REQUIRE(q.dout); REQUIRE(q.out_x); REQUIRE(q.dz); REQUIRE(q.dout_x); REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.CB);
+        TRY(launch_bwd_dz_bmm(&q));
+    } else if (q.has_z) TRY(bimamba2_chunk_scan_bwd_dz(&q));
+    // the last launch adds up the head slices of dCB where it is the one that does so
+    const bool tail_small = !bwd_tail_merged(&q) && bwd_tail_small(&q);
+    const int ncb = tail_small && !p->dCB && !p->dCBT && !bwd_dcb_sp_merged(&q) ? dcb_slices(&q) : 1;
     // the dCB kernel is bound by instruction issue and moves little data: right behind dz it runs while the memory system
     // still writes back dz's output, which the memory-bound kernels after it would otherwise wait behind
     if (bwd_dcb_sp_merged(&q)) {
@@ -469,7 +480,8 @@ int bimamba2_bwd(const bimamba2_params *p) {
         if (q.has_z) REQUIRE(q.dout_x); else REQUIRE(q.dout);
         TRY(launch_bwd_dcb_sp(&q, dcb16));
     } else {
-        TRY(bimamba2_chunk_scan_bwd_dcb(&q));
+        TRY(check_bwd_dcb(&q));
+        TRY(launch_bwd_dcb(&q, ncb == 1));
         if (!dz_dstates) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
         TRY(bimamba2_chunk_scan_bwd_dc(&q));           // (between the two memory-bound state kernels: measured best)
         TRY(bimamba2_state_passing_bwd(&q));
@@ -497,6 +509,10 @@ int bimamba2_bwd(const bimamba2_params *p) {
         REQUIRE(q.ddt); REQUIRE(q.dA); REQUIRE(q.dB); REQUIRE(q.dC);
         if (bwd_tail_merged(&q)) {
             TRY(launch_bwd_tail(&qc, &jobs, dcb16));
+        } else if (tail_small) {
+            REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dt); REQUIRE(q.A);
+            if (q.has_dt_bias) REQUIRE(q.dt_bias);
+            TRY(launch_bwd_tail_small(&qc, &jobs, ncb));
         } else {
             TRY(bimamba2_bmm_chunk_bwd(&q));
             TRY(launch_chunk_cumsum_bwd(&qc, &jobs));

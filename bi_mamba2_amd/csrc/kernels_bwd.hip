@@ -10,6 +10,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
+#include "bmm_fwd_body.hpp"
 #include "dbdc_body.hpp"
 #include "dcb_body.hpp"
 
@@ -88,7 +89,7 @@ int launch_reduce_jobs(const ReduceJobs &jobs, hipStream_t stream) {
 // dz = dout * out_x * sigmoid(z) (1 + z (1 - sigmoid(z)));  dout_x = dout * z * sigmoid(z)
 // =========================================================================================================
 template <typename T>
-__global__ __launch_bounds__(NTHREADS) void bwd_dz_kernel(const bimamba2_params p) {
+__device__ __forceinline__ void bwd_dz_body(const bimamba2_params &p, int id, int nblocks) {
     constexpr int VS = 16 / sizeof(T);
     const int P = p.headdim;
     const int pv = (P + VS - 1) / VS;
@@ -103,7 +104,7 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dz_kernel(const bimamba2_params 
     // the kernel's instructions otherwise)
     const bool packed = P % VS == 0 && p.z_sh == P && p.z_sl == (int64_t)p.nheads * P && p.z_sb == (int64_t)p.seqlen * p.nheads * P &&
                         p.dout_sh == P && p.dout_sl == p.z_sl && p.dout_sb == p.z_sb;
-    for (int64_t idx = blockIdx.x * (int64_t)NTHREADS + threadIdx.x; idx < nrows * pv; idx += (int64_t)gridDim.x * NTHREADS) {
+    for (int64_t idx = id * (int64_t)NTHREADS + threadIdx.x; idx < nrows * pv; idx += (int64_t)nblocks * NTHREADS) {
         const T *zp, *dp;
         int64_t o;
         int c0;
@@ -157,9 +158,40 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dz_kernel(const bimamba2_params 
     }
 }
 
-int launch_bwd_dz(const bimamba2_params *p) {
+template <typename T>
+__global__ __launch_bounds__(NTHREADS) void bwd_dz_kernel(const bimamba2_params p) {
+    bwd_dz_body<T>(p, blockIdx.x, gridDim.x);
+}
+
+// dz and C.B^T (where the forward pass did not keep it) in one launch: the tiles first, they are chains, the rest streams.
+// 4 x 2048, bfloat16, 16 heads of 16, dstate 16: 6 + 7 -> 9 us.
+template <typename T>
+__global__ __launch_bounds__(NTHREADS) void bwd_dz_bmm_kernel(const bimamba2_params p, int nc, int nqt, int nbmm) {
+    __shared__ __attribute__((aligned(16))) char lds[BMM_FWD_LDS<T>];
+    const int id = blockIdx.x;
+    if (id < nbmm) bmm_chunk_fwd_body<T>(p, nc, id % nqt, id / nqt % nqt, id / (nqt * nqt), lds);
+    else bwd_dz_body<T>(p, id - nbmm, gridDim.x - nbmm);
+}
+
+static int dz_blocks(const bimamba2_params *p) {
     const int64_t n = (int64_t)p->batch * p->seqlen * p->nheads * ((p->headdim + 3) / 4);
-    const int blocks = (int)std::min<int64_t>((n + NTHREADS - 1) / NTHREADS, 8192);
+    return (int)std::min<int64_t>((n + NTHREADS - 1) / NTHREADS, 8192);
+}
+
+int launch_bwd_dz_bmm(const bimamba2_params *p) {
+    const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, nbmm = nqt * nqt * p->batch * nc * p->ngroups;
+    const dim3 grid(nbmm + dz_blocks(p));
+    switch (p->dtype) {
+        case BIMAMBA2_F32: hipLaunchKernelGGL(bwd_dz_bmm_kernel<float>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, nbmm); break;
+        case BIMAMBA2_BF16: hipLaunchKernelGGL(bwd_dz_bmm_kernel<bf16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, nbmm); break;
+        case BIMAMBA2_F16: hipLaunchKernelGGL(bwd_dz_bmm_kernel<f16_t>, grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, nbmm); break;
+        default: return BIMAMBA2_EUNSUPPORTED;
+    }
+    return check_launch();
+}
+
+int launch_bwd_dz(const bimamba2_params *p) {
+    const int blocks = dz_blocks(p);
     switch (p->dtype) {
         case BIMAMBA2_F32: hipLaunchKernelGGL(bwd_dz_kernel<float>, dim3(blocks), dim3(NTHREADS), 0, stream_of(p), *p); break;
         case BIMAMBA2_BF16: hipLaunchKernelGGL(bwd_dz_kernel<bf16_t>, dim3(blocks), dim3(NTHREADS), 0, stream_of(p), *p); break;
@@ -937,7 +969,7 @@ bool dcb_recomputes_cb(const bimamba2_params *p) {
 }
 
 template <typename T>
-static int launch_dcb_t(const bimamba2_params *p) {
+static int launch_dcb_t(const bimamba2_params *p, bool add_up) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64;
     const int slices = dcb_slices(p);
     dim3 grid(p->batch * nc * p->ngroups, nqt * nqt, slices);
@@ -952,7 +984,7 @@ static int launch_dcb_t(const bimamba2_params *p) {
     if (ring) launch_dcb_ring<T>(grid, p, nc, nqt);
     else if (fast) hipLaunchKernelGGL((bwd_dcb_kernel<T, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
     else hipLaunchKernelGGL((bwd_dcb_kernel<T, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
-    if (slices > 1) {
+    if (slices > 1 && add_up) {
         // (Q*Q is a multiple of 4 only when Q is even; odd chunk sizes are rejected by the 16-byte requirement below)
         const size_t n = (size_t)p->batch * nc * p->ngroups * p->chunk_size * p->chunk_size;
         if (n % 4) return BIMAMBA2_EUNSUPPORTED;
@@ -1019,11 +1051,11 @@ int launch_bwd_dcb_sp(const bimamba2_params *p, bool out16) {
     return check_launch();
 }
 
-int launch_bwd_dcb(const bimamba2_params *p) {
+int launch_bwd_dcb(const bimamba2_params *p, bool add_up) {
     switch (p->dtype) {
-        case BIMAMBA2_F32: return launch_dcb_t<float>(p);
-        case BIMAMBA2_BF16: return launch_dcb_t<bf16_t>(p);
-        case BIMAMBA2_F16: return launch_dcb_t<f16_t>(p);
+        case BIMAMBA2_F32: return launch_dcb_t<float>(p, add_up);
+        case BIMAMBA2_BF16: return launch_dcb_t<bf16_t>(p, add_up);
+        case BIMAMBA2_F16: return launch_dcb_t<f16_t>(p, add_up);
         default: return BIMAMBA2_EUNSUPPORTED;
     }
 }
@@ -1058,7 +1090,8 @@ template <typename T> __device__ __forceinline__ void split_operand(const float 
 // the general variant fits two (with few heads per group the launch has thousands of workgroups: 83 -> 76 us at 8 groups
 // of 4 heads, batch 4 x 4096, where the launch moves 250 MB).
 template <typename T, int QP, bool FAST, bool SLIM = false>
-__device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int nc, int nslices, BlockId bid, bool in16 = false) {
+__device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int nc, int nslices, BlockId bid, bool in16 = false, int ncb = 1) {
+    // ncb: head slices of dCB / dCBT (float32) that are still to be added up
     typedef Mma<T> M;
     constexpr int KPL = M::KPL, KSTEP = M::KSTEP;
     constexpr int LDX = QP + 16 / (int)sizeof(T);
@@ -1080,6 +1113,7 @@ __device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int
     if (which == 0) { os = p.C_sl; op = reinterpret_cast<const T *>(p.Cm) + b * p.C_sb + (int64_t)c * Q * os + g * p.C_sg + nt * 64; }
     else { os = p.B_sl; op = reinterpret_cast<const T *>(p.Bm) + b * p.B_sb + (int64_t)c * Q * os + g * p.B_sg + nt * 64; }
     const float *arow = (which == 0 ? p.dCBT : p.dCB) + (int64_t)bcg * Q * Q + (int64_t)min(r0 + wave * 16 + lr, Q - 1) * Q;
+    const int64_t cb_slice = (int64_t)p.batch * nc * p.ngroups * Q * Q;
     const float *res = which == 0 ? p.dBs : p.dCs;
     T *out = reinterpret_cast<T *>(which == 0 ? p.dB : p.dC);
     // (dB / dC may be slices of a wider buffer: their own position and batch strides; 0 = contiguous)
@@ -1101,6 +1135,16 @@ __device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int
             for (int s = 0; s < NS; ++s) {
                 raw[s][0] = *reinterpret_cast<const float4 *>(arow + s * KSTEP + lg * KPL);
                 raw[s][1] = *reinterpret_cast<const float4 *>(arow + s * KSTEP + lg * KPL + 4);
+            }
+            for (int sl = 1; sl < ncb; ++sl) {
+                const float *more = arow + sl * cb_slice;
+#pragma unroll
+                for (int s = 0; s < NS; ++s)
+#pragma unroll
+                    for (int half = 0; half < 2; ++half) {
+                        const float4 u = *reinterpret_cast<const float4 *>(more + s * KSTEP + lg * KPL + 4 * half);
+                        raw[s][half].x += u.x; raw[s][half].y += u.y; raw[s][half].z += u.z; raw[s][half].w += u.w;
+                    }
             }
         }
         // slices: the first half is requested here, the second half after the products, into the registers of the row pieces
@@ -1198,7 +1242,11 @@ __device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int
             if (KPL >= 4) {
 #pragma unroll
                 for (int i = 0; i < KPL; i += 4) {
-                    const float4 t4 = *reinterpret_cast<const float4 *>(arow + kb + i);
+                    float4 t4 = *reinterpret_cast<const float4 *>(arow + kb + i);
+                    for (int sl = 1; sl < ncb; ++sl) {
+                        const float4 u = *reinterpret_cast<const float4 *>(arow + sl * cb_slice + kb + i);
+                        t4.x += u.x; t4.y += u.y; t4.z += u.z; t4.w += u.w;
+                    }
                     v[i] = t4.x; v[(i + 1) % KPL] = t4.y; v[(i + 2) % KPL] = t4.z; v[(i + 3) % KPL] = t4.w;
                 }
             } else {
@@ -1206,7 +1254,11 @@ __device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int
             }
         } else {
 #pragma unroll
-            for (int i = 0; i < KPL; ++i) v[i] = kb + i < Q ? arow[kb + i] : 0.f;
+            for (int i = 0; i < KPL; ++i) {
+                v[i] = kb + i < Q ? arow[kb + i] : 0.f;
+                for (int sl = 1; sl < ncb; ++sl)
+                    if (kb + i < Q) v[i] += arow[sl * cb_slice + kb + i];
+            }
         }
         typename M::Frag af, rest{};
         split_operand<T>(v, af, rest);
@@ -1473,6 +1525,20 @@ __global__ __launch_bounds__(NTHREADS) void bwd_tail_kernel(const bimamba2_param
     }
 }
 
+// The same for chunks of up to 128 positions and any type and shape, with the head slices of dCB added up by their reader (instead of
+// a launch of their own): what ends a pass whose kernels for wide 16-bit heads and states do not apply.  4 x 2048, bfloat16, 16 heads
+// of 16, dstate 16: 10 + 8 + 5 -> 14 us; float32, 16 heads of 64, dstate 64: 14 + 9 + 6 -> 18.
+template <typename T, int QP, bool FAST, typename DT>
+__global__ __launch_bounds__(NTHREADS) void bwd_tail_small_kernel(const bimamba2_params p, int nc, int nslices, int nqt, int nsplit, int nbmm,
+                                                                  int nnt, int cs_gx, int ncb) {
+    const int id = blockIdx.x;
+    if (id < nbmm) bmm_chunk_bwd_body<T, QP, FAST>(p, nc, nslices, BlockId{id % nnt, id / nnt % nqt, id / (nnt * nqt)}, false, ncb);
+    else {
+        const int k = id - nbmm;                  // cumsum grid (cs_gx, nc, batch)
+        chunk_cumsum_bwd_body<DT>(p, nc, nqt, nsplit, BlockId{k % cs_gx, (k / cs_gx) % nc, k / (cs_gx * nc)});
+    }
+}
+
 static bool bmm_bwd_fast(const bimamba2_params *p) {
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     auto mult = [](int64_t a, int64_t b, int64_t c) { return a % 8 == 0 && b % 8 == 0 && c % 8 == 0; };
@@ -1507,6 +1573,42 @@ static int launch_bwd_tail_t(const bimamba2_params *p, int nc, int nqt, int nspl
         default: return BIMAMBA2_EUNSUPPORTED;
     }
     return check_launch();
+}
+
+// dt in float32 or in the type of x (two instantiations of each)
+bool bwd_tail_small(const bimamba2_params *p) {
+    return !p->causal && p->chunk_size <= 128 && (p->dt_dtype == BIMAMBA2_F32 || p->dt_dtype == p->dtype);
+}
+
+template <typename T, int QP, bool FAST>
+static void launch_bwd_tail_small_t(const bimamba2_params *p, int nc, int nsplit, int ncb) {
+    const int nqt = (p->chunk_size + 63) / 64, nnt = (p->dstate + 63) / 64, nbmm = nnt * nqt * p->batch * nc * p->ngroups * 2;
+    const int cs_gx = (p->nheads + 3) / 4;
+    const dim3 grid(nbmm + cs_gx * nc * p->batch);
+    if (p->dt_dtype == BIMAMBA2_F32) hipLaunchKernelGGL((bwd_tail_small_kernel<T, QP, FAST, float>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, dbdc_slices(p), nqt, nsplit, nbmm, nnt, cs_gx, ncb);
+    else hipLaunchKernelGGL((bwd_tail_small_kernel<T, QP, FAST, T>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, dbdc_slices(p), nqt, nsplit, nbmm, nnt, cs_gx, ncb);
+}
+
+// ncb: head slices of dCB that nobody has added up yet
+int launch_bwd_tail_small(const bimamba2_params *p, ReduceJobs *defer, int ncb) {
+    const int nc = nchunks(p), nsplit = (p->headdim * p->dstate + SP_EPT * NTHREADS - 1) / (SP_EPT * NTHREADS);
+    const bool fast = bmm_bwd_fast(p), half = p->chunk_size <= 64;
+    switch (p->dtype) {
+        case BIMAMBA2_F32: if (half) launch_bwd_tail_small_t<float, 64, false>(p, nc, nsplit, ncb); else launch_bwd_tail_small_t<float, 128, false>(p, nc, nsplit, ncb); break;
+#define BM2_TAIL(TT)                                                                                                                   \
+    if (fast && half) launch_bwd_tail_small_t<TT, 64, true>(p, nc, nsplit, ncb); else if (fast) launch_bwd_tail_small_t<TT, 128, true>(p, nc, nsplit, ncb); \
+    else if (half) launch_bwd_tail_small_t<TT, 64, false>(p, nc, nsplit, ncb); else launch_bwd_tail_small_t<TT, 128, false>(p, nc, nsplit, ncb)
+        case BIMAMBA2_BF16: BM2_TAIL(bf16_t); break;
+        case BIMAMBA2_F16: BM2_TAIL(f16_t); break;
+#undef BM2_TAIL
+        default: return BIMAMBA2_EUNSUPPORTED;
+    }
+    const int rc = check_launch();
+    if (rc) return rc;
+    const int ni = p->batch * nc;
+    defer->job[defer->n++] = ReduceJob{p->red, p->dA, ni, p->nheads, 1};
+    if (p->has_dt_bias && p->ddt_bias) defer->job[defer->n++] = ReduceJob{p->red + (int64_t)ni * p->nheads, p->ddt_bias, ni, p->nheads, 1};
+    return BIMAMBA2_OK;
 }
 
 // bmm_chunk_bwd + chunk_cumsum_bwd in one launch (the caller checked bwd_tail_merged()); reductions as in

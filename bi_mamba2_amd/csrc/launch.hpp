@@ -48,12 +48,13 @@ bool scan_recomputes_cb(const bimamba2_params *p, bool bwd);
 bool dcb_recomputes_cb(const bimamba2_params *p);
 
 int launch_bwd_dz(const bimamba2_params *p);
+int launch_bwd_dz_bmm(const bimamba2_params *p);       // dz and C.B^T in one launch
 bool bwd_dz_dstates_fused(const bimamba2_params *p);   // dz and dstates as one launch
 int launch_bwd_dz_dstates(const bimamba2_params *p);
 int launch_state_passing_bwd(const bimamba2_params *p);
 int choose_dbdc_heads(const bimamba2_params *p);   // heads per slice of the dB / dC partial sums
 int launch_bwd_dbdc(const bimamba2_params *p, bool is_db);
-int launch_bwd_dcb(const bimamba2_params *p);
+int launch_bwd_dcb(const bimamba2_params *p, bool add_up = true);   // add_up: also the launch that adds several head slices up
 int choose_dcb_slices(const bimamba2_params *p);
 int dcb_slices(const bimamba2_params *p);   // head slices whose dCB partial sums the kernel keeps apart
 int launch_bmm_chunk_bwd(const bimamba2_params *p);
@@ -71,6 +72,9 @@ bool bwd_dcb_sp_merged(const bimamba2_params *p);
 int launch_bwd_dcb_sp(const bimamba2_params *p, bool out16 = false);
 bool bwd_tail_merged(const bimamba2_params *p);
 int launch_bwd_tail(const bimamba2_params *p, ReduceJobs *defer, bool in16 = false);
+// the same for chunks of up to 128 positions, any type and shape (ncb: head slices of dCB still to be added up)
+bool bwd_tail_small(const bimamba2_params *p);
+int launch_bwd_tail_small(const bimamba2_params *p, ReduceJobs *defer, int ncb);
 int launch_fill(float *ptr, size_t n, float value, hipStream_t stream);
 // out[j] = sum_{i<ni} sum_{k<nk} in[(i*nj + j)*nk + k]
 int launch_reduce(const float *in, float *out, int ni, int nj, int nk, hipStream_t stream);

@@ -143,3 +143,37 @@ def test_backward_takes_a_misaligned_gradient_view(ops):
         res.append({k: v.grad for k, v in leaves.items()})
     for k in res[0]:
         assert torch.equal(res[0][k], res[1][k]), k
+
+
+@pytest.mark.parametrize("b,L,H,P,G,N,Q,dtype,dt_dtype,z", [
+    (1, 130, 4, 16, 2, 16, 64, torch.float32, torch.float32, True),        # two row tiles, nothing to add up
+    (2, 75, 8, 16, 1, 24, 50, torch.float32, torch.float32, False),        # head slices of dCB, chunk no whole tile
+    (1, 257, 12, 24, 1, 72, 128, torch.bfloat16, torch.bfloat16, True),    # slices, two tiles of the state
+    (1, 100, 16, 32, 1, 64, 64, torch.float16, torch.float32, False),      # slices with unconditional loads
+    (1, 100, 6, 16, 1, 16, 64, torch.bfloat16, torch.float16, True),       # dt of a third type: the two launches
+])
+def test_last_launch_adds_up_head_slices(ops, b, L, H, P, G, N, Q, dtype, dt_dtype, z):
+    """bimamba2_bwd against a caller that brings its own dCB and dCBT, which are added up by a launch of their own, in four slices"""
+    d = to_dev(make_case(b, L, H, P, G, N, dtype, with_z=z))
+    dt = d["dt"].to(dt_dtype)
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(7)).to(dtype).cuda()
+    args, kw = (d["x"], dt, d["A"], d["B"], d["C"]), dict(D=d["D"], z=d["z"], dt_bias=d["dt_bias"], dt_softplus=True)
+    res = ops._mamba_chunk_scan_combined_fwd(*args, Q, return_intermediates=False, keep_for_bwd=True, **kw)
+    bwd = lambda: ops._mamba_chunk_scan_combined_bwd(dout, *args, res[1] if z else res[0], Q, saved=res[9], **kw)
+    own, ws = bwd(), ops._Call.workspace
+
+    def with_dcb(call, is_bwd):
+        call.p.dcb_slices = min(4, H // G)
+        for field in ("dCB", "dCBT"):
+            call.new(field, (call.p.dcb_slices, b, -(-L // Q), G, Q, Q))
+        return ws(call, is_bwd)
+
+    ops._Call.workspace = with_dcb
+    try:
+        brought = bwd()
+    finally:
+        ops._Call.workspace = ws
+    tol = {torch.float32: 1e-5, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]      # (four slices: another order of the same sum, rounded once)
+    for a, c in zip(own, brought):
+        if a is not None:
+            assert float((a.double() - c.double()).norm()) <= tol * float(c.double().norm())
