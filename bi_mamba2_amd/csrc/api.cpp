@@ -470,9 +470,10 @@ int bimamba2_bwd(const bimamba2_params *p) {
     const int ncb = tail_small && !p->dCB && !p->dCBT && !bwd_dcb_sp_merged(&q) ? dcb_slices(&q) : 1;
     // the dCB kernel is bound by instruction issue and moves little data: right behind dz it runs while the memory system
     // still writes back dz's output, which the memory-bound kernels after it would otherwise wait behind
+    const bool dx_db_dc = dx_db_dc_merged(&q);      // (one launch at the end)
     if (bwd_dcb_sp_merged(&q)) {
         // the backward state passing (streams, few instructions) rides along with the dCB kernel in one launch
-        TRY(bimamba2_chunk_scan_bwd_dc(&q));
+        if (!dx_db_dc) TRY(bimamba2_chunk_scan_bwd_dc(&q));
         if (!dz_dstates) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
         REQUIRE(q.x); REQUIRE(q.dt_out); REQUIRE(q.cs_f); REQUIRE(q.cs_b); REQUIRE(q.dCB); REQUIRE(q.dCBT); REQUIRE(q.da_intra);
         if (!q.dstates16_f) REQUIRE(q.dstates_f);
@@ -481,12 +482,20 @@ int bimamba2_bwd(const bimamba2_params *p) {
         TRY(launch_bwd_dcb_sp(&q, dcb16));
     } else {
         TRY(check_bwd_dcb(&q));
-        TRY(launch_bwd_dcb(&q, ncb == 1));
-        if (!dz_dstates) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
-        TRY(bimamba2_chunk_scan_bwd_dc(&q));           // (between the two memory-bound state kernels: measured best)
+        if (!dz_dstates && ncb == dcb_slices(&q) && dcb_dstates_merged(&q)) {
+            REQUIRE(q.Cm);
+            TRY(launch_dcb_dstates(&q));
+        } else {
+            TRY(launch_bwd_dcb(&q, ncb == 1));
+            if (!dz_dstates) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
+        }
+        if (!dx_db_dc) TRY(bimamba2_chunk_scan_bwd_dc(&q));           // (between the two memory-bound state kernels: measured best)
         TRY(bimamba2_state_passing_bwd(&q));
     }
-    TRY(bimamba2_chunk_state_bwd_db(&q));
+    if (dx_db_dc) {
+        REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dBs); REQUIRE(q.dCs); REQUIRE(q.u_f); REQUIRE(q.u_b); REQUIRE(q.v_f); REQUIRE(q.v_b);
+        REQUIRE(q.states_f); REQUIRE(q.states_b); REQUIRE(q.dstates_f); REQUIRE(q.dstates_b);
+    } else TRY(bimamba2_chunk_state_bwd_db(&q));
     ReduceJobs jobs;
     {
         // as bimamba2_chunk_scan_bwd_dx, with the reduction of the dD partial sums left for the end
@@ -495,7 +504,7 @@ int bimamba2_bwd(const bimamba2_params *p) {
         REQUIRE(qx.dx); REQUIRE(qx.ddt_direct);
         if (qx.has_D) { REQUIRE(qx.D); REQUIRE(qx.dD); }
         const int nc = nchunks(&q);
-        TRY(launch_chunk_scan(&qx, true));
+        TRY(dx_db_dc ? launch_dx_db_dc(&qx) : launch_chunk_scan(&qx, true));
         if (q.has_D) {
             if (q.D_has_hdim) jobs.job[jobs.n++] = ReduceJob{q.red, q.dD, q.batch * nc, q.nheads * q.headdim, 1};
             else jobs.job[jobs.n++] = ReduceJob{q.red, q.dD, q.batch * nc, q.nheads, q.headdim};

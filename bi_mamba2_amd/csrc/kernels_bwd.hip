@@ -968,18 +968,24 @@ bool dcb_recomputes_cb(const bimamba2_params *p) {
     return al(p->Bm) && mult(p->B_sb, p->B_sl, p->B_sg) && al(p->Cm) && mult(p->C_sb, p->C_sl, p->C_sg);
 }
 
+static bool dcb_aligned(const bimamba2_params *p) {
+    const int vs = p->dtype == BIMAMBA2_F32 ? 4 : 8;
+    auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    const bool x = al(p->x) && p->x_sb % vs == 0 && p->x_sl % vs == 0 && p->x_sh % vs == 0;
+    return x && (p->has_z ? al(p->dout_x) : (al(p->dout) && p->dout_sb % vs == 0 && p->dout_sl % vs == 0 && p->dout_sh % vs == 0));
+}
+static bool dcb_ring_applies(const bimamba2_params *p) {
+    return p->dtype != BIMAMBA2_F32 && dcb_aligned(p) && p->chunk_size % 64 == 0 && p->headdim % 8 == 0 && dcb_rows_in_32bit(p);
+}
+
 template <typename T>
 static int launch_dcb_t(const bimamba2_params *p, bool add_up) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64;
     const int slices = dcb_slices(p);
     dim3 grid(p->batch * nc * p->ngroups, nqt * nqt, slices);
-    constexpr int VS = 16 / (int)sizeof(T);
-    auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
-    bool aligned = al(p->x) && p->x_sb % VS == 0 && p->x_sl % VS == 0 && p->x_sh % VS == 0;
-    aligned = aligned && (p->has_z ? al(p->dout_x) : (al(p->dout) && p->dout_sb % VS == 0 && p->dout_sl % VS == 0 && p->dout_sh % VS == 0));
-    const bool fast = aligned && p->headdim % (sizeof(T) == 2 ? 64 : 16) == 0;
+    const bool fast = dcb_aligned(p) && p->headdim % (sizeof(T) == 2 ? 64 : 16) == 0;
     if (!p->CB && !dcb_recomputes_cb(p)) return BIMAMBA2_EINVAL;
-    const bool ring = aligned && sizeof(T) == 2 && p->chunk_size % 64 == 0 && p->headdim % 8 == 0 && dcb_rows_in_32bit(p);
+    const bool ring = dcb_ring_applies(p);
     if (p->causal && !(ring && fast)) return BIMAMBA2_EUNSUPPORTED;
     if (ring) launch_dcb_ring<T>(grid, p, nc, nqt);
     else if (fast) hipLaunchKernelGGL((bwd_dcb_kernel<T, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
@@ -1649,6 +1655,60 @@ int launch_chunk_cumsum_bwd(const bimamba2_params *p, ReduceJobs *defer) {
     if (rc) return rc;
     if (p->has_dt_bias && p->ddt_bias) rc = launch_reduce(p->red + (int64_t)ni * p->nheads, p->ddt_bias, ni, p->nheads, 1, stream_of(p));
     return rc;
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// launches of several roles (roles.hpp)
+// ---------------------------------------------------------------------------------------------------------
+static bool dbdc_wide16(const bimamba2_params *p) {      // the dB / dC kernels with the ring of state tiles
+    return p->dtype != BIMAMBA2_F32 && p->headdim % 64 == 0 && (p->dstate == 64 || p->dstate == 128);
+}
+static RolesShape roles_shape(const bimamba2_params *p) {
+    const int vs = p->dtype == BIMAMBA2_F32 ? 4 : 8;
+    RolesShape r;
+    r.nchunks = nchunks(p);
+    r.dcb_slices = dcb_slices(p);
+    r.dbdc_slices = dbdc_slices(p);
+    r.dbdc_heads = dbdc_heads(p);
+    r.dcb_ring = dcb_ring_applies(p);
+    r.dcb_fast = dcb_aligned(p) && p->headdim % 16 == 0;
+    auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    r.dstates_fast = dcb_aligned(p) && p->headdim % 64 == 0 && p->dstate % 64 == 0 && al(p->Cm) && p->C_sb % vs == 0 && p->C_sl % vs == 0 && p->C_sg % vs == 0;
+    r.dbdc_fast = dcb_aligned(p) && p->headdim % 64 == 0 && p->dstate % 64 == 0;
+    return r;
+}
+
+// (faster at every size measured, 1 x 300 to 8 x 2048 with 8 to 32 heads of 16 to 128 and dstate 16 to 128: 4 x 2048, 16 heads of 16, dstate 16,
+// bfloat16 158 -> 150 us a pass, float32 174 -> 171; 8 x 2048, 32 heads of 64, dstate 64, float32 1544 -> 1513)
+bool dcb_dstates_merged(const bimamba2_params *p) {
+    if (p->causal || p->chunk_size > 128 || !p->CB || !p->dstates_f || !p->dstates_b || p->dstates16_f) return false;
+    // 16 bits: the ring variant of dCB, and the generic kernel of the states' gradients
+    return p->dtype == BIMAMBA2_F32 || (dcb_ring_applies(p) && !(p->headdim % 64 == 0 && p->dstate % 64 == 0));
+}
+int launch_dcb_dstates(const bimamba2_params *p) {
+    const RolesShape r = roles_shape(p);
+    return p->dtype == BIMAMBA2_F32 ? launch_dcb_dstates_f32(p, r) : p->dtype == BIMAMBA2_BF16 ? launch_dcb_dstates_bf16(p, r) : launch_dcb_dstates_f16(p, r);
+}
+
+// One launch holds the registers of the dB / dC role (128 for states of up to 32 columns, 165 for 64, 245 for 128) for the dx role too,
+// which then has one workgroup a CU above 128: it pays while most of the dx workgroups are on the chip at once anyway.
+// us a pass over 16 heads, three launches -> one: 16 bits, heads of 16, dstate 16: 4 x 1024 (512 dx workgroups) 122 -> 101, 4 x 2048 (1024) 153 ->
+// 149, 32 heads 8 x 2048 (4096) 398 -> 395, but heads of 64, dstate 32 573 -> 580; heads of 128, dstate 32: 4 x 2048 (2048) 306 -> 302.  dstate 64,
+// heads of 32: 4 x 1024 (512) 123 -> 121, but 4 x 2048 186 -> 192.  dstate 128: 163 -> 170 (512).  float32, heads of 64, dstate 32: 4 x 1024 (1024)
+// 204 -> 198, 4 x 2048 (2048) 323 -> 324; dstate 64: 4 x 1024 (1024) 238 -> 246.
+static bool dx_db_dc_pays(const bimamba2_params *p) {
+    const int pw = scan_col_tile_of(p->headdim, p->dtype);
+    const int64_t dx = (int64_t)p->batch * nchunks(p) * p->nheads * ((p->headdim + pw - 1) / pw);
+    return dx <= (p->dstate <= 32 ? 2048 : p->dstate <= 64 ? 512 : 256);
+}
+
+bool dx_db_dc_merged(const bimamba2_params *p) {
+    if (p->causal || p->chunk_size > 128 || !p->CBT || p->states16_f || p->dstates16_f || dbdc_wide16(p) || p->dstate > 128 || dbdc_heads(p) > DBDC_HEADS) return false;
+    return dx_db_dc_pays(p) && scan_is_fast(p, true);
+}
+int launch_dx_db_dc(const bimamba2_params *p) {
+    const RolesShape r = roles_shape(p);
+    return p->dtype == BIMAMBA2_F32 ? launch_dx_db_dc_f32(p, r) : p->dtype == BIMAMBA2_BF16 ? launch_dx_db_dc_bf16(p, r) : launch_dx_db_dc_f16(p, r);
 }
 
 }  // namespace bm2

@@ -42,6 +42,8 @@ static bool scan_fast(const bimamba2_params *p, bool bwd, int pw, int vs) {
     return fast;
 }
 
+bool scan_is_fast(const bimamba2_params *p, bool bwd) { return scan_fast(p, bwd, scan_col_tile(p), p->dtype == BIMAMBA2_F32 ? 4 : 8); }
+
 // the conditions of the kernels that rebuild C.B^T, apart from the state dimension
 static bool scan_rebuild_shape(const bimamba2_params *p, bool bwd) {
     if (p->dtype == BIMAMBA2_F32 || scan_col_tile(p) != 64) return false;

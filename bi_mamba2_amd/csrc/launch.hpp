@@ -75,6 +75,22 @@ int launch_bwd_tail(const bimamba2_params *p, ReduceJobs *defer, bool in16 = fal
 // the same for chunks of up to 128 positions, any type and shape (ncb: head slices of dCB still to be added up)
 bool bwd_tail_small(const bimamba2_params *p);
 int launch_bwd_tail_small(const bimamba2_params *p, ReduceJobs *defer, int ncb);
+// launches of several roles (roles.hpp), with what their kernels' own launches know about the problem
+struct RolesShape {
+    int nchunks, dcb_slices, dbdc_slices, dbdc_heads;
+    bool dcb_ring, dcb_fast, dstates_fast, dbdc_fast;
+};
+bool dcb_dstates_merged(const bimamba2_params *p);      // dCB and dstates in one launch
+int launch_dcb_dstates(const bimamba2_params *p);
+bool dx_db_dc_merged(const bimamba2_params *p);         // dx, dB and dC in one launch
+int launch_dx_db_dc(const bimamba2_params *p);
+int launch_dcb_dstates_f32(const bimamba2_params *p, const RolesShape &r);
+int launch_dcb_dstates_bf16(const bimamba2_params *p, const RolesShape &r);
+int launch_dcb_dstates_f16(const bimamba2_params *p, const RolesShape &r);
+int launch_dx_db_dc_f32(const bimamba2_params *p, const RolesShape &r);
+int launch_dx_db_dc_bf16(const bimamba2_params *p, const RolesShape &r);
+int launch_dx_db_dc_f16(const bimamba2_params *p, const RolesShape &r);
+bool scan_is_fast(const bimamba2_params *p, bool bwd);  // the scan kernel without guarded fallbacks applies
 int launch_fill(float *ptr, size_t n, float value, hipStream_t stream);
 // out[j] = sum_{i<ni} sum_{k<nk} in[(i*nj + j)*nk + k]
 int launch_reduce(const float *in, float *out, int ni, int nj, int nk, hipStream_t stream);

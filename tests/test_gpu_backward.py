@@ -177,3 +177,37 @@ def test_last_launch_adds_up_head_slices(ops, b, L, H, P, G, N, Q, dtype, dt_dty
     for a, c in zip(own, brought):
         if a is not None:
             assert float((a.double() - c.double()).norm()) <= tol * float(c.double().norm())
+
+
+@pytest.mark.parametrize("b,L,H,P,G,N,Q,dtype,z", [
+    (1, 130, 4, 16, 2, 16, 64, torch.float32, True),          # one column tile of the state, two chunks and a rest
+    (1, 128, 3, 64, 1, 32, 128, torch.float32, False),        # two; two headdim tiles a dx workgroup owns one of
+    (1, 100, 2, 128, 1, 64, 64, torch.float32, True),         # four, unconditional loads
+    (1, 70, 2, 64, 1, 128, 64, torch.float32, False),         # two tiles of 64
+    (1, 200, 4, 32, 2, 128, 128, torch.bfloat16, True),
+    (1, 65, 5, 128, 5, 16, 64, torch.float16, False),
+    (2, 96, 6, 16, 1, 40, 96, torch.bfloat16, True),          # chunk no whole tile: dCB and the states' gradients on their own
+])
+def test_launches_of_several_roles(ops, b, L, H, P, G, N, Q, dtype, z):
+    """bimamba2_bwd with dCB and the states' gradients in one launch and dx, dB and dC in another against the stages one by one: the
+    same work in other workgroups, so the same bits where a stage's result is the call's"""
+    d = to_dev(make_case(b, L, H, P, G, N, dtype, with_z=z))
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(7)).to(dtype).cuda()
+    args, kw = (d["x"], d["dt"], d["A"], d["B"], d["C"]), dict(D=d["D"], z=d["z"], dt_bias=d["dt_bias"], dt_softplus=True)
+    res = ops._mamba_chunk_scan_combined_fwd(*args, Q, keep_for_bwd=True, **kw)
+    dt_out, csf, csb, sf, sb = res[2:7]
+    got = ops._mamba_chunk_scan_combined_bwd(dout, *args, res[1] if z else res[0], Q, saved=res[9], **kw)
+    dox = ops._chunk_scan_bwd_dz(res[1], d["z"], res[1], dout, Q)[1] if z else dout
+    dpf, dpb = ops._chunk_scan_bwd_dstates(d["C"], csf, csb, dox)
+    dsf, dsb = ops._state_passing_bwd(sf, sb, csf, csb, dpf, dpb)[:2]
+    CB = ops._bmm_chunk_fwd(d["C"], d["B"], Q)
+    dx, _, dD = ops._chunk_scan_chunk_state_bwd_dx(d["x"], dt_out, csf, csb, d["B"], CB, dox, dsf, dsb, D=d["D"])
+    assert torch.equal(got[0], dx) and torch.equal(got[5], dD)
+    # dB and dC: the slices of heads differ between the two (their sum is rounded in another order)
+    dBs = ops._chunk_state_bwd_db(d["x"], dt_out, csf, csb, dsf, dsb, B=d["B"], ngroups=G)[0]
+    dCs = ops._chunk_scan_bwd_dC(sf, sb, csf, csb, dox, C=d["C"], ngroups=G)[0]
+    dCB = ops._chunk_scan_bwd_dcb(d["x"], dt_out, csf, csb, dox, CB, ngroups=G)[0]
+    dB, dC = ops._bmm_chunk_bwd(d["B"], d["C"], dCB, dBs, dCs)
+    tol = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]      # (now and then one unit of the result's type)
+    for g, w in ((got[3], dB), (got[4], dC)):
+        assert float((g.double() - w.double()).norm()) <= tol * float(w.double().norm())
