@@ -8,6 +8,8 @@
 //   chunk_cumsum_bwd   assembles d(dt*A) from its pieces with wavefront scans; ddt, dA, ddt_bias
 #include <type_traits>
 
+#include <type_traits>
+
 #include "common.hpp"
 #include "launch.hpp"
 #include "bmm_fwd_body.hpp"
@@ -274,10 +276,15 @@ __global__ __launch_bounds__(NTHREADS) void state_passing_bwd_kernel(const bimam
 // DP16 (with DS16): the per-chunk gradients lie in dstates16_* in the 16-bit type as well (no float32 tensors): every one is
 // read once and replaced in place by the gradient with respect to the state entering its chunk.
 constexpr int SP_CH = 8;
-template <typename T16, bool PREV16, bool DS16, bool DP16 = false>
+// AHEAD: the next SP_CH chunks are on their way while the present ones are worked on, and the inner products are handed out every
+// SP_FLUSH chunks instead of every SP_CH (a barrier waits for the loads in flight): the launch of its own, whose workgroups have nothing
+// else to cover a round trip with.  As a role beside dCB the kernel keeps to that one's registers and LDS.
+constexpr int SP_FLUSH = 64;
+template <typename T16, bool PREV16, bool DS16, bool DP16 = false, bool AHEAD = false>
 __device__ __forceinline__ void state_passing_bwd_vec_body(const bimamba2_params &p, int nc, int nsplit, int ndir, BlockId bid) {
     struct alignas(8) V4 { T16 v[4]; };
-    __shared__ float red[SP_CH][4];
+    constexpr int FLUSH = AHEAD ? SP_FLUSH : SP_CH;
+    __shared__ float red[FLUSH][4];
     const int PN = p.headdim * p.dstate;
     const int split = bid.x, h = bid.y, b = bid.z / ndir, dir = bid.z % ndir;   // ndir = 1: forward direction only
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -298,66 +305,104 @@ __device__ __forceinline__ void state_passing_bwd_vec_body(const bimamba2_params
     const int64_t bh = ((int64_t)b * p.nheads + h) * PN + e;
     f32x4 g = {0.f, 0.f, 0.f, 0.f};
     if (dfin) g = *reinterpret_cast<const f32x4 *>(dfin + bh);
-    for (int s0 = 0; s0 < nc; s0 += SP_CH) {
-        const int nb = min(SP_CH, nc - s0);
-        f32x4 dp[SP_CH], pv[SP_CH];
-        float dec[SP_CH];
+    struct Batch { f32x4 dp[SP_CH], pv[SP_CH]; float dec[SP_CH]; };
+    auto load = [&](int s0, Batch &r) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < SP_CH; ++j) {
             const int sj = min(s0 + j, nc - 1);            // past the last chunk: a valid chunk again, never used
             const int c = dir == 0 ? nc - 1 - sj : sj;
-            dec[j] = cs[(int64_t)c * Q];
+            r.dec[j] = cs[(int64_t)c * Q];
             // (both are read for the last time in the pass: past the caches)
             if constexpr (DP16) {
                 const V4 t = *reinterpret_cast<const V4 *>(ds16 + c * cstride);
 #pragma unroll
-                for (int k = 0; k < 4; ++k) dp[j][k] = to_f(t.v[k]);
+                for (int k = 0; k < 4; ++k) r.dp[j][k] = to_f(t.v[k]);
             } else {
-                dp[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(ds + c * cstride));
+                r.dp[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(ds + c * cstride));
             }
             if constexpr (PREV16) {
                 typedef float f32x2 __attribute__((ext_vector_type(2)));
                 const V4 t = __builtin_bit_cast(V4, __builtin_nontemporal_load(reinterpret_cast<const f32x2 *>(prev16 + c * cstride)));
 #pragma unroll
-                for (int k = 0; k < 4; ++k) pv[j][k] = to_f(t.v[k]);
+                for (int k = 0; k < 4; ++k) r.pv[j][k] = to_f(t.v[k]);
             } else {
-                pv[j] = *reinterpret_cast<const f32x4 *>(prev + c * cstride);
+                r.pv[j] = *reinterpret_cast<const f32x4 *>(prev + c * cstride);
             }
         }
+    };
+    // (the recurrence and its stores first, then all inner products' sums side by side: one after the other, each a chain of six
+    // exchanges between the lanes, they were half of the kernel's time.  1 x 16384 in chunks of 128, 16 heads of 32, dstate 32: 61 -> 50 us
+    // with the next chunks under way, -> 27 with the sums side by side; beside dCB, 1 x 16384, 8 heads of 64, the pass 186 -> 172)
+    auto recur = [&](int s0, int nb, const Batch &r, float (&dot)[SP_CH], auto WHOLE) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < SP_CH; ++j) {
-            if (j < nb) {
+            if (decltype(WHOLE)::value || j < nb) {
                 const int c = dir == 0 ? nc - 1 - (s0 + j) : s0 + j;
-                const float d = __expf(dec[j]);
-                float dot = 0.f;
-                if (live) {
-                    dot = g[0] * pv[j][0] + g[1] * pv[j][1] + g[2] * pv[j][2] + g[3] * pv[j][3];
-                    if constexpr (DS16) {
-                        V4 t;
+                const float d = __expf(r.dec[j]);
+                dot[j] = (g[0] * r.pv[j][0] + g[1] * r.pv[j][1] + g[2] * r.pv[j][2] + g[3] * r.pv[j][3]) * d;
+                if constexpr (DS16) {
+                    V4 t;
 #pragma unroll
-                        for (int k = 0; k < 4; ++k) t.v[k] = from_f<T16>(g[k]);
-                        *reinterpret_cast<V4 *>(ds16 + c * cstride) = t;
-                    } else {
-                        *reinterpret_cast<f32x4 *>(ds + c * cstride) = g;
-                    }
-                    g = dp[j] + d * g;
+                    for (int k = 0; k < 4; ++k) t.v[k] = from_f<T16>(g[k]);
+                    *reinterpret_cast<V4 *>(ds16 + c * cstride) = t;
+                } else {
+                    *reinterpret_cast<f32x4 *>(ds + c * cstride) = g;
                 }
-                dot = wave_sum(dot) * d;
-                if (lane == 0) red[j][wave] = dot;
+                g = r.dp[j] + d * g;
             }
         }
-        __syncthreads();
-        if ((int)threadIdx.x < nb) {
-            const int c = dir == 0 ? nc - 1 - (s0 + (int)threadIdx.x) : s0 + (int)threadIdx.x;
-            dda[(int64_t)c * nsplit] = red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3];
+    };
+    auto work = [&](int s0, const Batch &r) __attribute__((always_inline)) {
+        const int nb = min(SP_CH, nc - s0);
+        float dot[SP_CH] = {};
+        if (live) {
+            if (nb == SP_CH) recur(s0, nb, r, dot, std::true_type());
+            else recur(s0, nb, r, dot, std::false_type());
         }
-        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < SP_CH; ++j) dot[j] = row16_sum(dot[j]);
+#pragma unroll
+        for (int m = 16; m <= 32; m <<= 1)
+#pragma unroll
+            for (int j = 0; j < SP_CH; ++j) dot[j] += __shfl_xor(dot[j], m, 64);
+        if (lane == 0) {
+#pragma unroll
+            for (int j = 0; j < SP_CH; ++j) red[s0 % FLUSH + j][wave] = dot[j];      // (behind the last chunk: never read)
+        }
+        // chunks up to s0 + nb: hand the inner products out when their place is full, or at the end
+        const int done = s0 + nb;
+        if (done % FLUSH == 0 || done == nc) {
+            __syncthreads();
+            const int from = (done - 1) / FLUSH * FLUSH;
+            if ((int)threadIdx.x < done - from) {
+                const int c = dir == 0 ? nc - 1 - (from + (int)threadIdx.x) : from + (int)threadIdx.x;
+                dda[(int64_t)c * nsplit] = red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3];
+            }
+            __syncthreads();
+        }
+    };
+    if constexpr (AHEAD) {
+        Batch one, two;
+        load(0, one);
+        for (int s0 = 0; s0 < nc; s0 += 2 * SP_CH) {
+            if (s0 + SP_CH < nc) load(s0 + SP_CH, two);
+            work(s0, one);
+            if (s0 + SP_CH >= nc) break;
+            if (s0 + 2 * SP_CH < nc) load(s0 + 2 * SP_CH, one);
+            work(s0 + SP_CH, two);
+        }
+    } else {
+        for (int s0 = 0; s0 < nc; s0 += SP_CH) {
+            Batch one;
+            load(s0, one);
+            work(s0, one);
+        }
     }
     if (dini && live) *reinterpret_cast<f32x4 *>(dini + bh) = g;
 }
 template <typename T16, bool PREV16, bool DS16, bool DP16 = false>
 __global__ __launch_bounds__(NTHREADS) void state_passing_bwd_vec_kernel(const bimamba2_params p, int nc, int nsplit, int ndir) {
-    state_passing_bwd_vec_body<T16, PREV16, DS16, DP16>(p, nc, nsplit, ndir, BlockId{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z});
+    state_passing_bwd_vec_body<T16, PREV16, DS16, DP16, true>(p, nc, nsplit, ndir, BlockId{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z});
 }
 
 int launch_state_passing_bwd(const bimamba2_params *p) {

@@ -259,3 +259,33 @@ def test_state_parts_of_db_and_dc_with_narrow_states(ops, N, H, G, P, L, Q, dtyp
         for g, w, t in ((got[1], wf, tf), (got[2], wb, tb)):
             want = (w * (t * wide(mate)).sum(-1)).permute(0, 3, 1, 2).reshape(b, H, -1)[:, :, :L]
             assert float((g.reshape(b, H, -1)[:, :, :L] - want).norm() / want.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("nc", [1, 7, 8, 9, 16, 17, 63, 64, 65, 129])
+@pytest.mark.parametrize("PN", [(8, 4), (40, 30)])
+def test_state_passing_over_many_chunks(ops, nc, PN):
+    """both recurrences and their gradients at the edges of what is loaded ahead (8 chunks) and handed out together (64), with one
+    partly filled workgroup and with two"""
+    b, H, Q, (P, N) = 2, 3, 32, PN
+    gen = torch.Generator().manual_seed(nc)
+    r = lambda *s: torch.randn(*s, generator=gen).cuda()
+    cs = [-0.1 * torch.rand(b, H, nc, Q, generator=gen).cuda().cumsum(-1) for _ in range(2)]
+    csf, csb = cs[0], cs[1].flip(-1).contiguous()                  # the reverse sums' total stands at the first position
+    st, dprev = [r(b, nc, H, P, N) for _ in range(2)], [r(b, nc, H, P, N) for _ in range(2)]
+    ef, eb = csf[..., -1].double().exp(), csb[..., 0].double().exp()
+    got = ops._state_passing_fwd(*st, csf, csb)
+    back = ops._state_passing_bwd(got[0], got[1], csf, csb, *dprev)
+    for k, (e, order) in enumerate(((ef, range(nc)), (eb, reversed(range(nc))))):
+        order, s, enter = list(order), torch.zeros(b, H, P, N, dtype=torch.float64).cuda(), {}
+        for c in order:
+            enter[c] = s
+            s = e[:, :, c, None, None] * s + st[k][:, c].double()
+        g, ds, dda = torch.zeros_like(s), {}, {}
+        for c in reversed(order):
+            ds[c] = g
+            dda[c] = e[:, :, c] * (g * got[k][:, c].double()).sum((-1, -2))
+            g = dprev[k][:, c].double() + e[:, :, c, None, None] * g
+        stack = lambda d, dim: torch.stack([d[c] for c in range(nc)], dim)
+        # float32 recurrences whose terms shrink by e^-1.6 a chunk; inner products of P N terms
+        for have, want in ((got[k], stack(enter, 1)), (got[2 + k], s), (back[k], stack(ds, 1)), (back[2 + k], stack(dda, 2))):
+            assert float((have - want).norm()) <= 1e-5 * float(want.norm())
