@@ -192,4 +192,118 @@ __device__ __forceinline__ void chunk_state_body(const bimamba2_params &p, int n
         }
 }
 
+// ---------------------------------------------------------------------------------------------------------
+// The same for 16-bit types in chunks of up to 128 positions, headdim and dstate multiples of 8, aligned rows: the whole x tile and
+// the whole B tile of the chunk come by direct loads, all requested at once, and the operands are LDS transpose reads (no registers
+// to stage in, 143 of them above: four workgroups fit a CU instead of three, and each waits for memory once).  A row's units past
+// headdim or dstate are not requested: what lies there gives outputs that nobody stores.
+// 4 x 2048 in chunks of 128, bfloat16, 16 heads, headdim 16, dstate 16: the forward launch 24 -> 15 us, beside dCB 27 -> 22; headdim 128, dstate 32: 35 -> 27 and 26 -> 18.
+// ---------------------------------------------------------------------------------------------------------
+struct ChunkStateNarrowMap {
+    static constexpr int ROWS = 128, TILE = ROWS * 128;                                  // rows of 64 elements, tile64 swizzle
+    static constexpr int WF = 2 * TILE, WB = WF + 4 * BIMAMBA2_MAX_CHUNK, LDS = WB + 4 * BIMAMBA2_MAX_CHUNK;
+};
+template <typename T, bool DSTATES, bool CUMSUM = false>
+__device__ __forceinline__ void chunk_state_narrow_body(const bimamba2_params &p, int nc, int nt, int pt, int bch, char *lds) {
+    typedef Mma<T> M;
+    typedef typename M::Frag Frag;
+    typedef ChunkStateNarrowMap Map;
+    static_assert(sizeof(T) == 2, "16-bit operands");
+    T *xt = reinterpret_cast<T *>(lds), *bt = reinterpret_cast<T *>(lds + Map::TILE);
+    float *wf = reinterpret_cast<float *>(lds + Map::WF), *wb = reinterpret_cast<float *>(lds + Map::WB);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 15, lg = lane >> 4;
+    const int h = bch % p.nheads, bc = bch / p.nheads, c = bc % nc, b = bc / nc;
+    const int g = h / (p.nheads / p.ngroups);
+    const int Q = p.chunk_size, N = p.dstate, P = p.headdim;
+    const int limit = min(Q, p.seqlen - c * Q), rows = (limit + 31) & ~31;
+    const int64_t o = (((int64_t)b * p.nheads + h) * nc + c) * Q;
+    const T *xp, *bp;
+    int64_t xs, bs;
+    if (DSTATES) {
+        if (p.has_z) { xs = (int64_t)p.nheads * P; xp = reinterpret_cast<const T *>(p.dout_x) + ((int64_t)b * p.seqlen + (int64_t)c * Q) * xs + (int64_t)h * P; }
+        else { xs = p.dout_sl; xp = reinterpret_cast<const T *>(p.dout) + b * p.dout_sb + (int64_t)c * Q * xs + h * p.dout_sh; }
+        bs = p.C_sl;
+        bp = reinterpret_cast<const T *>(p.Cm) + b * p.C_sb + (int64_t)c * Q * bs + g * p.C_sg;
+    } else {
+        xs = p.x_sl;
+        xp = reinterpret_cast<const T *>(p.x) + b * p.x_sb + (int64_t)c * Q * xs + h * p.x_sh;
+        bs = p.B_sl;
+        bp = reinterpret_cast<const T *>(p.Bm) + b * p.B_sb + (int64_t)c * Q * bs + g * p.B_sg;
+    }
+    // unit of 8 rows: lane l brings 16 bytes of row l / 8 (rows behind the sequence's end read its last row: weight 0)
+    for (int u = wave; u < rows / 8; u += NTHREADS / 64) {
+        const int row = u * 8 + (lane >> 3), col = ((lane & 7) ^ tile64_swz(row)) << 3;
+        const int64_t r = min(row, limit - 1);
+        if (pt * 64 + col < P) load16_to_lds(xp + r * xs + pt * 64 + col, xt + u * 512);
+        if (nt * 64 + col < N) load16_to_lds(bp + r * bs + nt * 64 + col, bt + u * 512);
+    }
+    if constexpr (CUMSUM && !DSTATES) {
+        if (wave == 0) {
+            float v[4], cf[4], cb[4];
+            if (p.dt_dtype == BIMAMBA2_F32) chunk_cumsum_wave<float, float>(p, b, c, h, lane, v, cf, cb);
+            else if (p.dt_dtype == BIMAMBA2_BF16) chunk_cumsum_wave<bf16_t, float>(p, b, c, h, lane, v, cf, cb);
+            else chunk_cumsum_wave<f16_t, float>(p, b, c, h, lane, v, cf, cb);
+            if (nt == 0 && pt == 0) chunk_cumsum_store(p, o, lane, v, cf, cb);
+            const float ef = __shfl(cf[(Q - 1) & 3], (Q - 1) >> 2, 64), eb = __shfl(cb[0], 0, 64);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                wf[lane * 4 + e] = __expf(ef - cf[e]) * v[e];              // (v is 0 past the end)
+                wb[lane * 4 + e] = __expf(eb - cb[e]) * v[e];
+            }
+        }
+    } else {
+        for (int q = threadIdx.x; q < rows; q += NTHREADS) {
+            const int qc = min(q, limit - 1);
+            const float cf = p.cs_f[o + qc], cb = p.cs_b[o + qc];
+            float f, r;
+            if (DSTATES) { f = __expf(cf); r = __expf(cb); }
+            else {
+                const float d = p.dt_out[o + qc];
+                f = __expf(p.cs_f[o + Q - 1] - cf) * d;
+                r = __expf(p.cs_b[o] - cb) * d;
+            }
+            wf[q] = q < limit ? f : 0.f;
+            wb[q] = q < limit ? r : 0.f;
+        }
+    }
+    wait_vmcnt<0>();
+    __syncthreads();
+    if (pt * 64 + wave * 16 >= P) return;
+    f32x4 accf[4] = {}, accb[4] = {};
+    for (int ks = 0; ks < rows; ks += 32) {
+        const Frag a = tile64_tr_frag<Frag>(xt, ks, wave * 16, lr, lg);
+        float vf[8], vb[8];
+#pragma unroll
+        for (int i = 0; i < 8; i += 4) {
+            const f32x4 f4 = *reinterpret_cast<const f32x4 *>(wf + ks + lg * 8 + i), b4 = *reinterpret_cast<const f32x4 *>(wb + ks + lg * 8 + i);
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const T x = a[i + k];
+                vf[i + k] = to_f(x) * f4[k];
+                vb[i + k] = to_f(x) * b4[k];
+            }
+        }
+        const Frag af = M::pack(vf), ab = M::pack(vb);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            if (nt * 64 + j * 16 >= N) continue;               // (uniform)
+            const Frag bf = tile64_tr_frag<Frag>(bt, ks, j * 16, lr, lg);
+            accf[j] = M::mma(af, bf, accf[j]);
+            accb[j] = M::mma(ab, bf, accb[j]);
+        }
+    }
+    float *of = (DSTATES ? p.dstates_f : p.states_f) + (int64_t)bch * P * N, *ob = (DSTATES ? p.dstates_b : p.states_b) + (int64_t)bch * P * N;
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int pp = pt * 64 + wave * 16 + lg * 4 + i, n = nt * 64 + j * 16 + lr;
+            if (pp < P && n < N) {
+                of[(int64_t)pp * N + n] = accf[j][i];
+                ob[(int64_t)pp * N + n] = accb[j][i];
+            }
+        }
+}
+
 }  // namespace bm2

@@ -1719,6 +1719,7 @@ static RolesShape roles_shape(const bimamba2_params *p) {
     r.dcb_fast = dcb_aligned(p) && p->headdim % 16 == 0;
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     r.dstates_fast = dcb_aligned(p) && p->headdim % 64 == 0 && p->dstate % 64 == 0 && al(p->Cm) && p->C_sb % vs == 0 && p->C_sl % vs == 0 && p->C_sg % vs == 0;
+    r.dstates_narrow = chunk_state_narrow(p, true);
     r.dbdc_fast = dcb_aligned(p) && p->headdim % 64 == 0 && p->dstate % 64 == 0;
     return r;
 }

@@ -51,6 +51,12 @@ __global__ __launch_bounds__(NTHREADS) void bmm_chunk_fwd_kernel(const bimamba2_
     bmm_chunk_fwd_body<T>(p, nc, blockIdx.x, blockIdx.y, blockIdx.z, lds);
 }
 
+template <typename T, bool DSTATES>
+__global__ __launch_bounds__(NTHREADS) void chunk_state_narrow_kernel(const bimamba2_params p, int nc) {
+    __shared__ __attribute__((aligned(16))) char lds[ChunkStateNarrowMap::LDS];
+    chunk_state_narrow_body<T, DSTATES>(p, nc, blockIdx.x, blockIdx.y, blockIdx.z, lds);
+}
+
 template <typename T, bool DSTATES, bool FAST>
 __global__ __launch_bounds__(NTHREADS) void chunk_state_kernel(const bimamba2_params p, int nc) {
     __shared__ __attribute__((aligned(16))) char lds[ChunkStateMap<T>::LDS];
@@ -60,13 +66,15 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_kernel(const bimamba2_pa
 // The forward pass's first kernels in one launch, where the scan kernel reads C.B^T: the first nstate workgroups form chunk states
 // (and the cumulative sums), the others the tiles of C.B^T.  Neither needs the other, none of them fills the chip at the sizes
 // where it matters, and a launch is 3 to 5 us.
-template <typename T, bool FAST>
+template <typename T, bool FAST, bool NARROW>
 __global__ __launch_bounds__(NTHREADS) void fwd_front_kernel(const bimamba2_params p, int nc, int nnt, int npt, int nstate, int nqt) {
-    constexpr int LDS = ChunkStateMap<T>::LDS > BMM_FWD_LDS<T> ? ChunkStateMap<T>::LDS : BMM_FWD_LDS<T>;
-    __shared__ __attribute__((aligned(16))) char lds[LDS];
+    constexpr int STATE_LDS = NARROW ? ChunkStateNarrowMap::LDS : ChunkStateMap<T>::LDS;
+    __shared__ __attribute__((aligned(16))) char lds[STATE_LDS > BMM_FWD_LDS<T> ? STATE_LDS : BMM_FWD_LDS<T>];
     const int id = blockIdx.x;
-    if (id < nstate) chunk_state_body<T, false, FAST, true>(p, nc, id % nnt, id / nnt % npt, id / (nnt * npt), lds);
-    else {
+    if (id < nstate) {
+        if constexpr (NARROW) chunk_state_narrow_body<T, false, true>(p, nc, id % nnt, id / nnt % npt, id / (nnt * npt), lds);
+        else chunk_state_body<T, false, FAST, true>(p, nc, id % nnt, id / nnt % npt, id / (nnt * npt), lds);
+    } else {
         const int k = id - nstate;
         bmm_chunk_fwd_body<T>(p, nc, k % nqt, k / nqt % nqt, k / (nqt * nqt), lds);
     }
@@ -880,6 +888,15 @@ int launch_chunk_state_heads(const bimamba2_params *p) {
 }
 
 
+// whether the kernel with direct loads of whole tiles takes the place of the generic one
+bool chunk_state_narrow(const bimamba2_params *p, bool dstates) {
+    auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    auto mult = [](int64_t a, int64_t b, int64_t c) { return a % 8 == 0 && b % 8 == 0 && c % 8 == 0; };
+    if (p->dtype == BIMAMBA2_F32 || p->chunk_size > ChunkStateNarrowMap::ROWS || p->headdim % 8 || p->dstate % 8) return false;
+    if (!dstates) return al(p->Bm) && mult(p->B_sb, p->B_sl, p->B_sg) && al(p->x) && mult(p->x_sb, p->x_sl, p->x_sh);
+    return al(p->Cm) && mult(p->C_sb, p->C_sl, p->C_sg) && (p->has_z ? al(p->dout_x) : (al(p->dout) && mult(p->dout_sb, p->dout_sl, p->dout_sh)));
+}
+
 template <typename T>
 static int launch_chunk_state_t(const bimamba2_params *p, bool dstates, bool cumsum) {
     const int nc = nchunks(p);
@@ -928,6 +945,13 @@ static int launch_chunk_state_t(const bimamba2_params *p, bool dstates, bool cum
     if (cumsum) return BIMAMBA2_EINVAL;      // the caller checked chunk_state_does_cumsum()
     if (!dstates && !(p->states_f && p->states_b)) return BIMAMBA2_EINVAL;   // (16-bit per-chunk states: the kernel above only)
     if (dstates && !(p->dstates_f && p->dstates_b)) return BIMAMBA2_EINVAL;
+    if constexpr (sizeof(T) == 2) {
+        if (chunk_state_narrow(p, dstates)) {
+            if (dstates) hipLaunchKernelGGL((chunk_state_narrow_kernel<T, true>), grid, dim3(NTHREADS), 0, s, *p, nc);
+            else hipLaunchKernelGGL((chunk_state_narrow_kernel<T, false>), grid, dim3(NTHREADS), 0, s, *p, nc);
+            return check_launch();
+        }
+    }
     if (dstates) {
         if (fast) hipLaunchKernelGGL((chunk_state_kernel<T, true, true>), grid, dim3(NTHREADS), 0, s, *p, nc);
         else hipLaunchKernelGGL((chunk_state_kernel<T, true, false>), grid, dim3(NTHREADS), 0, s, *p, nc);
@@ -968,11 +992,16 @@ template <typename T> static int launch_fwd_front_t(const bimamba2_params *p, bo
     const dim3 grid(nstate + nqt * nqt * p->batch * nc * p->ngroups);
     if constexpr (sizeof(T) == 4) {
         if (fast) {
-            hipLaunchKernelGGL((fwd_front_kernel<T, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
+            hipLaunchKernelGGL((fwd_front_kernel<T, true, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
+            return check_launch();
+        }
+    } else {
+        if (chunk_state_narrow(p, false)) {
+            hipLaunchKernelGGL((fwd_front_kernel<T, false, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
             return check_launch();
         }
     }
-    hipLaunchKernelGGL((fwd_front_kernel<T, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
+    hipLaunchKernelGGL((fwd_front_kernel<T, false, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
     return check_launch();
 }
 

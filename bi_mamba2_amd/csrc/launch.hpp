@@ -26,6 +26,7 @@ int launch_seq_boundaries(const bimamba2_params *p, int32_t *counts);
 int launch_bmm_chunk_fwd(const bimamba2_params *p);
 int launch_chunk_state(const bimamba2_params *p, bool dstates, bool cumsum = false);   // cumsum: also does the chunk cumsum
 bool chunk_state_does_cumsum(const bimamba2_params *p);
+bool chunk_state_narrow(const bimamba2_params *p, bool dstates);
 // chunk cumsum, chunk states and C.B^T as one launch, where fwd_front_merged() says it exists
 bool fwd_front_merged(const bimamba2_params *p);
 int launch_fwd_front(const bimamba2_params *p);
@@ -78,7 +79,7 @@ int launch_bwd_tail_small(const bimamba2_params *p, ReduceJobs *defer, int ncb);
 // launches of several roles (roles.hpp), with what their kernels' own launches know about the problem
 struct RolesShape {
     int nchunks, dcb_slices, dbdc_slices, dbdc_heads;
-    bool dcb_ring, dcb_fast, dstates_fast, dbdc_fast;
+    bool dcb_ring, dcb_fast, dstates_fast, dstates_narrow, dbdc_fast;
 };
 bool dcb_dstates_merged(const bimamba2_params *p);      // dCB and dstates in one launch
 int launch_dcb_dstates(const bimamba2_params *p);

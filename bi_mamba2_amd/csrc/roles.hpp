@@ -18,11 +18,13 @@ static inline bool roles_al16(const void *q) { return (reinterpret_cast<uintptr_
 
 // ---- dCB and the gradients of the states entering the chunks ----
 // RING: columns per step of the ring variant (16-bit types; WHOLE: headdim a multiple of 64), 0: the variant through registers
-// DFAST, CFAST: unconditional loads in that one and in the kernel of the states' gradients
+// DFAST, CFAST: unconditional loads in that one and in the kernel of the states' gradients (16 bits: the one with direct loads)
 template <typename T, int RING, bool WHOLE, bool DFAST, bool CFAST>
 __global__ __launch_bounds__(NTHREADS) void bwd_dcb_dstates_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int gdz, int nnt, int npt, int ndcb) {
     constexpr int DCB_LDS = RING ? DcbRingMap<RING ? RING : 64>::LDS : DcbMap::LDS;
-    __shared__ __attribute__((aligned(16))) char lds[DCB_LDS > ChunkStateMap<T>::LDS ? DCB_LDS : ChunkStateMap<T>::LDS];
+    constexpr bool NARROW = sizeof(T) == 2 && CFAST;
+    constexpr int STATE_LDS = NARROW ? ChunkStateNarrowMap::LDS : ChunkStateMap<T>::LDS;
+    __shared__ __attribute__((aligned(16))) char lds[DCB_LDS > STATE_LDS ? DCB_LDS : STATE_LDS];
     const int id = blockIdx.x;
     if (id < ndcb) {
         const int per = gdx * nqt * nqt;
@@ -35,7 +37,8 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_dstates_kernel(const bimamba
         }
     } else {
         const int k = id - ndcb;
-        chunk_state_body<T, true, CFAST>(p, nc, k % nnt, k / nnt % npt, k / (nnt * npt), lds);
+        if constexpr (NARROW) chunk_state_narrow_body<T, true>(p, nc, k % nnt, k / nnt % npt, k / (nnt * npt), lds);
+        else chunk_state_body<T, true, CFAST>(p, nc, k % nnt, k / nnt % npt, k / (nnt * npt), lds);
     }
 }
 
@@ -64,7 +67,11 @@ template <typename T> int launch_dcb_dstates_t(const bimamba2_params *p, const R
 #define BM2_R(RING, WHOLE, DFAST, CFAST) hipLaunchKernelGGL((bwd_dcb_dstates_kernel<T, RING, WHOLE, DFAST, CFAST>), grid, dim3(NTHREADS), 0, s, *p, nc, nqt, gdx, gdz, nnt, npt, ndcb)
     if constexpr (sizeof(T) == 2) {
         if (!r.dcb_ring) return BIMAMBA2_EINVAL;
-        if (p->headdim <= 32) BM2_R(32, false, false, false);
+        if (r.dstates_narrow) {
+            if (p->headdim <= 32) BM2_R(32, false, false, true);
+            else if (p->headdim % 64) BM2_R(64, false, false, true);
+            else BM2_R(64, true, false, true);
+        } else if (p->headdim <= 32) BM2_R(32, false, false, false);
         else if (p->headdim % 64) BM2_R(64, false, false, false);
         else BM2_R(64, true, false, false);
     } else {

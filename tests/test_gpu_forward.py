@@ -181,3 +181,23 @@ def test_first_kernels_in_one_launch(b, L, H, P, G, N, Q, dtype, dt_dtype):
     # the weights of the states come from the sums in registers instead of memory: the same values, the same order of products
     for got, want in zip((res[5], res[6], res[0]), (sf, sb, out)):
         assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("P,N", [(8, 8), (16, 72), (24, 16), (64, 40), (72, 64), (128, 136)])
+@pytest.mark.parametrize("L,Q,dtype", [(1, 32, torch.bfloat16), (95, 64, torch.float16), (129, 128, torch.bfloat16), (100, 50, torch.bfloat16)])
+def test_chunk_states_of_narrow_tiles(P, N, L, Q, dtype):
+    """the kernel with direct loads of whole tiles (16 bits, up to 128 positions, sizes that are multiples of 8) for states and for
+    their gradients, rows and columns that are no whole tile included, against float64"""
+    from bi_mamba2_amd import ops
+    b, H, G = 2, 4, 2
+    d = to_dev(make_case(b, L, H, P, G, N, dtype))
+    csf, csb, dt = ops._chunk_cumsum_fwd(d["dt"], d["A"], Q, dt_bias=d["dt_bias"], dt_softplus=True)
+    nc = csf.shape[2]
+    pad = lambda t: torch.nn.functional.pad(t.double(), (0, 0, 0, 0, 0, nc * Q - L)).view(b, nc, Q, *t.shape[2:])
+    rows = lambda e: e.double().permute(0, 2, 3, 1)                                        # (b, nc, Q, H)
+    for got, x, mate, wf, wb in ((ops._chunk_state_fwd(d["B"], d["x"], dt, csf, csb), d["x"], d["B"], dt.double() * (csf[..., -1:] - csf).double().exp(), dt.double() * (csb[..., :1] - csb).double().exp()),
+                                 (ops._chunk_scan_bwd_dstates(d["C"], csf, csb, d["x"]), d["x"], d["C"], csf.double().exp(), csb.double().exp())):
+        for g, w in zip(got, (wf, wb)):
+            want = torch.einsum("bcqhp,bcqhn->bchpn", pad(x) * rows(w)[..., None], pad(mate).repeat_interleave(H // G, 3))
+            # one operand carries the weight and is rounded to the inputs' type (at most half a unit in its last place)
+            assert float((g - want).norm() / want.norm()) < {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
