@@ -452,7 +452,8 @@ int bimamba2_bwd(const bimamba2_params *p) {
     }
     // dCB / dCBT in the 16-bit element type where this call owns them and the two launches that write and read them are the
     // merged ones (their reader rounds them to that type for its MFMA anyway)
-    const bool dcb16 = !p->dCB && !p->dCBT && bwd_dcb_sp_merged(&q) && bwd_tail_merged(&q);
+    const bool own_dcb = !p->dCB && !p->dCBT, dcb_sp = bwd_dcb_sp_merged(&q) && (own_dcb || dcb_slices(&q) == 1);
+    const bool dcb16 = own_dcb && dcb_sp && dcb_slices(&q) == 1 && bwd_tail_merged(&q);
     const bool need_cbt = !scan_recomputes_cb(&q, true), need_cb = need_cbt || !dcb_recomputes_cb(&q);
     const bool saved_cb = (p->fwd_saved & 2) && p->CB && p->CBT;
     const bool form_cb = need_cb && !saved_cb;     // (else left there by the forward pass)
@@ -465,13 +466,13 @@ int bimamba2_bwd(const bimamba2_params *p) {
         REQUIRE(q.z); REQUIRE(q.dout); REQUIRE(q.out_x); REQUIRE(q.dz); REQUIRE(q.dout_x); REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.CB);
         TRY(launch_bwd_dz_bmm(&q));
     } else if (q.has_z) TRY(bimamba2_chunk_scan_bwd_dz(&q));
-    // the last launch adds up the head slices of dCB where it is the one that does so
+    // the last launch adds up the head slices of dCB
     const bool tail_small = !bwd_tail_merged(&q) && bwd_tail_small(&q);
-    const int ncb = tail_small && !p->dCB && !p->dCBT && !bwd_dcb_sp_merged(&q) ? dcb_slices(&q) : 1;
+    const int ncb = own_dcb && (tail_small || bwd_tail_merged(&q)) ? dcb_slices(&q) : 1;
     // the dCB kernel is bound by instruction issue and moves little data: right behind dz it runs while the memory system
     // still writes back dz's output, which the memory-bound kernels after it would otherwise wait behind
     const bool dx_db_dc = dx_db_dc_merged(&q);      // (one launch at the end)
-    if (bwd_dcb_sp_merged(&q)) {
+    if (dcb_sp && (ncb == dcb_slices(&q))) {
         // the backward state passing (streams, few instructions) rides along with the dCB kernel in one launch
         if (!dx_db_dc) TRY(bimamba2_chunk_scan_bwd_dc(&q));
         if (!dz_dstates) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
@@ -517,7 +518,7 @@ int bimamba2_bwd(const bimamba2_params *p) {
         qc.red = q.red + (size_t)q.batch * nchunks(&q) * q.nheads * q.headdim;
         REQUIRE(q.ddt); REQUIRE(q.dA); REQUIRE(q.dB); REQUIRE(q.dC);
         if (bwd_tail_merged(&q)) {
-            TRY(launch_bwd_tail(&qc, &jobs, dcb16));
+            TRY(launch_bwd_tail(&qc, &jobs, dcb16, ncb));
         } else if (tail_small) {
             REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dt); REQUIRE(q.A);
             if (q.has_dt_bias) REQUIRE(q.dt_bias);

@@ -961,16 +961,19 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_ring_kernel(const bimamba2_p
     bwd_dcb_ring_body<T, UNI, KC, WHOLE>(p, nc, nqt, bid, gridDim.x, gridDim.z, smem);
 }
 
-// The dCB kernel and the backward state passing as roles of one launch (one head slice): the first is bound by instruction issue and moves little data, the second streams
+// The dCB kernel and the backward state passing as roles of one launch: the first is bound by instruction issue and moves little data, the second streams
 // 70 MB and needs few instructions, and the two depend on different kernels before them.  The first ndcb blocks are the
 // dCB tiles in the order of their own grid (so they are placed first, two per CU as when alone), the rest are the state
 // passing's blocks, which take what is left of each CU.
 template <typename T, bool UNI>
-__device__ __forceinline__ void bwd_dcb_sp_body(const bimamba2_params &p, int nc, int nqt, int gdx, int ndcb, int nsplit, int ndir, bool out16) {
+__device__ __forceinline__ void bwd_dcb_sp_body(const bimamba2_params &p, int nc, int nqt, int gdx, int ndcb, int nslices, int nsplit, int ndir, bool out16) {
     const int id = blockIdx.x;
     if (id < ndcb) {
         __shared__ __attribute__((aligned(16))) unsigned char smem[DcbRingMap<64>::LDS];
-        bwd_dcb_ring_body<T, UNI, 64, true>(p, nc, nqt, dcb_block_of(id, gdx, nqt * nqt, ndcb), gdx, 1, smem, out16);
+        const int ntiles = gdx * nqt * nqt;
+        BlockId tile = dcb_block_of(id % ntiles, gdx, nqt * nqt, ntiles);
+        tile.z = id / ntiles;
+        bwd_dcb_ring_body<T, UNI, 64, true>(p, nc, nqt, tile, gdx, nslices, smem, out16);
     } else {
         const int k = id - ndcb;                  // grid (nsplit, nheads, batch * ndir) of the state passing
         const BlockId sb{k % nsplit, (k / nsplit) % p.nheads, k / (nsplit * p.nheads)};
@@ -981,8 +984,8 @@ __device__ __forceinline__ void bwd_dcb_sp_body(const bimamba2_params &p, int nc
 }
 
 template <typename T, bool UNI>
-__global__ __launch_bounds__(NTHREADS) void bwd_dcb_sp_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int ndcb, int nsplit, int ndir, bool out16) {
-    bwd_dcb_sp_body<T, UNI>(p, nc, nqt, gdx, ndcb, nsplit, ndir, out16);
+__global__ __launch_bounds__(NTHREADS) void bwd_dcb_sp_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int ndcb, int nslices, int nsplit, int ndir, bool out16) {
+    bwd_dcb_sp_body<T, UNI>(p, nc, nqt, gdx, ndcb, nslices, nsplit, ndir, out16);
 }
 // Narrow heads (16-bit) take the ring as well: through registers a workgroup waits for its operands head by head.  4 x 2048 in chunks of
 // 128, 16 heads of 16: 46 -> 21 us; 48 heads of 16: the whole pass 497 -> 389 us; in 8 groups (two heads a tile) 43 -> 28 us.
@@ -1045,10 +1048,14 @@ static int launch_dcb_t(const bimamba2_params *p, bool add_up) {
     return check_launch();
 }
 
-// Head slices where bimamba2_bwd owns dCB and the kernel reads C.B^T: float32, and 16-bit shapes whose state or headdim is no
-// multiple of what the rebuilding kernel takes (the ring with a narrow state or narrow heads; through registers where rows are
-// not aligned).  Where C.B^T is rebuilt the
-// number is dcb_slices()'s: every slice would rebuild it, and one slice shares its launch with the state passing.
+// Head slices where bimamba2_bwd owns dCB.
+// The kernel rebuilds C.B^T (16 bits, wide heads): a slice starts with its own copy of the tile, and the last launch reads the slices in
+// float32 instead of one in 16 bits; they pay while compute units are left without two workgroups.  us a training pass with 1 / 2 / 4
+// slices, heads of 64, dstate 64, chunks of 256: 48 heads, 64 tiles 161 / 135 / 124, 128 tiles 183 / 158 / 152, 384 tiles 312 / 297 / 314;
+// 32 heads of 128, dstate 128, 96 tiles 264 / 240 / 234; from 512 tiles on they cost (32 heads 244 / 249 / 271; 16 heads 154 / 157 / 167).
+// Between 256 and 384 tiles few heads give little (24 heads 150 / 143 / 146, with dstate 128 306 / 302 / 316): one slice up to 31 heads.
+// The kernel reads C.B^T (float32, and 16-bit shapes whose state or headdim is no multiple of what the rebuilding kernel takes: the ring
+// with a narrow state or narrow heads; through registers where rows are not aligned).
 // A workgroup is one chain over its heads, 5 to 7 us a head through registers in float32, 3 to 5 in 16 bits and 1.5 in the ring,
 // so slices pay on a small grid until there are three workgroups on every CU; against them stands a launch that adds them up
 // (4 us, and 0.03 us per tile and slice), which few heads do not earn: in 16 bits a slice wants a head per 32 tiles of the grid,
@@ -1062,20 +1069,25 @@ static int launch_dcb_t(const bimamba2_params *p, bool add_up) {
 int choose_dcb_slices(const bimamba2_params *p) {
     const int usual = dcb_slices(p), hpg = p->nheads / p->ngroups, nqt = (p->chunk_size + 63) / 64;
     const int64_t n = (int64_t)p->batch * nchunks(p) * p->ngroups * p->chunk_size * p->chunk_size;
-    if (dcb_recomputes_cb(p) || p->causal || n % 4) return usual;
+    if (p->causal || n % 4) return usual;
     const int64_t wgs = (int64_t)p->batch * nchunks(p) * p->ngroups * nqt * nqt;
-    const int most = p->dtype == BIMAMBA2_F32 ? (hpg < 6 ? 256 : 768) : std::min(768, 32 * hpg);      // workgroups
-    const int wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, most / wgs}));
+    int wanted = usual;
+    if (dcb_recomputes_cb(p)) {
+        if (wgs < 256 || (wgs <= 384 && hpg >= DCB_SLICE_HEADS)) wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 4, 4, std::max<int64_t>(512 / wgs, 2)}));
+    } else {
+        const int most = p->dtype == BIMAMBA2_F32 ? (hpg < 6 ? 256 : 768) : std::min(768, 32 * hpg);      // workgroups
+        wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, most / wgs}));
+    }
     const int heads = (hpg + wanted - 1) / wanted;               // (9 heads in 4 slices: three of 3, the fourth would be empty)
     return (hpg + heads - 1) / heads;
 }
 
-// whether bwd_dcb_sp_kernel exists for the problem (the ring variant of the dCB kernel with one head slice, the vector
+// whether bwd_dcb_sp_kernel exists for the problem (the ring variant of the dCB kernel, the vector
 // variant of the state passing)
 bool bwd_dcb_sp_merged(const bimamba2_params *p) {
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     if (p->dtype != BIMAMBA2_BF16 && p->dtype != BIMAMBA2_F16) return false;
-    if (!dcb_recomputes_cb(p) || dcb_slices(p) != 1) return false;       // (implies the conditions of the ring variant)
+    if (!dcb_recomputes_cb(p)) return false;                             // (implies the conditions of the ring variant)
     // the entering states and their gradients both in 16 bits, or (state dimension 128) both in float32
     if (p->states16_f && p->dstates16_f ? !(p->causal || (p->states16_b && p->dstates16_b))
                                         : p->states16_f || p->dstates16_f || p->causal || !p->states_f || !p->states_b || !p->dstates_f || !p->dstates_b)
@@ -1090,12 +1102,12 @@ bool bwd_dcb_sp_merged(const bimamba2_params *p) {
 int launch_bwd_dcb_sp(const bimamba2_params *p, bool out16) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, PN = p->headdim * p->dstate;
     const int nsplit = (PN + SP_EPT * NTHREADS - 1) / (SP_EPT * NTHREADS), ndir = p->causal ? 1 : 2;
-    const int gdx = p->batch * nc * p->ngroups, ndcb = gdx * nqt * nqt, nsp = nsplit * p->nheads * p->batch * ndir;
+    const int slices = dcb_slices(p), gdx = p->batch * nc * p->ngroups, ndcb = gdx * nqt * nqt * slices, nsp = nsplit * p->nheads * p->batch * ndir;
     dim3 grid(ndcb + nsp);
 #define BM2_DS(TT)                                                                                                                     \
     do {                                                                                                                               \
-        if (p->causal) hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, ndcb, nsplit, ndir, out16);  \
-        else hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, ndcb, nsplit, ndir, out16);           \
+        if (p->causal) hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, ndcb, slices, nsplit, ndir, out16);  \
+        else hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, ndcb, slices, nsplit, ndir, out16);           \
     } while (0)
     if (p->dtype == BIMAMBA2_BF16) BM2_DS(bf16_t); else BM2_DS(f16_t);
 #undef BM2_DS
@@ -1560,7 +1572,7 @@ __global__ __launch_bounds__(NTHREADS) void chunk_cumsum_bwd_kernel(const bimamb
 // other, both are short and latency-bound, and together they fit the machine in one wave of workgroups.
 template <typename T, typename DT, bool SLIM = false>
 __global__ __launch_bounds__(NTHREADS) void bwd_tail_kernel(const bimamba2_params p, int nc, int nslices, int nqt, int nsplit, int nbmm,
-                                                            int bmm_gy, int cs_gx, bool in16) {
+                                                            int bmm_gy, int cs_gx, bool in16, int ncb) {
     const int id = blockIdx.x;
     if (id < nbmm) {
         // bmm grid (n tiles, bmm_gy, z), bmm_gy here counting both.  The bmm_gy tiles of one z = (which, b, c, g) stage the same
@@ -1569,7 +1581,7 @@ __global__ __launch_bounds__(NTHREADS) void bwd_tail_kernel(const bimamba2_param
         const int nz = nbmm / bmm_gy, k = id >> 3;
         const int t = nz % 8 == 0 ? k % bmm_gy : id % bmm_gy, ntiles = p.dstate >> 6;
         const BlockId bb{t % ntiles, t / ntiles, nz % 8 == 0 ? (k / bmm_gy) * 8 + (id & 7) : id / bmm_gy};
-        bmm_chunk_bwd_body<T, 256, true, SLIM>(p, nc, nslices, bb, in16);
+        bmm_chunk_bwd_body<T, 256, true, SLIM>(p, nc, nslices, bb, in16, ncb);
     } else {
         const int k = id - nbmm;                  // cumsum grid (cs_gx, nc, batch)
         chunk_cumsum_bwd_body<DT>(p, nc, nqt, nsplit, BlockId{k % cs_gx, (k / cs_gx) % nc, k / (cs_gx * nc)});
@@ -1603,24 +1615,24 @@ static bool bmm_bwd_fast(const bimamba2_params *p) {
 bool bwd_tail_merged(const bimamba2_params *p) { return bmm_bwd_fast(p) && p->chunk_size == 256 && (p->dstate == 64 || p->dstate == 128); }
 
 template <typename T>
-static int launch_bwd_tail_t(const bimamba2_params *p, int nc, int nqt, int nsplit, bool in16) {
+static int launch_bwd_tail_t(const bimamba2_params *p, int nc, int nqt, int nsplit, bool in16, int ncb) {
     const int bmm_gy = (p->chunk_size + 63) / 64 * (p->dstate / 64), nbmm = bmm_gy * p->batch * nc * p->ngroups * 2;
     const int cs_gx = (p->nheads + 3) / 4, ncs = cs_gx * nc * p->batch;
     dim3 grid(nbmm + ncs);
     const int nsl = dbdc_slices(p);
     if (in16 && nsl <= 2) {
         switch (p->dt_dtype) {
-            case BIMAMBA2_F32: hipLaunchKernelGGL((bwd_tail_kernel<T, float, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16); break;
-            case BIMAMBA2_BF16: hipLaunchKernelGGL((bwd_tail_kernel<T, bf16_t, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16); break;
-            case BIMAMBA2_F16: hipLaunchKernelGGL((bwd_tail_kernel<T, f16_t, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16); break;
+            case BIMAMBA2_F32: hipLaunchKernelGGL((bwd_tail_kernel<T, float, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16, ncb); break;
+            case BIMAMBA2_BF16: hipLaunchKernelGGL((bwd_tail_kernel<T, bf16_t, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16, ncb); break;
+            case BIMAMBA2_F16: hipLaunchKernelGGL((bwd_tail_kernel<T, f16_t, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16, ncb); break;
             default: return BIMAMBA2_EUNSUPPORTED;
         }
         return check_launch();
     }
     switch (p->dt_dtype) {
-        case BIMAMBA2_F32: hipLaunchKernelGGL((bwd_tail_kernel<T, float>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16); break;
-        case BIMAMBA2_BF16: hipLaunchKernelGGL((bwd_tail_kernel<T, bf16_t>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16); break;
-        case BIMAMBA2_F16: hipLaunchKernelGGL((bwd_tail_kernel<T, f16_t>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16); break;
+        case BIMAMBA2_F32: hipLaunchKernelGGL((bwd_tail_kernel<T, float>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16, ncb); break;
+        case BIMAMBA2_BF16: hipLaunchKernelGGL((bwd_tail_kernel<T, bf16_t>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16, ncb); break;
+        case BIMAMBA2_F16: hipLaunchKernelGGL((bwd_tail_kernel<T, f16_t>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16, ncb); break;
         default: return BIMAMBA2_EUNSUPPORTED;
     }
     return check_launch();
@@ -1664,11 +1676,11 @@ int launch_bwd_tail_small(const bimamba2_params *p, ReduceJobs *defer, int ncb) 
 
 // bmm_chunk_bwd + chunk_cumsum_bwd in one launch (the caller checked bwd_tail_merged()); reductions as in
 // launch_chunk_cumsum_bwd
-int launch_bwd_tail(const bimamba2_params *p, ReduceJobs *defer, bool in16) {
+int launch_bwd_tail(const bimamba2_params *p, ReduceJobs *defer, bool in16, int ncb) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64;
     const int PN = p->headdim * p->dstate;
     const int nsplit = (PN + SP_EPT * NTHREADS - 1) / (SP_EPT * NTHREADS);
-    int rc = p->dtype == BIMAMBA2_BF16 ? launch_bwd_tail_t<bf16_t>(p, nc, nqt, nsplit, in16) : launch_bwd_tail_t<f16_t>(p, nc, nqt, nsplit, in16);
+    int rc = p->dtype == BIMAMBA2_BF16 ? launch_bwd_tail_t<bf16_t>(p, nc, nqt, nsplit, in16, ncb) : launch_bwd_tail_t<f16_t>(p, nc, nqt, nsplit, in16, ncb);
     if (rc) return rc;
     const int ni = p->batch * nc;
     defer->job[defer->n++] = ReduceJob{p->red, p->dA, ni, p->nheads, 1};

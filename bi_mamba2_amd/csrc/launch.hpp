@@ -72,7 +72,7 @@ bool bwd_dcb_sp_merged(const bimamba2_params *p);
 // them to that type anyway)
 int launch_bwd_dcb_sp(const bimamba2_params *p, bool out16 = false);
 bool bwd_tail_merged(const bimamba2_params *p);
-int launch_bwd_tail(const bimamba2_params *p, ReduceJobs *defer, bool in16 = false);
+int launch_bwd_tail(const bimamba2_params *p, ReduceJobs *defer, bool in16 = false, int ncb = 1);
 // the same for chunks of up to 128 positions, any type and shape (ncb: head slices of dCB still to be added up)
 bool bwd_tail_small(const bimamba2_params *p);
 int launch_bwd_tail_small(const bimamba2_params *p, ReduceJobs *defer, int ncb);

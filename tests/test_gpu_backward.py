@@ -179,6 +179,17 @@ def test_last_launch_adds_up_head_slices(ops, b, L, H, P, G, N, Q, dtype, dt_dty
             assert float((a.double() - c.double()).norm()) <= tol * float(c.double().norm())
 
 
+@pytest.mark.parametrize("case", [
+    (1, 300, 13, 64, 1, 64, 256, torch.bfloat16, torch.float32, True),     # three slices, the last with fewer heads; a ragged chunk
+    (1, 257, 16, 128, 2, 128, 256, torch.float16, torch.float16, False),   # two slices a group; float32 states and gradients
+    (1, 130, 24, 64, 1, 64, 128, torch.bfloat16, torch.bfloat16, True),    # the last launch for chunks of up to 128
+    (2, 65, 8, 64, 1, 64, 64, torch.bfloat16, torch.float16, False),       # a dt type without it: the slices' own launch
+])
+def test_head_slices_of_wide_heads(ops, case):
+    """the same for the launch that rebuilds C.B^T and passes the states beside it, on grids small enough for slices"""
+    test_last_launch_adds_up_head_slices(ops, *case)
+
+
 @pytest.mark.parametrize("b,L,H,P,G,N,Q,dtype,z", [
     (1, 130, 4, 16, 2, 16, 64, torch.float32, True),          # one column tile of the state, two chunks and a rest
     (1, 128, 3, 64, 1, 32, 128, torch.float32, False),        # two; two headdim tiles a dx workgroup owns one of
