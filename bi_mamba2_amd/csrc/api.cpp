@@ -436,7 +436,8 @@ int bimamba2_fwd_static(const bimamba2_params *p) {
     return bimamba2_fwd(&q);
 }
 
-int bimamba2_bwd(const bimamba2_params *p) {
+// leave: the final sums are appended to it instead of being launched
+static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     TRY(check_problem(p));
     bimamba2_params q = *p;
     q.final_f = q.final_b = nullptr;
@@ -528,9 +529,12 @@ int bimamba2_bwd(const bimamba2_params *p) {
             TRY(launch_chunk_cumsum_bwd(&qc, &jobs));
         }
     }
-    TRY(launch_reduce_jobs(jobs, stream_of(&q)));
+    if (leave) *leave = jobs;
+    else TRY(launch_reduce_jobs(jobs, stream_of(&q)));
     return BIMAMBA2_OK;
 }
+
+int bimamba2_bwd(const bimamba2_params *p) { return backward(p, nullptr); }
 
 size_t bimamba2_norm_params_size(void) { return sizeof(bimamba2_norm_params); }
 
@@ -555,13 +559,18 @@ int bimamba2_rmsnorm_gated_fwd(const bimamba2_norm_params *p) {
     return launch_rmsnorm_gated(p, false);
 }
 
-int bimamba2_rmsnorm_gated_bwd(const bimamba2_norm_params *p) {
+static int check_norm_bwd(const bimamba2_norm_params *p) {
     TRY(check_norm(p));
     REQUIRE(p->dout); REQUIRE(p->rstd); REQUIRE(p->dx); REQUIRE(p->dweight);
     if (p->layer_norm) REQUIRE(p->mean);
     if (p->has_z) REQUIRE(p->dz);
     if (p->has_bias) REQUIRE(p->dbias);
     if (!p->workspace || p->workspace_bytes < norm_workspace_bytes(p)) return BIMAMBA2_EWORKSPACE;
+    return BIMAMBA2_OK;
+}
+
+int bimamba2_rmsnorm_gated_bwd(const bimamba2_norm_params *p) {
+    TRY(check_norm_bwd(p));
     return launch_rmsnorm_gated(p, true);
 }
 
@@ -569,7 +578,7 @@ size_t bimamba2_conv_params_size(void) { return sizeof(bimamba2_conv_params); }
 
 size_t bimamba2_cast_params_size(void) { return sizeof(bimamba2_cast_params); }
 
-int bimamba2_cast_many(const bimamba2_cast_params *p) {
+static int check_cast(const bimamba2_cast_params *p) {
     if (!p || p->count < 0 || p->count > BIMAMBA2_CAST_MAX) return BIMAMBA2_EINVAL;
     auto known = [](int d) { return d == BIMAMBA2_F32 || d == BIMAMBA2_BF16 || d == BIMAMBA2_F16; };
     for (int k = 0; k < p->count; ++k) {
@@ -579,6 +588,11 @@ int bimamba2_cast_many(const bimamba2_cast_params *p) {
         if (it.op < BIMAMBA2_CAST_COPY || it.op > BIMAMBA2_CAST_MUL) return BIMAMBA2_EINVAL;
         if (it.op == BIMAMBA2_CAST_MUL && it.n > 0 && !it.aux) return BIMAMBA2_EINVAL;
     }
+    return BIMAMBA2_OK;
+}
+
+int bimamba2_cast_many(const bimamba2_cast_params *p) {
+    TRY(check_cast(p));
     return launch_cast_many(p);
 }
 
@@ -604,17 +618,37 @@ int bimamba2_conv1d_silu_fwd(const bimamba2_conv_params *p) {
     return launch_conv1d_silu(p, false);
 }
 
-int bimamba2_conv1d_silu_bwd(const bimamba2_conv_params *p) {
+static int check_conv_bwd(const bimamba2_conv_params *p) {
     TRY(check_conv(p));
     REQUIRE(p->dout); REQUIRE(p->dx); REQUIRE(p->dweight);
     if (p->has_bias) REQUIRE(p->dbias);
     if (!p->workspace || p->workspace_bytes < conv_workspace_bytes(p)) return BIMAMBA2_EWORKSPACE;
+    return BIMAMBA2_OK;
+}
+
+int bimamba2_conv1d_silu_bwd(const bimamba2_conv_params *p) {
+    TRY(check_conv_bwd(p));
     if (p->batch == 0 || p->seqlen == 0) {
         TRY(launch_fill(p->dweight, (size_t)p->channels * p->width, 0.f, reinterpret_cast<hipStream_t>(p->stream)));
         if (p->has_bias) TRY(launch_fill(p->dbias, (size_t)p->channels, 0.f, reinterpret_cast<hipStream_t>(p->stream)));
         return BIMAMBA2_OK;
     }
     return launch_conv1d_silu(p, true);
+}
+
+int bimamba2_norm_scan_conv_bwd(const bimamba2_norm_params *norm, const bimamba2_params *scan, const bimamba2_conv_params *conv,
+                                const bimamba2_cast_params *casts) {
+    TRY(check_norm_bwd(norm));
+    TRY(check_problem(scan));
+    TRY(check_conv_bwd(conv));
+    TRY(check_cast(casts));
+    if (norm->rows == 0 || conv->batch == 0 || conv->seqlen == 0) return BIMAMBA2_EINVAL;
+    if (norm->stream != scan->stream || conv->stream != scan->stream) return BIMAMBA2_EINVAL;
+    LayerSums sums;
+    TRY(launch_rmsnorm_gated(norm, true, &sums));
+    TRY(backward(scan, &sums.jobs));
+    TRY(launch_conv1d_silu(conv, true, &sums));
+    return launch_layer_sums(sums, casts, stream_of(scan));
 }
 
 size_t bimamba2_gemm_params_size(void) { return sizeof(bimamba2_gemm_params); }

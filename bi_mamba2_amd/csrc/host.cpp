@@ -50,12 +50,11 @@ struct Api {
     decltype(&bimamba2_seq_boundaries) seq_boundaries = nullptr;
     decltype(&bimamba2_strerror) strerror = nullptr;
     decltype(&bimamba2_rmsnorm_gated_fwd) norm_fwd = nullptr;
-    decltype(&bimamba2_rmsnorm_gated_bwd) norm_bwd = nullptr;
     decltype(&bimamba2_rmsnorm_gated_workspace_bytes) norm_workspace = nullptr;
     decltype(&bimamba2_conv1d_silu_fwd) conv_fwd = nullptr;
-    decltype(&bimamba2_conv1d_silu_bwd) conv_bwd = nullptr;
     decltype(&bimamba2_conv1d_silu_workspace_bytes) conv_workspace = nullptr;
     decltype(&bimamba2_cast_many) cast_many = nullptr;
+    decltype(&bimamba2_norm_scan_conv_bwd) norm_scan_conv_bwd = nullptr;
     decltype(&bimamba2_gemm) gemm = nullptr;
     decltype(&bimamba2_gemm_workspace_bytes) gemm_workspace = nullptr;
 } api;
@@ -86,12 +85,11 @@ void load(const std::string &path) {
     get(api.seq_boundaries, "bimamba2_seq_boundaries");
     get(api.strerror, "bimamba2_strerror");
     get(api.norm_fwd, "bimamba2_rmsnorm_gated_fwd");
-    get(api.norm_bwd, "bimamba2_rmsnorm_gated_bwd");
     get(api.norm_workspace, "bimamba2_rmsnorm_gated_workspace_bytes");
     get(api.conv_fwd, "bimamba2_conv1d_silu_fwd");
-    get(api.conv_bwd, "bimamba2_conv1d_silu_bwd");
     get(api.conv_workspace, "bimamba2_conv1d_silu_workspace_bytes");
     get(api.cast_many, "bimamba2_cast_many");
+    get(api.norm_scan_conv_bwd, "bimamba2_norm_scan_conv_bwd");
     get(api.gemm, "bimamba2_gemm");
     get(api.gemm_workspace, "bimamba2_gemm_workspace_bytes");
 }
@@ -824,51 +822,44 @@ public:
         const Tensor dyn = device_empty({s.rows, s.inner}, u.scalar_type(), u), dy = device_empty({s.rows, s.inner}, u.scalar_type(), u);
         const Tensor dzx = device_empty({s.rows, s.pitch}, u.scalar_type(), u).narrow(1, 0, s.proj);
         product_nn(dout, w_out, dyn);
-        {
-            bimamba2_norm_params n = layer_norm_params(s, o, zx, y, w, stream);
-            n.rstd = rstd.mutable_data_ptr<float>();
-            n.dout = dyn.const_data_ptr(); n.dout_rs = s.inner;
-            n.dx = dy.mutable_data_ptr(); n.dx_rs = s.inner;
-            n.dz = at_byte(dzx, 0); n.dz_rs = s.pitch;
-            n.dweight = g + off[5];
-            const Tensor ws = device_empty({(int64_t)std::max<size_t>(api.norm_workspace(&n), 1)}, at::kByte, u);
-            n.workspace = ws.mutable_data_ptr();
-            n.workspace_bytes = ws.numel();
-            check(api.norm_bwd(&n), "bimamba2_rmsnorm_gated_bwd");
-        }
+        bimamba2_norm_params n = layer_norm_params(s, o, zx, y, w, stream);
+        n.rstd = rstd.mutable_data_ptr<float>();
+        n.dout = dyn.const_data_ptr(); n.dout_rs = s.inner;
+        n.dx = dy.mutable_data_ptr(); n.dx_rs = s.inner;
+        n.dz = at_byte(dzx, 0); n.dz_rs = s.pitch;
+        n.dweight = g + off[5];
+        const Tensor norm_ws = device_empty({(int64_t)std::max<size_t>(api.norm_workspace(&n), 1)}, at::kByte, u);
+        n.workspace = norm_ws.mutable_data_ptr();
+        n.workspace_bytes = norm_ws.numel();
+
         const Tensor dxbc = device_empty({s.rows, s.conv}, u.scalar_type(), u);
-        {
-            bimamba2_params p = layer_scan_params(s, o, zx, xbc, w, stream);
-            const Kept k(p, o.copies, o.cb);
-            k.point(p, kept.mutable_data_ptr<float>());
-            p.fwd_saved = k.saved();
-            p.dout = dy.const_data_ptr();
-            p.dout_sb = s.seqlen * s.inner; p.dout_sl = s.inner; p.dout_sh = o.headdim;
-            p.dx = at_byte(dxbc, 0);
-            p.dB = at_byte(dxbc, s.inner);
-            p.dC = at_byte(dxbc, s.inner + o.ngroups * o.dstate);
-            p.dx_sb = p.dB_sb = p.dC_sb = s.seqlen * s.conv;
-            p.dx_sl = p.dB_sl = p.dC_sl = s.conv;
-            p.ddt = at_byte(dzx, s.inner + s.conv);
-            p.ddt_sb = s.seqlen * s.pitch; p.ddt_sl = s.pitch;
-            p.dA = g + off[0]; p.dD = g + off[1]; p.ddt_bias = g + off[2];
-            const Tensor ws = attach_workspace(p, true, u);
-            check(api.bwd(&p), "bimamba2_bwd");
-        }
-        {
-            bimamba2_conv_params c = conv_params(s, zx, w, stream);
-            c.dout = dxbc.const_data_ptr();
-            c.dout_sb = s.seqlen * s.conv; c.dout_sl = s.conv;
-            c.dx = at_byte(dzx, s.inner);
-            c.dx_sb = s.seqlen * s.pitch; c.dx_sl = s.pitch;
-            c.dweight = g + off[3];
-            if (prm[4].defined()) c.dbias = g + off[4];
-            const Tensor ws = device_empty({(int64_t)std::max<size_t>(api.conv_workspace(&c), 1)}, at::kByte, u);
-            c.workspace = ws.mutable_data_ptr();
-            c.workspace_bytes = ws.numel();
-            check(api.conv_bwd(&c), "bimamba2_conv1d_silu_bwd");
-        }
-        // the small gradients into their parameters' types, one launch; dA_log = dA * A
+        bimamba2_params p = layer_scan_params(s, o, zx, xbc, w, stream);
+        const Kept k(p, o.copies, o.cb);
+        k.point(p, kept.mutable_data_ptr<float>());
+        p.fwd_saved = k.saved();
+        p.dout = dy.const_data_ptr();
+        p.dout_sb = s.seqlen * s.inner; p.dout_sl = s.inner; p.dout_sh = o.headdim;
+        p.dx = at_byte(dxbc, 0);
+        p.dB = at_byte(dxbc, s.inner);
+        p.dC = at_byte(dxbc, s.inner + o.ngroups * o.dstate);
+        p.dx_sb = p.dB_sb = p.dC_sb = s.seqlen * s.conv;
+        p.dx_sl = p.dB_sl = p.dC_sl = s.conv;
+        p.ddt = at_byte(dzx, s.inner + s.conv);
+        p.ddt_sb = s.seqlen * s.pitch; p.ddt_sl = s.pitch;
+        p.dA = g + off[0]; p.dD = g + off[1]; p.ddt_bias = g + off[2];
+        const Tensor scan_ws = attach_workspace(p, true, u);
+
+        bimamba2_conv_params cv = conv_params(s, zx, w, stream);
+        cv.dout = dxbc.const_data_ptr();
+        cv.dout_sb = s.seqlen * s.conv; cv.dout_sl = s.conv;
+        cv.dx = at_byte(dzx, s.inner);
+        cv.dx_sb = s.seqlen * s.pitch; cv.dx_sl = s.pitch;
+        cv.dweight = g + off[3];
+        if (prm[4].defined()) cv.dbias = g + off[4];
+        const Tensor conv_ws = device_empty({(int64_t)std::max<size_t>(api.conv_workspace(&cv), 1)}, at::kByte, u);
+        cv.workspace = conv_ws.mutable_data_ptr();
+        cv.workspace_bytes = conv_ws.numel();
+        // the small gradients in their parameters' types; dA_log = dA * A
         std::array<Tensor, Params32::N> dprm;
         bimamba2_cast_params c{};
         c.stream = stream;
@@ -884,7 +875,7 @@ public:
             add_cast(c, part, dprm[i].mutable_data_ptr(), dtype_code(prm[i].scalar_type(), "parameter dtype"),
                      i == 0 ? BIMAMBA2_CAST_MUL : BIMAMBA2_CAST_COPY, i == 0 ? w.ptr[0] : nullptr);
         }
-        if (c.count) check(api.cast_many(&c), "bimamba2_cast_many");
+        check(api.norm_scan_conv_bwd(&n, &p, &cv, &c), "bimamba2_norm_scan_conv_bwd");
         if (needs(0)) {
             du = device_empty(u.sizes(), u.scalar_type(), u);
             product_nn(dzx, w_in, du.view({s.rows, u.size(2)}));

@@ -18,6 +18,7 @@
 
 #include "common.hpp"
 #include "launch.hpp"
+#include "sums_body.hpp"
 
 namespace bm2 {
 
@@ -308,35 +309,17 @@ size_t conv_workspace_bytes(const bimamba2_conv_params *p) {
     return (size_t)p->batch * conv_ntl(p, true) * p->channels * (p->width + 1) * sizeof(float);
 }
 
-// dweight[c][k], dbias[c] = sums over the tiles of part[tile][c][W + 1]: 16 columns x 16 slices of the tiles per workgroup, the
-// slices added in a fixed order
+// dweight[c][k], dbias[c] = sums over the tiles of part[tile][c][W + 1]
 __global__ __launch_bounds__(NTHREADS) void conv_sums_kernel(const float *part, float *dweight, float *dbias, int ntiles, int channels, int W) {
-    __shared__ float red[16][17];
-    const int jl = threadIdx.x & 15, sl = threadIdx.x >> 4, j = blockIdx.x * 16 + jl, nj = channels * (W + 1);
-    float s = 0.f;
-    if (j < nj) {
-        int i = sl;
-        for (; i + 48 < ntiles; i += 64) {
-            const float a = part[(int64_t)i * nj + j], b = part[(int64_t)(i + 16) * nj + j], c = part[(int64_t)(i + 32) * nj + j],
-                        d = part[(int64_t)(i + 48) * nj + j];
-            s += (a + b) + (c + d);
-        }
-        for (; i < ntiles; i += 16) s += part[(int64_t)i * nj + j];
-    }
-    red[sl][jl] = s;
-    __syncthreads();
-    if (sl == 0 && j < nj) {
-        float t = 0.f;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) t += red[q][jl];
+    column_sums_body(part, ntiles, channels * (W + 1), blockIdx.x, [&](int j, float t) {
         const int c = j / (W + 1), k = j - c * (W + 1);
         if (k < W) dweight[(int64_t)c * W + k] = t;
         else if (dbias) dbias[c] = t;
-    }
+    });
 }
 
 template <typename T, int W, int VS>
-static int launch_conv_w(const bimamba2_conv_params *p, bool bwd) {
+static int launch_conv_w(const bimamba2_conv_params *p, bool bwd, LayerSums *leave) {
     const int ntl = conv_ntl(p, bwd), tl = conv_tile_len(p, bwd);
     const int64_t threads = (int64_t)p->batch * ntl * (p->channels / VS);
     const int64_t blocks = (threads + NTHREADS - 1) / NTHREADS;
@@ -364,20 +347,24 @@ static int launch_conv_w(const bimamba2_conv_params *p, bool bwd) {
                        *p, ntl, tl, nwc, part);
     int rc = check_launch();
     if (rc) return rc;
+    if (leave) {
+        leave->cols[leave->ncols++] = ColumnSums{part, p->dweight, p->has_bias ? p->dbias : nullptr, (int)ntiles, nj, W};
+        return BIMAMBA2_OK;
+    }
     hipLaunchKernelGGL(conv_sums_kernel, dim3((nj + 15) / 16), dim3(NTHREADS), 0, s, part, p->dweight, p->has_bias ? p->dbias : nullptr,
                        (int)ntiles, p->channels, W);
     return check_launch();
 }
 
 template <typename T, int VS>
-static int launch_conv_vs(const bimamba2_conv_params *p, bool bwd) {
+static int launch_conv_vs(const bimamba2_conv_params *p, bool bwd, LayerSums *leave) {
     auto al = [](const void *q, size_t a) { return (reinterpret_cast<uintptr_t>(q) % a) == 0; };
     const size_t va = sizeof(T) * VS;
     bool vec = p->channels % VS == 0 && al(p->x, va) && p->x_sb % VS == 0 && p->x_sl % VS == 0;
     if (bwd) vec = vec && al(p->dout, va) && p->dout_sb % VS == 0 && p->dout_sl % VS == 0 && al(p->dx, va) && p->dx_sb % VS == 0 && p->dx_sl % VS == 0;
     else vec = vec && al(p->out, va);
 #define BM2_CONV(WV)                                                      \
-    case WV: return vec ? launch_conv_w<T, WV, VS>(p, bwd) : launch_conv_w<T, WV, 1>(p, bwd)
+    case WV: return vec ? launch_conv_w<T, WV, VS>(p, bwd, leave) : launch_conv_w<T, WV, 1>(p, bwd, leave)
     switch (p->width) {
         BM2_CONV(1);
         BM2_CONV(3);
@@ -392,8 +379,8 @@ static int launch_conv_vs(const bimamba2_conv_params *p, bool bwd) {
 // two channels per thread when the rows allow it (else one): measured faster than four or eight - the backward pass has
 // three register windows plus the filter-gradient sums per channel, and more, narrower threads hide the load latency better
 template <typename T>
-static int launch_conv_t(const bimamba2_conv_params *p, bool bwd) {
-    return launch_conv_vs<T, 2>(p, bwd);
+static int launch_conv_t(const bimamba2_conv_params *p, bool bwd, LayerSums *leave) {
+    return launch_conv_vs<T, 2>(p, bwd, leave);
 }
 
 // ---- several small element-wise conversions in one launch (bimamba2_cast_many) -------------------------------------
@@ -437,11 +424,11 @@ int launch_cast_many(const bimamba2_cast_params *p) {
     return check_launch();
 }
 
-int launch_conv1d_silu(const bimamba2_conv_params *p, bool bwd) {
+int launch_conv1d_silu(const bimamba2_conv_params *p, bool bwd, LayerSums *leave) {
     switch (p->dtype) {
-        case BIMAMBA2_F32: return launch_conv_t<float>(p, bwd);
-        case BIMAMBA2_BF16: return launch_conv_t<bf16_t>(p, bwd);
-        case BIMAMBA2_F16: return launch_conv_t<f16_t>(p, bwd);
+        case BIMAMBA2_F32: return launch_conv_t<float>(p, bwd, leave);
+        case BIMAMBA2_BF16: return launch_conv_t<bf16_t>(p, bwd, leave);
+        case BIMAMBA2_F16: return launch_conv_t<f16_t>(p, bwd, leave);
         default: return BIMAMBA2_EUNSUPPORTED;
     }
 }

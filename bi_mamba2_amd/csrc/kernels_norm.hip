@@ -14,6 +14,7 @@
 // reduction adds them up (no atomics).
 #include "common.hpp"
 #include "launch.hpp"
+#include "sums_body.hpp"
 
 namespace bm2 {
 
@@ -488,31 +489,20 @@ size_t norm_workspace_bytes(const bimamba2_norm_params *p) {
     return (size_t)norm_partial_rows(p) * p->cols * sizeof(float) * (p->has_bias ? 2 : 1);
 }
 
-// out[j] = sum_i in[i * nj + j] for many columns j: 16 columns x 16 row slices per workgroup, the slices added in a fixed
-// order; blockIdx.y selects one of up to two (in, out) pairs
+// out[j] = sum_i in[i * nj + j] for many columns j; blockIdx.y selects one of up to two (in, out) pairs
 __global__ __launch_bounds__(NTHREADS) void colsum_kernel(const float *in0, float *out0, const float *in1, float *out1, int ni, int nj) {
-    __shared__ float red[16][17];
-    const float *in = blockIdx.y ? in1 : in0;
     float *out = blockIdx.y ? out1 : out0;
-    const int jl = threadIdx.x & 15, sl = threadIdx.x >> 4, j = blockIdx.x * 16 + jl;
-    float s = 0.f;
-    if (j < nj) {
-        int i = sl;
-        for (; i + 48 < ni; i += 64) {
-            const float a = in[(int64_t)i * nj + j], b = in[(int64_t)(i + 16) * nj + j], c = in[(int64_t)(i + 32) * nj + j],
-                        d = in[(int64_t)(i + 48) * nj + j];
-            s += (a + b) + (c + d);
-        }
-        for (; i < ni; i += 16) s += in[(int64_t)i * nj + j];
+    column_sums_body(blockIdx.y ? in1 : in0, ni, nj, blockIdx.x, [&](int j, float t) { out[j] = t; });
+}
+static int launch_norm_sums(const bimamba2_norm_params *p, float *part_w, float *part_b, int npr, LayerSums *leave) {
+    if (leave) {
+        leave->cols[leave->ncols++] = ColumnSums{part_w, p->dweight, nullptr, npr, p->cols, 0};
+        if (p->has_bias) leave->cols[leave->ncols++] = ColumnSums{part_b, p->dbias, nullptr, npr, p->cols, 0};
+        return BIMAMBA2_OK;
     }
-    red[sl][jl] = s;
-    __syncthreads();
-    if (sl == 0 && j < nj) {
-        float t = 0.f;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) t += red[q][jl];
-        out[j] = t;
-    }
+    hipLaunchKernelGGL(colsum_kernel, dim3((p->cols + 15) / 16, p->has_bias ? 2 : 1), dim3(NTHREADS), 0, stream_of(p), part_w, p->dweight,
+                       part_b, p->dbias, npr, p->cols);
+    return check_launch();
 }
 
 static bool norm_vec_ok(const bimamba2_norm_params *p, bool bwd, int elem) {
@@ -524,7 +514,7 @@ static bool norm_vec_ok(const bimamba2_norm_params *p, bool bwd, int elem) {
 }
 
 template <typename T, int NCH>
-static int launch_norm_nch(const bimamba2_norm_params *p, bool bwd) {
+static int launch_norm_nch(const bimamba2_norm_params *p, bool bwd, LayerSums *leave) {
     const bool vec = norm_vec_ok(p, bwd, (int)sizeof(T));
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     const bool wvec = p->group_size % 4 == 0 && al(p->weight) && (!p->has_bias || al(p->bias));
@@ -551,14 +541,12 @@ static int launch_norm_nch(const bimamba2_norm_params *p, bool bwd) {
     }
     int rc = check_launch();
     if (rc) return rc;
-    hipLaunchKernelGGL(colsum_kernel, dim3((p->cols + 15) / 16, p->has_bias ? 2 : 1), dim3(NTHREADS), 0, stream_of(p), part_w, p->dweight,
-                       part_b, p->dbias, npr, p->cols);
-    return check_launch();
+    return launch_norm_sums(p, part_w, part_b, npr, leave);
 }
 
 // groups of more than 8192 columns: NCH chunks of 512 per wave, four waves per (row, group)
 template <typename T, int NCH>
-static int launch_norm_wide(const bimamba2_norm_params *p, bool bwd) {
+static int launch_norm_wide(const bimamba2_norm_params *p, bool bwd, LayerSums *leave) {
     const bool vec = norm_vec_ok(p, bwd, (int)sizeof(T));
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     const bool wvec = p->group_size % 4 == 0 && al(p->weight) && (!p->has_bias || al(p->bias));
@@ -578,33 +566,31 @@ static int launch_norm_wide(const bimamba2_norm_params *p, bool bwd) {
     else hipLaunchKernelGGL((rmsnorm_gated_bwd_wide_kernel<T, NCH, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, vec, wvec, part_w, part_b);
     int rc = check_launch();
     if (rc) return rc;
-    hipLaunchKernelGGL(colsum_kernel, dim3((p->cols + 15) / 16, p->has_bias ? 2 : 1), dim3(NTHREADS), 0, stream_of(p), part_w, p->dweight,
-                       part_b, p->dbias, npr, p->cols);
-    return check_launch();
+    return launch_norm_sums(p, part_w, part_b, npr, leave);
 }
 
 template <typename T>
-static int launch_norm_t(const bimamba2_norm_params *p, bool bwd) {
+static int launch_norm_t(const bimamba2_norm_params *p, bool bwd, LayerSums *leave) {
     const int nch = (p->group_size + 511) / 512;
     if (nch > 16) {
-        if (nch <= 32) return launch_norm_wide<T, 8>(p, bwd);
-        if (nch <= 64) return launch_norm_wide<T, 16>(p, bwd);
+        if (nch <= 32) return launch_norm_wide<T, 8>(p, bwd, leave);
+        if (nch <= 64) return launch_norm_wide<T, 16>(p, bwd, leave);
         return BIMAMBA2_EUNSUPPORTED;
     }
-    if (nch <= 1) return launch_norm_nch<T, 1>(p, bwd);
-    if (nch <= 2) return launch_norm_nch<T, 2>(p, bwd);
-    if (nch == 3) return launch_norm_nch<T, 3>(p, bwd);    // 1536 columns: expand 2 x d_model 768, the benchmark layer's width
-    if (nch <= 4) return launch_norm_nch<T, 4>(p, bwd);
-    if (nch <= 8) return launch_norm_nch<T, 8>(p, bwd);
-    if (nch <= 16) return launch_norm_nch<T, 16>(p, bwd);
+    if (nch <= 1) return launch_norm_nch<T, 1>(p, bwd, leave);
+    if (nch <= 2) return launch_norm_nch<T, 2>(p, bwd, leave);
+    if (nch == 3) return launch_norm_nch<T, 3>(p, bwd, leave);    // 1536 columns: expand 2 x d_model 768, the benchmark layer's width
+    if (nch <= 4) return launch_norm_nch<T, 4>(p, bwd, leave);
+    if (nch <= 8) return launch_norm_nch<T, 8>(p, bwd, leave);
+    if (nch <= 16) return launch_norm_nch<T, 16>(p, bwd, leave);
     return BIMAMBA2_EUNSUPPORTED;
 }
 
-int launch_rmsnorm_gated(const bimamba2_norm_params *p, bool bwd) {
+int launch_rmsnorm_gated(const bimamba2_norm_params *p, bool bwd, LayerSums *leave) {
     switch (p->dtype) {
-        case BIMAMBA2_F32: return launch_norm_t<float>(p, bwd);
-        case BIMAMBA2_BF16: return launch_norm_t<bf16_t>(p, bwd);
-        case BIMAMBA2_F16: return launch_norm_t<f16_t>(p, bwd);
+        case BIMAMBA2_F32: return launch_norm_t<float>(p, bwd, leave);
+        case BIMAMBA2_BF16: return launch_norm_t<bf16_t>(p, bwd, leave);
+        case BIMAMBA2_F16: return launch_norm_t<f16_t>(p, bwd, leave);
         default: return BIMAMBA2_EUNSUPPORTED;
     }
 }

@@ -63,6 +63,13 @@ int launch_bmm_chunk_bwd(const bimamba2_params *p);
 struct ReduceJob { const float *in; float *out; int ni, nj, nk; };
 struct ReduceJobs { ReduceJob job[4]; int n = 0; };
 int launch_reduce_jobs(const ReduceJobs &jobs, hipStream_t stream);
+// out[j] = sum_i in[i*nj + j]; width > 0: columns are rows of width + 1, whose last goes to extra (NULL: nowhere) and the others to out
+struct ColumnSums { const float *in; float *out, *extra; int ni, nj, width; };
+// the final sums that several backward stages leave to one launch
+struct LayerSums { ReduceJobs jobs; ColumnSums cols[3]; int ncols = 0; };
+// casts: which of the sums leave in another type or multiplied (the item's source is the float32 place, which is not written then);
+// BIMAMBA2_EINVAL where an item is none of the sums
+int launch_layer_sums(const LayerSums &sums, const bimamba2_cast_params *casts, hipStream_t stream);
 // defer != NULL: the final reductions of dA and ddt_bias are appended to *defer instead of being launched
 int launch_chunk_cumsum_bwd(const bimamba2_params *p, ReduceJobs *defer = nullptr);
 // bmm_chunk_bwd and chunk_cumsum_bwd as one launch, where bwd_tail_merged() says it exists
@@ -97,11 +104,11 @@ int launch_fill(float *ptr, size_t n, float value, hipStream_t stream);
 int launch_reduce(const float *in, float *out, int ni, int nj, int nk, hipStream_t stream);
 
 // gated RMSNorm (kernels_norm.hip)
-int launch_rmsnorm_gated(const bimamba2_norm_params *p, bool bwd);
+int launch_rmsnorm_gated(const bimamba2_norm_params *p, bool bwd, LayerSums *leave = nullptr);   // leave: the sums are appended instead of launched
 size_t norm_workspace_bytes(const bimamba2_norm_params *p);
 
 // depthwise conv1d + SiLU (kernels_conv.hip)
-int launch_conv1d_silu(const bimamba2_conv_params *p, bool bwd);
+int launch_conv1d_silu(const bimamba2_conv_params *p, bool bwd, LayerSums *leave = nullptr);
 size_t conv_workspace_bytes(const bimamba2_conv_params *p);
 // several small element-wise conversions in one launch (kernels_conv.hip)
 int launch_cast_many(const bimamba2_cast_params *p);

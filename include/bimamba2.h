@@ -398,6 +398,14 @@ typedef struct bimamba2_cast_params {
 size_t bimamba2_cast_params_size(void);
 int bimamba2_cast_many(const bimamba2_cast_params *p);
 
+/* bimamba2_rmsnorm_gated_bwd, bimamba2_bwd and bimamba2_conv1d_silu_bwd one after the other on one stream, with the sums that end
+ * each of them (the gradients of the norm's weight, of A, D and dt_bias, of the convolution's filter and bias) in one launch
+ * behind all three.  casts: those of them that leave in another type or times a vector (BIMAMBA2_CAST_COPY, BIMAMBA2_CAST_MUL):
+ * an item's src is the float32 place given to the stage, which stays unwritten then.  The three workspaces are in use at the
+ * same time.  At least one row. */
+int bimamba2_norm_scan_conv_bwd(const bimamba2_norm_params *norm, const bimamba2_params *scan, const bimamba2_conv_params *conv,
+                                const bimamba2_cast_params *casts);
+
 /* ---------------------------------------------------------------------------------------------------------
  * Matrix product for the layer's projections, 16-bit operands, float32 accumulation:
  *   c[m, n] = sum_k A(m, k) B(n, k) (+ bias[n])

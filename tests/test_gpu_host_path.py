@@ -49,6 +49,34 @@ def test_layer_equals_its_composition(case, monkeypatch):
         assert_close(a, b.double(), dtype, name, scaled=True)
 
 
+@pytest.mark.parametrize("batch,seqlen,kw,dtype,frozen", [
+    (1, 1, dict(d_model=64, d_state=16, headdim=32), torch.float32, ()),                             # one row of partial sums; only A_log converted
+    (2, 70, dict(d_model=64, d_state=16, headdim=16, conv_bias=False), torch.bfloat16, ()),
+    (3, 301, dict(d_model=192, d_state=64, headdim=64), torch.float16, ("D", "conv1d.bias", "norm.weight")),
+    (2, 1030, dict(d_model=128, d_state=64, headdim=64, d_conv=3), torch.bfloat16, ("A_log",)),      # more partial sums than one round of loads
+])
+def test_layer_sums_in_one_launch(batch, seqlen, kw, dtype, frozen, monkeypatch):
+    """the sums that end the stages of a layer's backward pass and their conversions in one launch against a launch each: the same
+    order of additions, one rounding to the parameter's type, the same bits.  A_log and the norm's weight stay float32."""
+    from bi_mamba2_amd.modules import BiMamba2, _GradPieces
+    torch.manual_seed(0)
+    m = BiMamba2(**kw).cuda().to(dtype)
+    m.A_log.data = m.A_log.data.float()
+    m.norm.weight.data = m.norm.weight.data.float()
+    small = {n: p for n, p in m.named_parameters() if n.split(".")[0] in ("A_log", "D", "dt_bias", "conv1d", "norm")}
+    for n, p in small.items():
+        p.requires_grad_(n not in frozen)
+    live = [p for p in small.values() if p.requires_grad]
+    u = torch.randn(batch, seqlen, kw["d_model"], device="cuda").to(dtype).requires_grad_(True)
+    dy = torch.randn_like(u)
+    step = lambda: torch.autograd.grad(m(u), live, dy)
+    assert m._native_tensors(u) is not None
+    native = step()
+    monkeypatch.setattr(_GradPieces, "on_copied", staticmethod(lambda copied: None))
+    for a, b in zip(native, step()):
+        assert a.dtype == b.dtype and torch.equal(a, b)
+
+
 def test_layer_with_hooks_or_autocast_is_composed():
     from bi_mamba2_amd.modules import BiMamba2
     m = BiMamba2(d_model=64, d_state=16, headdim=16, chunk_size=64).cuda()
