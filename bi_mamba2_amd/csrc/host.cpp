@@ -828,7 +828,7 @@ public:
         n.dx = dy.mutable_data_ptr(); n.dx_rs = s.inner;
         n.dz = at_byte(dzx, 0); n.dz_rs = s.pitch;
         n.dweight = g + off[5];
-        const Tensor norm_ws = device_empty({(int64_t)std::max<size_t>(api.norm_workspace(&n), 1)}, at::kByte, u);
+        Tensor norm_ws = device_empty({(int64_t)std::max<size_t>(api.norm_workspace(&n), 1)}, at::kByte, u);
         n.workspace = norm_ws.mutable_data_ptr();
         n.workspace_bytes = norm_ws.numel();
 
@@ -847,7 +847,7 @@ public:
         p.ddt = at_byte(dzx, s.inner + s.conv);
         p.ddt_sb = s.seqlen * s.pitch; p.ddt_sl = s.pitch;
         p.dA = g + off[0]; p.dD = g + off[1]; p.ddt_bias = g + off[2];
-        const Tensor scan_ws = attach_workspace(p, true, u);
+        Tensor scan_ws = attach_workspace(p, true, u);
 
         bimamba2_conv_params cv = conv_params(s, zx, w, stream);
         cv.dout = dxbc.const_data_ptr();
@@ -856,7 +856,7 @@ public:
         cv.dx_sb = s.seqlen * s.pitch; cv.dx_sl = s.pitch;
         cv.dweight = g + off[3];
         if (prm[4].defined()) cv.dbias = g + off[4];
-        const Tensor conv_ws = device_empty({(int64_t)std::max<size_t>(api.conv_workspace(&cv), 1)}, at::kByte, u);
+        Tensor conv_ws = device_empty({(int64_t)std::max<size_t>(api.conv_workspace(&cv), 1)}, at::kByte, u);
         cv.workspace = conv_ws.mutable_data_ptr();
         cv.workspace_bytes = conv_ws.numel();
         // the small gradients in their parameters' types; dA_log = dA * A
@@ -876,6 +876,7 @@ public:
                      i == 0 ? BIMAMBA2_CAST_MUL : BIMAMBA2_CAST_COPY, i == 0 ? w.ptr[0] : nullptr);
         }
         check(api.norm_scan_conv_bwd(&n, &p, &cv, &c), "bimamba2_norm_scan_conv_bwd");
+        norm_ws = scan_ws = conv_ws = Tensor();           // (what follows may have their memory)
         if (needs(0)) {
             du = device_empty(u.sizes(), u.scalar_type(), u);
             product_nn(dzx, w_in, du.view({s.rows, u.size(2)}));

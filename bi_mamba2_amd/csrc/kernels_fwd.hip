@@ -88,7 +88,9 @@ __global__ __launch_bounds__(NTHREADS) void fwd_front_kernel(const bimamba2_para
 // ---------------------------------------------------------------------------------------------------------
 // CUMSUM (states only): the workgroup also does the work of chunk_cumsum_fwd_kernel for its (b, c, h) - wave 0 transforms
 // dt and scans it while the tiles are under way - and the first tile's workgroup writes dt_out, cs_f, cs_b for the later
-// kernels: one launch less in front of the forward pass.
+// kernels: one launch less in front of the forward pass.  Packed sequences too, which took
+// the stand-alone kernel before: 1 x 8192, 24 heads of 64, dstate 64, bfloat16 67.5 -> 65 us a forward pass, 219 -> 214 in training;
+// 2 x 1000, 8 heads of 128 38 -> 35.
 // UNI: forward direction only (single-direction comparator).
 // OUT16 (chunk states of the forward pass only): the per-chunk states leave in the inputs' 16-bit type, into states16_f/b
 // (where the inter-chunk scan turns them into the entering states in place) - half the bytes of the float32 tensors; the
@@ -159,6 +161,7 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bima
     // make an access it knows of wait for all outstanding requests).
     float r_cf = 0.f, r_cb = 0.f, r_dt = 0.f, e_f = 0.f, e_b = 0.f, A_h = 0.f, bias_h = 0.f;
     unsigned dt_raw[4] = {0u, 0u, 0u, 0u};                   // DO_CUMSUM, wave 0: bits of dt at this lane's four positions
+    float sid[6] = {};                                       // ... and of seq_idx there, at the position before and the one behind
     if constexpr (DO_CUMSUM) {
         if (wave == 0) {
             const int64_t dto = b * p.dt_sb + (int64_t)c * Q * p.dt_sl + h * p.dt_sh;
@@ -171,6 +174,11 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bima
             } else {
 #pragma unroll
                 for (int e = 0; e < 4; ++e) dt_raw[e] = raw_global_load_u16(reinterpret_cast<const uint16_t *>(p.dt) + at[e]);
+            }
+            if (p.seq_idx) {
+                const float *si = reinterpret_cast<const float *>(p.seq_idx + (int64_t)b * p.seqlen);
+#pragma unroll
+                for (int e = 0; e < 6; ++e) sid[e] = raw_global_load_f32(si + min(max(c * Q + lane * 4 + e - 1, 0), p.seqlen - 1));
             }
             A_h = raw_global_load_f32(p.A + h);
             bias_h = raw_global_load_f32(p.has_dt_bias ? p.dt_bias + h : p.A + h);
@@ -220,7 +228,9 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bima
             for (int e = 0; e < 4; ++e) raw_lds_use(dt_raw[e]);
             const float A = A_h;
             const float bias = p.has_dt_bias ? bias_h : 0.f;
-            float a[4];
+            float a[4], ar[4];                               // (differ with seq_idx only, see chunk_cumsum_wave)
+#pragma unroll
+            for (int e = 0; e < 6; ++e) raw_lds_use(sid[e]);
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const int q = lane * 4 + e;
@@ -232,13 +242,17 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bima
                 d = fminf(fmaxf(d, p.dt_min), p.dt_max);
                 if (q >= limit) d = 0.f;
                 keep_dt[e] = d;
-                a[e] = d * A;
+                a[e] = ar[e] = d * A;
+                if (p.seq_idx && q < limit) {
+                    if (__float_as_uint(sid[e]) != __float_as_uint(sid[e + 1])) a[e] += BIMAMBA2_SEQ_CUT;
+                    if (__float_as_uint(sid[e + 2]) != __float_as_uint(sid[e + 1])) ar[e] += BIMAMBA2_SEQ_CUT;
+                }
             }
             float pf[4], sb[4];
             pf[0] = a[0]; pf[1] = pf[0] + a[1]; pf[2] = pf[1] + a[2]; pf[3] = pf[2] + a[3];
-            sb[3] = a[3]; sb[2] = sb[3] + a[2]; sb[1] = sb[2] + a[1]; sb[0] = sb[1] + a[0];
-            const float tot = pf[3];
-            const float before = wave_incl_prefix(tot, lane) - tot, after = wave_incl_suffix(tot, lane) - tot;
+            sb[3] = ar[3]; sb[2] = sb[3] + ar[2]; sb[1] = sb[2] + ar[1]; sb[0] = sb[1] + ar[0];
+            const float tot = pf[3], tot_r = sb[0];
+            const float before = wave_incl_prefix(tot, lane) - tot, after = wave_incl_suffix(tot_r, lane) - tot_r;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 keep_f[e] = before + pf[e];
@@ -1021,7 +1035,6 @@ int launch_fwd_front(const bimamba2_params *p) {
 bool chunk_state_does_cumsum(const bimamba2_params *p) {
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     auto mult = [](int64_t a, int64_t b, int64_t c) { return a % 8 == 0 && b % 8 == 0 && c % 8 == 0; };
-    if (p->seq_idx) return false;                 // packed sequences: the stand-alone cumsum kernel applies the cuts
     // (the kernel that walks through several heads per workgroup reads the cumulative sums: the stand-alone launch comes first)
     if (!p->states_f && p->states16_f && p->states16_b && chunk_state_uses_heads_kernel(p)) return false;
     return p->dtype != BIMAMBA2_F32 && p->headdim % 64 == 0 && p->dstate % 64 == 0 && p->chunk_size % 32 == 0 && al(p->Bm) &&

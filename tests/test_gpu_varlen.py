@@ -64,6 +64,29 @@ def test_packed_sequences_forward_and_backward(ops, case):
             assert_close(leaves[k].grad, r[k].grad, dtype, "d" + k, scaled=is_reduced("d" + k, dtype))
 
 
+@pytest.mark.parametrize("L,P,N,Q,dtype,dt_dtype,bounds", [
+    (1, 64, 64, 64, torch.bfloat16, torch.float32, ()),
+    (300, 64, 64, 256, torch.bfloat16, torch.bfloat16, (1, 3, 4, 255, 256, 299)),          # both sides of a lane's four positions, of a chunk and of the row's end
+    (257, 128, 128, 128, torch.float16, torch.float32, (127, 128, 129, 252)),
+    (200, 64, 128, 96, torch.bfloat16, torch.float16, tuple(range(5, 200, 5))),            # a chunk that is no power of two
+])
+def test_cuts_beside_the_chunk_states(ops, L, P, N, Q, dtype, dt_dtype, bounds):
+    """the sums that the chunk-state launch forms with the cuts of packed sequences against float64"""
+    H, nc = 4, -(-L // Q)
+    d = to_dev(make_case(2, L, H, P, 2, N, dtype))
+    si = _seq_idx(2, L, [bounds, ()]).cuda()
+    dt = d["dt"].to(dt_dtype)
+    res = ops._mamba_chunk_scan_combined_fwd(d["x"], dt, d["A"], d["B"], d["C"], Q, D=d["D"], dt_bias=d["dt_bias"], dt_softplus=True, seq_idx=si)
+    # (2, H, nc, Q), zeros behind the sequence; -20 at a sequence's first position and, for the reverse sums, its last
+    assert torch.allclose(res[2], ops._chunk_cumsum_fwd(dt, d["A"], Q, dt_bias=d["dt_bias"], dt_softplus=True)[2], rtol=2.0 ** -22, atol=0)
+    change = -20.0 * (si[:, 1:] != si[:, :-1]).double()
+    cut = lambda front, back: torch.nn.functional.pad(change, (front, back + nc * Q - L)).view(2, 1, nc, Q)
+    a = res[2].double() * d["A"].double()[:, None, None]
+    for got, want in ((res[3], (a + cut(1, 0)).cumsum(-1)), (res[4], (a + cut(0, 1)).flip(-1).cumsum(-1).flip(-1))):
+        # (each of up to 256 float32 additions rounds, at the size of the largest sum)
+        assert float((got - want).abs().max()) <= 256 * 2.0 ** -24 * float(want.abs().max())
+
+
 def test_packed_equals_one_by_one(ops):
     b, L, H, P, G, N, Q, dtype = 1, 768, 8, 64, 1, 64, 256, torch.bfloat16
     d = to_dev(make_case(b, L, H, P, G, N, dtype, with_z=True))
