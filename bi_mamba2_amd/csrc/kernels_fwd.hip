@@ -95,14 +95,16 @@ __global__ __launch_bounds__(NTHREADS) void fwd_front_kernel(const bimamba2_para
 // OUT16 (chunk states of the forward pass only): the per-chunk states leave in the inputs' 16-bit type, into states16_f/b
 // (where the inter-chunk scan turns them into the entering states in place) - half the bytes of the float32 tensors; the
 // tile passes through LDS so that it is written as 16-byte vectors, a whole 128-byte row piece per eight lanes.
-template <typename T, bool DSTATES, bool CUMSUM, bool UNI = false, bool OUT16 = false>
-__global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bimamba2_params p, int nc) {
+constexpr int DIRECT_RING = 4;                             // K steps (32 positions each): requests run DIRECT_RING - 1 steps ahead
+constexpr int DIRECT_LDS = 2 * DIRECT_RING * 32 * 64 * 2;
+// lds: DIRECT_LDS bytes; workgroup (nt, pt, bch) of the grid (dstate tiles gx, headdim tiles gy, (batch, chunk, head) gz)
+template <typename T, bool DSTATES, bool CUMSUM, bool UNI, bool OUT16>
+__device__ __forceinline__ void chunk_state_direct_body(const bimamba2_params &p, int nc, int nt, int pt, int bch, int gx, int gy, int gz, char *lds) {
     typedef Mma<T> M;
     typedef typename M::Frag Frag;
     static_assert(sizeof(T) == 2, "16-bit operands");
-    constexpr int KR = 4;                                  // ring of K steps (32 positions each): requests run KR - 1 steps ahead
-    __shared__ __attribute__((aligned(16))) T xt[KR * 32 * 64];
-    __shared__ __attribute__((aligned(16))) T bt[KR * 32 * 64];
+    constexpr int KR = DIRECT_RING;
+    T *xt = reinterpret_cast<T *>(lds), *bt = xt + KR * 32 * 64;
     __shared__ __attribute__((aligned(16))) float wf[BIMAMBA2_MAX_CHUNK], wb[BIMAMBA2_MAX_CHUNK];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 15, lg = lane >> 4;
@@ -114,22 +116,20 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bima
     // With large groups only the tiles of one (b, c, h) are kept together: the heads of a (b, c) spread over the dies,
     // a few per die, and the B rows are a small part of the traffic (all 32 heads of a one-group (b, c) on one die, asking
     // for the same B tile at the same time, made the launch slower: 16.3 -> 18.7 us).
-    int nt = blockIdx.x, pt = blockIdx.y, bch = blockIdx.z;
     {
-        const int tiles = gridDim.x * gridDim.y;
-        const int lin = blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z);
+        const int tiles = gx * gy, lin = nt + gx * (pt + gy * bch);
         if (p.nheads <= 8 * p.ngroups) {
             int inner, bc_;
-            xcd_order(lin, tiles * p.nheads, (int)gridDim.z / p.nheads, inner, bc_);
+            xcd_order(lin, tiles * p.nheads, gz / p.nheads, inner, bc_);
             const int tile = inner % tiles;
             bch = bc_ * p.nheads + inner / tiles;
-            nt = tile % (int)gridDim.x;
-            pt = tile / (int)gridDim.x;
+            nt = tile % gx;
+            pt = tile / gx;
         } else if (tiles > 1) {
             int tile;
-            xcd_order(lin, tiles, (int)gridDim.z, tile, bch);
-            nt = tile % (int)gridDim.x;
-            pt = tile / (int)gridDim.x;
+            xcd_order(lin, tiles, gz, tile, bch);
+            nt = tile % gx;
+            pt = tile / gx;
         }
     }
     const int h = bch % p.nheads, bc = bch / p.nheads, c = bc % nc, b = bc / nc;
@@ -389,6 +389,25 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bima
                 }
             }
         }
+    }
+}
+
+template <typename T, bool DSTATES, bool CUMSUM, bool UNI = false, bool OUT16 = false>
+__global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bimamba2_params p, int nc) {
+    __shared__ __attribute__((aligned(16))) char lds[DIRECT_LDS];
+    chunk_state_direct_body<T, DSTATES, CUMSUM, UNI, OUT16>(p, nc, blockIdx.x, blockIdx.y, blockIdx.z, gridDim.x, gridDim.y, gridDim.z, lds);
+}
+
+// The cumulative sums, the states and C.B^T in one launch, as fwd_front_kernel (the scan kernels of training at dstate 128 read
+// C.B^T): 2 x 3001, 24 heads of 64, dstate 128, bfloat16 21 + 14 -> 26 us, the training pass 306.6 -> 298; 4 x 1024, 32 heads in 4 groups 290 -> 261.
+template <typename T>
+__global__ __launch_bounds__(NTHREADS) void chunk_state_direct_cb_kernel(const bimamba2_params p, int nc, int nnt, int npt, int nstate, int nqt) {
+    __shared__ __attribute__((aligned(16))) char lds[DIRECT_LDS > BMM_FWD_LDS<T> ? DIRECT_LDS : BMM_FWD_LDS<T>];
+    const int id = blockIdx.x;
+    if (id < nstate) chunk_state_direct_body<T, false, true, false, false>(p, nc, id % nnt, id / nnt % npt, id / (nnt * npt), nnt, npt, nstate / (nnt * npt), lds);
+    else {
+        const int k = id - nstate;
+        bmm_chunk_fwd_body<T>(p, nc, k % nqt, k / nqt % nqt, k / (nqt * nqt), lds);
     }
 }
 
@@ -997,13 +1016,19 @@ static bool chunk_state_generic(const bimamba2_params *p, bool &fast) {
 // chunk cumsum, chunk states and C.B^T as one launch
 bool fwd_front_merged(const bimamba2_params *p) {
     bool fast;
-    return p->CB && p->states_f && p->states_b && chunk_state_generic(p, fast);
+    return p->CB && !p->causal && p->states_f && p->states_b && (chunk_state_generic(p, fast) || chunk_state_does_cumsum(p));
 }
 
 template <typename T> static int launch_fwd_front_t(const bimamba2_params *p, bool fast) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, nnt = (p->dstate + 63) / 64, npt = (p->headdim + 63) / 64;
     const int nstate = nnt * npt * p->batch * nc * p->nheads;
     const dim3 grid(nstate + nqt * nqt * p->batch * nc * p->ngroups);
+    if constexpr (sizeof(T) == 2) {
+        if (chunk_state_does_cumsum(p)) {
+            hipLaunchKernelGGL((chunk_state_direct_cb_kernel<T>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
+            return check_launch();
+        }
+    }
     if constexpr (sizeof(T) == 4) {
         if (fast) {
             hipLaunchKernelGGL((fwd_front_kernel<T, true, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);
@@ -1021,7 +1046,7 @@ template <typename T> static int launch_fwd_front_t(const bimamba2_params *p, bo
 
 int launch_fwd_front(const bimamba2_params *p) {
     bool fast;
-    if (!chunk_state_generic(p, fast)) return BIMAMBA2_EINVAL;          // (the caller checked fwd_front_merged())
+    if (!chunk_state_generic(p, fast) && !chunk_state_does_cumsum(p)) return BIMAMBA2_EINVAL;          // (the caller checked fwd_front_merged())
     switch (p->dtype) {
         case BIMAMBA2_F32: return launch_fwd_front_t<float>(p, fast);
         case BIMAMBA2_BF16: return launch_fwd_front_t<bf16_t>(p, fast);

@@ -183,6 +183,16 @@ def test_first_kernels_in_one_launch(b, L, H, P, G, N, Q, dtype, dt_dtype):
         assert torch.equal(got, want)
 
 
+@pytest.mark.parametrize("case", [
+    (1, 257, 4, 64, 2, 128, 256, torch.bfloat16, torch.float32),     # two tiles of states, sixteen of C.B^T, one of them past the end
+    (2, 33, 9, 128, 1, 128, 32, torch.float16, torch.float16),       # more than eight heads a group: the other order of tiles
+    (1, 200, 2, 64, 1, 192, 96, torch.bfloat16, torch.bfloat16),     # a chunk that is no whole tile of C.B^T
+])
+def test_first_kernels_of_wide_heads_in_one_launch(case):
+    """the same for the states by direct loads"""
+    test_first_kernels_in_one_launch(*case)
+
+
 @pytest.mark.parametrize("P,N", [(8, 8), (16, 72), (24, 16), (64, 40), (72, 64), (128, 136)])
 @pytest.mark.parametrize("L,Q,dtype", [(1, 32, torch.bfloat16), (95, 64, torch.float16), (129, 128, torch.bfloat16), (100, 50, torch.bfloat16)])
 def test_chunk_states_of_narrow_tiles(P, N, L, Q, dtype):
