@@ -399,7 +399,8 @@ __global__ __launch_bounds__(NTHREADS) void chunk_state_direct_kernel(const bima
 }
 
 // The cumulative sums, the states and C.B^T in one launch, as fwd_front_kernel (the scan kernels of training at dstate 128 read
-// C.B^T): 2 x 3001, 24 heads of 64, dstate 128, bfloat16 21 + 14 -> 26 us, the training pass 306.6 -> 298; 4 x 1024, 32 heads in 4 groups 290 -> 261.
+// C.B^T): 2 x 3001, 24 heads of 64, dstate 128, bfloat16 21 + 14 -> 26 us, the training pass 302 -> 293;
+// 1 x 2000, 16 heads in 2 groups, float16 151 -> 143; 4 x 1024, 32 heads in 4 groups 263 -> 258; 1 x 1024, 8 heads: host time.
 template <typename T>
 __global__ __launch_bounds__(NTHREADS) void chunk_state_direct_cb_kernel(const bimamba2_params p, int nc, int nnt, int npt, int nstate, int nqt) {
     __shared__ __attribute__((aligned(16))) char lds[DIRECT_LDS > BMM_FWD_LDS<T> ? DIRECT_LDS : BMM_FWD_LDS<T>];
