@@ -514,4 +514,29 @@ __device__ __forceinline__ void xcd_order(int lin, int ninner, int nouter, int &
     }
 }
 
+// A float32 operand of a 16-bit product as two 16-bit ones, the value rounded and what the rounding left: it enters with 16 (22)
+// bits instead of 8 (11).  For kernels that wait for memory or for each other, where a second product costs little.
+// The remainder is that of the very number in `hi`: the value is made opaque first, because a product that is converted right away
+// may be rounded once (multiply and convert in one instruction) where it goes into `hi` and twice where it is subtracted from;
+// one operand in some ten thousand was then off by a unit of the 16-bit type.
+template <typename T> __device__ __forceinline__ void split_operand(const float (&v)[Mma<T>::KPL], typename Mma<T>::Frag &hi, typename Mma<T>::Frag &rest) {
+    float e[Mma<T>::KPL];
+#pragma unroll
+    for (int i = 0; i < Mma<T>::KPL; ++i) {
+        e[i] = v[i];
+        asm volatile("" : "+v"(e[i]));
+    }
+    hi = Mma<T>::pack(e);
+    if constexpr (sizeof(T) == 2) {
+        float r[Mma<T>::KPL];
+#pragma unroll
+        for (int i = 0; i < Mma<T>::KPL; ++i) {
+            const T part = hi[i];
+            const float h = to_f(part);
+            r[i] = __builtin_isfinite(h) ? e[i] - h : 0.f;          // (what overflows the 16-bit type stays an infinity)
+        }
+        rest = Mma<T>::pack(r);
+    }
+}
+
 }  // namespace bm2

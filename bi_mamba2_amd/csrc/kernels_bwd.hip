@@ -1184,23 +1184,6 @@ int launch_bwd_dcb(const bimamba2_params *p, bool add_up) {
 // FAST (16-bit types, chunk_size == QP, dstate a multiple of 64, aligned operands, at most 8 slices): every global load
 // of a thread (its dCB row pieces, the slices it adds, the K operand) is requested before the first one is used.
 
-
-// A float32 operand of a 16-bit product as two 16-bit ones, the value rounded and what the rounding left: dCB in float32 enters
-// with 16 (22) bits instead of 8 (11).  The kernel waits for memory, the second product costs it nothing that can be measured,
-// and dB and dC are a fifth closer to the exact ones.
-template <typename T> __device__ __forceinline__ void split_operand(const float (&v)[Mma<T>::KPL], typename Mma<T>::Frag &hi, typename Mma<T>::Frag &rest) {
-    hi = Mma<T>::pack(v);
-    if constexpr (sizeof(T) == 2) {
-        float r[Mma<T>::KPL];
-#pragma unroll
-        for (int i = 0; i < Mma<T>::KPL; ++i) {
-            const float h = to_f(from_f<T>(v[i]));
-            r[i] = __builtin_isfinite(h) ? v[i] - h : 0.f;          // (what overflows the 16-bit type stays an infinity)
-        }
-        rest = Mma<T>::pack(r);
-    }
-}
-
 // SLIM (with FAST): dCB / dCBT hold 16-bit elements (in16) and there are at most two slices to add: a quarter of the
 // registers, and the staging tile of the result shares the LDS of the K operand, so that three workgroups fit a CU where
 // the general variant fits two (with few heads per group the launch has thousands of workgroups: 83 -> 76 us at 8 groups
