@@ -218,16 +218,20 @@ int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd) {
 // Where the lines lie, us a pass with chunks of 64 / 128 / 256 (z gate, D; forward alone and, second, with the backward pass; one
 // group unless said otherwise).  A chunk costs its pairs of positions (they grow with the chunk) and its states (which do not);
 // small calls want many workgroups, i.e. small chunks.
-//  * float32: pairs run at the float32 matrix rate.  4 x 2048, 16 heads of 64, dstate 64: 147 / 111 / 129, 526 / 412 / 488; heads of 16,
-//    dstate 16: 58 / 49 / 56, 240 / 211 / 252; 2 x 512, 8 heads of 64, dstate 64: 34 / 37 / 55, 141 / 143 / 185; 4 x 1024, 8 heads of 32:
-//    45 / 43 / 61.  Never above the caller's: the result is off by the resolution of sums over a chunk (1.6 times as much in
+//  * float32: pairs run at the float32 matrix rate.  4 x 2048, 16 heads of 64, dstate 64: 142 / 99 / 118, 478 / 384 / 477; heads of 16,
+//    dstate 16: 49 / 39 / 48, 192 / 168 / 250; 2 x 512, 8 heads of 64, dstate 64: 25 / 29 / 47, 120 / 120 / 180; 4 x 1024, 8 heads of 32:
+//    29 / 29 / 45.  Never above the caller's: the result is off by the resolution of sums over a chunk (1.6 times as much in
 //    chunks twice as long).
 //  * 16 bits, the kernels that rebuild C.B^T (dstate 64, headdim 64 or 128; forward also dstate 128): 4 x 2048, 16 heads of 64, dstate 64:
-//    61 / 44 / 39, 206 / 163 / 153; 4 x 1024, 8 heads: 31 / 25 / 29, 133 / 126 / 125; 2 x 512: 22 / 22 / 27; dstate 128, 4 x 2048: 86 / 65 / 63.
-//    Never below the caller's (their states are kept in 16 bits: a rounding per chunk).
-//  * other 16-bit shapes: 4 x 2048, 16 heads of 32, dstate 32: 66 / 52 / 53, 267 / 222 / 258; 8 groups, 4 x 4096: 126 / 101 / 119, 583 / 545 /
-//    719; 4 x 1024, 8 heads: 31 / 29 / 40, 139 / 129 / 167; 2 x 512: 27 / 28 / 38.  Training at dstate 128: 4 x 2048, 16 heads of 64: 433 / 278 /
-//    251; of 128: 894 / 496 / 408; 16 heads in 8 groups, 4 x 4096, of 64: 1093 / 783 / 877, of 128: 1903 / 1253 / 1218.
+//    63 / 44 / 40, 198 / 159 / 152; 4 x 1024, 8 heads: 30 / 25 / 28, 118 / 118 / 118 (host time); 2 x 512: 21 / 22 / 27; dstate 128, 4 x 2048:
+//    88 / 65 / 62.  Never below the caller's, where small calls would be faster: their result is 0.4 % (128) and 1.5 % (64) further from
+//    float64 in bfloat16 (1 x 197, 12 heads: 2.013e-3 / 2.023e-3 / 2.048e-3), most of it from the states in 16 bits.
+//  * other 16-bit shapes: 4 x 2048, 16 heads of 32, dstate 32: 53 / 41 / 45, 178 / 145 / 194; 8 groups, 4 x 4096: 185 / 149 / 178 and 659 / 580 /
+//    784 (32 heads); 4 x 1024, 8 heads: 21 / 20 / 34, 117 / 117 / 136; 2 x 512: 17 / 19 / 32.  Below the caller's chunk only where the
+//    chunk states take their weighted operand in two 16-bit parts: with one, dA was 5 to 32 % further from float64 in chunks of 128
+//    than of 256 (900 positions, 8 heads, 400 inputs); with two no output is (dA -0.3 to -7 %, out -0.4 to -0.8 %, dB and dC -18 to -28 %).
+//    Training at dstate 128 with heads of 64 or 128 and few of them a group stays as asked: 16 heads in 8 groups, 4 x 4096, of 64 1104 /
+//    784 / 880 would gain, with dA 5 % further off.
 int bimamba2_chunk_for(const bimamba2_params *p, int training) {
     if (check_problem(p)) return p ? p->chunk_size : 0;
     const int Q = p->chunk_size, P = p->headdim, N = p->dstate;
@@ -241,7 +245,11 @@ int bimamba2_chunk_for(const bimamba2_params *p, int training) {
     const bool whole = P == 64 || P == 128;
     if (whole && (N == 64 || (N == 128 && (!training || P == 128 || p->nheads >= 8 * p->ngroups))))
         return std::max(Q, workgroups(256, 64) >= CUS ? 256 : workgroups(128, 64) >= CUS / 2 ? 128 : Q);
-    return Q > 128 || workgroups(128, 64) >= CUS ? 128 : Q;
+    if (Q <= 128) return workgroups(128, 64) >= CUS ? 128 : Q;
+    bimamba2_params q = *p;
+    q.chunk_size = 128;
+    const bool exact_states = !(P % 64 == 0 && N % 64 == 0) && chunk_state_narrow(&q, false) && chunk_state_narrow(&q, true);
+    return exact_states ? 128 : Q;
 }
 
 int bimamba2_ddt_direct_planes(const bimamba2_params *p) {

@@ -197,6 +197,9 @@ __device__ __forceinline__ void chunk_state_body(const bimamba2_params &p, int n
 // the whole B tile of the chunk come by direct loads, all requested at once, and the operands are LDS transpose reads (no registers
 // to stage in, 143 of them above: four workgroups fit a CU instead of three, and each waits for memory once).  A row's units past
 // headdim or dstate are not requested: what lies there gives outputs that nobody stores.
+// The weighted operand enters in two 16-bit parts: the kernel waits for memory, and states that were off by its rounding made dA up to
+// 32 % less exact in chunks of 128 than in the ones of 256 that a caller asked for.  Time with two parts and one: 39.5 and 38.3 us a
+// forward pass over 4 x 2048, 16 heads of 16, dstate 16, two boxes; 134 and 133.5 in training.
 // 4 x 2048 in chunks of 128, bfloat16, 16 heads, headdim 16, dstate 16: the forward launch 24 -> 15 us, beside dCB 27 -> 22; headdim 128, dstate 32: 35 -> 27 and 26 -> 18.
 // ---------------------------------------------------------------------------------------------------------
 struct ChunkStateNarrowMap {
@@ -284,13 +287,15 @@ __device__ __forceinline__ void chunk_state_narrow_body(const bimamba2_params &p
                 vb[i + k] = to_f(x) * b4[k];
             }
         }
-        const Frag af = M::pack(vf), ab = M::pack(vb);
+        Frag af, ab, af_rest, ab_rest;
+        split_operand<T>(vf, af, af_rest);
+        split_operand<T>(vb, ab, ab_rest);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             if (nt * 64 + j * 16 >= N) continue;               // (uniform)
             const Frag bf = tile64_tr_frag<Frag>(bt, ks, j * 16, lr, lg);
-            accf[j] = M::mma(af, bf, accf[j]);
-            accb[j] = M::mma(ab, bf, accb[j]);
+            accf[j] = M::mma(af_rest, bf, M::mma(af, bf, accf[j]));
+            accb[j] = M::mma(ab_rest, bf, M::mma(ab, bf, accb[j]));
         }
     }
     float *of = (DSTATES ? p.dstates_f : p.states_f) + (int64_t)bch * P * N, *ob = (DSTATES ? p.dstates_b : p.states_b) + (int64_t)bch * P * N;

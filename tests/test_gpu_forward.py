@@ -205,14 +205,16 @@ def test_chunk_states_of_narrow_tiles(P, N, L, Q, dtype):
     nc = csf.shape[2]
     pad = lambda t: torch.nn.functional.pad(t.double(), (0, 0, 0, 0, 0, nc * Q - L)).view(b, nc, Q, *t.shape[2:])
     rows = lambda e: e.double().permute(0, 2, 3, 1)                                        # (b, nc, Q, H)
-    for got, x, mate, wf, wb in ((ops._chunk_state_fwd(d["B"], d["x"], dt, csf, csb), d["x"], d["B"], dt.double() * (csf[..., -1:] - csf).double().exp(), dt.double() * (csb[..., :1] - csb).double().exp()),
-                                 (ops._chunk_scan_bwd_dstates(d["C"], csf, csb, d["x"]), d["x"], d["C"], csf.double().exp(), csb.double().exp())):
-        for g, w in zip(got, (wf, wb)):
-            xs, ms = pad(x) * rows(w)[..., None], pad(mate).repeat_interleave(H // G, 3)
-            want, size = (torch.einsum("bcqhp,bcqhn->bchpn", f(xs), f(ms)) for f in (lambda t: t, torch.abs))
-            # One operand carries the weight and is rounded to the inputs' type: at most half a unit in its last place, 2^-8 (8 bits
-            # of significand) or 2^-11 (11 bits) of each product, or 2^-25, half of float16's smallest number, where it is subnormal.
-            # The weight and up to 128 sums in float32 add at most 2^-16 of the products' sizes.
-            u, tiny = {torch.bfloat16: (2.0 ** -8, 0.0), torch.float16: (2.0 ** -11, 2.0 ** -25)}[dtype]
-            bound = (u + 2.0 ** -16) * size + tiny * ms.abs().sum(2)[..., None, :] + 1e-30
+    ends = dict(x=(csf[..., -1:] - csf, csb[..., :1] - csb, dt), d=(csf, csb, torch.ones_like(dt)))      # exponents of the weights and their factor
+    for got, mate, (ef, eb, d0) in ((ops._chunk_state_fwd(d["B"], d["x"], dt, csf, csb), d["B"], ends["x"]), (ops._chunk_scan_bwd_dstates(d["C"], csf, csb, d["x"]), d["C"], ends["d"])):
+        for g, e in zip(got, (ef, eb)):
+            xs, ms = pad(d["x"]) * rows(d0.double() * e.double().exp())[..., None], pad(mate).repeat_interleave(H // G, 3)
+            want = torch.einsum("bcqhp,bcqhn->bchpn", xs, ms)
+            # One operand carries the weight and enters as two numbers of the inputs' type: each rounds by at most half a unit in its
+            # last place, 2^-8 (8 bits of significand) or 2^-11 (11 bits), the second of what the first left: 2^-16 or 2^-22 of
+            # each product, or 2^-25, half of float16's smallest number, where that is subnormal.  The weight is off by the
+            # rounding of its exponent's multiple (2^-23 of it) and a few roundings of its own, 256 sums in float32 by 2^-16.
+            u, tiny = {torch.bfloat16: (2.0 ** -16, 0.0), torch.float16: (2.0 ** -22, 2.0 ** -25)}[dtype]
+            off = u + 2.0 ** -16 + (rows(e).abs()[..., None] + 4) * 2.0 ** -23
+            bound = torch.einsum("bcqhp,bcqhn->bchpn", xs.abs() * off, ms.abs()) + tiny * ms.abs().sum(2)[..., None, :] + 1e-30
             assert float(((g - want).abs() / bound).max()) <= 1.0

@@ -249,12 +249,14 @@ def test_head_slices_of_dcb(heads, rows, chunk, headdim, dstate, dtype, slices):
     # kernels that rebuild C.B^T: up to 256 or 128 where that leaves enough workgroups; never down
     (4, 1024, 16, 64, 1, 64, "BF16", 1, 64, 256), (4, 1024, 15, 64, 1, 64, "BF16", 1, 64, 128), (1, 300, 4, 64, 1, 64, "F16", 0, 64, 64),
     (1, 300, 4, 64, 1, 64, "F16", 0, 256, 256), (4, 1024, 8, 128, 1, 64, "F16", 1, 128, 256),
-    # state dimension 128: training with few heads of 64 in a group stays at 128
-    (4, 2048, 16, 64, 8, 128, "BF16", 0, 64, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 256, 128), (4, 2048, 16, 64, 2, 128, "BF16", 1, 64, 256),
+    # state dimension 128: training with few heads of 64 in a group goes up to 128 at most, and not down (one-part chunk states)
+    (4, 2048, 16, 64, 8, 128, "BF16", 0, 64, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 256, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 64, 128), (4, 2048, 16, 64, 2, 128, "BF16", 1, 64, 256),
     (4, 2048, 16, 128, 8, 128, "BF16", 1, 64, 256),
     # the other 16-bit shapes: 128, from below only where that fills the chip
     (1, 300, 4, 16, 1, 16, "BF16", 1, 256, 128), (1, 300, 4, 16, 1, 16, "BF16", 1, 64, 64), (4, 1024, 8, 32, 1, 16, "BF16", 0, 64, 128),
     (4, 1024, 8, 96, 1, 64, "BF16", 0, 224, 128), (4, 1024, 8, 64, 1, 80, "F16", 1, 32, 128),
+    # ... and from above only where the chunk states take their weighted operand in two parts
+    (1, 300, 4, 20, 1, 16, "BF16", 1, 256, 256), (1, 300, 4, 16, 1, 20, "BF16", 0, 256, 256), (1, 300, 4, 64, 1, 192, "F16", 0, 256, 256),
     # sizes that are no whole steps of the kernels stay
     (4, 2048, 16, 64, 1, 64, "F32", 1, 200, 200), (4, 2048, 16, 16, 1, 64, "BF16", 1, 33, 33),
 ])
