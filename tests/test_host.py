@@ -248,7 +248,7 @@ def test_head_slices_of_dcb(heads, rows, chunk, headdim, dstate, dtype, slices):
     (1, 100, 1, 16, 1, 16, "F32", 0, 128, 64), (4, 2048, 16, 64, 1, 64, "F32", 1, 64, 64), (4, 2048, 16, 64, 1, 64, "F32", 1, 32, 32),
     # kernels that rebuild C.B^T: up to 256 or 128 where that leaves enough workgroups; never down
     (4, 1024, 16, 64, 1, 64, "BF16", 1, 64, 256), (4, 1024, 15, 64, 1, 64, "BF16", 1, 64, 128), (1, 300, 4, 64, 1, 64, "F16", 0, 64, 64),
-    (1, 300, 4, 64, 1, 64, "F16", 0, 256, 256), (4, 1024, 8, 128, 1, 64, "F16", 1, 128, 256),
+    (1, 300, 4, 64, 1, 64, "F16", 0, 256, 256), (4, 1024, 8, 128, 1, 64, "F16", 1, 128, 256), (4, 136, 8, 128, 2, 128, "BF16", 0, 64, 64),
     # state dimension 128: training with few heads of 64 in a group goes up to 128 at most, and not down (one-part chunk states)
     (4, 2048, 16, 64, 8, 128, "BF16", 0, 64, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 256, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 64, 128), (4, 2048, 16, 64, 2, 128, "BF16", 1, 64, 256),
     (4, 2048, 16, 128, 8, 128, "BF16", 1, 64, 256),
