@@ -557,15 +557,28 @@ def _point_into(c, blob, offs, fields=_BLOB_FIELDS):
 MAX_SEQ_BOUNDARIES_PER_CHUNK = 32
 
 
-def _chunk_for(x, dt, A, B, C, chunk_size, D, z, dt_bias, seq_idx):
-    """The chunk size that the kernels run the problem with (bimamba2_chunk_for), as the native route chooses it."""
+def _chunk_for(x, dt, A, B, C, chunk_size, D, z, dt_bias, seq_idx, initial_states=(None, None)):
+    """The chunk size that the kernels run the problem with (bimamba2_chunk_for), as the native route chooses it: which kernels run,
+    and with them the choice, depends on the operands' strides and alignment as well."""
     if x.shape[-1] > MAX_HEADDIM or B.shape[-1] > MAX_DSTATE or x.dtype not in _DT:
         return chunk_size                                          # (the pieces that such a call is made of choose theirs)
     p = _lib.Params()
     p.batch, p.seqlen, p.nheads, p.headdim = (int(n) for n in x.shape)
     p.ngroups, p.dstate, p.chunk_size, p.dtype = int(B.shape[2]), int(B.shape[3]), chunk_size, _DT[x.dtype]
+    for field, prefix, t in (("x", "x_s", x), ("Bm", "B_s", B), ("Cm", "C_s", C), ("z", "z_s", z)):
+        if t is None:
+            continue
+        # (as _Call._strided leaves them: what it converts or copies lies in memory of its own, which is aligned)
+        strides = t.stride() if t.dtype == x.dtype else torch.empty_like(t, dtype=x.dtype, device="meta").stride()
+        moved = t.dtype != x.dtype or strides[-1] != 1
+        if strides[-1] != 1:
+            strides = torch.empty(t.shape, device="meta").stride()
+        setattr(p, field, None if moved else t.data_ptr())
+        for name, n in zip(("b", "l", "g" if field in ("Bm", "Cm") else "h"), strides):
+            setattr(p, prefix + name, n)
+    p.has_z = int(z is not None)
     p.seq_idx = seq_idx.data_ptr() if seq_idx is not None else None
-    training = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, dt, A, B, C, D, z, dt_bias))
+    training = torch.is_grad_enabled() and any(t is not None and t.requires_grad for t in (x, dt, A, B, C, D, z, dt_bias, *initial_states))
     return int(_lib.load().bimamba2_chunk_for(p, 1 if training else 0))
 
 
@@ -706,9 +719,10 @@ def _mamba_chunk_scan_combined_bwd(dout, x, dt, A, B, C, out, chunk_size, D=None
         sshape = (batch, nheads, headdim, B.shape[3])
         dinit = tuple(c.new(f, sshape) if t is not None else None
                       for f, t in zip(("dinitial_f", "dinitial_b"), initial_states))
-    if blob is not None and x.element_size() == 2 and (dout.data_ptr() % 16 or any(s % 8 for s in dout.stride()[:3])):
-        # the forward kept the 16-bit copies of the entering states only, which the kernels for aligned operands know:
-        # a gradient view that breaks their alignment (e.g. a slice of a wider tensor at an odd offset) is copied
+    if x.element_size() == 2 and (dout.data_ptr() % 16 or any(s % 8 for s in dout.stride()[:3])):
+        # a gradient view that breaks the alignment of the kernels' rows (e.g. a slice of a wider tensor at an odd offset) is copied: the
+        # kernels that read the 16-bit copies of the entering states take aligned rows, and so do those that the chunk size was
+        # chosen for
         dout = dout.contiguous()
     c.set_dout(dout)
     if blob is not None:
@@ -869,7 +883,7 @@ def bimamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_b
         res = _lib.host().scan(x, dt, A, B, C, chunk_size, D, z, dt_bias, dt_softplus, dt_limit[0], dt_limit[1],
                                return_final_states, initial_states_f, initial_states_b, seq_idx)
         return tuple(res) if return_final_states else res[0]
-    chunk_size = _chunk_for(x, dt, A, B, C, chunk_size, D, z, dt_bias, seq_idx)
+    chunk_size = _chunk_for(x, dt, A, B, C, chunk_size, D, z, dt_bias, seq_idx, (initial_states_f, initial_states_b))
     if seq_idx is not None:
         # many short packed sequences: a smaller chunk keeps the boundaries per chunk inside what the mechanism resolves
         chunk_size = chunk_size_for_seq_idx(seq_idx, chunk_size)

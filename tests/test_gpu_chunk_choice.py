@@ -44,3 +44,29 @@ def test_results_do_not_depend_on_the_choice(monkeypatch, b, L, H, P, G, N, Q, r
         for name, g, w in zip(["out"] + names, got, want):
             err = (g.double() - w).norm() / w.norm()
             assert err < REL[dtype], (name, float(err))
+
+
+@pytest.mark.parametrize("odd", [(), ("x",), ("B",), ("dout",)])
+def test_both_routes_choose_the_same(monkeypatch, odd):
+    """operands at an odd element, which another kernel of the chunk states takes: the route through Python runs in the chunks that
+    the native one runs in, with the same kernels, so that the results are equal in bits"""
+    from bi_mamba2_amd import ops
+    b, L, H, P, N, dtype = 2, 900, 8, 16, 16, torch.bfloat16
+
+    def place(name, t):
+        if t is None or name not in odd:
+            return t
+        return torch.cat([t.new_zeros(1), t.flatten()])[1:].view(t.shape)
+    d = {k: None if v is None else place(k, v.cuda()).requires_grad_(True) for k, v in make_case(b, L, H, P, 1, N, dtype).items()}
+    dout = place("dout", torch.randn(b, L, H, P, generator=torch.Generator().manual_seed(3)).to(dtype).cuda())
+    leaves = [v for v in d.values() if v is not None]
+
+    def run(**kw):
+        out = ops.bimamba_chunk_scan_combined(d["x"], d["dt"], d["A"], d["B"], d["C"], 256, D=d["D"], dt_bias=d["dt_bias"], dt_softplus=True, **kw)
+        return (out.detach(),) + torch.autograd.grad(out, leaves, dout)
+    native, places = run(), run(grad_places={})
+    monkeypatch.setattr(ops, "KEEP_FORWARD_INTERMEDIATES", False)
+    for route in (places, run()):
+        for k, a, w in zip(["out"] + [k for k, v in d.items() if v is not None], route, native):
+            assert torch.equal(a, w), k
+

@@ -269,3 +269,35 @@ def test_chunk_size_that_the_kernels_run_with(batch, seqlen, heads, headdim, gro
     p.causal, p.seq_idx = 0, 4096
     assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == (chunk if chunk <= 32 else runs)   # 32: needs no count of boundaries
     assert lib.bimamba2_chunk_for(ctypes.byref(_params(chunk_size=16)), training) == 16            # (refused by the entry points)
+
+
+@pytest.mark.parametrize("training", [False, True])
+def test_python_route_chooses_the_chunk_by_the_operands_themselves(training):
+    """bfloat16, 900 positions, 8 heads of 16: chunks of 256 become 128 only where the kernel with two-part operands runs, which takes
+    aligned rows; the native route hands the strides and addresses over, and so does the Python one"""
+    def at(shape, offset=0, width=None, dtype=torch.bfloat16):         # offset: elements behind an aligned address; width: of a wider row
+        rows, n = shape[0] * shape[1], shape[2] * shape[3]
+        width = width or n
+        return torch.zeros(rows * width + offset, dtype=dtype)[offset:].view(*shape[:2], width)[..., :n].unflatten(-1, shape[2:])
+    X, N = (2, 900, 8, 16), (2, 900, 1, 16)
+    dt, A = torch.zeros(2, 900, 8), torch.zeros(8)
+
+    def chosen(x, B, C, z=None, **kw):
+        leaf = A.clone().requires_grad_(training)
+        return ops._chunk_for(x, dt, leaf, B, C, 256, None, z, None, None, **kw)
+    assert chosen(at(X), at(N), at(N)) == 128
+    assert chosen(at(X), at(N), at(N), at(X)) == 128
+    for odd in (dict(offset=1), dict(width=132)):
+        assert chosen(at(X, **odd), at(N), at(N)) == 256
+    assert chosen(at(X), at(N, offset=1), at(N)) == 256 and chosen(at(X), at(N), at(N, offset=4)) == 256
+    # what is converted or copied on its way to the kernels arrives aligned
+    assert chosen(at(X), at(N, offset=1, dtype=torch.float32), at(N)) == 128
+    assert chosen(at(X), at(N), torch.zeros(2, 16, 1, 901, dtype=torch.bfloat16)[..., 1:].permute(0, 3, 2, 1)) == 128
+
+
+def test_initial_states_count_as_training():
+    """heads of 64 at dstate 128, few of them a group: chunks grow to 256 in a pass without gradients only"""
+    x, bc = torch.zeros(4, 2048, 16, 64, dtype=torch.bfloat16), torch.zeros(4, 2048, 8, 128, dtype=torch.bfloat16)
+    dt, A, state = torch.zeros(4, 2048, 16), torch.zeros(16), torch.zeros(4, 16, 64, 128)
+    assert ops._chunk_for(x, dt, A, bc, bc, 64, None, None, None, None, (state, None)) == 256
+    assert ops._chunk_for(x, dt, A, bc, bc, 64, None, None, None, None, (None, state.requires_grad_(True))) == 128
