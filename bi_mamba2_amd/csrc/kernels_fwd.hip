@@ -228,7 +228,8 @@ __device__ __forceinline__ void chunk_state_direct_body(const bimamba2_params &p
             for (int e = 0; e < 4; ++e) raw_lds_use(dt_raw[e]);
             const float A = A_h;
             const float bias = p.has_dt_bias ? bias_h : 0.f;
-            float a[4], ar[4];                               // (differ with seq_idx only, see chunk_cumsum_wave)
+            // cuts of packed sequences in front of a position in the forward sums and behind it in the reverse ones (see chunk_cumsum_wave)
+            float cut_f[4] = {}, cut_b[4] = {};
 #pragma unroll
             for (int e = 0; e < 6; ++e) raw_lds_use(sid[e]);
 #pragma unroll
@@ -242,21 +243,29 @@ __device__ __forceinline__ void chunk_state_direct_body(const bimamba2_params &p
                 d = fminf(fmaxf(d, p.dt_min), p.dt_max);
                 if (q >= limit) d = 0.f;
                 keep_dt[e] = d;
-                a[e] = ar[e] = d * A;
                 if (p.seq_idx && q < limit) {
-                    if (__float_as_uint(sid[e]) != __float_as_uint(sid[e + 1])) a[e] += BIMAMBA2_SEQ_CUT;
-                    if (__float_as_uint(sid[e + 2]) != __float_as_uint(sid[e + 1])) ar[e] += BIMAMBA2_SEQ_CUT;
+                    if (__float_as_uint(sid[e]) != __float_as_uint(sid[e + 1])) cut_f[e] = BIMAMBA2_SEQ_CUT;
+                    if (__float_as_uint(sid[e + 2]) != __float_as_uint(sid[e + 1])) cut_b[e] = BIMAMBA2_SEQ_CUT;
                 }
             }
+            // The products dt * A enter their sums unrounded.  (Written out: with the cuts' conditions between product and sum the compiler
+            // does not fuse the two by itself.)
             float pf[4], sb[4];
-            pf[0] = a[0]; pf[1] = pf[0] + a[1]; pf[2] = pf[1] + a[2]; pf[3] = pf[2] + a[3];
-            sb[3] = ar[3]; sb[2] = sb[3] + ar[2]; sb[1] = sb[2] + ar[1]; sb[0] = sb[1] + ar[0];
+            pf[0] = fmaf(keep_dt[0], A, cut_f[0]);
+            sb[3] = fmaf(keep_dt[3], A, cut_b[3]);
+#pragma unroll
+            for (int e = 1; e < 4; ++e) {
+                pf[e] = fmaf(keep_dt[e], A, pf[e - 1] + cut_f[e]);
+                sb[3 - e] = fmaf(keep_dt[3 - e], A, sb[4 - e] + cut_b[3 - e]);
+            }
             const float tot = pf[3], tot_r = sb[0];
             const float before = wave_incl_prefix(tot, lane) - tot, after = wave_incl_suffix(tot_r, lane) - tot_r;
+            keep_f[0] = fmaf(keep_dt[0], A, before + cut_f[0]);
+            keep_b[3] = fmaf(keep_dt[3], A, after + cut_b[3]);
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
+            for (int e = 1; e < 4; ++e) {
                 keep_f[e] = before + pf[e];
-                keep_b[e] = after + sb[e];
+                keep_b[3 - e] = after + sb[3 - e];
             }
             raw_lds_write128_at<0>(dts_a + lane * 16, f32x4{keep_dt[0], keep_dt[1], keep_dt[2], keep_dt[3]});
             raw_lds_write128_at<0>(csf_a + lane * 16, f32x4{keep_f[0], keep_f[1], keep_f[2], keep_f[3]});

@@ -218,3 +218,28 @@ def test_chunk_states_of_narrow_tiles(P, N, L, Q, dtype):
             off = u + 2.0 ** -16 + (rows(e).abs()[..., None] + 4) * 2.0 ** -23
             bound = torch.einsum("bcqhp,bcqhn->bchpn", xs.abs() * off, ms.abs()) + tiny * ms.abs().sum(2)[..., None, :] + 1e-30
             assert float(((g - want).abs() / bound).max()) <= 1.0
+
+
+@pytest.mark.parametrize("L,Q,N,dtype,one_row", [(300, 256, 64, torch.bfloat16, False), (100, 64, 64, torch.float16, False),
+                                                 (257, 128, 128, torch.bfloat16, True)])
+def test_sums_beside_the_chunk_states_take_the_products_unrounded(ops, L, Q, N, dtype, one_row):
+    """Pairs of dt that cancel: 1 and -(1 - k / 65536).  1 * A is exact, so a sum that takes the second product unrounded is off by
+    its additions alone, at the size of the small sums; a rounded product is off by 2^-25 |A|.  one_row: seq_idx without a boundary."""
+    H, nc = 4, -(-L // Q)
+    d = to_dev(make_case(2, L, H, 64, 2, N, dtype))
+    k = torch.randint(1, 9, (2, nc * Q // 4, H), generator=torch.Generator().manual_seed(4)).float()
+    dt = torch.zeros(2, nc * Q // 4, 4, H)
+    dt[:, :, 0, 0::2], dt[:, :, 1, 0::2] = 1.0, k[..., 0::2] / 65536 - 1.0        # even heads: the exact product comes first
+    dt[:, :, 2, 1::2], dt[:, :, 3, 1::2] = k[..., 1::2] / 65536 - 1.0, 1.0        # odd heads: ... first in the reverse sums
+    dt = dt.flatten(1, 2)[:, :L // 4 * 4]
+    dt = torch.nn.functional.pad(dt, (0, 0, 0, L - dt.shape[1])).cuda()
+    A = -torch.rand(H, generator=torch.Generator().manual_seed(5)).cuda() - 1.0
+    si = torch.zeros(2, L, dtype=torch.int32, device="cuda") if one_row else None
+    res = ops._mamba_chunk_scan_combined_fwd(d["x"], dt, A, d["B"], d["C"], Q, dt_limit=(-INF, INF), seq_idx=si)
+    a = torch.nn.functional.pad(dt, (0, 0, 0, nc * Q - L)).double().view(2, nc, Q, H).permute(0, 3, 1, 2) * A.double()[:, None, None]
+    for got, want, heads, big in ((res[3], a.cumsum(-1), slice(0, None, 2), 0), (res[4], a.flip(-1).cumsum(-1).flip(-1), slice(1, None, 2), 3)):
+        got, want = (t[:, heads].unflatten(-1, (Q // 4, 4)) for t in (got.double(), want))
+        small = [e for e in range(4) if e != big]                                # (the sum behind the first of a pair is about A)
+        # (four positions of a lane, six steps over the wave, what is in front of the lane by a difference, and their sum)
+        err, bound = float((got - want)[..., small].abs().max()), 12 * 2.0 ** -24 * float(want[..., small].abs().max())
+        assert err <= bound
