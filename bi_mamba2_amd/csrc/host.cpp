@@ -425,11 +425,11 @@ public:
         BM2_ASSERT(dout.sizes() == x.sizes(), "gradient of the output: expected the shape of x");
         dout = as_type(dout, x.scalar_type());
         // the kernels that read the kept 16-bit states take aligned rows: a gradient view that is not (a slice of a wider
-        // tensor at an odd offset) is copied
+        // tensor at an odd offset) is copied (clone: contiguous() leaves a contiguous tensor at an odd address where it is)
         bool even = dout.stride(-1) == 1;
         if (even && p.dtype != BIMAMBA2_F32)
             even = aligned16(dout.const_data_ptr()) && dout.stride(0) % 8 == 0 && dout.stride(1) % 8 == 0 && dout.stride(2) % 8 == 0;
-        if (!even) dout = dout.contiguous();
+        if (!even) dout = dout.clone(at::MemoryFormat::Contiguous);
         p.dout = dout.const_data_ptr();
         p.dout_sb = dout.stride(0); p.dout_sl = dout.stride(1); p.dout_sh = dout.stride(2);
         Tensor dfin_f, dfin_b, dinit_f, dinit_b;

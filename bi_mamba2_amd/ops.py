@@ -722,8 +722,8 @@ def _mamba_chunk_scan_combined_bwd(dout, x, dt, A, B, C, out, chunk_size, D=None
     if x.element_size() == 2 and (dout.data_ptr() % 16 or any(s % 8 for s in dout.stride()[:3])):
         # a gradient view that breaks the alignment of the kernels' rows (e.g. a slice of a wider tensor at an odd offset) is copied: the
         # kernels that read the 16-bit copies of the entering states take aligned rows, and so do those that the chunk size was
-        # chosen for
-        dout = dout.contiguous()
+        # chosen for (clone: contiguous() leaves a contiguous tensor at an odd address where it is)
+        dout = dout.clone(memory_format=torch.contiguous_format)
     c.set_dout(dout)
     if blob is not None:
         _point_into(c, blob, snap[2], snap[3])

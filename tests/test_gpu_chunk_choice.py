@@ -70,3 +70,18 @@ def test_both_routes_choose_the_same(monkeypatch, odd):
         for k, a, w in zip(["out"] + [k for k, v in d.items() if v is not None], route, native):
             assert torch.equal(a, w), k
 
+
+@pytest.mark.parametrize("keep", [True, False])
+@pytest.mark.parametrize("L,H,P,N", [(900, 8, 16, 16), (300, 4, 64, 64)])        # two-part chunk states; 16-bit states kept for the backward pass
+def test_a_contiguous_gradient_at_an_odd_address_is_copied(monkeypatch, keep, L, H, P, N):
+    from bi_mamba2_amd import ops
+    monkeypatch.setattr(ops, "KEEP_FORWARD_INTERMEDIATES", keep)
+    d = {k: None if v is None else v.cuda().requires_grad_(True) for k, v in make_case(2, L, H, P, 1, N, torch.bfloat16).items()}
+    dout = torch.randn(2, L, H, P, generator=torch.Generator().manual_seed(3)).bfloat16().cuda()
+    odd = torch.cat([dout.new_zeros(1), dout.flatten()])[1:].view(dout.shape)
+    leaves = [v for v in d.values() if v is not None]
+    out = ops.bimamba_chunk_scan_combined(d["x"], d["dt"], d["A"], d["B"], d["C"], 256, D=d["D"], dt_bias=d["dt_bias"], dt_softplus=True)
+    want, got = (torch.autograd.grad(out, leaves, g, retain_graph=True) for g in (dout, odd))
+    for name, a, w in zip([k for k, v in d.items() if v is not None], got, want):
+        assert torch.equal(a, w), name
+
