@@ -106,7 +106,8 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     }
     if (is_bwd) {
         const size_t nqt = (Q + 63) / 64;
-        if (!q->dCB && !q->dCBT) q->dcb_slices = choose_dcb_slices(q);
+        if (!q->dBs && !q->dCs) q->dbdc_heads = choose_dbdc_heads(q);
+        if (!q->dCB && !q->dCBT) q->dcb_slices = choose_dcb_slices(q);      // (which asks about the last launch, and that about the slices of dB and dC)
         need_f(q->dCB, cbn * dcb_slices(q));
         need_f(q->dCBT, cbn * dcb_slices(q));
         if (!scan_recomputes_cb(q, true)) need_f(q->CBT, cbn);
@@ -129,7 +130,6 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
         need_f(q->da_intra, (size_t)q->batch * q->nheads * nc * nqt * nqt * 128);
         need_f(q->ddA_chunk_f, (size_t)q->batch * q->nheads * nc * sp_nsplit(q));
         need_f(q->ddA_chunk_b, (size_t)q->batch * q->nheads * nc * sp_nsplit(q));
-        if (!q->dBs && !q->dCs) q->dbdc_heads = choose_dbdc_heads(q);
         const int hps = q->dbdc_heads > 0 ? q->dbdc_heads : 8;
         const size_t slices = (q->nheads / q->ngroups + hps - 1) / hps;   // head slices of the dB / dC partial sums
         const size_t bn = slices * q->batch * q->seqlen * q->ngroups * q->dstate;

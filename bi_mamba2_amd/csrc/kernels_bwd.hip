@@ -1107,6 +1107,11 @@ static int launch_dcb_t(const bimamba2_params *p, bool add_up) {
 // slices, heads of 64, dstate 64, chunks of 256: 48 heads, 64 tiles 161 / 135 / 124, 128 tiles 183 / 158 / 152, 384 tiles 312 / 297 / 314;
 // 32 heads of 128, dstate 128, 96 tiles 264 / 240 / 234; from 512 tiles on they cost (32 heads 244 / 249 / 271; 16 heads 154 / 157 / 167).
 // Between 256 and 384 tiles few heads give little (24 heads 150 / 143 / 146, with dstate 128 306 / 302 / 316): one slice up to 31 heads.
+// All of these are chunks of 256, where the last launch adds the slices up.  Where none does (dt of a type of its own in chunks of up to
+// 128, chunks between, state dimensions other than 64 and 128 in chunks of 256) they take a launch for it and part the dCB launch from
+// the state passing, 5 us that 16 heads do not earn; 1 slice -> as above: 8 heads of 64, 2048 positions, dstate 192 181 -> 184, 12 heads 207 -> 211,
+// 16 heads 223 -> 226, 24 heads 259 -> 254; float16 dt beside bfloat16, dstate 64, 1024 positions 8 heads 85 -> 90, 32 heads 133 -> 113, 48
+// heads 161 -> 128; 3000 positions, 16 heads 123 -> 124, 20 heads 131 -> 129.
 // The kernel reads C.B^T (float32, and 16-bit shapes whose state or headdim is no multiple of what the rebuilding kernel takes: the ring
 // with a narrow state or narrow heads; through registers where rows are not aligned).
 // A workgroup is one chain over its heads, 5 to 7 us a head through registers in float32, 3 to 5 in 16 bits and 1.5 in the ring,
@@ -1126,6 +1131,7 @@ int choose_dcb_slices(const bimamba2_params *p) {
     const int64_t wgs = (int64_t)p->batch * nchunks(p) * p->ngroups * nqt * nqt;
     int wanted = usual;
     if (dcb_recomputes_cb(p)) {
+        if (hpg <= 16 && !bwd_tail_merged(p) && !bwd_tail_small(p)) return usual;
         if (wgs < 256 || (wgs <= 384 && hpg >= DCB_SLICE_HEADS)) wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 4, 4, std::max<int64_t>(512 / wgs, 2)}));
     } else {
         const int most = p->dtype == BIMAMBA2_F32 ? (hpg < 6 ? 256 : 768) : std::min(768, 32 * hpg);      // workgroups

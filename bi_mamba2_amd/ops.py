@@ -161,11 +161,11 @@ class _Call:
         # the size depends on the problem and on which intermediates the caller brought; ask the library once per such key
         # (which kernels run, and with them what is carved, also depends on strides and on 16-byte alignment)
         al = lambda v: (v or 0) & 15
-        key = (is_bwd, p.batch, p.seqlen, p.nheads, p.headdim, p.ngroups, p.dstate, p.chunk_size, p.dtype, p.has_z, p.causal,
+        key = (is_bwd, p.batch, p.seqlen, p.nheads, p.headdim, p.ngroups, p.dstate, p.chunk_size, p.dtype, p.dt_dtype, p.has_z, p.causal,
                bool(p.dt_out), bool(p.cs_f), bool(p.states_f), bool(p.states_b), bool(p.CB), bool(p.CBT), bool(p.dCB), bool(p.dCBT),
                bool(p.dstates_f), bool(p.dout_x), bool(p.red), bool(p.dBs), bool(p.da_intra),
                p.x_sb, p.x_sl, p.x_sh, p.z_sb, p.z_sl, p.z_sh, p.dout_sb, p.dout_sl, p.dout_sh, p.B_sb, p.B_sl, p.B_sg,
-               p.C_sb, p.C_sl, p.C_sg, al(p.x), al(p.z), al(p.dout), al(p.Bm), al(p.Cm), al(p.out), al(p.out_x), al(p.dx),
+               p.C_sb, p.C_sl, p.C_sg, p.dx_sb, p.dx_sl, p.dB_sb, p.dB_sl, p.dC_sb, p.dC_sl, al(p.dB), al(p.dC), al(p.x), al(p.z), al(p.dout), al(p.Bm), al(p.Cm), al(p.out), al(p.out_x), al(p.dx),
                al(p.states_f), al(p.states_b), al(p.dstates_f), al(p.dstates_b),
                bool(p.states16_f), bool(p.dstates16_f), p.fwd_saved, al(p.states16_f), al(p.states16_b), al(p.final_f), al(p.final_b),
                al(p.initial_f), al(p.initial_b), al(p.dfinal_f), al(p.dfinal_b), al(p.dinitial_f), al(p.dinitial_b))

@@ -241,6 +241,29 @@ def test_head_slices_of_dcb(heads, rows, chunk, headdim, dstate, dtype, slices):
     assert _dcb_slices(**_contiguous(rows, chunk, heads, headdim, 1, dstate, chunk, dtype)) == slices
 
 
+# wide 16-bit heads over 4 (batch, chunk) pairs: up to 16 heads are cut only where the last launch adds the slices up
+@pytest.mark.parametrize("chunk,dstate,more,added", [
+    (256, 64, {}, True), (256, 64, dict(dt_dtype=_lib.F16), True), (128, 64, dict(dt_dtype=_lib.BF16), True), (64, 64, {}, True), (128, 96, {}, True),
+    (128, 64, dict(dt_dtype=_lib.F16), False), (64, 128, dict(dt_dtype=_lib.F16), False),       # chunks of up to 128: dt in float32 or the type of x
+    (192, 64, {}, False), (256, 96, {}, False), (256, 64, dict(dB=258), False), (256, 64, dict(dC_sl=1028), False)])
+def test_head_slices_of_dcb_where_nothing_adds_them_up(chunk, dstate, more, added):
+    for heads, slices in ((8, 2 if added else 1), (16, 4 if added else 1), (17, 4), (48, 4)):
+        assert _dcb_slices(**_contiguous(4, chunk, heads, 64, 1, dstate, chunk, _lib.BF16), **more) == slices, heads
+
+
+def test_workspace_sizes_are_kept_apart_by_what_the_slices_depend_on():
+    """16 heads of 64 in chunks of 128: four slices of dCB with dt in float32, one with dt of a type of its own, or dB at an odd address in chunks of 256"""
+    def size(chunk, dt_dtype, dB):
+        c = ops._Call(1, 512, 16, 64, 1, 64, chunk, torch.bfloat16, torch.device("cpu"), dt_dtype)
+        for name, n in _contiguous(1, 512, 16, 64, 1, 64, chunk, _lib.BF16).items():
+            setattr(c.p, name, n)
+        c.p.dB = dB
+        c.workspace(True)
+        return c.p.workspace_bytes
+    assert size(128, torch.float16, 256) < size(128, torch.float32, 256)
+    assert size(256, torch.float32, 258) < size(256, torch.float32, 256)
+
+
 # what a caller asks for -> what the kernels run with, at the lines of the rule: workgroups of one launch against the chip's 256
 @pytest.mark.parametrize("batch,seqlen,heads,headdim,groups,dstate,dtype,training,chunk,runs", [
     # float32: down to 128 where that fills the chip, else to 64; never up
