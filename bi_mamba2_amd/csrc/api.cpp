@@ -244,8 +244,25 @@ int bimamba2_chunk_for(const bimamba2_params *p, int training) {
     };
     constexpr int CUS = 256;
     if (p->dtype == BIMAMBA2_F32) return Q > 64 ? std::min(Q, workgroups(128, 32) >= CUS ? 128 : 64) : Q;
-    const bool whole = P == 64 || P == 128;
-    if (whole && (N == 64 || (N == 128 && (!training || P == 128 || p->nheads >= 8 * p->ngroups))))
+    // whether the kernels for whole 64 x 64 tiles of aligned rows are the ones that run; the generic ones, which take the other rows, are
+    // among the other shapes below (x at an odd element, one group, a pass with gradients: 4 x 2048, 16 heads of 64, dstate 64 444 / 416 / 555, dstate
+    // 128 672 / 543 / 677; 2 x 2048, 8 heads of 128 256 / 241 / 341; 8 groups, 4 x 4096, 32 heads of 64 1947 / 1738 / 2339)
+    auto whole = [&] {
+        if (!(P == 64 || P == 128) || !(N == 64 || N == 128)) return false;
+        bimamba2_params q = *p;
+        q.chunk_size = 256;
+        // (an operand that is not named yet will be contiguous)
+        auto rows = [&](const void *t, int64_t &sb, int64_t &sl, int64_t &si, int heads, int width) {
+            if (!t && !sb && !sl && !si) sb = (int64_t)p->seqlen * (sl = (int64_t)heads * (si = width));
+        };
+        rows(q.x, q.x_sb, q.x_sl, q.x_sh, p->nheads, P);
+        rows(q.Bm, q.B_sb, q.B_sl, q.B_sg, p->ngroups, N);
+        rows(q.Cm, q.C_sb, q.C_sl, q.C_sg, p->ngroups, N);
+        if (!training) return chunk_scan_uses_scan16(&q, false);
+        if (N == 64) return scan_recomputes_cb(&q, false) && scan_recomputes_cb(&q, true) && dcb_recomputes_cb(&q);
+        return chunk_state_does_cumsum(&q) && dcb_recomputes_cb(&q);
+    };
+    if ((N == 64 || !training || P == 128 || p->nheads >= 8 * p->ngroups) && whole())
         return std::max(Q, workgroups(256, 64) >= CUS ? 256 : workgroups(128, 64) >= CUS / 2 ? 128 : Q);
     if (Q <= 128) return workgroups(128, 64) >= CUS ? 128 : Q;
     bimamba2_params q = *p;

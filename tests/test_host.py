@@ -324,3 +324,22 @@ def test_initial_states_count_as_training():
     dt, A, state = torch.zeros(4, 2048, 16), torch.zeros(16), torch.zeros(4, 16, 64, 128)
     assert ops._chunk_for(x, dt, A, bc, bc, 64, None, None, None, None, (state, None)) == 256
     assert ops._chunk_for(x, dt, A, bc, bc, 64, None, None, None, None, (None, state.requires_grad_(True))) == 128
+
+
+@pytest.mark.parametrize("heads,headdim,groups,dstate", [(16, 64, 1, 64), (16, 64, 1, 128), (8, 128, 1, 64)])
+@pytest.mark.parametrize("training", [0, 1])
+def test_chunks_of_wide_heads_grow_only_where_their_kernels_run(heads, headdim, groups, dstate, training):
+    """4 x 2048 in bfloat16, chunks of 128 asked for: 256 with the kernels for aligned rows, as asked with those for any rows"""
+    lib, named = _lib.load(), dict(x=256, Bm=256, Cm=256, z=256, has_z=1)
+
+    def chosen(**kw):
+        p = _contiguous(4, 2048, heads, headdim, groups, dstate, 128, _lib.BF16)
+        z = {"z" + k[1:]: v for k, v in p.items() if k.startswith("x_")}
+        return lib.bimamba2_chunk_for(ctypes.byref(_params(**{**p, **z, **named, **kw})), training)
+    assert chosen() == 256 and chosen(x_sl=heads * headdim + 8, B_sl=2 * groups * dstate) == 256
+    assert lib.bimamba2_chunk_for(ctypes.byref(_params(**_contiguous(4, 2048, heads, headdim, groups, dstate, 128, _lib.BF16))), training) == 256
+    for odd in (dict(x=258), dict(Bm=264), dict(Cm=258), dict(x_sl=heads * headdim + 4), dict(B_sl=groups * dstate + 1), dict(C_sb=4097)):
+        assert chosen(**odd) == 128, odd
+    if dstate == 64 or not training:           # (the scan kernel that rebuilds C.B^T)
+        assert chosen(z=258) == 128 and chosen(z_sl=heads * headdim + 2) == 128 and chosen(B_sl=1 << 22) == 128
+
