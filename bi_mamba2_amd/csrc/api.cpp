@@ -215,35 +215,39 @@ int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd) {
     return chunk_scan_uses_scan16(p, bwd != 0) ? chunk_scan16_heads_per_workgroup(p) : 1;
 }
 
-// Where the lines lie, us a pass with chunks of 64 / 128 / 256 (z gate, D; forward alone and, second, with the backward pass; one
-// group unless said otherwise).  A chunk costs its pairs of positions (they grow with the chunk) and its states (which do not);
-// small calls want many workgroups, i.e. small chunks.
-//  * float32: pairs run at the float32 matrix rate.  4 x 2048, 16 heads of 64, dstate 64: 142 / 99 / 118, 478 / 384 / 477; heads of 16,
-//    dstate 16: 49 / 39 / 48, 192 / 168 / 250; 2 x 512, 8 heads of 64, dstate 64: 25 / 29 / 47, 120 / 120 / 180; 4 x 1024, 8 heads of 32:
-//    29 / 29 / 45.  Never above the caller's: the result is off by the resolution of sums over a chunk (1.6 times as much in
-//    chunks twice as long).
-//  * 16 bits, the kernels that rebuild C.B^T (dstate 64, headdim 64 or 128; forward also dstate 128): 4 x 2048, 16 heads of 64, dstate 64:
-//    63 / 44 / 40, 198 / 159 / 152; 4 x 1024, 8 heads: 30 / 25 / 28, 118 / 118 / 118 (host time); 2 x 512: 21 / 22 / 27; dstate 128, 4 x 2048:
-//    88 / 65 / 62.  Never below the caller's, where small calls would be faster: their result is 0.4 % (128) and 1.5 % (64) further from
-//    float64 in bfloat16 (1 x 197, 12 heads: 2.013e-3 / 2.023e-3 / 2.048e-3), most of it from the states in 16 bits.
-//  * other 16-bit shapes: 4 x 2048, 16 heads of 32, dstate 32: 53 / 41 / 45, 178 / 145 / 194; 8 groups, 4 x 4096: 185 / 149 / 178 and 659 / 580 /
-//    784 (32 heads); 4 x 1024, 8 heads: 21 / 20 / 34, 117 / 117 / 136; 2 x 512: 17 / 19 / 32.  Below the caller's chunk only where the
-//    chunk states take their weighted operand in two 16-bit parts: with one, dA was 5 to 32 % further from float64 in chunks of 128
-//    than of 256 (900 positions, 8 heads, 400 inputs); with two no output is (dA -0.3 to -7 %, out -0.4 to -0.8 %, dB and dC -18 to -28 %).
-//    Training at dstate 128 with heads of 64 or 128 and few of them a group stays as asked: 16 heads in 8 groups, 4 x 4096, of 64 1104 /
-//    784 / 880 would gain, with dA 5 % further off.
+// A chunk costs its pairs of positions (they grow with the chunk) and its states (which do not); small calls want many workgroups, i.e. small
+// chunks.  The lines follow the length, the heads and the operands of a row but not the number of rows, so that a row's result is the same
+// alone and in any batch; where they lie is therefore between what one row and what many rows want.  us a pass with chunks of 64 / 128 / 256
+// (z gate, D, one group; forward alone and, second, with the backward pass; workgroups: of one row in chunks of 128, for wide heads
+// 256, as counted below):
+//  * float32: pairs run at the float32 matrix rate.  Heads of 64, dstate 64: 1024 positions, 8 heads (128 workgroups) 30 / 33, 98 / 101, four
+//    rows 52 / 45, 171 / 150; 2048, 8 heads (256) 41 / 37, 131 / 118; 512, 8 heads (64) 27 / 32, 80 / 91, four rows 39 / 36, 126 / 118, sixteen 79 / 65,
+//    270 / 235.  Heads of 32, dstate 16: 2048, 24 heads (384) 37 / 36, 133 / 136; 1024, 8 heads (64) 23 / 27, 74 / 83, four rows 30 / 30, 106 / 108.
+//    Chunks of 256: 118, 477 where 128 takes 99, 384 (4 x 2048, 16 heads of 64).  Never above the caller's: the result is off by the
+//    resolution of sums over a chunk (1.6 times as much in chunks twice as long).
+//  * 16 bits, the kernels that rebuild C.B^T (dstate 64, headdim 64 or 128; forward also dstate 128), heads of 64, dstate 64: 2048, 24 heads (192)
+//    43 / 37 / 35, 119 / 112 / 120, four rows 87 / 64 / 56, 280 / 215 / 201; 1024, 24 heads (96) 34 / 28 / 32, 101 / 96 / 112; 8192, 8 heads (256) 58 / 44 / 40,
+//    168 / 130 / 124; 512, 8 heads (16; 32 in chunks of 128) 24 / 25 / 30, 72 / 75 / 89, sixteen rows 43 / 37 / 36, 128 / 117 / 119; 200, 8 heads 23 / 24 / 29,
+//    71 / 73 / 84.  dstate 128: 2048, 24 heads 55 / 49 / 49, 197 / 154 / 160, four rows 122 / 91 / 85, 657 / 394 / 348.  Never below the caller's, where small
+//    calls would be faster: their result is 0.4 % (128) and 1.5 % (64) further from float64 in bfloat16 (1 x 197, 12 heads:
+//    2.013e-3 / 2.023e-3 / 2.048e-3), most of it from the states in 16 bits.
+//  * other 16-bit shapes, 64 / 128, heads of 32, dstate 32: 1024, 8 heads (64) 22 / 24, 61 / 67, four rows 26 / 25, 89 / 84; 2048, 8 heads (128) 25 / 25,
+//    79 / 79; 2048, 24 heads (384) 34 / 29, 114 / 106; 512, 8 heads (32) 21 / 23, 57 / 64, sixteen rows 38 / 31, 116 / 101.  128 and 256: 41 / 45, 145 / 194 (4 x
+//    2048, 16 heads); 8 groups, 4 x 4096, 32 heads 149 / 178, 580 / 784; 4 x 1024, 8 heads 20 / 34, 117 / 136; 2 x 512 19 / 32.  Below the
+//    caller's chunk only where the chunk states take their weighted operand in two 16-bit parts: with one, dA was 5 to 32 % further from
+//    float64 in chunks of 128 than of 256 (900 positions, 8 heads, 400 inputs); with two no output is (dA -0.3 to -7 %, out -0.4 to
+//    -0.8 %, dB and dC -18 to -28 %).  Training at dstate 128 with heads of 64 or 128 and few of them a group stays as asked: 16 heads
+//    in 8 groups, 4 x 4096, of 64 1104 / 784 / 880 would gain, with dA 5 % further off.
 int bimamba2_chunk_for(const bimamba2_params *p, int training) {
     if (check_problem(p)) return p ? p->chunk_size : 0;
     const int Q = p->chunk_size, P = p->headdim, N = p->dstate;
     // (packed sequences that need no count of their boundaries keep their size: counting them synchronises)
     if (p->causal || Q % 32 || (p->seq_idx && Q <= BIMAMBA2_MAX_SEQ_BOUNDARIES)) return Q;
-    // of one launch over (batch, chunk, head, headdim tile), in whole chunks' worth of positions: the rest of a sequence is a workgroup that
-    // fills nothing (4 x 136, 8 heads of 128, dstate 128: 30.5 us in chunks of 64, 31.2 in a whole chunk of 128 and one of 8 positions)
-    auto workgroups = [&](int q, int columns) {
-        return (int64_t)p->batch * p->seqlen * p->nheads * ((P + columns - 1) / columns) / q;
-    };
+    // of one row in one launch over (chunk, head, headdim tile), in whole chunks' worth of positions: the rest of a sequence is a workgroup
+    // that fills nothing (4 x 136, 8 heads of 128, dstate 128: 30.5 us in chunks of 64, 31.2 in a whole chunk of 128 and one of 8 positions)
+    auto workgroups = [&](int q, int columns) { return (int64_t)p->seqlen * p->nheads * ((P + columns - 1) / columns) / q; };
     constexpr int CUS = 256;
-    if (p->dtype == BIMAMBA2_F32) return Q > 64 ? std::min(Q, workgroups(128, 32) >= CUS ? 128 : 64) : Q;
+    if (p->dtype == BIMAMBA2_F32) return Q > 64 ? std::min(Q, workgroups(128, 32) >= CUS / 2 ? 128 : 64) : Q;
     // whether the kernels for whole 64 x 64 tiles of aligned rows are the ones that run; the generic ones, which take the other rows, are
     // among the other shapes below (x at an odd element, one group, a pass with gradients: 4 x 2048, 16 heads of 64, dstate 64 444 / 416 / 555, dstate
     // 128 672 / 543 / 677; 2 x 2048, 8 heads of 128 256 / 241 / 341; 8 groups, 4 x 4096, 32 heads of 64 1947 / 1738 / 2339)
@@ -263,8 +267,8 @@ int bimamba2_chunk_for(const bimamba2_params *p, int training) {
         return chunk_state_does_cumsum(&q) && dcb_recomputes_cb(&q);
     };
     if ((N == 64 || !training || P == 128 || p->nheads >= 8 * p->ngroups) && whole())
-        return std::max(Q, workgroups(256, 64) >= CUS ? 256 : workgroups(128, 64) >= CUS / 2 ? 128 : Q);
-    if (Q <= 128) return workgroups(128, 64) >= CUS ? 128 : Q;
+        return std::max(Q, workgroups(256, 64) >= CUS / 2 ? 256 : workgroups(128, 64) >= CUS / 8 ? 128 : Q);
+    if (Q <= 128) return workgroups(128, 64) >= CUS / 4 ? 128 : Q;
     bimamba2_params q = *p;
     q.chunk_size = 128;
     const bool exact_states = !(P % 64 == 0 && N % 64 == 0) && chunk_state_narrow(&q, false) && chunk_state_narrow(&q, true);

@@ -843,8 +843,9 @@ def bimamba_chunk_scan_combined(x, dt, A, B, C, chunk_size, D=None, z=None, dt_b
         A: (nheads)
         B: (batch, seqlen, ngroups, dstate)
         C: (batch, seqlen, ngroups, dstate)   (dstate above the kernels' 256: computed in pieces of the state dimension)
-        chunk_size: int, at least 32.  The result does not depend on it, and the kernels may run with another one (at most 256) that
-            is faster for the problem and no less exact
+        chunk_size: int, at least 32.  The result does not depend on it but for rounding, and the kernels may run with another one (at most
+            256) that is faster for the problem and no less exact.  Which one does not depend on the number of rows: out and the final
+            states of a row are the same, in bits, alone and in any batch (with seq_idx: of rows whose boundaries need no smaller chunk)
         D: (nheads, headdim) or (nheads,)
         z: (batch, seqlen, nheads, headdim)
         dt_bias: (nheads,)

@@ -85,3 +85,21 @@ def test_a_contiguous_gradient_at_an_odd_address_is_copied(monkeypatch, keep, L,
     for name, a, w in zip([k for k, v in d.items() if v is not None], got, want):
         assert torch.equal(a, w), name
 
+
+@pytest.mark.parametrize("L,H,P,N,Q,dtype", [
+    (1024, 8, 64, 64, 256, torch.float32), (1024, 16, 32, 16, 128, torch.float32), (1024, 8, 64, 64, 64, torch.bfloat16), (520, 8, 64, 128, 64, torch.bfloat16),
+    (1024, 8, 32, 16, 64, torch.float16), (300, 12, 20, 16, 64, torch.bfloat16)])
+@pytest.mark.parametrize("training", [False, True])
+def test_a_row_does_not_depend_on_the_batch(L, H, P, N, Q, dtype, training):
+    """forward results of a row alone, in two rows and in eight: equal in bits, at sizes on both sides of the lines of the chunk choice"""
+    from bi_mamba2_amd import ops
+    d = {k: None if v is None else v.cuda() for k, v in make_case(8, L, H, P, 1, N, dtype, with_z=True).items()}
+
+    def run(rows):
+        x, dt, B, C, z = (d[k][rows].requires_grad_(training) for k in ("x", "dt", "B", "C", "z"))
+        return ops.bimamba_chunk_scan_combined(x, dt, d["A"], B, C, Q, D=d["D"], z=z, dt_bias=d["dt_bias"], dt_softplus=True, return_final_states=True)
+    alone = run(slice(7, 8))
+    for rows in (slice(6, 8), slice(0, 8)):
+        for name, got, want in zip(("out", "final_f", "final_b"), run(rows), alone):
+            assert torch.equal(got[-1:], want), (name, rows)
+

@@ -264,19 +264,20 @@ def test_workspace_sizes_are_kept_apart_by_what_the_slices_depend_on():
     assert size(256, torch.float32, 258) < size(256, torch.float32, 256)
 
 
-# what a caller asks for -> what the kernels run with, at the lines of the rule: workgroups of one launch against the chip's 256
+# what a caller asks for -> what the kernels run with, at the lines of the rule: workgroups of one row in a launch against the chip's 256
 @pytest.mark.parametrize("batch,seqlen,heads,headdim,groups,dstate,dtype,training,chunk,runs", [
     # float32: down to 128 where that fills the chip, else to 64; never up
-    (2, 1111, 16, 64, 2, 64, "F32", 1, 256, 128), (1, 8192, 4, 32, 1, 16, "F32", 1, 256, 128), (1, 8064, 4, 32, 1, 16, "F32", 0, 256, 64),
+    (2, 1111, 16, 64, 2, 64, "F32", 1, 256, 128), (1, 4096, 4, 32, 1, 16, "F32", 1, 256, 128), (1, 4064, 4, 32, 1, 16, "F32", 0, 256, 64),
     (1, 100, 1, 16, 1, 16, "F32", 0, 128, 64), (4, 2048, 16, 64, 1, 64, "F32", 1, 64, 64), (4, 2048, 16, 64, 1, 64, "F32", 1, 32, 32),
     # kernels that rebuild C.B^T: up to 256 or 128 where that leaves enough workgroups; never down
-    (4, 1024, 16, 64, 1, 64, "BF16", 1, 64, 256), (4, 1024, 15, 64, 1, 64, "BF16", 1, 64, 128), (1, 300, 4, 64, 1, 64, "F16", 0, 64, 64),
-    (1, 300, 4, 64, 1, 64, "F16", 0, 256, 256), (4, 1024, 8, 128, 1, 64, "F16", 1, 128, 256), (4, 136, 8, 128, 2, 128, "BF16", 0, 64, 64),
+    (4, 2048, 16, 64, 1, 64, "BF16", 1, 64, 256), (4, 2048, 15, 64, 1, 64, "BF16", 1, 64, 128), (1, 512, 8, 64, 1, 64, "BF16", 1, 64, 128),
+    (1, 508, 8, 64, 1, 64, "BF16", 1, 64, 64), (1, 300, 4, 64, 1, 64, "F16", 0, 64, 64),
+    (1, 300, 4, 64, 1, 64, "F16", 0, 256, 256), (4, 2048, 8, 128, 1, 64, "F16", 1, 128, 256), (4, 136, 8, 128, 2, 128, "BF16", 0, 64, 64),
     # state dimension 128: training with few heads of 64 in a group goes up to 128 at most, and not down (one-part chunk states)
     (4, 2048, 16, 64, 8, 128, "BF16", 0, 64, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 256, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 64, 128), (4, 2048, 16, 64, 2, 128, "BF16", 1, 64, 256),
     (4, 2048, 16, 128, 8, 128, "BF16", 1, 64, 256),
     # the other 16-bit shapes: 128, from below only where that fills the chip
-    (1, 300, 4, 16, 1, 16, "BF16", 1, 256, 128), (1, 300, 4, 16, 1, 16, "BF16", 1, 64, 64), (4, 1024, 8, 32, 1, 16, "BF16", 0, 64, 128),
+    (1, 300, 4, 16, 1, 16, "BF16", 1, 256, 128), (1, 300, 4, 16, 1, 16, "BF16", 1, 64, 64), (4, 1024, 8, 32, 1, 16, "BF16", 0, 64, 128), (4, 1016, 8, 32, 1, 16, "BF16", 0, 64, 64),
     (4, 1024, 8, 96, 1, 64, "BF16", 0, 224, 128), (4, 1024, 8, 64, 1, 80, "F16", 1, 32, 128),
     # ... and from above only where the chunk states take their weighted operand in two parts
     (1, 300, 4, 20, 1, 16, "BF16", 1, 256, 256), (1, 300, 4, 16, 1, 20, "BF16", 0, 256, 256), (1, 300, 4, 64, 1, 192, "F16", 0, 256, 256),
@@ -287,6 +288,8 @@ def test_chunk_size_that_the_kernels_run_with(batch, seqlen, heads, headdim, gro
     lib = _lib.load()
     p = _params(batch=batch, seqlen=seqlen, nheads=heads, headdim=headdim, ngroups=groups, dstate=dstate, dtype=getattr(_lib, dtype), chunk_size=chunk)
     assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == runs
+    for p.batch in (1, 2, 64, batch):                                          # (a row runs as it would alone)
+        assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == runs
     p.causal = 1                                                               # (the comparator runs as it is asked to)
     assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == chunk
     p.causal, p.seq_idx = 0, 4096
