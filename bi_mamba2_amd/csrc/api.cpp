@@ -225,19 +225,23 @@ int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd) {
 //    270 / 235.  Heads of 32, dstate 16: 2048, 24 heads (384) 37 / 36, 133 / 136; 1024, 8 heads (64) 23 / 27, 74 / 83, four rows 30 / 30, 106 / 108.
 //    Chunks of 256: 118, 477 where 128 takes 99, 384 (4 x 2048, 16 heads of 64).  Never above the caller's: the result is off by the
 //    resolution of sums over a chunk (1.6 times as much in chunks twice as long).
-//  * 16 bits, the kernels that rebuild C.B^T (dstate 64, headdim 64 or 128; forward also dstate 128), heads of 64, dstate 64: 2048, 24 heads (192)
+//  * 16 bits, heads of 64 or 128 with dstate 64 or 128; heads of 64, dstate 64: 2048, 24 heads (192)
 //    43 / 37 / 35, 119 / 112 / 120, four rows 87 / 64 / 56, 280 / 215 / 201; 1024, 24 heads (96) 34 / 28 / 32, 101 / 96 / 112; 8192, 8 heads (256) 58 / 44 / 40,
 //    168 / 130 / 124; 512, 8 heads (16; 32 in chunks of 128) 24 / 25 / 30, 72 / 75 / 89, sixteen rows 43 / 37 / 36, 128 / 117 / 119; 200, 8 heads 23 / 24 / 29,
 //    71 / 73 / 84.  dstate 128: 2048, 24 heads 55 / 49 / 49, 197 / 154 / 160, four rows 122 / 91 / 85, 657 / 394 / 348.  Never below the caller's, where small
 //    calls would be faster: their result is 0.4 % (128) and 1.5 % (64) further from float64 in bfloat16 (1 x 197, 12 heads:
-//    2.013e-3 / 2.023e-3 / 2.048e-3), most of it from the states in 16 bits.
+//    2.013e-3 / 2.023e-3 / 2.048e-3), most of it from the states in 16 bits (float16, 520 positions, 16 heads: 3.03e-4 / 3.02e-4 / 3.01e-4).
+//    A pass with gradients grows to 128 at most: the last launch of chunks of 256 takes dCB rounded to 16 bits, that of up to 128 in two
+//    parts, and dB and dC are 14 to 21 % further off in 256 (2.40e-3 against 2.89e-3 at any number of heads, groups and both state
+//    dimensions), for 3 to 8 % of the time at dstate 64 and 3 to 13 % at 128 (4 x 4096, 32 heads in 8 groups 617 / 584; 2 x 2048, 8 heads of 128,
+//    dstate 128 177 / 172).  In chunks that are no multiples of 64 its states stay in float32 at dstate 64: they are kept (float16, 640
+//    positions, 16 heads: out 2.58e-4 in chunks of 160, 3.08e-4 in 128).
 //  * other 16-bit shapes, 64 / 128, heads of 32, dstate 32: 1024, 8 heads (64) 22 / 24, 61 / 67, four rows 26 / 25, 89 / 84; 2048, 8 heads (128) 25 / 25,
 //    79 / 79; 2048, 24 heads (384) 34 / 29, 114 / 106; 512, 8 heads (32) 21 / 23, 57 / 64, sixteen rows 38 / 31, 116 / 101.  128 and 256: 41 / 45, 145 / 194 (4 x
 //    2048, 16 heads); 8 groups, 4 x 4096, 32 heads 149 / 178, 580 / 784; 4 x 1024, 8 heads 20 / 34, 117 / 136; 2 x 512 19 / 32.  Below the
 //    caller's chunk only where the chunk states take their weighted operand in two 16-bit parts: with one, dA was 5 to 32 % further from
 //    float64 in chunks of 128 than of 256 (900 positions, 8 heads, 400 inputs); with two no output is (dA -0.3 to -7 %, out -0.4 to
-//    -0.8 %, dB and dC -18 to -28 %).  Training at dstate 128 with heads of 64 or 128 and few of them a group stays as asked: 16 heads
-//    in 8 groups, 4 x 4096, of 64 1104 / 784 / 880 would gain, with dA 5 % further off.
+//    -0.8 %, dB and dC -18 to -28 %).
 int bimamba2_chunk_for(const bimamba2_params *p, int training) {
     if (check_problem(p)) return p ? p->chunk_size : 0;
     const int Q = p->chunk_size, P = p->headdim, N = p->dstate;
@@ -248,13 +252,11 @@ int bimamba2_chunk_for(const bimamba2_params *p, int training) {
     auto workgroups = [&](int q, int columns) { return (int64_t)p->seqlen * p->nheads * ((P + columns - 1) / columns) / q; };
     constexpr int CUS = 256;
     if (p->dtype == BIMAMBA2_F32) return Q > 64 ? std::min(Q, workgroups(128, 32) >= CUS / 2 ? 128 : 64) : Q;
-    // whether the kernels for whole 64 x 64 tiles of aligned rows are the ones that run; the generic ones, which take the other rows, are
-    // among the other shapes below (x at an odd element, one group, a pass with gradients: 4 x 2048, 16 heads of 64, dstate 64 444 / 416 / 555, dstate
-    // 128 672 / 543 / 677; 2 x 2048, 8 heads of 128 256 / 241 / 341; 8 groups, 4 x 4096, 32 heads of 64 1947 / 1738 / 2339)
-    auto whole = [&] {
-        if (!(P == 64 || P == 128) || !(N == 64 || N == 128)) return false;
+    const bool wide = (P == 64 || P == 128) && (N == 64 || N == 128);
+    if (wide && !training) {
+        // the kernel that rebuilds C.B^T takes aligned rows; others run the generic one, which is among the other shapes below (x at an odd
+        // element, a pass with gradients: 4 x 2048, 16 heads of 64, dstate 64 444 / 416 / 555, dstate 128 672 / 543 / 677)
         bimamba2_params q = *p;
-        q.chunk_size = 256;
         // (an operand that is not named yet will be contiguous)
         auto rows = [&](const void *t, int64_t &sb, int64_t &sl, int64_t &si, int heads, int width) {
             if (!t && !sb && !sl && !si) sb = (int64_t)p->seqlen * (sl = (int64_t)heads * (si = width));
@@ -262,13 +264,12 @@ int bimamba2_chunk_for(const bimamba2_params *p, int training) {
         rows(q.x, q.x_sb, q.x_sl, q.x_sh, p->nheads, P);
         rows(q.Bm, q.B_sb, q.B_sl, q.B_sg, p->ngroups, N);
         rows(q.Cm, q.C_sb, q.C_sl, q.C_sg, p->ngroups, N);
-        if (!training) return chunk_scan_uses_scan16(&q, false);
-        if (N == 64) return scan_recomputes_cb(&q, false) && scan_recomputes_cb(&q, true) && dcb_recomputes_cb(&q);
-        return chunk_state_does_cumsum(&q) && dcb_recomputes_cb(&q);
-    };
-    if ((N == 64 || !training || P == 128 || p->nheads >= 8 * p->ngroups) && whole())
-        return std::max(Q, workgroups(256, 64) >= CUS / 2 ? 256 : workgroups(128, 64) >= CUS / 8 ? 128 : Q);
-    if (Q <= 128) return workgroups(128, 64) >= CUS / 4 ? 128 : Q;
+        if (chunk_scan_uses_scan16(&q, false))
+            return std::max(Q, workgroups(256, 64) >= CUS / 2 ? 256 : workgroups(128, 64) >= CUS / 8 ? 128 : Q);
+    }
+    // (in chunks that are no multiples of 64 such a pass keeps its states in float32)
+    if (training && N == 64 && P % 64 == 0 && Q % 64) return Q;
+    if (Q <= 128) return workgroups(128, 64) >= (wide ? CUS / 8 : CUS / 4) ? 128 : Q;
     bimamba2_params q = *p;
     q.chunk_size = 128;
     const bool exact_states = !(P % 64 == 0 && N % 64 == 0) && chunk_state_narrow(&q, false) && chunk_state_narrow(&q, true);

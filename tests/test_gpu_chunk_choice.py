@@ -18,7 +18,7 @@ REL = {torch.float32: 2e-5, torch.bfloat16: 1e-2, torch.float16: 2e-3}
     (2, 260, 64, 32, 1, 16, 256, 128, torch.float32, False, False),      # down to 128
     (1, 300, 6, 32, 2, 32, 256, 128, torch.bfloat16, True, False),       # another 16-bit shape: down
     (2, 257, 64, 16, 8, 80, 64, 128, torch.float16, True, False),        # and up, dstate no multiple of 32
-    (2, 520, 64, 64, 8, 64, 64, 256, torch.bfloat16, True, False),       # kernels that rebuild C.B^T: up
+    (2, 520, 64, 64, 8, 64, 64, 128, torch.bfloat16, True, False),       # kernels that rebuild C.B^T: up
     (2, 300, 64, 64, 64, 128, 64, 128, torch.bfloat16, False, False),    # state dimension 128 with one head a group
     (2, 300, 64, 16, 8, 16, 64, 128, torch.bfloat16, False, True),       # packed sequences
 ])
@@ -44,6 +44,37 @@ def test_results_do_not_depend_on_the_choice(monkeypatch, b, L, H, P, G, N, Q, r
         for name, g, w in zip(["out"] + names, got, want):
             err = (g.double() - w).norm() / w.norm()
             assert err < REL[dtype], (name, float(err))
+
+
+@pytest.mark.parametrize("L,H,P,G,N,Q,dtype", [
+    (520, 128, 64, 8, 64, 64, torch.bfloat16), (300, 128, 64, 1, 128, 64, torch.bfloat16), (300, 128, 64, 2, 64, 64, torch.float16), (520, 128, 64, 8, 64, 160, torch.float16),
+    (300, 128, 64, 1, 64, 96, torch.float16), (300, 128, 32, 2, 32, 256, torch.bfloat16), (300, 128, 16, 8, 16, 256, torch.float16), (300, 128, 16, 2, 16, 256, torch.float32)])
+def test_no_result_is_further_off_than_in_the_chunks_asked_for(monkeypatch, L, H, P, G, N, Q, dtype):
+    """errors against float64 in the chunks that the rule takes over those in the caller's, of a pass with and one without gradients.
+    Tensors of tens of thousands of elements and more agree to a percent, with float16's 0.4 % for chunks twice as long; dA and ddt_bias
+    have 256 values here, and two root mean squares of 256 independent errors differ by 1 / sqrt(256) = 6 %: 2.5 times that.  (dD takes
+    the same sums over a chunk's positions whatever the chunks are.)"""
+    from bi_mamba2_amd import ops
+    chosen, errors = ops._chunk_for, {}
+    monkeypatch.setattr(ops, "KEEP_FORWARD_INTERMEDIATES", False)
+    for seed in (0, 1):
+        d = {k: None if v is None else v.cuda().requires_grad_(True) for k, v in make_case(1, L, H, P, G, N, dtype, with_z=True, seed=seed).items()}
+        dout = torch.randn(1, L, H, P, generator=torch.Generator().manual_seed(seed)).to(dtype).cuda()
+        r = {k: v.detach().double().requires_grad_(True) for k, v in d.items()}
+        want = O.bimamba2_sequential(r["x"], r["dt"], r["A"], r["B"], r["C"], D=r["D"], z=r["z"], dt_bias=r["dt_bias"], dt_softplus=True)[0]
+        want = (want.detach(),) * 2 + torch.autograd.grad(want, list(r.values()), dout.double())
+        for side, rule in ((0, chosen), (1, lambda x, dt, A, B, C, chunk_size, *a: chunk_size)):
+            monkeypatch.setattr(ops, "_chunk_for", rule)
+            call = lambda: ops.bimamba_chunk_scan_combined(d["x"], d["dt"], d["A"], d["B"], d["C"], Q, D=d["D"], z=d["z"], dt_bias=d["dt_bias"], dt_softplus=True)
+            with torch.no_grad():
+                alone = call()
+            out = call()
+            got = (alone, out.detach()) + torch.autograd.grad(out, list(d.values()), dout)
+            for name, g, w in zip(["out without gradients", "out"] + list(d), got, want):
+                errors.setdefault(name, [0.0, 0.0])[side] += float((g.double() - w).norm() ** 2 / w.norm() ** 2)
+    for name, (ours, asked) in errors.items():
+        if name != "D":
+            assert ours ** 0.5 <= (1.15 if name in ("A", "dt_bias") else 1.01) * asked ** 0.5, (name, ours ** 0.5, asked ** 0.5)
 
 
 @pytest.mark.parametrize("odd", [(), ("x",), ("B",), ("dout",)])

@@ -269,13 +269,14 @@ def test_workspace_sizes_are_kept_apart_by_what_the_slices_depend_on():
     # float32: down to 128 where that fills the chip, else to 64; never up
     (2, 1111, 16, 64, 2, 64, "F32", 1, 256, 128), (1, 4096, 4, 32, 1, 16, "F32", 1, 256, 128), (1, 4064, 4, 32, 1, 16, "F32", 0, 256, 64),
     (1, 100, 1, 16, 1, 16, "F32", 0, 128, 64), (4, 2048, 16, 64, 1, 64, "F32", 1, 64, 64), (4, 2048, 16, 64, 1, 64, "F32", 1, 32, 32),
-    # kernels that rebuild C.B^T: up to 256 or 128 where that leaves enough workgroups; never down
-    (4, 2048, 16, 64, 1, 64, "BF16", 1, 64, 256), (4, 2048, 15, 64, 1, 64, "BF16", 1, 64, 128), (1, 512, 8, 64, 1, 64, "BF16", 1, 64, 128),
+    # wide heads: up to 256 (without gradients) or 128 where that leaves enough workgroups; never down
+    (4, 2048, 16, 64, 1, 64, "BF16", 0, 64, 256), (4, 2048, 16, 64, 1, 64, "BF16", 1, 64, 128), (4, 2048, 15, 64, 1, 64, "BF16", 0, 64, 128), (1, 512, 8, 64, 1, 64, "BF16", 1, 64, 128),
     (1, 508, 8, 64, 1, 64, "BF16", 1, 64, 64), (1, 300, 4, 64, 1, 64, "F16", 0, 64, 64),
-    (1, 300, 4, 64, 1, 64, "F16", 0, 256, 256), (4, 2048, 8, 128, 1, 64, "F16", 1, 128, 256), (4, 136, 8, 128, 2, 128, "BF16", 0, 64, 64),
-    # state dimension 128: training with few heads of 64 in a group goes up to 128 at most, and not down (one-part chunk states)
-    (4, 2048, 16, 64, 8, 128, "BF16", 0, 64, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 256, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 64, 128), (4, 2048, 16, 64, 2, 128, "BF16", 1, 64, 256),
-    (4, 2048, 16, 128, 8, 128, "BF16", 1, 64, 256),
+    (1, 300, 4, 64, 1, 64, "F16", 0, 256, 256), (4, 2048, 8, 128, 1, 64, "F16", 0, 128, 256), (4, 2048, 8, 128, 1, 64, "F16", 1, 128, 128), (4, 2048, 8, 128, 1, 64, "F16", 1, 192, 192), (4, 136, 8, 128, 2, 128, "BF16", 0, 64, 64),
+    (4, 2048, 16, 64, 8, 128, "BF16", 0, 64, 256), (4, 2048, 16, 64, 8, 128, "BF16", 1, 256, 256), (4, 2048, 16, 64, 2, 128, "BF16", 1, 64, 128),
+    (4, 2048, 16, 128, 8, 128, "BF16", 1, 64, 128), (1, 1024, 4, 64, 1, 128, "BF16", 1, 64, 128), (1, 1023, 4, 64, 1, 64, "BF16", 1, 64, 64),
+    # ... and in training from multiples of 64 only at state dimension 64 (other sizes keep its states in float32)
+    (4, 2048, 16, 64, 1, 64, "F16", 1, 96, 96), (4, 2048, 16, 64, 1, 64, "F16", 1, 160, 160), (4, 2048, 16, 64, 1, 64, "F16", 0, 160, 256), (4, 2048, 16, 64, 1, 128, "F16", 1, 96, 128),
     # the other 16-bit shapes: 128, from below only where that fills the chip
     (1, 300, 4, 16, 1, 16, "BF16", 1, 256, 128), (1, 300, 4, 16, 1, 16, "BF16", 1, 64, 64), (4, 1024, 8, 32, 1, 16, "BF16", 0, 64, 128), (4, 1016, 8, 32, 1, 16, "BF16", 0, 64, 64),
     (4, 1024, 8, 96, 1, 64, "BF16", 0, 224, 128), (4, 1024, 8, 64, 1, 80, "F16", 1, 32, 128),
@@ -332,17 +333,17 @@ def test_initial_states_count_as_training():
 @pytest.mark.parametrize("heads,headdim,groups,dstate", [(16, 64, 1, 64), (16, 64, 1, 128), (8, 128, 1, 64)])
 @pytest.mark.parametrize("training", [0, 1])
 def test_chunks_of_wide_heads_grow_only_where_their_kernels_run(heads, headdim, groups, dstate, training):
-    """4 x 2048 in bfloat16, chunks of 128 asked for: 256 with the kernels for aligned rows, as asked with those for any rows"""
+    """4 x 2048 in bfloat16, chunks of 128 asked for, without gradients: 256 with the kernel for aligned rows, as asked with those for any rows"""
     lib, named = _lib.load(), dict(x=256, Bm=256, Cm=256, z=256, has_z=1)
 
     def chosen(**kw):
         p = _contiguous(4, 2048, heads, headdim, groups, dstate, 128, _lib.BF16)
         z = {"z" + k[1:]: v for k, v in p.items() if k.startswith("x_")}
         return lib.bimamba2_chunk_for(ctypes.byref(_params(**{**p, **z, **named, **kw})), training)
-    assert chosen() == 256 and chosen(x_sl=heads * headdim + 8, B_sl=2 * groups * dstate) == 256
-    assert lib.bimamba2_chunk_for(ctypes.byref(_params(**_contiguous(4, 2048, heads, headdim, groups, dstate, 128, _lib.BF16))), training) == 256
+    grown = 128 if training else 256
+    assert chosen() == grown and chosen(x_sl=heads * headdim + 8, B_sl=2 * groups * dstate) == grown
+    assert lib.bimamba2_chunk_for(ctypes.byref(_params(**_contiguous(4, 2048, heads, headdim, groups, dstate, 128, _lib.BF16))), training) == grown
     for odd in (dict(x=258), dict(Bm=264), dict(Cm=258), dict(x_sl=heads * headdim + 4), dict(B_sl=groups * dstate + 1), dict(C_sb=4097)):
         assert chosen(**odd) == 128, odd
-    if dstate == 64 or not training:           # (the scan kernel that rebuilds C.B^T)
-        assert chosen(z=258) == 128 and chosen(z_sl=heads * headdim + 2) == 128 and chosen(B_sl=1 << 22) == 128
+    assert chosen(z=258) == 128 and chosen(z_sl=heads * headdim + 2) == 128 and chosen(B_sl=1 << 22) == 128
 
