@@ -233,8 +233,8 @@ int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd) {
 //    2.013e-3 / 2.023e-3 / 2.048e-3), most of it from the states in 16 bits (float16, 520 positions, 16 heads: 3.03e-4 / 3.02e-4 / 3.01e-4).
 //    A pass with gradients grows to 128 at most: the last launch of chunks of 256 takes dCB rounded to 16 bits, that of up to 128 in two
 //    parts, and dB and dC are 14 to 21 % further off in 256 (2.40e-3 against 2.89e-3 at any number of heads, groups and both state
-//    dimensions), for 3 to 8 % of the time at dstate 64 and 3 to 13 % at 128 (4 x 4096, 32 heads in 8 groups 617 / 584; 2 x 2048, 8 heads of 128,
-//    dstate 128 177 / 172).  In chunks that are no multiples of 64 its states stay in float32 at dstate 64: they are kept (float16, 640
+//    dimensions), for 3 to 8 % of the time at dstate 64 and 3 to 21 % at 128 (4 x 4096, 32 heads in 8 groups 617 / 584; dstate 128, 2 x 2048,
+//    8 heads of 128 177 / 172, 2 x 7236, 42 heads of 64 1334 / 1102).  In chunks that are no multiples of 64 its states stay in float32 at dstate 64: they are kept (float16, 640
 //    positions, 16 heads: out 2.58e-4 in chunks of 160, 3.08e-4 in 128).
 //  * other 16-bit shapes, 64 / 128, heads of 32, dstate 32: 1024, 8 heads (64) 22 / 24, 61 / 67, four rows 26 / 25, 89 / 84; 2048, 8 heads (128) 25 / 25,
 //    79 / 79; 2048, 24 heads (384) 34 / 29, 114 / 106; 512, 8 heads (32) 21 / 23, 57 / 64, sixteen rows 38 / 31, 116 / 101.  128 and 256: 41 / 45, 145 / 194 (4 x

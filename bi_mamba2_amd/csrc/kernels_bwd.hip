@@ -71,7 +71,7 @@ int launch_reduce_jobs(const ReduceJobs &jobs, hipStream_t stream) {
 // The sums of a layer's backward pass in one launch, each in its parameter's type: those of the norm's weight, of the convolution's
 // filter and bias, of A, D and dt_bias, and what were a conversion of each afterwards.  Every one of them is a launch of 4 to 7 us
 // of which the chip is busy for less than one.  16 x 1024 positions, d_model 768, bfloat16: 24 -> 11 us,
-// the layer 904 -> 892; 4 x 2000, 640: 554 -> 540; 16 x 4000, 256: 969 -> 950.
+// the layer 938 -> 930 (two runs of one build differ by 1); 4 x 2000, 640: 554 -> 540; 16 x 4000, 256: 969 -> 950.
 struct SumTarget { void *out; const float *mul; int dtype; };
 struct SumArgs {
     ColumnSums cols[3];
