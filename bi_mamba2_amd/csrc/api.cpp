@@ -241,7 +241,11 @@ int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd) {
 //    2048, 16 heads); 8 groups, 4 x 4096, 32 heads 149 / 178, 580 / 784; 4 x 1024, 8 heads 20 / 34, 117 / 136; 2 x 512 19 / 32.  Below the
 //    caller's chunk only where the chunk states take their weighted operand in two 16-bit parts: with one, dA was 5 to 32 % further from
 //    float64 in chunks of 128 than of 256 (900 positions, 8 heads, 400 inputs); with two no output is (dA -0.3 to -7 %, out -0.4 to
-//    -0.8 %, dB and dC -18 to -28 %).
+//    -0.8 %, dB and dC -18 to -28 %).  Nor in training without a gate where one chunk, or little more, holds the sequence: dA is made of
+//    products of the operands themselves within a chunk, and only what crosses a boundary has been rounded (200 positions, 64 heads of 64 in 8 groups,
+//    dstate 32, bfloat16: 1.2e-6 in chunks of 256, 7.3e-4 in 128; 257 three times as far off in 128, 270 1.3, 288 1.1, 320 and 384 1.0, 512 1.1, 900 0.84
+//    times; with a gate, whose product with the gradient is rounded, 1.0 at all of them).  128 / 256 there, heads of 32, dstate 16: 200 positions, 8
+//    heads 63 / 106, sixteen rows 78 / 132; 24 heads of 64, dstate 32 142 / 188.
 int bimamba2_chunk_for(const bimamba2_params *p, int training) {
     if (check_problem(p)) return p ? p->chunk_size : 0;
     const int Q = p->chunk_size, P = p->headdim, N = p->dstate;
@@ -270,6 +274,8 @@ int bimamba2_chunk_for(const bimamba2_params *p, int training) {
     // (in chunks that are no multiples of 64 such a pass keeps its states in float32)
     if (training && N == 64 && P % 64 == 0 && Q % 64) return Q;
     if (Q <= 128) return workgroups(128, 64) >= (wide ? CUS / 8 : CUS / 4) ? 128 : Q;
+    // (a sequence that one chunk holds, or little more, in training without a gate: see above)
+    if (training && !p->has_z && p->seqlen > 128 && 4 * (int64_t)p->seqlen < 5 * (int64_t)Q) return Q;
     bimamba2_params q = *p;
     q.chunk_size = 128;
     const bool exact_states = !(P % 64 == 0 && N % 64 == 0) && chunk_state_narrow(&q, false) && chunk_state_narrow(&q, true);

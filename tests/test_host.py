@@ -278,10 +278,13 @@ def test_workspace_sizes_are_kept_apart_by_what_the_slices_depend_on():
     # ... and in training from multiples of 64 only at state dimension 64 (other sizes keep its states in float32)
     (4, 2048, 16, 64, 1, 64, "F16", 1, 96, 96), (4, 2048, 16, 64, 1, 64, "F16", 1, 160, 160), (4, 2048, 16, 64, 1, 64, "F16", 0, 160, 256), (4, 2048, 16, 64, 1, 128, "F16", 1, 96, 128),
     # the other 16-bit shapes: 128, from below only where that fills the chip
-    (1, 300, 4, 16, 1, 16, "BF16", 1, 256, 128), (1, 300, 4, 16, 1, 16, "BF16", 1, 64, 64), (4, 1024, 8, 32, 1, 16, "BF16", 0, 64, 128), (4, 1016, 8, 32, 1, 16, "BF16", 0, 64, 64),
+    (1, 320, 4, 16, 1, 16, "BF16", 1, 256, 128), (1, 300, 4, 16, 1, 16, "BF16", 1, 64, 64), (4, 1024, 8, 32, 1, 16, "BF16", 0, 64, 128), (4, 1016, 8, 32, 1, 16, "BF16", 0, 64, 64),
     (4, 1024, 8, 96, 1, 64, "BF16", 0, 224, 128), (4, 1024, 8, 64, 1, 80, "F16", 1, 32, 128),
     # ... and from above only where the chunk states take their weighted operand in two parts
     (1, 300, 4, 20, 1, 16, "BF16", 1, 256, 256), (1, 300, 4, 16, 1, 20, "BF16", 0, 256, 256), (1, 300, 4, 64, 1, 192, "F16", 0, 256, 256),
+    # ... nor in training without a gate where the sequence is hardly longer than one chunk and does not fit into 128
+    (1, 319, 4, 16, 1, 16, "BF16", 1, 256, 256), (1, 129, 4, 16, 1, 16, "BF16", 1, 256, 256), (1, 128, 4, 16, 1, 16, "BF16", 1, 256, 128), (1, 129, 4, 16, 1, 16, "BF16", 0, 256, 128),
+    (1, 199, 4, 16, 1, 16, "F16", 1, 160, 160), (1, 200, 4, 16, 1, 16, "F16", 1, 160, 128),
     # sizes that are no whole steps of the kernels stay
     (4, 2048, 16, 64, 1, 64, "F32", 1, 200, 200), (4, 2048, 16, 16, 1, 64, "BF16", 1, 33, 33),
 ])
@@ -291,6 +294,10 @@ def test_chunk_size_that_the_kernels_run_with(batch, seqlen, heads, headdim, gro
     assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == runs
     for p.batch in (1, 2, 64, batch):                                          # (a row runs as it would alone)
         assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == runs
+    if training and dtype != "F32" and 128 < seqlen < 1.25 * chunk and runs == chunk and headdim == dstate == 16:
+        p.has_z = 1
+        assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == 128
+        p.has_z = 0
     p.causal = 1                                                               # (the comparator runs as it is asked to)
     assert lib.bimamba2_chunk_for(ctypes.byref(p), training) == chunk
     p.causal, p.seq_idx = 0, 4096
