@@ -186,8 +186,8 @@ int bimamba2_seq_boundaries(const bimamba2_params *p, int32_t *counts);
 
 /* The chunk size to run the problem of `p` with where a caller asks for p->chunk_size but only wants the result, which does not
  * depend on it: the faster one of 64, 128 and 256 where that is no less exact, else p->chunk_size.  training: a backward pass
- * follows.  Reads the sizes other than batch, dtype, causal and seq_idx of `p` and, where they are set, the operands' strides and
- * alignment: a row of a batch runs in the chunks that it would run in alone.  No counterpart in the reference. */
+ * follows.  Reads the sizes other than batch, dtype, has_z, causal and seq_idx of `p` and, where they are set, the operands' strides
+ * and alignment: a row of a batch runs in the chunks that it would run in alone.  No counterpart in the reference. */
 int bimamba2_chunk_for(const bimamba2_params *p, int training);
 
 /* 1 if the kernels of this problem can keep the entering states in 16-bit copies (see states16_f), else 0 */
