@@ -301,7 +301,8 @@ __device__ __forceinline__ void bwd_dcb_body(const bimamba2_params &p, int nc, i
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// Variant for 16-bit types with headdim % 8 == 0, chunk_size % 64 == 0 and aligned operands.
+// Variant for 16-bit types with headdim % 8 == 0, chunk_size % 64 == 0 and aligned operands (heads of 64: dcb_heads_body.hpp, but for the
+// launches of several roles).
 //
 // The kernel is bound by its instruction count, not by memory, so everything per head is pared down:
 //  * the dout tile, the x tile and the decay vectors of each (head, KC-wide headdim chunk) step travel from global memory
@@ -325,7 +326,6 @@ __device__ __forceinline__ float lanegroup_sum_mfma(float v) {
 // Slots of the ring.  Two (the step being multiplied and the one after it, requested right after the barrier that frees
 // its slot) measured 60 us against 62 us for three slots requested two steps ahead.
 constexpr int DCB_RING = 2;
-constexpr int DCB_RESIDENT_BLOCKS = 1024;                 // a dCB grid up to this size is on the chip all at once
 constexpr int DCB_PART_B = 10 * 64 * 4;                   // per-wave column sums (f: 0-3, b: 4-7), row sums (f: 8, b: 9)
 
 
@@ -333,13 +333,13 @@ constexpr int DCB_PART_B = 10 * 64 * 4;                   // per-wave column sum
 // bid / gdx / gdz: block index and grid extents (x: batch * chunks * groups, y: tiles, z: head slices)
 // Which (batch, chunk, group) and which tile the id-th workgroup of the dCB grid takes.  Workgroups are dealt round-robin to
 // the 8 XCDs in id order, and the tiles of one (b, c, g) read the same dout and x rows (each row tile four times at chunk
-// 256), so they belong on one XCD, close in time.  A grid that is resident all at once (two or three workgroups per CU)
-// has (b, c, g) fastest: equal ids modulo 8 share an XCD, and all diagonal tiles, which cost more, come first and spread
+// 256), so they belong on one XCD, close in time.  A grid that is resident all at once (up to
+// `resident` workgroups) has (b, c, g) fastest: equal ids modulo 8 share an XCD, and all diagonal tiles, which cost more, come first and spread
 // over the CUs.  A larger grid runs in several rounds, and with that order a row tile's readers are rounds apart and
 // each fetches it from memory again (768 MB of reads at 8 groups of 4 heads, batch 4 x 4096; 172 -> 155 us): there
 // eight (b, c, g) at a time, one per XCD, go through all their tiles before the next eight start.
-__device__ __forceinline__ BlockId dcb_block_of(int id, int gdx, int ntiles, int nblocks) {
-    if (nblocks <= DCB_RESIDENT_BLOCKS || gdx % 8) return BlockId{id % gdx, id / gdx, 0};
+__device__ __forceinline__ BlockId dcb_block_of(int id, int gdx, int ntiles, int nblocks, int resident = 1024) {
+    if (nblocks <= resident || gdx % 8) return BlockId{id % gdx, id / gdx, 0};
     const int k = id >> 3;
     return BlockId{(k / ntiles) * 8 + (id & 7), k % ntiles, 0};
 }

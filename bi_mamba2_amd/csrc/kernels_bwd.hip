@@ -14,6 +14,7 @@
 #include "bmm_fwd_body.hpp"
 #include "dbdc_body.hpp"
 #include "dcb_body.hpp"
+#include "dcb_heads_body.hpp"
 
 namespace bm2 {
 
@@ -1014,19 +1015,30 @@ __global__ __launch_bounds__(NTHREADS) void bwd_dcb_ring_kernel(const bimamba2_p
     bwd_dcb_ring_body<T, UNI, KC, WHOLE>(p, nc, nqt, bid, gridDim.x, gridDim.z, smem);
 }
 
-// The dCB kernel and the backward state passing as roles of one launch: the first is bound by instruction issue and moves little data, the second streams
-// 70 MB and needs few instructions, and the two depend on different kernels before them.  The first ndcb blocks are the
-// dCB tiles in the order of their own grid (so they are placed first, two per CU as when alone), the rest are the state
-// passing's blocks, which take what is left of each CU.
-template <typename T, bool UNI>
-__device__ __forceinline__ void bwd_dcb_sp_body(const bimamba2_params &p, int nc, int nqt, int gdx, int ndcb, int nslices, int nsplit, int ndir, bool out16) {
-    const int id = blockIdx.x;
+template <typename T, bool UNI, int W>
+__global__ __launch_bounds__(NTHREADS, 2) void bwd_dcb_heads_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int gdy, int gdz) {
+    __shared__ __attribute__((aligned(16))) unsigned char smem[DcbHeadsMap<W>::LDS];
+    const int id = blockIdx.x, per = gdx * gdy;
+    BlockId bid = dcb_block_of(id % per, gdx, gdy, per, DCB_HEADS_RESIDENT);
+    bid.z = id / per;
+    bwd_dcb_heads_body<T, UNI, W>(p, nc, nqt, bid, gdx, gdz, smem, false);
+}
+
+// The dCB kernel and the backward state passing as roles of one launch: the first is bound by instruction issue and moves little data, the
+// second streams 70 MB and needs few instructions, and the two depend on different kernels before them.  The first ndcb blocks are the
+// dCB tiles, the rest are the state passing's, which take the places that the tiles leave one after the other: heads of 64, 45 us for both
+// against 41 + 13 in two launches (4 x 2048, 32 heads), 121 against 109 + 23 (4 x 4096, 8 groups); with the state passing's blocks first
+// 50 and 122, and 47 against 34 at dstate 128 (2 x 3001, 24 heads).
+// W: the waves that share a tile in the kernel above (gdy: workgroups a (b, c, g)); 0: the ring, a tile a workgroup
+template <typename T, bool UNI, int W>
+__global__ __launch_bounds__(NTHREADS, W ? 2 : 1) void bwd_dcb_sp_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int gdy, int gdz, int nsplit, int ndir, bool out16) {
+    const int id = blockIdx.x, per = gdx * gdy, ndcb = per * gdz;
     if (id < ndcb) {
-        __shared__ __attribute__((aligned(16))) unsigned char smem[DcbRingMap<64>::LDS];
-        const int ntiles = gdx * nqt * nqt;
-        BlockId tile = dcb_block_of(id % ntiles, gdx, nqt * nqt, ntiles);
-        tile.z = id / ntiles;
-        bwd_dcb_ring_body<T, UNI, 64, true>(p, nc, nqt, tile, gdx, nslices, smem, out16);
+        __shared__ __attribute__((aligned(16))) unsigned char smem[W ? DcbHeadsMap<W ? W : 1>::LDS : DcbRingMap<64>::LDS];
+        BlockId tile = dcb_block_of(id % per, gdx, gdy, per, W ? DCB_HEADS_RESIDENT : 1024);
+        tile.z = id / per;
+        if constexpr (W > 0) bwd_dcb_heads_body<T, UNI, W>(p, nc, nqt, tile, gdx, gdz, smem, out16);
+        else bwd_dcb_ring_body<T, UNI, 64, true>(p, nc, nqt, tile, gdx, gdz, smem, out16);
     } else {
         const int k = id - ndcb;                  // grid (nsplit, nheads, batch * ndir) of the state passing
         const BlockId sb{k % nsplit, (k / nsplit) % p.nheads, k / (nsplit * p.nheads)};
@@ -1035,16 +1047,39 @@ __device__ __forceinline__ void bwd_dcb_sp_body(const bimamba2_params &p, int nc
         else state_passing_bwd_vec_body<T, true, true>(p, nc, nsplit, ndir, sb);
     }
 }
-
-template <typename T, bool UNI>
-__global__ __launch_bounds__(NTHREADS) void bwd_dcb_sp_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int ndcb, int nslices, int nsplit, int ndir, bool out16) {
-    bwd_dcb_sp_body<T, UNI>(p, nc, nqt, gdx, ndcb, nslices, nsplit, ndir, out16);
+// Waves that share a tile of the kernel above.  More of them split a tile's heads and finish sooner, fewer leave out the exchange at the end
+// and the repeated C.B^T and keep their requests under way over more heads.  What is compared is rounds of the 512 workgroups that the
+// chip holds times a workgroup's start and end (8 us) and heads (2.9 us each), and a tile to every wave pays for the unequal
+// tiles (those on the diagonal take longer) while there are few rounds.  us with 4 / 2 / 1 waves (heads of 64, dstate 64):
+//   512 tiles: 4 heads 12 / 14 / 19, 32 heads 34 / 51 / 90; 1024: 4 heads 20 / 16 / 20, 24 heads 47 / 45 / 70; 2048: 4 heads 37 / 27 / 27,
+//   24 heads 93 / 78 / 102; 4096: 2 heads 62 / 41 / 34, 8 heads 90 / 80 / 72; 8192: 4 heads 130 / 98 / 81, 8 heads 181 / 149 / 137
+static int dcb_waves(const bimamba2_params *p, int slices) {
+    const int nqt = (p->chunk_size + 63) / 64, heads = (p->nheads / p->ngroups + slices - 1) / slices;
+    const double tiles = (double)p->batch * nchunks(p) * p->ngroups * nqt * nqt * slices;
+    int best = 4;
+    double best_cost = 0;
+    for (int w = 4; w >= 1; w /= 2) {
+        const double full = tiles * w / (4 * DCB_HEADS_RESIDENT), rounds = (full + std::ceil(full)) / 2;      // (a last round that is nearly empty costs more than its share)
+        const double cost = (std::max(1.0, rounds) + (w == 1 ? 0.3 : 0.0)) * (8 + 2.9 * ((heads + w - 1) / w));
+        if (w == 4 || cost < best_cost) { best = w; best_cost = cost; }
+    }
+    return best;
+}
+template <typename T, bool UNI> static void launch_dcb_heads(const bimamba2_params *p, int nc, int nqt, int slices) {
+    const int W = dcb_waves(p, slices), gdx = p->batch * nc * p->ngroups, gdy = (nqt * nqt * W + 3) / 4;
+    const dim3 g(gdx * gdy * slices);
+    if (W == 4) hipLaunchKernelGGL((bwd_dcb_heads_kernel<T, UNI, 4>), g, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, gdy, slices);
+    else if (W == 2) hipLaunchKernelGGL((bwd_dcb_heads_kernel<T, UNI, 2>), g, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, gdy, slices);
+    else hipLaunchKernelGGL((bwd_dcb_heads_kernel<T, UNI, 1>), g, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, gdy, slices);
 }
 // Narrow heads (16-bit) take the ring as well: through registers a workgroup waits for its operands head by head.  4 x 2048 in chunks of
 // 128, 16 heads of 16: 46 -> 21 us; 48 heads of 16: the whole pass 497 -> 389 us; in 8 groups (two heads a tile) 43 -> 28 us.
 template <typename T> static void launch_dcb_ring(dim3 grid, const bimamba2_params *p, int nc, int nqt) {
     if constexpr (sizeof(T) == 2) {
-        if (p->causal) hipLaunchKernelGGL((bwd_dcb_ring_kernel<T, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
+        if (p->headdim == 64) {
+            if (p->causal) launch_dcb_heads<T, true>(p, nc, nqt, grid.z);
+            else launch_dcb_heads<T, false>(p, nc, nqt, grid.z);
+        } else if (p->causal) hipLaunchKernelGGL((bwd_dcb_ring_kernel<T, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
         else if (p->headdim <= 32) hipLaunchKernelGGL((bwd_dcb_ring_kernel<T, false, 32, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
         else if (p->headdim % 64) hipLaunchKernelGGL((bwd_dcb_ring_kernel<T, false, 64, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
         else hipLaunchKernelGGL((bwd_dcb_ring_kernel<T>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt);
@@ -1161,15 +1196,21 @@ bool bwd_dcb_sp_merged(const bimamba2_params *p) {
 int launch_bwd_dcb_sp(const bimamba2_params *p, bool out16) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, PN = p->headdim * p->dstate;
     const int nsplit = (PN + SP_EPT * NTHREADS - 1) / (SP_EPT * NTHREADS), ndir = p->causal ? 1 : 2;
-    const int slices = dcb_slices(p), gdx = p->batch * nc * p->ngroups, ndcb = gdx * nqt * nqt * slices, nsp = nsplit * p->nheads * p->batch * ndir;
-    dim3 grid(ndcb + nsp);
-#define BM2_DS(TT)                                                                                                                     \
-    do {                                                                                                                               \
-        if (p->causal) hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, ndcb, slices, nsplit, ndir, out16);  \
-        else hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, ndcb, slices, nsplit, ndir, out16);           \
+    const int slices = dcb_slices(p), W = p->headdim == 64 ? dcb_waves(p, slices) : 0;
+    const int gdx = p->batch * nc * p->ngroups, gdy = W ? (nqt * nqt * W + 3) / 4 : nqt * nqt, nsp = nsplit * p->nheads * p->batch * ndir;
+    dim3 grid(gdx * gdy * slices + nsp);
+#define BM2_D(TT, UNI, WV) hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, UNI, WV>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, gdy, slices, nsplit, ndir, out16)
+#define BM2_DS(TT, UNI)                \
+    do {                               \
+        if (W == 4) BM2_D(TT, UNI, 4); \
+        else if (W == 2) BM2_D(TT, UNI, 2); \
+        else if (W == 1) BM2_D(TT, UNI, 1); \
+        else BM2_D(TT, UNI, 0);        \
     } while (0)
-    if (p->dtype == BIMAMBA2_BF16) BM2_DS(bf16_t); else BM2_DS(f16_t);
+    if (p->dtype == BIMAMBA2_BF16) { if (p->causal) BM2_DS(bf16_t, true); else BM2_DS(bf16_t, false); }
+    else { if (p->causal) BM2_DS(f16_t, true); else BM2_DS(f16_t, false); }
 #undef BM2_DS
+#undef BM2_D
     return check_launch();
 }
 

@@ -233,6 +233,25 @@ def test_dcb_of_heads_that_are_no_whole_steps(ops, P, L, Q, dtype):
         assert float((g - w).norm() / w.norm()) < 4e-6
 
 
+@pytest.mark.parametrize("b,H,G,P,L,Q,dtype", [
+    (1, 5, 1, 64, 65, 64, torch.bfloat16),        # few tiles: four waves share one, one of them with two heads; one row in the last chunk
+    (1, 3, 1, 64, 449, 256, torch.float16),       # fewer heads than waves, a ragged tile on the diagonal
+    (16, 6, 2, 64, 1030, 128, torch.bfloat16),    # 1152 tiles of 3 heads: two waves a tile
+    (16, 16, 8, 64, 1030, 64, torch.float16),     # 2176 tiles of 2 heads: one wave a tile
+    (4, 9, 9, 64, 1030, 256, torch.bfloat16),     # 2880 tiles of 1 head
+])
+def test_dcb_by_waves_that_share_a_tile(ops, b, H, G, P, L, Q, dtype):
+    """4, 2 or 1 waves take the heads of a tile in turn (bounds as in the test above); rows behind the end of the sequence count nothing"""
+    d = to_dev(make_case(b, L, H, P, G, 16, dtype))
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(5)).to(dtype).cuda()
+    csf, csb, dt = ops._chunk_cumsum_fwd(d["dt"], d["A"], Q, dt_bias=d["dt_bias"], dt_softplus=True)
+    CB = torch.randn(b, -(-L // Q), G, Q, Q, generator=torch.Generator().manual_seed(6)).cuda()
+    want = ops._chunk_scan_bwd_dcb(d["x"].float(), dt, csf, csb, dout.float(), CB, ngroups=G)
+    got = ops._chunk_scan_bwd_dcb(d["x"], dt, csf, csb, dout, CB, ngroups=G)
+    for g, w in zip(got, want):
+        assert float((g - w).norm() / w.norm()) < 4e-6
+
+
 @pytest.mark.parametrize("N", [8, 16, 20, 32, 36, 64])
 @pytest.mark.parametrize("H,G,P,L,Q,dtype", [(6, 2, 16, 130, 128, torch.bfloat16), (8, 1, 72, 75, 64, torch.float32), (3, 3, 32, 257, 256, torch.float16)])
 def test_state_parts_of_db_and_dc_with_narrow_states(ops, N, H, G, P, L, Q, dtype):
