@@ -334,125 +334,170 @@ constexpr int SP_CH = 8;
 // SP_FLUSH chunks instead of every SP_CH (a barrier waits for the loads in flight): the launch of its own, whose workgroups have nothing
 // else to cover a round trip with.  As a role beside dCB the kernel keeps to that one's registers and LDS.
 constexpr int SP_FLUSH = 64;
-template <typename T16, bool PREV16, bool DS16, bool DP16 = false, bool AHEAD = false>
-__device__ __forceinline__ void state_passing_bwd_vec_body(const bimamba2_params &p, int nc, int nsplit, int ndir, BlockId bid) {
+// A workgroup takes one or several groups of SP_EPT * NTHREADS elements of a head.  Bound by the time of its one round trip to memory, so what
+// counts is how much it asks for at once.  Short sequences: several groups, so that all its loads in flight are of use (with
+// one group, and the loads behind the last chunk repeating it, a pass over one chunk asked eight times for everything).  As a role
+// of the dCB launch, which has room for two of these a CU: two groups of long sequences too.  Both roles, heads of 64, bfloat16: 32 x 256, 24 heads,
+// one chunk 60 -> 37 us; 16 x 512, 24 heads, 2 chunks 46 -> 36; 16 x 1024, 24 heads, 4 chunks 71 -> 64; 4 x 2048, 32 heads, 8 chunks 49 -> 43; 4 x 4096, 8
+// groups, 16 chunks 129 -> 125; dstate 128, 2 x 3001, 24 heads 36 -> 34.
+inline int sp_bwd_groups(int nc) { return nc <= 2 ? 4 : nc <= 4 ? 2 : 1; }
+template <typename T16, bool PREV16, bool DS16, bool DP16, bool AHEAD, int NCH, int NG>
+__device__ __forceinline__ void state_passing_bwd_groups(const bimamba2_params &p, int nc, int nsplit, int ndir, BlockId bid) {
     struct alignas(8) V4 { T16 v[4]; };
-    constexpr int FLUSH = AHEAD ? SP_FLUSH : SP_CH;
+    constexpr int NU = NCH * NG, FLUSH = AHEAD && NG == 1 ? SP_FLUSH : NU > SP_CH ? NU : SP_CH;
     __shared__ float red[FLUSH][4];
     const int PN = p.headdim * p.dstate;
-    const int split = bid.x, h = bid.y, b = bid.z / ndir, dir = bid.z % ndir;   // ndir = 1: forward direction only
+    const int split = bid.x * NG, h = bid.y, b = bid.z / ndir, dir = bid.z % ndir;   // ndir = 1: forward direction only
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int Q = p.chunk_size;
     const float *cs = (dir == 0 ? p.cs_f : p.cs_b) + ((int64_t)b * p.nheads + h) * nc * Q + (dir == 0 ? Q - 1 : 0);
     const int64_t cstride = (int64_t)p.nheads * PN;
     const int64_t base = ((int64_t)b * nc * p.nheads + h) * PN;
-    const int e_own = (split * NTHREADS + threadIdx.x) * SP_EPT;
-    const bool live = e_own < PN;
-    const int e = live ? e_own : PN - SP_EPT;              // loads are unconditional (so that they all go out together)
-    const float *prev = (dir == 0 ? p.states_f : p.states_b) + base + e;
-    const T16 *prev16 = reinterpret_cast<const T16 *>(dir == 0 ? p.states16_f : p.states16_b) + base + e;
-    float *ds = (dir == 0 ? p.dstates_f : p.dstates_b) + base + e;
-    T16 *ds16 = reinterpret_cast<T16 *>(dir == 0 ? p.dstates16_f : p.dstates16_b) + base + e;
+    const float *prev = (dir == 0 ? p.states_f : p.states_b) + base;
+    const T16 *prev16 = reinterpret_cast<const T16 *>(dir == 0 ? p.states16_f : p.states16_b) + base;
+    float *ds = (dir == 0 ? p.dstates_f : p.dstates_b) + base;
+    T16 *ds16 = reinterpret_cast<T16 *>(dir == 0 ? p.dstates16_f : p.dstates16_b) + base;
     float *dda = (dir == 0 ? p.ddA_chunk_f : p.ddA_chunk_b) + ((int64_t)b * p.nheads + h) * nc * nsplit + split;
     const float *dfin = dir == 0 ? p.dfinal_f : p.dfinal_b;
     float *dini = dir == 0 ? p.dinitial_f : p.dinitial_b;
-    const int64_t bh = ((int64_t)b * p.nheads + h) * PN + e;
-    f32x4 g = {0.f, 0.f, 0.f, 0.f};
-    if (dfin) g = *reinterpret_cast<const f32x4 *>(dfin + bh);
-    struct Batch { f32x4 dp[SP_CH], pv[SP_CH]; float dec[SP_CH]; };
+    const int64_t bh = ((int64_t)b * p.nheads + h) * PN;
+    bool live[NG];
+    int e[NG];
+    f32x4 g[NG];
+#pragma unroll
+    for (int u = 0; u < NG; ++u) {
+        const int own = ((split + u) * NTHREADS + threadIdx.x) * SP_EPT;
+        live[u] = own < PN;
+        e[u] = live[u] ? own : PN - SP_EPT;                // loads are unconditional (so that they all go out together)
+        g[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (dfin) g[u] = *reinterpret_cast<const f32x4 *>(dfin + bh + e[u]);
+    }
+    // the gradient of the recurrence's last chunk leads to the initial states only: without them its neighbour is read in its place
+    const int last = dini || nc == 1 ? nc - 1 : nc - 2;
+    // (as they lie in memory, converted where they are used: a conversion beside its load waits for it, and the loads went out one by one)
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    struct Batch {
+        typename std::conditional<DP16, f32x2, f32x4>::type dp[NU];
+        typename std::conditional<PREV16, f32x2, f32x4>::type pv[NU];
+        float dec[NCH];
+    };
+    auto wide = [](auto v) __attribute__((always_inline)) {
+        if constexpr (sizeof(v) == 16) return v;
+        else {
+            const V4 t = __builtin_bit_cast(V4, v);
+            return f32x4{to_f(t.v[0]), to_f(t.v[1]), to_f(t.v[2]), to_f(t.v[3])};
+        }
+    };
     auto load = [&](int s0, Batch &r) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < SP_CH; ++j) {
+        for (int j = 0; j < NCH; ++j) {
             const int sj = min(s0 + j, nc - 1);            // past the last chunk: a valid chunk again, never used
             const int c = dir == 0 ? nc - 1 - sj : sj;
             r.dec[j] = cs[(int64_t)c * Q];
-            // (both are read for the last time in the pass: past the caches)
-            if constexpr (DP16) {
-                const V4 t = *reinterpret_cast<const V4 *>(ds16 + c * cstride);
+            const int sd = min(sj, last);
+            const int64_t od = (dir == 0 ? nc - 1 - sd : sd) * cstride, op = c * cstride;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) r.dp[j][k] = to_f(t.v[k]);
-            } else {
-                r.dp[j] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(ds + c * cstride));
-            }
-            if constexpr (PREV16) {
-                typedef float f32x2 __attribute__((ext_vector_type(2)));
-                const V4 t = __builtin_bit_cast(V4, __builtin_nontemporal_load(reinterpret_cast<const f32x2 *>(prev16 + c * cstride)));
-#pragma unroll
-                for (int k = 0; k < 4; ++k) r.pv[j][k] = to_f(t.v[k]);
-            } else {
-                r.pv[j] = *reinterpret_cast<const f32x4 *>(prev + c * cstride);
+            for (int u = 0; u < NG; ++u) {
+                const int k = j * NG + u;
+                // (both are read for the last time in the pass: past the caches)
+                if constexpr (DP16) r.dp[k] = *reinterpret_cast<const f32x2 *>(ds16 + e[u] + od);
+                else r.dp[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4 *>(ds + e[u] + od));
+                if constexpr (PREV16) r.pv[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x2 *>(prev16 + e[u] + op));
+                else r.pv[k] = *reinterpret_cast<const f32x4 *>(prev + e[u] + op);
             }
         }
     };
     // (the recurrence and its stores first, then all inner products' sums side by side: one after the other, each a chain of six
     // exchanges between the lanes, they were half of the kernel's time.  1 x 16384 in chunks of 128, 16 heads of 32, dstate 32: 61 -> 50 us
     // with the next chunks under way, -> 27 with the sums side by side; beside dCB, 1 x 16384, 8 heads of 64, the pass 186 -> 172)
-    auto recur = [&](int s0, int nb, const Batch &r, float (&dot)[SP_CH], auto WHOLE) __attribute__((always_inline)) {
+    auto recur = [&](int s0, int nb, const Batch &r, float (&dot)[NU], auto WHOLE) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < SP_CH; ++j) {
+        for (int j = 0; j < NCH; ++j) {
             if (decltype(WHOLE)::value || j < nb) {
                 const int c = dir == 0 ? nc - 1 - (s0 + j) : s0 + j;
                 const float d = __expf(r.dec[j]);
-                dot[j] = (g[0] * r.pv[j][0] + g[1] * r.pv[j][1] + g[2] * r.pv[j][2] + g[3] * r.pv[j][3]) * d;
-                if constexpr (DS16) {
-                    V4 t;
 #pragma unroll
-                    for (int k = 0; k < 4; ++k) t.v[k] = from_f<T16>(g[k]);
-                    *reinterpret_cast<V4 *>(ds16 + c * cstride) = t;
-                } else {
-                    *reinterpret_cast<f32x4 *>(ds + c * cstride) = g;
+                for (int u = 0; u < NG; ++u) {
+                    if (NG > 1 && !live[u]) continue;
+                    const int k = j * NG + u;
+                    f32x4 &gu = g[u];
+                    const f32x4 pv = wide(r.pv[k]);
+                    dot[k] = (gu[0] * pv[0] + gu[1] * pv[1] + gu[2] * pv[2] + gu[3] * pv[3]) * d;
+                    if constexpr (DS16) {
+                        V4 t;
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) t.v[i] = from_f<T16>(gu[i]);
+                        *reinterpret_cast<V4 *>(ds16 + e[u] + c * cstride) = t;
+                    } else {
+                        *reinterpret_cast<f32x4 *>(ds + e[u] + c * cstride) = gu;
+                    }
+                    gu = wide(r.dp[k]) + d * gu;
                 }
-                g = r.dp[j] + d * g;
             }
         }
     };
     auto work = [&](int s0, const Batch &r) __attribute__((always_inline)) {
-        const int nb = min(SP_CH, nc - s0);
-        float dot[SP_CH] = {};
-        if (live) {
-            if (nb == SP_CH) recur(s0, nb, r, dot, std::true_type());
+        const int nb = min(NCH, nc - s0);
+        float dot[NU] = {};
+        if (NG > 1 || live[0]) {
+            if (nb == NCH) recur(s0, nb, r, dot, std::true_type());
             else recur(s0, nb, r, dot, std::false_type());
         }
 #pragma unroll
-        for (int j = 0; j < SP_CH; ++j) dot[j] = row16_sum(dot[j]);
+        for (int j = 0; j < NU; ++j) dot[j] = row16_sum(dot[j]);
 #pragma unroll
         for (int m = 16; m <= 32; m <<= 1)
 #pragma unroll
-            for (int j = 0; j < SP_CH; ++j) dot[j] += __shfl_xor(dot[j], m, 64);
+            for (int j = 0; j < NU; ++j) dot[j] += __shfl_xor(dot[j], m, 64);
         if (lane == 0) {
 #pragma unroll
-            for (int j = 0; j < SP_CH; ++j) red[s0 % FLUSH + j][wave] = dot[j];      // (behind the last chunk: never read)
+            for (int j = 0; j < NU; ++j) red[s0 * NG % FLUSH + j][wave] = dot[j];      // (behind the last chunk: never read)
         }
         // chunks up to s0 + nb: hand the inner products out when their place is full, or at the end
         const int done = s0 + nb;
-        if (done % FLUSH == 0 || done == nc) {
+        if (done * NG % FLUSH == 0 || done == nc) {
             __syncthreads();
-            const int from = (done - 1) / FLUSH * FLUSH;
-            if ((int)threadIdx.x < done - from) {
-                const int c = dir == 0 ? nc - 1 - (from + (int)threadIdx.x) : from + (int)threadIdx.x;
-                dda[(int64_t)c * nsplit] = red[threadIdx.x][0] + red[threadIdx.x][1] + red[threadIdx.x][2] + red[threadIdx.x][3];
+            const int from = (done - 1) / (FLUSH / NG) * (FLUSH / NG), i = threadIdx.x;
+            if (i < (done - from) * NG && split + i % NG < nsplit) {
+                const int c = dir == 0 ? nc - 1 - (from + i / NG) : from + i / NG;
+                dda[(int64_t)c * nsplit + i % NG] = red[i][0] + red[i][1] + red[i][2] + red[i][3];
             }
             __syncthreads();
         }
     };
-    if constexpr (AHEAD) {
+    if constexpr (AHEAD && NG == 1) {
         Batch one, two;
         load(0, one);
-        for (int s0 = 0; s0 < nc; s0 += 2 * SP_CH) {
-            if (s0 + SP_CH < nc) load(s0 + SP_CH, two);
+        for (int s0 = 0; s0 < nc; s0 += 2 * NCH) {
+            if (s0 + NCH < nc) load(s0 + NCH, two);
             work(s0, one);
-            if (s0 + SP_CH >= nc) break;
-            if (s0 + 2 * SP_CH < nc) load(s0 + 2 * SP_CH, one);
-            work(s0 + SP_CH, two);
+            if (s0 + NCH >= nc) break;
+            if (s0 + 2 * NCH < nc) load(s0 + 2 * NCH, one);
+            work(s0 + NCH, two);
         }
     } else {
-        for (int s0 = 0; s0 < nc; s0 += SP_CH) {
+        for (int s0 = 0; s0 < nc; s0 += NCH) {
             Batch one;
             load(s0, one);
             work(s0, one);
         }
     }
-    if (dini && live) *reinterpret_cast<f32x4 *>(dini + bh) = g;
+    if (dini)
+#pragma unroll
+        for (int u = 0; u < NG; ++u)
+            if (live[u]) *reinterpret_cast<f32x4 *>(dini + bh + e[u]) = g[u];
+}
+// ngr: groups a workgroup (2 also for long sequences, where TWO)
+template <typename T16, bool PREV16, bool DS16, bool DP16 = false, bool AHEAD = false, bool TWO = false>
+__device__ __forceinline__ void state_passing_bwd_vec_body(const bimamba2_params &p, int nc, int nsplit, int ndir, BlockId bid, int ngr = 1) {
+    if (nc == 1) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 1, 4>(p, nc, nsplit, ndir, bid);
+    else if (nc == 2) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 2, 4>(p, nc, nsplit, ndir, bid);
+    else if (nc <= 4) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 4, 2>(p, nc, nsplit, ndir, bid);
+    else {
+        if constexpr (TWO)
+            if (ngr == 2) return state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, SP_CH, 2>(p, nc, nsplit, ndir, bid);
+        state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, SP_CH, 1>(p, nc, nsplit, ndir, bid);
+    }
 }
 template <typename T16, bool PREV16, bool DS16, bool DP16 = false>
 __global__ __launch_bounds__(NTHREADS) void state_passing_bwd_vec_kernel(const bimamba2_params p, int nc, int nsplit, int ndir) {
@@ -466,7 +511,8 @@ int launch_state_passing_bwd(const bimamba2_params *p) {
     const int ndir = p->causal ? 1 : 2;
     if (PN % 4 == 0 && al(p->states_f) && al(p->states_b) && al(p->dstates_f) && al(p->dstates_b) && al(p->dfinal_f) && al(p->dfinal_b) &&
         al(p->dinitial_f) && al(p->dinitial_b)) {
-        dim3 grid(nsplit, p->nheads, p->batch * ndir);
+        const int ngr = sp_bwd_groups(nc);
+        dim3 grid((nsplit + ngr - 1) / ngr, p->nheads, p->batch * ndir);
         const bool prev16 = p->states16_f != nullptr, ds16 = p->dstates16_f != nullptr;
         if (prev16 && (!(p->causal || p->states16_b) || !al(p->states16_f) || !al(p->states16_b))) return BIMAMBA2_EINVAL;
         if (ds16 && (!(p->causal || p->dstates16_b) || !al(p->dstates16_f) || !al(p->dstates16_b))) return BIMAMBA2_EINVAL;
@@ -1031,7 +1077,7 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_dcb_heads_kernel(const bimamb
 // 50 and 122, and 47 against 34 at dstate 128 (2 x 3001, 24 heads).
 // W: the waves that share a tile in the kernel above (gdy: workgroups a (b, c, g)); 0: the ring, a tile a workgroup
 template <typename T, bool UNI, int W>
-__global__ __launch_bounds__(NTHREADS, W ? 2 : 1) void bwd_dcb_sp_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int gdy, int gdz, int nsplit, int ndir, bool out16) {
+__global__ __launch_bounds__(NTHREADS, W ? 2 : 1) void bwd_dcb_sp_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int gdy, int gdz, int nsplit, int nspx, int ndir, bool out16) {
     const int id = blockIdx.x, per = gdx * gdy, ndcb = per * gdz;
     if (id < ndcb) {
         __shared__ __attribute__((aligned(16))) unsigned char smem[W ? DcbHeadsMap<W ? W : 1>::LDS : DcbRingMap<64>::LDS];
@@ -1040,10 +1086,11 @@ __global__ __launch_bounds__(NTHREADS, W ? 2 : 1) void bwd_dcb_sp_kernel(const b
         if constexpr (W > 0) bwd_dcb_heads_body<T, UNI, W>(p, nc, nqt, tile, gdx, gdz, smem, out16);
         else bwd_dcb_ring_body<T, UNI, 64, true>(p, nc, nqt, tile, gdx, gdz, smem, out16);
     } else {
-        const int k = id - ndcb;                  // grid (nsplit, nheads, batch * ndir) of the state passing
-        const BlockId sb{k % nsplit, (k / nsplit) % p.nheads, k / (nsplit * p.nheads)};
-        if (p.dstates_f == nullptr) state_passing_bwd_vec_body<T, true, true, true>(p, nc, nsplit, ndir, sb);
-        else if (p.dstates16_f == nullptr) state_passing_bwd_vec_body<T, false, false>(p, nc, nsplit, ndir, sb);
+        const int k = id - ndcb;                  // grid (nspx, nheads, batch * ndir) of the state passing
+        const BlockId sb{k % nspx, (k / nspx) % p.nheads, k / (nspx * p.nheads)};
+        const int ngr = (nsplit + nspx - 1) / nspx;
+        if (p.dstates_f == nullptr) state_passing_bwd_vec_body<T, true, true, true, false, W != 0>(p, nc, nsplit, ndir, sb, ngr);
+        else if (p.dstates16_f == nullptr) state_passing_bwd_vec_body<T, false, false, false, false, W != 0>(p, nc, nsplit, ndir, sb, ngr);
         else state_passing_bwd_vec_body<T, true, true>(p, nc, nsplit, ndir, sb);
     }
 }
@@ -1197,9 +1244,13 @@ int launch_bwd_dcb_sp(const bimamba2_params *p, bool out16) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, PN = p->headdim * p->dstate;
     const int nsplit = (PN + SP_EPT * NTHREADS - 1) / (SP_EPT * NTHREADS), ndir = p->causal ? 1 : 2;
     const int slices = dcb_slices(p), W = p->headdim == 64 ? dcb_waves(p, slices) : 0;
-    const int gdx = p->batch * nc * p->ngroups, gdy = W ? (nqt * nqt * W + 3) / 4 : nqt * nqt, nsp = nsplit * p->nheads * p->batch * ndir;
+    const int gdx = p->batch * nc * p->ngroups, gdy = W ? (nqt * nqt * W + 3) / 4 : nqt * nqt, nsp1 = nsplit * p->nheads * p->batch * ndir;
+    // (two groups a workgroup of the state passing where that leaves as many workgroups as the chip holds beside the tiles, else fewer are
+    // under way at once: 1 x 8192, 24 heads, 192 -> 96 workgroups 36.8 -> 37.5)
+    const int ngr = nc > 4 && W && !(p->dstates_f && p->dstates16_f) && nsplit % 2 == 0 && nsp1 >= DCB_HEADS_RESIDENT ? 2 : sp_bwd_groups(nc);
+    const int nspx = (nsplit + ngr - 1) / ngr, nsp = nspx * p->nheads * p->batch * ndir;
     dim3 grid(gdx * gdy * slices + nsp);
-#define BM2_D(TT, UNI, WV) hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, UNI, WV>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, gdy, slices, nsplit, ndir, out16)
+#define BM2_D(TT, UNI, WV) hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, UNI, WV>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, gdy, slices, nsplit, nspx, ndir, out16)
 #define BM2_DS(TT, UNI)                \
     do {                               \
         if (W == 4) BM2_D(TT, UNI, 4); \

@@ -1183,17 +1183,22 @@ __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_inplace16_kernel(c
 #pragma unroll
         for (int k = 0; k < 4; ++k) { s[k] = a[k]; s[4 + k] = c4[k]; }
     }
-    for (int s0 = 0; s0 < nc; s0 += 8) {
-        Vec16<T16> v[8];
-        float d[8];
+    float *fin = dir == 0 ? p.final_f : p.final_b;
+    // (the recurrence's last chunk leads to the final state only: without one its neighbour is read in its place)
+    const int last = fin || nc == 1 ? nc - 1 : nc - 2;
+    // as many loads as there are chunks, up to 8 (behind the last chunk a load repeats it: one chunk cost eight loads of it)
+    auto batch = [&](int s0, auto N) __attribute__((always_inline)) {
+        constexpr int CH = decltype(N)::value;
+        Vec16<T16> v[CH];
+        float d[CH];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int si = min(s0 + i, nc - 1), c = dir == 0 ? si : nc - 1 - si;
+        for (int i = 0; i < CH; ++i) {
+            const int si = min(s0 + i, last), c = dir == 0 ? si : nc - 1 - si;
             v[i] = *reinterpret_cast<const Vec16<T16> *>(st + c * cstride);
             d[i] = cs[(int64_t)c * Q];
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
+        for (int i = 0; i < CH; ++i)
             if (s0 + i < nc) {
                 const int c = dir == 0 ? s0 + i : nc - 1 - (s0 + i);
                 Vec16<T16> o;
@@ -1204,8 +1209,14 @@ __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_inplace16_kernel(c
 #pragma unroll
                 for (int k = 0; k < 8; ++k) s[k] = dec * s[k] + to_f(v[i].v[k]);
             }
+    };
+    for (int s0 = 0; s0 < nc; s0 += 8) {
+        const int left = nc - s0;
+        if (left <= 1) batch(s0, std::integral_constant<int, 1>());
+        else if (left <= 2) batch(s0, std::integral_constant<int, 2>());
+        else if (left <= 4) batch(s0, std::integral_constant<int, 4>());
+        else batch(s0, std::integral_constant<int, 8>());
     }
-    float *fin = dir == 0 ? p.final_f : p.final_b;
     if (fin) {
         *reinterpret_cast<f32x4 *>(fin + ((int64_t)b * p.nheads + h) * PN + e) = f32x4{s[0], s[1], s[2], s[3]};
         *reinterpret_cast<f32x4 *>(fin + ((int64_t)b * p.nheads + h) * PN + e + 4) = f32x4{s[4], s[5], s[6], s[7]};

@@ -308,3 +308,33 @@ def test_state_passing_over_many_chunks(ops, nc, PN):
         # float32 recurrences whose terms shrink by e^-1.6 a chunk; inner products of P N terms
         for have, want in ((got[k], stack(enter, 1)), (got[2 + k], s), (back[k], stack(ds, 1)), (back[2 + k], stack(dda, 2))):
             assert float((have - want).norm()) <= 1e-5 * float(want.norm())
+
+
+@pytest.mark.parametrize("PN", [(64, 16), (64, 64), (72, 68)])
+@pytest.mark.parametrize("nc", [1, 2, 3, 4, 5])
+def test_state_passing_over_few_chunks(ops, nc, PN):
+    """several groups of 1024 elements a workgroup: one group of the state, four, and five (a workgroup with a group behind the end)"""
+    test_state_passing_over_many_chunks(ops, nc, PN)
+
+
+@pytest.mark.parametrize("L", [100, 333, 1000])
+def test_state_passing_beside_dcb_does_not_depend_on_the_batch(L):
+    """many rows: several groups of 1024 elements a workgroup in the launch of dCB; one row: one group where the sequence is long.  The
+    gradients of the states, and what is made of them alone, are the same bits"""
+    from bi_mamba2_amd.ops import bimamba_chunk_scan_combined
+    b, H, P, N = 32, 4, 64, 64
+    gen = torch.Generator().manual_seed(L)
+    inp = to_dev(make_case(b, L, H, P, 1, N, torch.bfloat16))
+    init = [torch.randn(b, H, P, N, generator=gen).cuda() for _ in range(2)]
+    dout = torch.randn(b, L, H, P, generator=gen).bfloat16().cuda()
+    dfin = [torch.randn(b, H, P, N, generator=gen).cuda() for _ in range(2)]
+
+    def grads(rows):
+        x = inp["x"][:rows].clone().requires_grad_(True)
+        st = [t[:rows].clone().requires_grad_(True) for t in init]
+        out = bimamba_chunk_scan_combined(x, inp["dt"][:rows], inp["A"], inp["B"][:rows], inp["C"][:rows], 128, dt_bias=inp["dt_bias"], dt_softplus=True,
+                                          initial_states_f=st[0], initial_states_b=st[1], return_final_states=True)
+        return torch.autograd.grad(out, [x] + st, [dout[:rows]] + [t[:rows] for t in dfin])
+
+    for many, one in zip(grads(b), grads(1)):
+        assert torch.equal(many[:1], one)
