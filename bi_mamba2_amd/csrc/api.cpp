@@ -38,6 +38,23 @@ int check_problem(const bimamba2_params *p) {
     return BIMAMBA2_OK;
 }
 
+// A sequence that one chunk holds, without states going in or out and without tensors for the states entering the chunks: these are
+// zero, nothing crosses a chunk boundary, and neither the chunk states and their passing nor the state parts of the backward pass are
+// formed (the sums are the same but for terms of zero).  us of kernels a pass, bfloat16, heads of 64, z gate: 1 x 197, 12 heads, dstate 64 25 -> 17
+// forward, 91 -> 60 in training (10 -> 7 launches); 8 x 250, 24 heads, dstate 128 48 -> 27, 168 -> 90; layer 16 x 200, d_model 768 109 -> 95,
+// 363 -> 303.  What follows from it is which pointers are NULL: the scan kernels' states, the last launch's state parts.
+inline bool one_chunk(const bimamba2_params *p) {
+    return p->seqlen <= p->chunk_size && !p->causal && !p->initial_f && !p->initial_b && !p->final_f && !p->final_b && !p->dfinal_f && !p->dfinal_b &&
+           !p->dinitial_f && !p->dinitial_b && !p->states_f && !p->states_b && !p->states16_f && !p->states16_b && !p->dstates_f && !p->dstates_b &&
+           !p->dstates16_f && !p->dstates16_b;
+}
+// whether such a problem's entering states would travel as 16-bit copies, i.e. which scan kernel is the one to run without any
+// (a forward pass that a backward pass follows keeps them in float32 at other shapes than bimamba2_state_copies()'s)
+inline bool one_chunk_free16(const bimamba2_params *p, bool is_bwd) {
+    if (p->dtype == BIMAMBA2_F32) return false;
+    return bimamba2_state_copies(p) != 0 || (!is_bwd && !(p->fwd_saved & 4) && (p->headdim * p->dstate) % 4 == 0);
+}
+
 #define REQUIRE(ptr)                        \
     do {                                    \
         if (!(ptr)) return BIMAMBA2_EINVAL; \
@@ -63,6 +80,7 @@ struct Carver {
 // Assigns every intermediate that is NULL in `q` from the workspace; returns the bytes used.
 size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     Carver cv(ws);
+    const bool one = one_chunk(q);
     const size_t nc = nchunks(q), Q = q->chunk_size;
     const size_t bhcq = (size_t)q->batch * q->nheads * nc * Q;
     const size_t cbn = (size_t)q->batch * nc * q->ngroups * Q * Q;
@@ -83,10 +101,11 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     const bool fwd_only_copies = !is_bwd && !q->causal && (q->dtype == BIMAMBA2_BF16 || q->dtype == BIMAMBA2_F16) &&
                                  (q->headdim * q->dstate) % 4 == 0 && al16(q->final_f) && al16(q->final_b) &&
                                  al16(q->initial_f) && al16(q->initial_b) && !q->states_b && !q->states16_b;
-    const bool carve16 = (copies || fwd_only_copies) && !q->states_f && !q->states16_f;
+    const bool carve16 = !one && (copies || fwd_only_copies) && !q->states_f && !q->states16_f;
     // CB: read by the forward scan and by the dCB kernel unless they rebuild it; CB^T: by the dx kernel, likewise.  (The
     // forward scan kernel for state dimension 128 rebuilds it as well, and runs where the entering states travel as copies.)
-    const bool fwd_scan16 = !is_bwd && chunk_scan_uses_scan16(q, false) && (carve16 || q->states16_f) && (q->causal || carve16 || q->states16_b);
+    const bool fwd_scan16 = !is_bwd && chunk_scan_uses_scan16(q, false) &&
+                            (one ? one_chunk_free16(q, false) : (carve16 || q->states16_f) && (q->causal || carve16 || q->states16_b));
     if (is_bwd ? !(scan_recomputes_cb(q, true) && dcb_recomputes_cb(q)) : !(scan_recomputes_cb(q, false) || fwd_scan16)) need_f(q->CB, cbn);
     if (carve16) {
         q->states16_f = cv.take<char>(stn * 2);
@@ -96,11 +115,11 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     // too (the chunk-state kernel writes them there, the inter-chunk scan replaces them by the entering states)
     const bool states16_only = !is_bwd && !q->states_f && !q->states_b && (carve16 || (q->states16_f && q->states16_b)) &&
                                chunk_states_in_16bit(q);
-    if (!saved_copies && !states16_only) {
+    if (!saved_copies && !states16_only && !one) {
         need_f(q->states_f, stn);
         need_f(q->states_b, stn);
     }
-    if (is_bwd && copies && !q->dstates_f && !q->dstates16_f) {
+    if (is_bwd && copies && !q->dstates_f && !q->dstates16_f && !one) {
         q->dstates16_f = cv.take<char>(stn * 2);
         q->dstates16_b = cv.take<char>(stn * 2);
     }
@@ -116,25 +135,29 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
         // inter-chunk scan): no float32 tensors at all
         // (the in-place kernel of the backward inter-chunk scan reads the entering states from their copies as well)
         const bool dstates16_only = copies && !q->dstates_f && !q->dstates_b && (carve16 || q->states16_f);
-        if (!dstates16_only) {
+        if (!dstates16_only && !one) {
             need_f(q->dstates_f, stn);
             need_f(q->dstates_b, stn);
         }
         if (q->has_z && !q->dout_x)
             q->dout_x = cv.take<char>((size_t)q->batch * q->seqlen * q->nheads * q->headdim * elem_size(q->dtype));
         need_f(q->ddt_direct, bhcq * ddt_direct_planes(*q));
-        need_f(q->u_f, bhcq);
-        need_f(q->u_b, bhcq);
-        need_f(q->v_f, bhcq);
-        need_f(q->v_b, bhcq);
         need_f(q->da_intra, (size_t)q->batch * q->nheads * nc * nqt * nqt * 128);
-        need_f(q->ddA_chunk_f, (size_t)q->batch * q->nheads * nc * sp_nsplit(q));
-        need_f(q->ddA_chunk_b, (size_t)q->batch * q->nheads * nc * sp_nsplit(q));
-        const int hps = q->dbdc_heads > 0 ? q->dbdc_heads : 8;
-        const size_t slices = (q->nheads / q->ngroups + hps - 1) / hps;   // head slices of the dB / dC partial sums
-        const size_t bn = slices * q->batch * q->seqlen * q->ngroups * q->dstate;
-        need_f(q->dBs, bn);
-        need_f(q->dCs, bn);
+        if (one) {
+            q->u_f = q->u_b = q->v_f = q->v_b = q->ddA_chunk_f = q->ddA_chunk_b = q->dBs = q->dCs = nullptr;
+        } else {
+            need_f(q->u_f, bhcq);
+            need_f(q->u_b, bhcq);
+            need_f(q->v_f, bhcq);
+            need_f(q->v_b, bhcq);
+            need_f(q->ddA_chunk_f, (size_t)q->batch * q->nheads * nc * sp_nsplit(q));
+            need_f(q->ddA_chunk_b, (size_t)q->batch * q->nheads * nc * sp_nsplit(q));
+            const int hps = q->dbdc_heads > 0 ? q->dbdc_heads : 8;
+            const size_t slices = (q->nheads / q->ngroups + hps - 1) / hps;   // head slices of the dB / dC partial sums
+            const size_t bn = slices * q->batch * q->seqlen * q->ngroups * q->dstate;
+            need_f(q->dBs, bn);
+            need_f(q->dCs, bn);
+        }
         // partial sums of dD, then those of dA and ddt_bias (the composite reduces all three in one launch at the end)
         need_f(q->red, (size_t)q->batch * nc * q->nheads * q->headdim + (size_t)2 * q->batch * nc * q->nheads);
     }
@@ -444,6 +467,16 @@ int bimamba2_fwd(const bimamba2_params *p) {
     bimamba2_params q = *p;
     const size_t need = carve(&q, 0, p->workspace);
     if (need > 256 && (!p->workspace || p->workspace_bytes < need)) return BIMAMBA2_EWORKSPACE;
+    if (one_chunk(&q)) {
+        REQUIRE(q.dt); REQUIRE(q.A); REQUIRE(q.x); REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.out);
+        if (q.has_dt_bias) REQUIRE(q.dt_bias);
+        if (q.has_D) REQUIRE(q.D);
+        if (q.has_z) REQUIRE(q.z);
+        const bool free16 = one_chunk_free16(&q, false);
+        TRY(launch_fwd_cumsum_cb(&q, free16));
+        if (scan_recomputes_cb(&q, false) || (free16 && chunk_scan_uses_scan16(&q, false))) q.CB = nullptr;
+        return launch_chunk_scan(&q, false, free16);
+    }
     if (fwd_front_merged(&q)) {
         REQUIRE(q.dt); REQUIRE(q.A); REQUIRE(q.x); REQUIRE(q.Bm); REQUIRE(q.Cm);
         if (q.has_dt_bias) REQUIRE(q.dt_bias);
@@ -481,9 +514,15 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     q.final_f = q.final_b = nullptr;
     const size_t need = carve(&q, 1, p->workspace);
     if (need > 256 && (!p->workspace || p->workspace_bytes < need)) return BIMAMBA2_EWORKSPACE;
+    // (a forward pass over one chunk leaves no states: its caller says so)
+    const bool one = one_chunk(&q) && (!p->fwd_saved || (p->fwd_saved & 4));
     if (p->fwd_saved) {
         REQUIRE(p->dt_out); REQUIRE(p->cs_f); REQUIRE(p->cs_b);
-        if (!p->states16_f) { REQUIRE(p->states_f); REQUIRE(p->states_b); }
+        if (!p->states16_f && !one) { REQUIRE(p->states_f); REQUIRE(p->states_b); }
+    } else if (one) {
+        bimamba2_params qs = q;
+        qs.CB = nullptr;
+        TRY(launch_fwd_cumsum_cb(&qs, one_chunk_free16(&q, true)));
     } else {
         // recompute the forward intermediates (the reference does the same, src/ssd/bi/ssd_combined.py:373-380)
         TRY(forward_cumsum_and_states(&q));
@@ -491,14 +530,16 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     }
     // dCB / dCBT in the 16-bit element type where this call owns them and the two launches that write and read them are the
     // merged ones (their reader rounds them to that type for its MFMA anyway)
-    const bool own_dcb = !p->dCB && !p->dCBT, dcb_sp = bwd_dcb_sp_merged(&q) && (own_dcb || dcb_slices(&q) == 1);
+    // (without states to pass the launch is dCB's alone, with its place for 16-bit results)
+    const bool own_dcb = !p->dCB && !p->dCBT;
+    const bool dcb_sp = (one ? dcb_recomputes_cb(&q) && (q.headdim * q.dstate) % 4 == 0 : bwd_dcb_sp_merged(&q)) && (own_dcb || dcb_slices(&q) == 1);
     const bool dcb16 = own_dcb && dcb_sp && dcb_slices(&q) == 1 && bwd_tail_merged(&q);
     const bool need_cbt = !scan_recomputes_cb(&q, true), need_cb = need_cbt || !dcb_recomputes_cb(&q);
     const bool saved_cb = (p->fwd_saved & 2) && p->CB && p->CBT;
     const bool form_cb = need_cb && !saved_cb;     // (else left there by the forward pass)
     if (!need_cb) q.CB = nullptr;
     // dz and dstates as one launch where the kernel for it exists (dout_x goes from the first to the second inside the workgroup)
-    const bool dz_dstates = q.has_z && bwd_dz_dstates_fused(&q), dz_bmm = q.has_z && !dz_dstates && form_cb;
+    const bool dz_dstates = q.has_z && !one && bwd_dz_dstates_fused(&q), dz_bmm = q.has_z && !dz_dstates && form_cb;
     if (form_cb && !dz_bmm) TRY(bimamba2_bmm_chunk_fwd(&q));  // CB for the dCB kernel, CB^T for the dx kernel, unless they rebuild it
     if (dz_dstates) TRY(bimamba2_chunk_scan_bwd_dz_dstates(&q));
     else if (dz_bmm) {
@@ -510,32 +551,37 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     const int ncb = own_dcb && (tail_small || bwd_tail_merged(&q)) ? dcb_slices(&q) : 1;
     // the dCB kernel is bound by instruction issue and moves little data: right behind dz it runs while the memory system
     // still writes back dz's output, which the memory-bound kernels after it would otherwise wait behind
-    const bool dx_db_dc = dx_db_dc_merged(&q);      // (one launch at the end)
+    const bool dx_db_dc = !one && dx_db_dc_merged(&q);      // (one launch at the end)
     if (dcb_sp && (ncb == dcb_slices(&q))) {
         // the backward state passing (streams, few instructions) rides along with the dCB kernel in one launch
-        if (!dx_db_dc) TRY(bimamba2_chunk_scan_bwd_dc(&q));
-        if (!dz_dstates) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
+        if (!dx_db_dc && !one) TRY(bimamba2_chunk_scan_bwd_dc(&q));
+        if (!dz_dstates && !one) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
         REQUIRE(q.x); REQUIRE(q.dt_out); REQUIRE(q.cs_f); REQUIRE(q.cs_b); REQUIRE(q.dCB); REQUIRE(q.dCBT); REQUIRE(q.da_intra);
-        if (!q.dstates16_f) REQUIRE(q.dstates_f);
-        REQUIRE(q.ddA_chunk_f); REQUIRE(q.ddA_chunk_b);
+        if (!one) {
+            if (!q.dstates16_f) REQUIRE(q.dstates_f);
+            REQUIRE(q.ddA_chunk_f); REQUIRE(q.ddA_chunk_b);
+        }
         if (q.has_z) REQUIRE(q.dout_x); else REQUIRE(q.dout);
         TRY(launch_bwd_dcb_sp(&q, dcb16));
     } else {
         TRY(check_bwd_dcb(&q));
-        if (!dz_dstates && ncb == dcb_slices(&q) && dcb_dstates_merged(&q)) {
+        if (one) TRY(launch_bwd_dcb(&q, ncb == 1));
+        else if (!dz_dstates && ncb == dcb_slices(&q) && dcb_dstates_merged(&q)) {
             REQUIRE(q.Cm);
             TRY(launch_dcb_dstates(&q));
         } else {
             TRY(launch_bwd_dcb(&q, ncb == 1));
             if (!dz_dstates) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
         }
-        if (!dx_db_dc) TRY(bimamba2_chunk_scan_bwd_dc(&q));           // (between the two memory-bound state kernels: measured best)
-        TRY(bimamba2_state_passing_bwd(&q));
+        if (!one) {
+            if (!dx_db_dc) TRY(bimamba2_chunk_scan_bwd_dc(&q));           // (between the two memory-bound state kernels: measured best)
+            TRY(bimamba2_state_passing_bwd(&q));
+        }
     }
     if (dx_db_dc) {
         REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dBs); REQUIRE(q.dCs); REQUIRE(q.u_f); REQUIRE(q.u_b); REQUIRE(q.v_f); REQUIRE(q.v_b);
         REQUIRE(q.states_f); REQUIRE(q.states_b); REQUIRE(q.dstates_f); REQUIRE(q.dstates_b);
-    } else TRY(bimamba2_chunk_state_bwd_db(&q));
+    } else if (!one) TRY(bimamba2_chunk_state_bwd_db(&q));
     ReduceJobs jobs;
     {
         // as bimamba2_chunk_scan_bwd_dx, with the reduction of the dD partial sums left for the end
@@ -544,7 +590,7 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
         REQUIRE(qx.dx); REQUIRE(qx.ddt_direct);
         if (qx.has_D) { REQUIRE(qx.D); REQUIRE(qx.dD); }
         const int nc = nchunks(&q);
-        TRY(dx_db_dc ? launch_dx_db_dc(&qx) : launch_chunk_scan(&qx, true));
+        TRY(dx_db_dc ? launch_dx_db_dc(&qx) : launch_chunk_scan(&qx, true, one && one_chunk_free16(&q, true)));
         if (q.has_D) {
             if (q.D_has_hdim) jobs.job[jobs.n++] = ReduceJob{q.red, q.dD, q.batch * nc, q.nheads * q.headdim, 1};
             else jobs.job[jobs.n++] = ReduceJob{q.red, q.dD, q.batch * nc, q.nheads, q.headdim};
@@ -562,6 +608,11 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
             REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dt); REQUIRE(q.A);
             if (q.has_dt_bias) REQUIRE(q.dt_bias);
             TRY(launch_bwd_tail_small(&qc, &jobs, ncb));
+        } else if (one) {
+            REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dt); REQUIRE(q.A);
+            if (q.has_dt_bias) REQUIRE(q.dt_bias);
+            TRY(launch_bmm_chunk_bwd(&q));
+            TRY(launch_chunk_cumsum_bwd(&qc, &jobs));
         } else {
             TRY(bimamba2_bmm_chunk_bwd(&q));
             TRY(launch_chunk_cumsum_bwd(&qc, &jobs));

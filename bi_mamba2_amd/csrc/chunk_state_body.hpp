@@ -13,7 +13,30 @@ namespace bm2 {
 // ACC: the type of the sums.  float32 problems take them in 64 bits and round once: a result there is off by little else than the
 // resolution of these sums (their differences are exponents), and with every addition rounded it was off by 1.7 times as much.
 // 16-bit results are not, and 64 bits would cost them 2 of 13 us over 2 x 16384 positions of 48 heads.
-template <typename DT, typename ACC>
+// The sums of a lane's four positions with the products dt * A unrounded, as the chunk-state kernel with direct loads takes them.  (Written
+// out: with the cuts' conditions between product and sum the compiler does not fuse the two by itself.)  cut_*: of packed sequences, in
+// front of a position in the forward sums and behind it in the reverse ones.
+__device__ __forceinline__ void chunk_sums_unrounded(const float (&dt)[4], float A, const float (&cut_f)[4], const float (&cut_b)[4], int lane, float (&cf)[4], float (&cb)[4]) {
+    float pf[4], sb[4];
+    pf[0] = fmaf(dt[0], A, cut_f[0]);
+    sb[3] = fmaf(dt[3], A, cut_b[3]);
+#pragma unroll
+    for (int e = 1; e < 4; ++e) {
+        pf[e] = fmaf(dt[e], A, pf[e - 1] + cut_f[e]);
+        sb[3 - e] = fmaf(dt[3 - e], A, sb[4 - e] + cut_b[3 - e]);
+    }
+    const float tot = pf[3], tot_r = sb[0];
+    const float before = wave_incl_prefix(tot, lane) - tot, after = wave_incl_suffix(tot_r, lane) - tot_r;
+    cf[0] = fmaf(dt[0], A, before + cut_f[0]);
+    cb[3] = fmaf(dt[3], A, after + cut_b[3]);
+#pragma unroll
+    for (int e = 1; e < 4; ++e) {
+        cf[e] = before + pf[e];
+        cb[3 - e] = after + sb[3 - e];
+    }
+}
+// UNROUNDED: the sums as above
+template <typename DT, typename ACC, bool UNROUNDED = false>
 __device__ __forceinline__ void chunk_cumsum_wave(const bimamba2_params &p, int b, int c, int h, int lane, float (&v)[4], float (&cf)[4], float (&cb)[4]) {
     const int Q = p.chunk_size;
     const int limit = min(Q, p.seqlen - c * Q);
@@ -21,6 +44,7 @@ __device__ __forceinline__ void chunk_cumsum_wave(const bimamba2_params &p, int 
     const float A = p.A[h];
     const float bias = p.has_dt_bias ? p.dt_bias[h] : 0.f;
     ACC a[4], ar[4];                                  // ar: exponents of the reverse direction (differ with seq_idx only)
+    float cut_f[4] = {}, cut_b[4] = {};
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int q = lane * 4 + e;
@@ -38,10 +62,11 @@ __device__ __forceinline__ void chunk_cumsum_wave(const bimamba2_params &p, int 
             const int l = c * Q + q;
             const int32_t *si = p.seq_idx + (int64_t)b * p.seqlen + l;
             const int32_t cur = si[0];
-            if (l > 0 && si[-1] != cur) a[e] += BIMAMBA2_SEQ_CUT;
-            if (l + 1 < p.seqlen && si[1] != cur) ar[e] += BIMAMBA2_SEQ_CUT;
+            if (l > 0 && si[-1] != cur) { a[e] += BIMAMBA2_SEQ_CUT; cut_f[e] = BIMAMBA2_SEQ_CUT; }
+            if (l + 1 < p.seqlen && si[1] != cur) { ar[e] += BIMAMBA2_SEQ_CUT; cut_b[e] = BIMAMBA2_SEQ_CUT; }
         }
     }
+    if constexpr (UNROUNDED) return chunk_sums_unrounded(v, A, cut_f, cut_b, lane, cf, cb);
     // forward inclusive scan, reverse inclusive scan
     ACC pf[4], sb[4];
     pf[0] = a[0]; pf[1] = pf[0] + a[1]; pf[2] = pf[1] + a[2]; pf[3] = pf[2] + a[3];

@@ -251,15 +251,16 @@ struct Problem {
 
 // What the forward pass leaves for the backward pass besides its operands, in one float32 allocation: dt_out, cs_f, cs_b, the
 // states entering the chunks (copies: in the operands' 16-bit type, where the kernels can keep them that way) and, with cb,
-// C.B^T and its transpose.
+// C.B^T and its transpose.  One chunk without states of its own (final: the caller takes the final states) has no states to keep.
 struct Kept {
     size_t n1 = 0, ns = 0, ncb = 0;
     bool copies = false;
-    Kept(const bimamba2_params &p, bool copies_, bool cb) : copies(copies_) {
+    Kept(const bimamba2_params &p, bool copies_, bool cb, bool final) : copies(copies_) {
         const size_t nc = (p.seqlen + p.chunk_size - 1) / p.chunk_size;
         n1 = round_up((size_t)p.batch * p.nheads * nc * p.chunk_size, 64);
         ns = round_up((size_t)p.batch * nc * p.nheads * p.headdim * p.dstate, 64);
         if (copies) ns /= 2;
+        if (p.seqlen <= p.chunk_size && !p.initial_f && !p.initial_b && !final) ns = 0;
         if (cb) ncb = round_up((size_t)p.batch * nc * p.ngroups * p.chunk_size * p.chunk_size, 64);
     }
     int64_t floats() const { return (int64_t)(3 * n1 + 2 * ns + 2 * ncb); }
@@ -268,10 +269,10 @@ struct Kept {
         p.cs_f = base + n1;
         p.cs_b = base + 2 * n1;
         float *st = base + 3 * n1;
-        if (copies) {
+        if (ns && copies) {
             p.states16_f = st;
             p.states16_b = st + ns;
-        } else {
+        } else if (ns) {
             p.states_f = st;
             p.states_b = st + ns;
         }
@@ -280,8 +281,9 @@ struct Kept {
             p.CBT = p.CB + ncb;
         }
     }
-    // what bimamba2_bwd is told about these
-    int saved() const { return ncb ? 3 : 1; }
+    // what bimamba2_fwd and bimamba2_bwd are told about these
+    int kept() const { return ns ? 0 : 4; }
+    int saved() const { return kept() | (ncb ? 3 : 1); }
 };
 
 // Whether the forward pass keeps C.B^T and its transpose for the backward pass: where the backward's kernels read them and they
@@ -292,7 +294,8 @@ struct Kept {
 bool keeps_cb(const bimamba2_params &p) {
     if (!api.reads_cb(&p, 0) || !api.reads_cb(&p, 1)) return false;
     const size_t e = p.dtype == BIMAMBA2_F32 ? 4 : 2, x = e * p.batch * p.seqlen * p.nheads * p.headdim;
-    const Kept without(p, false, false), with(p, false, true);
+    // (beside the states of the chunks, also where there are none to keep)
+    const Kept without(p, false, false, true), with(p, false, true, true);
     return 8 * with.ncb <= x + 4 * (size_t)without.floats();
 }
 
@@ -313,9 +316,10 @@ ScanResult scan_forward(Problem &q, ScanOpts &o, bool keep) {
     if (keep) {
         o.copies = api.state_copies(&p) != 0;
         o.cb = !o.copies && keeps_cb(p);
-        const Kept k(p, o.copies, o.cb);
+        const Kept k(p, o.copies, o.cb, o.want_final);
         r.kept = device_empty({k.floats()}, at::kFloat, q.x);
         k.point(p, r.kept.mutable_data_ptr<float>());
+        p.fwd_saved = k.kept();
     }
     r.out = device_empty(q.x.sizes(), q.x.scalar_type(), q.x);
     p.out = r.out.mutable_data_ptr();
@@ -445,7 +449,7 @@ public:
             p.dinitial_b = dinit_b.mutable_data_ptr<float>();
         }
         Tensor kept = s[12].contiguous();
-        const Kept k(p, o.copies, o.cb);
+        const Kept k(p, o.copies, o.cb, o.want_final);
         k.point(p, kept.mutable_data_ptr<float>());
         p.fwd_saved = k.saved();
         Tensor dz, dD, dbias, out_x = s[11];
@@ -752,9 +756,10 @@ Tensor layer_forward(const Tensor &u, const Tensor &w_in, const Tensor &b_in, st
     if (keep) {
         o.copies = api.state_copies(&p) != 0;
         o.cb = !o.copies && keeps_cb(p);
-        const Kept k(p, o.copies, o.cb);
+        const Kept k(p, o.copies, o.cb, false);
         kept = device_empty({k.floats()}, at::kFloat, u);
         k.point(p, kept.mutable_data_ptr<float>());
+        p.fwd_saved = k.kept();
     }
     const Tensor ws = attach_workspace(p, false, u);
     check(api.fwd(&p), "bimamba2_fwd");
@@ -834,7 +839,7 @@ public:
 
         const Tensor dxbc = device_empty({s.rows, s.conv}, u.scalar_type(), u);
         bimamba2_params p = layer_scan_params(s, o, zx, xbc, w, stream);
-        const Kept k(p, o.copies, o.cb);
+        const Kept k(p, o.copies, o.cb, false);
         k.point(p, kept.mutable_data_ptr<float>());
         p.fwd_saved = k.saved();
         p.dout = dy.const_data_ptr();

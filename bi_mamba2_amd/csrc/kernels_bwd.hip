@@ -548,6 +548,8 @@ int launch_state_passing_bwd(const bimamba2_params *p) {
 // =========================================================================================================
 static inline int dbdc_heads(const bimamba2_params *p) { return p->dbdc_heads > 0 ? p->dbdc_heads : DBDC_HEADS; }
 static inline int dbdc_slices(const bimamba2_params *p) { return (p->nheads / p->ngroups + dbdc_heads(p) - 1) / dbdc_heads(p); }
+// of them, those there are to add up: none where nothing wrote a state part (one_chunk())
+static inline int state_slices(const bimamba2_params *p) { return p->dBs ? dbdc_slices(p) : 0; }
 
 // Heads per slice where the caller leaves the choice (the partial sums are bimamba2_bwd's own).  A workgroup of the dB / dC
 // kernels fills a CU, needs about three head steps to start (measured: 17 us for 8 heads, of which 5 before the first) and
@@ -1248,7 +1250,7 @@ int launch_bwd_dcb_sp(const bimamba2_params *p, bool out16) {
     // (two groups a workgroup of the state passing where that leaves as many workgroups as the chip holds beside the tiles, else fewer are
     // under way at once: 1 x 8192, 24 heads, 192 -> 96 workgroups 36.8 -> 37.5)
     const int ngr = nc > 4 && W && !(p->dstates_f && p->dstates16_f) && nsplit % 2 == 0 && nsp1 >= DCB_HEADS_RESIDENT ? 2 : sp_bwd_groups(nc);
-    const int nspx = (nsplit + ngr - 1) / ngr, nsp = nspx * p->nheads * p->batch * ndir;
+    const int nspx = (nsplit + ngr - 1) / ngr, nsp = p->ddA_chunk_f ? nspx * p->nheads * p->batch * ndir : 0;      // (0: one_chunk())
     dim3 grid(gdx * gdy * slices + nsp);
 #define BM2_D(TT, UNI, WV) hipLaunchKernelGGL((bwd_dcb_sp_kernel<TT, UNI, WV>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, gdx, gdy, slices, nsplit, nspx, ndir, out16)
 #define BM2_DS(TT, UNI)                \
@@ -1357,6 +1359,7 @@ __device__ __forceinline__ void bmm_chunk_bwd_body(const bimamba2_params &p, int
             oa[it] = (((int64_t)b * p.seqlen + (int64_t)c * Q + r) * p.ngroups + g) * N + nt * 64 + cc;
 #pragma unroll
             for (int sl = 0; sl < HSL; ++sl) {
+                if (nslices == 0) continue;        // (uniform) no state part: a sequence of one chunk
                 const float *q = res + oa[it] + (int64_t)min(sl, nslices - 1) * slice;
                 sv[it][sl][0] = *reinterpret_cast<const float4 *>(q);
                 sv[it][sl][1] = *reinterpret_cast<const float4 *>(q + 4);
@@ -1514,7 +1517,7 @@ __global__ __launch_bounds__(NTHREADS) void bmm_chunk_bwd_kernel(const bimamba2_
 
 template <typename T>
 static int launch_bmm_bwd_t(const bimamba2_params *p) {
-    const int nc = nchunks(p), Q = p->chunk_size, nsl = dbdc_slices(p);
+    const int nc = nchunks(p), Q = p->chunk_size, nsl = state_slices(p);
     dim3 grid((p->dstate + 63) / 64, (Q + 63) / 64, p->batch * nc * p->ngroups * 2);
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     auto mult = [](int64_t a, int64_t b, int64_t c) { return a % 8 == 0 && b % 8 == 0 && c % 8 == 0; };
@@ -1565,16 +1568,27 @@ __device__ __forceinline__ void chunk_cumsum_bwd_body(const bimamba2_params &p, 
     const int nplanes = ddt_direct_planes(p);
     const int64_t plane = (int64_t)p.batch * H * nc * Q;
     const DT *dt = reinterpret_cast<const DT *>(p.dt) + b * p.dt_sb + (int64_t)c * Q * p.dt_sl + h * p.dt_sh;
+    const bool state_terms = p.u_f != nullptr;     // (else a sequence of one chunk: nothing crosses a boundary)
+    if (state_terms) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int qc = min(lane * 4 + e, limit - 1);
+            vf[e] = p.v_f[o + qc];
+            vb[e] = p.v_b[o + qc];
+            uf[e] = p.u_f[o + qc];
+            ub[e] = p.u_b[o + qc];
+        }
+    }
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const int qc = min(lane * 4 + e, limit - 1);
-        vf[e] = p.v_f[o + qc];
-        vb[e] = p.v_b[o + qc];
-        uf[e] = p.u_f[o + qc];
-        ub[e] = p.u_b[o + qc];
         ddr[e] = p.ddt_direct[o + qc];
         for (int pl = 1; pl < nplanes; ++pl) ddr[e] += p.ddt_direct[pl * plane + o + qc];    // one plane per headdim tile of the dx kernel
         dtr[e] = to_f(dt[(int64_t)qc * p.dt_sl]);
+    }
+    if (!state_terms) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) vf[e] = vb[e] = uf[e] = ub[e] = 0.f;
     }
     if (p.causal) {                   // single-direction operator: nothing wrote the reverse direction's terms
 #pragma unroll
@@ -1583,7 +1597,7 @@ __device__ __forceinline__ void chunk_cumsum_bwd_body(const bimamba2_params &p, 
     const float A = p.A[h];
     const float bias = p.has_dt_bias ? p.dt_bias[h] : 0.f;
     float chunk_term = 0.f;
-    for (int s = 0; s < nsplit; ++s)
+    for (int s = 0; state_terms && s < nsplit; ++s)
     {
         const float cf = p.ddA_chunk_f[(((int64_t)b * H + h) * nc + c) * nsplit + s], cr = p.ddA_chunk_b[(((int64_t)b * H + h) * nc + c) * nsplit + s];
         chunk_term += cf + (p.causal ? 0.f : cr);
@@ -1753,7 +1767,7 @@ static int launch_bwd_tail_t(const bimamba2_params *p, int nc, int nqt, int nspl
     const int bmm_gy = (p->chunk_size + 63) / 64 * (p->dstate / 64), nbmm = bmm_gy * p->batch * nc * p->ngroups * 2;
     const int cs_gx = (p->nheads + 3) / 4, ncs = cs_gx * nc * p->batch;
     dim3 grid(nbmm + ncs);
-    const int nsl = dbdc_slices(p);
+    const int nsl = state_slices(p);
     if (in16 && nsl <= 2) {
         switch (p->dt_dtype) {
             case BIMAMBA2_F32: hipLaunchKernelGGL((bwd_tail_kernel<T, float, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nsl, nqt, nsplit, nbmm, bmm_gy, cs_gx, in16, ncb); break;
@@ -1782,8 +1796,8 @@ static void launch_bwd_tail_small_t(const bimamba2_params *p, int nc, int nsplit
     const int nqt = (p->chunk_size + 63) / 64, nnt = (p->dstate + 63) / 64, nbmm = nnt * nqt * p->batch * nc * p->ngroups * 2;
     const int cs_gx = (p->nheads + 3) / 4;
     const dim3 grid(nbmm + cs_gx * nc * p->batch);
-    if (p->dt_dtype == BIMAMBA2_F32) hipLaunchKernelGGL((bwd_tail_small_kernel<T, QP, FAST, float>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, dbdc_slices(p), nqt, nsplit, nbmm, nnt, cs_gx, ncb);
-    else hipLaunchKernelGGL((bwd_tail_small_kernel<T, QP, FAST, T>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, dbdc_slices(p), nqt, nsplit, nbmm, nnt, cs_gx, ncb);
+    if (p->dt_dtype == BIMAMBA2_F32) hipLaunchKernelGGL((bwd_tail_small_kernel<T, QP, FAST, float>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, state_slices(p), nqt, nsplit, nbmm, nnt, cs_gx, ncb);
+    else hipLaunchKernelGGL((bwd_tail_small_kernel<T, QP, FAST, T>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, state_slices(p), nqt, nsplit, nbmm, nnt, cs_gx, ncb);
 }
 
 // ncb: head slices of dCB that nobody has added up yet

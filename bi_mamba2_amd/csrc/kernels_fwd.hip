@@ -80,6 +80,25 @@ __global__ __launch_bounds__(NTHREADS) void fwd_front_kernel(const bimamba2_para
     }
 }
 
+// The cumulative sums and, where C.B^T is read, its tiles in one launch: the front of a pass over one chunk, which has no states to form.  UNROUNDED: the
+// sums as the chunk-state launch that takes them at such shapes.
+template <typename T, typename DT, bool UNROUNDED>
+__global__ __launch_bounds__(NTHREADS) void fwd_cumsum_cb_kernel(const bimamba2_params p, int nc, int gx, int ncs, int nqt) {
+    __shared__ __attribute__((aligned(16))) char lds[BMM_FWD_LDS<T>];
+    const int id = blockIdx.x;
+    if (id >= ncs) {
+        const int k = id - ncs;
+        bmm_chunk_fwd_body<T>(p, nc, k % nqt, k / nqt % nqt, k / (nqt * nqt), lds);
+        return;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int h = id % gx * 4 + wave, c = id / gx % nc, b = id / (gx * nc);
+    if (h >= p.nheads) return;
+    float v[4], cf[4], cb[4];
+    chunk_cumsum_wave<DT, typename std::conditional<sizeof(T) == 4, double, float>::type, UNROUNDED>(p, b, c, h, lane, v, cf, cb);
+    chunk_cumsum_store(p, (((int64_t)b * p.nheads + h) * nc + c) * p.chunk_size, lane, v, cf, cb);
+}
+
 // ---------------------------------------------------------------------------------------------------------
 // The same for 16-bit types with headdim % 64 == 0, dstate % 64 == 0, chunk_size % 32 == 0 and aligned operands: both
 // tiles travel as they are from global memory into LDS (direct loads: no registers, nothing to wait for until all of
@@ -248,25 +267,7 @@ __device__ __forceinline__ void chunk_state_direct_body(const bimamba2_params &p
                     if (__float_as_uint(sid[e + 2]) != __float_as_uint(sid[e + 1])) cut_b[e] = BIMAMBA2_SEQ_CUT;
                 }
             }
-            // The products dt * A enter their sums unrounded.  (Written out: with the cuts' conditions between product and sum the compiler
-            // does not fuse the two by itself.)
-            float pf[4], sb[4];
-            pf[0] = fmaf(keep_dt[0], A, cut_f[0]);
-            sb[3] = fmaf(keep_dt[3], A, cut_b[3]);
-#pragma unroll
-            for (int e = 1; e < 4; ++e) {
-                pf[e] = fmaf(keep_dt[e], A, pf[e - 1] + cut_f[e]);
-                sb[3 - e] = fmaf(keep_dt[3 - e], A, sb[4 - e] + cut_b[3 - e]);
-            }
-            const float tot = pf[3], tot_r = sb[0];
-            const float before = wave_incl_prefix(tot, lane) - tot, after = wave_incl_suffix(tot_r, lane) - tot_r;
-            keep_f[0] = fmaf(keep_dt[0], A, before + cut_f[0]);
-            keep_b[3] = fmaf(keep_dt[3], A, after + cut_b[3]);
-#pragma unroll
-            for (int e = 1; e < 4; ++e) {
-                keep_f[e] = before + pf[e];
-                keep_b[3 - e] = after + sb[3 - e];
-            }
+            chunk_sums_unrounded(keep_dt, A, cut_f, cut_b, lane, keep_f, keep_b);
             raw_lds_write128_at<0>(dts_a + lane * 16, f32x4{keep_dt[0], keep_dt[1], keep_dt[2], keep_dt[3]});
             raw_lds_write128_at<0>(csf_a + lane * 16, f32x4{keep_f[0], keep_f[1], keep_f[2], keep_f[3]});
             raw_lds_write128_at<0>(csb_a + lane * 16, f32x4{keep_b[0], keep_b[1], keep_b[2], keep_b[3]});
@@ -712,6 +713,29 @@ int launch_bmm_chunk_fwd(const bimamba2_params *p) {
         default: return BIMAMBA2_EUNSUPPORTED;
     }
     return check_launch();
+}
+
+template <typename T, bool UNROUNDED> static int launch_fwd_cumsum_cb_t(const bimamba2_params *p) {
+    const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, gx = (p->nheads + 3) / 4, ncs = gx * nc * p->batch;
+    const dim3 grid(ncs + (p->CB ? nqt * nqt * p->batch * nc * p->ngroups : 0));
+    switch (p->dt_dtype) {
+        case BIMAMBA2_F32: hipLaunchKernelGGL((fwd_cumsum_cb_kernel<T, float, UNROUNDED>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, gx, ncs, nqt); break;
+        case BIMAMBA2_BF16: hipLaunchKernelGGL((fwd_cumsum_cb_kernel<T, bf16_t, UNROUNDED>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, gx, ncs, nqt); break;
+        case BIMAMBA2_F16: hipLaunchKernelGGL((fwd_cumsum_cb_kernel<T, f16_t, UNROUNDED>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, gx, ncs, nqt); break;
+        default: return BIMAMBA2_EUNSUPPORTED;
+    }
+    return check_launch();
+}
+// states16: the states would travel in 16 bits, formed by the kernel that walks through several heads where it exists (which leaves
+// the sums to the stand-alone launch)
+int launch_fwd_cumsum_cb(const bimamba2_params *p, bool states16) {
+    const bool unrounded = chunk_state_does_cumsum(p) && !(states16 && chunk_state_uses_heads_kernel(p));
+    switch (p->dtype) {
+        case BIMAMBA2_F32: return launch_fwd_cumsum_cb_t<float, false>(p);
+        case BIMAMBA2_BF16: return unrounded ? launch_fwd_cumsum_cb_t<bf16_t, true>(p) : launch_fwd_cumsum_cb_t<bf16_t, false>(p);
+        case BIMAMBA2_F16: return unrounded ? launch_fwd_cumsum_cb_t<f16_t, true>(p) : launch_fwd_cumsum_cb_t<f16_t, false>(p);
+        default: return BIMAMBA2_EUNSUPPORTED;
+    }
 }
 
 // Whether the forward pass of this problem can keep its per-chunk states in the 16-bit type only, in states16_f/b: written

@@ -61,7 +61,7 @@ bool chunk_scan_uses_scan16(const bimamba2_params *p, bool bwd) {
 }
 
 template <typename T, bool BWD>
-static int launch_scan_t(const bimamba2_params *p) {
+static int launch_scan_t(const bimamba2_params *p, bool free16) {
     const int nc = nchunks(p);
     const int P = p->headdim, Q = p->chunk_size, N = p->dstate;
     constexpr int VS = 16 / (int)sizeof(T);
@@ -82,7 +82,7 @@ static int launch_scan_t(const bimamba2_params *p) {
     if constexpr (sizeof(T) == 2) {
         // the shapes of the 16-bit kernel with transposed products and a raw operand tile: it needs the 16-bit copies of the
         // entering states (the composites keep them at these shapes) and no CB
-        if (c16f && (BWD ? p->CBT : p->CB) == nullptr && chunk_scan_uses_scan16(p, BWD) && (p->causal || c16b))
+        if ((free16 || (c16f && (p->causal || c16b))) && (BWD ? p->CBT : p->CB) == nullptr && chunk_scan_uses_scan16(p, BWD))
             return launch_chunk_scan16(p, BWD);
         if (p->causal) {                                // single-direction comparator: the fused kernels only
             if (!scan_recomputes_cb(p, BWD)) return BIMAMBA2_EUNSUPPORTED;
@@ -107,11 +107,12 @@ static int launch_scan_t(const bimamba2_params *p) {
     return check_launch();
 }
 
-int launch_chunk_scan(const bimamba2_params *p, bool bwd) {
+// free16: the entering states are zero and have no tensors (one_chunk()), at a shape where they would travel as 16-bit copies
+int launch_chunk_scan(const bimamba2_params *p, bool bwd, bool free16) {
     switch (p->dtype) {
-        case BIMAMBA2_F32: return bwd ? launch_scan_t<float, true>(p) : launch_scan_t<float, false>(p);
-        case BIMAMBA2_BF16: return bwd ? launch_scan_t<bf16_t, true>(p) : launch_scan_t<bf16_t, false>(p);
-        case BIMAMBA2_F16: return bwd ? launch_scan_t<f16_t, true>(p) : launch_scan_t<f16_t, false>(p);
+        case BIMAMBA2_F32: return bwd ? launch_scan_t<float, true>(p, free16) : launch_scan_t<float, false>(p, free16);
+        case BIMAMBA2_BF16: return bwd ? launch_scan_t<bf16_t, true>(p, free16) : launch_scan_t<bf16_t, false>(p, free16);
+        case BIMAMBA2_F16: return bwd ? launch_scan_t<f16_t, true>(p, free16) : launch_scan_t<f16_t, false>(p, free16);
         default: return BIMAMBA2_EUNSUPPORTED;
     }
 }

@@ -118,6 +118,8 @@ __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba
     // One pair of state tiles where the map has room for one only (DS = 128) and the z-row area is in use; without a z gate
     // that area (32 KB, free once the K rows are done with) holds the second pair.
     const bool st_single = L::ST_BUFS == 1 && (BWD || p.has_z);
+    // (a sequence of one chunk without states of its own: the states entering it are zero and have no tensors)
+    const bool has_states = BWD ? p.dstates16_f != nullptr : p.states16_f != nullptr;
     auto st_buf_off = [&](int buf) __attribute__((always_inline)) {
         return L::ST_BUFS == 2 ? buf * 2 * L::ST_TILE : st_single ? 0 : buf * (L::ZR - L::ST);
     };
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba
             load16_to_lds_at<BWD>(kp, tile_off(ln, part, ks_bytes), smem + L::XR0 + buf * L::XR_STRIDE + wave * 2048 + part * 1024);
         } else if (part == 2) {
             const int dir = wave >> 3;
-            if (!(UNI && dir)) {
+            if (has_states && !(UNI && dir)) {
                 const int64_t so = ((int64_t)(b * nc + c) * H + h) * P * DS + (int64_t)p0 * DS;
                 const T *src = reinterpret_cast<const T *>(BWD ? (dir ? p.dstates16_b : p.dstates16_f) : (dir ? p.states16_b : p.states16_f));
                 const int sboff = st_buf_off(buf);
@@ -201,7 +203,7 @@ __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba
         for (int part = 0; part < 4; ++part) request_part(h, buf, part);
     };
     // requests of a head this wave issues (the vmcnt a wait for something older has to leave outstanding)
-    const int head_requests = 2 + ((UNI && wave >= 8) ? 0 : (DS == 64 ? 1 : 2)) + (wave < 3 ? 1 : 0);
+    const int head_requests = 2 + ((!has_states || (UNI && wave >= 8)) ? 0 : (DS == 64 ? 1 : 2)) + (wave < 3 ? 1 : 0);
 
     // ---- prologue: the K rows of the chunk (B, resp. C), this lane's own rows (C, resp. B), the first head's operands.  The
     // products below wait for the first two only; the head's operands land meanwhile.  (LDS accesses are raw from here on.)
@@ -428,7 +430,12 @@ __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba
             // row = [32 (j/2) + 4 (j%2)] + [8 (lr/4) + lr%4] the lane's part is one address and everything else a constant:
             // (row % 8) = lr%4 + 4 (j%2), so the chunk is (lg ^ lr%4) + 4 ((s%2) ^ (j%2)) + 8 (s/2).
             const unsigned st_lane = sb + L::ST + st_buf_off(cur) + (8 * (lr >> 2) + (lr & 3)) * ROWB + ((lg ^ (lr & 3)) << 4);
-            static_for<0, (UNI ? 1 : 2)>([&](auto DIR) __attribute__((always_inline)) {
+            if (!has_states) {
+                raw_lds_wait();
+                raw_lds_use(lor); raw_lds_use(upr);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+            } else static_for<0, (UNI ? 1 : 2)>([&](auto DIR) __attribute__((always_inline)) {
                 constexpr int dir = decltype(DIR)::value;
                 f32x4 tmp[4];
 #pragma unroll

@@ -24,6 +24,7 @@ __host__ __device__ inline int ddt_direct_planes(const bimamba2_params &p) {
 int launch_chunk_cumsum_fwd(const bimamba2_params *p);
 int launch_seq_boundaries(const bimamba2_params *p, int32_t *counts);
 int launch_bmm_chunk_fwd(const bimamba2_params *p);
+int launch_fwd_cumsum_cb(const bimamba2_params *p, bool states16);     // chunk cumsum and, with p->CB, C.B^T in one launch
 int launch_chunk_state(const bimamba2_params *p, bool dstates, bool cumsum = false);   // cumsum: also does the chunk cumsum
 bool chunk_state_does_cumsum(const bimamba2_params *p);
 bool chunk_state_narrow(const bimamba2_params *p, bool dstates);
@@ -36,7 +37,7 @@ bool chunk_states_in_16bit(const bimamba2_params *p);
 bool chunk_state_uses_heads_kernel(const bimamba2_params *p);
 int launch_chunk_state_heads(const bimamba2_params *p);
 int launch_state_passing_fwd(const bimamba2_params *p);
-int launch_chunk_scan(const bimamba2_params *p, bool bwd);
+int launch_chunk_scan(const bimamba2_params *p, bool bwd, bool free16 = false);
 // the 16-bit kernel of kernels_scan16.hip (launch_chunk_scan picks it where it applies)
 int launch_chunk_scan16(const bimamba2_params *p, bool bwd);
 // heads of one group that a workgroup of that kernel walks through (they share one C.B^T product)

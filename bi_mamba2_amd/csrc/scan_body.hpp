@@ -179,7 +179,10 @@ __device__ __forceinline__ void chunk_scan_work(const bimamba2_params &p, int nc
     f32x4 acc[QT][NJ] = {};
 
     // ---- part 1: states.  A = (C or B rows) * row scale, K = dstate; B operand = state tiles [p][n] in LDS ----
-    {
+    // (a sequence of one chunk without states of its own: the states entering it are zero and have no tensors)
+    const bool has_states = BWD ? p.dstates_f != nullptr || (NF > 0 && p.dstates16_f != nullptr) : p.states_f != nullptr || p.states16_f != nullptr;
+    if (!has_states) __syncthreads();
+    else {
         const int64_t so = ((int64_t)(b * nc + c) * H + h) * P * N + (int64_t)p0 * N;
         const float *stf = (BWD ? p.dstates_f : p.states_f) + so, *stb = (BWD ? p.dstates_b : p.states_b) + so;
         // one direction's product of the rows with the state tile in LDS, scaled row by row (rows 4*(l/16)+i of each tile) on

@@ -168,7 +168,9 @@ class _Call:
                p.C_sb, p.C_sl, p.C_sg, p.dx_sb, p.dx_sl, p.dB_sb, p.dB_sl, p.dC_sb, p.dC_sl, al(p.dB), al(p.dC), al(p.x), al(p.z), al(p.dout), al(p.Bm), al(p.Cm), al(p.out), al(p.out_x), al(p.dx),
                al(p.states_f), al(p.states_b), al(p.dstates_f), al(p.dstates_b),
                bool(p.states16_f), bool(p.dstates16_f), p.fwd_saved, al(p.states16_f), al(p.states16_b), al(p.final_f), al(p.final_b),
-               al(p.initial_f), al(p.initial_b), al(p.dfinal_f), al(p.dfinal_b), al(p.dinitial_f), al(p.dinitial_b))
+               al(p.initial_f), al(p.initial_b), al(p.dfinal_f), al(p.dfinal_b), al(p.dinitial_f), al(p.dinitial_b),
+               bool(p.final_f), bool(p.final_b), bool(p.initial_f), bool(p.initial_b), bool(p.dfinal_f), bool(p.dfinal_b), bool(p.dinitial_f),
+               bool(p.dinitial_b), bool(p.states16_b), bool(p.dstates16_b), bool(p.dstates_b))
         n = _WS_CACHE.get(key)
         if n is None:
             n = _WS_CACHE[key] = self._workspace_bytes(is_bwd)

@@ -64,9 +64,12 @@ typedef struct bimamba2_params {
     int32_t dtype;          /* BIMAMBA2_* : x, z, Bm, Cm, out, out_x, dout and their gradients */
     int32_t dt_dtype;       /* BIMAMBA2_* : dt and ddt */
     int32_t has_D, D_has_hdim, has_z, has_dt_bias, dt_softplus;
-    int32_t fwd_saved;      /* bimamba2_bwd only: dt_out, cs_f, cs_b, states_f, states_b hold what bimamba2_fwd left in
+    int32_t fwd_saved;      /* bimamba2_bwd: dt_out, cs_f, cs_b, states_f, states_b hold what bimamba2_fwd left in
                                them, so the backward pass does not recompute them.  3: CB and CBT hold what it left there too
-                               (1: they are recomputed where a kernel reads them) */
+                               (1: they are recomputed where a kernel reads them).
+                               4 is added where seqlen <= chunk_size, no states go in or out and the states' pointers are
+                               NULL in both passes (the states entering the one chunk are zero: none are kept or formed);
+                               bimamba2_fwd then takes 4 alone: a backward pass follows */
     int32_t causal;         /* 0: the bidirectional operator.  1: the single-direction (causal) operator built from the same
                                kernels with the reverse direction left out - the comparator the bidirectional pass is
                                timed against.  Every entry point follows it, but only for the shapes whose scan
