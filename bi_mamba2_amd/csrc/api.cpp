@@ -107,6 +107,10 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     const bool fwd_scan16 = !is_bwd && chunk_scan_uses_scan16(q, false) &&
                             (one ? one_chunk_free16(q, false) : (carve16 || q->states16_f) && (q->causal || carve16 || q->states16_b));
     if (is_bwd ? !(scan_recomputes_cb(q, true) && dcb_recomputes_cb(q)) : !(scan_recomputes_cb(q, false) || fwd_scan16)) need_f(q->CB, cbn);
+    // whether dbdc_both_by_heads() will hold (what is carved is aligned)
+    const bool by_heads = is_bwd && copies && !one && !q->dstates_f && dbdc_by_heads(q) &&
+                          (carve16 || (q->states16_f && q->states16_b && al16(q->states16_f) && al16(q->states16_b))) &&
+                          (!q->dstates16_f || (q->dstates16_b && al16(q->dstates16_f) && al16(q->dstates16_b)));
     if (carve16) {
         q->states16_f = cv.take<char>(stn * 2);
         q->states16_b = cv.take<char>(stn * 2);
@@ -125,7 +129,7 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     }
     if (is_bwd) {
         const size_t nqt = (Q + 63) / 64;
-        if (!q->dBs && !q->dCs) q->dbdc_heads = choose_dbdc_heads(q);
+        if (!q->dBs && !q->dCs) q->dbdc_heads = choose_dbdc_heads(q, by_heads);
         if (!q->dCB && !q->dCBT) q->dcb_slices = choose_dcb_slices(q);      // (which asks about the last launch, and that about the slices of dB and dC)
         need_f(q->dCB, cbn * dcb_slices(q));
         need_f(q->dCBT, cbn * dcb_slices(q));
@@ -552,9 +556,10 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     // the dCB kernel is bound by instruction issue and moves little data: right behind dz it runs while the memory system
     // still writes back dz's output, which the memory-bound kernels after it would otherwise wait behind
     const bool dx_db_dc = !one && dx_db_dc_merged(&q);      // (one launch at the end)
+    const bool both = !one && !dx_db_dc && dbdc_both_by_heads(&q);      // dC with dB
     if (dcb_sp && (ncb == dcb_slices(&q))) {
         // the backward state passing (streams, few instructions) rides along with the dCB kernel in one launch
-        if (!dx_db_dc && !one) TRY(bimamba2_chunk_scan_bwd_dc(&q));
+        if (!dx_db_dc && !one && !both) TRY(bimamba2_chunk_scan_bwd_dc(&q));
         if (!dz_dstates && !one) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
         REQUIRE(q.x); REQUIRE(q.dt_out); REQUIRE(q.cs_f); REQUIRE(q.cs_b); REQUIRE(q.dCB); REQUIRE(q.dCBT); REQUIRE(q.da_intra);
         if (!one) {
@@ -574,13 +579,16 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
             if (!dz_dstates) TRY(bimamba2_chunk_scan_bwd_dstates(&q));
         }
         if (!one) {
-            if (!dx_db_dc) TRY(bimamba2_chunk_scan_bwd_dc(&q));           // (between the two memory-bound state kernels: measured best)
+            if (!dx_db_dc && !both) TRY(bimamba2_chunk_scan_bwd_dc(&q));           // (between the two memory-bound state kernels: measured best)
             TRY(bimamba2_state_passing_bwd(&q));
         }
     }
     if (dx_db_dc) {
         REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dBs); REQUIRE(q.dCs); REQUIRE(q.u_f); REQUIRE(q.u_b); REQUIRE(q.v_f); REQUIRE(q.v_b);
         REQUIRE(q.states_f); REQUIRE(q.states_b); REQUIRE(q.dstates_f); REQUIRE(q.dstates_b);
+    } else if (both) {
+        REQUIRE(q.x); REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dBs); REQUIRE(q.dCs); REQUIRE(q.u_f); REQUIRE(q.u_b); REQUIRE(q.v_f); REQUIRE(q.v_b);
+        TRY(launch_dbdc_both(&q));
     } else if (!one) TRY(bimamba2_chunk_state_bwd_db(&q));
     ReduceJobs jobs;
     {

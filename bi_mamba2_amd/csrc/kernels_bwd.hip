@@ -15,6 +15,7 @@
 #include "dbdc_body.hpp"
 #include "dcb_body.hpp"
 #include "dcb_heads_body.hpp"
+#include "dbdc_heads_body.hpp"
 
 namespace bm2 {
 
@@ -546,6 +547,14 @@ int launch_state_passing_bwd(const bimamba2_params *p) {
 // =========================================================================================================
 // dB and dC, state part (the kernel for float32 state tensors: dbdc_body.hpp)
 // =========================================================================================================
+static bool dcb_aligned(const bimamba2_params *p);
+static bool dcb_rows_in_32bit(const bimamba2_params *p);
+static double dbdc_heads_cost(const bimamba2_params *p, int w, int hps);
+// 16-byte aligned rows of B and C
+static bool bmm_rows_aligned(const bimamba2_params *p) {
+    auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    return al(p->Bm) && al(p->Cm) && p->B_sb % 8 == 0 && p->B_sl % 8 == 0 && p->B_sg % 8 == 0 && p->C_sb % 8 == 0 && p->C_sl % 8 == 0 && p->C_sg % 8 == 0;
+}
 static inline int dbdc_heads(const bimamba2_params *p) { return p->dbdc_heads > 0 ? p->dbdc_heads : DBDC_HEADS; }
 static inline int dbdc_slices(const bimamba2_params *p) { return (p->nheads / p->ngroups + dbdc_heads(p) - 1) / dbdc_heads(p); }
 // of them, those there are to add up: none where nothing wrote a state part (one_chunk())
@@ -556,8 +565,23 @@ static inline int state_slices(const bimamba2_params *p) { return p->dBs ? dbdc_
 // then one per head; each slice more is a partial sum of each of dB and dC that is written and read again.  With eight heads
 // a slice, small problems leave most of the chip idle: 24 workgroups at batch 2 x 1500 with 8 heads of 128 channels, where the
 // two kernels took 22 us each and take 12 with one head a slice.
-int choose_dbdc_heads(const bimamba2_params *p) {
+int choose_dbdc_heads(const bimamba2_params *p, bool by_heads) {
     const int hpg = p->nheads / p->ngroups, nc = nchunks(p);
+    if (by_heads) {
+        // the same for the kernel whose waves take whole heads, dB and dC in one launch (us; a partial sum of each at 5 TB/s)
+        const double slice_cost = (double)p->batch * p->seqlen * p->ngroups * p->dstate * 8 * 2 / 5e6;
+        int best = hpg;
+        double best_cost = 0;
+        for (int s = 1; s <= std::min(hpg, DBDC_SLICES_MAX); ++s) {
+            const int hps = (hpg + s - 1) / s;
+            if ((hpg + hps - 1) / hps != s) continue;
+            double cost = dbdc_heads_cost(p, 4, hps);
+            for (int w = 2; w >= 1; w /= 2) cost = std::min(cost, dbdc_heads_cost(p, w, hps));
+            cost += s * slice_cost;
+            if (s == 1 || cost < best_cost) { best = hps; best_cost = cost; }
+        }
+        return best;
+    }
     const int64_t tiles = (int64_t)p->batch * nc * p->ngroups * ((p->chunk_size + 127) / 128);
     const double steps = ((p->headdim + 63) / 64) * ((p->dstate + 63) / 64);                             // per head
     const double slice_cost = (double)p->batch * p->seqlen * p->ngroups * p->dstate * 8 / 5e6 / 1.5;     // one partial sum at 5 TB/s, in steps of 1.5 us
@@ -572,6 +596,61 @@ int choose_dbdc_heads(const bimamba2_params *p) {
         if (k == DBDC_HEADS || cost < best_cost) { best = k; best_cost = cost; }
     }
     return best;
+}
+
+// dB and dC by waves that take whole heads (dbdc_heads_body.hpp): headdim and dstate 64, the states and their gradients in 16-bit
+// copies.  bwd_dbdc_dma_kernel below took 20.6 + 18.8 us for dC and dB at 4 x 2048 with 32 heads: its x and dout fragments come straight
+// from memory, 16 bytes of 16 different rows to a request, so the address unit was busy four times as long as the bytes
+// need, and a third of its life went by before the first product.  Here every request is of whole rows, a wave waits for nobody, and
+// both roles share a launch: 28.7; 4 x 4096, 8 groups of 4 heads 108 -> 70; 16 x 1024, 24 heads 61.5 -> 37.8.  What is left is the sums:
+// 32 additions of a state's product into the lane's sums and 32 into the rows' per 16 matrix instructions of 8 cycles.
+// (dC's workgroups in front)
+template <typename T, int W>
+__global__ __launch_bounds__(NTHREADS, 2) void bwd_dbdc_heads_kernel(const bimamba2_params p, int nc, int nqt, int hps, int gdx, int gdy, int gdz) {
+    __shared__ __attribute__((aligned(16))) unsigned char smem[DbdcHeadsMap<W>::LDS];
+    const int per = gdx * gdy, half = per * gdz, id = blockIdx.x % half;
+    BlockId bid = dcb_block_of(id % per, gdx, gdy, per, DCB_HEADS_RESIDENT);
+    bid.z = id / per;
+    if ((int)blockIdx.x >= half) bwd_dbdc_heads_body<T, true, W>(p, nc, nqt, hps, bid, smem);
+    else bwd_dbdc_heads_body<T, false, W>(p, nc, nqt, hps, bid, smem);
+}
+// us: with the chip full (two workgroups on a CU) a wave's head takes 5.6, with one on a CU 3.8, start and end 6.  dC and dB
+// in one launch: 4 x 2048, 32 heads, two slices: 28.7 with four waves to a tile (four heads each), one slice 34.5; with two waves
+// 36.6, with one 58.4; 4 x 4096 with 8 groups of 4 heads: 96, 77, 70 with four, two and one.
+static double dbdc_heads_cost(const bimamba2_params *p, int w, int hps) {
+    const int hpg = p->nheads / p->ngroups, nqt = (p->chunk_size + 63) / 64, slices = (hpg + hps - 1) / hps;
+    const double full = (double)p->batch * nchunks(p) * p->ngroups * nqt * w / 4 * slices * 2 / DCB_HEADS_RESIDENT;
+    const double rounds = std::max(1.0, (full + std::ceil(full)) / 2);      // (a last round that is nearly empty costs more than its share)
+    return rounds * (6 + (2 + 3.6 * std::min(std::max(full, 0.5), 1.0)) * ((std::min(hps, hpg) + w - 1) / w));
+}
+static int dbdc_waves(const bimamba2_params *p, int hps) {
+    int best = 4;
+    for (int w = 2; w >= 1; w /= 2)
+        if (dbdc_heads_cost(p, w, hps) < dbdc_heads_cost(p, best, hps)) best = w;
+    return best;
+}
+// the states' copies aside, which a caller may bring
+bool dbdc_by_heads(const bimamba2_params *p) {
+    return p->dtype != BIMAMBA2_F32 && !p->causal && p->headdim == 64 && p->dstate == 64 && p->chunk_size % 64 == 0 && dcb_aligned(p) && dcb_rows_in_32bit(p) &&
+           bmm_rows_aligned(p);
+}
+bool dbdc_both_by_heads(const bimamba2_params *p) {
+    auto al = [](const void *q) { return q && (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
+    return dbdc_by_heads(p) && al(p->states16_f) && al(p->states16_b) && al(p->dstates16_f) && al(p->dstates16_b);
+}
+template <typename T, int W> static void launch_dbdc_both_w(const bimamba2_params *p, int nqt, int hps) {
+    const int nc = nchunks(p), gdx = p->batch * nc * p->ngroups, gdy = (nqt * W + 3) / 4, gdz = dbdc_slices(p);
+    hipLaunchKernelGGL((bwd_dbdc_heads_kernel<T, W>), dim3(2 * gdx * gdy * gdz), dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, hps, gdx, gdy, gdz);
+}
+template <typename T> static int launch_dbdc_both_t(const bimamba2_params *p) {
+    const int nqt = p->chunk_size / 64, hps = dbdc_heads(p), W = dbdc_waves(p, hps);
+    if (W == 4) launch_dbdc_both_w<T, 4>(p, nqt, hps);
+    else if (W == 2) launch_dbdc_both_w<T, 2>(p, nqt, hps);
+    else launch_dbdc_both_w<T, 1>(p, nqt, hps);
+    return check_launch();
+}
+int launch_dbdc_both(const bimamba2_params *p) {
+    return p->dtype == BIMAMBA2_BF16 ? launch_dbdc_both_t<bf16_t>(p) : launch_dbdc_both_t<f16_t>(p);
 }
 
 // Two waves to a SIMD, said explicitly: with the bound left out the two-tile variant takes 140 us instead of 40 (float32, heads of 16,

@@ -54,7 +54,10 @@ int launch_bwd_dz_bmm(const bimamba2_params *p);       // dz and C.B^T in one la
 bool bwd_dz_dstates_fused(const bimamba2_params *p);   // dz and dstates as one launch
 int launch_bwd_dz_dstates(const bimamba2_params *p);
 int launch_state_passing_bwd(const bimamba2_params *p);
-int choose_dbdc_heads(const bimamba2_params *p);   // heads per slice of the dB / dC partial sums
+int choose_dbdc_heads(const bimamba2_params *p, bool by_heads);   // heads per slice of the dB / dC partial sums; by_heads: for the next three
+bool dbdc_by_heads(const bimamba2_params *p);       // dB and dC by waves that take whole heads, given 16-bit copies of the states
+bool dbdc_both_by_heads(const bimamba2_params *p);  // with them given
+int launch_dbdc_both(const bimamba2_params *p);     // both in one launch
 int launch_bwd_dbdc(const bimamba2_params *p, bool is_db);
 int launch_bwd_dcb(const bimamba2_params *p, bool add_up = true);   // add_up: also the launch that adds several head slices up
 int choose_dcb_slices(const bimamba2_params *p);

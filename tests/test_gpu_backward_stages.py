@@ -280,6 +280,55 @@ def test_state_parts_of_db_and_dc_with_narrow_states(ops, N, H, G, P, L, Q, dtyp
             assert float((g.reshape(b, H, -1)[:, :, :L] - want).norm() / want.norm()) < 1e-5
 
 
+@pytest.mark.parametrize("b,H,G,L,Q,hps,dtype", [
+    (1, 5, 1, 129, 64, 5, torch.bfloat16),        # four waves share a tile, one of them with two heads; one row in the last chunk
+    (1, 3, 1, 449, 256, 2, torch.float16),        # fewer heads than waves, the second slice with one; a ragged tile and one with no rows
+    (2, 26, 1, 300, 128, 13, torch.bfloat16),     # slices of more than eight heads
+    (16, 4, 2, 1030, 128, 2, torch.bfloat16),     # 576 tiles of two heads and role: two waves a tile
+    (16, 16, 8, 1030, 64, 2, torch.float16),      # 2176 tiles of two heads: one wave a tile
+    (4, 18, 9, 1030, 256, 1, torch.bfloat16),     # 900 tiles, two slices of one head each
+])
+def test_state_parts_of_db_and_dc_by_waves_that_take_heads(ops, monkeypatch, b, H, G, L, Q, hps, dtype):
+    """headdim and dstate 64 with the states and their gradients in 16-bit copies, both in one launch: against float64 on the
+    copies as they are.  Exact products, float32 sums over 64 terms and the heads: 1e-5 as above.  (Behind the sequence's end the rows'
+    sums are whatever they are: nothing reads them.)"""
+    P = N = 64
+    d = to_dev(make_case(b, L, H, P, G, N, dtype))
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(5)).to(dtype).cuda()
+    nc, hpg, kept = -(-L // Q), H // G, {}
+    own = ops._Call.workspace
+
+    def workspace(c, is_bwd):
+        if is_bwd:
+            c.p.dbdc_heads = hps
+            for name in ("dBs", "dCs"):
+                kept[name] = c.new(name, (-(-hpg // hps), b, L, G, N)).fill_(float("nan"))
+            for name in ("u_f", "u_b", "v_f", "v_b", "dt_out", "cs_f", "cs_b"):
+                kept[name] = c.new(name, (b, H, nc, Q))
+            for name in ("states16_f", "states16_b", "dstates16_f", "dstates16_b"):
+                kept[name] = c.new(name, (b, nc, H, P, N), dtype)
+        return own(c, is_bwd)
+
+    monkeypatch.setattr(ops._Call, "workspace", workspace)
+    ops._mamba_chunk_scan_combined_bwd(dout, d["x"], d["dt"], d["A"], d["B"], d["C"], None, Q, dt_bias=d["dt_bias"], dt_softplus=True)
+    k = {n: t.double() for n, t in kept.items()}
+    pad = lambda t: F.pad(t.double(), (0, 0, 0, 0, 0, nc * Q - L)).view(b, nc, Q, *t.shape[2:])
+    rows_of = lambda t: t.permute(0, 2, 3, 1)                                               # (b, nc, Q, H)
+    csf, csb, dt = (k[n] for n in ("cs_f", "cs_b", "dt_out"))
+    for out, name, rows, mate, w, states in (
+            ("dCs", "u", dout, d["C"], (csf.exp(), csb.exp()), "states16"),
+            ("dBs", "v", d["x"], d["B"], (dt * (csf[..., -1:] - csf).exp(), dt * (csb[..., :1] - csb).exp()), "dstates16")):
+        total = 0
+        for way, weight in zip("fb", w):
+            t = torch.matmul(pad(rows).transpose(2, 3), k[f"{states}_{way}"]).transpose(2, 3)              # (b, nc, Q, H, N)
+            total = total + rows_of(weight)[..., None] * t
+            want = (rows_of(weight) * (t * pad(mate).repeat_interleave(hpg, 3)).sum(-1)).permute(0, 3, 1, 2).reshape(b, H, -1)[:, :, :L]
+            got = k[f"{name}_{way}"].reshape(b, H, -1)
+            assert float((got[:, :, :L] - want).norm() / want.norm()) < 1e-5
+        total = total.view(b, nc, Q, G, hpg, N).sum(4).reshape(b, nc * Q, G, N)[:, :L]
+        assert float((k[out].sum(0) - total).norm() / total.norm()) < 1e-5
+
+
 @pytest.mark.parametrize("nc", [1, 7, 8, 9, 16, 17, 63, 64, 65, 129])
 @pytest.mark.parametrize("PN", [(8, 4), (40, 30)])
 def test_state_passing_over_many_chunks(ops, nc, PN):
