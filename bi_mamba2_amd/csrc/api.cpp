@@ -129,7 +129,7 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     }
     if (is_bwd) {
         const size_t nqt = (Q + 63) / 64;
-        if (!q->dBs && !q->dCs) q->dbdc_heads = choose_dbdc_heads(q, by_heads);
+        if (!q->dBs && !q->dCs) q->dbdc_heads = choose_dbdc_heads(q, by_heads, db_dc_roles(q, q->states16_f || q->dstates16_f));
         if (!q->dCB && !q->dCBT) q->dcb_slices = choose_dcb_slices(q);      // (which asks about the last launch, and that about the slices of dB and dC)
         need_f(q->dCB, cbn * dcb_slices(q));
         need_f(q->dCBT, cbn * dcb_slices(q));
@@ -556,7 +556,7 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     // the dCB kernel is bound by instruction issue and moves little data: right behind dz it runs while the memory system
     // still writes back dz's output, which the memory-bound kernels after it would otherwise wait behind
     const bool dx_db_dc = !one && dx_db_dc_merged(&q);      // (one launch at the end)
-    const bool both = !one && !dx_db_dc && dbdc_both_by_heads(&q);      // dC with dB
+    const bool by_heads = !one && !dx_db_dc && dbdc_both_by_heads(&q), both = by_heads || (!one && !dx_db_dc && db_dc_merged(&q));      // dC with dB
     if (dcb_sp && (ncb == dcb_slices(&q))) {
         // the backward state passing (streams, few instructions) rides along with the dCB kernel in one launch
         if (!dx_db_dc && !one && !both) TRY(bimamba2_chunk_scan_bwd_dc(&q));
@@ -588,7 +588,8 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
         REQUIRE(q.states_f); REQUIRE(q.states_b); REQUIRE(q.dstates_f); REQUIRE(q.dstates_b);
     } else if (both) {
         REQUIRE(q.x); REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dBs); REQUIRE(q.dCs); REQUIRE(q.u_f); REQUIRE(q.u_b); REQUIRE(q.v_f); REQUIRE(q.v_b);
-        TRY(launch_dbdc_both(&q));
+        if (!by_heads) { REQUIRE(q.states_f); REQUIRE(q.states_b); REQUIRE(q.dstates_f); REQUIRE(q.dstates_b); }
+        TRY(by_heads ? launch_dbdc_both(&q) : launch_db_dc(&q));
     } else if (!one) TRY(bimamba2_chunk_state_bwd_db(&q));
     ReduceJobs jobs;
     {

@@ -565,7 +565,8 @@ static inline int state_slices(const bimamba2_params *p) { return p->dBs ? dbdc_
 // then one per head; each slice more is a partial sum of each of dB and dC that is written and read again.  With eight heads
 // a slice, small problems leave most of the chip idle: 24 workgroups at batch 2 x 1500 with 8 heads of 128 channels, where the
 // two kernels took 22 us each and take 12 with one head a slice.
-int choose_dbdc_heads(const bimamba2_params *p, bool by_heads) {
+static int dbdc_places(const bimamba2_params *p) { return p->dstate <= 32 ? 512 : 256; }      // workgroups on the chip at once (narrow states: two to a CU)
+int choose_dbdc_heads(const bimamba2_params *p, bool by_heads, bool together) {
     const int hpg = p->nheads / p->ngroups, nc = nchunks(p);
     if (by_heads) {
         // the same for the kernel whose waves take whole heads, dB and dC in one launch (us; a partial sum of each at 5 TB/s)
@@ -585,7 +586,10 @@ int choose_dbdc_heads(const bimamba2_params *p, bool by_heads) {
     const int64_t tiles = (int64_t)p->batch * nc * p->ngroups * ((p->chunk_size + 127) / 128);
     const double steps = ((p->headdim + 63) / 64) * ((p->dstate + 63) / 64);                             // per head
     const double slice_cost = (double)p->batch * p->seqlen * p->ngroups * p->dstate * 8 / 5e6 / 1.5;     // one partial sum at 5 TB/s, in steps of 1.5 us
-    const int64_t places = p->dstate <= 32 ? 512 : 256;       // workgroups on the chip at once (narrow states: two to a CU)
+    // where both roles share a launch (db_dc_roles()) they share the chip, and half the slices are less to add up.  us a pass with one
+    // launch, slices as for two launches and as here: float32, 2 x 1111, 16 heads of 64, dstate 64, 190 -> 181; 4 x 1024, 8 heads of 128
+    // 231 -> 225; bfloat16, 4 x 2048, 16 heads of 16, dstate 16 139 -> 135
+    const int64_t places = dbdc_places(p) / (together ? 2 : 1);
     int best = DBDC_HEADS;
     double best_cost = 0;
     for (int k = DBDC_HEADS; k >= 1; --k) {
@@ -1959,6 +1963,7 @@ static RolesShape roles_shape(const bimamba2_params *p) {
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     r.dstates_fast = dcb_aligned(p) && p->headdim % 64 == 0 && p->dstate % 64 == 0 && al(p->Cm) && p->C_sb % vs == 0 && p->C_sl % vs == 0 && p->C_sg % vs == 0;
     r.dstates_narrow = chunk_state_narrow(p, true);
+    r.dx = true;
     r.dbdc_fast = dcb_aligned(p) && p->headdim % 64 == 0 && p->dstate % 64 == 0;
     return r;
 }
@@ -1987,9 +1992,24 @@ static bool dx_db_dc_pays(const bimamba2_params *p) {
     return dx <= (p->dstate <= 32 ? 2048 : p->dstate <= 64 ? 512 : 256);
 }
 
+// dB and dC in one launch, without dx where that does not pay (us a pass, two launches -> one: float32, 2 x 1111, 16 heads of 64, dstate
+// 64 190 -> 181; 4 x 1024, 8 heads of 128 235 -> 225; 4 x 2048, 16 heads of 64, dstate 128 598 -> 586; bfloat16, 8 x 1000, 16 heads
+// of 32, dstate 64 176 -> 169): neither role fills the chip for long, and each alone ends with a wait for its slowest workgroup.
+// 16-bit types lose by it where a role is many rounds of workgroups by itself, counted in heads of a place (8 x 2048: 32 heads of 64,
+// dstate 32, eight of them, 554 -> 567; 16 heads of 40, dstate 48, eight, 345 -> 349; the case above four); float32 does
+// not (8 x 2048, 32 heads of 64, dstate 64, sixteen, 1356 -> 1358; 2 x 3000, 8 groups of 8 heads of 32, twelve, 762 -> 716).
+bool db_dc_roles(const bimamba2_params *p, bool states16) {
+    const int64_t heads = (int64_t)p->batch * nchunks(p) * p->nheads * ((p->headdim + 63) / 64) * ((p->dstate + 63) / 64);
+    return !p->causal && p->chunk_size <= 128 && !states16 && !dbdc_wide16(p) && p->dstate <= 128 && (p->dtype == BIMAMBA2_F32 || heads <= 4 * dbdc_places(p));
+}
+bool db_dc_merged(const bimamba2_params *p) { return db_dc_roles(p, p->states16_f || p->dstates16_f) && dbdc_heads(p) <= DBDC_HEADS; }
 bool dx_db_dc_merged(const bimamba2_params *p) {
-    if (p->causal || p->chunk_size > 128 || !p->CBT || p->states16_f || p->dstates16_f || dbdc_wide16(p) || p->dstate > 128 || dbdc_heads(p) > DBDC_HEADS) return false;
-    return dx_db_dc_pays(p) && scan_is_fast(p, true);
+    return db_dc_merged(p) && p->CBT && dx_db_dc_pays(p) && scan_is_fast(p, true);
+}
+int launch_db_dc(const bimamba2_params *p) {
+    RolesShape r = roles_shape(p);
+    r.dx = false;
+    return p->dtype == BIMAMBA2_F32 ? launch_dx_db_dc_f32(p, r) : p->dtype == BIMAMBA2_BF16 ? launch_dx_db_dc_bf16(p, r) : launch_dx_db_dc_f16(p, r);
 }
 int launch_dx_db_dc(const bimamba2_params *p) {
     const RolesShape r = roles_shape(p);

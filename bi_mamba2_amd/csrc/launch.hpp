@@ -54,7 +54,7 @@ int launch_bwd_dz_bmm(const bimamba2_params *p);       // dz and C.B^T in one la
 bool bwd_dz_dstates_fused(const bimamba2_params *p);   // dz and dstates as one launch
 int launch_bwd_dz_dstates(const bimamba2_params *p);
 int launch_state_passing_bwd(const bimamba2_params *p);
-int choose_dbdc_heads(const bimamba2_params *p, bool by_heads);   // heads per slice of the dB / dC partial sums; by_heads: for the next three
+int choose_dbdc_heads(const bimamba2_params *p, bool by_heads, bool together);   // heads per slice of the dB / dC partial sums; by_heads: for the next three; together: db_dc_roles()
 bool dbdc_by_heads(const bimamba2_params *p);       // dB and dC by waves that take whole heads, given 16-bit copies of the states
 bool dbdc_both_by_heads(const bimamba2_params *p);  // with them given
 int launch_dbdc_both(const bimamba2_params *p);     // both in one launch
@@ -90,12 +90,15 @@ int launch_bwd_tail_small(const bimamba2_params *p, ReduceJobs *defer, int ncb);
 // launches of several roles (roles.hpp), with what their kernels' own launches know about the problem
 struct RolesShape {
     int nchunks, dcb_slices, dbdc_slices, dbdc_heads;
-    bool dcb_ring, dcb_fast, dstates_fast, dstates_narrow, dbdc_fast;
+    bool dcb_ring, dcb_fast, dstates_fast, dstates_narrow, dbdc_fast, dx;
 };
 bool dcb_dstates_merged(const bimamba2_params *p);      // dCB and dstates in one launch
 int launch_dcb_dstates(const bimamba2_params *p);
 bool dx_db_dc_merged(const bimamba2_params *p);         // dx, dB and dC in one launch
 int launch_dx_db_dc(const bimamba2_params *p);
+bool db_dc_roles(const bimamba2_params *p, bool states16);      // dB and dC in one launch, with dx or without; states16: the states in 16-bit copies
+bool db_dc_merged(const bimamba2_params *p);
+int launch_db_dc(const bimamba2_params *p);
 int launch_dcb_dstates_f32(const bimamba2_params *p, const RolesShape &r);
 int launch_dcb_dstates_bf16(const bimamba2_params *p, const RolesShape &r);
 int launch_dcb_dstates_f16(const bimamba2_params *p, const RolesShape &r);

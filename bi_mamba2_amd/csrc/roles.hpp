@@ -85,7 +85,7 @@ template <typename T> int launch_dcb_dstates_t(const bimamba2_params *p, const R
 
 template <typename T> int launch_dx_db_dc_t(const bimamba2_params *p, const RolesShape &r) {
     const int nc = r.nchunks, pw = scan_col_tile_of(p->headdim, p->dtype), npt = (p->headdim + pw - 1) / pw;
-    const int gdx = p->batch * nc * p->ngroups, ndx = p->batch * nc * p->nheads * npt, ndb = gdx * r.dbdc_slices;
+    const int gdx = p->batch * nc * p->ngroups, ndx = r.dx ? p->batch * nc * p->nheads * npt : 0, ndb = gdx * r.dbdc_slices;
     const dim3 grid(ndx + 2 * ndb);
     hipStream_t s = reinterpret_cast<hipStream_t>(p->stream);
 #define BM2_R(NJS, NT, NJ, FAST) hipLaunchKernelGGL((bwd_dx_db_dc_kernel<T, NJS, NT, NJ, FAST>), grid, dim3(DBDC_THREADS), 0, s, *p, nc, npt, ndx, ndb, gdx, r.dbdc_heads)

@@ -222,3 +222,15 @@ def test_launches_of_several_roles(ops, b, L, H, P, G, N, Q, dtype, z):
     tol = {torch.float32: 1e-6, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]      # (now and then one unit of the result's type)
     for g, w in ((got[3], dB), (got[4], dC)):
         assert float((g.double() - w.double()).norm()) <= tol * float(w.double().norm())
+
+
+@pytest.mark.parametrize("case", [
+    (3, 700, 16, 64, 2, 64, 128, torch.float32, True),        # 576 dx workgroups: dB and dC share a launch, dx has its own
+    (2, 260, 12, 128, 1, 128, 128, torch.float32, False),     # 288 of dstate 128
+    (3, 333, 30, 24, 3, 40, 64, torch.float32, True),         # no whole tiles
+    (8, 500, 20, 32, 1, 64, 128, torch.bfloat16, False),      # 640 heads' tiles of 16 bits: one launch
+    (9, 500, 32, 32, 1, 64, 128, torch.float16, True),        # 1152: two
+])
+def test_db_and_dc_in_one_launch(ops, case):
+    """the same where dx does not ride along"""
+    test_launches_of_several_roles(ops, *case)
