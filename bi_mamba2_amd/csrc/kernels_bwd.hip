@@ -1185,7 +1185,7 @@ __global__ __launch_bounds__(NTHREADS, W ? 2 : 1) void bwd_dcb_sp_kernel(const b
 // tiles (those on the diagonal take longer) while there are few rounds.  us with 4 / 2 / 1 waves (heads of 64, dstate 64):
 //   512 tiles: 4 heads 12 / 14 / 19, 32 heads 34 / 51 / 90; 1024: 4 heads 20 / 16 / 20, 24 heads 47 / 45 / 70; 2048: 4 heads 37 / 27 / 27,
 //   24 heads 93 / 78 / 102; 4096: 2 heads 62 / 41 / 34, 8 heads 90 / 80 / 72; 8192: 4 heads 130 / 98 / 81, 8 heads 181 / 149 / 137
-static int dcb_waves(const bimamba2_params *p, int slices) {
+static int dcb_waves(const bimamba2_params *p, int slices, double *us = nullptr) {
     const int nqt = (p->chunk_size + 63) / 64, heads = (p->nheads / p->ngroups + slices - 1) / slices;
     const double tiles = (double)p->batch * nchunks(p) * p->ngroups * nqt * nqt * slices;
     int best = 4;
@@ -1195,7 +1195,18 @@ static int dcb_waves(const bimamba2_params *p, int slices) {
         const double cost = (std::max(1.0, rounds) + (w == 1 ? 0.3 : 0.0)) * (8 + 2.9 * ((heads + w - 1) / w));
         if (w == 4 || cost < best_cost) { best = w; best_cost = cost; }
     }
+    if (us) *us = best_cost;
     return best;
+}
+// Whether the state passing that shares dCB's launch is the longer part: float32 states (their gradients read and written, the states read:
+// 12 bytes an element at 5 TB/s).  The ring's workgroups are four to a CU and stay so beside it, those of the kernel above fill the LDS by
+// twos and it has to wait for them.  us ring / heads: 8 x 2048, 32 heads, dstate 32 (200 MB) 65 / 76; 4 x 2048, dstate 96 (300 MB) 66 / 74; but
+// 4 x 2048, 8 groups, dstate 32 (100 MB) 54 / 51
+static bool dcb_sp_streams(const bimamba2_params *p, int slices) {
+    if (p->dstates16_f || !p->dstates_f) return false;
+    double us;
+    dcb_waves(p, slices, &us);
+    return (double)p->batch * nchunks(p) * p->nheads * p->headdim * p->dstate * (p->causal ? 12 : 24) / 5e6 > us;
 }
 template <typename T, bool UNI> static void launch_dcb_heads(const bimamba2_params *p, int nc, int nqt, int slices) {
     const int W = dcb_waves(p, slices), gdx = p->batch * nc * p->ngroups, gdy = (nqt * nqt * W + 3) / 4;
@@ -1328,7 +1339,7 @@ bool bwd_dcb_sp_merged(const bimamba2_params *p) {
 int launch_bwd_dcb_sp(const bimamba2_params *p, bool out16) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, PN = p->headdim * p->dstate;
     const int nsplit = (PN + SP_EPT * NTHREADS - 1) / (SP_EPT * NTHREADS), ndir = p->causal ? 1 : 2;
-    const int slices = dcb_slices(p), W = p->headdim == 64 ? dcb_waves(p, slices) : 0;
+    const int slices = dcb_slices(p), W = p->headdim == 64 && !dcb_sp_streams(p, slices) ? dcb_waves(p, slices) : 0;
     const int gdx = p->batch * nc * p->ngroups, gdy = W ? (nqt * nqt * W + 3) / 4 : nqt * nqt, nsp1 = nsplit * p->nheads * p->batch * ndir;
     // (two groups a workgroup of the state passing where that leaves as many workgroups as the chip holds beside the tiles, else fewer are
     // under way at once: 1 x 8192, 24 heads, 192 -> 96 workgroups 36.8 -> 37.5)

@@ -230,6 +230,7 @@ def test_launches_of_several_roles(ops, b, L, H, P, G, N, Q, dtype, z):
     (3, 333, 30, 24, 3, 40, 64, torch.float32, True),         # no whole tiles
     (8, 500, 20, 32, 1, 64, 128, torch.bfloat16, False),      # 640 heads' tiles of 16 bits: one launch
     (9, 500, 32, 32, 1, 64, 128, torch.float16, True),        # 1152: two
+    (4, 1030, 32, 64, 16, 96, 128, torch.bfloat16, True),     # two; the state passing is the longer part of dCB's launch
 ])
 def test_db_and_dc_in_one_launch(ops, case):
     """the same where dx does not ride along"""
