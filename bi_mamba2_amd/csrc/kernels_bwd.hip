@@ -343,10 +343,10 @@ constexpr int SP_FLUSH = 64;
 // groups, 16 chunks 129 -> 125; dstate 128, 2 x 3001, 24 heads 36 -> 34.
 inline int sp_bwd_groups(int nc) { return nc <= 2 ? 4 : nc <= 4 ? 2 : 1; }
 template <typename T16, bool PREV16, bool DS16, bool DP16, bool AHEAD, int NCH, int NG>
-__device__ __forceinline__ void state_passing_bwd_groups(const bimamba2_params &p, int nc, int nsplit, int ndir, BlockId bid) {
+__device__ __forceinline__ void state_passing_bwd_groups(const bimamba2_params &p, int nc, int nsplit, int ndir, BlockId bid, float (*red)[4]) {
     struct alignas(8) V4 { T16 v[4]; };
     constexpr int NU = NCH * NG, FLUSH = AHEAD && NG == 1 ? SP_FLUSH : NU > SP_CH ? NU : SP_CH;
-    __shared__ float red[FLUSH][4];
+    static_assert(FLUSH <= SP_FLUSH, "rows of red");
     const int PN = p.headdim * p.dstate;
     const int split = bid.x * NG, h = bid.y, b = bid.z / ndir, dir = bid.z % ndir;   // ndir = 1: forward direction only
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -488,21 +488,22 @@ __device__ __forceinline__ void state_passing_bwd_groups(const bimamba2_params &
         for (int u = 0; u < NG; ++u)
             if (live[u]) *reinterpret_cast<f32x4 *>(dini + bh + e[u]) = g[u];
 }
-// ngr: groups a workgroup (2 also for long sequences, where TWO)
+// red: SP_FLUSH rows of LDS; ngr: groups a workgroup (2 also for long sequences, where TWO)
 template <typename T16, bool PREV16, bool DS16, bool DP16 = false, bool AHEAD = false, bool TWO = false>
-__device__ __forceinline__ void state_passing_bwd_vec_body(const bimamba2_params &p, int nc, int nsplit, int ndir, BlockId bid, int ngr = 1) {
-    if (nc == 1) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 1, 4>(p, nc, nsplit, ndir, bid);
-    else if (nc == 2) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 2, 4>(p, nc, nsplit, ndir, bid);
-    else if (nc <= 4) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 4, 2>(p, nc, nsplit, ndir, bid);
+__device__ __forceinline__ void state_passing_bwd_vec_body(const bimamba2_params &p, int nc, int nsplit, int ndir, BlockId bid, float (*red)[4], int ngr = 1) {
+    if (nc == 1) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 1, 4>(p, nc, nsplit, ndir, bid, red);
+    else if (nc == 2) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 2, 4>(p, nc, nsplit, ndir, bid, red);
+    else if (nc <= 4) state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, 4, 2>(p, nc, nsplit, ndir, bid, red);
     else {
         if constexpr (TWO)
-            if (ngr == 2) return state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, SP_CH, 2>(p, nc, nsplit, ndir, bid);
-        state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, SP_CH, 1>(p, nc, nsplit, ndir, bid);
+            if (ngr == 2) return state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, SP_CH, 2>(p, nc, nsplit, ndir, bid, red);
+        state_passing_bwd_groups<T16, PREV16, DS16, DP16, AHEAD, SP_CH, 1>(p, nc, nsplit, ndir, bid, red);
     }
 }
 template <typename T16, bool PREV16, bool DS16, bool DP16 = false>
 __global__ __launch_bounds__(NTHREADS) void state_passing_bwd_vec_kernel(const bimamba2_params p, int nc, int nsplit, int ndir) {
-    state_passing_bwd_vec_body<T16, PREV16, DS16, DP16, true>(p, nc, nsplit, ndir, BlockId{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z});
+    __shared__ float red[SP_FLUSH][4];
+    state_passing_bwd_vec_body<T16, PREV16, DS16, DP16, true>(p, nc, nsplit, ndir, BlockId{(int)blockIdx.x, (int)blockIdx.y, (int)blockIdx.z}, red);
 }
 
 int launch_state_passing_bwd(const bimamba2_params *p) {
@@ -1164,8 +1165,9 @@ __global__ __launch_bounds__(NTHREADS, 2) void bwd_dcb_heads_kernel(const bimamb
 template <typename T, bool UNI, int W>
 __global__ __launch_bounds__(NTHREADS, W ? 2 : 1) void bwd_dcb_sp_kernel(const bimamba2_params p, int nc, int nqt, int gdx, int gdy, int gdz, int nsplit, int nspx, int ndir, bool out16) {
     const int id = blockIdx.x, per = gdx * gdy, ndcb = per * gdz;
+    // (one place for both roles: with 1 KB more the ring's workgroups are three to a CU instead of four: 2 x 8192, 24 heads of 128 160 us instead of 148)
+    __shared__ __attribute__((aligned(16))) unsigned char smem[W ? DcbHeadsMap<W ? W : 1>::LDS : DcbRingMap<64>::LDS];
     if (id < ndcb) {
-        __shared__ __attribute__((aligned(16))) unsigned char smem[W ? DcbHeadsMap<W ? W : 1>::LDS : DcbRingMap<64>::LDS];
         BlockId tile = dcb_block_of(id % per, gdx, gdy, per, W ? DCB_HEADS_RESIDENT : 1024);
         tile.z = id / per;
         if constexpr (W > 0) bwd_dcb_heads_body<T, UNI, W>(p, nc, nqt, tile, gdx, gdz, smem, out16);
@@ -1174,9 +1176,10 @@ __global__ __launch_bounds__(NTHREADS, W ? 2 : 1) void bwd_dcb_sp_kernel(const b
         const int k = id - ndcb;                  // grid (nspx, nheads, batch * ndir) of the state passing
         const BlockId sb{k % nspx, (k / nspx) % p.nheads, k / (nspx * p.nheads)};
         const int ngr = (nsplit + nspx - 1) / nspx;
-        if (p.dstates_f == nullptr) state_passing_bwd_vec_body<T, true, true, true, false, W != 0>(p, nc, nsplit, ndir, sb, ngr);
-        else if (p.dstates16_f == nullptr) state_passing_bwd_vec_body<T, false, false, false, false, W != 0>(p, nc, nsplit, ndir, sb, ngr);
-        else state_passing_bwd_vec_body<T, true, true>(p, nc, nsplit, ndir, sb);
+        float (*red)[4] = reinterpret_cast<float (*)[4]>(smem);
+        if (p.dstates_f == nullptr) state_passing_bwd_vec_body<T, true, true, true, false, W != 0>(p, nc, nsplit, ndir, sb, red, ngr);
+        else if (p.dstates16_f == nullptr) state_passing_bwd_vec_body<T, false, false, false, false, W != 0>(p, nc, nsplit, ndir, sb, red, ngr);
+        else state_passing_bwd_vec_body<T, true, true>(p, nc, nsplit, ndir, sb, red);
     }
 }
 // Waves that share a tile of the kernel above.  More of them split a tile's heads and finish sooner, fewer leave out the exchange at the end
