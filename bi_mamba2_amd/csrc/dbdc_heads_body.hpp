@@ -1,4 +1,4 @@
-// The work of one workgroup of the dB / dC kernel (state parts) for 16-bit types, headdim and dstate 64: a wave takes whole heads.
+// The work of one workgroup of the dB / dC kernel (state parts) for 16-bit types, dstate 64 and headdim 64 or 128: a wave takes whole heads.
 #pragma once
 #include "common.hpp"
 #include "dcb_heads_body.hpp"
@@ -10,7 +10,7 @@ namespace bm2 {
 // direction after the other.  Its rows' B (C) values (64 registers) and the sums of dB (dC) (64) stay in registers over the heads, a product
 // takes another 64; a head's x (dout) rows and a state tile come by direct loads into the wave's own 16 KB of LDS, the second direction's
 // tile into the place of the first one's as soon as that has been read, the next head's operands behind them.  The waves' sums are added
-// up in wave order at the end.
+// up in wave order at the end.  A wider head is taken 64 columns of it at a time: its pieces' products add up in the same registers.
 // W waves share 64 rows, so a workgroup of four waves has 4 / W row tiles.
 template <int W> struct DbdcHeadsMap {
     static constexpr int TILES = 4 / W, TILE = 64 * 64 * 2, RING = 2 * TILE;
@@ -27,7 +27,8 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
     typedef typename M::Frag Frag;
     typedef DbdcHeadsMap<W> L;
     static_assert(sizeof(T) == 2, "16-bit operands");
-    constexpr int N = 64, P = 64;
+    constexpr int N = 64;
+    const int P = p.headdim, np = P / 64;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int hw = wave % W, ti = wave / W;
     const int rt = bid.y * L::TILES + ti;
@@ -38,7 +39,7 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
     const int hh0 = bid.z * hps, nhs = max(min(hpg, hh0 + hps) - hh0, 0), nhw = nhs > hw ? (nhs - hw + W - 1) / W : 0;
     const int h0 = g * hpg + hh0 + hw;
     const bool live = rt < nqt && valid > 0;
-    const int nit = live ? nhw : 0;
+    const int nit = live ? nhw * np : 0;
 
     unsigned char *ring = smem + wave * L::RING, *vec = smem + L::VEC + wave * L::VEC_WAVE;
     const unsigned ring_a = lds_addr(ring), vec_a = lds_addr(vec);
@@ -63,6 +64,9 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
         c2 = uniform_ptr(p.cs_b + o);
         c3 = uniform_ptr(p.dt_out + o);
     }
+    // from a head's last piece to the first one of the wave's next head
+    const int64_t x_wrap = (x_head * W - (np - 1) * 64) * (int64_t)sizeof(T), s_wrap = ((int64_t)P * W - (np - 1) * 64) * N * (int64_t)sizeof(T);
+    int asked = 0, piece = 0;                      // of the head to come, of the one in hand
     // rows of 128 bytes to their place, 8 a request: 16-byte unit u of row r at u ^ r % 8
     auto request_rows = [&](const char *base, unsigned stride, int valid, unsigned char *to) __attribute__((always_inline)) {
         const int ln = lane_number();
@@ -94,11 +98,17 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
             __builtin_amdgcn_global_load_lds((gbl_ptr_t)(c1 + (Q - 1) * 4), (lds_ptr_t)(vec + 1280), 4, 0, 0);
             __builtin_amdgcn_global_load_lds((gbl_ptr_t)c2, (lds_ptr_t)(vec + 1536), 4, 0, 0);
         }
-        c1 += cs_head * 4;
-        c2 += cs_head * 4;
-        c3 += cs_head * 4;
-        xbase += x_head * W * (int64_t)sizeof(T);
-        sf += (int64_t)P * N * W * (int64_t)sizeof(T);
+        if (++asked < np) {
+            xbase += 64 * sizeof(T);
+            sf += 64 * N * sizeof(T);
+        } else {
+            asked = 0;
+            c1 += cs_head * 4;
+            c2 += cs_head * 4;
+            c3 += cs_head * 4;
+            xbase += x_wrap;
+            sf += s_wrap;
+        }
     };
 
     // ---- this lane's B (C) values: row 16 q + 4 lg + i, column 16 j + lr; the rows pass through the ring
@@ -129,6 +139,7 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
     }
     const int64_t uv0 = (((int64_t)b * H + h0) * nc + c) * Q + r0;
     float *uf = (IS_DB ? p.v_f : p.u_f) + uv0, *ub = (IS_DB ? p.v_b : p.u_b) + uv0;
+    float part[2] = {0.f, 0.f};                    // of a row's sum: the head's pieces so far
 #pragma unroll 1
     for (int it = 0; it < nit; ++it) {
         const int ln = lane_number(), lr = ln & 15, lg = ln >> 4;
@@ -185,7 +196,7 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
                 if (q0 == 2) {
                     if (dir == 0) {
                         request_state(sb);
-                        sb += (int64_t)P * N * W * (int64_t)sizeof(T);
+                        sb += piece + 1 < np ? 64 * N * (int64_t)sizeof(T) : s_wrap;
                     } else if (it + 1 < nit) request_head();
                 }
                 f32x4 s4[2] = {raw_lds_read_at<f32x4, q0 * 64>(va + lg * 16), raw_lds_read_at<f32x4, q0 * 64 + 64>(va + lg * 16)};
@@ -212,10 +223,14 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
             raw_lds_wait();
             raw_lds_use(srow);
             const float v = dpp_fold<0xb1>(dpp_fold<0x4e>(u[0], u[1], ln & 2), dpp_fold<0x4e>(u[2], u[3], ln & 2), ln & 1) * srow;
-            (dir ? ub : uf)[row] = row < valid ? v : 0.f;         // (without a branch: the waits count this store)
+            part[dir] = piece ? part[dir] + v : v;
+            (dir ? ub : uf)[row] = row < valid ? part[dir] : 0.f;         // (without a branch: the waits count this store)
         });
-        uf += cs_head;
-        ub += cs_head;
+        if (++piece == np) {
+            piece = 0;
+            uf += cs_head;
+            ub += cs_head;
+        }
     }
     // ---- the waves' shares are added up: wave hw owns the stripes q with q % W == hw
     const int le = lane_number(), lre = le & 15, lge = le >> 4;

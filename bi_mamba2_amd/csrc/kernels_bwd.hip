@@ -603,11 +603,12 @@ int choose_dbdc_heads(const bimamba2_params *p, bool by_heads, bool together) {
     return best;
 }
 
-// dB and dC by waves that take whole heads (dbdc_heads_body.hpp): headdim and dstate 64, the states and their gradients in 16-bit
+// dB and dC by waves that take whole heads (dbdc_heads_body.hpp): headdim 64 or 128, dstate 64, the states and their gradients in 16-bit
 // copies.  bwd_dbdc_dma_kernel below took 20.6 + 18.8 us for dC and dB at 4 x 2048 with 32 heads: its x and dout fragments come straight
 // from memory, 16 bytes of 16 different rows to a request, so the address unit was busy four times as long as the bytes
 // need, and a third of its life went by before the first product.  Here every request is of whole rows, a wave waits for nobody, and
-// both roles share a launch: 28.7; 4 x 4096, 8 groups of 4 heads 108 -> 70; 16 x 1024, 24 heads 61.5 -> 37.8.  What is left is the sums:
+// both roles share a launch: 28.7; 4 x 4096, 8 groups of 4 heads 108 -> 70; 16 x 1024, 24 heads 61.5 -> 37.8; heads
+// of 128: 2 x 1500, 8 heads 18.6 -> 13.5; 4 x 2048, 16 heads 33.5 -> 28.5; 2 x 8192, 24 heads in 4 groups 97 -> 82.  What is left is the sums:
 // 32 additions of a state's product into the lane's sums and 32 into the rows' per 16 matrix instructions of 8 cycles.
 // (dC's workgroups in front)
 template <typename T, int W>
@@ -626,7 +627,7 @@ static double dbdc_heads_cost(const bimamba2_params *p, int w, int hps) {
     const int hpg = p->nheads / p->ngroups, nqt = (p->chunk_size + 63) / 64, slices = (hpg + hps - 1) / hps;
     const double full = (double)p->batch * nchunks(p) * p->ngroups * nqt * w / 4 * slices * 2 / DCB_HEADS_RESIDENT;
     const double rounds = std::max(1.0, (full + std::ceil(full)) / 2);      // (a last round that is nearly empty costs more than its share)
-    return rounds * (6 + (2 + 3.6 * std::min(std::max(full, 0.5), 1.0)) * ((std::min(hps, hpg) + w - 1) / w));
+    return rounds * (6 + (2 + 3.6 * std::min(std::max(full, 0.5), 1.0)) * ((std::min(hps, hpg) + w - 1) / w) * (p->headdim / 64));
 }
 static int dbdc_waves(const bimamba2_params *p, int hps) {
     int best = 4;
@@ -636,7 +637,7 @@ static int dbdc_waves(const bimamba2_params *p, int hps) {
 }
 // the states' copies aside, which a caller may bring
 bool dbdc_by_heads(const bimamba2_params *p) {
-    return p->dtype != BIMAMBA2_F32 && !p->causal && p->headdim == 64 && p->dstate == 64 && p->chunk_size % 64 == 0 && dcb_aligned(p) && dcb_rows_in_32bit(p) &&
+    return p->dtype != BIMAMBA2_F32 && !p->causal && p->headdim % 64 == 0 && p->dstate == 64 && p->chunk_size % 64 == 0 && dcb_aligned(p) && dcb_rows_in_32bit(p) &&
            bmm_rows_aligned(p);
 }
 bool dbdc_both_by_heads(const bimamba2_params *p) {

@@ -280,19 +280,21 @@ def test_state_parts_of_db_and_dc_with_narrow_states(ops, N, H, G, P, L, Q, dtyp
             assert float((g.reshape(b, H, -1)[:, :, :L] - want).norm() / want.norm()) < 1e-5
 
 
-@pytest.mark.parametrize("b,H,G,L,Q,hps,dtype", [
-    (1, 5, 1, 129, 64, 5, torch.bfloat16),        # four waves share a tile, one of them with two heads; one row in the last chunk
-    (1, 3, 1, 449, 256, 2, torch.float16),        # fewer heads than waves, the second slice with one; a ragged tile and one with no rows
-    (2, 26, 1, 300, 128, 13, torch.bfloat16),     # slices of more than eight heads
-    (16, 4, 2, 1030, 128, 2, torch.bfloat16),     # 576 tiles of two heads and role: two waves a tile
-    (16, 16, 8, 1030, 64, 2, torch.float16),      # 2176 tiles of two heads: one wave a tile
-    (4, 18, 9, 1030, 256, 1, torch.bfloat16),     # 900 tiles, two slices of one head each
+@pytest.mark.parametrize("b,H,G,L,Q,hps,dtype,P", [
+    (1, 5, 1, 129, 64, 5, torch.bfloat16, 64),        # four waves share a tile, one of them with two heads; one row in the last chunk
+    (1, 3, 1, 449, 256, 2, torch.float16, 64),        # fewer heads than waves, the second slice with one; a ragged tile and one with no rows
+    (2, 26, 1, 300, 128, 13, torch.bfloat16, 64),     # slices of more than eight heads
+    (16, 4, 2, 1030, 128, 2, torch.bfloat16, 64),     # 576 tiles of two heads and role: two waves a tile
+    (16, 16, 8, 1030, 64, 2, torch.float16, 64),      # 2176 tiles of two heads: one wave a tile
+    (4, 18, 9, 1030, 256, 1, torch.bfloat16, 64),     # 900 tiles, two slices of one head each
+    (1, 7, 1, 200, 128, 7, torch.float16, 128),       # heads in two pieces
+    (8, 4, 2, 1030, 64, 2, torch.bfloat16, 128),
 ])
-def test_state_parts_of_db_and_dc_by_waves_that_take_heads(ops, monkeypatch, b, H, G, L, Q, hps, dtype):
-    """headdim and dstate 64 with the states and their gradients in 16-bit copies, both in one launch: against float64 on the
-    copies as they are.  Exact products, float32 sums over 64 terms and the heads: 1e-5 as above.  (Behind the sequence's end the rows'
+def test_state_parts_of_db_and_dc_by_waves_that_take_heads(ops, monkeypatch, b, H, G, L, Q, hps, dtype, P):
+    """dstate 64, headdim 64 and 128 with the states and their gradients in 16-bit copies, both in one launch: against float64 on the
+    copies as they are.  Exact products, float32 sums over P terms and the heads: 1e-5 as above.  (Behind the sequence's end the rows'
     sums are whatever they are: nothing reads them.)"""
-    P = N = 64
+    N = 64
     d = to_dev(make_case(b, L, H, P, G, N, dtype))
     dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(5)).to(dtype).cuda()
     nc, hpg, kept = -(-L // Q), H // G, {}
