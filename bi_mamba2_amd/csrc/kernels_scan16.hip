@@ -105,7 +105,9 @@ template <int I, int N, class F> __device__ __forceinline__ void static_for(F &&
 // hpw: heads per workgroup (divides nheads / ngroups, <= S16_MAX_HEADS); blockIdx.x = ((pt * nslices + slice) * nbc + bc).
 // DCOLS (mirror): dD per (head, headdim column); else one value per head.
 // DS: the state dimension, 64 or 128 (128: forward only).
-template <typename T, bool BWD, bool UNI, bool DCOLS = false, int DS = 64>
+// STATES = false: a sequence of one chunk without states of its own: the states entering it are zero and have no tensors.  (A kernel of its own: asked at
+// run time the question costs the others 1 to 2 %, 42.6 -> 43.6 us at 4 x 2048, 32 heads.)
+template <typename T, bool BWD, bool UNI, bool DCOLS = false, int DS = 64, bool STATES = true>
 __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba2_params p, int nc, int npt, int hpw) {
     typedef Mma<T> M;
     typedef typename M::Frag Frag;
@@ -118,8 +120,6 @@ __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba
     // One pair of state tiles where the map has room for one only (DS = 128) and the z-row area is in use; without a z gate
     // that area (32 KB, free once the K rows are done with) holds the second pair.
     const bool st_single = L::ST_BUFS == 1 && (BWD || p.has_z);
-    // (a sequence of one chunk without states of its own: the states entering it are zero and have no tensors)
-    const bool has_states = BWD ? p.dstates16_f != nullptr : p.states16_f != nullptr;
     auto st_buf_off = [&](int buf) __attribute__((always_inline)) {
         return L::ST_BUFS == 2 ? buf * 2 * L::ST_TILE : st_single ? 0 : buf * (L::ZR - L::ST);
     };
@@ -173,7 +173,7 @@ __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba
             load16_to_lds_at<BWD>(kp, tile_off(ln, part, ks_bytes), smem + L::XR0 + buf * L::XR_STRIDE + wave * 2048 + part * 1024);
         } else if (part == 2) {
             const int dir = wave >> 3;
-            if (has_states && !(UNI && dir)) {
+            if (STATES && !(UNI && dir)) {
                 const int64_t so = ((int64_t)(b * nc + c) * H + h) * P * DS + (int64_t)p0 * DS;
                 const T *src = reinterpret_cast<const T *>(BWD ? (dir ? p.dstates16_b : p.dstates16_f) : (dir ? p.states16_b : p.states16_f));
                 const int sboff = st_buf_off(buf);
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba
         for (int part = 0; part < 4; ++part) request_part(h, buf, part);
     };
     // requests of a head this wave issues (the vmcnt a wait for something older has to leave outstanding)
-    const int head_requests = 2 + ((!has_states || (UNI && wave >= 8)) ? 0 : (DS == 64 ? 1 : 2)) + (wave < 3 ? 1 : 0);
+    const int head_requests = 2 + ((!STATES || (UNI && wave >= 8)) ? 0 : (DS == 64 ? 1 : 2)) + (wave < 3 ? 1 : 0);
 
     // ---- prologue: the K rows of the chunk (B, resp. C), this lane's own rows (C, resp. B), the first head's operands.  The
     // products below wait for the first two only; the head's operands land meanwhile.  (LDS accesses are raw from here on.)
@@ -430,7 +430,7 @@ __global__ __launch_bounds__(S16_THREADS) void chunk_scan16_kernel(const bimamba
             // row = [32 (j/2) + 4 (j%2)] + [8 (lr/4) + lr%4] the lane's part is one address and everything else a constant:
             // (row % 8) = lr%4 + 4 (j%2), so the chunk is (lg ^ lr%4) + 4 ((s%2) ^ (j%2)) + 8 (s/2).
             const unsigned st_lane = sb + L::ST + st_buf_off(cur) + (8 * (lr >> 2) + (lr & 3)) * ROWB + ((lg ^ (lr & 3)) << 4);
-            if (!has_states) {
+            if constexpr (!STATES) {
                 raw_lds_wait();
                 raw_lds_use(lor); raw_lds_use(upr);
 #pragma unroll
@@ -752,21 +752,24 @@ static int launch_scan16_t(const bimamba2_params *p, int nc) {
     const int npt = p->headdim / 64, hpw = scan16_heads_per_block(p, nc);
     dim3 grid(p->batch * nc * (p->nheads / hpw) * npt);
     hipStream_t s = reinterpret_cast<hipStream_t>(p->stream);
+    const bool states = BWD ? p->dstates16_f != nullptr : p->states16_f != nullptr;
+#define BM2_S16(DCOLS, DS)                                                                                                                        \
+    do {                                                                                                                                          \
+        if (p->causal) hipLaunchKernelGGL((chunk_scan16_kernel<T, BWD, true, DCOLS, DS>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);         \
+        else if (states) hipLaunchKernelGGL((chunk_scan16_kernel<T, BWD, false, DCOLS, DS>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);      \
+        else hipLaunchKernelGGL((chunk_scan16_kernel<T, BWD, false, DCOLS, DS, false>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);           \
+    } while (0)
+    if (p->causal && !states) return BIMAMBA2_EINVAL;
     if (p->dstate == 128) {
         // the forward kernel only (launch_chunk_scan sends the mirror of this shape elsewhere)
-        if constexpr (!BWD) {
-            if (p->causal) hipLaunchKernelGGL((chunk_scan16_kernel<T, false, true, false, 128>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);
-            else hipLaunchKernelGGL((chunk_scan16_kernel<T, false, false, false, 128>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);
-        } else {
-            return BIMAMBA2_EUNSUPPORTED;
-        }
+        if constexpr (!BWD) BM2_S16(false, 128);
+        else return BIMAMBA2_EUNSUPPORTED;
     } else if (BWD && p->has_D && p->D_has_hdim) {
-        if (p->causal) hipLaunchKernelGGL((chunk_scan16_kernel<T, BWD, true, BWD>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);
-        else hipLaunchKernelGGL((chunk_scan16_kernel<T, BWD, false, BWD>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);
+        BM2_S16(BWD, 64);
     } else {
-        if (p->causal) hipLaunchKernelGGL((chunk_scan16_kernel<T, BWD, true>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);
-        else hipLaunchKernelGGL((chunk_scan16_kernel<T, BWD, false>), grid, dim3(S16_THREADS), 0, s, *p, nc, npt, hpw);
+        BM2_S16(false, 64);
     }
+#undef BM2_S16
     return check_launch();
 }
 
