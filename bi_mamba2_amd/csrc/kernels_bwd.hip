@@ -1314,18 +1314,12 @@ int choose_dcb_slices(const bimamba2_params *p) {
     int wanted = usual;
     if (dcb_recomputes_cb(p)) {
         if (hpg <= 16 && !bwd_tail_merged(p) && !bwd_tail_small(p)) return usual;
-        if (p->headdim == 64) {
-            // Waves that take whole heads: their cost against that of a slice more to write and add up.  us of dCB with the state passing beside it
-            // + the last launch, 1 / 2 / 4 slices: 64 tiles of 64 heads 62 / 43 / 37; 128 of 24 heads 35 / 30 / 34; 144 of 16 30 / 29 / 34; 256 of 24
-            // 37 / 36 / 41; 384 of 32 49 / 54 / 65
-            double best = 0;
-            for (int sl = usual; sl <= std::min(hpg, std::max(usual, 8)); ++sl) {
-                double us;
-                dcb_waves(p, sl, &us);
-                us += (sl - 1) * (2.2 + 0.006 * wgs);
-                if (sl == usual || us < best) { best = us; wanted = sl; }
-            }
-        } else if (wgs < 256 || (wgs <= 384 && hpg >= DCB_SLICE_HEADS)) wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 4, 4, std::max<int64_t>(512 / wgs, 2)}));
+        // (heads of 64: waves that take whole heads split a tile's heads themselves.  us of dCB with the state passing beside it + the last launch with
+        // 1 / 2 / 4 slices: 64 tiles of 64 heads 62 / 43 / 37; 128 of 24 heads 35 / 30 / 34; 144 of 16 30 / 29 / 34; 256 of 24 37 / 36 / 41;
+        // 384 of 32 49 / 54 / 65)
+        const bool heads = p->headdim == 64;
+        if (wgs < 256 || (wgs <= (heads ? 256 : 384) && hpg >= DCB_SLICE_HEADS))
+            wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 4, 4, heads && wgs >= 128 ? 2 : std::max<int64_t>(512 / wgs, 2)}));
     } else {
         const int most = p->dtype == BIMAMBA2_F32 ? (hpg < 6 ? 256 : 768) : std::min(768, 32 * hpg);      // workgroups
         wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, most / wgs}));
