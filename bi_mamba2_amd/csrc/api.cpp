@@ -518,6 +518,7 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     q.final_f = q.final_b = nullptr;
     const size_t need = carve(&q, 1, p->workspace);
     if (need > 256 && (!p->workspace || p->workspace_bytes < need)) return BIMAMBA2_EWORKSPACE;
+    if ((p->dBs || p->dCs) && p->dbdc_heads > 8) return BIMAMBA2_EINVAL;      // (a caller's slices; this call's own may be longer)
     // (a forward pass over one chunk leaves no states: its caller says so)
     const bool one = one_chunk(&q) && (!p->fwd_saved || (p->fwd_saved & 4));
     if (p->fwd_saved) {

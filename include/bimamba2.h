@@ -164,7 +164,7 @@ typedef struct bimamba2_params {
     int64_t dx_sb, dx_sl, dB_sb, dB_sl, dC_sb, dC_sl;
     int64_t ddt_sb, ddt_sl;         /* likewise of ddt (batch, seqlen, nheads): 0 means contiguous */
     int32_t dbdc_heads;             /* heads per slice of dBs / dCs (1..8): S = ceil(H/G/dbdc_heads); 0 means 8.  bimamba2_bwd
-                                       chooses it itself where dBs and dCs are its own. */
+                                       chooses it itself where dBs and dCs are its own (and may take more than 8). */
     int32_t dcb_slices;             /* head slices of dCB / dCBT, one copy of each per slice; 0 means min(4, max(1, H/G/32)).
                                        A slice holds ceil(H/G/dcb_slices) heads; one that is left without any adds zeros.
                                        bimamba2_bwd chooses it itself where dCB and dCBT are its own. */

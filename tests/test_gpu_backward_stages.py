@@ -283,7 +283,7 @@ def test_state_parts_of_db_and_dc_with_narrow_states(ops, N, H, G, P, L, Q, dtyp
 @pytest.mark.parametrize("b,H,G,L,Q,hps,dtype,P", [
     (1, 5, 1, 129, 64, 5, torch.bfloat16, 64),        # four waves share a tile, one of them with two heads; one row in the last chunk
     (1, 3, 1, 449, 256, 2, torch.float16, 64),        # fewer heads than waves, the second slice with one; a ragged tile and one with no rows
-    (2, 26, 1, 300, 128, 13, torch.bfloat16, 64),     # slices of more than eight heads
+    (2, 26, 1, 300, 128, 8, torch.bfloat16, 64),      # four slices, the last with two heads
     (16, 4, 2, 1030, 128, 2, torch.bfloat16, 64),     # 576 tiles of two heads and role: two waves a tile
     (16, 16, 8, 1030, 64, 2, torch.float16, 64),      # 2176 tiles of two heads: one wave a tile
     (4, 18, 9, 1030, 256, 1, torch.bfloat16, 64),     # 900 tiles, two slices of one head each

@@ -201,6 +201,15 @@ def test_chunk_size_follows_the_number_of_sequence_boundaries():
     assert ops.chunk_size_for_seq_idx(four, 64) == 64                       # never above what the caller asked for
 
 
+def test_a_callers_slices_of_db_and_dc_hold_eight_heads():
+    """bimamba2_bwd's own slices may be longer; a caller's are refused, before any launch, also where the kernel would take them"""
+    lib = _lib.load()
+    for more in (dict(dBs=256, dCs=256), dict(dBs=256), dict(dCs=256)):
+        p = _params(batch=2, seqlen=512, nheads=26, headdim=64, ngroups=1, dstate=64, chunk_size=256, dbdc_heads=13, workspace=256, workspace_bytes=1 << 40, **more,
+                    **dict.fromkeys("x dt A Bm Cm dout dx ddt dA dB dC".split(), 256))
+        assert lib.bimamba2_bwd(ctypes.byref(p)) == -1
+
+
 def _dcb_slices(**kw):
     """head slices of dCB that bimamba2_bwd works with: what its workspace holds beside a caller's dCB and dCBT"""
     lib = _lib.load()
