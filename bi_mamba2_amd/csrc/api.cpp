@@ -519,6 +519,12 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     const size_t need = carve(&q, 1, p->workspace);
     if (need > 256 && (!p->workspace || p->workspace_bytes < need)) return BIMAMBA2_EWORKSPACE;
     if ((p->dBs || p->dCs) && p->dbdc_heads > 8) return BIMAMBA2_EINVAL;      // (a caller's slices; this call's own may be longer)
+    // what a caller has to bring, before any launch: which stages run, and with them whose checks, depends on the problem
+    REQUIRE(q.x); REQUIRE(q.dt); REQUIRE(q.A); REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dout);
+    REQUIRE(q.dx); REQUIRE(q.ddt); REQUIRE(q.dA); REQUIRE(q.dB); REQUIRE(q.dC);
+    if (q.has_dt_bias) REQUIRE(q.dt_bias);
+    if (q.has_D) { REQUIRE(q.D); REQUIRE(q.dD); }
+    if (q.has_z) { REQUIRE(q.z); REQUIRE(q.out_x); REQUIRE(q.dz); }
     // (a forward pass over one chunk leaves no states: its caller says so)
     const bool one = one_chunk(&q) && (!p->fwd_saved || (p->fwd_saved & 4));
     if (p->fwd_saved) {

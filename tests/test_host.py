@@ -210,6 +210,22 @@ def test_a_callers_slices_of_db_and_dc_hold_eight_heads():
         assert lib.bimamba2_bwd(ctypes.byref(p)) == -1
 
 
+@pytest.mark.parametrize("seqlen,chunk,saved", [(100, 128, 0), (100, 256, 0), (100, 256, 5), (100, 72, 0), (64, 64, 5), (600, 256, 0), (600, 256, 1), (600, 128, 1)])
+@pytest.mark.parametrize("dtype,headdim,dstate", [(_lib.BF16, 64, 64), (_lib.F16, 128, 128), (_lib.BF16, 16, 16), (_lib.F32, 64, 64)])
+def test_a_backward_pass_asks_for_every_operand_before_any_launch(dtype, headdim, dstate, seqlen, chunk, saved):
+    """rows as the fast kernels take them, over one chunk and over several, with the forward pass's intermediates and without"""
+    p = dict(_contiguous(2, seqlen, 4, headdim, 1, dstate, chunk, dtype), has_z=1, has_D=1, has_dt_bias=1, fwd_saved=saved, workspace=256, workspace_bytes=1 << 40)
+    p.update({"z" + k[1:]: v for k, v in p.items() if k.startswith("x_")}, **{"dout" + k[1:]: v for k, v in p.items() if k.startswith("x_")})
+    if saved:
+        p.update(dt_out=256, cs_f=256, cs_b=256)
+    if saved & 4 == 0 and saved:
+        p.update(states_f=256, states_b=256)
+    named = "x dt A Bm Cm dout dx ddt dA dB dC dt_bias D dD z out_x dz".split()
+    for missing in named:
+        got = _lib.load().bimamba2_bwd(ctypes.byref(_params(**p, **dict.fromkeys(set(named) - {missing}, 256))))
+        assert got == -1, (missing, got)
+
+
 def _dcb_slices(**kw):
     """head slices of dCB that bimamba2_bwd works with: what its workspace holds beside a caller's dCB and dCBT"""
     lib = _lib.load()
