@@ -77,10 +77,28 @@ struct Carver {
     }
 };
 
+inline bool al16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
+
+// What the tensors of states that a caller brings, or leaves out, decide about a pass
+struct StateForm {
+    bool one;           // one_chunk()
+    bool by_heads;      // dbdc_both_by_heads() will hold (what is carved is aligned)
+    bool together;      // db_dc_roles()
+};
+StateForm state_form(const bimamba2_params *q, int is_bwd) {
+    StateForm f{one_chunk(q), false, false};
+    if (!is_bwd) return f;
+    const bool copies = bimamba2_state_copies(q) != 0, brought = q->states16_f && q->states16_b && al16(q->states16_f) && al16(q->states16_b);
+    f.by_heads = copies && !q->dstates_f && dbdc_by_heads(q) && (q->states16_f ? brought : !q->states_f) &&
+                 (!q->dstates16_f || (q->dstates16_b && al16(q->dstates16_f) && al16(q->dstates16_b)));
+    f.together = db_dc_roles(q, copies || q->states16_f || q->dstates16_f);
+    return f;
+}
+
 // Assigns every intermediate that is NULL in `q` from the workspace; returns the bytes used.
-size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
+size_t carve(bimamba2_params *q, int is_bwd, void *ws, const StateForm &form) {
     Carver cv(ws);
-    const bool one = one_chunk(q);
+    const bool one = form.one;
     const size_t nc = nchunks(q), Q = q->chunk_size;
     const size_t bhcq = (size_t)q->batch * q->nheads * nc * Q;
     const size_t cbn = (size_t)q->batch * nc * q->ngroups * Q * Q;
@@ -97,7 +115,6 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     // a forward pass whose caller keeps no states (no pointer given for them) has one reader of the entering states, the scan
     // kernel, and every 16-bit scan kernel reads the copies: the state passing then writes half the bytes, the scan reads half
     // (under the conditions of the state-passing kernel that writes them)
-    auto al16 = [](const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
     const bool fwd_only_copies = !is_bwd && !q->causal && (q->dtype == BIMAMBA2_BF16 || q->dtype == BIMAMBA2_F16) &&
                                  (q->headdim * q->dstate) % 4 == 0 && al16(q->final_f) && al16(q->final_b) &&
                                  al16(q->initial_f) && al16(q->initial_b) && !q->states_b && !q->states16_b;
@@ -107,10 +124,6 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     const bool fwd_scan16 = !is_bwd && chunk_scan_uses_scan16(q, false) &&
                             (one ? one_chunk_free16(q, false) : (carve16 || q->states16_f) && (q->causal || carve16 || q->states16_b));
     if (is_bwd ? !(scan_recomputes_cb(q, true) && dcb_recomputes_cb(q)) : !(scan_recomputes_cb(q, false) || fwd_scan16)) need_f(q->CB, cbn);
-    // whether dbdc_both_by_heads() will hold (what is carved is aligned)
-    const bool by_heads = is_bwd && copies && !one && !q->dstates_f && dbdc_by_heads(q) &&
-                          (carve16 || (q->states16_f && q->states16_b && al16(q->states16_f) && al16(q->states16_b))) &&
-                          (!q->dstates16_f || (q->dstates16_b && al16(q->dstates16_f) && al16(q->dstates16_b)));
     if (carve16) {
         q->states16_f = cv.take<char>(stn * 2);
         q->states16_b = cv.take<char>(stn * 2);
@@ -129,7 +142,7 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     }
     if (is_bwd) {
         const size_t nqt = (Q + 63) / 64;
-        if (!q->dBs && !q->dCs) q->dbdc_heads = choose_dbdc_heads(q, by_heads, db_dc_roles(q, q->states16_f || q->dstates16_f));
+        if (!q->dBs && !q->dCs) q->dbdc_heads = choose_dbdc_heads(q, !one && form.by_heads, form.together);
         if (!q->dCB && !q->dCBT) q->dcb_slices = choose_dcb_slices(q);      // (which asks about the last launch, and that about the slices of dB and dC)
         need_f(q->dCB, cbn * dcb_slices(q));
         need_f(q->dCBT, cbn * dcb_slices(q));
@@ -167,6 +180,7 @@ size_t carve(bimamba2_params *q, int is_bwd, void *ws) {
     }
     return (cv.off + 255) & ~size_t(255);
 }
+size_t carve(bimamba2_params *q, int is_bwd, void *ws) { return carve(q, is_bwd, ws, state_form(q, is_bwd)); }
 
 // Device memory that lives as long as the process: the workspace of bimamba2_fwd_static.  Every GPU the library runs on
 // holds its own copy at its own address; in host code the array's name is not a device address, so the address is asked
@@ -211,8 +225,22 @@ size_t bimamba2_params_size(void) { return sizeof(bimamba2_params); }
 
 size_t bimamba2_workspace_bytes(const bimamba2_params *p, int is_bwd) {
     if (check_problem(p)) return 0;
-    bimamba2_params q = *p;
-    return carve(&q, is_bwd, nullptr);
+    bimamba2_params asked = *p;
+    if (is_bwd) asked.final_f = asked.final_b = nullptr;      // (as the pass does)
+    // the most that any form takes which tensors of states set after the question can lead to
+    const StateForm now = state_form(&asked, is_bwd);
+    size_t most = 0;
+    for (int k = 0; k < 8; ++k) {
+        if (((k & 1) && !now.one) || ((k & 2) && !now.by_heads) || ((k & 4) && !now.together)) continue;
+        bimamba2_params q = asked;
+        most = std::max(most, carve(&q, is_bwd, nullptr, StateForm{now.one && !(k & 1), now.by_heads && !(k & 2), now.together && !(k & 4)}));
+    }
+    if (!is_bwd && !asked.states_f && !asked.states16_f) {
+        // float32 states of the caller's: no copies, and a scan kernel that reads CB where the one for copies would not (dstate 128, few heads)
+        asked.states_f = asked.states_b = reinterpret_cast<float *>(256);
+        most = std::max(most, carve(&asked, is_bwd, nullptr));
+    }
+    return most;
 }
 
 int bimamba2_state_copies(const bimamba2_params *p) {

@@ -177,7 +177,9 @@ int bimamba2_version(void);
 /* sizeof(bimamba2_params) as compiled into the library, for bindings to check their mirror of the struct */
 size_t bimamba2_params_size(void);
 
-/* bytes of workspace the composite entry points need (is_bwd = 0: forward, 1: backward) */
+/* bytes of workspace the composite entry points need (is_bwd = 0: forward, 1: backward).  Reads `p` as it will be passed, fwd_saved and the operands'
+ * strides and alignment included; the tensors of states (initial_*, final_*, their gradients, states*, dstates*) may be set after the question, to
+ * 16-byte aligned addresses: the answer is enough with them and without. */
 size_t bimamba2_workspace_bytes(const bimamba2_params *p, int is_bwd);
 
 /* Packed sequences: counts[b * nchunks + c] = the larger of the numbers of sequence boundaries that the forward and the reverse

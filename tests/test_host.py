@@ -226,6 +226,22 @@ def test_a_backward_pass_asks_for_every_operand_before_any_launch(dtype, headdim
         assert got == -1, (missing, got)
 
 
+@pytest.mark.parametrize("dtype,headdim,dstate", [(_lib.BF16, 64, 64), (_lib.F16, 128, 64), (_lib.BF16, 64, 128), (_lib.BF16, 16, 16), (_lib.F32, 64, 64)])
+@pytest.mark.parametrize("batch,seqlen,chunk", [(2, 100, 128), (2, 100, 256), (2, 100, 72), (4, 2048, 256), (1, 1000, 128)])
+@pytest.mark.parametrize("is_bwd", [0, 1])
+def test_a_workspace_asked_for_before_the_states_are_named_is_enough(is_bwd, batch, seqlen, chunk, dtype, headdim, dstate):
+    """no operand is named either, so that a workspace that is taken leads to the refusal of these, before any launch"""
+    lib = _lib.load()
+    pairs = ["initial", "final", "states", "states16"] + (["dstates", "dstates16", "dinitial", "dfinal"] if is_bwd else [])
+    for heads, groups in ((4, 1), (32, 1), (24, 8)):
+        p = dict(_contiguous(batch, seqlen, heads, headdim, groups, dstate, chunk, dtype), workspace=256)
+        asked = lib.bimamba2_workspace_bytes(ctypes.byref(_params(**p)), is_bwd)
+        for subset in range(1 << len(pairs)):
+            named = {f"{n}_{way}": 256 for i, n in enumerate(pairs) if subset >> i & 1 for way in "fb"}
+            got = (lib.bimamba2_bwd if is_bwd else lib.bimamba2_fwd)(ctypes.byref(_params(**p, **named, workspace_bytes=asked)))
+            assert got == -1, (heads, groups, sorted(named))
+
+
 def _dcb_slices(**kw):
     """head slices of dCB that bimamba2_bwd works with: what its workspace holds beside a caller's dCB and dCBT"""
     lib = _lib.load()
