@@ -567,6 +567,17 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
         TRY(forward_cumsum_and_states(&q));
         TRY(bimamba2_state_passing_fwd(&q));
     }
+    if (one) {
+        // state parts that the caller has places for (the pass itself neither forms nor reads them): nothing crosses a chunk boundary
+        const size_t rows = (size_t)q.batch * q.nheads * q.chunk_size, heads = q.nheads / q.ngroups, hps = p->dbdc_heads > 0 ? p->dbdc_heads : 8;
+        const size_t sums = (heads + hps - 1) / hps * q.batch * q.seqlen * q.ngroups * q.dstate;
+        for (float *t : {p->u_f, p->u_b, p->v_f, p->v_b})
+            if (t) TRY(launch_fill(t, rows, 0.f, stream_of(&q)));
+        for (float *t : {p->ddA_chunk_f, p->ddA_chunk_b})
+            if (t) TRY(launch_fill(t, (size_t)q.batch * q.nheads * sp_nsplit(&q), 0.f, stream_of(&q)));
+        for (float *t : {p->dBs, p->dCs})
+            if (t) TRY(launch_fill(t, sums, 0.f, stream_of(&q)));
+    }
     // dCB / dCBT in the 16-bit element type where this call owns them and the two launches that write and read them are the
     // merged ones (their reader rounds them to that type for its MFMA anyway)
     // (without states to pass the launch is dCB's alone, with its place for 16-bit results)

@@ -74,3 +74,28 @@ def test_the_same_call_with_and_without_states_in_turn():
     kw = dict(D=inp["D"], dt_bias=inp["dt_bias"], dt_softplus=True, return_intermediates=False)
     outs = [ops._mamba_chunk_scan_combined_fwd(*args, **kw, want_final=f)[0] for f in (False, True, False)]
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("H,P,G,N,Q,heads_per_slice", [(4, 64, 1, 64, 256, 0), (6, 32, 2, 16, 128, 2), (26, 64, 1, 128, 64, 8)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_state_parts_that_the_caller_has_places_for_are_zero(monkeypatch, dtype, H, P, G, N, Q, heads_per_slice):
+    """through bimamba2_bwd with buffers of the caller's; the gradients are those without them"""
+    b, L = 2, 57
+    inp = to_dev(make_case(b, L, H, P, G, N, dtype))
+    dout = torch.randn(inp["x"].shape, generator=torch.Generator().manual_seed(2)).to(dtype).cuda()
+    rows, sums = (b, H, 1, Q), (-(-(H // G) // (heads_per_slice or 8)), b, L, G, N)
+    shapes = {**dict.fromkeys(("u_f", "u_b", "v_f", "v_b"), rows), **dict.fromkeys(("ddA_chunk_f", "ddA_chunk_b"), (b, H, 1, -(-P * N // 1024))), "dBs": sums, "dCs": sums}
+    own, kept = ops._Call.workspace, {}
+
+    def workspace(c, is_bwd):
+        c.p.dbdc_heads = heads_per_slice
+        for name, shape in shapes.items():
+            kept[name] = c.new(name, shape).fill_(float("nan"))
+        return own(c, is_bwd)
+
+    grads = lambda: ops._mamba_chunk_scan_combined_bwd(dout, inp["x"], inp["dt"], inp["A"], inp["B"], inp["C"], None, Q, dt_bias=inp["dt_bias"], dt_softplus=True)
+    want = grads()
+    monkeypatch.setattr(ops._Call, "workspace", workspace)
+    got = grads()
+    assert len(kept) == 8 and all(bool((t == 0).all()) for t in kept.values())
+    assert all(a is b or torch.equal(a, b) for a, b in zip(got, want))
