@@ -1234,13 +1234,15 @@ __global__ __launch_bounds__(NTHREADS) void state_passing_fwd_inplace16_kernel(c
                 for (int k = 0; k < 8; ++k) s[k] = dec * s[k] + to_f(v[i].v[k]);
             }
     };
-    for (int s0 = 0; s0 < nc; s0 += 8) {
-        const int left = nc - s0;
-        if (left <= 1) batch(s0, std::integral_constant<int, 1>());
-        else if (left <= 2) batch(s0, std::integral_constant<int, 2>());
-        else if (left <= 4) batch(s0, std::integral_constant<int, 4>());
-        else batch(s0, std::integral_constant<int, 8>());
-    }
+    // (the remainder's size is asked for behind the whole batches: inside the loop 64 chunks, 12 heads, dstate 64 took 14.3 us instead of 13.0;
+    // 9 chunks, 16 rows of 12 heads 10.9 with the remainder as a batch of 8, 9.5 by its size)
+    int s0 = 0;
+    for (; nc - s0 >= 8; s0 += 8) batch(s0, std::integral_constant<int, 8>());
+    const int left = nc - s0;
+    if (left > 4) batch(s0, std::integral_constant<int, 8>());
+    else if (left > 2) batch(s0, std::integral_constant<int, 4>());
+    else if (left == 2) batch(s0, std::integral_constant<int, 2>());
+    else if (left == 1) batch(s0, std::integral_constant<int, 1>());
     if (fin) {
         *reinterpret_cast<f32x4 *>(fin + ((int64_t)b * p.nheads + h) * PN + e) = f32x4{s[0], s[1], s[2], s[3]};
         *reinterpret_cast<f32x4 *>(fin + ((int64_t)b * p.nheads + h) * PN + e + 4) = f32x4{s[4], s[5], s[6], s[7]};
