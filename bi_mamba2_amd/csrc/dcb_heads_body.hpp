@@ -83,15 +83,15 @@ __device__ __forceinline__ void bwd_dcb_heads_body(const bimamba2_params &p, int
     const int hw = wave % W, ti = wave / W;
     // the tiles on the diagonal cost more: they come first in launch order, which spreads them over the compute units
     const int tid = bid.y * L::TILES + ti;
-    int tt, st;
+    const bool mine = tid < nqt * nqt;             // (else a place behind the last tile: with one tile a plane the division would be by zero)
+    int tt = 0, st = 0;
     if (tid < nqt) tt = st = tid;
-    else {
+    else if (mine) {
         const int k = tid - nqt;
         tt = k / (nqt - 1);
         st = k % (nqt - 1);
         st += st >= tt;
     }
-    const bool mine = tid < nqt * nqt;
     const int tile = tt * nqt + st;
     const int g = bid.x % p.ngroups, bc = bid.x / p.ngroups, c = bc % nc, b = bc / nc;
     const int Q = p.chunk_size, P = p.headdim, H = p.nheads, hpg = H / p.ngroups;
