@@ -24,6 +24,12 @@ __device__ __forceinline__ float to_f(float v) { return v; }
 __device__ __forceinline__ float to_f(bf16_t v) { return static_cast<float>(v); }
 __device__ __forceinline__ float to_f(f16_t v) { return static_cast<float>(v); }
 template <typename T> __device__ __forceinline__ T from_f(float v) { return static_cast<T>(v); }
+// The same from the float32 value.  float16 has an instruction for multiply, add and convert with one rounding, which the compiler takes for some
+// results of a kernel and not for others: where two kernels, or two variants of one, have to give the same bits, both convert by this.
+template <typename T> __device__ __forceinline__ T from_f32(float v) {
+    if constexpr (std::is_same<T, f16_t>::value) asm("" : "+v"(v));
+    return from_f<T>(v);
+}
 
 // ---- direct global -> LDS loads (global_load_lds): lane l's 16 bytes land at the wave-uniform LDS address + 16*l ----
 typedef __attribute__((address_space(3))) void *lds_ptr_t;

@@ -426,8 +426,9 @@ __device__ __forceinline__ void state_passing_bwd_groups(const bimamba2_params &
                     dot[k] = (gu[0] * pv[0] + gu[1] * pv[1] + gu[2] * pv[2] + gu[3] * pv[3]) * d;
                     if constexpr (DS16) {
                         V4 t;
+                        // (by the float32 value: a row's gradients do not depend on how many rows there are, i.e. on NG)
 #pragma unroll
-                        for (int i = 0; i < 4; ++i) t.v[i] = from_f<T16>(gu[i]);
+                        for (int i = 0; i < 4; ++i) t.v[i] = from_f32<T16>(gu[i]);
                         *reinterpret_cast<V4 *>(ds16 + e[u] + c * cstride) = t;
                     } else {
                         *reinterpret_cast<f32x4 *>(ds + e[u] + c * cstride) = gu;

@@ -369,15 +369,16 @@ def test_state_passing_over_few_chunks(ops, nc, PN):
 
 
 @pytest.mark.parametrize("L", [100, 333, 1000])
-def test_state_passing_beside_dcb_does_not_depend_on_the_batch(L):
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_state_passing_beside_dcb_does_not_depend_on_the_batch(L, dtype):
     """many rows: several groups of 1024 elements a workgroup in the launch of dCB; one row: one group where the sequence is long.  The
     gradients of the states, and what is made of them alone, are the same bits"""
     from bi_mamba2_amd.ops import bimamba_chunk_scan_combined
     b, H, P, N = 32, 4, 64, 64
     gen = torch.Generator().manual_seed(L)
-    inp = to_dev(make_case(b, L, H, P, 1, N, torch.bfloat16))
+    inp = to_dev(make_case(b, L, H, P, 1, N, dtype))
     init = [torch.randn(b, H, P, N, generator=gen).cuda() for _ in range(2)]
-    dout = torch.randn(b, L, H, P, generator=gen).bfloat16().cuda()
+    dout = torch.randn(b, L, H, P, generator=gen).to(dtype).cuda()
     dfin = [torch.randn(b, H, P, N, generator=gen).cuda() for _ in range(2)]
 
     def grads(rows):
