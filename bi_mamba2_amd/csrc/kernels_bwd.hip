@@ -144,6 +144,7 @@ int launch_layer_sums(const LayerSums &sums, const bimamba2_cast_params *casts, 
 
 // =========================================================================================================
 // dz = dout * out_x * sigmoid(z) (1 + z (1 - sigmoid(z)));  dout_x = dout * z * sigmoid(z)
+// (by their float32 values: the same bits as from the kernel that also forms the states' gradients)
 // =========================================================================================================
 template <typename T>
 __device__ __forceinline__ void bwd_dz_body(const bimamba2_params &p, int id, int nblocks) {
@@ -200,8 +201,8 @@ __device__ __forceinline__ void bwd_dz_body(const bimamba2_params &p, int id, in
 #pragma unroll
         for (int i = 0; i < VS; ++i) {
             const float sg = sigmoid_f(zv[i]);
-            r1.v[i] = from_f<T>(dv[i] * ov[i] * sg * (1.f + zv[i] * (1.f - sg)));
-            r2.v[i] = from_f<T>(dv[i] * zv[i] * sg);
+            r1.v[i] = from_f32<T>(dv[i] * ov[i] * sg * (1.f + zv[i] * (1.f - sg)));
+            r2.v[i] = from_f32<T>(dv[i] * zv[i] * sg);
         }
         if (vec) {
             // dz is not read again inside the pass, dout_x by four kernels: the first goes past the caches

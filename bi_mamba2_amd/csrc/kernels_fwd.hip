@@ -523,8 +523,8 @@ __global__ __launch_bounds__(NTHREADS) __attribute__((amdgpu_waves_per_eu(4, 4))
             for (int i = 0; i < 8; ++i) {
                 const float zv = to_f(a.v[i]), dv = to_f(d.v[i]), ov = to_f(e.v[i]);
                 const float sg = sigmoid_f(zv);
-                r1.v[i] = from_f<T>(dv * ov * sg * (1.f + zv * (1.f - sg)));
-                r2.v[i] = from_f<T>(dv * zv * sg);
+                r1.v[i] = from_f32<T>(dv * ov * sg * (1.f + zv * (1.f - sg)));
+                r2.v[i] = from_f32<T>(dv * zv * sg);
             }
             raw_lds_write128_at<XO>(xw, __builtin_bit_cast(f32x4, r2));
             const int row = 32 * s + row0;

@@ -17,19 +17,10 @@ SHAPES = [(4, 64, 1, 64, 256), (8, 64, 2, 128, 256), (3, 128, 1, 64, 128), (6, 3
           (36, 64, 1, 64, 256)]
 
 
-def same(a, b, gated_half):
-    """In bits.  float16 gradients with a z gate: dz and dout * silu(z) come from another kernel where no states' gradients are formed with
-    them, and a float16 product of float32 values may be rounded once or twice (multiply and convert in one instruction or two).  Elements are
-    then off by one unit, 2^-11 of the value at most; fewer than one in a hundred of them make 5e-5 of a tensor's norm."""
-    if gated_half:
-        return float((a.double() - b.double()).norm()) <= 5e-5 * float(b.double().norm())
-    return torch.equal(a, b)
-
-
-def passes(inp, Q, dout, final, training):
+def passes(inp, Q, dout, final, training, seq_idx=None):
     leaves = {k: v.clone().requires_grad_(training) for k, v in inp.items()}
     out = bimamba_chunk_scan_combined(leaves["x"], leaves["dt"], leaves["A"], leaves["B"], leaves["C"], Q, D=leaves["D"], z=leaves.get("z"),
-                                      dt_bias=leaves["dt_bias"], dt_softplus=True, return_final_states=final)
+                                      dt_bias=leaves["dt_bias"], dt_softplus=True, return_final_states=final, seq_idx=seq_idx)
     out = out[0] if final else out
     return [out] + (list(torch.autograd.grad(out, list(leaves.values()), dout)) if training else [])
 
@@ -46,7 +37,22 @@ def test_same_bits_as_with_states(dtype, shape, L):
         dout = torch.randn(inp["x"].shape, generator=torch.Generator().manual_seed(L)).to(dtype).cuda()
         for training in (False, True):
             for a, b in zip(passes(inp, Q, dout, False, training), passes(inp, Q, dout, True, training)):
-                assert same(a, b, training and with_z and dtype == torch.float16)
+                assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("bounds", [((), ()), ((1,), (56,)), ((5, 6, 7), (22,)), ((4, 32), (3, 31, 55))])      # inside a lane's four positions, between them, at both ends
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_same_bits_as_with_states_where_sequences_are_packed(dtype, shape, bounds):
+    H, P, G, N, Q = shape
+    L = 57
+    seq_idx = torch.stack([sum((torch.arange(L) >= at).int() for at in (0,) + row) for row in bounds]).int().cuda()
+    assert ops.chunk_size_for_seq_idx(seq_idx, Q) >= L
+    inp = {k: v for k, v in to_dev(make_case(2, L, H, P, G, N, dtype, with_z=True)).items() if v is not None}
+    dout = torch.randn(inp["x"].shape, generator=torch.Generator().manual_seed(L)).to(dtype).cuda()
+    for training in (False, True):
+        for a, b in zip(passes(inp, Q, dout, False, training, seq_idx), passes(inp, Q, dout, True, training, seq_idx)):
+            assert torch.equal(a, b)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -64,7 +70,7 @@ def test_rows_at_odd_addresses(dtype):
         return [out] + list(torch.autograd.grad(out, list(leaves.values()), dout))
 
     for a, b in zip(grads(False), grads(True)):
-        assert same(a, b, dtype == torch.float16)
+        assert torch.equal(a, b)
 
 
 def test_the_same_call_with_and_without_states_in_turn():
