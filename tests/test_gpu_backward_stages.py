@@ -252,6 +252,25 @@ def test_dcb_by_waves_that_share_a_tile(ops, b, H, G, P, L, Q, dtype):
         assert float((g - w).norm() / w.norm()) < 4e-6
 
 
+@pytest.mark.parametrize("b,H,G,L,Q", [(1, 5, 1, 449, 256), (16, 6, 2, 1030, 128), (16, 16, 8, 1030, 64)])      # four waves, two, one to a tile
+@pytest.mark.parametrize("N", [32, 64, 96, 160])
+def test_dcb_that_rebuilds_cb(ops, N, b, H, G, L, Q):
+    """C.B^T from the rows of C and B, 64 columns at a time, the last 32 of a dstate that is no multiple of 64 by themselves: against the tiles as
+    they are computed in float64 from the same values.  The kernel's own are sums of N exact products in float32 (relative to their
+    norm within 2^-24 sqrt(N), 1e-6), which adds to the bound of the test above only in the vectors they enter."""
+    dtype = torch.bfloat16 if N % 64 else torch.float16
+    d = to_dev(make_case(b, L, H, 64, G, N, dtype))
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(5)).to(dtype).cuda()
+    csf, csb, dt = ops._chunk_cumsum_fwd(d["dt"], d["A"], Q, dt_bias=d["dt_bias"], dt_softplus=True)
+    nc = -(-L // Q)
+    rows = lambda t: F.pad(t.double(), (0, 0, 0, 0, 0, nc * Q - L)).view(b, nc, Q, G, N).transpose(2, 3)
+    CB = torch.matmul(rows(d["C"]), rows(d["B"]).transpose(-1, -2).contiguous()).float()
+    want = ops._chunk_scan_bwd_dcb(d["x"].float(), dt, csf, csb, dout.float(), CB, ngroups=G)
+    got = ops._chunk_scan_bwd_dcb(d["x"], dt, csf, csb, dout, None, ngroups=G, B=d["B"], C=d["C"])
+    for g, w in zip(got, want):
+        assert float((g - w).norm() / w.norm()) < 5e-6
+
+
 @pytest.mark.parametrize("N", [8, 16, 20, 32, 36, 64])
 @pytest.mark.parametrize("H,G,P,L,Q,dtype", [(6, 2, 16, 130, 128, torch.bfloat16), (8, 1, 72, 75, 64, torch.float32), (3, 3, 32, 257, 256, torch.float16)])
 def test_state_parts_of_db_and_dc_with_narrow_states(ops, N, H, G, P, L, Q, dtype):
@@ -390,3 +409,30 @@ def test_state_passing_beside_dcb_does_not_depend_on_the_batch(L, dtype):
 
     for many, one in zip(grads(b), grads(1)):
         assert torch.equal(many[:1], one)
+
+
+@pytest.mark.parametrize("H,L,dtype", [(24, 1500, torch.bfloat16), (24, 2700, torch.float16), (20, 4343, torch.bfloat16)])      # 6, 11 and 17 chunks
+def test_state_passing_of_float32_states_beside_dcb_does_not_depend_on_the_batch(ops, monkeypatch, H, L, dtype):
+    """the same at dstate 128, whose states and their gradients are float32: two rows have 512 workgroups or more of one group, so that a workgroup takes
+    two; one row has fewer and keeps one.  The inner products that it leaves for d(dt A) are compared as well"""
+    b, P, N, Q, nsplit = 2, 64, 128, 256, 8
+    gen = torch.Generator().manual_seed(L)
+    inp = to_dev(make_case(b, L, H, P, 1, N, dtype))
+    states = lambda: [torch.randn(b, H, P, N, generator=gen).cuda() for _ in range(2)]
+    init, dfin, dout = states(), states(), torch.randn(b, L, H, P, generator=gen).to(dtype).cuda()
+    own, kept = ops._Call.workspace, {}
+
+    def workspace(c, is_bwd):
+        for name in ("ddA_chunk_f", "ddA_chunk_b"):
+            kept[name] = c.new(name, (c.p.batch, H, -(-L // Q), nsplit)).fill_(float("nan"))
+        return own(c, is_bwd)
+
+    monkeypatch.setattr(ops._Call, "workspace", workspace)
+
+    def results(rows):
+        res = ops._mamba_chunk_scan_combined_bwd(dout[:rows], inp["x"][:rows], inp["dt"][:rows], inp["A"], inp["B"][:rows], inp["C"][:rows], None, Q,
+                                                 dt_bias=inp["dt_bias"], dt_softplus=True, initial_states=[t[:rows] for t in init], dfinal_states=[t[:rows] for t in dfin])
+        return [res[0], *res[8], *kept.values()]
+
+    for many, one in zip(results(b), results(1)):
+        assert torch.isfinite(many).all() and torch.equal(many[:1], one)

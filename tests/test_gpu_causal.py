@@ -44,6 +44,29 @@ def test_causal_forward_and_backward(ops, case):
             assert_close(leaves[k].grad, ref["d" + k], dtype, "d" + k, scaled=is_reduced("d" + k, dtype))
 
 
+@pytest.mark.parametrize("H,G,Q,dtype", [(6, 2, 128, torch.bfloat16), (16, 8, 64, torch.float16)])      # two waves a 64 x 64 tile, one
+def test_causal_gradients_do_not_depend_on_the_batch(ops, H, G, Q, dtype):
+    """16 rows have tiles enough for two waves or one to a tile in the dCB kernel; a row by itself, as in the cases above, has four.  What a wave leaves
+    by heads is the same in bits; the heads of a group are added up in another order, so dB and dC may be off by a unit of their type
+    now and then"""
+    b, L = 16, 1030
+    d = to_dev(make_case(b, L, H, 64, G, 64, dtype, with_z=True))
+    dout = torch.randn(d["x"].shape, generator=torch.Generator().manual_seed(5)).to(dtype).cuda()
+
+    def grads(rows):
+        leaves = [d[k][rows].clone().requires_grad_(True) for k in ("x", "dt", "z", "B", "C")]
+        x, dt, z, B, C = leaves
+        out = ops.causal_chunk_scan_combined(x, dt, d["A"], B, C, Q, D=d["D"], z=z, dt_bias=d["dt_bias"], dt_softplus=True)
+        return torch.autograd.grad(out, leaves, dout[rows])
+
+    many = grads(slice(0, b))
+    for row in (0, b - 1):
+        one = grads(slice(row, row + 1))
+        assert all(torch.equal(m[row:row + 1], o) for m, o in zip(many[:3], one))
+        for m, o in zip(many[3:], one[3:]):
+            assert float((m[row].double() - o[0].double()).norm()) <= (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12) * float(o.double().norm())
+
+
 def test_causal_refuses_shapes_without_kernels(ops):
     inp = to_dev(make_case(1, 128, 2, 32, 1, 16, torch.float32))
     with pytest.raises(ValueError):
