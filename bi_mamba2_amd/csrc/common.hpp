@@ -31,6 +31,17 @@ template <typename T> __device__ __forceinline__ T from_f32(float v) {
     return from_f<T>(v);
 }
 
+// f(integral_constant<int, I>) for I = 0 .. N - 1 (until it returns false, where it returns anything): a loop whose index is a constant expression
+// inside the body (LDS offsets become immediates)
+template <int I, int N, class F> __device__ __forceinline__ void static_for(F &&f) {
+    if constexpr (I < N) {
+        typedef std::integral_constant<int, I> Index;
+        if constexpr (std::is_void<decltype(f(Index()))>::value) f(Index());
+        else if (!f(Index())) return;
+        static_for<I + 1, N>(f);
+    }
+}
+
 // ---- direct global -> LDS loads (global_load_lds): lane l's 16 bytes land at the wave-uniform LDS address + 16*l ----
 typedef __attribute__((address_space(3))) void *lds_ptr_t;
 typedef const __attribute__((address_space(1))) void *gbl_ptr_t;

@@ -157,18 +157,18 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
             raw_lds_write_at<0>(a, in ? (IS_DB ? d * __expf(ef - f) : __expf(f)) : 0.f);
             raw_lds_write_at<256>(a, in ? (IS_DB ? d * __expf(eb - r) : __expf(r)) : 0.f);
         }
-        dcb_static_for<0, 2>([&](auto DIR) __attribute__((always_inline)) {
+        static_for<0, 2>([&](auto DIR) __attribute__((always_inline)) {
             constexpr int dir = decltype(DIR)::value;
             if (dir == 1) wait_vmcnt<1>();        // the second direction's tile (younger is the store of the first one's sums)
             const unsigned ta = ring_a + L::TILE, va = vec_a + dir * 256;
             const int kk = 8 * lg + (lr >> 2), nn = 4 * (lr & 3);
             float u[4];
             // 32 rows at a time (with 64 the product's registers are too many)
-            dcb_static_for<0, 2>([&](auto HALF) __attribute__((always_inline)) {
+            static_for<0, 2>([&](auto HALF) __attribute__((always_inline)) {
                 constexpr int q0 = 2 * decltype(HALF)::value;
                 f32x4 acc[2][4];
                 __builtin_amdgcn_sched_barrier(0);
-                dcb_static_for<0, 2>([&](auto KS) __attribute__((always_inline)) {
+                static_for<0, 2>([&](auto KS) __attribute__((always_inline)) {
                     constexpr int ks = decltype(KS)::value;
                     const unsigned fa = ring_a + lr * 128 + (((ks * 4 + lg) ^ (ln & 7)) << 4);        // row 16 q + lr, unit 4 ks + lg
                     Frag x0 = raw_lds_read_at<Frag, q0 * 2048>(fa), x1 = raw_lds_read_at<Frag, q0 * 2048 + 2048>(fa);

@@ -42,13 +42,6 @@ __device__ __forceinline__ int lane_number() {
     asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(n));
     return n;
 }
-// f(integral_constant<int, I>) for I = 0 .. N - 1 (LDS offsets become immediates)
-template <int I, int N, class F> __device__ __forceinline__ void dcb_static_for(F &&f) {
-    if constexpr (I < N) {
-        f(std::integral_constant<int, I>());
-        dcb_static_for<I + 1, N>(f);
-    }
-}
 template <int CTRL> __device__ __forceinline__ float dpp_of(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
@@ -331,7 +324,7 @@ __device__ __forceinline__ void bwd_dcb_heads_body(const bimamba2_params &p, int
             const unsigned ra = vec_a + lg * 16, ca = vec_a + lr * 4;
             f32x4 colf = {}, colb = {};
             float uf[4], ub[4];
-            dcb_static_for<0, 4>([&](auto QQ) __attribute__((always_inline)) {
+            static_for<0, 4>([&](auto QQ) __attribute__((always_inline)) {
                 constexpr int q = decltype(QQ)::value;
                 float df[4] = {0.f, 0.f, 0.f, 0.f}, db[4] = {0.f, 0.f, 0.f, 0.f};
                 // the blocks of the other half of the columns (j0, j0 + 1), the one beside the diagonal in the same half (j2)

@@ -90,14 +90,6 @@ __device__ __forceinline__ int tile64_row_offset(int r, int n) {
 // Output rows m = 4 g + i of lane group g are then the columns 32 t + 8 g + i (tile 2t) and 32 t + 8 g + 4 + i (tile 2t + 1).
 __device__ __forceinline__ constexpr int s16_col(int j, int m) { return 32 * (j >> 1) + 8 * (m >> 2) + 4 * (j & 1) + (m & 3); }
 
-// f(integral_constant<int, I>) for I = 0 .. N - 1, until it returns false: a loop whose index is a constant expression inside
-// the body (LDS offsets become immediates)
-template <int I, int N, class F> __device__ __forceinline__ void static_for(F &&f) {
-    if constexpr (I < N) {
-        if (f(std::integral_constant<int, I>())) static_for<I + 1, N>(f);
-    }
-}
-
 }  // namespace
 
 // UNI: the single-direction (causal) operator: the reverse direction's state product, the K steps on the far side of the
