@@ -553,6 +553,7 @@ int launch_state_passing_bwd(const bimamba2_params *p) {
 static bool dcb_aligned(const bimamba2_params *p);
 static bool dcb_rows_in_32bit(const bimamba2_params *p);
 static double dbdc_heads_cost(const bimamba2_params *p, int w, int hps);
+static bool dx_db_dc_pays(const bimamba2_params *p);
 // 16-byte aligned rows of B and C
 static bool bmm_rows_aligned(const bimamba2_params *p) {
     auto al = [](const void *q) { return (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
@@ -589,17 +590,22 @@ int choose_dbdc_heads(const bimamba2_params *p, bool by_heads, bool together) {
     const int64_t tiles = (int64_t)p->batch * nc * p->ngroups * ((p->chunk_size + 127) / 128);
     const double steps = ((p->headdim + 63) / 64) * ((p->dstate + 63) / 64);                             // per head
     const double slice_cost = (double)p->batch * p->seqlen * p->ngroups * p->dstate * 8 / 5e6 / 1.5;     // one partial sum at 5 TB/s, in steps of 1.5 us
-    // where both roles share a launch (db_dc_roles()) they share the chip, and half the slices are less to add up.  us a pass with one
-    // launch, slices as for two launches and as here: float32, 2 x 1111, 16 heads of 64, dstate 64, 190 -> 181; 4 x 1024, 8 heads of 128
-    // 231 -> 225; bfloat16, 4 x 2048, 16 heads of 16, dstate 16 139 -> 135
+    // Where both roles share a launch (db_dc_roles()) they share the chip, and half the slices are less to add up.  us a pass with one
+    // launch, slices as for two launches and as here: float32, 2 x 1111, 16 heads of 64, dstate 64, 187 -> 177; 4 x 1024, 8 heads of 128
+    // 222 -> 213.  With dx in front of them in it no round of theirs starts at once: they take the places that dx leaves one after the other, so
+    // what counts is their work over all places, and the last workgroup, which ends alone.  us a pass, slices as for two launches / by half
+    // the places / as here: bfloat16, heads of 32, dstate 16, two groups, 16 x 520, 16 heads 162 / 167 / 164; 20 x 500, heads of 16, dstate 32
+    // 173 / 178 / 173; 4 x 2048, 16 heads of 16, dstate 16 137 / 132 / 133; float32, 1 x 6000, 16 heads of 32 179 / 182 / 180; 16 x 520
+    // 265 / 247 / 247; 8 x 520 157 / 161 / 159.
     const int64_t places = dbdc_places(p) / (together ? 2 : 1);
+    const bool behind_dx = together && dx_db_dc_pays(p);
     int best = DBDC_HEADS;
     double best_cost = 0;
     for (int k = DBDC_HEADS; k >= 1; --k) {
         const int slices = (hpg + k - 1) / k;
         if (k < DBDC_HEADS && (slices > DBDC_SLICES_MAX || (hpg + slices - 1) / slices != k)) continue;  // (the fewest heads for this many slices)
-        const double rounds = (double)((tiles * slices + places - 1) / places);
-        const double cost = rounds * (3 + steps * std::min(k, hpg)) + slices * slice_cost;
+        const double life = 3 + steps * std::min(k, hpg);
+        const double cost = (behind_dx ? (double)(tiles * slices) / places + 1.5 : (double)((tiles * slices + places - 1) / places)) * life + slices * slice_cost;
         if (k == DBDC_HEADS || cost < best_cost) { best = k; best_cost = cost; }
     }
     return best;
