@@ -1293,15 +1293,22 @@ static int launch_dcb_t(const bimamba2_params *p, bool add_up) {
 
 // Head slices where bimamba2_bwd owns dCB.
 // The kernel rebuilds C.B^T (16 bits, wide heads): a slice starts with its own copy of the tile, and the last launch reads the slices in
-// float32 instead of one in 16 bits; they pay while compute units are left without two workgroups.  us a training pass with 1 / 2 / 4
-// slices, heads of 64, dstate 64, chunks of 256: 48 heads, 64 tiles 161 / 135 / 124, 128 tiles 183 / 158 / 152, 384 tiles 312 / 297 / 314;
-// 32 heads of 128, dstate 128, 96 tiles 264 / 240 / 234; from 512 tiles on they cost (32 heads 244 / 249 / 271; 16 heads 154 / 157 / 167).
-// Between 256 and 384 tiles few heads give little (24 heads 150 / 143 / 146, with dstate 128 306 / 302 / 316): one slice up to 31 heads.
+// float32 instead of one in 16 bits; they pay while compute units are left without two workgroups.  us with 1 / 2 / 4 slices, chunks of 256:
+//   heads of 128 (the ring), a training pass: dstate 64, 24 heads, 64 tiles 136 / 118 / 112, 128 tiles 157 / 138 / 136, 384 tiles 264 / 258 / 279; 16 heads, 512
+//     tiles 214 / 222 / 244; dstate 128, 32 heads, 96 tiles 258 / 235 / 231
+//   heads of 64 (waves that take whole heads split a tile's heads themselves), dCB with the state passing beside it + the last launch, dstate 64: 24 heads, 16
+//     tiles 31 / 25 / 26, 32 tiles 33 / 27 / 28; 64 tiles: 12 heads 25 / 24 / 28, 24 34 / 28 / 28, 32 39 / 31 / 30, 48 50 / 36 / 33; 96 tiles: 16 heads 28 / 26 / 28,
+//     24 34 / 29 / 33, 48 50 / 38 / 40; 128 tiles: 12 heads 26 / 25 / 29, 24 35 / 29 / 33, 48 51 / 38 / 38; 192 of 24 35 / 31 / 38; 256 of 24 36 / 34 / 41, of 32 43 / 40 / 46; 384
+//     of 24 41 / 46 / 54, of 32 48 / 51 / 59; 512 of 16 36 / 47 / 54
+// So four up to 95 tiles (fewer heads than 16 make fewer), then for heads of 64 two below 256 (at 256 from 32 heads on) and one beyond; for heads of
+// 128 four up to 128, three up to 170, two up to 255, or 384 from 32 heads on.
 // All of these are chunks of 256, where the last launch adds the slices up.  Where none does (dt of a type of its own in chunks of up to
 // 128, chunks between, state dimensions other than 64 and 128 in chunks of 256) they take a launch for it and part the dCB launch from
-// the state passing, 5 us that 16 heads do not earn; 1 slice -> as above: 8 heads of 64, 2048 positions, dstate 192 181 -> 184, 12 heads 207 -> 211,
-// 16 heads 223 -> 226, 24 heads 259 -> 254; float16 dt beside bfloat16, dstate 64, 1024 positions 8 heads 85 -> 90, 32 heads 133 -> 113, 48
-// heads 161 -> 128; 3000 positions, 16 heads 123 -> 124, 20 heads 131 -> 129.
+// the state passing.  us a pass with one slice -> with the number chosen where a launch adds up (heads of 64, dstate 192): 8 heads, 64 tiles and up lose; 64
+// tiles: 17 heads 218 -> 217, 24 228 -> 228, 32 255 -> 251, 48 310 -> 302; 128 tiles: 17 heads 241 -> 246, 24 260 -> 268, 48 401 -> 405; 224 tiles: 24 heads 340 ->
+// 353, 48 573 -> 603; float16 dt beside bfloat16, dstate 64, chunks of 128: 32 tiles: 8 heads 81 -> 89, 32 112 -> 103, 48 135 -> 122; 96 tiles: 16 heads 114 -> 122,
+// 24 134 -> 143, 32 150 -> 155, 48 194 -> 193.  So 16 heads or fewer are not cut, and up to 64 (of 64 channels) not from 96
+// tiles on.
 // The kernel reads C.B^T (float32, and 16-bit shapes whose state or headdim is no multiple of what the rebuilding kernel takes: the ring
 // with a narrow state or narrow heads; through registers where rows are not aligned).
 // A workgroup is one chain over its heads, 5 to 7 us a head through registers in float32, 3 to 5 in 16 bits and 1.5 in the ring,
@@ -1321,13 +1328,13 @@ int choose_dcb_slices(const bimamba2_params *p) {
     const int64_t wgs = (int64_t)p->batch * nchunks(p) * p->ngroups * nqt * nqt;
     int wanted = usual;
     if (dcb_recomputes_cb(p)) {
-        if (hpg <= 16 && !bwd_tail_merged(p) && !bwd_tail_small(p)) return usual;
-        // (heads of 64: waves that take whole heads split a tile's heads themselves.  us of dCB with the state passing beside it + the last launch with
-        // 1 / 2 / 4 slices: 64 tiles of 64 heads 62 / 43 / 37; 128 of 24 heads 35 / 30 / 34; 144 of 16 30 / 29 / 34; 256 of 24 37 / 36 / 41;
-        // 384 of 32 49 / 54 / 65)
         const bool heads = p->headdim == 64;
+        if (!bwd_tail_merged(p) && !bwd_tail_small(p)) {
+            if (hpg <= 16) return usual;
+            if (heads && wgs >= 96 && hpg <= 64) return 1;
+        }
         if (wgs < 256 || (wgs <= (heads ? 256 : 384) && hpg >= DCB_SLICE_HEADS))
-            wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 4, 4, heads && wgs >= 128 ? 2 : std::max<int64_t>(512 / wgs, 2)}));
+            wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 4, 4, heads && wgs >= 96 ? 2 : std::max<int64_t>(512 / wgs, 2)}));
     } else {
         const int most = p->dtype == BIMAMBA2_F32 ? (hpg < 6 ? 256 : 768) : std::min(768, 32 * hpg);      // workgroups
         wanted = (int)std::max<int64_t>(usual, std::min<int64_t>({hpg / 2, 8, most / wgs}));

@@ -292,6 +292,14 @@ def test_head_slices_of_dcb_where_nothing_adds_them_up(chunk, dstate, more, adde
         assert _dcb_slices(**_contiguous(4, chunk, heads, 64, 1, dstate, chunk, _lib.BF16), **more) == slices, heads
 
 
+# heads of 64 at the line between 64 and 96 tiles: fewer slices behind it, one where no launch adds them up
+@pytest.mark.parametrize("heads,rows,chunk,dstate,slices", [(24, 4, 256, 64, 4), (24, 6, 256, 64, 2), (48, 6, 256, 128, 2), (24, 15, 256, 64, 2), (24, 16, 256, 64, 1), (32, 16, 256, 64, 2),
+                                                            (32, 17, 256, 64, 1), (48, 4, 256, 192, 4),
+                                                            (24, 6, 256, 192, 1), (64, 6, 256, 192, 1), (65, 6, 256, 192, 2), (24, 32, 256, 192, 1), (24, 7, 192, 64, 4), (24, 11, 192, 64, 1)])
+def test_head_slices_of_dcb_of_heads_of_64(heads, rows, chunk, dstate, slices):
+    assert _dcb_slices(**_contiguous(rows, chunk, heads, 64, 1, dstate, chunk, _lib.BF16)) == slices
+
+
 def test_workspace_sizes_are_kept_apart_by_what_the_slices_depend_on():
     """16 heads of 64 in chunks of 128: four slices of dCB with dt in float32, one with dt of a type of its own, or dB at an odd address in chunks of 256"""
     def size(chunk, dt_dtype, dB):
