@@ -16,10 +16,10 @@ static inline hipStream_t stream_of(const bimamba2_params *p) { return reinterpr
 constexpr int scan_waves_per_simd(int bytes, int qt, int nj, int nf) { return nf > 0 || qt > 1 || bytes == 2 ? 4 : 8; }
 
 // (what a workgroup does: scan_body.hpp)
-template <typename T, int QT, int NJ, bool BWD, bool FAST, int NF, bool UNI = false>
+template <typename T, int QT, int NJ, bool BWD, bool FAST, int NF, bool UNI = false, bool STATES = true>
 __global__ __launch_bounds__(SCAN_THREADS, scan_waves_per_simd(sizeof(T), QT, NJ, NF)) void chunk_scan_kernel(const bimamba2_params p, int nc, int npt) {
     __shared__ __attribute__((aligned(16))) char lds[ScanMap<T, QT, NJ, BWD, NF>::LDS];
-    chunk_scan_body<T, QT, NJ, BWD, FAST, NF, UNI>(p, nc, npt, blockIdx.x, lds);
+    chunk_scan_body<T, QT, NJ, BWD, FAST, NF, UNI, STATES>(p, nc, npt, blockIdx.x, lds);
 }
 
 static inline bool al16(const void *ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; }
@@ -70,10 +70,16 @@ static int launch_scan_t(const bimamba2_params *p, bool free16) {
     dim3 grid(p->batch * nc * p->nheads * npt);
     hipStream_t s = reinterpret_cast<hipStream_t>(p->stream);
     const bool fast = scan_fast(p, BWD, pw, VS);
-#define BM2_SCAN(QTV, NJV)                                                                                                        \
-    do {                                                                                                                          \
-        if (fast) hipLaunchKernelGGL((chunk_scan_kernel<T, QTV, NJV, BWD, true, 0>), grid, dim3(SCAN_THREADS), 0, s, *p, nc, npt); \
-        else hipLaunchKernelGGL((chunk_scan_kernel<T, QTV, NJV, BWD, false, 0>), grid, dim3(SCAN_THREADS), 0, s, *p, nc, npt);     \
+    const bool states = BWD ? p->dstates_f || p->dstates16_f : p->states_f || p->states16_f;       // (else one_chunk())
+#define BM2_SCAN_K(QTV, NJV, FAST, NF)                                                                                                          \
+    do {                                                                                                                                        \
+        if (states) hipLaunchKernelGGL((chunk_scan_kernel<T, QTV, NJV, BWD, FAST, NF>), grid, dim3(SCAN_THREADS), 0, s, *p, nc, npt);             \
+        else hipLaunchKernelGGL((chunk_scan_kernel<T, QTV, NJV, BWD, FAST, NF, false, false>), grid, dim3(SCAN_THREADS), 0, s, *p, nc, npt);      \
+    } while (0)
+#define BM2_SCAN(QTV, NJV)                          \
+    do {                                            \
+        if (fast) BM2_SCAN_K(QTV, NJV, true, 0);    \
+        else BM2_SCAN_K(QTV, NJV, false, 0);        \
     } while (0)
     const int qt = Q <= 128 ? 1 : 2;             // 16-row tiles per wave (8 waves)
     // 16-bit copies of the entering states: known to the kernels that rebuild CB only
@@ -85,6 +91,7 @@ static int launch_scan_t(const bimamba2_params *p, bool free16) {
         if ((free16 || (c16f && (p->causal || c16b))) && (BWD ? p->CBT : p->CB) == nullptr && chunk_scan_uses_scan16(p, BWD))
             return launch_chunk_scan16(p, BWD);
         if (p->causal) {                                // single-direction comparator: the fused kernels only
+            if (!states) return BIMAMBA2_EINVAL;
             if (!scan_recomputes_cb(p, BWD)) return BIMAMBA2_EUNSUPPORTED;
             if (qt == 1) hipLaunchKernelGGL((chunk_scan_kernel<T, 1, 4, BWD, true, 2, true>), grid, dim3(SCAN_THREADS), 0, s, *p, nc, npt);
             else hipLaunchKernelGGL((chunk_scan_kernel<T, 2, 4, BWD, true, 2, true>), grid, dim3(SCAN_THREADS), 0, s, *p, nc, npt);
@@ -92,8 +99,8 @@ static int launch_scan_t(const bimamba2_params *p, bool free16) {
         }
         if ((BWD ? p->CBT : p->CB) == nullptr) {
             if (!scan_recomputes_cb(p, BWD)) return BIMAMBA2_EINVAL;   // (the kernels below rebuild C.B^T at state dimension 64 only)
-            if (qt == 1) hipLaunchKernelGGL((chunk_scan_kernel<T, 1, 4, BWD, true, 2>), grid, dim3(SCAN_THREADS), 0, s, *p, nc, npt);
-            else hipLaunchKernelGGL((chunk_scan_kernel<T, 2, 4, BWD, true, 2>), grid, dim3(SCAN_THREADS), 0, s, *p, nc, npt);
+            if (qt == 1) BM2_SCAN_K(1, 4, true, 2);
+            else BM2_SCAN_K(2, 4, true, 2);
             return check_launch();
         }
     }
@@ -104,6 +111,7 @@ static int launch_scan_t(const bimamba2_params *p, bool free16) {
     else if (pw == 32) { if (qt == 1) BM2_SCAN(1, 2); else BM2_SCAN(2, 2); }
     else if constexpr (sizeof(T) == 2) { if (qt == 1) BM2_SCAN(1, 4); else BM2_SCAN(2, 4); }   // (float32: 32 columns at most)
 #undef BM2_SCAN
+#undef BM2_SCAN_K
     return check_launch();
 }
 
