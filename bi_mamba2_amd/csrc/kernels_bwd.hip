@@ -596,9 +596,11 @@ int choose_dbdc_heads(const bimamba2_params *p, bool by_heads, bool together) {
     // what counts is their work over all places, and the last workgroup, which ends alone.  us a pass, slices as for two launches / by half
     // the places / as here: bfloat16, heads of 32, dstate 16, two groups, 16 x 520, 16 heads 162 / 167 / 164; 20 x 500, heads of 16, dstate 32
     // 173 / 178 / 173; 4 x 2048, 16 heads of 16, dstate 16 137 / 132 / 133; float32, 1 x 6000, 16 heads of 32 179 / 182 / 180; 16 x 520
-    // 265 / 247 / 247; 8 x 520 157 / 161 / 159.
+    // 265 / 247 / 247; 8 x 520 157 / 161 / 159.  (Wider states, whose workgroups have a CU each, keep to rounds: float32, 2 x 196, 8 groups of
+    // 2 heads of 64, dstate 64 89 / 89, by the work 93; 2 x 300, 16 heads of 16 in two groups, dstate 96 103 / 101; bfloat16, 2 x 900, 16 heads of 16 in four, dstate 48
+    // 91 / 86.)
     const int64_t places = dbdc_places(p) / (together ? 2 : 1);
-    const bool behind_dx = together && dx_db_dc_pays(p);
+    const bool behind_dx = together && p->dstate <= 32 && dx_db_dc_pays(p);
     int best = DBDC_HEADS;
     double best_cost = 0;
     for (int k = DBDC_HEADS; k >= 1; --k) {
