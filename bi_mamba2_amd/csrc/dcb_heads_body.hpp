@@ -18,8 +18,9 @@ namespace bm2 {
 //    tiles of 32 heads): there neighbouring lanes hold different rows, so each 16 bytes are a request of their own.
 //  * Off the diagonal the decay is a row factor times a column factor about the tile's edge, so a position has one exponential.
 // Bound by instruction issue: 480 vector instructions and 32 products (16 x 16 x 32) a head and wave off the diagonal, 1.25 us at two
-// waves a SIMD, 1.45 with the loads.  16-row stripes of a tile to four waves, all of them on the same head with a barrier each (the
-// kernel before this one): 51 us against 34 for 512 tiles of 32 heads, 134 against 88 for 8192 tiles of 4 (heads of 64, bfloat16).
+// waves a SIMD, 1.45 with the loads.  (Counters of the launch with the state passing, 4 x 2048, 32 heads: vector units busy 58 % of the time, matrix
+// units 11 %, LDS 22 %, 28 % of the waves' time waiting for an instruction; 8 groups of 4 heads, 4 x 4096: 46, 8, 23 and 25 %.)  16-row
+// stripes of a tile to four waves, all of them on the same head with a barrier each (the kernel before this one): 51 us against 34 for 512 tiles of 32 heads, 134 against 88 for 8192 tiles of 4 (heads of 64, bfloat16).
 // At headdim 128 a tile and head are 32 KB, and a wave waits for the second half of them: 88 us instead of 86 with the state passing (1024
 // tiles of 16 heads), 70 without it; with 32 KB of LDS a wave, i.e. one workgroup a CU, 87 without it: such heads stay with that kernel.
 // Errors against 64 bits are those of that kernel (the sums of a tile's heads are split over W waves and added up in wave order).
