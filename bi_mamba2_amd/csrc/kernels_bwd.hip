@@ -1216,8 +1216,8 @@ static int dcb_waves(const bimamba2_params *p, int slices, double *us = nullptr)
 }
 // Whether the state passing that shares dCB's launch is the longer part: float32 states (their gradients read and written, the states read:
 // 12 bytes an element at 5 TB/s).  The ring's workgroups are four to a CU and stay so beside it, those of the kernel above fill the LDS by
-// twos and it has to wait for them.  us ring / heads: 8 x 2048, 32 heads, dstate 32 (200 MB) 65 / 76; 4 x 2048, dstate 96 (300 MB) 66 / 74; but
-// 4 x 2048, 8 groups, dstate 32 (100 MB) 54 / 51
+// twos and it has to wait for them.  us ring / heads: 4 x 2048, 32 heads, dstate 96 (300 MB) 66 / 70, 12 heads in 4 groups, 2 x 8192, chunks of 128, dstate 96 (230 MB) 77 / 75
+// to 91; but 8 groups of 4, dstate 32 (100 MB) 50 / 50, 1 x 4096, 24 heads, dstate 128 (75 MB) 40 / 30
 static bool dcb_sp_streams(const bimamba2_params *p, int slices) {
     if (p->dstates16_f || !p->dstates_f) return false;
     double us;

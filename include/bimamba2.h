@@ -236,7 +236,8 @@ int bimamba2_fwd(const bimamba2_params *p);
  * `workspace` / `workspace_bytes` are ignored: the intermediates that the caller does not bring live in a buffer of
  * BIMAMBA2_STATIC_SCRATCH_BYTES that is part of the library's device image (each GPU the library runs on holds one until
  * the process ends).  Calls no hipMalloc / hipFree or any other allocating routine.  Returns BIMAMBA2_ESCRATCH when
- * bimamba2_workspace_bytes(p, 0) exceeds the buffer.  All calls on one GPU share that GPU's buffer: calls that overlap
+ * this pass needs more than the buffer (bimamba2_workspace_bytes(p, 0), enough for tensors of states named later, may be more than the pass needs).
+ * All calls on one GPU share that GPU's buffer: calls that overlap
  * on one GPU (two streams, two host threads) race; calls on one stream, one after the other, are safe. */
 #define BIMAMBA2_STATIC_SCRATCH_BYTES (64u << 20)
 int bimamba2_fwd_static(const bimamba2_params *p);
