@@ -436,3 +436,33 @@ def test_state_passing_of_float32_states_beside_dcb_does_not_depend_on_the_batch
 
     for many, one in zip(results(b), results(1)):
         assert torch.isfinite(many).all() and torch.equal(many[:1], one)
+
+
+@pytest.mark.parametrize("H,L,N,dtype", [(17, 1536, 192, torch.bfloat16), (24, 1700, 160, torch.float16), (64, 1600, 192, torch.bfloat16)])      # 6 and 7 chunks: 96 and 112 tiles
+def test_heads_of_64_in_one_slice_of_dcb_where_no_launch_adds_slices_up(ops, monkeypatch, H, L, N, dtype):
+    """more than 16 heads, dCB in the launch of the state passing; against two slices in buffers of the caller's, a launch that adds them up and a state passing of
+    its own.  dB and dC enter the sums of a tile's heads in another order: a float32 sum off by its last bits rounds to another unit of the type now and then"""
+    b, G, P, Q = 1, 1, 64, 256
+    nc = -(-L // Q)
+    inp = to_dev(make_case(b, L, H, P, G, N, dtype))
+    dout = torch.randn(b, L, H, P, generator=torch.Generator().manual_seed(L)).to(dtype).cuda()
+    grads = lambda: ops._mamba_chunk_scan_combined_bwd(dout, inp["x"], inp["dt"], inp["A"], inp["B"], inp["C"], None, Q, dt_bias=inp["dt_bias"], dt_softplus=True)
+    got, own, kept = grads(), ops._Call.workspace, {}
+
+    def workspace(c, is_bwd):
+        c.p.dcb_slices = 2
+        for name in ("dCB", "dCBT"):
+            kept[name] = c.new(name, (2, b, nc, G, Q, Q))
+        return own(c, is_bwd)
+
+    monkeypatch.setattr(ops._Call, "workspace", workspace)
+    want = grads()
+    assert len(kept) == 2
+    for i, (g, w) in enumerate(zip(got, want)):
+        if not torch.is_tensor(g):
+            continue
+        assert torch.isfinite(g.float()).all()
+        if g.shape == inp["B"].shape:
+            assert float((g.double() - w.double()).norm()) <= (2.0 ** -9 if dtype == torch.bfloat16 else 2.0 ** -12) * float(w.double().norm())
+        else:
+            assert torch.equal(g, w), i
