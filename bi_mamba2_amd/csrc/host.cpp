@@ -648,8 +648,8 @@ bimamba2_norm_params layer_norm_params(const LayerShape &s, const LayerOpts &o, 
 
 // ---- the projections' matrix products -------------------------------------------------------------------------------
 // c (m x n, row pitch ldc) = sum_k A(m, k) B(n, k) (+ bias), by this library's kernel; false where it does not take the problem.
-// a, b: 2-d with unit stride along columns; a_kc: k along a's columns (else along its rows), b_kc likewise.
-bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const Tensor &bias, const Tensor &c) {
+// a, b: 2-d with unit stride along columns; a_kc: k along a's columns (else along its rows), b_kc likewise.  uncut: nor one whose sum it cuts in slices.
+bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const Tensor &bias, const Tensor &c, bool uncut = false) {
     if (c.scalar_type() == at::kFloat || a.stride(1) != 1 || b.stride(1) != 1 || c.stride(1) != 1) return false;
     bimamba2_gemm_params g{};
     g.m = c.size(0);
@@ -667,6 +667,7 @@ bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const T
     g.c = c.mutable_data_ptr();
     g.stream = stream_of(c);
     const size_t need = api.gemm_workspace(&g);
+    if (need && uncut) return false;
     Tensor ws;
     if (need) {
         ws = device_empty({(int64_t)need}, at::kByte, c);
@@ -690,6 +691,13 @@ bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const T
 //   gradients of the inputs: 197 x 384 241 -> 214, 170 -> 163; 512 x 768 240 -> 230, 231 -> 228; 512 x 1024 273 -> 264, 270 -> 262; 2048 x 768 (4.8 for
 //     the second) 314 -> 316, 313 -> 314
 constexpr double OWN_INFERENCE_FLOPS = 1.5e9, OWN_TRAINING_FLOPS = 3e9, OWN_GRADIENT_FLOPS = 5e9;
+// Two kinds go further (replayed graphs, operands from memory; own over library):
+//   forward products whose columns are no multiple of 64, below 16384 rows: 0.89 of the better of the library alone and in two parts (see SPLIT_ROWS) over the 14
+//     of 60 sampled ones with 3 to 20 GFLOP, 0.69 (8572 x 512 by 2192) to 1.11 (488 x 960 by 4382); above 20 1.0 to 1.27
+//   gradients of inputs with twice as many terms as columns (in front of the first projection): 0.84 over 44, 0.63 (155 x 960 from 3998) to 1.06; where
+//     the sum is cut and has more than 20 GFLOP up to 1.30 (5448 x 896 from 3868), and the library keeps it
+constexpr double OWN_RAGGED_FLOPS = 20e9, OWN_CUT_GRADIENT_FLOPS = 20e9;
+constexpr int64_t OWN_RAGGED_ROWS = 16384;
 
 // From so many rows or operations on, the columns of a forward product behind the last multiple of 256 go to the own kernel where the
 // number of columns is no multiple of 64: the library has fast kernels for some of these numbers only.  us, library alone -> in
@@ -704,7 +712,8 @@ constexpr double SPLIT_FLOPS = 25e9;
 void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c, bool training) {
     const int64_t m = c.size(0), n = c.size(1), whole = n / 256 * 256;
     const double per_column = 2.0 * m * x.size(1);
-    if (per_column * n <= (training ? OWN_TRAINING_FLOPS : OWN_INFERENCE_FLOPS) && own_product(x, true, w, true, bias, c)) return;
+    const bool ragged = n % 64 && m < OWN_RAGGED_ROWS;
+    if (per_column * n <= (ragged ? OWN_RAGGED_FLOPS : training ? OWN_TRAINING_FLOPS : OWN_INFERENCE_FLOPS) && own_product(x, true, w, true, bias, c)) return;
     if ((m >= SPLIT_ROWS || per_column * whole >= SPLIT_FLOPS) && n % 64 && whole && c.scalar_type() != at::kFloat && !bias.defined() &&
         own_product(x, true, w.narrow(0, whole, n - whole), true, Tensor(), c.narrow(1, whole, n - whole))) {
         Tensor front = c.narrow(1, 0, whole);
@@ -717,13 +726,15 @@ void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c, 
 
 // c = dy w: the gradient of a projection's input
 void product_nn(const Tensor &dy, const Tensor &w, Tensor c) {
-    if (2.0 * c.size(0) * c.size(1) * dy.size(1) <= OWN_GRADIENT_FLOPS && own_product(dy, true, w, false, Tensor(), c)) return;
+    const double flops = 2.0 * c.size(0) * c.size(1) * dy.size(1);
+    const bool longer = dy.size(1) >= 2 * c.size(1);
+    if ((longer || flops <= OWN_GRADIENT_FLOPS) && own_product(dy, true, w, false, Tensor(), c, flops > OWN_CUT_GRADIENT_FLOPS)) return;
     at::mm_out(c, dy, w);
 }
 
 // c = dy^T x: the gradient of a projection's weight.  Always the own kernel where it exists: the library does not cut the long
-// sum over the rows.  us, library -> own: 3224 x 768 over 16384 rows 149 -> 94, over 4096 43 -> 35, over 1024 16 -> 19, over 197
-// 10 -> 10; 768 x 1536 122 -> 51, 34 -> 25, 13 -> 12, 8 -> 7; 4384 x 1024 over 65536 693 -> 554; 644 x 128 over 4096 31 -> 11.
+// sum over the rows.  us, library -> own: 3224 x 768 over 16384 rows 185 -> 88; 768 x 1536 145 -> 54; 4256 x 1024 over 65536 706 -> 493;
+// 2320 x 512 over 4096 35 -> 27; 1676 x 384 over 992 15 -> 11; 1676 x 384 over 197 7.6 -> 5.9.
 void product_tn(const Tensor &dy, const Tensor &x, Tensor c) {
     if (own_product(dy, false, x, false, Tensor(), c)) return;
     at::mm_out(c, dy.t(), x);

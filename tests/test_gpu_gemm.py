@@ -50,6 +50,38 @@ def test_product(m, n, k, a_kc, b_kc, dtype):
     assert (got - want).abs().max() <= (8e-3 if dtype == torch.bfloat16 else 1e-3) * want.abs().max()
 
 
+# Shapes that take the 256 x 192 (first two lines) and 256 x 256 tiles uncut, with edges in both directions and sums that end in every place of the ring of five
+# steps, a whole last step among them; sums cut in slices, the last one ragged
+@pytest.mark.parametrize("m,n,k", [(11016, 649, 40), (13379, 514, 72), (13816, 543, 104), (13374, 522, 128), (7406, 1064, 168), (13854, 513, 200),
+                                   (12357, 643, 232), (11150, 641, 264),
+                                   (6402, 1775, 24), (5960, 1935, 72), (4621, 2537, 104), (6675, 1750, 136), (8281, 1347, 168), (5897, 1937, 192),
+                                   (7246, 1555, 232), (4865, 2324, 264), (700, 1500, 16381), (1700, 2100, 9001), (3224, 768, 4100)])
+@pytest.mark.parametrize("a_kc,b_kc", [(1, 1), (1, 0), (0, 0)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_product_large_tiles(m, n, k, a_kc, b_kc, dtype):
+    test_product(m, n, k, a_kc, b_kc, dtype)
+
+
+# a last step of 256 x 256 tiles that is not whole: infinities behind its end
+@pytest.mark.parametrize("a_kc,b_kc", [(1, 1), (1, 0), (0, 0)])
+def test_large_tiles_infinities_behind_the_end(a_kc, b_kc):
+    m, n, k = 4865, 2324, 200
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    # the operand's last 8 (or the last rows) hold infinities where k ends; k = 200 of 224 elements
+    a = torch.randint(-3, 4, (m, 224) if a_kc else (224, 4872), device="cuda", generator=gen).bfloat16()
+    b = torch.randint(-3, 4, (n, 224) if b_kc else (224, 2328), device="cuda", generator=gen).bfloat16()
+    for t, kc in ((a, a_kc), (b, b_kc)):
+        (t[:, k:] if kc else t[k:]).fill_(float("inf"))
+    c = torch.empty(m, 2328, device="cuda", dtype=torch.bfloat16)
+    lib, p = _lib.load(), _lib.GemmParams()
+    p.m, p.n, p.k, p.a_kcontig, p.b_kcontig, p.dtype = m, n, k, a_kc, b_kc, _lib.BF16
+    p.lda, p.ldb, p.ldc = a.stride(0), b.stride(0), c.stride(0)
+    p.a, p.b, p.c, p.stream = a.data_ptr(), b.data_ptr(), c.data_ptr(), torch.cuda.current_stream().cuda_stream
+    assert lib.bimamba2_gemm_workspace_bytes(ctypes.byref(p)) == 0 and lib.bimamba2_gemm(ctypes.byref(p)) == 0
+    af, bf = (a[:, :k].float() if a_kc else a[:k, :m].float().t()), (b[:, :k].float().t() if b_kc else b[:k, :n].float())
+    assert torch.equal(c[:, :n], (af @ bf).bfloat16())
+
+
 @pytest.mark.parametrize("b_kc", [1, 0])
 def test_infinities_in_the_last_step(b_kc):
     """what the loads find behind a k that is no multiple of a step takes no part, infinities included"""
