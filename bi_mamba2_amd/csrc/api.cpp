@@ -499,6 +499,18 @@ int bimamba2_fwd(const bimamba2_params *p) {
     bimamba2_params q = *p;
     const size_t need = carve(&q, 0, p->workspace);
     if (need > 256 && (!p->workspace || p->workspace_bytes < need)) return BIMAMBA2_EWORKSPACE;
+    if (scan_once_applies(p)) {
+        REQUIRE(p->dt); REQUIRE(p->A); REQUIRE(p->x); REQUIRE(p->Bm); REQUIRE(p->Cm); REQUIRE(p->out);
+        if (p->has_dt_bias) REQUIRE(p->dt_bias);
+        if (p->has_D) REQUIRE(p->D);
+        if (p->has_z) REQUIRE(p->z);
+        if (q.final_f || q.final_b) {
+            // (the result of such a call is the same in bits whether or not the final states are asked for)
+            TRY(forward_cumsum_and_states(&q));
+            TRY(bimamba2_state_passing_fwd(&q));
+        }
+        return launch_scan_once(p);
+    }
     if (one_chunk(&q)) {
         REQUIRE(q.dt); REQUIRE(q.A); REQUIRE(q.x); REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.out);
         if (q.has_dt_bias) REQUIRE(q.dt_bias);

@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256, 1) void gemm_big_kernel(const bimamba2_gemm_pa
         if constexpr (i < AL) load16_to_lds_at(abase + (size_t)it * astep, ao[i], smem + so + (wave + 4 * i) * 1024);
         else load16_to_lds_at(bbase + (size_t)it * bstep, bo[i - AL], smem + so + G::A_B + (wave + 4 * (i - AL)) * 1024);
     };
-    // The last tile of a k that is no multiple of 64, once this wave's share of it has landed: the elements behind the end
+    // The last step of a k that is no multiple of 32, once this wave's share of it has landed: the elements behind the end
     // become zero (what the loads found there may be an infinity, or no number at all).
     auto clear_tail = [&](unsigned so) __attribute__((always_inline)) {
         typedef unsigned u32x4 __attribute__((ext_vector_type(4)));

@@ -1,0 +1,104 @@
+"""The forward pass of short sequences in one launch, against the quadratic form in float64 and against the chunked launches (which run where
+initial states go in: zeros here), at the edges of its row tiles, steps and operands."""
+
+import pytest
+import torch
+
+from bi_mamba2_amd.ops import bimamba_chunk_scan_combined
+from oracle import bimamba2_oracle as O
+
+pytestmark = pytest.mark.gpu
+
+# Relative 2-norm.  float32: sums of up to 256 products in any order, about sqrt(256) 2^-24 = 1e-6 at worst.  16 bits: the decayed products and the
+# result are rounded once each, 2^-9 (2^-12) uniform: at most sqrt(2) 2^-9 = 2.8e-3 (3.5e-4).
+BOUND = {torch.float32: 1e-6, torch.bfloat16: 2.8e-3, torch.float16: 3.5e-4}
+# the chunked launches round C.B^T or the states to 16 bits besides
+CHUNKED = {torch.float32: 2e-6, torch.bfloat16: 5e-3, torch.float16: 1e-3}
+
+
+def call(t, chunk, initial=False, final=False):
+    (b, _, H, P), N = t["x"].shape, t["B"].shape[-1]
+    zeros = torch.zeros(b, H, P, N, device="cuda") if initial else None
+    with torch.no_grad():
+        return bimamba_chunk_scan_combined(t["x"], t["dt"], t["A"], t["B"], t["C"], chunk, D=t.get("D"), z=t.get("z"), dt_bias=t["dt_bias"],
+                                           dt_softplus=True, initial_states_f=zeros, initial_states_b=zeros, return_final_states=final)
+
+
+def check(t, dtype, chunk, D=True, z=True):
+    t = dict(t)
+    if not D:
+        t.pop("D")
+    if not z:
+        t.pop("z")
+    dev = {k: v.cuda() if not v.is_cuda else v for k, v in t.items()}
+    r = {k: v.double().cpu() for k, v in t.items()}
+    want, _ = O.bimamba2_quadratic(r["x"], r["dt"], r["A"], r["B"], r["C"], D=r.get("D"), z=r.get("z"), dt_bias=r["dt_bias"], dt_softplus=True)
+    got, general = call(dev, chunk), call(dev, chunk, initial=True)
+    assert bool(torch.isfinite(got).all())
+    for a, b, bound in ((got.double().cpu(), want, BOUND[dtype]), (got.double(), general.double(), CHUNKED[dtype])):
+        assert (a - b).norm() <= bound * b.norm(), ((a - b).norm() / b.norm()).item()
+
+
+SHAPES = [  # heads, headdim, groups, dstate
+    (torch.float32, 4, 32, 1, 16), (torch.float32, 2, 16, 2, 32), (torch.float32, 1, 64, 1, 64), (torch.float32, 2, 48, 1, 16),
+    (torch.bfloat16, 4, 64, 1, 64), (torch.bfloat16, 2, 128, 2, 128), (torch.float16, 3, 64, 3, 32), (torch.float16, 2, 64, 1, 64)]
+
+
+@pytest.mark.parametrize("L", [1, 15, 16, 17, 32, 33, 64, 65, 100, 127, 129, 197, 224, 255, 256])
+@pytest.mark.parametrize("dtype,H,P,G,N", SHAPES)
+def test_lengths(L, dtype, H, P, G, N):
+    check(O.make_inputs(2, L, H, P, G, N, seed=L, dtype=dtype, with_z=True), dtype, 64 if dtype == torch.float32 else 256)
+
+
+@pytest.mark.parametrize("dtype,H,P,G,N", SHAPES)
+@pytest.mark.parametrize("D,z", [("none", True), ("hp", False), ("h", False), ("hp", True)])
+def test_operands(dtype, H, P, G, N, D, z):
+    t = O.make_inputs(1, 130, H, P, G, N, seed=3, dtype=dtype, with_z=True)
+    if D == "hp":
+        t["D"] = torch.randn(H, P, generator=torch.Generator().manual_seed(4))
+    check(t, dtype, 128, D=D != "none", z=z)
+
+
+@pytest.mark.parametrize("dt_dtype", [torch.float32, torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dtype,H,P,G,N", [SHAPES[0], SHAPES[4], SHAPES[7]])
+def test_views_and_what_lies_behind_the_end(dt_dtype, dtype, H, P, G, N):
+    """operands as slices of wider buffers, heads and positions at other strides, NaN in every element that is not theirs"""
+    b, L = 3, 77
+    t = O.make_inputs(b, L, H, P, G, N, seed=5, dtype=dtype, with_z=True)
+    t["dt"] = t["dt"].to(dt_dtype)
+
+    def inside(v, spare):
+        wide = torch.full((b, L + 60) + v.shape[2:-1] + (v.shape[-1] + spare,), float("nan"), dtype=v.dtype, device="cuda")
+        wide[:, :L, ..., :v.shape[-1]] = v.cuda()
+        return wide[:, :L, ..., :v.shape[-1]]
+
+    for k, spare in (("x", 16), ("z", 8), ("B", 8), ("C", 24), ("dt", 3)):
+        t[k] = inside(t[k], spare)
+    check(t, dtype, 64)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_strong_decay(dtype):
+    """sums of up to -4000 over the sequence: neither side's factor may overflow, and neighbours keep their weight"""
+    t = O.make_inputs(1, 256, 2, 64, 1, 64, seed=6, dtype=dtype, with_z=False)
+    t["A"] = torch.tensor([-16.0, -1.0])
+    t["dt_bias"] = torch.tensor([1.0, 1.0])
+    check(t, dtype, 256, z=False)
+
+
+@pytest.mark.parametrize("dtype,H,P,G,N", SHAPES)
+def test_a_row_does_not_depend_on_the_batch(dtype, H, P, G, N):
+    t = {k: v.cuda() for k, v in O.make_inputs(7, 200, H, P, G, N, seed=8, dtype=dtype, with_z=True).items()}
+    row = {k: v[4:5] if k in ("x", "dt", "B", "C", "z") else v for k, v in t.items()}
+    assert torch.equal(call(t, 256)[4:5], call(row, 256))
+
+
+@pytest.mark.parametrize("L", [40, 256])
+@pytest.mark.parametrize("dtype,H,P,G,N", SHAPES)
+def test_final_states_besides(dtype, H, P, G, N, L):
+    """the same result in bits, and the final states of the chunked launches"""
+    t = {k: v.cuda() for k, v in O.make_inputs(2, L, H, P, G, N, seed=9, dtype=dtype, with_z=True).items()}
+    out, *final = call(t, 64, final=True)
+    assert torch.equal(out, call(t, 64))
+    for a, b in zip(final, call(t, 64, initial=True, final=True)[1:]):
+        assert torch.equal(a, b)
