@@ -615,6 +615,8 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     // still writes back dz's output, which the memory-bound kernels after it would otherwise wait behind
     const bool dx_db_dc = !one && dx_db_dc_merged(&q);      // (one launch at the end)
     const bool by_heads = !one && !dx_db_dc && dbdc_both_by_heads(&q), both = by_heads || (!one && !dx_db_dc && db_dc_merged(&q));      // dC with dB
+    // and the part of both inside the chunks with them, where dCB is there in 16 bits and nobody asked for the partial sums
+    const bool product = by_heads && dcb16 && !p->dBs && !p->dCs && dbdc_with_product(&q);
     if (dcb_sp && (ncb == dcb_slices(&q))) {
         // the backward state passing (streams, few instructions) rides along with the dCB kernel in one launch
         if (!dx_db_dc && !one && !both) TRY(bimamba2_chunk_scan_bwd_dc(&q));
@@ -625,7 +627,9 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
             REQUIRE(q.ddA_chunk_f); REQUIRE(q.ddA_chunk_b);
         }
         if (q.has_z) REQUIRE(q.dout_x); else REQUIRE(q.dout);
-        TRY(launch_bwd_dcb_sp(&q, dcb16));
+        bimamba2_params qd = q;
+        if (product) qd.dCBT = nullptr;      // (nobody reads it)
+        TRY(launch_bwd_dcb_sp(&qd, dcb16));
     } else {
         TRY(check_bwd_dcb(&q));
         if (one) TRY(launch_bwd_dcb(&q, ncb == 1));
@@ -647,7 +651,7 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     } else if (both) {
         REQUIRE(q.x); REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dBs); REQUIRE(q.dCs); REQUIRE(q.u_f); REQUIRE(q.u_b); REQUIRE(q.v_f); REQUIRE(q.v_b);
         if (!by_heads) { REQUIRE(q.states_f); REQUIRE(q.states_b); REQUIRE(q.dstates_f); REQUIRE(q.dstates_b); }
-        TRY(by_heads ? launch_dbdc_both(&q) : launch_db_dc(&q));
+        TRY(by_heads ? launch_dbdc_both(&q, product) : launch_db_dc(&q));
     } else if (!one) TRY(bimamba2_chunk_state_bwd_db(&q));
     ReduceJobs jobs;
     {
@@ -669,7 +673,9 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
         bimamba2_params qc = q;
         qc.red = q.red + (size_t)q.batch * nchunks(&q) * q.nheads * q.headdim;
         REQUIRE(q.ddt); REQUIRE(q.dA); REQUIRE(q.dB); REQUIRE(q.dC);
-        if (bwd_tail_merged(&q)) {
+        if (product) {
+            TRY(launch_chunk_cumsum_bwd(&qc, &jobs));
+        } else if (bwd_tail_merged(&q)) {
             TRY(launch_bwd_tail(&qc, &jobs, dcb16, ncb));
         } else if (tail_small) {
             REQUIRE(q.Bm); REQUIRE(q.Cm); REQUIRE(q.dt); REQUIRE(q.A);

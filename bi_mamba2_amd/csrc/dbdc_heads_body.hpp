@@ -20,8 +20,14 @@ template <int W> struct DbdcHeadsMap {
     static_assert(COMB <= VEC, "the exchange lies over the rings");
 };
 
+// PRODUCT: the part of dB (dC) inside the chunk, sum_t dCB[t, s] C[t, n] (sum_s dCB[t, s] B[s, n]), is formed here as well, the sums over the
+// heads are added to it from their registers and the result leaves in its own type, with the bits that two launches give.  That takes one slice of heads,
+// chunks of 256 and dCB in 16 bits, of which no transpose is needed: dC reads its tiles as they lie, dB by transpose reads.  The
+// chunk's C (B) rows lie in the second halves of the four rings, 64 rows in each, for all waves; the 64 x 64 pieces of dCB in the first
+// halves, W of a tile's four at a time, with one wave to a tile asked for under the last head and under the products.  Bound by
+// memory with one wave to a tile (4 x 4096, 32 heads in 8 groups: 82 us, 71 without the product; 450 MB), by its waits else (16 x 1024, 24 heads: 41.5, 38.6 without).
 // bid.x: (batch, chunk, group), bid.y: row tiles, bid.z: slice of hps heads
-template <typename T, bool IS_DB, int W>
+template <typename T, bool IS_DB, int W, bool PRODUCT>
 __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, int nc, int nqt, int hps, BlockId bid, unsigned char *smem) {
     typedef Mma<T> M;
     typedef typename M::Frag Frag;
@@ -111,6 +117,29 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
         }
     };
 
+    // ---- PRODUCT: this wave's 64 of the chunk's C (B) rows, and the piece of dCB at k rows (columns) that it brings
+    const char *krows = nullptr, *cb = nullptr;
+    if constexpr (PRODUCT) {
+        const int k0 = min(wave * 64, limit - 1);
+        krows = uniform_ptr(IS_DB ? reinterpret_cast<const T *>(p.Cm) + b * p.C_sb + ((int64_t)c * Q + k0) * p.C_sl + g * p.C_sg
+                                  : reinterpret_cast<const T *>(p.Bm) + b * p.B_sb + ((int64_t)c * Q + k0) * p.B_sl + g * p.B_sg);
+        cb = uniform_ptr(reinterpret_cast<const T *>(p.dCB) + (int64_t)bid.x * Q * Q + (IS_DB ? r0 : (int64_t)r0 * Q));
+    }
+    auto request_krows = [&]() __attribute__((always_inline)) {
+        const int ln = lane_number(), r = ln >> 3, last = max(limit - 1 - wave * 64, 0);
+        const unsigned stride = (unsigned)((IS_DB ? p.C_sl : p.B_sl) * (int64_t)sizeof(T));
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            load16_to_lds_at(krows, __umul24(min(k * 8 + r, last), stride) + (((ln & 7) ^ tile64_swz(k * 8 + r)) << 4), ring + L::TILE + k * 1024);
+    };
+    auto request_cb = [&](int piece) __attribute__((always_inline)) {      // (dB reads it transposed, dC as it lies)
+        const int ln = lane_number(), r = ln >> 3;
+        const char *base = cb + piece * (IS_DB ? 64 * 512 : 128);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            load16_to_lds_at(base + k * 8 * 512, r * 512 + (((ln & 7) ^ (IS_DB ? tile64_swz(k * 8 + r) : r)) << 4), ring + k * 1024);
+    };
+
     // ---- this lane's B (C) values: row 16 q + 4 lg + i, column 16 j + lr; the rows pass through the ring
     f32x4 cr[4][4];
     f32x4 tot[4][4] = {};
@@ -198,6 +227,10 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
                         request_state(sb);
                         sb += piece + 1 < np ? 64 * N * (int64_t)sizeof(T) : s_wrap;
                     } else if (it + 1 < nit) request_head();
+                    else if (PRODUCT && W == 1) {                  // (nobody else's: the ring is this wave's until the barrier)
+                        request_krows();
+                        request_cb(0);
+                    }
                 }
                 f32x4 s4[2] = {raw_lds_read_at<f32x4, q0 * 64>(va + lg * 16), raw_lds_read_at<f32x4, q0 * 64 + 64>(va + lg * 16)};
                 raw_lds_wait();
@@ -253,6 +286,103 @@ __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, in
 #pragma unroll
                     for (int j = 0; j < 4; ++j) tot[q][j] += comb[(((ti * 4 + q) * (W - 1) + sl) * 4 + j) * 64];
             }
+    }
+    if constexpr (PRODUCT) {
+        if constexpr (W > 1) __syncthreads();      // (everybody has read the stripes)
+        if (W > 1 || nit == 0) {
+            request_krows();
+            if (live) request_cb(hw);
+        }
+        const unsigned smem_a = lds_addr(smem);
+        const int kk = 8 * lge + (lre >> 2), nn = 4 * (lre & 3);
+        constexpr int NS = 4 / W;                  // this wave's stripes: 16 rows from 16 (W i + hw) on
+        f32x4 inner[NS][4] = {};
+#pragma unroll 1
+        for (int step = 0; step < 4 / W; ++step) {
+            wait_vmcnt<0>();
+            if (W > 1 || step == 0) __syncthreads();
+            if (live)
+#pragma unroll 1
+                for (int k = 0; k < W; ++k) {
+                    const int kb = step * W + k;
+                    const unsigned aa = smem_a + (ti * W + k) * L::RING, ka = smem_a + kb * L::RING + L::TILE;
+                    static_for<0, 2>([&](auto KS) __attribute__((always_inline)) {
+                        constexpr int ks = decltype(KS)::value;
+                        Frag av[NS];
+                        i16x4 alo[NS], ahi[NS], lo[4], hi[4];
+#pragma unroll
+                        for (int i = 0; i < NS; ++i) {
+                            const int q = i * W + hw;
+                            if constexpr (IS_DB) {
+                                alo[i] = raw_lds_tr16_read_at<ks * 4096>(aa + tile64_tr_offset(kk, q * 16 + nn));
+                                ahi[i] = raw_lds_tr16_read_at<ks * 4096>(aa + tile64_tr_offset(kk + 4, q * 16 + nn));
+                            } else av[i] = raw_lds_read_at<Frag, 0>(aa + (q * 16 + lre) * 128 + (((ks * 4 + lge) ^ (le & 7)) << 4));
+                        }
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            lo[j] = raw_lds_tr16_read_at<ks * 4096>(ka + tile64_tr_offset(kk, j * 16 + nn));
+                            hi[j] = raw_lds_tr16_read_at<ks * 4096>(ka + tile64_tr_offset(kk + 4, j * 16 + nn));
+                        }
+                        raw_lds_wait();
+#pragma unroll
+                        for (int i = 0; i < NS; ++i)
+                            if constexpr (IS_DB) { raw_lds_use(alo[i]); raw_lds_use(ahi[i]); }
+                            else raw_lds_use(av[i]);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) { raw_lds_use(lo[j]); raw_lds_use(hi[j]); }
+                        __builtin_amdgcn_sched_barrier(0);
+                        if (W == 1 && ks == 1 && step + 1 < 4) request_cb(step + 1);       // (the piece has been read)
+                        // rows behind the sequence hold its last one again
+                        const int n = limit - kb * 64 - ks * 32 - 8 * lge;
+                        if (kb * 64 + ks * 32 + 32 > limit)
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) {
+                                    lo[j][i] = i < n ? lo[j][i] : (short)0;
+                                    hi[j][i] = i + 4 < n ? hi[j][i] : (short)0;
+                                }
+#pragma unroll
+                        for (int i = 0; i < NS; ++i) {
+                            if constexpr (IS_DB) av[i] = __builtin_bit_cast(Frag, __builtin_shufflevector(alo[i], ahi[i], 0, 1, 2, 3, 4, 5, 6, 7));
+#pragma unroll
+                            for (int j = 0; j < 4; ++j)
+                                inner[i][j] = M::mma(av[i], __builtin_bit_cast(Frag, __builtin_shufflevector(lo[j], hi[j], 0, 1, 2, 3, 4, 5, 6, 7)), inner[i][j]);
+                        }
+                    });
+                }
+            if constexpr (W > 1) {
+                __syncthreads();                   // (the tile's waves have read the pieces)
+                if (live && step + 1 < 4 / W) request_cb((step + 1) * W + hw);
+            }
+        }
+        if (!live) return;
+        // out through this wave's piece of LDS as whole rows of 128 bytes; 16-byte unit u of row r at u ^ (r / 4) % 8
+        const int64_t o_sl = (IS_DB ? p.dB_sl : p.dC_sl) ? (IS_DB ? p.dB_sl : p.dC_sl) : (int64_t)p.ngroups * N;
+        const int64_t o_sb = (IS_DB ? p.dB_sl : p.dC_sl) ? (IS_DB ? p.dB_sb : p.dC_sb) : p.seqlen * o_sl;
+        T *out = reinterpret_cast<T *>(IS_DB ? p.dB : p.dC) + b * o_sb + ((int64_t)c * Q + r0) * o_sl + (int64_t)g * N;
+        T *img = reinterpret_cast<T *>(ring);
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (q % W == hw)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) inner[q / W][j] += tot[q][j];
+#pragma unroll
+        for (int k = 0; k < NS; ++k)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int t = k * 16 + lge * 4 + i, s = j * 16 + lre;
+                    img[t * 64 + (((s >> 3) ^ ((t >> 2) & 7)) << 3) + (s & 7)] = from_f<T>(inner[k][j][i]);
+                }
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int k = 0; k < 2 * NS; ++k) {
+            const int t = k * 8 + (le >> 3), u = le & 7, r = ((k >> 1) * W + hw) * 16 + (k & 1) * 8 + (le >> 3);
+            if (r < valid) *reinterpret_cast<f32x4 *>(out + r * o_sl + u * 8) = *reinterpret_cast<const f32x4 *>(img + t * 64 + ((u ^ ((t >> 2) & 7)) << 3));
+        }
+        return;
     }
     if (!live) return;
     float *out = (IS_DB ? p.dBs : p.dCs) + (int64_t)bid.z * p.batch * p.seqlen * p.ngroups * N;

@@ -735,7 +735,7 @@ __device__ __forceinline__ void bwd_dcb_ring_body(const bimamba2_params &p, int 
                 v4[i] = from_f<T>(dcb[j][i]);
                 out[(int64_t)(t0 + trow + i) * Q + s] = v4[i];
             }
-            *reinterpret_cast<uint2 *>(outT + (int64_t)s * Q + t0 + trow) = *reinterpret_cast<const uint2 *>(v4);
+            if (p.dCBT) *reinterpret_cast<uint2 *>(outT + (int64_t)s * Q + t0 + trow) = *reinterpret_cast<const uint2 *>(v4);
         }
         return;
     }

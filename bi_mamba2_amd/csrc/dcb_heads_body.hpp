@@ -437,7 +437,7 @@ __device__ __forceinline__ void bwd_dcb_heads_body(const bimamba2_params &p, int
     }
     // dCB / dCBT in the element type of the inputs (inside bimamba2_bwd, one head slice: their one reader rounds them to that type
     // for its MFMA anyway, so nothing changes but the bytes moved), through LDS as whole rows of 128 bytes.  16-byte units of a row lie
-    // at unit ^ (row / 4) % 8 (dCB, written four rows at a time) and unit ^ row % 8 (the transpose).
+    // at unit ^ (row / 4) % 8 (dCB, written four rows at a time) and unit ^ row % 8 (the transpose, where somebody reads it).
     T *img = reinterpret_cast<T *>(smem + L::IMG + ti * 16384), *imgT = img + 4096;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
@@ -451,7 +451,7 @@ __device__ __forceinline__ void bwd_dcb_heads_body(const bimamba2_params &p, int
                 v4[i] = from_f<T>(dcb[q][j][i]);
                 img[(t + i) * 64 + (((s >> 3) ^ ((t >> 2) & 7)) << 3) + (s & 7)] = v4[i];
             }
-            *reinterpret_cast<uint2 *>(imgT + s * 64 + (((t >> 3) ^ (s & 7)) << 3) + (t & 7)) = *reinterpret_cast<const uint2 *>(v4);
+            if (p.dCBT) *reinterpret_cast<uint2 *>(imgT + s * 64 + (((t >> 3) ^ (s & 7)) << 3) + (t & 7)) = *reinterpret_cast<const uint2 *>(v4);
         }
     }
     if constexpr (W > 1) __syncthreads();
@@ -462,7 +462,7 @@ __device__ __forceinline__ void bwd_dcb_heads_body(const bimamba2_params &p, int
     for (int k = 0; k < 8 / W; ++k) {
         const int r = (hw * (8 / W) + k) * 8 + (le >> 3), u = le & 7;
         *reinterpret_cast<f32x4 *>(out + r * Q + u * 8) = *reinterpret_cast<const f32x4 *>(img + r * 64 + ((u ^ ((r >> 2) & 7)) << 3));
-        *reinterpret_cast<f32x4 *>(outT + r * Q + u * 8) = *reinterpret_cast<const f32x4 *>(imgT + r * 64 + ((u ^ (r & 7)) << 3));
+        if (p.dCBT) *reinterpret_cast<f32x4 *>(outT + r * Q + u * 8) = *reinterpret_cast<const f32x4 *>(imgT + r * 64 + ((u ^ (r & 7)) << 3));
     }
 }
 

@@ -623,14 +623,14 @@ int choose_dbdc_heads(const bimamba2_params *p, bool by_heads, bool together) {
 // (Counters, 4 x 2048, 32 heads: vector units busy 42 % of the time, matrix units 14 %, LDS 29 % without conflicts, and a third of the waves' time is spent
 // waiting for an instruction: 219 registers leave two waves a SIMD, which do not cover each other.)
 // (dC's workgroups in front)
-template <typename T, int W>
+template <typename T, int W, bool PRODUCT>
 __global__ __launch_bounds__(NTHREADS, 2) void bwd_dbdc_heads_kernel(const bimamba2_params p, int nc, int nqt, int hps, int gdx, int gdy, int gdz) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[DbdcHeadsMap<W>::LDS];
     const int per = gdx * gdy, half = per * gdz, id = blockIdx.x % half;
     BlockId bid = dcb_block_of(id % per, gdx, gdy, per, DCB_HEADS_RESIDENT);
     bid.z = id / per;
-    if ((int)blockIdx.x >= half) bwd_dbdc_heads_body<T, true, W>(p, nc, nqt, hps, bid, smem);
-    else bwd_dbdc_heads_body<T, false, W>(p, nc, nqt, hps, bid, smem);
+    if ((int)blockIdx.x >= half) bwd_dbdc_heads_body<T, true, W, PRODUCT>(p, nc, nqt, hps, bid, smem);
+    else bwd_dbdc_heads_body<T, false, W, PRODUCT>(p, nc, nqt, hps, bid, smem);
 }
 // us: with the chip full (two workgroups on a CU) a wave's head takes 5.6, with one on a CU 3.8, start and end 6.  dC and dB
 // in one launch: 4 x 2048, 32 heads, two slices: 28.7 with four waves to a tile (four heads each), one slice 34.5; with two waves
@@ -656,19 +656,33 @@ bool dbdc_both_by_heads(const bimamba2_params *p) {
     auto al = [](const void *q) { return q && (reinterpret_cast<uintptr_t>(q) & 15) == 0; };
     return dbdc_by_heads(p) && al(p->states16_f) && al(p->states16_b) && al(p->dstates16_f) && al(p->dstates16_b);
 }
-template <typename T, int W> static void launch_dbdc_both_w(const bimamba2_params *p, int nqt, int hps) {
-    const int nc = nchunks(p), gdx = p->batch * nc * p->ngroups, gdy = (nqt * W + 3) / 4, gdz = dbdc_slices(p);
-    hipLaunchKernelGGL((bwd_dbdc_heads_kernel<T, W>), dim3(2 * gdx * gdy * gdz), dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, hps, gdx, gdy, gdz);
+// Where one slice holds all heads of a group, the workgroup that has summed a tile's state parts forms the part inside the chunk too and writes dB and
+// dC themselves: 16 MB of partial sums and 16 MB of dCB's transpose less per 64 (batch, chunk, group), and the last launch is left with the cumulative
+// sums.  Not below 16 (batch, chunk, group), where the last launch ran beside them for nothing and the product is one more chain of
+// waits.  us of the three launches (dCB, dB with dC, the last one), 16 bits, dstate 64, without -> with: 8 (b, c, g): 8 heads 29.1 -> 29.9, 4 heads 26.6 ->
+// 27.7; 16: 3 heads 28.8 -> 29.1, 4 heads 30.7 -> 30.2, 4 heads of 128 33.5 -> 32.2; 32: 8 heads 37.1 -> 36.4; 64 of 8 heads in two groups 47.4 -> 44.4, of 16 in
+// one 89.3 -> 90.1, of 24 130 -> 124; 128 of 4 heads 68 -> 58, of 8 heads 111 -> 98, of 4 heads of 128 104 -> 89; 512 of 4 heads 136 + 71 + 65 -> 131 + 82 + 17
+// (4 x 4096, 32 heads in 8 groups), a training pass there 523 -> 486.
+bool dbdc_with_product(const bimamba2_params *p) {
+    auto in32 = [](int64_t stride) { return stride >= 0 && stride < (1 << 22); };      // (its rows of B and C are 32-bit offsets, as those of x)
+    return dbdc_both_by_heads(p) && bwd_tail_merged(p) && dbdc_slices(p) == 1 && in32(p->B_sl) && in32(p->C_sl) &&
+           (int64_t)p->batch * nchunks(p) * p->ngroups >= 16;
 }
-template <typename T> static int launch_dbdc_both_t(const bimamba2_params *p) {
+template <typename T, int W> static void launch_dbdc_both_w(const bimamba2_params *p, int nqt, int hps, bool product) {
+    const int nc = nchunks(p), gdx = p->batch * nc * p->ngroups, gdy = (nqt * W + 3) / 4, gdz = dbdc_slices(p);
+    const dim3 grid(2 * gdx * gdy * gdz);
+    if (product) hipLaunchKernelGGL((bwd_dbdc_heads_kernel<T, W, true>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, hps, gdx, gdy, gdz);
+    else hipLaunchKernelGGL((bwd_dbdc_heads_kernel<T, W, false>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nqt, hps, gdx, gdy, gdz);
+}
+template <typename T> static int launch_dbdc_both_t(const bimamba2_params *p, bool product) {
     const int nqt = p->chunk_size / 64, hps = dbdc_heads(p), W = dbdc_waves(p, hps);
-    if (W == 4) launch_dbdc_both_w<T, 4>(p, nqt, hps);
-    else if (W == 2) launch_dbdc_both_w<T, 2>(p, nqt, hps);
-    else launch_dbdc_both_w<T, 1>(p, nqt, hps);
+    if (W == 4) launch_dbdc_both_w<T, 4>(p, nqt, hps, product);
+    else if (W == 2) launch_dbdc_both_w<T, 2>(p, nqt, hps, product);
+    else launch_dbdc_both_w<T, 1>(p, nqt, hps, product);
     return check_launch();
 }
-int launch_dbdc_both(const bimamba2_params *p) {
-    return p->dtype == BIMAMBA2_BF16 ? launch_dbdc_both_t<bf16_t>(p) : launch_dbdc_both_t<f16_t>(p);
+int launch_dbdc_both(const bimamba2_params *p, bool product) {
+    return p->dtype == BIMAMBA2_BF16 ? launch_dbdc_both_t<bf16_t>(p, product) : launch_dbdc_both_t<f16_t>(p, product);
 }
 
 // Two waves to a SIMD, said explicitly: with the bound left out the two-tile variant takes 140 us instead of 40 (float32, heads of 16,

@@ -60,7 +60,8 @@ int launch_state_passing_bwd(const bimamba2_params *p);
 int choose_dbdc_heads(const bimamba2_params *p, bool by_heads, bool together);   // heads per slice of the dB / dC partial sums; by_heads: for the next three; together: db_dc_roles()
 bool dbdc_by_heads(const bimamba2_params *p);       // dB and dC by waves that take whole heads, given 16-bit copies of the states
 bool dbdc_both_by_heads(const bimamba2_params *p);  // with them given
-int launch_dbdc_both(const bimamba2_params *p);     // both in one launch
+bool dbdc_with_product(const bimamba2_params *p);   // and one slice of heads, chunks of 256: with dCB in 16 bits it can write dB and dC themselves
+int launch_dbdc_both(const bimamba2_params *p, bool product);     // both in one launch
 int launch_bwd_dbdc(const bimamba2_params *p, bool is_db);
 int launch_bwd_dcb(const bimamba2_params *p, bool add_up = true);   // add_up: also the launch that adds several head slices up
 int choose_dcb_slices(const bimamba2_params *p);
