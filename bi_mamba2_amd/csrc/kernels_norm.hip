@@ -37,6 +37,23 @@ template <typename T> __device__ __forceinline__ void load8(const T *ptr, bool v
         for (int i = 0; i < 8; ++i) v[i] = i < ncol ? to_f(ptr[i]) : 0.f;
     }
 }
+// the same as they lie in memory: nothing waits for them before they are used
+template <typename T> __device__ __forceinline__ void load8_raw(const T *ptr, bool vec, int ncol, T (&v)[8]) {
+    if (vec && ncol >= 8) {
+        if constexpr (sizeof(T) == 2) {
+            const Vec16<T> raw = *reinterpret_cast<const Vec16<T> *>(ptr);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = raw.v[i];
+        } else {
+            const f32x4 a = *reinterpret_cast<const f32x4 *>(ptr), b = *reinterpret_cast<const f32x4 *>(ptr + 4);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) { v[i] = a[i]; v[i + 4] = b[i]; }
+        }
+    } else {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = i < ncol ? ptr[i] : from_f<T>(0.f);
+    }
+}
 template <typename T> __device__ __forceinline__ void store8(T *ptr, bool vec, int ncol, const float (&v)[8]) {
     if (vec && ncol >= 8) {
         if constexpr (sizeof(T) == 2) {
@@ -71,28 +88,31 @@ __global__ __launch_bounds__(NTHREADS) void rmsnorm_gated_fwd_kernel(const bimam
     T *out = reinterpret_cast<T *>(p.out) + row * p.out_rs + g * gs;
     const float *w = p.weight + g * gs, *bias = p.has_bias ? p.bias + g * gs : nullptr;
     const bool gate_first = p.has_z && !p.norm_before_gate;
-    // both operands are requested before anything is reduced; z is kept as loaded between the passes
+    // Everything is requested before anything is used; z is kept as loaded between the passes.  (A gate applied piece by piece waited for each piece
+    // of z before the next was asked for: 16384 rows of 1536 columns, bfloat16, 36.2 us, as here 29.5, 151 MB at 5.1 TB/s.)
     float xv[NCH][8];
-    T zk[NCH][8];
+    T xk[NCH][8], zk[NCH][8];
     float ss = 0.f;
 #pragma unroll
-    for (int k = 0; k < NCH; ++k) {
-        const int c = (k * 64 + lane) * 8;
-        load8(x + c, vec, FULL ? 8 : gs - c, xv[k]);
-        if (p.has_z) {
-            float zv[8];
-            load8(z + c, vec, FULL ? 8 : gs - c, zv);
+    for (int k = 0; k < NCH; ++k) load8_raw(x + (k * 64 + lane) * 8, vec, FULL ? 8 : gs - (k * 64 + lane) * 8, xk[k]);
+    if (p.has_z) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                if (gate_first) xv[k][i] *= silu_f(zv[i]);
-                else zk[k][i] = from_f<T>(zv[i]);      // exact: zv came from a T
-            }
-        }
+        for (int k = 0; k < NCH; ++k) load8_raw(z + (k * 64 + lane) * 8, vec, FULL ? 8 : gs - (k * 64 + lane) * 8, zk[k]);
     }
     float wk[FULL ? NCH : 1][8];
     if (FULL) {
 #pragma unroll
         for (int k = 0; k < NCH; ++k) load8(w + (k * 64 + lane) * 8, true, 8, wk[FULL ? k : 0]);
+    }
+#pragma unroll
+    for (int k = 0; k < NCH; ++k)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) xv[k][i] = to_f(xk[k][i]);
+    if (gate_first) {
+#pragma unroll
+        for (int k = 0; k < NCH; ++k)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) xv[k][i] *= silu_f(to_f(zk[k][i]));
     }
     if (p.layer_norm) {
         float sm = 0.f;
