@@ -25,7 +25,7 @@ template <int W> struct DbdcHeadsMap {
 // chunks of 256 and dCB in 16 bits, of which no transpose is needed: dC reads its tiles as they lie, dB by transpose reads.  The
 // chunk's C (B) rows lie in the second halves of the four rings, 64 rows in each, for all waves; the 64 x 64 pieces of dCB in the first
 // halves, W of a tile's four at a time, with one wave to a tile asked for under the last head and under the products.  Bound by
-// memory with one wave to a tile (4 x 4096, 32 heads in 8 groups: 82 us, 71 without the product; 450 MB), by its waits else (16 x 1024, 24 heads: 41.5, 38.6 without).
+// memory with one wave to a tile (4 x 4096, 32 heads in 8 groups: 81 us, 71 without the product; 405 MB), by its waits else (16 x 1024, 24 heads: 40.9, 39.5 without).
 // bid.x: (batch, chunk, group), bid.y: row tiles, bid.z: slice of hps heads
 template <typename T, bool IS_DB, int W, bool PRODUCT>
 __device__ __forceinline__ void bwd_dbdc_heads_body(const bimamba2_params &p, int nc, int nqt, int hps, BlockId bid, unsigned char *smem) {

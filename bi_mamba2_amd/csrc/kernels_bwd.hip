@@ -622,14 +622,22 @@ int choose_dbdc_heads(const bimamba2_params *p, bool by_heads, bool together) {
 // 32 additions of a state's product into the lane's sums and 32 into the rows' per 16 matrix instructions of 8 cycles.
 // (Counters, 4 x 2048, 32 heads: vector units busy 42 % of the time, matrix units 14 %, LDS 29 % without conflicts, and a third of the waves' time is spent
 // waiting for an instruction: 219 registers leave two waves a SIMD, which do not cover each other.)
-// (dC's workgroups in front)
+// (dC's workgroups in front, unless they form the product)
 template <typename T, int W, bool PRODUCT>
 __global__ __launch_bounds__(NTHREADS, 2) void bwd_dbdc_heads_kernel(const bimamba2_params p, int nc, int nqt, int hps, int gdx, int gdy, int gdz) {
     __shared__ __attribute__((aligned(16))) unsigned char smem[DbdcHeadsMap<W>::LDS];
-    const int per = gdx * gdy, half = per * gdz, id = blockIdx.x % half;
+    const int per = gdx * gdy, half = per * gdz, lin = blockIdx.x;
+    int id = lin % half;
+    bool is_db = lin >= half;
+    // With the product both roles read the (batch, chunk, group)'s dCB and its B and C rows: eight dC workgroups, one per XCD, then the eight of dB beside
+    // them.  4 x 4096, 32 heads in 8 groups: 414 -> 363 MB read, 82 -> 81 us; 16 x 1024, 24 heads 44.6 -> 40.9; 16 heads 31.2 -> 29.5.
+    if (PRODUCT && half % 8 == 0) {
+        is_db = (lin >> 3) & 1;
+        id = (lin >> 4) * 8 + (lin & 7);
+    }
     BlockId bid = dcb_block_of(id % per, gdx, gdy, per, DCB_HEADS_RESIDENT);
     bid.z = id / per;
-    if ((int)blockIdx.x >= half) bwd_dbdc_heads_body<T, true, W, PRODUCT>(p, nc, nqt, hps, bid, smem);
+    if (is_db) bwd_dbdc_heads_body<T, true, W, PRODUCT>(p, nc, nqt, hps, bid, smem);
     else bwd_dbdc_heads_body<T, false, W, PRODUCT>(p, nc, nqt, hps, bid, smem);
 }
 // us: with the chip full (two workgroups on a CU) a wave's head takes 5.6, with one on a CU 3.8, start and end 6.  dC and dB
@@ -661,8 +669,8 @@ bool dbdc_both_by_heads(const bimamba2_params *p) {
 // sums.  Not below 16 (batch, chunk, group), where the last launch ran beside them for nothing and the product is one more chain of
 // waits.  us of the three launches (dCB, dB with dC, the last one), 16 bits, dstate 64, without -> with: 8 (b, c, g): 8 heads 29.1 -> 29.9, 4 heads 26.6 ->
 // 27.7; 16: 3 heads 28.8 -> 29.1, 4 heads 30.7 -> 30.2, 4 heads of 128 33.5 -> 32.2; 32: 8 heads 37.1 -> 36.4; 64 of 8 heads in two groups 47.4 -> 44.4, of 16 in
-// one 89.3 -> 90.1, of 24 130 -> 124; 128 of 4 heads 68 -> 58, of 8 heads 111 -> 98, of 4 heads of 128 104 -> 89; 512 of 4 heads 136 + 71 + 65 -> 131 + 82 + 17
-// (4 x 4096, 32 heads in 8 groups), a training pass there 523 -> 486.
+// one 89.3 -> 90.1, of 24 130 -> 124; 128 of 4 heads 68 -> 58, of 8 heads 111 -> 98, of 4 heads of 128 104 -> 89; 512 of 4 heads 136 + 71 + 65 -> 131 + 81 + 15
+// (4 x 4096, 32 heads in 8 groups), a training pass there 526 -> 485.
 bool dbdc_with_product(const bimamba2_params *p) {
     auto in32 = [](int64_t stride) { return stride >= 0 && stride < (1 << 22); };      // (its rows of B and C are 32-bit offsets, as those of x)
     return dbdc_both_by_heads(p) && bwd_tail_merged(p) && dbdc_slices(p) == 1 && in32(p->B_sl) && in32(p->C_sl) &&
