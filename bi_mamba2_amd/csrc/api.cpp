@@ -270,6 +270,8 @@ int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd) {
     return chunk_scan_uses_scan16(p, bwd != 0) ? chunk_scan16_heads_per_workgroup(p) : 1;
 }
 
+int bimamba2_fwd_one_launch(const bimamba2_params *p) { return check_problem(p) || !scan_once_applies(p) ? 0 : scan_once_walks(p) ? 2 : 1; }
+
 // A chunk costs its pairs of positions (they grow with the chunk) and its states (which do not); small calls want many workgroups, i.e. small
 // chunks.  The lines follow the length, the heads and the operands of a row but not the number of rows, so that a row's result is the same
 // alone and in any batch; where they lie is therefore between what one row and what many rows want.  us a pass with chunks of 64 / 128 / 256

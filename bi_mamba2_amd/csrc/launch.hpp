@@ -40,6 +40,7 @@ int launch_state_passing_fwd(const bimamba2_params *p);
 int launch_chunk_scan(const bimamba2_params *p, bool bwd, bool free16 = false);
 // a forward pass over a short sequence in one launch (kernels_scan_once.hip), and where it is the one to run
 bool scan_once_applies(const bimamba2_params *p);
+bool scan_once_walks(const bimamba2_params *p);       // ... by workgroups that own whole sequences
 int launch_scan_once(const bimamba2_params *p);
 // the 16-bit kernel of kernels_scan16.hip (launch_chunk_scan picks it where it applies)
 int launch_chunk_scan16(const bimamba2_params *p, bool bwd);

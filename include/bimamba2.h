@@ -223,6 +223,10 @@ int bimamba2_ddt_direct_planes(const bimamba2_params *p);
  * src/ssd/bi/ssd_bmm.py:163-208). */
 int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd);
 
+/* Whether bimamba2_fwd forms `out` of this problem in one launch: 0 no, 1 yes, by workgroups that own 64 (float32: 32) positions, 2 yes, by
+ * workgroups that own whole sequences (the same result in bits).  Pointers that are not set yet count as aligned.  A measurement aid. */
+int bimamba2_fwd_one_launch(const bimamba2_params *p);
+
 /* Whole forward; replaces _mamba_chunk_scan_combined_fwd (src/ssd/bi/ssd_combined.py:297-331).
  * Needs: x dt A Bm Cm [D z dt_bias] out [out_x when has_z] [final_f final_b] workspace.  Intermediates given as
  * non-NULL pointers (dt_out cs_f cs_b CB CBT states_f states_b) are filled in place of workspace memory, so a

@@ -403,3 +403,21 @@ def test_chunks_of_wide_heads_grow_only_where_their_kernels_run(heads, headdim, 
         assert chosen(**odd) == 128, odd
     assert chosen(z=258) == 128 and chosen(z_sl=heads * headdim + 2) == 128 and chosen(B_sl=1 << 22) == 128
 
+
+
+# one row's workgroups of 64 (float32: 32) positions at the line up to which short sequences go in one launch
+ONE_LAUNCH = [(_lib.BF16, 256, 12, 64, 64), (_lib.BF16, 197, 12, 64, 64), (_lib.F16, 256, 8, 64, 128), (_lib.BF16, 256, 12, 64, 32), (_lib.BF16, 64, 48, 64, 64),
+              (_lib.BF16, 128, 24, 64, 64), (_lib.F32, 256, 16, 32, 16), (_lib.F32, 256, 10, 32, 32), (_lib.F32, 192, 4, 64, 64), (_lib.F32, 64, 24, 32, 16),
+              (_lib.F32, 64, 6, 64, 64)]
+
+
+@pytest.mark.parametrize("dtype,seqlen,heads,headdim,dstate", ONE_LAUNCH)
+def test_short_sequences_in_any_batch(dtype, seqlen, heads, headdim, dstate):
+    """few rows are cut into workgroups of some positions, many are not: there each would fetch the whole sequence and form C.B^T again (64 x 256
+    positions, 8 heads, dstate 128: 59 us where the chunked launches take 30).  Whether it is one launch does not follow the rows."""
+    lib = _lib.load()
+    form = lambda batch, heads=heads, **kw: lib.bimamba2_fwd_one_launch(ctypes.byref(
+        _params(batch=batch, seqlen=seqlen, nheads=heads, headdim=headdim, ngroups=1, dstate=dstate, chunk_size=64, dtype=dtype, **kw)))
+    assert [form(b) for b in (1, 2, 64, 256, 2200000)] == [1, 1, 2, 2, 2] if seqlen > 128 else [2] * 5
+    assert form(1, heads + 1) == form(64, heads + 1) == 0
+    assert form(64, causal=1) == form(64, initial_f=256) == form(64, states_f=256) == 0
