@@ -508,7 +508,11 @@ int bimamba2_fwd(const bimamba2_params *p) {
         if (p->has_z) REQUIRE(p->z);
         if (q.final_f || q.final_b) {
             // (the result of such a call is the same in bits whether or not the final states are asked for)
-            TRY(forward_cumsum_and_states(&q));
+            if (fwd_front_merged(&q)) {
+                bimamba2_params qs = q;
+                qs.CB = nullptr;      // (nobody reads it; float32, 1 x 256 positions, 4 heads of 32, us a call: chunked launches 17.1, cumsum and states apart 17.7, so 16.0)
+                TRY(launch_fwd_front(&qs));
+            } else TRY(forward_cumsum_and_states(&q));
             TRY(bimamba2_state_passing_fwd(&q));
         }
         return launch_scan_once(p);

@@ -1056,7 +1056,7 @@ bool fwd_front_merged(const bimamba2_params *p) {
 template <typename T> static int launch_fwd_front_t(const bimamba2_params *p, bool fast) {
     const int nc = nchunks(p), nqt = (p->chunk_size + 63) / 64, nnt = (p->dstate + 63) / 64, npt = (p->headdim + 63) / 64;
     const int nstate = nnt * npt * p->batch * nc * p->nheads;
-    const dim3 grid(nstate + nqt * nqt * p->batch * nc * p->ngroups);
+    const dim3 grid(nstate + (p->CB ? nqt * nqt * p->batch * nc * p->ngroups : 0));
     if constexpr (sizeof(T) == 2) {
         if (chunk_state_does_cumsum(p)) {
             hipLaunchKernelGGL((chunk_state_direct_cb_kernel<T>), grid, dim3(NTHREADS), 0, stream_of(p), *p, nc, nnt, npt, nstate, nqt);

@@ -563,8 +563,8 @@ bool scan_once_applies(const bimamba2_params *p) {
     //     1.48, 2.1; dstate 16: 128 (256, 16 heads) 2.6, 1.54, 1.60, 1.74; 48 (64, 24 heads) 2.0, 1.88, 1.64, 1.66
     // Below 1 are 16 bits over more than 128 positions at dstate 64 from some 200 rows on, where the chunked launches move two entries an instruction: the price of
     // the same bits in any batch.  Final states besides (the launches that form them stay, and the one launch takes the place of their scan only): bfloat16, 197
-    // positions, 12 heads 1.36, 1.12, 1.00, 0.97; float32 in one chunk, 64 positions, 6 heads 1.04, 1.01, 1.12, 1.31, in several chunks, where the
-    // chunked scan takes a quarter of the pairs, 256 positions, 4 heads of 32, dstate 16 0.96, 0.78, 0.87, 1.00, and 192 positions, 4 heads, dstate 64 0.91, 0.69, 0.88, 1.07: the
+    // positions, 12 heads 1.36, 1.12, 1.00, 0.97; float32 in one chunk, 64 positions, 6 heads 1.15, 1.16, 1.20, 1.38, in several chunks, where the
+    // chunked scan takes a quarter of the pairs, 256 positions, 4 heads of 32, dstate 16 1.07, 0.86, 0.92, 0.95, and 192 positions, 4 heads, dstate 64 0.99, 0.75, 0.89, 1.04: the
     // price of a result that is the same in bits whether or not they are asked for.
     const int per_row = p->nheads * once_tiles(p);
     if (e == 2) return per_row <= (ns == 4 ? 32 : 48);

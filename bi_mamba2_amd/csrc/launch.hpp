@@ -28,7 +28,7 @@ int launch_fwd_cumsum_cb(const bimamba2_params *p, bool states16);     // chunk 
 int launch_chunk_state(const bimamba2_params *p, bool dstates, bool cumsum = false);   // cumsum: also does the chunk cumsum
 bool chunk_state_does_cumsum(const bimamba2_params *p);
 bool chunk_state_narrow(const bimamba2_params *p, bool dstates);
-// chunk cumsum, chunk states and C.B^T as one launch, where fwd_front_merged() says it exists
+// chunk cumsum, chunk states and C.B^T (left out where CB is NULL) as one launch, where fwd_front_merged() says it exists
 bool fwd_front_merged(const bimamba2_params *p);
 int launch_fwd_front(const bimamba2_params *p);
 // the forward pass may keep its per-chunk states in states16_f/b only (16-bit type, no float32 state tensors)

@@ -122,6 +122,20 @@ def test_final_states_besides(dtype, H, P, G, N, L):
         assert torch.equal(a, b)
 
 
+def test_final_states_take_no_launch_more_than_the_chunked_pass():
+    """float32, chunks of 64: sums, states and their passing are two launches, as where the scan is the chunked one"""
+    t = {k: v.cuda() for k, v in O.make_inputs(2, 256, 4, 32, 1, 16, seed=9, with_z=False).items()}
+    call(t, 64, final=True)
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA, torch.profiler.ProfilerActivity.CPU]) as prof:
+        call(t, 64, final=True)
+        torch.cuda.synchronize()
+    names = [e.name for e in prof.events() if e.device_type == torch.autograd.DeviceType.CUDA and "bm2::" in e.name]
+    if not names:
+        pytest.skip("no kernels in the profiler's record")
+    assert len(names) == 3 and sum("scan_once" in n for n in names) == 1, names
+
+
 # rows from which on the workgroups own whole sequences and walk through several heads (up to 64, 128, 256 positions)
 ROWS = {64: 700, 128: 300, 256: 110}
 WALK_SHAPES = [(torch.float32, 5, 32, 1, 16), (torch.float32, 4, 48, 2, 32), (torch.float32, 3, 64, 1, 64),
