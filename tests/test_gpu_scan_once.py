@@ -124,7 +124,7 @@ def test_final_states_besides(dtype, H, P, G, N, L):
 
 def test_final_states_take_no_launch_more_than_the_chunked_pass():
     """float32, chunks of 64: sums, states and their passing are two launches, as where the scan is the chunked one"""
-    t = {k: v.cuda() for k, v in O.make_inputs(2, 256, 4, 32, 1, 16, seed=9, with_z=False).items()}
+    t = {k: v.cuda() for k, v in O.make_inputs(2, 256, 4, 32, 1, 16, seed=9, with_z=True).items()}
     call(t, 64, final=True)
     torch.cuda.synchronize()
     with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA, torch.profiler.ProfilerActivity.CPU]) as prof:
