@@ -201,6 +201,13 @@ template <bool RAW = true> __device__ __forceinline__ void raw_lds_barrier() {
     if constexpr (RAW) __builtin_amdgcn_s_barrier();
     else __syncthreads();
 }
+// The same between LDS accesses that the compiler knows of: settled in front of it, and none moved across it (the bare barrier orders nothing for the compiler).
+// Not __syncthreads(), which would wait for the loads from memory as well.
+__device__ __forceinline__ void ordered_lds_barrier() {
+    raw_lds_wait();
+    raw_lds_barrier();
+    asm volatile("" ::: "memory");
+}
 template <bool RAW = true, typename V> __device__ __forceinline__ void raw_lds_use(V &v) {
     if constexpr (RAW) asm volatile("" : "+v"(v));
 }

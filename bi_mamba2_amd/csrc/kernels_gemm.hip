@@ -102,7 +102,7 @@ __device__ __forceinline__ void store_tile(const bimamba2_gemm_params &p, f32x4 
         constexpr int MG = WAVES * MT * 16 * PITCH <= LDS_B ? MT : MT / 2;      // row tiles at a time
         static_assert(WAVES * MG * 16 * PITCH <= LDS_B && MG * 16 * RCH % 64 == 0, "staging of the result");
         unsigned char *mine = smem + wave * (MG * 16 * PITCH);
-        raw_lds_barrier();                                    // (the fragments that others read lie there)
+        ordered_lds_barrier();                                // (the fragments that others read lie there)
         static_for<0, MT / MG>([&](auto GI) __attribute__((always_inline)) {
             constexpr int g = decltype(GI)::value;
 #pragma unroll

@@ -72,12 +72,6 @@ __device__ __forceinline__ void once_decays(double step, double incl, const doub
     gf[q] = __expf(-f) * v; gb[q] = __expf(-r) * v;
     dts[q] = v;
 }
-// workgroup barrier behind LDS accesses of any kind (not __syncthreads(), which would wait for the loads from memory as well)
-__device__ __forceinline__ void once_barrier() {
-    raw_lds_wait();
-    raw_lds_barrier();
-    asm volatile("" ::: "memory");
-}
 
 }  // namespace
 
@@ -149,7 +143,7 @@ __global__ __launch_bounds__(ONCE_THREADS) void scan_once_kernel(const bimamba2_
         incl = wave_incl_prefix_dpp(step);
         if (lane == 63) totals[wave] = incl;
     }
-    once_barrier();
+    ordered_lds_barrier();
     if (wave < 4) once_decays(step, incl, totals, wave, lane, q, v, gf, gb, lf, lb, dts, sf, sb);
 #pragma unroll
     for (int i = 0; i < BI; ++i) {
@@ -367,7 +361,7 @@ __global__ __launch_bounds__((WalkMap<T, NS, LP>::THREADS), LP == 256 ? 2 : 4) v
             if (id < LP * BC) *reinterpret_cast<u32x4 *>(bs + r * BP + c * VS) = r < L ? br[i] : zero;
         }
         store_x(0);
-        once_barrier();
+        ordered_lds_barrier();
         form_tables(0);
         if (nh > 1) request(h0 + 1);
 #pragma unroll
@@ -387,7 +381,7 @@ __global__ __launch_bounds__((WalkMap<T, NS, LP>::THREADS), LP == 256 ? 2 : 4) v
                     for (int j = 0; j < 4; ++j) cb[t][n][4 * hh + j] = d[j];
                 }
             }
-        once_barrier();                                       // (x of the next head lies where the B rows did)
+        ordered_lds_barrier();                                       // (x of the next head lies where the B rows did)
     }
 
     // ---- the heads ----
@@ -525,11 +519,11 @@ __global__ __launch_bounds__((WalkMap<T, NS, LP>::THREADS), LP == 256 ? 2 : 4) v
                 if (orow < L && p0 + column(k) < P) *reinterpret_cast<Vec16<T> *>(out + column(k)) = o[k];
             if (more) {
                 if (rt == 0) {
-                    once_barrier();
+                    ordered_lds_barrier();
                     form_tables(cur ^ 1);
                     if (hi + 2 < nh) request(h + 2);
                 }
-                if (rt == NRT - 1) once_barrier();
+                if (rt == NRT - 1) ordered_lds_barrier();
             }
         });
     }

@@ -421,3 +421,13 @@ def test_short_sequences_in_any_batch(dtype, seqlen, heads, headdim, dstate):
     assert [form(b) for b in (1, 2, 64, 256, 2200000)] == [1, 1, 2, 2, 2] if seqlen > 128 else [2] * 5
     assert form(1, heads + 1) == form(64, heads + 1) == 0
     assert form(64, causal=1) == form(64, initial_f=256) == form(64, states_f=256) == 0
+
+
+@pytest.mark.parametrize("name,function", [("kernels_gemm.hip", "store_tile"), ("kernels_scan_once.hip", "scan_once_kernel"), ("kernels_scan_once.hip", "scan_once_walk_kernel")])
+def test_no_bare_barrier_in_front_of_ordinary_lds_accesses(name, function):
+    """these write LDS by stores that the compiler knows of, where other waves read before: s_barrier alone does not keep it from moving them up"""
+    text = open(os.path.join(ROOT, "bi_mamba2_amd", "csrc", name)).read()
+    body = text[text.index(f" {function}("):]
+    body = body[:body.index("\n}\n")]
+    assert "ordered_lds_barrier()" in body or "__syncthreads()" in body
+    assert not re.search(r"raw_lds_barrier|amdgcn_s_barrier", body)
