@@ -54,7 +54,7 @@ ALL_SYMBOLS = ENTRY_POINTS + ("bimamba2_strerror", "bimamba2_version", "bimamba2
                               "bimamba2_chunk_scan_heads_per_workgroup", "bimamba2_fwd_one_launch", "bimamba2_ddt_direct_planes", "bimamba2_norm_params_size",
                               "bimamba2_rmsnorm_gated_workspace_bytes", "bimamba2_conv_params_size",
                               "bimamba2_conv1d_silu_workspace_bytes", "bimamba2_cast_params_size",
-                              "bimamba2_cast_many", "bimamba2_norm_scan_conv_bwd", "bimamba2_gemm_params_size", "bimamba2_gemm_workspace_bytes", "bimamba2_gemm") + NORM_ENTRY_POINTS + CONV_ENTRY_POINTS
+                              "bimamba2_cast_many", "bimamba2_norm_scan_conv_bwd", "bimamba2_gemm_params_size", "bimamba2_gemm_workspace_bytes", "bimamba2_gemm_plan", "bimamba2_gemm") + NORM_ENTRY_POINTS + CONV_ENTRY_POINTS
 
 _lib = None
 
@@ -162,6 +162,8 @@ def load():
         raise RuntimeError("bimamba2_gemm_params layout mismatch between the library and its Python mirror")
     lib.bimamba2_gemm_workspace_bytes.argtypes = [ctypes.POINTER(GemmParams)]
     lib.bimamba2_gemm_workspace_bytes.restype = ctypes.c_size_t
+    lib.bimamba2_gemm_plan.argtypes = [ctypes.POINTER(GemmParams), ctypes.POINTER(ctypes.c_int)]
+    lib.bimamba2_gemm_plan.restype = ctypes.c_int
     lib.bimamba2_gemm.argtypes = [ctypes.POINTER(GemmParams)]
     lib.bimamba2_gemm.restype = ctypes.c_int
     lib.bimamba2_cast_many.argtypes = [ctypes.POINTER(CastParams)]

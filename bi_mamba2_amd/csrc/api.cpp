@@ -838,6 +838,13 @@ static int check_gemm(const bimamba2_gemm_params *p) {
     return BIMAMBA2_OK;
 }
 
+int bimamba2_gemm_plan(const bimamba2_gemm_params *p, int *slices) {
+    if (!p || !slices || p->m <= 0 || p->n <= 0 || p->k <= 0) return BIMAMBA2_EINVAL;
+    int tile;
+    gemm_plan_of(p, &tile, slices);
+    return tile;
+}
+
 size_t bimamba2_gemm_workspace_bytes(const bimamba2_gemm_params *p) { return check_gemm(p) ? 0 : gemm_workspace_bytes(p); }
 
 int bimamba2_gemm(const bimamba2_gemm_params *p) {

@@ -620,11 +620,15 @@ struct GemmTileCost {
     double start_us, fixed_us, each_us;     // a round of workgroups: start and end, and per step fixed + each * (tiles that share the CU)
     double kcontig;                         // factor of a step where k is contiguous in an operand
     double slices_us;                       // the launch that adds the k slices up
+    double crowd;                           // what c tiles that share a CU cost each other beyond that: factor 1 + crowd c (c - 1) of a step
 };
 // fitted to 360 products of layers of 128 to 1024 columns over 72 to 65536 rows with operands from memory, every tile and number of slices
-// each: the plan chosen takes 1.012 of the best one's time in the geometric mean, 1.10 at worst
-constexpr GemmTileCost GEMM_TILES[4] = {{256, 256, 1, 3.1, 0.50, 0.12, 1.2, 8.5}, {256, 192, 1, 3.0, 0.40, 0.106, 1.4, 6.6},
-                                        {128, 128, 2, 3.0, 0.22, 0.11, 1.4, 6.6}, {64, 64, 4, 3.4, 0.12, 0.08, 1.3, 3.5}};
+// each.  Held against another 598 of layers of 128 to 4096 columns (weight gradients, and the input gradients and forward products that come here): the plan chosen
+// takes 1.006 of the best one's time in the geometric mean, 1.08 at the 98th percentile, 1.21 at worst.  Against the plan with 128 x 128 tiles as the largest, 400
+// weight gradients 0.85 (0.47 to 1.12, seven above 1.03: few columns over long sums, and 3000 rows where two slices more pay).  Without the crowd 64 x 64 tiles were
+// taken for more of those: 1546 x 320 over 9110 rows 34.3 -> 29.3 us, 1286 x 192 over 19392 40.6 -> 36.1 (33.0 in eleven slices of 128 x 128).
+constexpr GemmTileCost GEMM_TILES[4] = {{256, 256, 1, 3.1, 0.50, 0.12, 1.2, 8.5, 0.}, {256, 192, 1, 3.0, 0.40, 0.106, 1.4, 6.6, 0.},
+                                        {128, 128, 2, 3.0, 0.22, 0.11, 1.4, 6.6, 0.}, {64, 64, 4, 3.3, 0.12, 0.08, 1.3, 3.5, 0.025}};
 
 // Tile and number of k slices by the estimated time: per round of workgroups its start and end and its steps at the round's
 // occupancy; for k slices the partial tiles that are written and read again (5 TB/s) and the launch that adds them.  us, with 128 x 128 tiles as
@@ -642,7 +646,10 @@ GemmPlan gemm_plan(const bimamba2_gemm_params *p) {
             const int64_t per = (steps + s - 1) / s;
             if (s > 1 && (per < 8 || (steps + per - 1) / per != s)) continue;
             const int64_t full = tiles * s / slots, rest = tiles * s % slots;
-            auto round = [&](int64_t wgs) { return c.start_us + per * slow * (c.fixed_us + c.each_us * ((wgs + 255) / 256)); };
+            auto round = [&](int64_t wgs) {
+                const int64_t share = (wgs + 255) / 256;
+                return c.start_us + per * slow * (c.fixed_us + c.each_us * share) * (1. + c.crowd * (share * (share - 1)));
+            };
             double cost = full * round(slots) + (rest ? round(rest) : 0.0);
             if (s > 1) cost += c.slices_us + (double)m * n * 8 * s / 5e6;
             if (cost < best_cost) { best_cost = cost; best = GemmPlan{t, s, (int)(per * 32)}; }
@@ -686,6 +693,12 @@ template <typename T> int launch_gemm_t(const bimamba2_gemm_params *p) {
 }
 
 }  // namespace
+
+void gemm_plan_of(const bimamba2_gemm_params *p, int *tile, int *slices) {
+    const GemmPlan g = gemm_plan(p);
+    *tile = g.tile;
+    *slices = g.nsplit;
+}
 
 size_t gemm_workspace_bytes(const bimamba2_gemm_params *p) {
     const GemmPlan g = gemm_plan(p);

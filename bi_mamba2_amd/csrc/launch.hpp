@@ -128,5 +128,6 @@ int launch_cast_many(const bimamba2_cast_params *p);
 // matrix products of the layer's projections (kernels_gemm.hip)
 int launch_gemm(const bimamba2_gemm_params *p);
 size_t gemm_workspace_bytes(const bimamba2_gemm_params *p);
+void gemm_plan_of(const bimamba2_gemm_params *p, int *tile, int *slices);     // tile 0: 256 x 256, 1: 256 x 192, 2: 128 x 128, 3: 64 x 64
 
 }  // namespace bm2

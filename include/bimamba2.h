@@ -438,6 +438,9 @@ typedef struct bimamba2_gemm_params {
 } bimamba2_gemm_params;
 size_t bimamba2_gemm_params_size(void);
 size_t bimamba2_gemm_workspace_bytes(const bimamba2_gemm_params *p);
+/* How the product of these sizes (m n k a_kcontig, the rest is not looked at) is cut: returns the output tile - 0: 256 x 256, 1: 256 x 192, 2: 128 x 128,
+ * 3: 64 x 64 - and sets *slices to the number of pieces of the sum. */
+int bimamba2_gemm_plan(const bimamba2_gemm_params *p, int *slices);
 int bimamba2_gemm(const bimamba2_gemm_params *p);
 
 #ifdef __cplusplus

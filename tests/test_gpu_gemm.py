@@ -17,6 +17,13 @@ def rows_of(rows, cols, pad, dtype, gen):
     return t[:, :cols]
 
 
+def plan(m, n, k, a_kc):
+    """the tile (0: 256 x 256, 1: 256 x 192, 2: 128 x 128, 3: 64 x 64) and the slices of the sum"""
+    p, slices = _lib.GemmParams(), ctypes.c_int()
+    p.m, p.n, p.k, p.a_kcontig = m, n, k, a_kc
+    return _lib.load().bimamba2_gemm_plan(ctypes.byref(p), ctypes.byref(slices)), slices.value
+
+
 # one element; a whole 64 tile and one more than it; ragged k below, at and above one and four steps; many k slices with a
 # ragged last one; 128 and 256 tiles with remainders; few columns (the rest of a library product)
 @pytest.mark.parametrize("m,n,k", [(1, 1, 8), (64, 64, 32), (65, 70, 40), (197, 1688, 384), (300, 100, 33), (257, 259, 1000),
@@ -55,10 +62,13 @@ def test_product(m, n, k, a_kc, b_kc, dtype):
 @pytest.mark.parametrize("m,n,k", [(11016, 649, 40), (13379, 514, 72), (13816, 543, 104), (13374, 522, 128), (7406, 1064, 168), (13854, 513, 200),
                                    (12357, 643, 232), (11150, 641, 264),
                                    (6402, 1775, 24), (5960, 1935, 72), (4621, 2537, 104), (6675, 1750, 136), (8281, 1347, 168), (5897, 1937, 192),
-                                   (7246, 1555, 232), (4865, 2324, 264), (700, 1500, 16381), (1700, 2100, 9001), (3224, 768, 4100)])
+                                   (7246, 1555, 232), (4865, 2324, 264), (700, 1500, 16381), (1700, 2100, 9001), (3224, 768, 16373)])
 @pytest.mark.parametrize("a_kc,b_kc", [(1, 1), (1, 0), (0, 0)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_product_large_tiles(m, n, k, a_kc, b_kc, dtype):
+    tile, slices = plan(m, n, (k + 7) // 8 * 8 if b_kc else k, a_kc)
+    assert tile in (0, 1) if k > 9000 else tile == (n < 1100), tile
+    assert (slices > 1) == (k > 9000)
     test_product(m, n, k, a_kc, b_kc, dtype)
 
 
@@ -77,6 +87,7 @@ def test_large_tiles_infinities_behind_the_end(a_kc, b_kc):
     p.m, p.n, p.k, p.a_kcontig, p.b_kcontig, p.dtype = m, n, k, a_kc, b_kc, _lib.BF16
     p.lda, p.ldb, p.ldc = a.stride(0), b.stride(0), c.stride(0)
     p.a, p.b, p.c, p.stream = a.data_ptr(), b.data_ptr(), c.data_ptr(), torch.cuda.current_stream().cuda_stream
+    assert plan(m, n, k, a_kc) == (0, 1)
     assert lib.bimamba2_gemm_workspace_bytes(ctypes.byref(p)) == 0 and lib.bimamba2_gemm(ctypes.byref(p)) == 0
     af, bf = (a[:, :k].float() if a_kc else a[:k, :m].float().t()), (b[:, :k].float().t() if b_kc else b[:k, :n].float())
     assert torch.equal(c[:, :n], (af @ bf).bfloat16())

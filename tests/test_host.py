@@ -405,6 +405,18 @@ def test_chunks_of_wide_heads_grow_only_where_their_kernels_run(heads, headdim, 
 
 
 
+def gemm_plan(m, n, k, a_kcontig):
+    p, slices = _lib.GemmParams(), ctypes.c_int()
+    p.m, p.n, p.k, p.a_kcontig = m, n, k, a_kcontig
+    return _lib.load().bimamba2_gemm_plan(ctypes.byref(p), ctypes.byref(slices)), slices.value
+
+
+# 64 x 64 tiles that share a CU cost each other: the first two took 34 and 30 us in them, 29 and 28 in 128 x 128, the third 4.9 in 128 x 128
+@pytest.mark.parametrize("m,n,k,tile", [(1546, 320, 9110, 2), (1546, 320, 7808, 2), (1288, 256, 84, 3), (320, 640, 1300, 3), (3224, 768, 16384, 0), (768, 1536, 16384, 1)])
+def test_tiles_of_weight_gradients(m, n, k, tile):
+    assert gemm_plan(m, n, k, 0)[0] == tile
+
+
 # one row's workgroups of 64 (float32: 32) positions at the line up to which short sequences go in one launch
 ONE_LAUNCH = [(_lib.BF16, 256, 12, 64, 64), (_lib.BF16, 197, 12, 64, 64), (_lib.F16, 256, 8, 64, 128), (_lib.BF16, 256, 12, 64, 32), (_lib.BF16, 64, 48, 64, 64),
               (_lib.BF16, 128, 24, 64, 64), (_lib.F32, 256, 16, 32, 16), (_lib.F32, 256, 10, 32, 32), (_lib.F32, 192, 4, 64, 64), (_lib.F32, 64, 24, 32, 16),
