@@ -57,6 +57,7 @@ struct Api {
     decltype(&bimamba2_norm_scan_conv_bwd) norm_scan_conv_bwd = nullptr;
     decltype(&bimamba2_gemm) gemm = nullptr;
     decltype(&bimamba2_gemm_workspace_bytes) gemm_workspace = nullptr;
+    decltype(&bimamba2_gemm_plan) gemm_plan = nullptr;
 } api;
 
 void load(const std::string &path) {
@@ -92,6 +93,7 @@ void load(const std::string &path) {
     get(api.norm_scan_conv_bwd, "bimamba2_norm_scan_conv_bwd");
     get(api.gemm, "bimamba2_gemm");
     get(api.gemm_workspace, "bimamba2_gemm_workspace_bytes");
+    get(api.gemm_plan, "bimamba2_gemm_plan");
 }
 
 void check(int rc, const char *entry) {
@@ -648,8 +650,8 @@ bimamba2_norm_params layer_norm_params(const LayerShape &s, const LayerOpts &o, 
 
 // ---- the projections' matrix products -------------------------------------------------------------------------------
 // c (m x n, row pitch ldc) = sum_k A(m, k) B(n, k) (+ bias), by this library's kernel; false where it does not take the problem.
-// a, b: 2-d with unit stride along columns; a_kc: k along a's columns (else along its rows), b_kc likewise.  uncut: nor one whose sum it cuts in slices.
-bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const Tensor &bias, const Tensor &c, bool uncut = false) {
+// a, b: 2-d with unit stride along columns; a_kc: k along a's columns (else along its rows), b_kc likewise.
+bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const Tensor &bias, const Tensor &c) {
     if (c.scalar_type() == at::kFloat || a.stride(1) != 1 || b.stride(1) != 1 || c.stride(1) != 1) return false;
     bimamba2_gemm_params g{};
     g.m = c.size(0);
@@ -667,7 +669,6 @@ bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const T
     g.c = c.mutable_data_ptr();
     g.stream = stream_of(c);
     const size_t need = api.gemm_workspace(&g);
-    if (need && uncut) return false;
     Tensor ws;
     if (need) {
         ws = device_empty({(int64_t)need}, at::kByte, c);
@@ -694,9 +695,8 @@ constexpr double OWN_INFERENCE_FLOPS = 1.5e9, OWN_TRAINING_FLOPS = 3e9, OWN_GRAD
 // Two kinds go further (replayed graphs, operands from memory; own over library):
 //   forward products whose columns are no multiple of 64, below 16384 rows: 0.89 of the better of the library alone and in two parts (see SPLIT_ROWS) over the 14
 //     of 60 sampled ones with 3 to 20 GFLOP, 0.69 (8572 x 512 by 2192) to 1.11 (488 x 960 by 4382); above 20 1.0 to 1.27
-//   gradients of inputs with twice as many terms as columns (in front of the first projection): 0.84 over 44, 0.63 (155 x 960 from 3998) to 1.06; where
-//     the sum is cut and has more than 20 GFLOP up to 1.30 (5448 x 896 from 3868), and the library keeps it
-constexpr double OWN_RAGGED_FLOPS = 20e9, OWN_CUT_GRADIENT_FLOPS = 20e9;
+//   gradients of inputs: own_input_gradient()
+constexpr double OWN_RAGGED_FLOPS = 20e9;
 constexpr int64_t OWN_RAGGED_ROWS = 16384;
 
 // From so many rows or operations on, the columns of a forward product behind the last multiple of 256 go to the own kernel where the
@@ -724,11 +724,30 @@ void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c, 
     else at::mm_out(c, x, w.t());
 }
 
+// Whether the gradient of a projection's input (rows x columns, a sum of `terms`) goes to the own kernel.  Beyond the line above, with twice as many terms as columns (in
+// front of the first projection), own over library, replayed graphs, operands from memory, 403 products of layers of 128 to 4096 columns over 64 to 65536 rows:
+//   below 2560 rows, where the library does not cut the sum: 0.70 over 130, 0.37 (128 x 3328 from 13672) to 0.99
+//   large tiles, the sum in one piece, up to 1024 columns, 256 x 256 tiles from 384 columns on: 0.91 over 62, 0.74 (16960 x 1024 from 4384) to 1.09 (35085 x 512 from
+//     2320), six of them above 1.02; 16384 x 768 from 3224 82 -> 71 us
+//   the other 211, which the library keeps: 0.98, up to 1.31 (10736 x 576 from 2834; 14629 x 1280 from 5288 207 -> 258 us, 9152 x 1984 from 8126 285 -> 366)
+bool own_input_gradient(int64_t rows, int64_t columns, int64_t terms) {
+    if (2.0 * rows * columns * terms <= OWN_GRADIENT_FLOPS) return true;
+    if (terms < 2 * columns || columns > 4096) return false;
+    if (rows < 2560) return true;
+    if (columns > 1024) return false;
+    bimamba2_gemm_params g{};
+    g.m = rows;
+    g.n = columns;
+    g.k = terms;
+    g.a_kcontig = 1;
+    int slices = 0;
+    const int tile = api.gemm_plan(&g, &slices);
+    return slices == 1 && (tile == 1 || (tile == 0 && columns >= 384));
+}
+
 // c = dy w: the gradient of a projection's input
 void product_nn(const Tensor &dy, const Tensor &w, Tensor c) {
-    const double flops = 2.0 * c.size(0) * c.size(1) * dy.size(1);
-    const bool longer = dy.size(1) >= 2 * c.size(1);
-    if ((longer || flops <= OWN_GRADIENT_FLOPS) && own_product(dy, true, w, false, Tensor(), c, flops > OWN_CUT_GRADIENT_FLOPS)) return;
+    if (own_input_gradient(c.size(0), c.size(1), dy.size(1)) && own_product(dy, true, w, false, Tensor(), c)) return;
     at::mm_out(c, dy, w);
 }
 
@@ -973,5 +992,6 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     });
     m.def("load", &load);
     m.def("scan", &scan, py::call_guard<py::gil_scoped_release>());
+    m.def("own_input_gradient", &own_input_gradient);
     m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
 }

@@ -417,6 +417,14 @@ def test_tiles_of_weight_gradients(m, n, k, tile):
     assert gemm_plan(m, n, k, 0)[0] == tile
 
 
+# us by the library and by the own kernel: 207 and 258, 285 and 366, 776 and 879, 42 and 53, 129 and 150; 128 and 47, 82 and 71; then the edges of the rule
+@pytest.mark.parametrize("rows,columns,terms,own", [(14629, 1280, 5288, False), (9152, 1984, 8126, False), (21882, 2176, 8900, False), (30528, 256, 1544, False), (5760, 1600, 6706, False),
+                                                    (128, 3328, 13672, True), (16384, 768, 3224, True),
+                                                    (2559, 1536, 6320, True), (2560, 1536, 6320, False), (1000, 4160, 20600, False), (512, 768, 1536, True), (65536, 384, 300, False)])
+def test_input_gradients_that_go_to_the_own_kernel(rows, columns, terms, own):
+    assert _lib.host().own_input_gradient(rows, columns, terms) == own
+
+
 # one row's workgroups of 64 (float32: 32) positions at the line up to which short sequences go in one launch
 ONE_LAUNCH = [(_lib.BF16, 256, 12, 64, 64), (_lib.BF16, 197, 12, 64, 64), (_lib.F16, 256, 8, 64, 128), (_lib.BF16, 256, 12, 64, 32), (_lib.BF16, 64, 48, 64, 64),
               (_lib.BF16, 128, 24, 64, 64), (_lib.F32, 256, 16, 32, 16), (_lib.F32, 256, 10, 32, 32), (_lib.F32, 192, 4, 64, 64), (_lib.F32, 64, 24, 32, 16),
