@@ -692,12 +692,11 @@ bool own_product(const Tensor &a, bool a_kc, const Tensor &b, bool b_kc, const T
 //   gradients of the inputs: 197 x 384 241 -> 214, 170 -> 163; 512 x 768 240 -> 230, 231 -> 228; 512 x 1024 273 -> 264, 270 -> 262; 2048 x 768 (4.8 for
 //     the second) 314 -> 316, 313 -> 314
 constexpr double OWN_INFERENCE_FLOPS = 1.5e9, OWN_TRAINING_FLOPS = 3e9, OWN_GRADIENT_FLOPS = 5e9;
-// Two kinds go further (replayed graphs, operands from memory; own over library):
-//   forward products whose columns are no multiple of 64, below 16384 rows: 0.89 of the better of the library alone and in two parts (see SPLIT_ROWS) over the 14
-//     of 60 sampled ones with 3 to 20 GFLOP, 0.69 (8572 x 512 by 2192) to 1.11 (488 x 960 by 4382); above 20 1.0 to 1.27
-//   gradients of inputs: own_input_gradient()
-constexpr double OWN_RAGGED_FLOPS = 20e9;
-constexpr int64_t OWN_RAGGED_ROWS = 16384;
+// Gradients of inputs go further: own_input_gradient().  So do forward products whose columns are no multiple of 64 (the library has fast kernels for some of these
+// numbers only), of 1024 to 4095 rows, 256 to 576 inputs and up to 2600 columns: 0.82 of the library's time over 30 with 3 GFLOP and more, 0.73 to 1.04, 0.77 over 16 with
+// 1.5 to 3 (replayed graphs, operands from memory).  The others of 227 such products of 3 to 20 GFLOP below 16384 rows: fewer rows 1.15, 0.93 to 1.53 (116 x 2176 by 8900 19 ->
+// 29 us), other inputs 0.99, 0.76 to 1.37, more rows 1.00 of what SPLIT_ROWS gives, 0.59 to 1.57 (15617 x 192 by 1030 16 -> 25).
+constexpr int64_t RAGGED_ROWS = 1024, RAGGED_ROWS_END = 4096, RAGGED_INPUTS = 256, RAGGED_INPUTS_END = 577, RAGGED_COLUMNS_END = 2601;
 
 // From so many rows or operations on, the columns of a forward product behind the last multiple of 256 go to the own kernel where the
 // number of columns is no multiple of 64: the library has fast kernels for some of these numbers only.  us, library alone -> in
@@ -708,12 +707,17 @@ constexpr int64_t OWN_RAGGED_ROWS = 16384;
 constexpr int64_t SPLIT_ROWS = 4096;
 constexpr double SPLIT_FLOPS = 25e9;
 
+// whether a forward product (rows x columns, a sum of `inputs`) goes to the own kernel
+bool own_forward_product(int64_t rows, int64_t columns, int64_t inputs, bool training) {
+    if (2.0 * rows * columns * inputs <= (training ? OWN_TRAINING_FLOPS : OWN_INFERENCE_FLOPS)) return true;
+    return columns % 64 && rows >= RAGGED_ROWS && rows < RAGGED_ROWS_END && inputs >= RAGGED_INPUTS && inputs < RAGGED_INPUTS_END && columns < RAGGED_COLUMNS_END;
+}
+
 // c = x w^T (+ bias): the forward product.  c may be a view with a row pitch.
 void product_nt(const Tensor &x, const Tensor &w, const Tensor &bias, Tensor c, bool training) {
     const int64_t m = c.size(0), n = c.size(1), whole = n / 256 * 256;
     const double per_column = 2.0 * m * x.size(1);
-    const bool ragged = n % 64 && m < OWN_RAGGED_ROWS;
-    if (per_column * n <= (ragged ? OWN_RAGGED_FLOPS : training ? OWN_TRAINING_FLOPS : OWN_INFERENCE_FLOPS) && own_product(x, true, w, true, bias, c)) return;
+    if (own_forward_product(m, n, x.size(1), training) && own_product(x, true, w, true, bias, c)) return;
     if ((m >= SPLIT_ROWS || per_column * whole >= SPLIT_FLOPS) && n % 64 && whole && c.scalar_type() != at::kFloat && !bias.defined() &&
         own_product(x, true, w.narrow(0, whole, n - whole), true, Tensor(), c.narrow(1, whole, n - whole))) {
         Tensor front = c.narrow(1, 0, whole);
@@ -992,6 +996,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     });
     m.def("load", &load);
     m.def("scan", &scan, py::call_guard<py::gil_scoped_release>());
+    m.def("own_forward_product", &own_forward_product);
     m.def("own_input_gradient", &own_input_gradient);
     m.def("layer", &layer, py::call_guard<py::gil_scoped_release>());
 }

@@ -425,6 +425,17 @@ def test_input_gradients_that_go_to_the_own_kernel(rows, columns, terms, own):
     assert _lib.host().own_input_gradient(rows, columns, terms) == own
 
 
+# us before and by the own kernel: 19 and 29, 32 and 41, 16 and 25, 28 and 38, 12 and 13; 21 and 16, 14 and 10; then the edges of the rule
+@pytest.mark.parametrize("rows,columns,inputs,own", [(116, 8900, 2176, False), (128, 13672, 3328, False), (15617, 1030, 192, False), (600, 7738, 1856, False), (1032, 2708, 640, False),
+                                                     (3712, 2062, 448, True), (1344, 2320, 512, True),
+                                                     (1000, 2578, 576, True), (1023, 4384, 576, False), (4095, 2318, 448, True), (4096, 2318, 448, False), (3000, 2304, 512, False),
+                                                     (3000, 2708, 640, False), (3000, 3000, 576, False)])
+def test_forward_products_that_go_to_the_own_kernel(rows, columns, inputs, own):
+    """in training; without gradients the line for small ones is at 1.5 GFLOP"""
+    assert _lib.host().own_forward_product(rows, columns, inputs, True) == own
+    assert _lib.host().own_forward_product(rows, columns, inputs, False) == (own and (rows >= 1024 or 2 * rows * columns * inputs <= 1.5e9))
+
+
 # one row's workgroups of 64 (float32: 32) positions at the line up to which short sequences go in one launch
 ONE_LAUNCH = [(_lib.BF16, 256, 12, 64, 64), (_lib.BF16, 197, 12, 64, 64), (_lib.F16, 256, 8, 64, 128), (_lib.BF16, 256, 12, 64, 32), (_lib.BF16, 64, 48, 64, 64),
               (_lib.BF16, 128, 24, 64, 64), (_lib.F32, 256, 16, 32, 16), (_lib.F32, 256, 10, 32, 32), (_lib.F32, 192, 4, 64, 64), (_lib.F32, 64, 24, 32, 16),
