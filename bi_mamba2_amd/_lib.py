@@ -51,7 +51,7 @@ NORM_ENTRY_POINTS = ("bimamba2_rmsnorm_gated_fwd", "bimamba2_rmsnorm_gated_bwd")
 CONV_ENTRY_POINTS = ("bimamba2_conv1d_silu_fwd", "bimamba2_conv1d_silu_bwd")
 ALL_SYMBOLS = ENTRY_POINTS + ("bimamba2_strerror", "bimamba2_version", "bimamba2_params_size",
                               "bimamba2_workspace_bytes", "bimamba2_chunk_for", "bimamba2_seq_boundaries", "bimamba2_chunk_scan_reads_cb", "bimamba2_state_copies",
-                              "bimamba2_chunk_scan_heads_per_workgroup", "bimamba2_fwd_one_launch", "bimamba2_ddt_direct_planes", "bimamba2_norm_params_size",
+                              "bimamba2_chunk_scan_heads_per_workgroup", "bimamba2_fwd_one_launch", "bimamba2_bwd_db_dc_complete", "bimamba2_ddt_direct_planes", "bimamba2_norm_params_size",
                               "bimamba2_rmsnorm_gated_workspace_bytes", "bimamba2_conv_params_size",
                               "bimamba2_conv1d_silu_workspace_bytes", "bimamba2_cast_params_size",
                               "bimamba2_cast_many", "bimamba2_norm_scan_conv_bwd", "bimamba2_gemm_params_size", "bimamba2_gemm_workspace_bytes", "bimamba2_gemm_plan", "bimamba2_gemm") + NORM_ENTRY_POINTS + CONV_ENTRY_POINTS
@@ -123,6 +123,8 @@ def load():
     lib.bimamba2_chunk_scan_heads_per_workgroup.restype = ctypes.c_int
     lib.bimamba2_fwd_one_launch.argtypes = [ctypes.POINTER(Params)]
     lib.bimamba2_fwd_one_launch.restype = ctypes.c_int
+    lib.bimamba2_bwd_db_dc_complete.argtypes = [ctypes.POINTER(Params)]
+    lib.bimamba2_bwd_db_dc_complete.restype = ctypes.c_int
     lib.bimamba2_ddt_direct_planes.argtypes = [ctypes.POINTER(Params)]
     lib.bimamba2_ddt_direct_planes.restype = ctypes.c_int
     lib.bimamba2_seq_boundaries.argtypes = [ctypes.POINTER(Params), _vp]

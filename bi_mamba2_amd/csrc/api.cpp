@@ -557,6 +557,36 @@ int bimamba2_fwd_static(const bimamba2_params *p) {
     return bimamba2_fwd(&q);
 }
 
+// Which launches of a backward pass are there in a merged form; q: the caller's p with what it leaves to the pass carved
+struct BwdForm {
+    bool one;           // one chunk without states (a forward pass over one chunk leaves none: its caller says so)
+    bool own_dcb;       // dCB and dCB^T are the pass's own
+    bool dcb_sp;        // dCB with the backward state passing (one chunk: dCB's alone, with its place for 16-bit results)
+    bool dcb16;         // dCB in the 16-bit element type: the two launches that write and read it are the merged ones (their reader rounds it to that type for its MFMA anyway)
+    bool dx_db_dc;      // dx, dB and dC in one launch at the end
+    bool by_heads;      // dB and dC in one launch, heads in turn
+    bool product;       // and the part of both inside the chunks with them, where nobody asked for the partial sums
+};
+static BwdForm bwd_form(const bimamba2_params *p, const bimamba2_params *q) {
+    BwdForm f;
+    f.one = one_chunk(q) && (!p->fwd_saved || (p->fwd_saved & 4));
+    f.own_dcb = !p->dCB && !p->dCBT;
+    f.dcb_sp = (f.one ? dcb_recomputes_cb(q) && (q->headdim * q->dstate) % 4 == 0 : bwd_dcb_sp_merged(q)) && (f.own_dcb || dcb_slices(q) == 1);
+    f.dcb16 = f.own_dcb && f.dcb_sp && dcb_slices(q) == 1 && bwd_tail_merged(q);
+    f.dx_db_dc = !f.one && dx_db_dc_merged(q);
+    f.by_heads = !f.one && !f.dx_db_dc && dbdc_both_by_heads(q);
+    f.product = f.by_heads && f.dcb16 && !p->dBs && !p->dCs && dbdc_with_product(q);
+    return f;
+}
+
+int bimamba2_bwd_db_dc_complete(const bimamba2_params *p) {
+    if (check_problem(p)) return 0;
+    bimamba2_params q = *p;
+    q.final_f = q.final_b = nullptr;
+    carve(&q, 1, reinterpret_cast<void *>(256));      // (a place to count from: nothing is read or written)
+    return bwd_form(p, &q).product ? 1 : 0;
+}
+
 // leave: the final sums are appended to it instead of being launched
 static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     TRY(check_problem(p));
@@ -571,8 +601,8 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     if (q.has_dt_bias) REQUIRE(q.dt_bias);
     if (q.has_D) { REQUIRE(q.D); REQUIRE(q.dD); }
     if (q.has_z) { REQUIRE(q.z); REQUIRE(q.out_x); REQUIRE(q.dz); }
-    // (a forward pass over one chunk leaves no states: its caller says so)
-    const bool one = one_chunk(&q) && (!p->fwd_saved || (p->fwd_saved & 4));
+    const BwdForm form = bwd_form(p, &q);
+    const bool one = form.one, own_dcb = form.own_dcb, dcb_sp = form.dcb_sp, dcb16 = form.dcb16;
     if (p->fwd_saved) {
         REQUIRE(p->dt_out); REQUIRE(p->cs_f); REQUIRE(p->cs_b);
         if (!p->states16_f && !one) { REQUIRE(p->states_f); REQUIRE(p->states_b); }
@@ -596,12 +626,6 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
         for (float *t : {p->dBs, p->dCs})
             if (t) TRY(launch_fill(t, sums, 0.f, stream_of(&q)));
     }
-    // dCB / dCBT in the 16-bit element type where this call owns them and the two launches that write and read them are the
-    // merged ones (their reader rounds them to that type for its MFMA anyway)
-    // (without states to pass the launch is dCB's alone, with its place for 16-bit results)
-    const bool own_dcb = !p->dCB && !p->dCBT;
-    const bool dcb_sp = (one ? dcb_recomputes_cb(&q) && (q.headdim * q.dstate) % 4 == 0 : bwd_dcb_sp_merged(&q)) && (own_dcb || dcb_slices(&q) == 1);
-    const bool dcb16 = own_dcb && dcb_sp && dcb_slices(&q) == 1 && bwd_tail_merged(&q);
     const bool need_cbt = !scan_recomputes_cb(&q, true), need_cb = need_cbt || !dcb_recomputes_cb(&q);
     const bool saved_cb = (p->fwd_saved & 2) && p->CB && p->CBT;
     const bool form_cb = need_cb && !saved_cb;     // (else left there by the forward pass)
@@ -619,10 +643,8 @@ static int backward(const bimamba2_params *p, ReduceJobs *leave) {
     const int ncb = own_dcb && (tail_small || bwd_tail_merged(&q)) ? dcb_slices(&q) : 1;
     // the dCB kernel is bound by instruction issue and moves little data: right behind dz it runs while the memory system
     // still writes back dz's output, which the memory-bound kernels after it would otherwise wait behind
-    const bool dx_db_dc = !one && dx_db_dc_merged(&q);      // (one launch at the end)
-    const bool by_heads = !one && !dx_db_dc && dbdc_both_by_heads(&q), both = by_heads || (!one && !dx_db_dc && db_dc_merged(&q));      // dC with dB
-    // and the part of both inside the chunks with them, where dCB is there in 16 bits and nobody asked for the partial sums
-    const bool product = by_heads && dcb16 && !p->dBs && !p->dCs && dbdc_with_product(&q);
+    const bool dx_db_dc = form.dx_db_dc, by_heads = form.by_heads, product = form.product;
+    const bool both = by_heads || (!one && !dx_db_dc && db_dc_merged(&q));      // dC with dB
     if (dcb_sp && (ncb == dcb_slices(&q))) {
         // the backward state passing (streams, few instructions) rides along with the dCB kernel in one launch
         if (!dx_db_dc && !one && !both) TRY(bimamba2_chunk_scan_bwd_dc(&q));

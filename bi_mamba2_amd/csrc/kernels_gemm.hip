@@ -34,7 +34,7 @@ template <int BM, int BN, int WR, int WC> struct GemmTile {
     static constexpr int A_B = BM * GK * 2, B_B = BN * GK * 2, SLOT = A_B + B_B;
     static constexpr int LOADS = (BM + BN) / 16 / WAVES;              // requests of a wave per step (1 KB each)
     static_assert((BM + BN) / 16 % WAVES == 0 && BM / 16 % WAVES == 0, "a wave's requests lie in one operand each");
-    static_assert(NT % 2 == 0 && MT >= 1, "pairs of column tiles");
+    static_assert(NT % 2 == 0 && NT <= 4 && MT <= 4, "pairs of column tiles; what the fragment reads below are written out for");
 };
 
 // the large kernel's tiles: MT x NT tiles of 16 a wave, 2 x 2 waves; BRING slots in its ring
@@ -226,7 +226,7 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const bimamba2_gemm_
         if constexpr (AKC) {
             const unsigned a0 = a_l[0] + so;
 #define BM2_RA(J) if constexpr (J < MT) f.a[J] = raw_lds_read_at<Frag, J * 1024>(a0)
-            BM2_RA(0); BM2_RA(1); BM2_RA(2); BM2_RA(3); BM2_RA(4); BM2_RA(5); BM2_RA(6); BM2_RA(7);
+            BM2_RA(0); BM2_RA(1); BM2_RA(2); BM2_RA(3);
 #undef BM2_RA
         } else {
             constexpr bool WHOLE = MT % 4 == 0;                // a wave owns whole 64-column blocks (else half of one)
@@ -234,12 +234,12 @@ __global__ __launch_bounds__(64 * WR * WC) void gemm_kernel(const bimamba2_gemm_
             unsigned ta[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) ta[j] = (WHOLE ? a_l[j] : a_l[(j + 2 * (wm & 1)) & 3]) + blk;
-#define BM2_RA(J)                                                                  \
-    if constexpr (J < MT) {                                                        \
-        f.al[J] = raw_lds_tr16_read_at<(J >> 2) * 4096>(ta[J & 3]);                \
-        f.ah[J] = raw_lds_tr16_read_at<(J >> 2) * 4096 + 512>(ta[(J & 3) ^ 2]);    \
+#define BM2_RA(J)                                          \
+    if constexpr (J < MT) {                                \
+        f.al[J] = raw_lds_tr16_read_at<0>(ta[J]);          \
+        f.ah[J] = raw_lds_tr16_read_at<512>(ta[J ^ 2]);    \
     }
-            BM2_RA(0) BM2_RA(1) BM2_RA(2) BM2_RA(3) BM2_RA(4) BM2_RA(5) BM2_RA(6) BM2_RA(7)
+            BM2_RA(0) BM2_RA(1) BM2_RA(2) BM2_RA(3)
 #undef BM2_RA
         }
     };

@@ -227,6 +227,10 @@ int bimamba2_chunk_scan_heads_per_workgroup(const bimamba2_params *p, int bwd);
  * workgroups that own whole sequences (the same result in bits).  Pointers that are not set yet count as aligned.  A measurement aid. */
 int bimamba2_fwd_one_launch(const bimamba2_params *p);
 
+/* Whether bimamba2_bwd of this problem writes dB and dC from the launch that sums their state parts (1), or leaves the part inside the chunks to
+ * its last launch (0).  `p` as it will be passed; the workspace may be missing.  A measurement aid. */
+int bimamba2_bwd_db_dc_complete(const bimamba2_params *p);
+
 /* Whole forward; replaces _mamba_chunk_scan_combined_fwd (src/ssd/bi/ssd_combined.py:297-331).
  * Needs: x dt A Bm Cm [D z dt_bias] out [out_x when has_z] [final_f final_b] workspace.  Intermediates given as
  * non-NULL pointers (dt_out cs_f cs_b CB CBT states_f states_b) are filled in place of workspace memory, so a

@@ -1,9 +1,12 @@
 """dB and dC complete from the launch that sums their state parts (one slice of heads, chunks of 256, 16 bits), against the two launches that
 run where the caller brings dCB in float32: the same products in the same order, so the same bits."""
 
+import ctypes
+
 import pytest
 import torch
 
+from bi_mamba2_amd import _lib
 from tests.helpers import make_case, to_dev
 
 pytestmark = pytest.mark.gpu
@@ -29,16 +32,25 @@ def grads(ops, d, dout, Q=256):
 def compare(ops, monkeypatch, d, dout):
     b, L = d["x"].shape[:2]
     G, N = d["B"].shape[2:]
-    got, ws = grads(ops, d, dout), ops._Call.workspace
+    ws, complete = ops._Call.workspace, []
+
+    def asked(call, is_bwd):
+        ws(call, is_bwd)
+        if is_bwd:
+            complete.append(_lib.load().bimamba2_bwd_db_dc_complete(ctypes.byref(call.p)))
+
+    monkeypatch.setattr(ops._Call, "workspace", asked)
+    got = grads(ops, d, dout)
 
     def with_dcb(call, is_bwd):
         if is_bwd:
             for field in ("dCB", "dCBT"):
                 call.new(field, (b, -(-L // 256), G, 256, 256))
-        return ws(call, is_bwd)
+        return asked(call, is_bwd)
 
     monkeypatch.setattr(ops._Call, "workspace", with_dcb)
     want = grads(ops, d, dout)
+    assert complete == [1, 0]
     seen = 0
     for a, c in zip(got, want):
         assert (a is None) == (c is None)

@@ -454,6 +454,16 @@ def test_short_sequences_in_any_batch(dtype, seqlen, heads, headdim, dstate):
     assert form(64, causal=1) == form(64, initial_f=256) == form(64, states_f=256) == 0
 
 
+def test_gradients_of_b_and_c_complete_from_one_launch():
+    """one slice of heads, chunks of 256, at least 16 (batch, chunk, group), and nobody asked for what the launch would leave out"""
+    lib = _lib.load()
+    form = lambda **kw: lib.bimamba2_bwd_db_dc_complete(ctypes.byref(_params(**{**dict(
+        batch=2, seqlen=2048, nheads=8, headdim=64, ngroups=2, dstate=64, chunk_size=256, x_sb=2048 * 512, x_sl=512, x_sh=64, dout_sb=2048 * 512, dout_sl=512, dout_sh=64,
+        B_sb=2048 * 128, B_sl=128, B_sg=64, C_sb=2048 * 128, C_sl=128, C_sg=64), **kw})))
+    assert form() == form(dtype=_lib.F16) == form(seqlen=1793) == 1
+    assert form(batch=1, seqlen=1792) == form(chunk_size=128) == form(dtype=_lib.F32) == form(dBs=256) == form(dCB=256) == form(dstates_f=256) == form(B_sl=129) == 0
+
+
 @pytest.mark.parametrize("name,function", [("kernels_gemm.hip", "store_tile"), ("kernels_scan_once.hip", "scan_once_kernel"), ("kernels_scan_once.hip", "scan_once_walk_kernel")])
 def test_no_bare_barrier_in_front_of_ordinary_lds_accesses(name, function):
     """these write LDS by stores that the compiler knows of, where other waves read before: s_barrier alone does not keep it from moving them up"""
