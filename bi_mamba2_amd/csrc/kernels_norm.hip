@@ -37,21 +37,16 @@ template <typename T> __device__ __forceinline__ void load8(const T *ptr, bool v
         for (int i = 0; i < 8; ++i) v[i] = i < ncol ? to_f(ptr[i]) : 0.f;
     }
 }
-// the same as they lie in memory: nothing waits for them before they are used
-template <typename T> __device__ __forceinline__ void load8_raw(const T *ptr, bool vec, int ncol, T (&v)[8]) {
-    if (vec && ncol >= 8) {
-        if constexpr (sizeof(T) == 2) {
-            const Vec16<T> raw = *reinterpret_cast<const Vec16<T> *>(ptr);
+// a whole piece as it lies in memory: nothing waits for it before it is used
+template <typename T> __device__ __forceinline__ void load8_raw(const T *ptr, T (&v)[8]) {
+    if constexpr (sizeof(T) == 2) {
+        const Vec16<T> raw = *reinterpret_cast<const Vec16<T> *>(ptr);
 #pragma unroll
-            for (int i = 0; i < 8; ++i) v[i] = raw.v[i];
-        } else {
-            const f32x4 a = *reinterpret_cast<const f32x4 *>(ptr), b = *reinterpret_cast<const f32x4 *>(ptr + 4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) { v[i] = a[i]; v[i + 4] = b[i]; }
-        }
+        for (int i = 0; i < 8; ++i) v[i] = raw.v[i];
     } else {
+        const f32x4 a = *reinterpret_cast<const f32x4 *>(ptr), b = *reinterpret_cast<const f32x4 *>(ptr + 4);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = i < ncol ? ptr[i] : from_f<T>(0.f);
+        for (int i = 0; i < 4; ++i) { v[i] = a[i]; v[i + 4] = b[i]; }
     }
 }
 template <typename T> __device__ __forceinline__ void store8(T *ptr, bool vec, int ncol, const float (&v)[8]) {
@@ -72,11 +67,20 @@ template <typename T> __device__ __forceinline__ void store8(T *ptr, bool vec, i
     }
 }
 
-// FULL: the group is exactly NCH * 512 columns wide and every access is a 16-byte one (the host checked it); the weights are
-// then requested together with the row, in front of the reduction.
-template <typename T, int NCH, bool FULL>
-__global__ __launch_bounds__(NTHREADS) void rmsnorm_gated_fwd_kernel(const bimamba2_norm_params p, bool vec_, bool wvec_) {
-    const bool vec = FULL || vec_, wvec = FULL || wvec_;
+// ROWS: what the host checked.  NORM_PIECES: groups of whole pieces, every access to a row a 16-byte one.  NORM_FULL: and the group is exactly
+// NCH * 512 columns wide; the weights are then requested together with the row, in front of the reduction.
+//
+// Everything of a row is requested before anything is used; z is kept as loaded between the passes.  (A gate applied piece by piece waits for each piece
+// of z before the next is asked for: 16384 rows of 1536 columns, bfloat16, 34.7 us, as here 30.0, 151 MB at 5.0 TB/s.)  That pays only where a request is no
+// branch: 16-bit values that leave one are taken apart inside it, each piece waited for.  So a piece behind the group's end asks for the last one and is
+// cleared, and rows without 16-byte accesses ask element by element only in the piece that the group's end cuts.  us, gate piece by piece / requested in
+// front but in branches / as here: bfloat16, 16384 rows of 768 columns 23.8 / 28.9 / 22.2, of 3072 128 / 140 / 75, 48864 of 1408 116 / 134 / 82, 16384 of 1001 (no
+// 16-byte accesses) 81 / 72 / 54; float32, 16384 of 1152 52 / 49 / 43, of 1001 111 / 111 / 74.  Fewer rows gain less (2000 of 768 6.3 / 6.8 / 5.3), none measured lost.
+enum { NORM_ANY, NORM_PIECES, NORM_FULL };
+template <typename T, int NCH, int ROWS>
+__global__ __launch_bounds__(NTHREADS) void rmsnorm_gated_fwd_kernel(const bimamba2_norm_params p, bool wvec_) {
+    constexpr bool FULL = ROWS == NORM_FULL, vec = ROWS != NORM_ANY;
+    const bool wvec = FULL || wvec_;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int ngroups = p.cols / p.group_size, gs = FULL ? NCH * 512 : p.group_size;
     const int64_t item = (int64_t)blockIdx.x * 4 + wave;
@@ -88,21 +92,31 @@ __global__ __launch_bounds__(NTHREADS) void rmsnorm_gated_fwd_kernel(const bimam
     T *out = reinterpret_cast<T *>(p.out) + row * p.out_rs + g * gs;
     const float *w = p.weight + g * gs, *bias = p.has_bias ? p.bias + g * gs : nullptr;
     const bool gate_first = p.has_z && !p.norm_before_gate;
-    // Everything is requested before anything is used; z is kept as loaded between the passes.  (A gate applied piece by piece waited for each piece
-    // of z before the next was asked for: 16384 rows of 1536 columns, bfloat16, 36.2 us, as here 29.5, 151 MB at 5.1 TB/s.)
     float xv[NCH][8];
-    T xk[NCH][8], zk[NCH][8];
+    T zk[NCH][8];
     float ss = 0.f;
+    float wk[FULL ? NCH : 1][8];
+    T xk[NCH][8];
+    auto request = [&](const T *r, int k, T (&v)[8]) {
+        const int c = (k * 64 + lane) * 8;
+        if constexpr (vec) load8_raw(r + (FULL ? c : min(c, gs - 8)), v);
+        else if (c + 8 <= gs) {
 #pragma unroll
-    for (int k = 0; k < NCH; ++k) load8_raw(x + (k * 64 + lane) * 8, vec, FULL ? 8 : gs - (k * 64 + lane) * 8, xk[k]);
+            for (int i = 0; i < 8; ++i) v[i] = r[c + i];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = c + i < gs ? r[c + i] : from_f<T>(0.f);
+        }
+    };
+#pragma unroll
+    for (int k = 0; k < NCH; ++k) request(x, k, xk[k]);
     if (p.has_z) {
 #pragma unroll
-        for (int k = 0; k < NCH; ++k) load8_raw(z + (k * 64 + lane) * 8, vec, FULL ? 8 : gs - (k * 64 + lane) * 8, zk[k]);
+        for (int k = 0; k < NCH; ++k) request(z, k, zk[k]);
     }
-    float wk[FULL ? NCH : 1][8];
-    if (FULL) {
+    if constexpr (FULL) {
 #pragma unroll
-        for (int k = 0; k < NCH; ++k) load8(w + (k * 64 + lane) * 8, true, 8, wk[FULL ? k : 0]);
+        for (int k = 0; k < NCH; ++k) load8(w + (k * 64 + lane) * 8, true, 8, wk[k]);
     }
 #pragma unroll
     for (int k = 0; k < NCH; ++k)
@@ -113,6 +127,12 @@ __global__ __launch_bounds__(NTHREADS) void rmsnorm_gated_fwd_kernel(const bimam
         for (int k = 0; k < NCH; ++k)
 #pragma unroll
             for (int i = 0; i < 8; ++i) xv[k][i] *= silu_f(to_f(zk[k][i]));
+    }
+    if constexpr (ROWS == NORM_PIECES) {
+#pragma unroll
+        for (int k = 0; k < NCH; ++k)
+#pragma unroll
+            for (int i = 0; i < 8; ++i) xv[k][i] = (k * 64 + lane) * 8 < gs ? xv[k][i] : 0.f;
     }
     if (p.layer_norm) {
         float sm = 0.f;
@@ -540,10 +560,11 @@ static int launch_norm_nch(const bimamba2_norm_params *p, bool bwd, LayerSums *l
     const bool wvec = p->group_size % 4 == 0 && al(p->weight) && (!p->has_bias || al(p->bias));
     if (!bwd) {
         const int64_t items = (int64_t)p->rows * (p->cols / p->group_size);
-        if (vec && wvec && p->group_size == NCH * 512 && NCH <= 4)
-            hipLaunchKernelGGL((rmsnorm_gated_fwd_kernel<T, NCH, true>), dim3((unsigned)((items + 3) / 4)), dim3(NTHREADS), 0, stream_of(p), *p, vec, wvec);
-        else
-            hipLaunchKernelGGL((rmsnorm_gated_fwd_kernel<T, NCH, false>), dim3((unsigned)((items + 3) / 4)), dim3(NTHREADS), 0, stream_of(p), *p, vec, wvec);
+        const dim3 grid((unsigned)((items + 3) / 4)), block(NTHREADS);
+        constexpr int FULL = NCH <= 4 ? NORM_FULL : NORM_PIECES;
+        if (vec && wvec && p->group_size == NCH * 512) hipLaunchKernelGGL((rmsnorm_gated_fwd_kernel<T, NCH, FULL>), grid, block, 0, stream_of(p), *p, wvec);
+        else if (vec) hipLaunchKernelGGL((rmsnorm_gated_fwd_kernel<T, NCH, NORM_PIECES>), grid, block, 0, stream_of(p), *p, wvec);
+        else hipLaunchKernelGGL((rmsnorm_gated_fwd_kernel<T, NCH, NORM_ANY>), grid, block, 0, stream_of(p), *p, wvec);
         return check_launch();
     }
     const int nb = norm_row_blocks(p);

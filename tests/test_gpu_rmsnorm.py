@@ -57,6 +57,30 @@ def test_rmsnorm_gated_forward_backward(case, rms):
             assert_close(got.grad, r.grad, dtype, name)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("width", [8, 504, 512, 520, 768, 1016, 1032, 2040, 3080, 8184, 7, 511, 1001, 1025, 2111, 8191])
+def test_rows_that_end_inside_a_wave(width, dtype):
+    """forward: pieces of eight columns behind a row's end ask for the last one inside it, or for nothing.  What lies behind the row is not a number, and one
+    element of the last piece is large, so that a piece counted twice would show in the row's sum."""
+    from bi_mamba2_amd.layernorm_gated import layernorm_fn
+    rows, pitch = 5, (width + 71) // 8 * 8
+    g = torch.Generator().manual_seed(width)
+    x, z = (torch.full((rows, pitch), float("nan"), dtype=dtype, device="cuda") for _ in range(2))
+    values = [torch.randn(rows, width, generator=g).to(dtype) for _ in range(2)]
+    values[0][1, -1] = 200.0
+    values[1][2, -1] = float("inf")
+    for wide, v in zip((x, z), values):
+        wide[:, :width] = v.cuda()
+    w, b = (1 + 0.3 * torch.randn(width, generator=g)).float(), (0.2 * torch.randn(width, generator=g)).float()
+    for gated, before, rms in ((True, True, True), (True, False, True), (False, True, True), (True, True, False)):
+        out = layernorm_fn(x[:, :width], w.cuda(), b.cuda(), z=z[:, :width] if gated else None, eps=1e-5, norm_before_gate=before, is_rms_norm=rms)
+        ref = rms_norm_gated(values[0].double(), w.double(), b.double(), values[1].double() if gated else None, eps=1e-5, norm_before_gate=before, is_rms_norm=rms)
+        keep = torch.tensor([0, 1, 3, 4]) if gated else torch.arange(rows)      # the row with an infinite gate has no finite result
+        assert_close(out[keep.cuda()], ref[keep], dtype, "out")
+        if gated and before:
+            assert_close(out[2, :-1], ref[2, :-1], dtype, "the row whose last gate is infinite")
+
+
 def test_rmsnorm_strided_rows_and_module():
     """Rows that are views into a wider projection output (as in the layer), and the module with its parameter."""
     from bi_mamba2_amd.layernorm_gated import RMSNorm
