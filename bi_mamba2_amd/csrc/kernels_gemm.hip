@@ -346,7 +346,7 @@ template <int N, int MT, int NT> __device__ __forceinline__ void big_settle(f32x
 }
 
 // 256 x (32 NT) tiles.  What bounds it: the products of a step take 1024 (NT = 8) cycles of a SIMD's matrix unit and the step 1480 (8192 cubed: 765 us, 1437 TFLOP/s;
-// the unit is busy 69 % of the time), waits 10 %; a round of tiles adds 10 to 14 us of start, end and stores.  Four waves instead of the eight
+// the unit is busy 73 % of the time there, counted); a round of tiles adds 10 to 14 us of start, end and stores.  Four waves instead of the eight
 // of 128 x 64 that stood here: a wave's fragments serve twice the products, and its sums fill the accumulation registers.  A wave that is
 // alone on its SIMD covers nothing but by its own order: reads and requests stand one by one between the products (all of a row tile's in front of
 // its eight products: 819 us at 8192 cubed, one behind each 778).  Steps of 64 with two slots: 802 us.  What it gives: gemm_plan.

@@ -7,11 +7,10 @@
 // scan_once_kernel, for few rows of more than 128 positions: a workgroup (8 waves) owns 64 positions (float32: 32) of one (batch, head) and a tile of headdim columns.  It brings the sequence's x and B rows into
 // LDS, forms the head's decays itself, and its waves take 16 rows and every second (fourth) step of columns each.  Everything else such a pass is made of - the
 // chunk cumsum, C.B^T, the states and their passing - would be a launch of 3 to 8 us of its own, of which the work is a fraction.
-// Bound by the chain load - decays - barrier - steps - barrier - store, 5.5 us at 197 positions, 12 heads of 64 (bfloat16, dstate 64): 2.5 until
-// the decays stand, 1.9 for the steps, 1.1 for the rest.  What made it short: loads without conditions and without the LDS copies that a
-// struct in a select became (13 -> 5.5 us to the barrier), decays by four waves with row shifts instead of LDS permutes, two steps at a
-// time.  us a call, from the chunked launches: 2 x 256, 4 heads of 32, dstate 16, float32 18.0 -> 7.2; 1 x 197, 12 heads of 64, dstate 64, bfloat16 17.0 -> 7.9; 4 x 256, 8 heads of 128,
-// dstate 128 24.0 -> 9.7.  Error against 64 bits: float32 0.60 to 0.78 of the chunked pass's, float16 0.81 to 0.86, bfloat16 0.98 to 1.003.
+// Bound by the chain load - decays - barrier - steps - barrier - store, a few hundred workgroups at most: 8.2 us in the trace of a layer at 197 positions,
+// 12 heads of 64 (bfloat16, dstate 64, 48 workgroups).  What made it short: loads without conditions and without the LDS copies that a
+// struct in a select became, decays by four waves with row shifts instead of LDS permutes, two steps at a time.  us a call, from the chunked launches: 2 x 256, 4 heads of 32, dstate 16, float32 18.0 -> 7.2; 1 x 197, 12 heads of 64, dstate 64, bfloat16 17.0 -> 7.9; 4 x 256, 8 heads of 128,
+// dstate 128 24.0 -> 9.7.  Error against 64 bits: float32 0.60 to 1.0 of the chunked pass's, float16 0.81 to 0.86, bfloat16 0.98 to 1.000.
 // The decays are exact to the last rounding of an exponent: the sums are kept in 64 bits and only differences within a block of 16
 // positions, or between a row and a block's edge, are rounded to 32 (the chunked pass rounds the sums of a chunk).
 #include <algorithm>
@@ -246,7 +245,7 @@ __global__ __launch_bounds__(ONCE_THREADS) void scan_once_kernel(const bimamba2_
 // than 128 positions two, one after the other) and all columns: C.B^T is formed once and stays in registers, nothing is exchanged between waves, and a head's x and
 // decays are brought while the head before is worked on.  Steps, and which of them add up to which sum, are those of scan_once_kernel, so that the results
 // are the same bits and the number of rows may choose between the two (launch_scan_once).
-// Bound by vector instructions: at 256 x 256 positions, 12 heads of 64 (bfloat16, dstate 64, two waves a SIMD) they are issued 61 % of the time, two products and
+// Bound by vector instructions: at 256 x 256 positions, 12 heads of 64 (bfloat16, dstate 64, two waves a SIMD) they are issued 62 % of the time, two products and
 // half a conversion per pair of positions most of them; a head takes 6.3 us with the chip half empty and 8 with 256 workgroups on it.  What made it so:
 // whole columns a wave instead of shares that meet in LDS (four barriers a head less, 159 -> 127 us), results as 16-byte stores from the sums of transposed products,
 // z and x never waited for behind stores (118 -> 101), addresses by immediates.  us a call, scan_once_kernel for every 64 positions -> this one (before: the chunked launches):
